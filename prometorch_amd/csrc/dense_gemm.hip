@@ -1,6 +1,7 @@
 // Prompt products over bfloat16 weights: C[M][N] = A[M][K] . W[N][K]^T on the matrix cores.
 //
-// dense_gemm_kernel (bfloat16 rows): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
+// dense_gemm_tiles_kernel (more than 64 bfloat16 rows): the tiles of gemm_tile.h, as plan_tiles lays them out.
+// dense_gemm_kernel (up to 64 bfloat16 rows): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
 // LDS; two register sets and two LDS buffers, so a step has one barrier and the loads of the next two steps are in flight
 // while its MFMAs run.
 // LDS rows are 128 bytes, the eight 16-byte pieces of row r stored at piece ^ (r % 8): the fragment reads (32 rows, one
@@ -8,6 +9,10 @@
 // holds four consecutive columns of one output row.
 // dense_gemm_f32_kernel (fp32 rows): the same product in fp32 on v_mfma_f32_32x32x2_f32, 64 x 64 tiles.
 #include "dense.h"
+#include "gemm_tile.h"
+
+#include <algorithm>
+#include <mutex>
 
 namespace ptm {
 
@@ -20,6 +25,15 @@ __device__ __forceinline__ void tile_of(int wg, int tiles_m, int tiles_n, int& t
     const int id = xcd * per + min(xcd, rem) + i;
     tm = id % tiles_m;
     tn = id / tiles_m;
+}
+
+// the same for the larger tiles: runs of bands of four row tiles, so that the 32 tiles an XCD works on are about as high as wide
+__device__ __forceinline__ void band_tile_of(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int total = tiles_m * tiles_n, per = total / 8, rem = total % 8, xcd = wg % 8, i = wg / 8;
+    const int id = xcd * per + min(xcd, rem) + i;
+    const int band = id / (4 * tiles_n), r = id - band * 4 * tiles_n, rows = min(4, tiles_m - 4 * band);
+    tm = 4 * band + r % rows;
+    tn = r / rows;
 }
 
 __device__ __forceinline__ float relu2(float v) { return v > 0.0f ? v * v : 0.0f; }
@@ -189,6 +203,89 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const DenseGemm g) {
     }
 }
 
+// The same product on the tiles of gemm_tile.h, which take rows of both sides from memory to LDS directly.  A launch covers its output
+// with up to four regions of equal tiles.
+typedef GemmTile<gt_b8, 8, 4, 2, 2, 2> Tile0;
+typedef GemmTile<gt_b8, 4, 6, 4, 2, 2> Tile1;
+typedef GemmTile<gt_b8, 4, 4, 2, 2, 3> Tile2;
+typedef GemmTile<gt_b8, 2, 6, 4, 3, 3> Tile3;
+typedef GemmTile<gt_b8, 2, 4, 4, 3, 3> Tile4;
+typedef GemmTile<gt_b8, 2, 4, 2, 3, 3> Tile5;
+typedef GemmTile<gt_b8, 2, 2, 2, 3, 3> Tile6;
+
+template <typename Tile>
+__device__ __forceinline__ void dense_tile(const DenseGemm& g, const GemmRegion& r, int wg, uint8_t* lds) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int split = wg / (r.tiles_m * r.tiles_n);
+    int tm, tn;
+    band_tile_of(wg - split * r.tiles_m * r.tiles_n, r.tiles_m, r.tiles_n, tm, tn);
+    const int m0 = r.m0 + tm * Tile::BM, n0 = r.n0 + tn * Tile::BN;
+    const int all = (g.K + 63) / 64, first = all * split / g.splits, steps = all * (split + 1) / g.splits - first;
+    const uint16_t* A = static_cast<const uint16_t*>(g.A) + (int64_t)m0 * g.lda + first * 64;
+    if (g.section_n > 0) A += n0 / g.section_n * g.section_a;
+    // two-byte results: a lane's two sums next to each other make one 16-byte store (1030 x 9728 x 2560 63.0 -> 57.7 us); fp32 sums of
+    // one fragment are 16 bytes already, and the four lanes of a row then store 64 in a row
+    const bool glu = g.epilogue == GEMM_SWIGLU, pairs = g.epilogue == GEMM_ELEM || g.epilogue == GEMM_RELU2;
+    const int w0 = weight_row(g, n0);  // GEMM_SWIGLU: tiles start with whole blocks of 32 columns, so no row of the tile lies in front of it
+    const gt_i4 xs = gt_buffer(A), ws = gt_buffer(g.W + (int64_t)w0 * g.ldw + first * 64);
+    const uint32_t piece = ((lane & 7) ^ (lane >> 3)) << 4;
+    uint32_t xo[Tile::NX], wo[Tile::NW];
+#pragma unroll
+    for (int i = 0; i < Tile::NX; ++i) xo[i] = (uint32_t)min(8 * (wave + 8 * i) + (lane >> 3), g.M - 1 - m0) * (uint32_t)g.lda * 2 + piece;
+#pragma unroll
+    for (int i = 0; i < Tile::NW; ++i) wo[i] = (uint32_t)(weight_row(g, n0 + (pairs ? gt_column(8 * (wave + 8 * i) + (lane >> 3)) : 8 * (wave + 8 * i) + (lane >> 3))) - w0) * (uint32_t)g.ldw * 2 + piece;
+    const uint32_t base = (uint32_t)(uintptr_t)lds + wave * 1024;
+    Tile t;
+    t.run(lds, steps, [&](int st, int i, int at) { gt_to_lds(base + at + i * 8192, (int)xo[i], xs, st * 128); },
+          [&](int st, int i, int at) { gt_to_lds(base + at + i * 8192, (int)wo[i], ws, st * 128); });
+    const int m1 = min(g.M, r.m0 + r.tiles_m * Tile::BM), n1 = min(g.N, r.n1);
+    if (glu) {  // even W fragments are gates, the odd ones behind them the ups of the same values
+        DenseGemm o = g;
+        o.epilogue = GEMM_ELEM;
+        o.N = g.N / 2;
+        t.each([&](int a, int b, int row, int c) {
+            const int m = m0 + row, n = n0 + c - 4 * (lane >> 4), v = n / 2 + 4 * (lane >> 4);
+            if (m >= m1 || n >= r.n1 || v >= o.N) return;
+            const gt_f4 x = t.acc[a][b], u = t.acc[a][b + 1];
+            store4<false>(o, 0, m, v, silu_f(x[0]) * u[0], silu_f(x[1]) * u[1], silu_f(x[2]) * u[2], silu_f(x[3]) * u[3]);
+        });
+        return;
+    }
+    t.each([&](int a, int b, int row, int c) {
+        const int m = m0 + row, n = n0 + (pairs ? gt_column(c) : c), next = pairs ? 4 : 16;
+        if (m >= m1) return;
+        const gt_f4 x = t.acc[a][b], y = t.acc[a][b + 1];
+        if (pairs && n + 7 < g.N && (g.ldc & 7) == 0) {
+            if (n >= n1) return;
+            auto two = [&](float lo, float hi) {
+                if (g.epilogue == GEMM_RELU2) lo = relu2(lo), hi = relu2(hi);
+                return (uint32_t)f_bf16(lo) | ((uint32_t)f_bf16(hi) << 16);
+            };
+            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.C) + (int64_t)m * g.ldc + n) = make_uint4(two(x[0], x[1]), two(x[2], x[3]), two(y[0], y[1]), two(y[2], y[3]));
+            return;
+        }
+        if (n < n1) store4<false>(g, split, m, n, x[0], x[1], x[2], x[3]);
+        if (n + next < n1) store4<false>(g, split, m, n + next, y[0], y[1], y[2], y[3]);
+    });
+}
+
+__global__ __launch_bounds__(512, 2) void dense_gemm_tiles_kernel(const DenseGemm g, const GemmRegions rs) {
+    extern __shared__ __align__(1024) uint8_t gt_lds[];
+    int i = 0;
+    while (i + 1 < rs.n && (int)blockIdx.x >= rs.r[i + 1].first) ++i;
+    const GemmRegion r = rs.r[i];
+    const int wg = blockIdx.x - r.first;
+    switch (r.kind) {
+        case 0: return dense_tile<Tile0>(g, r, wg, gt_lds);
+        case 1: return dense_tile<Tile1>(g, r, wg, gt_lds);
+        case 2: return dense_tile<Tile2>(g, r, wg, gt_lds);
+        case 3: return dense_tile<Tile3>(g, r, wg, gt_lds);
+        case 4: return dense_tile<Tile4>(g, r, wg, gt_lds);
+        case 5: return dense_tile<Tile5>(g, r, wg, gt_lds);
+        default: return dense_tile<Tile6>(g, r, wg, gt_lds);
+    }
+}
+
 __global__ __launch_bounds__(256) void dense_gemm_f32_kernel(const DenseGemm g) {
     constexpr int BK = 32, P = BK + 1;
     __shared__ float s_a[64 * P], s_b[64 * P];
@@ -229,6 +326,22 @@ __global__ __launch_bounds__(256) void dense_gemm_f32_kernel(const DenseGemm g) 
     }
 }
 
+// The times are those of 512 ... 2048 rows times 2560 ... 28672 columns, 40 and 152 steps, the chip nearly full (two thirds empty, a step
+// takes a fifth less: the CUs share the power).  Against 128 x 128 tiles of four waves, rows through registers, two workgroups a CU:
+// 2048 x 19456 x 2560 240 -> 175 us (gate, up; 1165 TFLOP/s), 2048 x 2560 x 9728 116 -> 85, 1030 x 9728 x 2560 84 -> 57 (895 TFLOP/s).
+static void launch_tiles(DenseGemm& g, int kp, bool may_split, hipStream_t s) {
+    static const TileKind kinds[] = {tile_kind<Tile0>(1300, 14000), tile_kind<Tile1>(1080, 11000), tile_kind<Tile2>(850, 8500), tile_kind<Tile3>(740, 6000),
+                                     tile_kind<Tile4>(500, 6000),   tile_kind<Tile5>(500, 6000),  tile_kind<Tile6>(340, 5000)};
+    static std::once_flag raised;
+    std::call_once(raised, [] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_gemm_tiles_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    });
+    const int most = may_split && g.slab > 0 ? (int)std::min<int64_t>(16, g.slab_room / g.slab) : 1;
+    const TilePlan p = plan_tiles(kinds, 7, g.M, g.tile_cols, kp / 64, most, g.section_n);
+    g.splits = p.splits;
+    hipLaunchKernelGGL(dense_gemm_tiles_kernel, dim3((unsigned)p.wgs), dim3(512), p.lds, s, g, p.regions);
+}
+
 int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (!g.A || !g.W || !g.C) return PTM_E_NULL;
     const int kp = up64(g.K);
@@ -262,12 +375,7 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
         split(tiles(64, 64), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<64, 64, 32, 32>), dim3((unsigned)(tiles(64, 64) * g.splits)), dim3(256), 0, s, g);
     } else {
-        const int64_t t = tiles(128, 128);
-        if (t < 192) split(t, 384);
-        if (t * g.splits >= 128)
-            hipLaunchKernelGGL((dense_gemm_kernel<128, 128, 64, 64>), dim3((unsigned)(t * g.splits)), dim3(256), 0, s, g);
-        else
-            hipLaunchKernelGGL((dense_gemm_kernel<64, 64, 32, 32>), dim3((unsigned)(tiles(64, 64) * g.splits)), dim3(256), 0, s, g);
+        launch_tiles(g, kp, splits != nullptr, s);
     }
     if (splits) *splits = g.splits;
     return launch_status();
