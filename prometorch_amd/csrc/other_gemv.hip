@@ -1,37 +1,48 @@
 // The GEMV dispatcher's other block formats: Q8_0 (34 B per 32 values), Q5_K (176 B per 256) and Q5_0 (22 B per 32),
 // fp32 activations, as the reference's q8_0_gemv_avx2 / q5k_gemv_avx2 / q5_0_gemv_scalar compute them
 // (torch/io/cpu_quant_gemv.h:784-826, :1091-1185, :1572-1630), and the dequantisers of the first two
-// (torch/io/gguf_dequant.h:237-255, :348-388).  A Qwen3 / Llama Q4_K_M file holds none of these, so the kernels are
-// plain: one wave per row, a lane per run of 32 values (a Q8_0 / Q5_0 block, or one of the eight sub-blocks of a
-// Q5_K block), the lane's runs striding the row by 64, x read through the cache, one wave reduction per row.
+// (torch/io/gguf_dequant.h:237-255, :348-388).
+//
+// slots_gemv_kernel: a lane takes 8 values of a row (16 of a Q5_K block: both nibbles of its bytes) at a time, so that neighbouring lanes read
+// neighbouring pieces of x and of the row, and a wave several rows, so that x is loaded once for all of them; two passes over the row are
+// requested together.  Bound by requests in flight: Q8_0 9728 x 2560 9.0 us = 2.9 TB/s, 30000 x 2560 23 us = 3.5 TB/s, 300 x 1024 1.9 us (19.4,
+// 51.5 and 2.4 with a lane per run of 32 values, as the exact Q4_K kernel below still has it: x and the row are then read in pieces 128
+// and 34 bytes apart, and every load instruction touches 64 cache lines).
 #include "ptm_common.h"
+
+#include <type_traits>
 
 namespace ptm {
 
 struct __attribute__((packed, aligned(2))) u32_a2 { uint32_t v; };
 
-// Σ q_i x_i over 32 values whose quants are 32 consecutive signed bytes at a 2-byte aligned address
-__device__ __forceinline__ float dot32_i8(const uint8_t* __restrict__ q, const float* __restrict__ x) {
-    float s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-        const uint32_t v = reinterpret_cast<const u32_a2*>(q + 4 * w)->v;
-        const float4 xv = *reinterpret_cast<const float4*>(x + 4 * w);
-        s = fmaf((float)(int8_t)(v & 0xffu), xv.x, s);
-        s = fmaf((float)(int8_t)((v >> 8) & 0xffu), xv.y, s);
-        s = fmaf((float)(int8_t)((v >> 16) & 0xffu), xv.z, s);
-        s = fmaf((float)(int8_t)(v >> 24), xv.w, s);
-    }
-    return s;
+struct __attribute__((packed, aligned(2))) u64_a2 { uint32_t lo, hi; };
+
+__device__ __forceinline__ void load8(const float* __restrict__ x, float (&v)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(x), b = *reinterpret_cast<const float4*>(x + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
+// A format: VALUES of a row per slot, ROWS per wave and from how many slots LONG rows are shared by waves (slots_launch), what a lane loads of the row for slot u, which values of x (two groups of 8 or 4), the slot's term.
 struct FmtQ8_0 {
-    static constexpr int UNIT_BYTES = 34, UNITS_PER_BLOCK = 1, BLOCK_BYTES = 34;
-    // contribution of run u (32 values) of a row
-    static __device__ __forceinline__ float term(const uint8_t* __restrict__ row, int u, const float* __restrict__ x) {
-        const uint8_t* p = row + (int64_t)u * 34;
-        const float d = h2f(reinterpret_cast<const u16_a2*>(p)->v);
-        return d * dot32_i8(p + 2, x + 32 * u);
+    static constexpr int BLOCK_BYTES = 34, VALUES = 8, ROWS = 4, LONG = 256;
+    struct Raw { u64_a2 q; uint32_t d; };
+    struct X { float v[8]; };
+    static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
+        const uint8_t* p = row + (int64_t)(u >> 2) * 34;
+        r.q = *reinterpret_cast<const u64_a2*>(p + 2 + 8 * (u & 3));
+        r.d = reinterpret_cast<const u16_a2*>(p)->v;
+    }
+    static __device__ __forceinline__ void load_x(const float* __restrict__ x, int u, X& o) { load8(x + 8 * u, o.v); }
+    static __device__ __forceinline__ float term(const Raw& r, const X& x, int) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            s = fmaf((float)(int8_t)((r.q.lo >> (8 * i)) & 0xffu), x.v[i], s);
+            s = fmaf((float)(int8_t)((r.q.hi >> (8 * i)) & 0xffu), x.v[4 + i], s);
+        }
+        return h2f(r.d) * s;
     }
     static __device__ __forceinline__ float value(const uint8_t* __restrict__ blocks, int64_t e) {
         const uint8_t* p = blocks + (e >> 5) * 34;
@@ -40,59 +51,80 @@ struct FmtQ8_0 {
 };
 
 struct FmtQ5_0 {
-    static constexpr int BLOCK_BYTES = 22;
-    static __device__ __forceinline__ float term(const uint8_t* __restrict__ row, int u, const float* __restrict__ x) {
-        const uint8_t* p = row + (int64_t)u * 22;
-        const float d = h2f(reinterpret_cast<const u16_a2*>(p)->v);
-        const uint32_t qh = reinterpret_cast<const u32_a2*>(p + 2)->v;
-        const float* xb = x + 32 * u;
+    static constexpr int BLOCK_BYTES = 22, VALUES = 8, ROWS = 2, LONG = 256;  // four low nibbles and the four high ones of the same bytes, 16 values on
+    struct Raw { uint32_t q, h, d; };
+    struct X { float v[8]; };
+    static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
+        const uint8_t* p = row + (int64_t)(u >> 2) * 22;
+        r.q = reinterpret_cast<const u32_a2*>(p + 6 + 4 * (u & 3))->v;
+        r.h = reinterpret_cast<const u32_a2*>(p + 2)->v;
+        r.d = reinterpret_cast<const u16_a2*>(p)->v;
+    }
+    static __device__ __forceinline__ void load_x(const float* __restrict__ x, int u, X& o) {
+        const float* p = x + 32 * (u >> 2) + 4 * (u & 3);
+        const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 16);
+        o.v[0] = a.x; o.v[1] = a.y; o.v[2] = a.z; o.v[3] = a.w;
+        o.v[4] = b.x; o.v[5] = b.y; o.v[6] = b.z; o.v[7] = b.w;
+    }
+    static __device__ __forceinline__ float term(const Raw& r, const X& x, int u) {
+        const uint32_t h = r.h >> (4 * (u & 3));
         float s = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t v = reinterpret_cast<const u32_a2*>(p + 6 + 4 * w)->v;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int j = 4 * w + i;
-                const uint32_t b = (v >> (8 * i)) & 0xffu;
-                const int q0 = (int)((b & 0xfu) | (((qh >> j) & 1u) << 4)) - 16;
-                const int q1 = (int)((b >> 4) | (((qh >> (j + 16)) & 1u) << 4)) - 16;
-                s = fmaf((float)q0, xb[j], s);
-                s = fmaf((float)q1, xb[j + 16], s);
-            }
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t b = (r.q >> (8 * i)) & 0xffu;
+            s = fmaf((float)((int)((b & 0xfu) | (((h >> i) & 1u) << 4)) - 16), x.v[i], s);
+            s = fmaf((float)((int)((b >> 4) | (((h >> (16 + i)) & 1u) << 4)) - 16), x.v[4 + i], s);
         }
-        return d * s;
+        return h2f(r.d) * s;
     }
 };
 
 struct FmtQ5_K {
-    static constexpr int BLOCK_BYTES = 176;
+    static constexpr int BLOCK_BYTES = 176, VALUES = 16, ROWS = 4, LONG = 512;  // eight low nibbles and the eight high ones of the same bytes, 32 values on
+    struct Raw { uint4 hdr; uint2 q, h; };
+    struct X { float lo[8], hi[8]; };
     // scale and min of sub-block sb from the 12 packed bytes at p + 4 (get_scale_min_k4, gguf_dequant.h:289-297)
     static __device__ __forceinline__ void scale_min(const uint8_t* __restrict__ p, int sb, int& sc, int& mn) {
         const uint32_t* s = reinterpret_cast<const uint32_t*>(p + 4);
         q4k_scale_min(s[0], s[1], s[2], sb, sc, mn);
     }
-    static __device__ __forceinline__ float term(const uint8_t* __restrict__ row, int u, const float* __restrict__ x) {
-        const int sb = u & 7, pair = sb >> 1, hi = sb & 1;
-        const uint8_t* p = row + (int64_t)(u >> 3) * 176;
-        const uint32_t dd = *reinterpret_cast<const uint32_t*>(p);
-        int sc, mn;
-        scale_min(p, sb, sc, mn);
-        const float ds = h2f(dd) * (float)sc, ms = h2f(dd >> 16) * (float)mn;
-        const float* xb = x + 32 * u;
-        float sq = 0.0f, sx = 0.0f;
+    // slot u: bytes 8 (u % 4) .. of the pair of sub-blocks u / 4 % 4 of block u / 16.  Rows are aligned to 4 bytes.
+    struct __attribute__((packed, aligned(4))) u128_a4 { uint32_t v[4]; };
+    static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
+        const uint8_t* p = row + (int64_t)(u >> 4) * 176;
+        const int at = 8 * (u & 3), pair = (u >> 2) & 3;
+        const u128_a4 h = *reinterpret_cast<const u128_a4*>(p);
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 48 + 32 * pair + at);
+        const uint32_t* b = reinterpret_cast<const uint32_t*>(p + 16 + at);
+        r.hdr = make_uint4(h.v[0], h.v[1], h.v[2], h.v[3]);
+        r.q = make_uint2(q[0], q[1]);
+        r.h = make_uint2(b[0], b[1]);
+    }
+    static __device__ __forceinline__ void load_x(const float* __restrict__ x, int u, X& o) {
+        const float* p = x + 256 * (u >> 4) + 64 * ((u >> 2) & 3) + 8 * (u & 3);
+        load8(p, o.lo);
+        load8(p + 32, o.hi);
+    }
+    static __device__ __forceinline__ float term(const Raw& r, const X& x, int u) {
+        const int pair = (u >> 2) & 3;
+        float out = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            const uint32_t nib = (*reinterpret_cast<const uint32_t*>(p + 48 + 32 * pair + 4 * w) >> (4 * hi)) & 0x0f0f0f0fu;
-            const uint32_t bit = (*reinterpret_cast<const uint32_t*>(p + 16 + 4 * w) >> (2 * pair + hi)) & 0x01010101u;
-            const uint32_t q = nib | (bit << 4);
-            const float4 xv = *reinterpret_cast<const float4*>(xb + 4 * w);
-            sq = fmaf((float)(q & 0xffu), xv.x, sq);
-            sq = fmaf((float)((q >> 8) & 0xffu), xv.y, sq);
-            sq = fmaf((float)((q >> 16) & 0xffu), xv.z, sq);
-            sq = fmaf((float)(q >> 24), xv.w, sq);
-            sx += (xv.x + xv.y) + (xv.z + xv.w);
+        for (int e = 0; e < 2; ++e) {
+            int sc, mn;
+            q4k_scale_min(r.hdr.y, r.hdr.z, r.hdr.w, 2 * pair + e, sc, mn);
+            const uint32_t q0 = ((r.q.x >> (4 * e)) & 0x0f0f0f0fu) | (((r.h.x >> (2 * pair + e)) & 0x01010101u) << 4);
+            const uint32_t q1 = ((r.q.y >> (4 * e)) & 0x0f0f0f0fu) | (((r.h.y >> (2 * pair + e)) & 0x01010101u) << 4);
+            const float* v = e ? x.hi : x.lo;
+            float sq = 0.0f, sx = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sq = fmaf((float)((q0 >> (8 * i)) & 0xffu), v[i], sq);
+                sq = fmaf((float)((q1 >> (8 * i)) & 0xffu), v[4 + i], sq);
+                sx += v[i] + v[4 + i];
+            }
+            out += fmaf(h2f(r.hdr.x) * (float)sc, sq, -((h2f(r.hdr.x >> 16) * (float)mn) * sx));
         }
-        return fmaf(ds, sq, -(ms * sx));
+        return out;
     }
     static __device__ __forceinline__ float value(const uint8_t* __restrict__ blocks, int64_t e) {
         const uint8_t* p = blocks + (e >> 8) * 176;
@@ -154,6 +186,60 @@ __global__ __launch_bounds__(256) void rowwave_gemv_kernel(const uint8_t* __rest
     }
 }
 
+// y[r] (+)= the row's terms; R rows per wave, four waves per workgroup, C of them (1 or 4) at the same rows
+template <typename Fmt, int R, int C, bool ACC>
+__global__ __launch_bounds__(256) void slots_gemv_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, float* __restrict__ y,
+                                                         int K, int N, int64_t stride) {
+    __shared__ float part[4][R];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r0 = (blockIdx.x * (4 / C) + wave / C) * R;
+    if (r0 >= N) return;  // a whole wave, and of C = 4 the whole workgroup
+    const uint8_t* row[R];
+    float acc[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        row[i] = W + (int64_t)min(r0 + i, N - 1) * stride;
+        acc[i] = 0.0f;
+    }
+    const int slots = K / Fmt::VALUES;
+    constexpr int U = 2;  // passes requested together; a lane beyond the row repeats the last slot and does not count it
+    for (int first = (wave % C) * 64 * U; first < slots; first += 64 * U * C) {
+        typename Fmt::X xv[U];
+        typename Fmt::Raw w[U][R];
+#pragma unroll
+        for (int p = 0; p < U; ++p) {
+            const int u = min(first + 64 * p + lane, slots - 1);
+            Fmt::load_x(x, u, xv[p]);
+#pragma unroll
+            for (int i = 0; i < R; ++i) Fmt::load(row[i], u, w[p][i]);
+        }
+#pragma unroll
+        for (int p = 0; p < U; ++p) {
+            const int at = first + 64 * p + lane, u = min(at, slots - 1);
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const float t = Fmt::term(w[p][i], xv[p], u);
+                acc[i] += at < slots ? t : 0.0f;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = sum64(acc[i]);
+    if constexpr (C > 1) {
+        if (lane == 0)
+#pragma unroll
+            for (int i = 0; i < R; ++i) part[wave][i] = acc[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < R; ++i) acc[i] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+        if (wave > 0) return;
+    }
+    if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (r0 + i < N) y[r0 + i] = ACC ? y[r0 + i] + acc[i] : acc[i];
+}
+
 template <typename Fmt>
 __global__ __launch_bounds__(256) void elementwise_dequant_kernel(const uint8_t* __restrict__ blocks, float* __restrict__ out,
                                                                   int64_t n) {
@@ -162,18 +248,42 @@ __global__ __launch_bounds__(256) void elementwise_dequant_kernel(const uint8_t*
 }
 
 template <typename Fmt>
-static int rowwave_launch(const void* W, const float* x, float* y, int K, int N, int64_t stride, int per_block,
-                          int w_align, bool accumulate, hipStream_t s) {
+static int gemv_check(const void* W, const float* x, const float* y, int K, int N, int64_t stride, int per_block, int w_align) {
     if (!W || !x || !y) return PTM_E_NULL;
     if (K <= 0 || N <= 0 || (K % per_block) != 0) return PTM_E_SHAPE;
     if (stride < (int64_t)(K / per_block) * Fmt::BLOCK_BYTES) return PTM_E_SHAPE;
     if ((stride % w_align) != 0 || (reinterpret_cast<uintptr_t>(W) % w_align) != 0 || !aligned16(x) ||
         (reinterpret_cast<uintptr_t>(y) & 3u))
         return PTM_E_ALIGN;
-    const dim3 grid((N + 3) / 4), block(256);
+    return PTM_OK;
+}
+
+template <typename Fmt>
+static int slots_launch(const void* W, const float* x, float* y, int K, int N, int64_t stride, int per_block, int w_align,
+                        bool accumulate, hipStream_t s) {
+    const int rc = gemv_check<Fmt>(W, x, y, K, N, stride, per_block, w_align);
+    if (rc != PTM_OK) return rc;
     const uint8_t* w = static_cast<const uint8_t*>(W);
-    if (accumulate) hipLaunchKernelGGL((rowwave_gemv_kernel<Fmt, true>), grid, block, 0, s, w, x, y, K, N, stride);
-    else hipLaunchKernelGGL((rowwave_gemv_kernel<Fmt, false>), grid, block, 0, s, w, x, y, K, N, stride);
+    auto go = [&](auto rows, auto waves) {
+        constexpr int R = decltype(rows)::value, C = decltype(waves)::value;
+        const dim3 grid((N + 4 / C * R - 1) / (4 / C * R)), block(256);
+        if (accumulate) hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, true>), grid, block, 0, s, w, x, y, K, N, stride);
+        else hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, false>), grid, block, 0, s, w, x, y, K, N, stride);
+    };
+    using std::integral_constant;
+    // Four waves at the same rows where a row has two requests or more for each of them, more rows to share x between the more rows there are.
+    // us for one / two rows a wave, then for one / two / four with four waves at them, Q8_0: 9728 x 2560 12.4 10.4 | 11.2 9.5 9.0, 2560 x 9728
+    // 12.6 15.4 | 11.9 10.9 10.5, 1024 x 2560 3.3 3.8 | 3.0 2.9 3.0, 700 x 14336 9.7 13.2 | 5.8 6.6 6.3, 9728 x 1024 5.3 5.0 | 7.2 6.2 5.0.
+    const int slots = K / Fmt::VALUES;
+    if (slots >= (N >= 2048 ? Fmt::LONG : 256)) {
+        if (N >= 2048) go(integral_constant<int, Fmt::ROWS>{}, integral_constant<int, 4>{});
+        else if (N >= 1024) go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+        else go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    } else if (N >= 2048) {
+        go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    } else {
+        go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    }
     return launch_status();
 }
 
@@ -197,22 +307,28 @@ extern "C" {
 
 int ptm_q8_0_gemv(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,
                   ptm_stream_t stream) {
-    return rowwave_launch<FmtQ8_0>(W, x, y, K, N, row_stride_bytes, 32, 2, accumulate != 0, as_stream(stream));
+    return slots_launch<FmtQ8_0>(W, x, y, K, N, row_stride_bytes, 32, 2, accumulate != 0, as_stream(stream));
 }
 
 int ptm_q5_0_gemv(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,
                   ptm_stream_t stream) {
-    return rowwave_launch<FmtQ5_0>(W, x, y, K, N, row_stride_bytes, 32, 2, accumulate != 0, as_stream(stream));
+    return slots_launch<FmtQ5_0>(W, x, y, K, N, row_stride_bytes, 32, 2, accumulate != 0, as_stream(stream));
 }
 
 int ptm_q5k_gemv(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,
                  ptm_stream_t stream) {
-    return rowwave_launch<FmtQ5_K>(W, x, y, K, N, row_stride_bytes, 256, 4, accumulate != 0, as_stream(stream));
+    return slots_launch<FmtQ5_K>(W, x, y, K, N, row_stride_bytes, 256, 4, accumulate != 0, as_stream(stream));
 }
 
 int ptm_q4k_gemv_f32act(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,
                         ptm_stream_t stream) {
-    return rowwave_launch<FmtQ4_K_F32>(W, x, y, K, N, row_stride_bytes, 256, 16, accumulate != 0, as_stream(stream));
+    const int rc = gemv_check<FmtQ4_K_F32>(W, x, y, K, N, row_stride_bytes, 256, 16);
+    if (rc != PTM_OK) return rc;
+    const dim3 grid((N + 3) / 4), block(256);
+    const uint8_t* w = static_cast<const uint8_t*>(W);
+    if (accumulate) hipLaunchKernelGGL((rowwave_gemv_kernel<FmtQ4_K_F32, true>), grid, block, 0, as_stream(stream), w, x, y, K, N, row_stride_bytes);
+    else hipLaunchKernelGGL((rowwave_gemv_kernel<FmtQ4_K_F32, false>), grid, block, 0, as_stream(stream), w, x, y, K, N, row_stride_bytes);
+    return launch_status();
 }
 
 int ptm_dequant_q8_0(const void* blocks, float* out, int64_t n, ptm_stream_t stream) {

@@ -52,6 +52,16 @@ def test_other_formats_gemv_shapes_vs_oracle(dev, po, qt, N, K):
     assert np.array_equal(gpu_gemv(qt, pad, x), gpu_gemv(qt, W, x))
 
 
+# either side of the row counts and row lengths at which other numbers of rows and waves share a workgroup; rows that end inside a request
+@pytest.mark.parametrize("qt,N,K", [(qt, N, K) for qt, per in ((8, 32), (6, 32), (13, 256)) for N, K in
+                                    ((1023, 2048), (1025, 2304), (2047, 2048), (2051, 2048 - per), (2051, 2048 + per), (2050, 8192), (3, 8192 + per))])
+def test_other_formats_gemv_rows_per_wave(dev, po, qt, N, K):
+    r = synth.rng_for(36, qt, N, K)
+    W = synth.make_weight(r, qt, N, K)
+    x = synth.make_x(r, K)
+    assert rel_err(gpu_gemv(qt, W, x), po.gemv(qt, W, x)) <= GEMV_TOL * 1e-2
+
+
 @pytest.mark.parametrize("qt,N,K", [(13, 24, 512), (13, 3, 2560), (8, 24, 512), (8, 5, 96)])
 def test_other_formats_dequant_bit_exact(dev, po, seeds, golden_formats, qt, N, K):
     r = synth.rng_for(seeds["blocks"], qt, N, K)
