@@ -474,19 +474,19 @@ __global__ __launch_bounds__(THREADS) void qgemm_prepare_fused_kernel(const floa
 // forms as qgemm_prepare_fused_kernel<1> produces them (same arithmetic, same reduction order: the row is staged in LDS
 // and walked with that kernel's two lane mappings).  One launch and one pass over the row instead of a reduction launch
 // and three sweeps of the conversion.
-template <int B>  // partial sums fetched per batch
-__global__ __launch_bounds__(256) void qgemm_reduce_norm_prepare_kernel(const float* __restrict__ P, int splits, float* __restrict__ X,
+template <int B, int THREADS>  // partial sums fetched per batch
+__global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(const float* __restrict__ P, int splits, float* __restrict__ X,
                                                                         int accumulate, const float* __restrict__ gamma, float eps,
                                                                         int add_one, _Float16* __restrict__ Xh_round,
                                                                         float* __restrict__ rs_round, _Float16* __restrict__ Xh_plain,
                                                                         float* __restrict__ rs_plain, int M, int K) {
     extern __shared__ __align__(16) float rn_row[];  // K floats
     __shared__ float red[4];
-    __shared__ float red2[4];
+    __shared__ float red2[THREADS / 64];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int n4 = K / 4;
     if (m >= M) {  // padding rows: zeros
-        for (int i = tid; i < n4; i += 256) {
+        for (int i = tid; i < n4; i += THREADS) {
             if (Xh_round) reinterpret_cast<uint2*>(Xh_round + (int64_t)m * K)[i] = make_uint2(0, 0);
             if (Xh_plain) reinterpret_cast<uint2*>(Xh_plain + (int64_t)m * K)[i] = make_uint2(0, 0);
         }
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void qgemm_reduce_norm_prepare_kernel(const fl
     }
     const int64_t total = (int64_t)M * K;
     float4* x4 = reinterpret_cast<float4*>(X + (int64_t)m * K);
-    for (int i = tid; i < n4; i += 256) {
+    for (int i = tid; i < n4; i += THREADS) {
         // B partial sums per batch, fetched unconditionally (the index clamped) so that they are in flight together; B = 4
         // where there are at most four slabs (half the clamped re-reads of the last one)
         const float4 o = accumulate ? x4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -514,9 +514,15 @@ __global__ __launch_bounds__(256) void qgemm_reduce_norm_prepare_kernel(const fl
         reinterpret_cast<float4*>(rn_row)[i] = a;
     }
     __syncthreads();
+    // the order of 256 threads whatever their number
     float ss = 0.0f;
-    for (int i = tid; i < K; i += 256) ss = fmaf(rn_row[i], rn_row[i], ss);
-    ss = block_sum256(ss, red);
+    if (tid < 256) {
+        for (int i = tid; i < K; i += 256) ss = fmaf(rn_row[i], rn_row[i], ss);
+        ss = sum64(ss);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+    }
+    __syncthreads();
+    ss = (red[0] + red[1]) + (red[2] + red[3]);
     const float rs = 1.0f / sqrtf(ss / (float)K + eps);
     const float one = add_one ? 1.0f : 0.0f;
     auto value4 = [&](int i) {
@@ -526,14 +532,16 @@ __global__ __launch_bounds__(256) void qgemm_reduce_norm_prepare_kernel(const fl
         return r;
     };
     float amax = 0.0f;
-    for (int i = tid; i < n4; i += 256) {
+    for (int i = tid; i < n4; i += THREADS) {
         const float4 v = value4(i);
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
     }
     amax = max64(amax);
     if ((tid & 63) == 0) red2[tid >> 6] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(red2[0], red2[1]), fmaxf(red2[2], red2[3]));
+    amax = red2[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / 64; ++w) amax = fmaxf(amax, red2[w]);
     int e = 0;
     if (amax > 16384.0f) { (void)frexpf(amax, &e); e -= 14; }
     const float down = ldexpf(1.0f, -e);
@@ -549,7 +557,7 @@ __global__ __launch_bounds__(256) void qgemm_reduce_norm_prepare_kernel(const fl
         o.h[3] = (_Float16)(v.w * down);
         reinterpret_cast<uint2*>(dst)[i] = o.u;
     };
-    for (int i = tid; i < n4; i += 256) {  // K % 256 == 0: whole waves, aligned groups of 8 lanes = one Q8 block
+    for (int i = tid; i < n4; i += THREADS) {  // K % 256 == 0: whole waves, aligned groups of 8 lanes = one Q8 block
         const float4 v = value4(i);
         if (Xh_plain) store4(Xh_plain + (int64_t)m * K, i, v);
         if (Xh_round) {
@@ -660,10 +668,10 @@ struct Q6Tile {  // Q6_K: the lane's 16 bytes of ql for each (half, pair), of qh
 // steps of the current block, followed by the next block's weights, and written to the other LDS buffer during the
 // later steps, so the block ends with the next tile complete behind the only workgroup barrier of the block.  (After the
 // last block the same code re-fetches the last tile into the idle buffer: no conditionals in the steady-state loop.)
-// WAVES = 8 (what is launched, for every tile height): waves w and w + 4 own one 32-column strip each of the same 64
-// columns and all MT row tiles, so a SIMD holds two waves and one's dequantisation and LDS reads run under the other's
-// MFMAs (the two pipes of a single wave barely overlap); no weight is dequantised twice, the X tile in LDS is read by twice
-// as many waves.  WAVES = 4 (a wave owns both strips) is the layout this grew from: slower at every height.
+// WAVES = 8: waves w and w + 4 own one 32-column strip each of the same 64 columns and all MT row tiles, so a SIMD holds two waves
+// and one's dequantisation and LDS reads run under the other's MFMAs (the two pipes of a single wave barely overlap); no weight is
+// dequantised twice.  WAVES = 4, up to 64 rows: 128 columns, one strip a wave.  There a workgroup's time is unpacking and requests (64
+// lanes are 64 rows of W), not MFMAs, and half as many columns on twice as many CUs halve it where 256 columns leave CUs idle.
 // (bx, by, bz) = (column tile, row tile, K split) of this workgroup; s_a = its dynamic LDS
 template <typename Tile, int MT, int WAVES>
 __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride, const _Float16* Xh,
@@ -673,15 +681,16 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     // W and Xh are deliberately not __restrict__: loads through a restrict pointer may be moved across the
     // compiler fences below, and the prefetch distance of this loop depends on those fences
     constexpr int TM = 32 * MT;                     // rows of X per workgroup (MT tiles of 32)
-    constexpr int NT = 2 / (WAVES / 4);             // 32-column tiles per wave
+    constexpr int NT = 1;                           // 32-column tiles per wave
+    constexpr int TN = 32 * WAVES;                  // columns per workgroup
     constexpr int RS = 2 * WAVES;                   // rows of the X tile that one fetch instruction of the workgroup covers
     constexpr int NPIECE = TM / RS;                 // 16-byte pieces of the X tile per thread
-    static_assert(WAVES == 4 || (WAVES == 8 && (MT == 4 || MT == 2 || MT == 1)), "wave layouts");
+    static_assert((WAVES == 4 && MT <= 2) || (WAVES == 8 && (MT == 4 || MT == 2 || MT == 1)), "wave layouts");
     static_assert(NPIECE == 2 || NPIECE == 4 || NPIECE == 8 || NPIECE == 16, "pieces per thread");
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;  // s_a: [2][TM * QF_PITCH]
     const int j = lane & 31, kh = lane >> 5;
     const int m0 = by * TM;
-    const int n_base = bx * QF_TN + wave * 64 + (WAVES == 8 ? 32 * (tid >> 8) : 0);
+    const int n_base = bx * TN + (WAVES == 8 ? wave * 64 + 32 * (tid >> 8) : wave * 32);
     // split K: workgroup z of the grid sums super-blocks [blk0, blk0 + nblk) into its own M x N partial
     const int blk0 = bz * blocks_per_split;
     const int nblk = min(K / 256 - blk0, blocks_per_split);
@@ -1053,6 +1062,11 @@ static int qgemm_f16_row_tiles(bool q4, int M, int N, int splits) {
     return (q4 && wgs < 128) ? 2 : 4;  // 512 x 2560 x 9728 (152 workgroups): 60 us with 128 rows, 70 with 64; 512 x 4096 x 4096 (64): 80 / 68
 }
 
+// Workgroups of 128 columns: always up to 32 rows, up to 64 where the chip then has a CU for each.  Prompts of 19 / 32 / 50 / 64 tokens,
+// Qwen3-4B shapes, 256 columns, this rule, 128 always: 3.53 / 3.67 / 3.97 / 4.12 ms, 3.32 / 3.45 / 3.89 / 4.00, 3.32 / 3.45 / 3.86 / 3.97;
+// Llama-3-8B shapes in 16 layers, 60 tokens: 2.28, 2.28, 2.31.  A row's sum does not depend on the choice.
+static bool qf_narrow(int M, int wide_workgroups) { return M <= 32 || (M <= 64 && wide_workgroups <= 128); }
+
 static int qgemm_check(const void* W, const void* X, const void* Y, int M, int K, int N, int64_t stride, int blk_bytes) {
     if (!W || !X || !Y) return PTM_E_NULL;
     if (M <= 0 || N <= 0 || K <= 0 || (K % 256) != 0) return PTM_E_SHAPE;
@@ -1107,21 +1121,28 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
     });
-    const dim3 grid((N + QF_TN - 1) / QF_TN, (M + tm - 1) / tm, splits);
+    const int wide = (N + QF_TN - 1) / QF_TN * splits;
+    const bool narrow = qf_narrow(M, wide);
+    const int tn = narrow ? 128 : QF_TN;
+    const dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm, splits);
     const uint8_t* Wb = static_cast<const uint8_t*>(W);
     // Every tile height runs with eight waves (two per SIMD, one 32-column strip each): against four waves owning two strips
     // each, 512 x 4096 x 14336 104 -> 92 us (128 rows), 512 x 4096 x 4096 59.8 -> 45.3 us and 96 x 4096 x 2560 57.0 -> 42.7 us
     // (64 rows), a 16-token prompt 4.09 -> 3.86 ms (32 rows); the 64-row Q6_K tile no longer spills.
-#define PTM_QF(TILE, MTV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, 8>), grid, dim3(512), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials)
+#define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials)
     if (q4) {
-        if (MT == 4) PTM_QF(Q4Tile, 4);
-        else if (MT == 2) PTM_QF(Q4Tile, 2);
-        else PTM_QF(Q4Tile, 1);
+        if (MT == 4) PTM_QF(Q4Tile, 4, 8);
+        else if (MT == 2 && narrow) PTM_QF(Q4Tile, 2, 4);
+        else if (MT == 2) PTM_QF(Q4Tile, 2, 8);
+        else PTM_QF(Q4Tile, 1, 4);
     } else {
-        if (MT == 4) PTM_QF(Q6Tile, 4);
-        else if (MT == 2) PTM_QF(Q6Tile, 2);
-        else PTM_QF(Q6Tile, 1);
+        if (MT == 4) PTM_QF(Q6Tile, 4, 8);
+        else if (MT == 2 && narrow) PTM_QF(Q6Tile, 2, 4);
+        else if (MT == 2) PTM_QF(Q6Tile, 2, 8);
+        else PTM_QF(Q6Tile, 1, 4);
     }
 #undef PTM_QF
     if (deferred_splits) *deferred_splits = partials ? splits : 0;
@@ -1146,12 +1167,14 @@ int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool acc
     _Float16* hp = static_cast<_Float16*>(ws_plain);
     float* rr = hr ? reinterpret_cast<float*>(hr + (int64_t)mp * K) : nullptr;
     float* rp = hp ? reinterpret_cast<float*>(hp + (int64_t)mp * K) : nullptr;
-    if (splits <= 4)
-        hipLaunchKernelGGL(qgemm_reduce_norm_prepare_kernel<4>, dim3(mp), dim3(256), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0,
-                           gamma, eps, add_one, hr, rr, hp, rp, M, K);
-    else
-        hipLaunchKernelGGL(qgemm_reduce_norm_prepare_kernel<8>, dim3(mp), dim3(256), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0,
-                           gamma, eps, add_one, hr, rr, hp, rp, M, K);
+#define PTM_RN(B, T) hipLaunchKernelGGL((qgemm_reduce_norm_prepare_kernel<B, T>), dim3(mp), dim3(T), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0, gamma, eps, add_one, hr, rr, hp, rp, M, K)
+    // up to 128 rows the launch lasts as long as one row's chain of requests: as many threads as the row has pieces (4 / 8 / 16 slabs of 2560
+    // values 9.4 -> 6.5 us)
+    if (M <= 128 && K > 2048) PTM_RN(16, 1024);
+    else if (M <= 128 && K > 1024) PTM_RN(16, 512);
+    else if (splits <= 4) PTM_RN(4, 256);
+    else PTM_RN(8, 256);
+#undef PTM_RN
     return launch_status();
 }
 
@@ -1178,6 +1201,10 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     int sp[3];
     qgemm_f16_multi_plan(n, N, types, K, M, sp);
     const int nblk = K / 256;
+    int wide = 0;
+    for (int i = 0; i < n; ++i) wide += (N[i] + QF_TN - 1) / QF_TN * sp[i];
+    const bool narrow = qf_narrow(M, wide);
+    const int tn = narrow ? 128 : QF_TN;
     QfMulti a{};
     QfRedMulti r{};
     a.n_mat = n;
@@ -1205,7 +1232,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
         m.N = N[i];
         m.bps = (nblk + sp[i] - 1) / sp[i];
         const int splits = (nblk + m.bps - 1) / m.bps;  // no empty split
-        m.ntiles = (N[i] + QF_TN - 1) / QF_TN;
+        m.ntiles = (N[i] + tn - 1) / tn;
         m.q6 = q6 ? 1 : 0;
         m.partials = splits > 1 ? part : nullptr;
         if (deferred_P) { deferred_P[i] = splits > 1 ? part : Y[i]; deferred_splits[i] = splits; }
@@ -1228,9 +1255,13 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
                                   2 * 128 * QF_PITCH + 4 * 128);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  2 * 64 * QF_PITCH + 4 * 64);
     });
-    if (M <= 32)  // short prompts: the 32-row tile (see qgemm_f16_row_tiles)
-        hipLaunchKernelGGL((qgemm_f16_multi_kernel<1, 8>), dim3(slots, 1), dim3(512), 2 * (size_t)32 * QF_PITCH + 4 * 32, s, a, M, K);
+    if (M <= 32)
+        hipLaunchKernelGGL((qgemm_f16_multi_kernel<1, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)32 * QF_PITCH + 4 * 32, s, a, M, K);
+    else if (narrow)
+        hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
     else if (M <= 64)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 8>), dim3(slots, 1), dim3(512), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
     else

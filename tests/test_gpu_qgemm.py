@@ -186,3 +186,17 @@ def test_qgemm_f16_llama3_8b_layer_shapes_m512(dev, po, qt, N, K):
     if qt == 12:
         Yx = gpu_qgemm(qt, W, xb, M, K, N)
         assert rel_err(Y, Yx) <= QGEMM_F16_EXPECT
+
+
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(1, 512, 127), (31, 2560, 129), (32, 512, 385), (33, 4096, 128), (63, 768, 255), (64, 2560, 641),
+                                   (33, 256, 128 * 256 + 1)])
+def test_short_prompt_tiles(dev, po, qt, M, K, N):
+    """Workgroups of 128 columns (up to 32 rows always, up to 64 where 256 columns leave CUs idle) and the last size's 256: rows are the
+    rows of a 65-row call, which no 128-column tile serves, bit for bit (K unsplit: a call without room for partial sums)."""
+    r = synth.rng_for(46, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    xb, _ = bf16_round(r.standard_normal((65, K), dtype=np.float32))
+    few = gpu_qgemm_f16(qt, W, xb[:M], M, K, N)
+    many = gpu_qgemm_f16(qt, W, xb, 65, K, N)
+    assert np.array_equal(bits(few), bits(many[:M]))
