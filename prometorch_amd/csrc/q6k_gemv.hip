@@ -327,7 +327,7 @@ static int q6k_launch_xch(const Q6KArgs& a, int grid, size_t lds, hipStream_t s)
 template <bool ACC, bool ARGMAX, bool NORM>
 static int q6k_launch_mfma(const Q6KArgs& a, hipStream_t s) {
     const int grid = q6k_mfma_workgroups(a.N);
-    const size_t lds = 4 * (size_t)a.K + 4 * 16 * Q6M_PITCH;   // x as two fp16 terms + a tile of 16 row-blocks per wave
+    const size_t lds = 4 * (size_t)a.K + 4 * 16 * Q6M_PITCH + Q6M_ZERO;   // x as two fp16 terms, a tile of 16 row-blocks per wave, zeros
     const int nblk = a.K / 256;
     const int nb = nblk >= 4 ? 4 : 2;   // blocks in flight per lane (even: a slot's block parity is fixed); they roll
 #define PTM_Q6M(XLV, NBV) hipLaunchKernelGGL((q6k_mfma_gemv_kernel<ACC, ARGMAX, NORM, XLV, NBV>), dim3(grid), dim3(Q6K_THREADS), lds, s, a)

@@ -15,13 +15,15 @@
 //   * it COMPUTES with lane l on row l % 16 and the quarter kq = l / 16 of the block: 64 weights from three 16-byte pieces
 //     (ql[64 h + 16 c ..], ql[64 h + 32 + 16 c ..], qh[32 h + 16 c ..], h = kq / 2, c = kq % 2), which are the groups
 //     y[128 h + 16 c + {0, 32, 64, 96} .. +15] with scales sc[8 h + c + {0, 2, 4, 6}] (gguf_dequant.h:392-430);
-//   * sc * (q - 32) is an integer of magnitude <= 1024, exact in fp16: the bytes of four assembled weights become the fp16
-//     values 1024 + q by a byte permute (0x6400 | q), and one packed fp16 FMA, (1024 + q) * sc - 1056 * sc, rounds once to
-//     the exact product - two instructions per pair of weights where the vector kernel needs four;
+//   * q - 32 is exact in fp16: the bytes of four assembled weights become the fp16 values 1024 + q by a byte permute (0x6400 | q)
+//     and one packed subtraction of 1056 - two instructions per pair of weights where the vector kernel needs four.  The scales
+//     (any int8: |sc (q - 32)| reaches 4096, which fp16 does not hold exactly) multiply the accumulators;
 //   * the activation vector is the OTHER operand: x * 2^k (k puts max |x| near 2^13) split into two fp16 terms,
-//     hi = fp16(x 2^k), lo = fp16((x 2^k - hi) 2^11) - 22 mantissa bits - as operand rows 0 and 1 (rows 2..15 are idle);
-//     after the eight products of a super-block, lanes 0..15 hold sum(hi) and sum(lo) of their own row in the accumulator's
-//     first two registers, and y += d * (sum_hi + 2^-11 sum_lo), scaled back by 2^-k at the end.
+//     hi = fp16(x 2^k), lo = fp16((x 2^k - hi) 2^11) - 22 mantissa bits.  A product's 32 values are 8 of each quarter, and each
+//     quarter has a scale of its own: operand rows 4 kq and 4 kq + 1 hold quarter kq's hi and lo and zeros for the other
+//     quarters, so the accumulator's first two registers in lane l are sum(hi) and sum(lo) over quarter l / 16 of row l % 16 - the
+//     quarter whose scales the lane has read - and y += d * sum over the groups of sc * (sum_hi + 2^-11 sum_lo), the four
+//     quarters added and scaled back by 2^-k at the end.
 // Products are exact and accumulate in fp32, so the result differs from the vector kernel's by summation order and by the
 // 2^-22 split of x (measured against the CPU oracle: ~1e-6 of rms(y), bar 1e-3).
 #pragma once
@@ -38,6 +40,7 @@ typedef float q6m_f4 __attribute__((ext_vector_type(4)));
 // is the dword that holds d (fetched as the last of 16 bytes that end inside the dword the block ends in: never past the
 // page); chunks 14, 15 repeat it.
 struct Q6MFetch { uint4 v[4]; };
+enum { Q6M_ZERO = 256 };   // bytes of zeros behind the tiles: as far as a block's reads of x reach
 enum { Q6M_PITCH = 240 };  // LDS bytes per staged row-block: 16 B more than 14 chunks -> the 16 rows start 4 banks apart
 
 // Per-lane addresses of the fetch.  Consecutive blocks of a row are 210 bytes apart, so their misalignment alternates:
@@ -91,34 +94,27 @@ __device__ __forceinline__ Q6MBlk q6m_pieces(const uint8_t* rowblk, int off_a, i
     return r;
 }
 
-// four assembled weights (bytes 0..63) of one scale group -> sc * (q - 32) as two pairs of fp16
-__device__ __forceinline__ void q6m_scale4(uint32_t q4, q6m_h2 sc2, q6m_h2 bias2, q6m_h2& lo, q6m_h2& hi) {
+// four assembled weights (bytes 0..63) -> q - 32 as two pairs of fp16
+__device__ __forceinline__ void q6m_center4(uint32_t q4, q6m_h2& lo, q6m_h2& hi) {
     const uint32_t b01 = __builtin_amdgcn_perm(0x64646464u, q4, 0x04010400u);  // halves 0x6400 | q = 1024 + q
     const uint32_t b23 = __builtin_amdgcn_perm(0x64646464u, q4, 0x04030402u);
-    lo = __builtin_elementwise_fma(__builtin_bit_cast(q6m_h2, b01), sc2, bias2);
-    hi = __builtin_elementwise_fma(__builtin_bit_cast(q6m_h2, b23), sc2, bias2);
+    const q6m_h2 bias = {(_Float16)1056.0f, (_Float16)1056.0f};
+    lo = __builtin_bit_cast(q6m_h2, b01) - bias;
+    hi = __builtin_bit_cast(q6m_h2, b23) - bias;
 }
 
-// The eight products of one super-block: returns this lane's accumulator (lanes 0..15: [0] = sum over the block of
-// w * x_hi, [1] = of w * x_lo, for row `lane` of the wave's tile).  xa: this lane's operand row in LDS at the block's first
-// value plus the lane's quarter offset.  The x fragments are requested four at a time ahead of the unpacking arithmetic that
+// The eight products of one super-block: returns sum over this lane's quarter of sc * (q - 32) * x, without d, of its own row.
+// xa: this lane's operand row in LDS at the block's first value plus the lane's quarter offset (lanes whose operand row belongs
+// to another quarter: a run of zeros, step 0).  The x fragments are requested four at a time ahead of the unpacking arithmetic that
 // covers their LDS round trip (read one by one in front of their products, each costs the wave a full LDS latency).
-__device__ __forceinline__ q6m_f4 q6m_block(const Q6MBlk& k, const uint8_t* __restrict__ xa) {
+__device__ __forceinline__ float q6m_block(const Q6MBlk& k, const uint8_t* __restrict__ xa) {
     q6m_h8 a8[8];
 #pragma unroll
     for (int s = 0; s < 4; ++s) a8[s] = *reinterpret_cast<const q6m_h8*>(xa + 64 * (s >> 1) + 16 * (s & 1));
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t qa[4] = {k.qa.x, k.qa.y, k.qa.z, k.qa.w}, qb[4] = {k.qb.x, k.qb.y, k.qb.z, k.qb.w},
                    qh[4] = {k.qh.x, k.qh.y, k.qh.z, k.qh.w};
-    q6m_h2 sc2[4], bias2[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const _Float16 s = (_Float16)(float)k.sc[g];             // |sc| <= 32: exact
-        const _Float16 b = (_Float16)(-1056.0f * (float)k.sc[g]);  // 33 * 32 * sc: at most 11 significant bits, exact
-        sc2[g] = q6m_h2{s, s};
-        bias2[g] = q6m_h2{b, b};
-    }
-    q6m_f4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+    float sum = 0.0f;
     // group g of the lane: 0 = low nibbles of piece a (y[l]), 1 = low nibbles of piece b (y[l + 32]), 2 = high nibbles of a
     // (y[l + 64]), 3 = high nibbles of b (y[l + 96]); its two bits are bits 2g, 2g + 1 of the qh bytes
 #pragma unroll
@@ -134,23 +130,25 @@ __device__ __forceinline__ q6m_f4 q6m_block(const Q6MBlk& k, const uint8_t* __re
             const uint32_t nib = g == 0 ? (qa[i] & 0x0f0f0f0fu) : g == 1 ? (qb[i] & 0x0f0f0f0fu)
                                : g == 2 ? ((qa[i] >> 4) & 0x0f0f0f0fu) : ((qb[i] >> 4) & 0x0f0f0f0fu);
             const uint32_t two = g == 0 ? (qh[i] << 4) : g == 1 ? (qh[i] << 2) : g == 2 ? qh[i] : (qh[i] >> 2);
-            q6m_scale4(nib | (two & 0x30303030u), sc2[g], bias2[g], w[2 * i], w[2 * i + 1]);
+            q6m_center4(nib | (two & 0x30303030u), w[2 * i], w[2 * i + 1]);
         }
+        q6m_f4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const q6m_h8 b8 = {w[4 * e][0], w[4 * e][1], w[4 * e + 1][0], w[4 * e + 1][1],
                                w[4 * e + 2][0], w[4 * e + 2][1], w[4 * e + 3][0], w[4 * e + 3][1]};
             c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a8[2 * g + e], b8, c, 0, 0, 0);
         }
+        sum = fmaf((float)k.sc[g], fmaf(c[1], 1.0f / 2048.0f, c[0]), sum);
     }
-    return c;
+    return sum;
 }
 
 // XL: float4 loads of x per thread (K <= 1024 XL); NB: super-blocks in flight per lane.
 template <bool ACC, bool ARGMAX, bool NORM, int XL, int NB>
 __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds_raw) {
     static_assert(NB % 2 == 0, "block parity is taken from the unrolled slot index");
-    // LDS: x_hi[K] fp16 | x_lo[K] fp16
+    // LDS: x_hi[K] fp16 | x_lo[K] fp16 | the waves' tiles | zeros
     uint8_t* s_hi = lds_raw;
     uint8_t* s_lo = lds_raw + 2 * (size_t)a.K;
     __shared__ float red[8];
@@ -179,6 +177,8 @@ __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds
     uint8_t* const stage = lds_raw + 4 * (size_t)a.K + (size_t)wave * 16 * Q6M_PITCH;   // this wave's tile of 16 row-blocks
     uint8_t* const stage_lane = stage + (lane >> 4) * Q6M_PITCH + 16 * min(chunk, 14);
     const uint8_t* const stage_row = stage + rl * Q6M_PITCH;
+    uint8_t* const s_zero = lds_raw + 4 * (size_t)a.K + 4 * 16 * Q6M_PITCH;
+    if (tid < Q6M_ZERO / 16) reinterpret_cast<uint4*>(s_zero)[tid] = make_uint4(0, 0, 0, 0);
 
     // ---- activation loads first (range-checked buffer loads, zeros past the end), then the first blocks ----
     const __amdgpu_buffer_rsrc_t x4 = make_rsrc(a.x, a.K * 4);
@@ -251,9 +251,10 @@ __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds
     }
     __syncthreads();
 
-    // this lane's operand row of x: rows 0 and 1 of the 16-row operand are x_hi and x_lo; rows 2..15 only feed accumulator
-    // rows that nobody reads, so their lanes fetch x_hi as well (no zero row, no per-lane address arithmetic)
-    const uint8_t* xa = (rl == 1 ? s_lo : s_hi) + 2 * (128 * h + 16 * c);
+    // this lane's operand row of x: x_hi or x_lo where the row is its quarter's (4 kq, 4 kq + 1), else 256 B of zeros
+    const bool own = (rl >> 2) == kq && (rl & 2) == 0;
+    const uint8_t* const xa = own ? ((rl & 1) ? s_lo : s_hi) + 2 * (128 * h + 16 * c) : s_zero;
+    const int xstep = own ? 512 : 0;
 
     // Blocks roll through NB register sets: block b is shifted into place and staged, its successor NB blocks on is
     // requested into the same registers, then the lanes read their pieces of block b back and compute.  LDS operations of
@@ -267,8 +268,8 @@ __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds
             if (u & 1) { q6m_stage<1>(ft[u], ad, chunk, stage_lane); ft[u] = q6m_fetch<1>(ad, clampb(b0 + NB + u)); }
             else { q6m_stage<0>(ft[u], ad, chunk, stage_lane); ft[u] = q6m_fetch<0>(ad, clampb(b0 + NB + u)); }
             const Q6MBlk k = q6m_pieces(stage_row, off_a, off_h, h, c);
-            const q6m_f4 cc = q6m_block(k, xa + 512 * (b0 + u));
-            acc = fmaf(h2f(k.d), fmaf(cc[1], 1.0f / 2048.0f, cc[0]), acc);
+            const float t = q6m_block(k, xa + xstep * (b0 + u));
+            acc = fmaf(h2f(k.d), t, acc);
         }
     }
 #pragma unroll
@@ -278,11 +279,13 @@ __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds
             if (u & 1) q6m_stage<1>(ft[u], ad, chunk, stage_lane);
             else q6m_stage<0>(ft[u], ad, chunk, stage_lane);
             const Q6MBlk k = q6m_pieces(stage_row, off_a, off_h, h, c);
-            const q6m_f4 cc = q6m_block(k, xa + 512 * b);
-            acc = fmaf(h2f(k.d), fmaf(cc[1], 1.0f / 2048.0f, cc[0]), acc);
+            const float t = q6m_block(k, xa + xstep * b);
+            acc = fmaf(h2f(k.d), t, acc);
         }
     }
-    const float p = acc * down;   // lanes 0..15: row rl of the tile
+    acc += __shfl_xor(acc, 16, 64);   // the four quarters
+    acc += __shfl_xor(acc, 32, 64);
+    const float p = acc * down;   // row rl of the tile
     if (kq == 0 && live && a.y) {
         if constexpr (ACC) a.y[rr] += p;
         else a.y[rr] = p;

@@ -722,3 +722,24 @@ def test_fused_argmax_of_nan_logits_publishes_a_row_inside_the_table(dev):
     ops.q6k_gemv_argmax(Wd, xd, logits, K, N, W.shape[1], idx, ws)
     torch.cuda.synchronize()
     assert bool(torch.isnan(logits).all()) and 0 <= int(idx.item()) < N
+
+
+@pytest.mark.parametrize("N,K", [(16384, 512), (16391, 768), (20000, 4352), (16400, 8192)])
+def test_q6k_tall_matrices_whole_scale_range(dev, N, K):
+    """Q6_K scales are any int8 (an encoder gives a block's largest group -128): scale x quant up to 4096, exact, on the matrix-core
+    path.  Bar: the 2^-22 split of x and fp32 sums of K products, as shares of the row's sum of |w x|."""
+    r = synth.rng_for(66, N, K)
+    W = synth.make_q6k(r, N, K)
+    blk = W.reshape(-1, 210)
+    blk[:, 192:208] = r.integers(-128, 128, size=(blk.shape[0], 16), dtype=np.int8).view(np.uint8)
+    blk[::3, 192:208:5] = 128   # -128
+    blk[1::3, 0:192] = 0        # quants of -32
+    x = r.standard_normal(K, dtype=np.float32)
+    Wd, xd, y = cu(W), cu(x), torch.full((N,), 7.0, device="cuda")
+    ops.launch_q6k_gemv(Wd, xd, y, K, N, W.shape[1])
+    torch.cuda.synchronize()
+    rows = np.concatenate([np.arange(0, 64), r.integers(0, N, size=400), np.arange(N - 64, N)])
+    w = synth.dequant_q6k_np(W[rows].reshape(-1)).reshape(len(rows), K).astype(np.float64)
+    ref, size = w @ x.astype(np.float64), np.abs(w) @ np.abs(x).astype(np.float64)
+    err = np.abs(y.cpu().numpy()[rows] - ref)
+    assert np.all(err <= (2.0 ** -21 + K * 2.0 ** -24) * size)
