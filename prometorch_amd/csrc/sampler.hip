@@ -11,7 +11,8 @@
 //   top_p, renormalised; the token is the first index whose running sum of p (index order) reaches the uniform
 //   draw r (index 0 when r <= 0, the last index when the sum never gets there).
 //   temperature < 1e-6: argmax (strict '>', lowest index) of the penalised logits.
-// Exact selection of the k-th largest x: a three-level radix select over the order-preserving integer image of x
+// Exact selection of the k-th largest x, top-k up to 64: per slice of the vocabulary, then among the slices' candidates (below).
+// Larger top-k: a three-level radix select over the order-preserving integer image of x
 // (11 + 11 + 10 bits: one histogram pass over the vocabulary per level), then a gather of everything at or above
 // the threshold (<= SAMPLER_MAX_CAND, normally exactly k) and ONE workgroup that finishes on that short list,
 // doing the reference's sequential fp32 sums in the reference's order (so results differ from the CPU's only
@@ -36,15 +37,17 @@ enum {
     // candidate arrays (the two paths never run in the same call)
     SW_WIDE = SW_CAND_IDX + SAMPLER_MAX_CAND,
     SW_MASS_HIST = SW_CAND_KEY,
-    SW_WORDS = SW_WIDE + 64,
+    SW_LOCAL = SW_WIDE + 64,      // the short path: [LOCAL_SLICES] of LOCAL_WORDS
     SW_CLEAR_WORDS = SW_COUNT + 8
 };
+// The short path: a slice of the vocabulary per workgroup, at most LOCAL_SLICES, and at most LOCAL_SLOTS candidates of each:
+// how many, the largest key that one left out may have (0: none left out), the largest key of each quarter, (key, index) pairs
+enum { LOCAL_MAX_TOPK = 64, LOCAL_SLICES = 128, LOCAL_SLOTS = 128, LOCAL_HEAD = 6, LOCAL_WORDS = LOCAL_HEAD + 2 * LOCAL_SLOTS, SW_WORDS = SW_LOCAL + LOCAL_SLICES * LOCAL_WORDS };
 // wide-path scalars (32-bit words from SW_WIDE): top-k threshold key, largest kept key, sum of exp (64-bit, 2^-32 units),
 // probability mass above the current prefix (64-bit, 2^-40 units), key prefix chosen so far, 1 when every eligible token stays
-// the narrow path's hand-over to its overflow kernel: 1 when more candidates tied at the threshold than the list holds, and the
-// threshold key itself (outside the words the wide threshold kernel zeroes)
+// the gathering path's threshold key (outside the words the wide threshold kernel zeroes)
 enum { WS_THR = 0, WS_MAXKEY = 1, WS_SUMEXP = 2, WS_MASS_ABOVE = 4, WS_PREFIX = 6, WS_KEEP_ALL = 7, WS_TSTAR = 8, WS_NTIE = 9,
-       WS_OVERFLOW = 16, WS_THR_SAVE = 17 };
+       WS_THR_SAVE = 16 };
 
 struct SamplerArgs {
     const float* logits;
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(256) void sampler_gather_kernel(SamplerArgs a) {
     select_bin(a.ws + SW_HIST1, 2048, k, b1, k, s_scan);
     select_bin(a.ws + SW_HIST2, 1024, k, b2, k, s_scan);
     const uint32_t threshold = ((uint32_t)b0 << 21) | ((uint32_t)b1 << 10) | (uint32_t)b2;
-    if (blockIdx.x == 0 && tid == 0) a.ws[SW_WIDE + WS_THR_SAVE] = threshold;   // for the overflow kernel
+    if (blockIdx.x == 0 && tid == 0) a.ws[SW_WIDE + WS_THR_SAVE] = threshold;   // should more tie there than the list holds
     const int base = blockIdx.x * SAMPLER_ELEMS_PER_WG;
 #pragma unroll
     for (int u = 0; u < SAMPLER_ELEMS_PER_WG / 256; ++u) {
@@ -208,7 +211,7 @@ struct SamplerOut {
 // what the last thread of a draw does with the chosen id: result, occurrence count, the decode loop's step bookkeeping
 __device__ __forceinline__ void sampler_publish(const SamplerOut& o, int token, int step, int64_t past_now) {
     if (o.out_token) *o.out_token = token;
-    if (o.counts_rw) o.counts_rw[token] += 1;
+    if (o.counts_rw) atomicAdd(&o.counts_rw[token], 1);  // no value needed back: nothing waits for it
     if (o.adv.d_step) {
         if (step < o.adv.cap) o.adv.tokens_out[step] = token;
         *o.adv.d_token = token;
@@ -217,111 +220,86 @@ __device__ __forceinline__ void sampler_publish(const SamplerOut& o, int token, 
     }
 }
 
-__global__ __launch_bounds__(1024) void sampler_finish_kernel(SamplerArgs a, SamplerOut o) {
-    __shared__ unsigned long long s_sort[SAMPLER_MAX_CAND];   // 16 KB
-    __shared__ float s_p[SAMPLER_MAX_CAND];                   // x, then p, in index order
-    __shared__ uint32_t s_idx[SAMPLER_MAX_CAND];
-    __shared__ uint8_t s_keep[SAMPLER_MAX_CAND];
-    const int tid = threadIdx.x;
-    // every load whose address is known goes out first, in one round trip; the draw follows as soon as the step is known
-    const ptm_sampling p = sampler_params(a);
-    const uint32_t total = a.ws[SW_COUNT];
-    const uint32_t key0 = a.ws[SW_CAND_KEY + (tid & 63)], idx0 = a.ws[SW_CAND_IDX + (tid & 63)];
-    const int step = o.d_step ? *o.d_step : 0;
-    const int64_t past_now = o.adv.d_past ? *o.adv.d_past : 0;
-    const float r_draw = o.uniforms[step];
-    if (total > SAMPLER_MAX_CAND) {
-        // more logits tie at the threshold than the candidate list holds: the kernel behind this one (sampler_overflow_kernel)
-        // draws from the whole vocabulary instead and publishes the token
-        if (tid == 0) a.ws[SW_WIDE + WS_OVERFLOW] = 1u;
-        if (o.leave_clean) for (int i = tid; i < SW_CLEAR_WORDS; i += 1024) a.ws[i] = 0;
-        return;
-    }
-    const int m = (int)total;
-    if (m <= 64) {
-        // The usual case (k candidates, k <= 64): one wave, one candidate per lane, no workgroup barrier.  Order by
-        // counting, sequential sums by reading lane after lane -- the same additions in the same order as below.
-        if (tid >= 64) {
-            if (o.leave_clean) for (int i = tid - 64; i < SW_CLEAR_WORDS; i += 1024 - 64) if (i != SW_COUNT) a.ws[i] = 0;
-            return;
-        }
-        const int lane = tid;
-        const bool valid = lane < m;
-        const uint32_t key = valid ? key0 : 0u, idx = valid ? idx0 : 0xffffffffu;
-        int rank = 0;
-        for (int j = 0; j < m; ++j) rank += lane_u(idx, j) < idx;
-        if (valid) { s_idx[rank] = idx; s_p[rank] = key_value(key); }
+// Running sums in lane order, one addition after the other, of the first n lanes' values: this lane's (total: the last one's).  A step
+// adds every lane's value to its lower neighbour's sum: after i steps the sums up to lane i are there, and stay.
+__device__ __forceinline__ float running_sums(float v, int n, float& total) {
+    float sum = v;
+    for (int i = 0; i < n; i += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum = dpp_f<0x138>(sum) + v;  // wave_shr:1, 0 into lane 0
+    total = n > 0 ? lane_f(sum, n - 1) : 0.0f;
+    return sum;
+}
+
+struct SamplerLds {
+    unsigned long long sort[SAMPLER_MAX_CAND];   // 16 KB
+    float p[SAMPLER_MAX_CAND];                   // x, then p, in index order
+    uint32_t idx[SAMPLER_MAX_CAND];
+    uint8_t keep[SAMPLER_MAX_CAND];
+};
+
+// Up to 64 candidates (the usual case), one per lane of one wave, in any order: no workgroup barrier.  Order by counting; the
+// sums are the reference's sequential ones, the running values kept in the lanes, so that each is walked once without a branch.
+__device__ __forceinline__ int sampler_draw64(const SamplerArgs& a, const ptm_sampling& p, SamplerLds& l, int m, uint32_t key, uint32_t idx, float r) {
+    const int lane = threadIdx.x & 63;
+    const bool valid = lane < m;
+    if (!valid) idx = 0xffffffffu;
+    int rank = 0;
+    for (int j = 0; j < m; j += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) rank += lane_u(idx, j + u) < idx;
+    if (valid) { l.idx[rank] = idx; l.p[rank] = key_value(key); }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t id = valid ? l.idx[lane] : 0u;   // index order from here on
+    if (!(p.temperature >= 1e-6f)) return (int)lane_u(id, 0);
+    const float x = valid ? l.p[lane] : -INFINITY;
+    const float mx = max64(x);
+    const float e = valid ? expf(x - mx) : 0.0f;
+    float sum;
+    running_sums(e, m, sum);
+    float pr = e * (1.0f / sum);
+    if (p.top_p < 1.0f) {
+        const bool elig = valid && pr > 1e-10f;
+        const uint32_t bits = elig ? __float_as_uint(pr) : 0u;   // positive floats order as their bits
+        const int n_elig = __popcll(__ballot(elig));
+        int r2 = 0;
+        for (int j = 0; j < m; j += 8)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) r2 += lane_u(bits, j + u) + (j + u < lane ? 1u : 0u) > bits;
+        float* s_q = reinterpret_cast<float*>(l.sort);
+        if (elig) s_q[r2] = pr;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const uint32_t id = valid ? s_idx[lane] : 0u;   // index order from here on
-        const float x = valid ? s_p[lane] : -INFINITY;
-        const bool greedy = !(p.temperature >= 1e-6f);
-        int token = a.vocab - 1;
-        if (greedy) {
-            token = (int)lane_u(id, 0);
-        } else {
-            const float mx = max64(x);
-            const float e = valid ? expf(x - mx) : 0.0f;
-            float sum = 0.0f;
-            for (int i = 0; i < m; ++i) sum += lane_f(e, i);
-            float pr = e * (1.0f / sum);
-            if (p.top_p < 1.0f) {
-                const bool elig = valid && pr > 1e-10f;
-                int r2 = 0, n_elig = 0;
-                for (int j = 0; j < m; ++j) {
-                    const float pj = lane_f(pr, j);
-                    const bool ej = pj > 1e-10f;
-                    n_elig += ej;
-                    r2 += ej && (pj > pr || (pj == pr && j < lane));
-                }
-                float* s_q = reinterpret_cast<float*>(s_sort);
-                if (elig) s_q[r2] = pr;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                const float q = lane < n_elig ? s_q[lane] : 0.0f;
-                float cum = 0.0f;
-                int n_keep = n_elig;
-                for (int k = 0; k < n_elig; ++k) {
-                    cum += lane_f(q, k);
-                    if (cum >= p.top_p) { n_keep = k + 1; break; }
-                }
-                pr = (elig && r2 < n_keep) ? pr : 0.0f;
-                float s2 = 0.0f;
-                for (int i = 0; i < m; ++i) s2 += lane_f(pr, i);
-                if (s2 > 0.0f) pr *= 1.0f / s2;
-            }
-            const float r = r_draw;
-            if (r <= 0.0f) {
-                token = 0;
-            } else {
-                float cum = 0.0f;
-                for (int i = 0; i < m; ++i) {
-                    cum += lane_f(pr, i);
-                    if (cum >= r) { token = (int)lane_u(id, i); break; }
-                }
-            }
-        }
-        if (lane == 0) {
-            if (o.out_token) *o.out_token = token;
-            if (o.counts_rw) atomicAdd(&o.counts_rw[token], 1);  // no value needed back: nothing waits for it
-            if (o.adv.d_step) {
-                if (step < o.adv.cap) o.adv.tokens_out[step] = token;
-                *o.adv.d_token = token;
-                *o.adv.d_past = past_now + 1;
-                *o.adv.d_step = step + 1;
-            }
-            if (o.leave_clean) a.ws[SW_COUNT] = 0;
-            a.ws[SW_WIDE + WS_OVERFLOW] = 0u;
-        }
-        return;
+        const float q = lane < n_elig ? s_q[lane] : 0.0f;
+        float total;
+        const float cum = running_sums(q, n_elig, total);
+        const unsigned long long full = __ballot(lane < n_elig && cum >= p.top_p);
+        const int n_keep = full ? (int)__builtin_ctzll(full) + 1 : n_elig;
+        pr = (elig && r2 < n_keep) ? pr : 0.0f;
+        running_sums(pr, m, total);
+        if (total > 0.0f) pr *= 1.0f / total;
     }
+    if (r <= 0.0f) return 0;
+    float total;
+    const float cum = running_sums(pr, m, total);
+    const unsigned long long hit = __ballot(valid && cum >= r);
+    return hit ? (int)lane_u(id, (int)__builtin_ctzll(hit)) : a.vocab - 1;
+}
+
+// Up to SAMPLER_MAX_CAND candidates in l.sort[0 .. m) as (index << 32 | key), by the whole workgroup; the result holds in thread 0.
+__device__ int sampler_draw_list(const SamplerArgs& a, const ptm_sampling& p, SamplerLds& l, int m, float r_draw) {
+    const int tid = threadIdx.x;
+    unsigned long long* s_sort = l.sort;
+    float* s_p = l.p;
+    uint32_t* s_idx = l.idx;
+    uint8_t* s_keep = l.keep;
     int n = 1;
     while (n < m) n <<= 1;
-    // ---- candidates in index order ----
-    for (int i = tid; i < n; i += 1024)
-        s_sort[i] = i < m ? (((unsigned long long)a.ws[SW_CAND_IDX + i] << 32) | a.ws[SW_CAND_KEY + i]) : ~0ull;
+    __syncthreads();
+    for (int i = m + tid; i < n; i += 1024) s_sort[i] = ~0ull;
     bitonic_sort_u64(s_sort, n);
     for (int i = tid; i < m; i += 1024) {
         s_idx[i] = (uint32_t)(s_sort[i] >> 32);
@@ -368,31 +346,22 @@ __global__ __launch_bounds__(1024) void sampler_finish_kernel(SamplerArgs a, Sam
             __syncthreads();
         }
     }
+    int token = a.vocab - 1;
     if (tid == 0) {
-        a.ws[SW_WIDE + WS_OVERFLOW] = 0u;
-        int token;
         if (greedy) {
             token = (int)s_idx[0];  // every candidate equals the maximum; index order -> the lowest index
+        } else if (r_draw <= 0.0f) {
+            token = 0;  // the running sum reaches r at the very first index
         } else {
-            const float r = r_draw;
-            token = a.vocab - 1;
-            if (r <= 0.0f) {
-                token = 0;  // the running sum reaches r at the very first index
-            } else {
-                float cum = 0.0f;
-                for (int i = 0; i < m; ++i) {
-                    cum += s_p[i];
-                    if (cum >= r) { token = (int)s_idx[i]; break; }
-                }
+            float cum = 0.0f;
+            for (int i = 0; i < m; ++i) {
+                cum += s_p[i];
+                if (cum >= r_draw) { token = (int)s_idx[i]; break; }
             }
         }
-        sampler_publish(o, token, step, past_now);
     }
-    if (o.leave_clean) {  // every thread read the candidate count long before (barriers above)
-        for (int i = tid; i < SW_CLEAR_WORDS; i += 1024) a.ws[i] = 0;
-    }
+    return token;
 }
-
 
 // ---------------------------------------------------------------------------------------------------------------------
 // Wide path: top-k off (top_k <= 0 or >= vocab) or a top-k beyond the candidate list.  The distribution then spans (almost)
@@ -690,22 +659,18 @@ __device__ __forceinline__ void sampler_wide_draw_body(const SamplerArgs& a, con
 
 __global__ __launch_bounds__(1024) void sampler_wide_draw_kernel(SamplerArgs a, SamplerOut o) { sampler_wide_draw_body(a, o); }
 
-// Behind the narrow path's finish kernel, always launched, one workgroup: returns at once unless that kernel found more
-// logits tied at the top-k threshold than its candidate list holds (a flat or constant stretch of logits at the cut: the
-// reference keeps every tie, gguf_model.h:7682-7691).  Then it does what the wide path does for a large top-k -- largest
+// More logits tie at the top-k threshold than a candidate list holds (a flat or constant stretch of logits at the cut: the
+// reference keeps every tie, gguf_model.h:7682-7691).  One workgroup does what the wide path does for a large top-k -- largest
 // kept value, fixed-point softmax denominator, the nucleus' last value by a three-level walk over per-key-bin mass -- with
-// loops of this one workgroup over the vocabulary (a rare case: no launch-level parallelism spent on it), and ends in the
-// wide path's draw.  Greedy (k = 1 with the maximum tied that often): the lowest index among the maxima, as argmax gives.
-__global__ __launch_bounds__(1024) void sampler_overflow_kernel(SamplerArgs a, SamplerOut o) {
+// loops over the vocabulary (a rare case: no launch-level parallelism spent on it), and ends in the wide path's draw.  Greedy
+// (k = 1 with the maximum tied that often): the lowest index among the maxima, as argmax gives.
+__device__ void sampler_overflow_body(const SamplerArgs& a, const SamplerOut& o, uint32_t thr, unsigned long long* s_hist) {
     uint32_t* w = a.ws + SW_WIDE;
-    if (w[WS_OVERFLOW] == 0u) return;
-    __shared__ unsigned long long s_hist[2048];
     __shared__ unsigned long long s_red64[16];
     __shared__ uint32_t s_red32[16];
     __shared__ uint32_t s_sel[2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const ptm_sampling p = sampler_params(a);
-    const uint32_t thr = w[WS_THR_SAVE];
     // largest kept key (and, for greedy, the lowest index that holds it)
     uint32_t best = 0;
     for (int i = tid; i < a.vocab; i += 1024) {
@@ -727,7 +692,6 @@ __global__ __launch_bounds__(1024) void sampler_overflow_kernel(SamplerArgs a, S
         __syncthreads();
         if (tid == 0) {
             for (int q = 1; q < 16; ++q) first = min(first, s_red32[q]);
-            w[WS_OVERFLOW] = 0u;
             sampler_publish(o, (int)first, o.d_step ? *o.d_step : 0, o.adv.d_past ? *o.adv.d_past : 0);
         }
         return;
@@ -796,11 +760,294 @@ __global__ __launch_bounds__(1024) void sampler_overflow_kernel(SamplerArgs a, S
         w[WS_KEEP_ALL] = keep_all;
         w[WS_TSTAR] = prefix;
         w[WS_NTIE] = ntie;
-        w[WS_OVERFLOW] = 0u;
     }
     __threadfence_block();
     __syncthreads();
     sampler_wide_draw_body(a, o);
+}
+
+// The gathering path's end: the draw from its candidates, or from the vocabulary where the list is too short.
+__global__ __launch_bounds__(1024) void sampler_finish_kernel(SamplerArgs a, SamplerOut o) {
+    __shared__ SamplerLds l;
+    const int tid = threadIdx.x;
+    // every load whose address is known goes out first, in one round trip; the draw follows as soon as the step is known
+    const ptm_sampling p = sampler_params(a);
+    const uint32_t total = a.ws[SW_COUNT], thr = a.ws[SW_WIDE + WS_THR_SAVE];
+    const uint32_t key0 = a.ws[SW_CAND_KEY + (tid & 63)], idx0 = a.ws[SW_CAND_IDX + (tid & 63)];
+    const int step = o.d_step ? *o.d_step : 0;
+    const int64_t past_now = o.adv.d_past ? *o.adv.d_past : 0;
+    const float r_draw = o.uniforms[step];
+    const int m = (int)min(total, (uint32_t)SAMPLER_MAX_CAND);
+    for (int i = tid; i < m; i += 1024) l.sort[i] = ((unsigned long long)a.ws[SW_CAND_IDX + i] << 32) | a.ws[SW_CAND_KEY + i];
+    __syncthreads();  // every thread has read the count
+    if (o.leave_clean)
+        for (int i = tid; i < SW_CLEAR_WORDS; i += 1024) a.ws[i] = 0;
+    if (total > SAMPLER_MAX_CAND) return sampler_overflow_body(a, o, thr, l.sort);
+    if (m <= 64) {
+        if (tid >= 64) return;
+        const int token = sampler_draw64(a, p, l, m, key0, idx0, r_draw);
+        if (tid == 0) sampler_publish(o, token, step, past_now);
+        return;
+    }
+    const int token = sampler_draw_list(a, p, l, m, r_draw);
+    if (tid == 0) sampler_publish(o, token, step, past_now);
+}
+
+// ---- the short path: top-k up to LOCAL_MAX_TOPK ------------------------------------------------------------------------
+// Two launches and one read of the logits instead of seven launches and four reads: a call is a chain of launches and latencies (151 936
+// logits, top-k 40: 34.2 us with histograms, 12.9 so; both read 1.2 MB, under a microsecond).  Beyond 64 candidates per slice the second
+// launch, a single workgroup, would read more than it saves.  What is at or above the k-th largest of the vocabulary is at
+// or above the k-th largest of its slice, so a workgroup leaves only those of its slice, and one workgroup selects among them.
+//
+// The largest T, as far as bits 31 .. low go, with at least k of the wave's R values per lane at or above it (0: fewer than k above 0).
+template <int R>
+__device__ __forceinline__ uint32_t kth_of_wave(const uint32_t (&v)[R], int k, int low) {
+    uint32_t t = 0;
+#pragma unroll 1
+    for (int bit = 31; bit >= low; --bit) {
+        const uint32_t with = t | 1u << bit;
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < R; ++i) n += __popcll(__ballot(v[i] >= with));
+        if (n >= k) t = with;
+    }
+    return t;
+}
+// The largest T, as far as its upper 16 bits go, with at least k of the workgroup's E keys per thread at or above it (0 if there are
+// fewer than k; keys left out are zeros): two bits at a time, from the top.  s_cnt: zeros.
+template <int E>
+__device__ __forceinline__ uint32_t kth_key_bits(const uint32_t (&key)[E], int k, uint32_t (&s_cnt)[8][4]) {
+    const int lane = threadIdx.x & 63;
+    uint32_t t = 0;
+#pragma unroll 1
+    for (int bit = 30, i = 0; bit >= 16; bit -= 2, ++i) {
+        uint32_t n[3] = {0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int e = 0; e < E; ++e) n[j] += (uint32_t)__popcll(__ballot(key[e] >= t + ((uint32_t)(j + 1) << bit)));
+        if (lane < 3) atomicAdd(&s_cnt[i][lane], lane == 0 ? n[0] : lane == 1 ? n[1] : n[2]);
+        __syncthreads();
+        const uint32_t c0 = s_cnt[i][0], c1 = s_cnt[i][1], c2 = s_cnt[i][2];
+        t += (uint32_t)((c0 >= (uint32_t)k) + (c1 >= (uint32_t)k) + (c2 >= (uint32_t)k)) << bit;
+    }
+    return t;
+}
+
+// grid: slices of 1024 E values.  Listed is what reaches the k-th largest of the maxima of four lanes, in its upper 16 bits: k values
+// and a tenth or so, found by one wave.  (Exactly, by all of them, takes eight barriers: 2.7 us against 1.)  Should they not fit, the
+// threshold is made exact, and should ties in its 16 bits still not fit, the list holds what is above them, and says so.
+template <int E>
+__global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
+    __shared__ uint32_t s_cnt[8][4];
+    __shared__ uint32_t s_max[256], s_bound, s_n[3];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, base = blockIdx.x * 1024 * E;
+    if (tid < 32) s_cnt[tid >> 2][tid & 3] = 0;
+    if (tid < 3) s_n[tid] = 0;
+    const ptm_sampling p = sampler_params(a);
+    uint32_t key[E], best = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = base + tid + 1024 * e;
+        key[e] = i < a.vocab ? order_key(sampler_value(a, p, i)) : 0u;
+        best = max(best, key[e]);
+    }
+    best = max(best, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)best, 0xB1, 0xf, 0xf, true));
+    best = max(best, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)best, 0x4E, 0xf, 0xf, true));
+    if ((tid & 3) == 0) s_max[tid >> 2] = best;
+    __syncthreads();
+    uint32_t* seg = a.ws + SW_LOCAL + blockIdx.x * LOCAL_WORDS;
+    if (wave == 0) {
+        const uint32_t v[4] = {s_max[lane], s_max[lane + 64], s_max[lane + 128], s_max[lane + 192]};
+        const uint32_t t = kth_of_wave(v, sampler_k(p), 16);
+        if (lane == 0) s_bound = t;
+    } else if (wave <= 4) {  // the quarters' maxima
+        uint32_t m = s_max[64 * (wave - 1) + lane];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor(m, off, 64));
+        if (lane == 0) seg[1 + wave] = m;
+    }
+    __syncthreads();
+    auto list = [&](uint32_t* count, uint32_t from) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = base + tid + 1024 * e;
+            if (i < a.vocab && key[e] >= from) {
+                const uint32_t slot = atomicAdd(count, 1u);
+                if (slot < LOCAL_SLOTS) reinterpret_cast<uint2*>(seg + LOCAL_HEAD)[slot] = make_uint2(key[e], (uint32_t)i);
+            }
+        }
+        __syncthreads();
+        return *count;
+    };
+    uint32_t n = list(&s_n[0], s_bound), left_out = 0;
+    if (n > LOCAL_SLOTS) {
+        const uint32_t thr = kth_key_bits(key, sampler_k(p), s_cnt);
+        n = list(&s_n[1], thr);
+        if (n > LOCAL_SLOTS) {  // (fewer than k <= 64 are above the whole of thr's 16 bits)
+            left_out = thr | 0xffffu;
+            n = left_out != 0xffffffffu ? list(&s_n[2], left_out + 1) : 0;
+        }
+    }
+    if (tid == 0) { seg[0] = n; seg[1] = left_out; }
+}
+
+// One workgroup: the candidates of all slices in registers.  A lower bound of the k-th largest is the k-th largest of the quarters'
+// maxima (one wave finds it), which leaves about k of some thousands; of those, the ones with fewer
+// than k greater ones.
+__global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs a, SamplerOut o, int slices) {
+    __shared__ SamplerLds l;
+    __shared__ uint32_t s_n[3];   // candidates at or above the bound, largest key left out, kept
+    __shared__ uint32_t s_bound;
+    constexpr int SEGS = LOCAL_SLICES / 16, MAXIMA = LOCAL_SLICES * 4 / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t* const seg0 = a.ws + SW_LOCAL;
+    uint2 head[SEGS], cand[2][SEGS];
+#pragma unroll
+    for (int g = 0; g < SEGS; ++g) {  // slots are fetched filled or not: one round trip, unless a slice has more than 64
+        head[g] = cand[0][g] = make_uint2(0, 0);
+        if (wave + 16 * g < slices) {
+            const uint32_t* seg = seg0 + (wave + 16 * g) * LOCAL_WORDS;
+            head[g] = *reinterpret_cast<const uint2*>(seg);
+            cand[0][g] = reinterpret_cast<const uint2*>(seg + LOCAL_HEAD)[lane];
+        }
+    }
+    if (tid < 3) s_n[tid] = 0;
+    const ptm_sampling p = sampler_params(a);
+    const int step = o.d_step ? *o.d_step : 0, k = sampler_k(p);
+    const int64_t past_now = o.adv.d_past ? *o.adv.d_past : 0;
+    const float r_draw = o.uniforms[step];
+    if (wave == 0) {
+        uint32_t v[MAXIMA];
+#pragma unroll
+        for (int t = 0; t < MAXIMA; ++t) v[t] = lane / 4 + 16 * t < slices ? seg0[(lane / 4 + 16 * t) * LOCAL_WORDS + 2 + lane % 4] : 0u;
+        const uint32_t t = kth_of_wave(v, k, 14);
+        if (lane == 0) s_bound = t;
+    }
+    __syncthreads();
+    const uint32_t bound = s_bound;
+    uint32_t most = 0, left_out = 0;
+#pragma unroll
+    for (int g = 0; g < SEGS; ++g) {
+        most = max(most, head[g].x);
+        left_out = max(left_out, head[g].y);
+    }
+    if (lane == 0 && left_out) atomicMax(&s_n[1], left_out);
+    auto list = [&](int h) {  // one reservation per wave
+        bool in[SEGS];
+        uint32_t count = 0;
+#pragma unroll
+        for (int g = 0; g < SEGS; ++g) {
+            in[g] = (uint32_t)(lane + 64 * h) < head[g].x && cand[h][g].x >= bound;
+            count += (uint32_t)__popcll(__ballot(in[g]));
+        }
+        if (count == 0) return;
+        uint32_t slot = 0;
+        if (lane == 0) slot = atomicAdd(&s_n[0], count);
+        slot = lane_u(slot, 0);
+#pragma unroll
+        for (int g = 0; g < SEGS; ++g) {
+            const unsigned long long who = __ballot(in[g]);
+            const uint32_t at = slot + (uint32_t)__popcll(who & ((1ull << lane) - 1ull));
+            if (in[g] && at < SAMPLER_MAX_CAND) l.sort[at] = ((unsigned long long)cand[h][g].y << 32) | cand[h][g].x;
+            slot += (uint32_t)__popcll(who);
+        }
+    };
+    list(0);
+    if (most > 64) {
+#pragma unroll
+        for (int g = 0; g < SEGS; ++g) cand[1][g] = wave + 16 * g < slices ? reinterpret_cast<const uint2*>(seg0 + (wave + 16 * g) * LOCAL_WORDS + LOCAL_HEAD)[lane + 64] : make_uint2(0, 0);
+        list(1);
+    }
+    __syncthreads();
+    const int n = (int)s_n[0];
+    left_out = s_n[1];
+    if (n <= 64 && left_out == 0u) {
+        if (tid >= 64) return;
+        const uint32_t key = lane < n ? (uint32_t)l.sort[lane] : 0u, idx = lane < n ? (uint32_t)(l.sort[lane] >> 32) : 0u;
+        int greater = 0;
+        for (int j = 0; j < n; j += 8)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) greater += lane_u(key, j + u) > key;
+        const bool keep = lane < n && greater < k;
+        const unsigned long long kept = __ballot(keep);
+        if (keep) l.sort[__popcll(kept & ((1ull << lane) - 1ull))] = ((unsigned long long)idx << 32) | key;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const unsigned long long c = l.sort[lane];
+        const int token = sampler_draw64(a, p, l, __popcll(kept), (uint32_t)c, (uint32_t)(c >> 32), r_draw);
+        if (tid == 0) sampler_publish(o, token, step, past_now);
+        return;
+    }
+    // Few slices, ties at the threshold, or a slice's list that was too short.  What was left out does not matter where k candidates are above it.
+    uint32_t thr = 0;
+    bool listed = n <= SAMPLER_MAX_CAND;
+    if (listed) {
+        unsigned long long c[2];
+        bool keep[2];
+        int above = 0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int i = tid + 1024 * q;
+            c[q] = l.sort[max(0, min(i, n - 1))];
+            int greater = 0;
+            for (int j = 0; j < n; ++j) greater += (uint32_t)l.sort[j] > (uint32_t)c[q];
+            keep[q] = i < n && greater < k;
+            above += i < n && (uint32_t)c[q] > left_out;
+        }
+        __syncthreads();
+        if (tid == 0) s_n[0] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (keep[q]) l.sort[atomicAdd(&s_n[2], 1u)] = c[q];
+        if (above) atomicAdd(&s_n[0], (uint32_t)above);
+        __syncthreads();
+        listed = left_out == 0u || s_n[0] >= (uint32_t)k;
+    }
+    if (!listed) {  // the vocabulary once more: its k-th largest key, three levels of bins walked from the top
+        uint32_t* hist = reinterpret_cast<uint32_t*>(l.sort);
+        int want = k;
+        for (int level = 0; level < 3; ++level) {
+            const int nb = level == 2 ? 1024 : 2048;
+            __syncthreads();
+            for (int i = tid; i < nb; i += 1024) hist[i] = 0;
+            __syncthreads();
+            for (int i = tid; i < a.vocab; i += 1024) {
+                const uint32_t key = order_key(sampler_value(a, p, i));
+                if (level == 0) atomicAdd(&hist[key >> 21], 1u);
+                else if (level == 1) { if (key >> 21 == thr) atomicAdd(&hist[key >> 10 & 0x7ffu], 1u); }
+                else if (key >> 10 == thr) atomicAdd(&hist[key & 0x3ffu], 1u);
+            }
+            __syncthreads();
+            int b = nb - 1;
+            while (b > 0 && hist[b] < (uint32_t)want) want -= (int)hist[b--];   // every thread the same walk
+            thr = level == 0 ? (uint32_t)b : thr << (level == 1 ? 11 : 10) | (uint32_t)b;
+        }
+        __syncthreads();
+        if (tid == 0) s_n[2] = 0;
+        __syncthreads();
+        for (int i = tid; i < a.vocab; i += 1024) {
+            const uint32_t key = order_key(sampler_value(a, p, i));
+            if (key >= thr) {
+                const uint32_t slot = atomicAdd(&s_n[2], 1u);
+                if (slot < SAMPLER_MAX_CAND) l.sort[slot] = ((unsigned long long)(uint32_t)i << 32) | key;
+            }
+        }
+        __syncthreads();
+        if (s_n[2] > SAMPLER_MAX_CAND) return sampler_overflow_body(a, o, thr, l.sort);
+    }
+    const int m = (int)s_n[2];
+    if (m <= 64) {
+        if (tid >= 64) return;
+        const unsigned long long c = l.sort[lane];
+        const int token = sampler_draw64(a, p, l, m, (uint32_t)c, (uint32_t)(c >> 32), r_draw);
+        if (tid == 0) sampler_publish(o, token, step, past_now);
+        return;
+    }
+    const int token = sampler_draw_list(a, p, l, m, r_draw);
+    if (tid == 0) sampler_publish(o, token, step, past_now);
 }
 
 static bool sampler_is_wide(const ptm_sampling& p, int vocab) {
@@ -814,11 +1061,16 @@ static int sampler_check(const ptm_sampling& p, int vocab) {
     return PTM_OK;
 }
 
-// Which launch sequence sampler_enqueue records for these parameters: 0 = candidate list (greedy included); otherwise the
-// whole-vocabulary passes, bit 1 = with the top-k select, bit 2 = with the nucleus walk.  A captured graph of one key must
+// The short path's slices hold up to two values per thread.
+static bool sampler_is_local(const ptm_sampling& p, int vocab) {
+    return vocab <= LOCAL_SLICES * 2048 && !(p.temperature >= 1e-6f && p.top_k > LOCAL_MAX_TOPK) && !sampler_is_wide(p, vocab);
+}
+
+// Which launch sequence sampler_enqueue records for these parameters: 0 = candidate list by slices (greedy included), 8 = by histograms;
+// otherwise the whole-vocabulary passes, bit 1 = with the top-k select, bit 2 = with the nucleus walk.  A captured graph of one key must
 // not be replayed for parameters of another.
 int sampler_launch_key(const ptm_sampling& p, int vocab) {
-    if (!sampler_is_wide(p, vocab)) return 0;
+    if (!sampler_is_wide(p, vocab)) return sampler_is_local(p, vocab) ? 0 : 8;
     return 1 | ((p.top_k > 0 && p.top_k < vocab) ? 2 : 0) | (p.top_p < 1.0f ? 4 : 0);
 }
 
@@ -835,6 +1087,13 @@ int sampler_enqueue(const float* logits, int vocab, const int32_t* counts, const
     SamplerArgs a{logits, counts, vocab, d_params, host_params, static_cast<uint32_t*>(workspace)};
     SamplerOut o{out_token, d_uniforms, d_step, counts_rw, adv, ws_kept_clean ? 1 : 0};
     const dim3 grid((vocab + SAMPLER_ELEMS_PER_WG - 1) / SAMPLER_ELEMS_PER_WG);
+    if (sampler_is_local(host_params, vocab)) {
+        const int per = vocab <= LOCAL_SLICES * 1024 ? 1024 : 2048, slices = (vocab + per - 1) / per;
+        if (per == 1024) hipLaunchKernelGGL(sampler_local_kernel<1>, dim3(slices), dim3(1024), 0, s, a);
+        else hipLaunchKernelGGL(sampler_local_kernel<2>, dim3(slices), dim3(1024), 0, s, a);
+        hipLaunchKernelGGL(sampler_local_finish_kernel, dim3(1), dim3(1024), 0, s, a, o, slices);
+        return launch_status();
+    }
     if (!ws_kept_clean) hipLaunchKernelGGL(sampler_clear_kernel, dim3(4), dim3(256), 0, s, a.ws);
     if (sampler_is_wide(host_params, vocab)) {
         // top-k off, or a top-k beyond the candidate list: passes over the whole vocabulary instead of a gathered list
@@ -863,7 +1122,6 @@ int sampler_enqueue(const float* logits, int vocab, const int32_t* counts, const
     hipLaunchKernelGGL(sampler_hist_kernel<2>, grid, dim3(256), 0, s, a);
     hipLaunchKernelGGL(sampler_gather_kernel, grid, dim3(256), 0, s, a);
     hipLaunchKernelGGL(sampler_finish_kernel, dim3(1), dim3(1024), 0, s, a, o);
-    hipLaunchKernelGGL(sampler_overflow_kernel, dim3(1), dim3(1024), 0, s, a, o);   // returns at once in the usual case
     return launch_status();
 }
 

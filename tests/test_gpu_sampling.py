@@ -342,3 +342,37 @@ def test_generate_loop_with_stop_tokens(dev, po, seeds):
     with pytest.raises(PtmError):
         dec.generate(prompt, [0.5] * 200, *params)          # does not fit the cache
     dec.close()
+
+
+@pytest.mark.parametrize("vocab,top_k", [(65, 64), (1023, 64), (1024, 1), (1025, 40), (2049, 64), (131072, 20), (131073, 64), (262144, 40),
+                                         (262145, 40), (20000, 65), (20000, 64)])
+@pytest.mark.parametrize("kind", ["normal", "one_slice", "close", "masked", "descending"])
+def test_candidates_by_slices(dev, po, vocab, top_k, kind):
+    """Top-k up to 64 selects per slice of the vocabulary first: the edges of its slices, its largest vocabulary and top-k and the first
+    beyond, all of the largest values in one slice, more values within a slice's 16-bit threshold than its list holds (with
+    the top k above them or among them), most of the vocabulary at -1e9, and sorted logits."""
+    g = synth.rng_for(92, vocab, top_k)
+    x = (2 * g.standard_normal(vocab, dtype=np.float32)).astype(np.float32)
+    if kind == "one_slice":
+        x[vocab // 2:vocab // 2 + 90] += 20.0
+    elif kind == "close":   # a quarter within 0.2 % of 3, fewer than k above them
+        x[::4] = 3.0 + 0.006 * g.random(len(x[::4]), dtype=np.float32)
+        x[g.integers(0, vocab, 30)] = 8.0
+    elif kind == "masked":
+        x[g.random(vocab) > 0.002] = -1e9
+        x[g.integers(0, vocab, 12)] = 5.0
+    elif kind == "descending":
+        x = np.sort(x)[::-1].copy()
+    tied = int((x >= np.sort(x)[-min(top_k, vocab)]).sum())
+    checked = 0
+    for r in (0.0031, 0.21371, 0.52193, 0.70937, 0.90173, 0.99731):  # (30 equal values share most of it: no multiples of 1 / n)
+        tok_o, gap, probs = po.sample_token(x, 0.8, top_k, 0.95, r, want_probs=True)
+        tok_g = gpu_sample(x, 0.8, top_k, 0.95, r)
+        if tied > 2048 or wide(vocab, 0.8, top_k):
+            check_wide_draw(tok_g, tok_o, gap, probs, r, max(GAP_TOL, 3e-9 * vocab), vocab)
+            checked += 1
+        elif gap > GAP_TOL:
+            assert tok_g == tok_o, (r, gap)
+            checked += 1
+    assert checked >= 4
+    assert gpu_sample(x, 0.0, 1, 1.0, 0.5) == int(np.argmax(x))
