@@ -189,6 +189,49 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage& st, const Q4KAr
     __syncthreads();
 }
 
+// The same for workgroups of more than four waves (RMSNorm, K <= 4096): the sum of squares is that of the form above, by the first
+// four waves, thread by thread and in the same order; the values are quantised four per thread by all of them.
+template <int NX>
+struct Q4KWideStage { float4 s[4], x[NX], g[NX]; };
+template <int NX>
+__device__ __forceinline__ Q4KWideStage<NX> q4k_wide_issue(const Q4KArgs& a) {
+    Q4KWideStage<NX> st;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, a.K * 4), rg = make_rsrc(a.gamma, a.K * 4);
+    const int tid = threadIdx.x, threads = blockDim.x;
+    q4k_load16(rx, 16 * tid, st.s);  // zeros from the fifth wave on
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rx, (tid + threads * u) * 16, 0, 0);
+        const u32x4 g = __builtin_amdgcn_raw_buffer_load_b128(rg, (tid + threads * u) * 16, 0, 0);
+        st.x[u] = make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
+        st.g[u] = make_float4(__uint_as_float(g.x), __uint_as_float(g.y), __uint_as_float(g.z), __uint_as_float(g.w));
+    }
+    return st;
+}
+template <int NX>
+__device__ __forceinline__ void q4k_wide_finish(const Q4KWideStage<NX>& st, const Q4KArgs& a, uint8_t* lds, float* red) {
+    const int tid = threadIdx.x, threads = blockDim.x;
+    float ss = sum64(q4k_sumsq16(st.s, 0.0f));
+    if ((tid & 63) == 0 && tid < 256) red[tid >> 6] = ss;
+    __syncthreads();
+    ss = (red[0] + red[1]) + (red[2] + red[3]);
+    const float rs = 1.0f / sqrtf(ss / (float)a.K + a.eps), one = a.add_one ? 1.0f : 0.0f;
+    float* xd = reinterpret_cast<float*>(lds + a.K);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+        const int i = tid + threads * u;
+        if (4 * i < a.K) {  // whole waves: K is a multiple of 256
+            float d, sum;
+            reinterpret_cast<uint32_t*>(lds)[i] = q8_quantize4(norm4(st.x[u], st.g[u], rs, one), d, sum);
+            if ((i & 7) == 0) {
+                xd[i >> 3] = d;
+                xd[a.K / 32 + (i >> 3)] = sum;
+            }
+        }
+    }
+    __syncthreads();
+}
+
 // contribution of one super-block to lane j's chain (sub-block j of the block)
 __device__ __forceinline__ float q4k_block_term(const uint4 hdr, const uint4 qv, const uint8_t* __restrict__ lds,
                                                 int K, int b, int j) {
@@ -245,7 +288,8 @@ __device__ __forceinline__ float silu_mul_ref(float g, float u) {
 //     passes roll ACROSS tiles - a consumed block's registers are refilled with the same slot of the NEXT tile's row, so a
 //     wave never stands with nothing in flight between two tiles (behind the last tile the refills repeat that tile: their
 //     number stays static, the lines are in cache, nothing consumes them).
-template <bool XQ8, bool NORM, bool ACC, int MODE, int NB, bool ROLLT = false, bool PRE = false>
+// NX > 0: workgroups of blockDim.x / 64 waves, x staged by q4k_wide_*<NX>, one tile each; else four waves.
+template <bool XQ8, bool NORM, bool ACC, int MODE, int NB, bool ROLLT = false, bool PRE = false, int NX = 0>
 __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int wg) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 7, grp = lane >> 3;
@@ -255,12 +299,13 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
     const int nblk = a.K / 256;
     const int nb_max = (nblk + S - 1) >> a.log2S;  // passes are sized for the group with the most blocks
     const int tpw = a.tiles_per_wg > 1 ? a.tiles_per_wg : 1;
-    const int n_tiles = (a.total_rows + 4 * rows_per_wave - 1) / (4 * rows_per_wave);
+    const int waves = NX > 0 ? (int)(blockDim.x >> 6) : 4;
+    const int n_tiles = (a.total_rows + waves * rows_per_wave - 1) / (waves * rows_per_wave);
 
     // One row tile: first pass of weight loads, `between` (the activation prologue on the first tile, nothing on the
     // others), block terms, reduction, store.
     auto run_tile = [&](int tile, auto&& between) {
-        const int r = (tile * 4 + wave) * rows_per_wave + (grp >> a.log2S);
+        const int r = (tile * waves + wave) * rows_per_wave + (grp >> a.log2S);
         const bool live = r < a.total_rows;
         const int rr = live ? r : a.total_rows - 1;
         int mat = 0, local = rr;
@@ -329,6 +374,12 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
     // ---- activation loads first, then the first tile's weight loads, then the activation prologue ----
     __shared__ float red[4];
     static_assert(!(PRE && ROLLT), "the deferred post-norm is built into the one-tile-at-a-time form only");
+    if constexpr (NX > 0) {
+        static_assert(NORM && !XQ8 && !PRE && !ROLLT, "what q4k_wide_* stages");
+        const Q4KWideStage<NX> wide = q4k_wide_issue<NX>(a);
+        run_tile(wg, [&] { q4k_wide_finish<NX>(wide, a, lds, red); });
+        return;
+    }
     const Q4KStage stg = q4k_stage_issue<XQ8, NORM, PRE>(a, lds, red);
     if constexpr (ROLLT) {
         // MODE 0: one matrix (a.W[0], a.y[0]); MODE 1: virtual row 2 r = gate row r (a.W[0]), 2 r + 1 = up row r (a.W[1]).

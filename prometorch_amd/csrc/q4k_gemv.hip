@@ -38,6 +38,16 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArg
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB, true>(a, lds, blockIdx.x);
 }
 
+// Gate / up behind RMSNorm, 5 to 16 waves per CU: in workgroups of four waves each of them normalises and quantises the whole
+// vector, 300 instructions per wave in front of a tile's 250.  One workgroup per CU shares that work; rows, lanes and sums are those
+// of q4k_gemv_kernel.  2816 x 1024 5.00 -> 4.32 us, 6144 x 1536 5.83 -> 5.50, 5632 x 2048 6.32 -> 6.05.  Its barriers cost more than it
+// saves with more waves (two workgroups of ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80).
+template <int NB, int NX>
+__global__ __launch_bounds__(1024) void q4k_gemv_wide_kernel(const Q4KArgs a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    q4k_gemv_body<false, true, false, 1, NB, false, false, NX>(a, lds, blockIdx.x);
+}
+
 // Few rows, long rows (a Q4_K down projection: 2560 x 9728, as in the layers of a Q4_K_M file whose ffn_down is Q4_K): with
 // four rows per workgroup, 640 workgroups would each quantise the whole 9728-value activation vector for four rows' worth
 // of weights.  Here a workgroup is `waves` waves of one row each (the row's super-blocks strided over the wave's 8 lane
@@ -176,6 +186,26 @@ static int q4k_launch(Q4KArgs& a, hipStream_t s) {
                 case 4: hipLaunchKernelGGL((q4k_gemv_tall_kernel<XQ8, NORM, ACC, MODE, 4>), grid, block, lds, s, a); break;
                 default: hipLaunchKernelGGL((q4k_gemv_tall_kernel<XQ8, NORM, ACC, MODE, 5>), grid, block, lds, s, a); break;
             }
+            return launch_status();
+        }
+    }
+    if constexpr (NORM && MODE == 1) {
+        const int rows_per_wave = 8 >> a.log2S, total = (a.total_rows + rows_per_wave - 1) / rows_per_wave, per_cu = (total + 255) / 256;
+        const int nx = (a.K + 256 * per_cu - 1) / (256 * per_cu);
+        if (per_cu >= 5 && per_cu <= 16 && nx <= 2 && nb <= 5) {
+            const dim3 grid((total + per_cu - 1) / per_cu);
+#define PTM_WIDE(NBV, NXV) hipLaunchKernelGGL((q4k_gemv_wide_kernel<NBV, NXV>), grid, dim3(64 * per_cu), lds, s, a)
+            switch (2 * nb + nx) {
+                case 5: PTM_WIDE(2, 1); break;
+                case 6: PTM_WIDE(2, 2); break;
+                case 7: PTM_WIDE(3, 1); break;
+                case 8: PTM_WIDE(3, 2); break;
+                case 9: PTM_WIDE(4, 1); break;
+                case 10: PTM_WIDE(4, 2); break;
+                case 11: PTM_WIDE(5, 1); break;
+                default: PTM_WIDE(5, 2); break;
+            }
+#undef PTM_WIDE
             return launch_status();
         }
     }

@@ -401,6 +401,23 @@ def test_fused_gate_up_silu_tall_shapes_vs_oracle(dev, po, N, K):
     assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2
 
 
+@pytest.mark.parametrize("N,K", [(5120, 256), (1281, 1024), (2816, 1024), (4096, 1024), (4097, 1024), (1900, 2560), (2100, 4096), (3333, 1536)])
+def test_fused_gate_up_silu_one_workgroup_per_cu(dev, po, N, K):
+    """5 to 16 waves per CU (4097 x 1024: the first beyond): one or two values of x per thread, rows that end inside a wave; bars as above."""
+    r = synth.rng_for(58, N, K)
+    Wg, Wu = synth.make_q4k(r, N, K), synth.make_q4k(r, N, K)
+    x = (synth.make_x(r, K) * 2.0).astype(np.float32)
+    gam = (1.0 + 0.1 * r.standard_normal(K)).astype(np.float32) * np.float32(0.05)
+    xn = po.rmsnorm(x, gam, 1e-6)
+    ref = po.silu_mul(po.gemv(12, Wg, xn), po.gemv(12, Wu, xn))
+    act = torch.full((N + 4,), 5.0, device="cuda")
+    ops.fused_rmsnorm_gate_up_silu(cu(x), cu(gam), cu(Wg), cu(Wu), act, K, N, Wg.shape[1], 1e-6, False)
+    torch.cuda.synchronize()
+    got = act.cpu().numpy()
+    err = np.abs(got[:N].astype(np.float64) - ref) / np.sqrt((ref.astype(np.float64) ** 2).mean())
+    assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[N:] == 5.0)
+
+
 # ---------------------------------------------------------------------------------------------
 # glue
 # ---------------------------------------------------------------------------------------------
