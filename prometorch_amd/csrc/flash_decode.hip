@@ -317,22 +317,19 @@ __global__ __launch_bounds__(FD_THREADS) void flash_decode_partial_kernel(
     }
 }
 
-// Merge of the active splits: grid n_heads, 256 threads = NSLOT split-slots x HD/4 float4 outputs.
-// Slot r sums splits r, r+NSLOT, ... in batches of 8 independent loads (the first batch is issued
-// before the max/denominator reductions so its latency overlaps them); slot sums are then added in
-// slot order, so the result does not depend on timing.
+// Merge of the active splits: a wave per 32 values of a head (one Q8 block), 8 split slots x 8 float4 outputs.  Slot r sums splits r,
+// r + 8, ... in batches of 8 independent loads; the slots are added in a fixed tree, so the result does not depend on timing.
+// The launch is one memory round trip and a chain of dependent instructions: no LDS, no barrier, and the loads spread over
+// HD / 32 CUs per head.  32 heads of 128, 33 splits: 3.2 us; a workgroup of four waves per head, sums through LDS behind three
+// barriers, 3.9.
 template <int HD>
-__global__ __launch_bounds__(256) void flash_decode_merge_kernel(const float* __restrict__ pO,
-                                                                 const float* __restrict__ pL,
-                                                                 const float* __restrict__ pM, float* __restrict__ O,
-                                                                 int n_heads, const int64_t* __restrict__ d_past,
-                                                                 int64_t past_host, int max_seq,
-                                                                 uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
-    constexpr int NOUT = HD / 4, NSLOT = 256 / NOUT;
-    __shared__ __align__(16) float4 s_stage[256];
-    __shared__ float s_red[8];
-    const int h = blockIdx.x, tid = threadIdx.x;
-    const int o_idx = tid % NOUT, slot = tid / NOUT;
+__global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __restrict__ pO, const float* __restrict__ pL,
+                                                                const float* __restrict__ pM, float* __restrict__ O,
+                                                                int n_heads, const int64_t* __restrict__ d_past,
+                                                                int64_t past_host, int max_seq,
+                                                                uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
+    constexpr int NOUT = HD / 4;
+    const int h = blockIdx.x, lane = threadIdx.x, slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
     const float4* pO4 = reinterpret_cast<const float4*>(pO);
     // Every load of the common case goes out before the position is known: chunk slots past the last active one
     // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the kernel makes one
@@ -346,46 +343,42 @@ __global__ __launch_bounds__(256) void flash_decode_merge_kernel(const float* __
     // partial maxima are natural-log scores, or base-2 ones (log2_units) from the matrix-core kernel
     const float ek = log2_units ? 1.0f : 1.44269504088896340736f;
     auto wexp = [ek](float x) { return __builtin_amdgcn_exp2f(x * ek); };
+    const int s_first = min(lane, ns_max - 1);
+    const float pm_first = pM[(int64_t)s_first * n_heads + h], pl_first = pL[(int64_t)s_first * n_heads + h];
     float4 v[8];
     float mm[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-        const int sc = min(slot + u * NSLOT, ns_max - 1);
+        const int sc = min(slot + 8 * u, ns_max - 1);
         v[u] = pO4[((int64_t)sc * n_heads + h) * NOUT + o_idx];
         mm[u] = pM[(int64_t)sc * n_heads + h];
     }
-    const int s_first = min(tid, ns_max - 1);
-    const float pm_first = pM[(int64_t)s_first * n_heads + h], pl_first = pL[(int64_t)s_first * n_heads + h];
     int64_t total = past + 1;
     if (total > max_seq) total = max_seq;
     if (total <= 0) return;
     const int n_chunks = (int)((total + chunk - 1) >> cs_);
     const int cpw_ = long_mode ? (n_chunks + (int)FD_LONG_SPLITS - 1) / (int)FD_LONG_SPLITS : 1;
     const int ns = long_mode ? (n_chunks + cpw_ - 1) / cpw_ : n_chunks;
-    float m = tid < ns ? pm_first : -INFINITY;
-    for (int sI = tid + 256; sI < ns; sI += 256) m = fmaxf(m, pM[(int64_t)sI * n_heads + h]);
-    m = max64(m);
-    if ((tid & 63) == 0) s_red[tid >> 6] = m;
-    __syncthreads();
-    const float M = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-    float den = tid < ns ? wexp(pm_first - M) * pl_first : 0.0f;
-    for (int sI = tid + 256; sI < ns; sI += 256)
+    float m = lane < ns ? pm_first : -INFINITY;
+    for (int sI = lane + 64; sI < ns; sI += 64) m = fmaxf(m, pM[(int64_t)sI * n_heads + h]);
+    const float M = max64(m);
+    float den = lane < ns ? wexp(pm_first - M) * pl_first : 0.0f;
+    for (int sI = lane + 64; sI < ns; sI += 64)
         den = fmaf(wexp(pM[(int64_t)sI * n_heads + h] - M), pL[(int64_t)sI * n_heads + h], den);
     den = sum64(den);
-    if ((tid & 63) == 0) s_red[4 + (tid >> 6)] = den;
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = slot; s0 < ns; s0 += NSLOT * 8) {
-        if (s0 != slot) {
+    for (int s0 = 0; s0 < ns; s0 += 64) {
+        if (s0 > 0) {
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int sc = min(s0 + u * NSLOT, ns - 1);
+                const int sc = min(s0 + slot + 8 * u, ns - 1);
                 v[u] = pO4[((int64_t)sc * n_heads + h) * NOUT + o_idx];
                 mm[u] = pM[(int64_t)sc * n_heads + h];
             }
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const bool on = (s0 + u * NSLOT) < ns;  // a select, not a zero weight: inactive slots may hold anything
+            const bool on = s0 + slot + 8 * u < ns;  // a select, not a zero weight: inactive slots may hold anything
             const float w = wexp(mm[u] - M);
             sum.x = on ? fmaf(w, v[u].x, sum.x) : sum.x;
             sum.y = on ? fmaf(w, v[u].y, sum.y) : sum.y;
@@ -393,31 +386,28 @@ __global__ __launch_bounds__(256) void flash_decode_merge_kernel(const float* __
             sum.w = on ? fmaf(w, v[u].w, sum.w) : sum.w;
         }
     }
-    s_stage[slot * NOUT + o_idx] = sum;
-    __syncthreads();
-    if (tid < NOUT) {
-        float4 t = s_stage[tid];
-        for (int r = 1; r < NSLOT; ++r) {
-            const float4 u = s_stage[r * NOUT + tid];
-            t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
-        }
-        const float dsum = (s_red[4] + s_red[5]) + (s_red[6] + s_red[7]);
-        const float inv = 1.0f / (dsum + 1e-10f);  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
-        const float4 o4 = make_float4(t.x * inv, t.y * inv, t.z * inv, t.w * inv);
-        reinterpret_cast<float4*>(O)[(int64_t)h * NOUT + tid] = o4;
-        if (q8_out) {
-            // the same vector as Q8 blocks (int8 qs[K] | float d[K/32] | float sum[K/32], K = n_heads * HD) for a Q4_K
-            // output projection, whose prologue then copies 1.25 bytes per value instead of quantising 4
-            const int K = n_heads * HD;
-            float d, sm;
-            const uint32_t packed = q8_quantize4(o4, d, sm);  // 8 consecutive lanes hold one block of 32
-            reinterpret_cast<uint32_t*>(q8_out)[(int64_t)h * NOUT + tid] = packed;
-            if ((tid & 7) == 0) {
-                float* dd = reinterpret_cast<float*>(q8_out + K);
-                const int blk = h * (HD / 32) + (tid >> 3);
-                dd[blk] = d;
-                dd[K / 32 + blk] = sm;
-            }
+    auto slots = [](float x) {  // over the lanes with equal lane % 8
+        x += dpp_f<0x128>(x);  // row_ror:8
+        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    const float inv = 1.0f / (den + 1e-10f);  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
+    const float4 o4 = make_float4(slots(sum.x) * inv, slots(sum.y) * inv, slots(sum.z) * inv, slots(sum.w) * inv);
+    if (lane < 8) reinterpret_cast<float4*>(O)[(int64_t)h * NOUT + o_idx] = o4;
+    if (q8_out) {
+        // the same vector as Q8 blocks (int8 qs[K] | float d[K/32] | float sum[K/32], K = n_heads * HD) for a Q4_K
+        // output projection, whose prologue then copies 1.25 bytes per value instead of quantising 4
+        const int K = n_heads * HD;
+        float d, sm;
+        const uint32_t packed = q8_quantize4(o4, d, sm);  // 8 consecutive lanes hold one block of 32
+        if (lane < 8) reinterpret_cast<uint32_t*>(q8_out)[(int64_t)h * NOUT + o_idx] = packed;
+        if (lane == 0) {
+            float* dd = reinterpret_cast<float*>(q8_out + K);
+            const int blk = h * (HD / 32) + blockIdx.y;
+            dd[blk] = d;
+            dd[K / 32 + blk] = sm;
         }
     }
 }
@@ -427,11 +417,11 @@ static int fd_merge(int head_dim, int n_heads, hipStream_t s, const float* pO, c
                     int chunk = FD_CHUNK, int log2_units = 0) {
     const int chunk_shift = chunk < 0 ? -1 : chunk == 128 ? 7 : 6;
     if (head_dim == 256)
-        hipLaunchKernelGGL(flash_decode_merge_kernel<256>, dim3(n_heads), dim3(256), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
+        hipLaunchKernelGGL(flash_decode_merge_kernel<256>, dim3(n_heads, 8), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
     else if (head_dim == 128)
-        hipLaunchKernelGGL(flash_decode_merge_kernel<128>, dim3(n_heads), dim3(256), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
+        hipLaunchKernelGGL(flash_decode_merge_kernel<128>, dim3(n_heads, 4), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
     else
-        hipLaunchKernelGGL(flash_decode_merge_kernel<64>, dim3(n_heads), dim3(256), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
+        hipLaunchKernelGGL(flash_decode_merge_kernel<64>, dim3(n_heads, 2), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
     return launch_status();
 }
 

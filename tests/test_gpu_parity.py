@@ -539,6 +539,12 @@ def test_flash_decode_vs_oracle(dev, po, kv_fp16, nh, nkv, hd, T):
     assert np.abs(got - want).max() <= 2e-5 * max(np.abs(want).max(), 1e-3) + 1e-6
 
 
+@pytest.mark.parametrize("nh,nkv,hd,T", [(8, 2, 128, 4096), (8, 2, 128, 4097), (4, 1, 64, 8300), (2, 2, 256, 4200)])
+def test_flash_decode_merges_any_number_of_splits(dev, po, nh, nkv, hd, T):
+    """64 splits are one batch of the merge's loads; 65 and more take further ones."""
+    test_flash_decode_vs_oracle(dev, po, True, nh, nkv, hd, T)
+
+
 def test_elementwise_embedding_argmax(dev, po):
     r = synth.rng_for(45)
     g = (synth.make_x(r, 9728) * 30).astype(np.float32)
