@@ -351,9 +351,9 @@ __global__ __launch_bounds__(256) void qgemm_prepare_rows_f16_kernel(const void*
 // rms_norm_kernel), PRE 2 = SiLU(gate) * up (the arithmetic of silu_mul_kernel), or tanh-GELU(gate) * up (that of
 // gelu_mul_kernel) when add_one, which has no other meaning for PRE 2, is set.  Writes the Q8-rounded form (for Q4_K
 // matrices) and / or the plain form (for Q6_K matrices) in one pass; either output may be NULL.
-// THREADS: 256, or 1024 for PRE 2 on short prompts (one workgroup per row: with few rows the launch lasts as long as one
-// row's dependent chain, which four times the threads shorten; the row maximum does not depend on the thread count).
-template <int PRE, int THREADS = 256>
+// PRE 2 has 1024 threads per row (256: 512 rows of 9728 16.9 us, 12.8 so; 2048 of 14336 69 -> 57, 252 MB), PRE 1 the 256 whose order
+// the RMSNorm's sum has.
+template <int PRE, int THREADS = PRE == 2 ? 1024 : 256>
 __global__ __launch_bounds__(THREADS) void qgemm_prepare_fused_kernel(const float* __restrict__ X, const float* __restrict__ X2,
                                                                   float eps, int add_one, _Float16* __restrict__ Xh_round,
                                                                   float* __restrict__ rs_round, _Float16* __restrict__ Xh_plain,
@@ -380,27 +380,28 @@ __global__ __launch_bounds__(THREADS) void qgemm_prepare_fused_kernel(const floa
         ss = block_sum256(ss, red);
         rs = 1.0f / sqrtf(ss / (float)K + eps);
     }
-    auto value4 = [&](int i) {
-        const float4 a = reinterpret_cast<const float4*>(x)[i], b = reinterpret_cast<const float4*>(x2)[i];
+    const bool gelu = PRE == 2 && add_one != 0;
+    auto value = [&](float4 a, float4 b) {
         float4 r;
         if constexpr (PRE == 1) {
             r.x = a.x * rs * (b.x + one); r.y = a.y * rs * (b.y + one); r.z = a.z * rs * (b.z + one); r.w = a.w * rs * (b.w + one);
         } else {
-            const bool gelu = add_one != 0;
-            auto silu_mul = [gelu](float g, float u) {
-                if (gelu) {
-                    const float x3 = g * g * g;
-                    const float t = tanhf(0.7978845608028654f * (g + 0.044715f * x3));
-                    return 0.5f * g * (1.0f + t) * u;
-                }
+            auto silu_mul = [](float g, float u) {
                 float ng = 0.0f - g;
                 ng = fminf(fmaxf(ng, -88.0f), 88.0f);
                 return (g * (1.0f / (1.0f + expf(ng)))) * u;
             };
-            r.x = silu_mul(a.x, b.x); r.y = silu_mul(a.y, b.y); r.z = silu_mul(a.z, b.z); r.w = silu_mul(a.w, b.w);
+            auto gelu_mul = [](float g, float u) {
+                const float x3 = g * g * g;
+                const float t = tanhf(0.7978845608028654f * (g + 0.044715f * x3));
+                return 0.5f * g * (1.0f + t) * u;
+            };
+            if (gelu) { r.x = gelu_mul(a.x, b.x); r.y = gelu_mul(a.y, b.y); r.z = gelu_mul(a.z, b.z); r.w = gelu_mul(a.w, b.w); }
+            else { r.x = silu_mul(a.x, b.x); r.y = silu_mul(a.y, b.y); r.z = silu_mul(a.z, b.z); r.w = silu_mul(a.w, b.w); }
         }
         return r;
     };
+    auto value4 = [&](int i) { return value(reinterpret_cast<const float4*>(x)[i], reinterpret_cast<const float4*>(x2)[i]); };
     // Rows of up to 16384 values are computed once and kept in registers between the maximum and the store pass: all of a
     // thread's loads go out together, and the exponentials of PRE 2 are paid once (the pass is otherwise two dependent
     // sweeps over 2 x 4 K bytes per row).
@@ -409,10 +410,19 @@ __global__ __launch_bounds__(THREADS) void qgemm_prepare_fused_kernel(const floa
     float4 hv[HOLD];
     float amax = 0.0f;
     if (held) {
+        float4 hx[HOLD];
+#pragma unroll
+        for (int u = 0; u < HOLD; ++u) {  // the loads go out together
+            const int i = tid + THREADS * u;
+            hv[u] = hx[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i < n4) {
+                hv[u] = reinterpret_cast<const float4*>(x)[i];
+                hx[u] = reinterpret_cast<const float4*>(x2)[i];
+            }
+        }
 #pragma unroll
         for (int u = 0; u < HOLD; ++u) {
-            const int i = tid + THREADS * u;
-            hv[u] = i < n4 ? value4(i) : make_float4(0.f, 0.f, 0.f, 0.f);
+            hv[u] = tid + THREADS * u < n4 ? value(hv[u], hx[u]) : make_float4(0.f, 0.f, 0.f, 0.f);
             amax = fmaxf(amax, fmaxf(fmaxf(fabsf(hv[u].x), fabsf(hv[u].y)), fmaxf(fabsf(hv[u].z), fabsf(hv[u].w))));
         }
     } else {
@@ -1169,11 +1179,12 @@ int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool acc
     float* rp = hp ? reinterpret_cast<float*>(hp + (int64_t)mp * K) : nullptr;
 #define PTM_RN(B, T) hipLaunchKernelGGL((qgemm_reduce_norm_prepare_kernel<B, T>), dim3(mp), dim3(T), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0, gamma, eps, add_one, hr, rr, hp, rp, M, K)
     // up to 128 rows the launch lasts as long as one row's chain of requests: as many threads as the row has pieces (4 / 8 / 16 slabs of 2560
-    // values 9.4 -> 6.5 us)
+    // values 9.4 -> 6.5 us).  Beyond, 512 (953 rows of 4096, two slabs: 256 threads 22.6 us, 512 20.8, 1024 22.3; 509 of 2560, six: 12.1,
+    // 11.6, 13.5)
     if (M <= 128 && K > 2048) PTM_RN(16, 1024);
     else if (M <= 128 && K > 1024) PTM_RN(16, 512);
-    else if (splits <= 4) PTM_RN(4, 256);
-    else PTM_RN(8, 256);
+    else if (splits <= 4) PTM_RN(4, 512);
+    else PTM_RN(8, 512);
 #undef PTM_RN
     return launch_status();
 }
@@ -1283,8 +1294,7 @@ int qgemm_f16_prepare_fused(int pre, const float* X, const float* X2, float eps,
     float* rr = hr ? reinterpret_cast<float*>(hr + (int64_t)mp * K) : nullptr;
     float* rp = hp ? reinterpret_cast<float*>(hp + (int64_t)mp * K) : nullptr;
     if (pre == 1) hipLaunchKernelGGL(qgemm_prepare_fused_kernel<1>, dim3(mp), dim3(256), 0, s, X, X2, eps, add_one, hr, rr, hp, rp, M, K);
-    else if (pre == 2 && M <= 128) hipLaunchKernelGGL((qgemm_prepare_fused_kernel<2, 1024>), dim3(mp), dim3(1024), 0, s, X, X2, eps, add_one, hr, rr, hp, rp, M, K);
-    else if (pre == 2) hipLaunchKernelGGL(qgemm_prepare_fused_kernel<2>, dim3(mp), dim3(256), 0, s, X, X2, eps, add_one, hr, rr, hp, rp, M, K);
+    else if (pre == 2) hipLaunchKernelGGL(qgemm_prepare_fused_kernel<2>, dim3(mp), dim3(1024), 0, s, X, X2, eps, add_one, hr, rr, hp, rp, M, K);
     else return PTM_E_UNSUPPORTED;
     return launch_status();
 }
