@@ -12,11 +12,10 @@
 //   draw r (index 0 when r <= 0, the last index when the sum never gets there).
 //   temperature < 1e-6: argmax (strict '>', lowest index) of the penalised logits.
 // Exact selection of the k-th largest x, top-k up to 64: per slice of the vocabulary, then among the slices' candidates (below).
-// Larger top-k: a three-level radix select over the order-preserving integer image of x
-// (11 + 11 + 10 bits: one histogram pass over the vocabulary per level), then a gather of everything at or above
-// the threshold (<= SAMPLER_MAX_CAND, normally exactly k) and ONE workgroup that finishes on that short list,
-// doing the reference's sequential fp32 sums in the reference's order (so results differ from the CPU's only
-// through expf's last bit).
+// Larger top-k: a three-level radix select over the order-preserving integer image of x (11 + 11 + 10 bits: one histogram pass over
+// the vocabulary per level), then a gather of everything at or above the threshold (<= SAMPLER_MAX_CAND, normally exactly k).
+// ONE workgroup finishes on the short list, doing the reference's sequential fp32 sums in the reference's order (so results differ
+// from the CPU's only through expf's last bit).
 #include "ptm_common.h"
 
 #include <random>
