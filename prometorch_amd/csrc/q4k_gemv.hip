@@ -38,10 +38,11 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArg
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB, true>(a, lds, blockIdx.x);
 }
 
-// Gate / up behind RMSNorm, 5 to 16 waves per CU: in workgroups of four waves each of them normalises and quantises the whole
+// Gate / up behind RMSNorm, 5 to 16 waves per CU, K <= 4096: in workgroups of four waves each of them normalises and quantises the whole
 // vector, 300 instructions per wave in front of a tile's 250.  One workgroup per CU shares that work; rows, lanes and sums are those
-// of q4k_gemv_kernel.  2816 x 1024 5.00 -> 4.32 us, 6144 x 1536 5.83 -> 5.50, 5632 x 2048 6.32 -> 6.05.  Its barriers cost more than it
-// saves with more waves (two workgroups of ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80).
+// of q4k_gemv_kernel.  2816 x 1024 4.68 -> 3.92 us, 6144 x 1536 5.10 -> 4.61, 4096 x 2560 6.02 -> 5.39, 4096 x 4096 6.61 -> 6.07 (in a
+// graph; of 99 sizes from 700 x 256 to 9728 x 4096 none slower).  Its barriers cost more than it saves with more waves (two workgroups of
+// ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80).
 template <int NB, int NX>
 __global__ __launch_bounds__(1024) void q4k_gemv_wide_kernel(const Q4KArgs a) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -192,7 +193,8 @@ static int q4k_launch(Q4KArgs& a, hipStream_t s) {
     if constexpr (NORM && MODE == 1) {
         const int rows_per_wave = 8 >> a.log2S, total = (a.total_rows + rows_per_wave - 1) / rows_per_wave, per_cu = (total + 255) / 256;
         const int nx = (a.K + 256 * per_cu - 1) / (256 * per_cu);
-        if (per_cu >= 5 && per_cu <= 16 && nx <= 2 && nb <= 5) {
+        // K: the sum of squares is taken from 16 values of each of the first 256 threads (longer vectors: the loop of the four-wave form)
+        if (per_cu >= 5 && per_cu <= 16 && nx <= 2 && nb <= 5 && a.K <= 16 * Q4K_THREADS) {
             const dim3 grid((total + per_cu - 1) / per_cu);
 #define PTM_WIDE(NBV, NXV) hipLaunchKernelGGL((q4k_gemv_wide_kernel<NBV, NXV>), grid, dim3(64 * per_cu), lds, s, a)
             switch (2 * nb + nx) {

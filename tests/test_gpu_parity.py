@@ -418,6 +418,24 @@ def test_fused_gate_up_silu_one_workgroup_per_cu(dev, po, N, K):
     assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[N:] == 5.0)
 
 
+@pytest.mark.parametrize("N,K", [(4096, 4096), (2049, 4352), (4096, 4352), (2304, 4608), (3456, 5120), (3000, 6144), (4096, 8192)])
+def test_fused_gate_up_silu_norm_of_long_vectors(dev, po, N, K):
+    """5 to 16 waves per CU on either side of the longest vector whose squares one round of 256 threads adds up (4096): the normalised
+    vector, and with it gate and up, must have the whole sum in it; bars as above."""
+    r = synth.rng_for(59, N, K)
+    Wg, Wu = synth.make_q4k(r, N, K), synth.make_q4k(r, N, K)
+    x = (synth.make_x(r, K) * 2.0).astype(np.float32)
+    gam = (1.0 + 0.1 * r.standard_normal(K)).astype(np.float32) * np.float32(0.05)
+    xn = po.rmsnorm(x, gam, 1e-6)
+    ref = po.silu_mul(po.gemv(12, Wg, xn), po.gemv(12, Wu, xn))
+    act = torch.full((N + 4,), 5.0, device="cuda")
+    ops.fused_rmsnorm_gate_up_silu(cu(x), cu(gam), cu(Wg), cu(Wu), act, K, N, Wg.shape[1], 1e-6, False)
+    torch.cuda.synchronize()
+    got = act.cpu().numpy()
+    err = np.abs(got[:N].astype(np.float64) - ref) / np.sqrt((ref.astype(np.float64) ** 2).mean())
+    assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[N:] == 5.0)
+
+
 # ---------------------------------------------------------------------------------------------
 # glue
 # ---------------------------------------------------------------------------------------------
