@@ -1,7 +1,7 @@
 // Prompt products over bfloat16 weights: C[M][N] = A[M][K] . W[N][K]^T on the matrix cores.
 //
 // dense_gemm_tiles_kernel (more than 64 bfloat16 rows): the tiles of gemm_tile.h, as plan_tiles lays them out.
-// dense_gemm_kernel (up to 64 bfloat16 rows): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
+// dense_gemm_kernel (up to 64 bfloat16 rows, or rows far apart): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
 // LDS; two register sets and two LDS buffers, so a step has one barrier and the loads of the next two steps are in flight
 // while its MFMAs run.
 // LDS rows are 128 bytes, the eight 16-byte pieces of row r stored at piece ^ (r % 8): the fragment reads (32 rows, one
@@ -226,7 +226,9 @@ __device__ __forceinline__ void dense_tile(const DenseGemm& g, const GemmRegion&
     // two-byte results: a lane's two sums next to each other make one 16-byte store (1030 x 9728 x 2560 63.0 -> 57.7 us); fp32 sums of
     // one fragment are 16 bytes already, and the four lanes of a row then store 64 in a row
     const bool glu = g.epilogue == GEMM_SWIGLU, pairs = g.epilogue == GEMM_ELEM || g.epilogue == GEMM_RELU2;
-    const int w0 = weight_row(g, n0);  // GEMM_SWIGLU: tiles start with whole blocks of 32 columns, so no row of the tile lies in front of it
+    // Offsets count from a wave's first row, which no other of its rows lies in front of (GEMM_SWIGLU: tiles start with whole blocks of 32
+    // columns, and an instruction's 8 rows are gates in the waves without bit 1 and ups, half of W further on, in those with it)
+    const int w0 = weight_row(g, n0 + (glu ? (wave & 2) << 3 : 0));
     const gt_i4 xs = gt_buffer(A), ws = gt_buffer(g.W + (int64_t)w0 * g.ldw + first * 64);
     const uint32_t piece = ((lane & 7) ^ (lane >> 3)) << 4;
     uint32_t xo[Tile::NX], wo[Tile::NW];
@@ -342,6 +344,9 @@ static void launch_tiles(DenseGemm& g, int kp, bool may_split, hipStream_t s) {
     hipLaunchKernelGGL(dense_gemm_tiles_kernel, dim3((unsigned)p.wgs), dim3(512), p.lds, s, g, p.regions);
 }
 
+// Offsets in a tile are 32 bits: 255 rows of up to 8 MiB stay under 2 GiB.
+static bool rows_close(const DenseGemm& g) { return g.lda <= 1 << 22 && g.ldw <= 1 << 22; }
+
 int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (!g.A || !g.W || !g.C) return PTM_E_NULL;
     const int kp = up64(g.K);
@@ -371,7 +376,7 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     } else if (g.M <= 32) {
         split(tiles(32, 128), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<32, 128, 32, 32>), dim3((unsigned)(tiles(32, 128) * g.splits)), dim3(256), 0, s, g);
-    } else if (g.M <= 64) {
+    } else if (g.M <= 64 || !rows_close(g)) {
         split(tiles(64, 64), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<64, 64, 32, 32>), dim3((unsigned)(tiles(64, 64) * g.splits)), dim3(256), 0, s, g);
     } else {

@@ -41,6 +41,26 @@ def test_tiles(dev, M, N, K):
     assert ((C[:M, :N].double() - want).abs() <= bound).all()
 
 
+# rows so far apart that the last of 64 lies 4 GiB and more behind the first, on either side; the longest rows that tiles take, and the next
+@pytest.mark.parametrize("lda,ldw", [(36 << 20, 128), (128, 36 << 20), (1 << 22, 1 << 22), ((1 << 22) + 8, 1 << 22)])
+def test_rows_far_apart(dev, lda, ldw):
+    M, N, K = 130, 140, 100
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rows = {}
+    for name, n, ld in (("A", M, lda), ("W", N, ldw)):
+        flat = torch.empty((n - 1) * ld + 128, dtype=torch.bfloat16, device="cuda")
+        rows[name] = flat.as_strided((n, 128), (ld, 1))
+        rows[name].copy_(torch.randn(n, 128, device="cuda", generator=g))
+        rows[name][:, K:] = 0
+    C = torch.full((M, N), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    _lib.check(dev.ptm_dense_gemm(rows["A"].data_ptr(), 0, lda, rows["W"].data_ptr(), ldw, C.data_ptr(), N, M, N, K, None), "dense_gemm")
+    torch.cuda.synchronize()
+    a, w = rows["A"].double(), rows["W"].double()
+    bound = (a.abs() @ w.abs().T) * (K * 2.0 ** -24) + 1e-30  # as above
+    assert ((C.double() - a @ w.T).abs() <= bound).all()
+
+
 # the results that are not plain sums (squared ReLU, gated SiLU, decays, 16-bit rows, sections of one product) and their odd sizes
 @pytest.mark.parametrize("design", ["tovasun", "nadozen"])
 def test_prompts_of_many_rows(dev, tmp_path, design):
