@@ -1,6 +1,7 @@
 // Interfaces between the block-decoder runtime (blocks.hip) and its kernels (dense_gemv.hip, dense_gemm.hip,
 // mixer_attention.hip).  Host side; not part of the C ABI.
 #pragma once
+#include "gemm_plan.h"
 #include "ptm_common.h"
 
 namespace ptm {
@@ -111,31 +112,6 @@ int latent_absorb(const LatentStep& a, hipStream_t s);
 // out[h * up8(vdim) + v] = W_uv[h] . merged latent of head h; pM / pL NULL: pO is the finished latent [heads][o_row]
 int latent_out(const LatentStep& a, const float* pO, const float* pM, const float* pL, int splits, int o_row, float* out,
                hipStream_t s);
-
-// C = epilogue(A . W^T): GEMM_F32 fp32 C; otherwise element type of the rows (bfloat16, or fp32 when a_fp32).
-// GEMM_SWIGLU: W holds N / 2 gate rows, then N / 2 up rows; C [M][N / 2] = silu(gate) * up.
-// GEMM_DECAY: fp32 C = exp(-exp(product + bias)).
-enum { GEMM_F32 = 0, GEMM_ELEM = 1, GEMM_RELU2 = 2, GEMM_SWIGLU = 3, GEMM_DECAY = 4 };
-struct DenseGemm {
-    const void* A = nullptr;
-    int a_fp32 = 0;
-    int64_t lda = 0;
-    const uint16_t* W = nullptr;
-    int64_t ldw = 0;
-    int M = 0, N = 0, K = 0;
-    int epilogue = GEMM_F32;
-    void* C = nullptr;
-    int64_t ldc = 0;
-    // K split over workgroups where the output has too few tiles (GEMM_F32 only): split z leaves its partial sums at
-    // C + z * slab; slab_room floats are available for all of them
-    int64_t slab = 0, slab_room = 0;
-    int splits = 1, tile_cols = 0;  // set by dense_gemm
-    // rows n of W take A + n / section_n * section_a (section_n a multiple of 128; 0: one section)
-    int section_n = 0;
-    int64_t section_a = 0;
-    const float* bias = nullptr;  // [N], GEMM_DECAY
-};
-int dense_gemm(DenseGemm g, hipStream_t s, int* splits = nullptr);
 
 // Attention of one decode token, position *d_past.  bfloat16 caches with tile classes the matrix-core kernel has: splits
 // partial results (decode_attention_splits); otherwise one finished result.

@@ -1,7 +1,7 @@
 // Prompt products over bfloat16 weights: C[M][N] = A[M][K] . W[N][K]^T on the matrix cores.
 //
 // dense_gemm_tiles_kernel (more than 64 bfloat16 rows): the tiles of gemm_tile.h, as plan_tiles lays them out.
-// dense_gemm_kernel (up to 64 bfloat16 rows, or rows far apart): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
+// dense_gemm_kernel (up to 64 bfloat16 rows, outputs of few tiles, rows far apart): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
 // LDS; two register sets and two LDS buffers, so a step has one barrier and the loads of the next two steps are in flight
 // while its MFMAs run.
 // LDS rows are 128 bytes, the eight 16-byte pieces of row r stored at piece ^ (r % 8): the fragment reads (32 rows, one
@@ -331,21 +331,45 @@ __global__ __launch_bounds__(256) void dense_gemm_f32_kernel(const DenseGemm g) 
 // The times are those of 512 ... 2048 rows times 2560 ... 28672 columns, 40 and 152 steps, the chip nearly full (two thirds empty, a step
 // takes a fifth less: the CUs share the power).  Against 128 x 128 tiles of four waves, rows through registers, two workgroups a CU:
 // 2048 x 19456 x 2560 240 -> 175 us (gate, up; 1165 TFLOP/s), 2048 x 2560 x 9728 116 -> 85, 1030 x 9728 x 2560 84 -> 57 (895 TFLOP/s).
-static void launch_tiles(DenseGemm& g, int kp, bool may_split, hipStream_t s) {
-    static const TileKind kinds[] = {tile_kind<Tile0>(1300, 14000), tile_kind<Tile1>(1080, 11000), tile_kind<Tile2>(850, 8500), tile_kind<Tile3>(740, 6000),
-                                     tile_kind<Tile4>(500, 6000),   tile_kind<Tile5>(500, 6000),  tile_kind<Tile6>(340, 5000)};
-    static std::once_flag raised;
-    std::call_once(raised, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_gemm_tiles_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    });
-    const int most = may_split && g.slab > 0 ? (int)std::min<int64_t>(16, g.slab_room / g.slab) : 1;
-    const TilePlan p = plan_tiles(kinds, 7, g.M, g.tile_cols, kp / 64, most, g.section_n);
-    g.splits = p.splits;
-    hipLaunchKernelGGL(dense_gemm_tiles_kernel, dim3((unsigned)p.wgs), dim3(512), p.lds, s, g, p.regions);
+static const TileKind kinds[] = {tile_kind<Tile0>(1300, 14000), tile_kind<Tile1>(1080, 11000), tile_kind<Tile2>(850, 8500), tile_kind<Tile3>(740, 6000),
+                                 tile_kind<Tile4>(500, 6000),   tile_kind<Tile5>(500, 6000),  tile_kind<Tile6>(340, 5000)};
+
+// K splits of 64 x 64 tiles of four waves, 0 where the plan's tiles are done first.  With a CU for each workgroup their step is the shortest
+// (330 ns and 4500 in the units above), and two that share a CU take 1.7 times one's: 128 x 1024 x 1024 9.0 us as the plan has it, 7.7 so,
+// 300 x 2560 x 2560 17.4 and 15.1, 1030 x 1024 x 128 5.05 and 4.6; split, 128 x 1024 x 2816 6.7 and 5.6.  With more of them a larger tile
+// wins: 512 x 2560 x 2560 (320 tiles) 18.1 and 23.1, 300 x 5000 x 320 (395) 6.5 and 7.0.
+static int four_wave_splits(const DenseGemm& g, int64_t tiles, int steps, int most, float plan_cost) {
+    int best = 0;
+    for (int splits = 1; splits == 1 || (splits <= most && splits * 4 <= steps); ++splits) {
+        if (tiles * splits > 512) break;
+        const float step = tiles * splits > 256 ? 1.7f * 330.0f : 330.0f;
+        const float sums = splits > 1 ? (float)splits * (float)g.M * (float)g.N * 2e-3f : 0.0f;
+        const float cost = (float)((steps + splits - 1) / splits) * step + 4500.0f + sums;
+        if (cost < plan_cost) best = splits, plan_cost = cost;
+    }
+    return best;
 }
 
-// Offsets in a tile are 32 bits: 255 rows of up to 8 MiB stay under 2 GiB.
-static bool rows_close(const DenseGemm& g) { return g.lda <= 1 << 22 && g.ldw <= 1 << 22; }
+// columns that tiles cover: gates and ups in whole blocks of 16
+static int tile_columns(const DenseGemm& g) { return g.epilogue == GEMM_SWIGLU ? (g.N / 2 + 15) / 16 * 32 : g.N; }
+
+TilePlan dense_gemm_plan(const DenseGemm& g, bool may_split) {
+    const int cols = tile_columns(g), steps = up64(g.K) / 64;
+    const int most = may_split && g.slab > 0 ? (int)std::min<int64_t>(16, g.slab_room / g.slab) : 1;
+    const int64_t small = ((int64_t)g.M + 63) / 64 * ((cols + 63) / 64);
+    TilePlan p{};
+    p.splits = 1;
+    // offsets in a tile are 32 bits: 255 rows of up to 8 MiB stay under 2 GiB
+    if (g.lda <= 1 << 22 && g.ldw <= 1 << 22) {
+        p = plan_tiles(kinds, sizeof kinds / sizeof *kinds, g.M, cols, steps, most, g.section_n);
+        const int splits = four_wave_splits(g, small, steps, most, p.cost);
+        if (splits == 0) return p;
+        p = TilePlan{};
+        p.splits = splits;
+    }
+    p.wgs = (int)(small * p.splits);
+    return p;
+}
 
 int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (!g.A || !g.W || !g.C) return PTM_E_NULL;
@@ -356,8 +380,7 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (g.epilogue != GEMM_F32 && splits) return PTM_E_SHAPE;  // partial sums have no epilogue
     if (g.epilogue == GEMM_DECAY && !g.bias) return PTM_E_NULL;
     if (!aligned16(g.A) || !aligned16(g.W) || !aligned16(g.C) || (g.lda & 7) || (g.ldw & 7)) return PTM_E_ALIGN;
-    const int cols = glu ? (g.N / 2 + 15) / 16 * 32 : g.N;  // gates and ups in whole blocks of 16
-    g.tile_cols = cols;
+    const int cols = g.tile_cols = tile_columns(g);
     auto tiles = [&](int bm, int bn) { return ((int64_t)g.M + bm - 1) / bm * ((cols + bn - 1) / bn); };
     if (tiles(32, 64) * 16 > 0x7fffffff) return PTM_E_UNSUPPORTED;
     // splits that bring `t` tiles to about `target` workgroups, each with at least four steps of K
@@ -376,11 +399,21 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     } else if (g.M <= 32) {
         split(tiles(32, 128), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<32, 128, 32, 32>), dim3((unsigned)(tiles(32, 128) * g.splits)), dim3(256), 0, s, g);
-    } else if (g.M <= 64 || !rows_close(g)) {
+    } else if (g.M <= 64) {
         split(tiles(64, 64), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<64, 64, 32, 32>), dim3((unsigned)(tiles(64, 64) * g.splits)), dim3(256), 0, s, g);
     } else {
-        launch_tiles(g, kp, splits != nullptr, s);
+        const TilePlan p = dense_gemm_plan(g, splits != nullptr);
+        g.splits = p.splits;
+        if (p.regions.n == 0) {
+            hipLaunchKernelGGL((dense_gemm_kernel<64, 64, 32, 32>), dim3((unsigned)p.wgs), dim3(256), 0, s, g);
+        } else {
+            static std::once_flag raised;
+            std::call_once(raised, [] {
+                (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_gemm_tiles_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            });
+            hipLaunchKernelGGL(dense_gemm_tiles_kernel, dim3((unsigned)p.wgs), dim3(512), p.lds, s, g, p.regions);
+        }
     }
     if (splits) *splits = g.splits;
     return launch_status();

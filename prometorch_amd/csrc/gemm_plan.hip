@@ -1,5 +1,5 @@
-// Host side of gemm_tile.h: which tiles cover a product.
-#include "gemm_tile.h"
+// Which tiles cover a product.
+#include "gemm_plan.h"
 
 namespace ptm {
 

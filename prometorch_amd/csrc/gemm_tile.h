@@ -12,6 +12,7 @@
 // ordered by rows alone, without bands, 900.  Small tiles are bound by how long a fetch takes: three steps in LDS against two
 // bring 128 x 128 from 545 to 760, 128 x 256 from 890 to 1050.
 #pragma once
+#include "gemm_plan.h"
 #include "ptm_common.h"
 
 namespace ptm {
@@ -142,66 +143,10 @@ struct GemmTile {
     }
 };
 
-// ---- how a launch covers its output ----------------------------------------------------------------------------------------
-// Rows m0 .. and columns n0 .. n1 - 1 in tiles_m x tiles_n tiles of one kind, workgroups first .. (the K splits one after the other).
-struct GemmRegion {
-    int kind, first, m0, n0, n1, tiles_m, tiles_n;
-};
-struct GemmRegions {
-    int n;
-    GemmRegion r[4];
-};
-
-// A kind of tile: its size, what a workgroup takes for a step of 64 values and for its start and end (ns), its LDS.
-struct TileKind {
-    int bm, bn;
-    float step, ends;
-    int lds;
-};
+// step, ends: what a workgroup takes for a step of 64 values and for its start and end (ns)
 template <typename Tile>
 constexpr TileKind tile_kind(float step, float ends) {
     return {Tile::BM, Tile::BN, step, ends, Tile::LDS};
 }
-
-struct TilePlan {
-    GemmRegions regions;
-    int splits, wgs, lds;
-    float cost;
-};
-
-// When the last of 256 CUs is done that take workgroups one after the other, `count` of `each` ns at a time
-class ChipTime {
-    struct Part { float t; int n; };
-    Part p[10];
-    int parts = 1;
-
-public:
-    ChipTime() { p[0] = {0.0f, 256}; }
-    void run(int64_t count, float each) {
-        while (count > 0) {
-            int i = 0;
-            for (int k = 1; k < parts; ++k)
-                if (p[k].t < p[i].t) i = k;
-            if (count >= p[i].n || parts == 10) {
-                count -= p[i].n;
-                p[i].t += each;
-            } else {
-                p[i].n -= (int)count;
-                p[parts++] = {p[i].t + each, (int)count};
-                count = 0;
-            }
-        }
-    }
-    float last() const {
-        float t = 0.0f;
-        for (int k = 0; k < parts; ++k) t = p[k].t > t ? p[k].t : t;
-        return t;
-    }
-};
-
-// The regions, kinds and K splits (at most most_splits) that bring M x N outputs of `steps` steps of K to the shortest time: whole
-// rounds of the chip in one kind of tile, the columns and rows left over in smaller ones, where a last round of the large tiles would leave
-// most of the chip idle or work on rows that are not there.  section_n > 0: no tile crosses a multiple of it.
-TilePlan plan_tiles(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n);
 
 }  // namespace ptm

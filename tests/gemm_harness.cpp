@@ -1,0 +1,56 @@
+// Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
+// splits, which the C ABI's plain product does not have, and how a launch would cover its output.  Host C++ only; built by
+// __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
+#include "gemm_plan.h"
+
+extern "C" {
+
+struct GemmCall {
+    const void* A;
+    const void* W;
+    void* C;
+    const float* bias;
+    int64_t lda, ldw, ldc, section_a, slab, slab_room;
+    int32_t M, N, K, epilogue, section_n, may_split;
+};
+
+static ptm::DenseGemm dense(const GemmCall* c) {
+    ptm::DenseGemm g;
+    g.A = c->A;
+    g.W = static_cast<const uint16_t*>(c->W);
+    g.C = c->C;
+    g.bias = c->bias;
+    g.lda = c->lda;
+    g.ldw = c->ldw;
+    g.ldc = c->ldc;
+    g.section_a = c->section_a;
+    g.slab = c->slab;
+    g.slab_room = c->slab_room;
+    g.M = c->M;
+    g.N = c->N;
+    g.K = c->K;
+    g.epilogue = c->epilogue;
+    g.section_n = c->section_n;
+    return g;
+}
+
+int gemm_run(const GemmCall* c, int32_t* splits, void* stream) {
+    int n = 1;
+    const int rc = ptm::dense_gemm(dense(c), static_cast<hipStream_t>(stream), c->may_split ? &n : nullptr);
+    *splits = n;
+    return rc;
+}
+
+// splits, workgroups, regions, and of each region its seven numbers
+void gemm_plan(const GemmCall* c, int32_t* out) {
+    const ptm::TilePlan p = ptm::dense_gemm_plan(dense(c), c->may_split != 0);
+    *out++ = p.splits;
+    *out++ = p.wgs;
+    *out++ = p.regions.n;
+    for (int i = 0; i < p.regions.n; ++i) {
+        const ptm::GemmRegion& r = p.regions.r[i];
+        for (int v : {r.kind, r.first, r.m0, r.n0, r.n1, r.tiles_m, r.tiles_n}) *out++ = v;
+    }
+}
+
+}  // extern "C"

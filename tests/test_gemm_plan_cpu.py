@@ -1,0 +1,54 @@
+"""CPU: which tiles cover a prompt product of more than 64 rows, and where a launch of 64 x 64 tiles of four waves takes it instead."""
+import random
+
+import pytest
+
+from gemm_helpers import DECAY, ELEM, F32, SWIGLU, TILES, plan
+
+
+# outputs of few tiles: up to 256 of 64 x 64, up to 512 where K is short; split, tiles x splits
+@pytest.mark.parametrize("M,N,K,slabs,splits", [(65, 64, 64, 0, 1), (128, 1024, 1024, 0, 1), (300, 2560, 2560, 0, 1), (256, 4096, 2560, 0, 1), (129, 2560, 9728, 0, 1),
+                                                (1500, 64, 2560, 0, 1), (1030, 1024, 128, 0, 1), (128, 1024, 1024, 16, 4), (128, 512, 1024, 16, 4)])
+def test_few_tiles_are_four_waves_each(M, N, K, slabs, splits):
+    got = plan(M, N, K, slabs=slabs)
+    assert got == (splits, (M + 63) // 64 * ((N + 63) // 64) * splits, [])
+
+
+@pytest.mark.parametrize("M,N,K,slabs", [(512, 2560, 2560, 0), (300, 5000, 320, 0), (2048, 2560, 1024, 0), (65, 2560, 9728, 16), (1030, 9728, 64, 0)])
+def test_more_tiles_are_not(M, N, K, slabs):
+    assert plan(M, N, K, slabs=slabs)[2]
+
+
+def test_rows_far_apart_are_four_waves_each():
+    """A tile's offsets are 32 bits; K of 2^22 + 8 values makes rows longer than the longest they take."""
+    assert plan(1000, 5000, (1 << 22) + 8)[2] == [] and plan(1000, 5000, 1 << 22)[2]
+
+
+def test_plans_cover_each_output():
+    r = random.Random(4)
+    for _ in range(4000):
+        M, N, K = r.randint(65, 3000), r.randint(1, 20000), r.randint(1, 10000)
+        epilogue, section, slabs = r.choice([(F32, 0, 16), (F32, 0, 0), (ELEM, 0, 0), (SWIGLU, 0, 0), (DECAY, 0, 0), (F32, 1, 0)])
+        if section:
+            section = 128 * r.randint(1, 40)
+            N = 4 * section
+        N += N & 1
+        cols = (N // 2 + 15) // 16 * 32 if epilogue == SWIGLU else N
+        splits, wgs, regions = plan(M, N, K, epilogue, section, slabs)
+        assert 1 <= splits <= max(1, slabs) and (splits == 1 or splits * 4 <= (K + 63) // 64)
+        at, covered = 0, {}
+        for kind, first, m0, n0, n1, tm, tn in regions:
+            bm, bn = TILES[kind]
+            assert first == at and tm > 0 and tn > 0 and m0 % 32 == n0 % 32 == 0
+            assert not section or (section % bn == 0 and n0 % bn == 0)
+            at += tm * tn * splits
+            m1, n1 = min(M, m0 + tm * bm), min(n1, n0 + tn * bn, cols)
+            for n in list(range(n0, n1, 32)):
+                covered.setdefault(n, []).append((m0, m1))
+        assert not regions or at == wgs
+        for n in range(0, cols, 32) if regions else ():
+            end = 0
+            for lo, hi in sorted(covered[n]):
+                assert lo <= end, (M, N, K, n)
+                end = max(end, hi)
+            assert end == M, (M, N, K, n)

@@ -1,9 +1,12 @@
 """Prompt products of more than 64 rows: every kind of tile, alone and beside others in one launch, at the edges of rows, columns and K."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from folder_helpers import errors, portions
+from gemm_helpers import DECAY, ELEM, F32, RELU2, SWIGLU, Call, harness
 from nadozen_models import model as nadozen, parallel, wkv
 from tovasun_models import attention, latent, layer, model as tovasun
 from oracle import nadozen_oracle, tovasun_oracle
@@ -59,6 +62,61 @@ def test_rows_far_apart(dev, lda, ldw):
     a, w = rows["A"].double(), rows["W"].double()
     bound = (a.abs() @ w.abs().T) * (K * 2.0 ** -24) + 1e-30  # as above
     assert ((C.double() - a @ w.T).abs() <= bound).all()
+
+
+def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0):
+    """One product as the block decoders' runtime calls it against 64 bits; how many K splits it took."""
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N * 3 + K + epilogue)
+    kp, S = (K + 63) // 64 * 64, N // section if section else 1
+    A, W = (torch.zeros(*shape, kp, dtype=torch.bfloat16, device="cuda") for shape in ((S, M), (N,)))
+    A[..., :K], W[:, :K] = torch.randn(S, M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g) * K ** -0.5
+    cols = N // 2 if epilogue == SWIGLU else N
+    ldc, bias = cols + pad, torch.randn(N, device="cuda", generator=g) - 1
+    out = torch.full((max(1, slabs), M, ldc), float("nan"), device="cuda", dtype=torch.float32 if epilogue in (F32, DECAY) else torch.bfloat16)
+    c = Call(A=A.data_ptr(), W=W.data_ptr(), C=out.data_ptr(), bias=bias.data_ptr(), lda=kp, ldw=kp, ldc=ldc, section_a=M * kp, slab=M * ldc,
+             slab_room=M * ldc * slabs, M=M, N=N, K=K, epilogue=epilogue, section_n=section, may_split=int(slabs > 0))
+    splits = C.c_int32()
+    torch.cuda.synchronize()
+    _lib.check(harness().gemm_run(C.byref(c), C.byref(splits), None), "gemm_run")
+    torch.cuda.synchronize()
+    splits = splits.value
+    assert splits <= max(1, slabs) and torch.isnan(out[:splits, :, cols:]).all() and torch.isnan(out[splits:]).all()
+    got = out[:splits, :, :cols].double().sum(0)
+    v, off = [], []  # the products, and how far sums of K of them in any order can be from them (as above; partial sums are added exactly here)
+    for i in range(S):
+        a, w = A[i].double(), W[i * (N // S):(i + 1) * (N // S)].double()
+        v.append(a @ w.T)
+        off.append(a.abs() @ w.abs().T * (K * 2.0 ** -24) + 1e-30)
+    v, off = torch.cat(v, 1), torch.cat(off, 1)
+    half = 2.0 ** -8  # bfloat16 has 8 significant bits: half of its last place is 2^-8 of the value, or less
+    if epilogue == F32:
+        want, bound = v, off
+    elif epilogue == ELEM:
+        want, bound = v, off + (v.abs() + off) * half
+    elif epilogue == RELU2:
+        want = v.clamp(min=0) ** 2
+        slack = 2 * v.abs() * off + off ** 2 + want * 2.0 ** -23
+        bound = slack + (want + slack) * half
+    elif epilogue == SWIGLU:  # |silu'| < 1.1; exponential, division and two products in 32 bits: 2^-20 of the result
+        (gate, up), (og, ou) = v.split(N // 2, 1), off.split(N // 2, 1)
+        want = gate / (1 + torch.exp(-gate)) * up
+        slack = 1.1 * og * (up.abs() + ou) + gate.abs() * ou + want.abs() * 2.0 ** -20
+        bound = slack + (want.abs() + slack) * half
+    else:  # the derivative of exp(-exp(v)) is at most 1 / e; each exponential 2^-22 off, the inner one times x exp(-x) <= 1 / e
+        want, bound = torch.exp(-torch.exp(v + bias.double())), 0.4 * (off + 2.0 ** -23 * (v.abs() + bias.double().abs())) + 2.0 ** -21
+    assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
+    return splits
+
+
+# outputs of few tiles (64 x 64, four waves each): one, all 256 of a round and a little more, split, and every kind of result
+FEW = [(65, 64, 64, F32, 0, 0, 0), (1024, 1024, 100, F32, 0, 0, 3), (1030, 1024, 128, ELEM, 0, 0, 0), (255, 4090, 1000, F32, 0, 0, 2), (129, 1023, 1030, F32, 0, 16, 1),
+       (128, 512, 2816, F32, 0, 16, 0), (97, 1500, 320, ELEM, 0, 0, 4), (200, 1001, 640, RELU2, 0, 0, 7), (130, 2022, 1024, SWIGLU, 0, 0, 5), (300, 999, 64, DECAY, 0, 0, 1),
+       (150, 1024, 256, F32, 256, 0, 0)]
+
+
+@pytest.mark.parametrize("case", FEW, ids=str)
+def test_few_tiles(dev, case):
+    assert check_product(*case) > 1 or not case[5]
 
 
 # the results that are not plain sums (squared ReLU, gated SiLU, decays, 16-bit rows, sections of one product) and their odd sizes
