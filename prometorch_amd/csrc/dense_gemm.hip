@@ -361,7 +361,11 @@ TilePlan dense_gemm_plan(const DenseGemm& g, bool may_split) {
     p.splits = 1;
     // offsets in a tile are 32 bits: 255 rows of up to 8 MiB stay under 2 GiB
     if (g.lda <= 1 << 22 && g.ldw <= 1 << 22) {
-        p = plan_tiles(kinds, sizeof kinds / sizeof *kinds, g.M, cols, steps, most, g.section_n);
+        // 32-bit results of 50 MB and more behind four steps or fewer are bound by their stores: a launch of two kinds takes 5 to 10 us more than
+        // the times above add up to, one of a single kind 2 to 3 less (1500 x 16384 x 64 36.2 us in two kinds, 24.4 in one; 700 x 32768 x 256
+        // 41.4 and 33.5).  From five steps on either may win by a tenth, and 16-bit results add up.
+        const bool stores = steps <= 4 && (g.epilogue == GEMM_F32 || g.epilogue == GEMM_DECAY) && (int64_t)g.M * cols * 4 >= 50000000;
+        p = plan_tiles(kinds, sizeof kinds / sizeof *kinds, g.M, cols, steps, most, g.section_n, stores ? 10000.0f : 0.0f);
         const int splits = four_wave_splits(g, small, steps, most, p.cost);
         if (splits == 0) return p;
         p = TilePlan{};

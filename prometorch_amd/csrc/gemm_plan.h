@@ -85,8 +85,9 @@ public:
 
 // The regions, kinds and K splits (at most most_splits) that bring M x N outputs of `steps` steps of K to the shortest time: whole
 // rounds of the chip in one kind of tile, the columns and rows left over in smaller ones, where a last round of the large tiles would leave
-// most of the chip idle or work on rows that are not there.  section_n > 0: no tile crosses a multiple of it.
-TilePlan plan_tiles(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n);
+// most of the chip idle or work on rows that are not there.  section_n > 0: no tile crosses a multiple of it.  second_kind: what a
+// launch of more than one kind takes beyond that (ns).
+TilePlan plan_tiles(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n, float second_kind);
 
 // What dense_gemm launches for more than 64 bfloat16 rows; may_split: the caller takes partial sums.  No regions: `splits` K splits of
 // 64 x 64 tiles of four waves.

@@ -21,7 +21,7 @@ static int best_kind(const TileKind* kinds, int n_kinds, int rows, int n0, int c
     return best;
 }
 
-static TilePlan find_plan(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n) {
+static TilePlan find_plan(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n, float second_kind) {
     TilePlan best{};
     best.splits = 0;
     for (int splits = 1; splits == 1 || (splits <= most_splits && splits * 4 <= steps); ++splits) {
@@ -64,6 +64,11 @@ static TilePlan find_plan(const TileKind* kinds, int n_kinds, int M, int N, int 
                         add(b, low, 0, N, up_div(M - low, kinds[b].bm), up_div(N, kinds[b].bn));
                     }
                     p.cost = t.last() + sums;
+                    for (int i = 1; i < p.regions.n; ++i)
+                        if (p.regions.r[i].kind != k) {
+                            p.cost += second_kind;
+                            break;
+                        }
                     if (!best.splits || p.cost < best.cost) best = p;
                 }
             }
@@ -73,20 +78,21 @@ static TilePlan find_plan(const TileKind* kinds, int n_kinds, int M, int N, int 
 }
 
 // A plan depends on its arguments alone, and a prompt asks for the same few in every layer: each thread keeps the last ones it made.
-TilePlan plan_tiles(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n) {
+TilePlan plan_tiles(const TileKind* kinds, int n_kinds, int M, int N, int steps, int most_splits, int section_n, float second_kind) {
     struct Made {
         const TileKind* kinds;
         int M, N, steps, most, section;
+        float second_kind;
         TilePlan plan;
     };
     constexpr int KEPT = 16;
     static thread_local Made made[KEPT];
     static thread_local int next = 0;
     for (const Made& m : made)
-        if (m.kinds == kinds && m.M == M && m.N == N && m.steps == steps && m.most == most_splits && m.section == section_n) return m.plan;
+        if (m.kinds == kinds && m.M == M && m.N == N && m.steps == steps && m.most == most_splits && m.section == section_n && m.second_kind == second_kind) return m.plan;
     Made& m = made[next];
     next = (next + 1) % KEPT;
-    m = {kinds, M, N, steps, most_splits, section_n, find_plan(kinds, n_kinds, M, N, steps, most_splits, section_n)};
+    m = {kinds, M, N, steps, most_splits, section_n, second_kind, find_plan(kinds, n_kinds, M, N, steps, most_splits, section_n, second_kind)};
     return m.plan;
 }
 

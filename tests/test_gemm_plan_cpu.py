@@ -19,6 +19,12 @@ def test_more_tiles_are_not(M, N, K, slabs):
     assert plan(M, N, K, slabs=slabs)[2]
 
 
+@pytest.mark.parametrize("M,N,K,epilogue,kinds", [(1500, 16384, 64, F32, 1), (700, 32768, 256, F32, 1), (700, 32768, 257, F32, 2), (1500, 16384, 64, ELEM, 2), (648, 8320, 64, F32, 2),
+                                                  (2048, 19456, 2560, F32, 2)])
+def test_large_32_bit_results_of_short_products_are_of_one_kind(M, N, K, epilogue, kinds):
+    assert len({r[0] for r in plan(M, N, K, epilogue)[2]}) == kinds
+
+
 def test_rows_far_apart_are_four_waves_each():
     """A tile's offsets are 32 bits; K of 2^22 + 8 values makes rows longer than the longest they take."""
     assert plan(1000, 5000, (1 << 22) + 8)[2] == [] and plan(1000, 5000, 1 << 22)[2]
