@@ -317,23 +317,26 @@ __global__ __launch_bounds__(FD_THREADS) void flash_decode_partial_kernel(
     }
 }
 
-// Merge of the active splits: a wave per 32 values of a head (one Q8 block), 8 split slots x 8 float4 outputs.  Slot r sums splits r,
-// r + 8, ... in batches of 8 independent loads; the slots are added in a fixed tree, so the result does not depend on timing.
-// The launch is one memory round trip and a chain of dependent instructions: no LDS, no barrier, and the loads spread over
-// HD / 32 CUs per head.  32 heads of 128, 33 splits: 3.2 us; a workgroup of four waves per head, sums through LDS behind three
-// barriers, 3.9.
-template <int HD>
-__global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __restrict__ pO, const float* __restrict__ pL,
-                                                                const float* __restrict__ pM, float* __restrict__ O,
-                                                                int n_heads, const int64_t* __restrict__ d_past,
-                                                                int64_t past_host, int max_seq,
-                                                                uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
+// Merge of the active splits: a workgroup per 32 values of a head (one Q8 block), 8 split slots x 8 float4 outputs per wave.  Slot r of
+// wave w sums splits 64 w + r, + 8, ... in batches of 8 independent loads; slots are added in a fixed tree and waves in their order, so the
+// result does not depend on timing.
+// The launch is one memory round trip and a chain of dependent instructions.  Up to 64 splits are one wave's batch, no LDS and no
+// barrier, the loads spread over HD / 32 CUs per head: 32 heads of 128, 33 splits, 3.2 us (a workgroup of four waves per head, sums through
+// LDS behind three barriers: 3.9).  Where a cache can hold more, four WAVES take 64 each in turn:
+// 16 heads of 64 over 4 kv heads, 33000 / 131072 positions, partials and merge 22.0 / 59.6 us (one wave 27.7 / 83.5, the workgroup of
+// four 23.2 / 64.0); the three waves cost 0.3 us where a cache that long is still short.
+template <int HD, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const float* __restrict__ pO, const float* __restrict__ pL,
+                                                                        const float* __restrict__ pM, float* __restrict__ O,
+                                                                        int n_heads, const int64_t* __restrict__ d_past,
+                                                                        int64_t past_host, int max_seq,
+                                                                        uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
     constexpr int NOUT = HD / 4;
-    const int h = blockIdx.x, lane = threadIdx.x, slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
+    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
     const float4* pO4 = reinterpret_cast<const float4*>(pO);
     // Every load of the common case goes out before the position is known: chunk slots past the last active one
-    // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the kernel makes one
-    // memory round trip, not one for the position and a second for the data.
+    // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the first wave makes one
+    // memory round trip, not one for the position and a second for the data; the others are there for long contexts only.
     // chunk_shift < 0: the partials of the looping kernel (at most FD_LONG_SPLITS of them, cpw chunks of 64 positions each)
     const bool long_mode = chunk_shift < 0;
     const int chunk = long_mode ? FD_CHUNK : 1 << chunk_shift;  // positions per chunk
@@ -343,15 +346,27 @@ __global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __r
     // partial maxima are natural-log scores, or base-2 ones (log2_units) from the matrix-core kernel
     const float ek = log2_units ? 1.0f : 1.44269504088896340736f;
     auto wexp = [ek](float x) { return __builtin_amdgcn_exp2f(x * ek); };
-    const int s_first = min(lane, ns_max - 1);
-    const float pm_first = pM[(int64_t)s_first * n_heads + h], pl_first = pL[(int64_t)s_first * n_heads + h];
+    const int mine = 64 * wave + lane;
+    float pm_first, pl_first;
     float4 v[8];
     float mm[8];
+    // what this wave's lanes and slots read of splits from .. from + 63, clamped to the first n
+    auto fetch_first = [&](int n) {
+        const int sI = min(mine, n - 1);
+        pm_first = pM[(int64_t)sI * n_heads + h];
+        pl_first = pL[(int64_t)sI * n_heads + h];
+    };
+    auto fetch = [&](int from, int n) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const int sc = min(slot + 8 * u, ns_max - 1);
-        v[u] = pO4[((int64_t)sc * n_heads + h) * NOUT + o_idx];
-        mm[u] = pM[(int64_t)sc * n_heads + h];
+        for (int u = 0; u < 8; ++u) {
+            const int sc = min(from + slot + 8 * u, n - 1);
+            v[u] = pO4[((int64_t)sc * n_heads + h) * NOUT + o_idx];
+            mm[u] = pM[(int64_t)sc * n_heads + h];
+        }
+    };
+    if (WAVES == 1 || wave == 0) {
+        fetch_first(ns_max);
+        fetch(0, ns_max);
     }
     int64_t total = past + 1;
     if (total > max_seq) total = max_seq;
@@ -359,23 +374,28 @@ __global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __r
     const int n_chunks = (int)((total + chunk - 1) >> cs_);
     const int cpw_ = long_mode ? (n_chunks + (int)FD_LONG_SPLITS - 1) / (int)FD_LONG_SPLITS : 1;
     const int ns = long_mode ? (n_chunks + cpw_ - 1) / cpw_ : n_chunks;
-    float m = lane < ns ? pm_first : -INFINITY;
-    for (int sI = lane + 64; sI < ns; sI += 64) m = fmaxf(m, pM[(int64_t)sI * n_heads + h]);
-    const float M = max64(m);
-    float den = lane < ns ? wexp(pm_first - M) * pl_first : 0.0f;
-    for (int sI = lane + 64; sI < ns; sI += 64)
+    const bool together = WAVES > 1 && ns > 64;  // the same in every thread
+    if (!together && wave > 0) return;
+    if (wave > 0) fetch_first(ns);
+    __shared__ float s_m[WAVES], s_den[WAVES];
+    __shared__ float4 s_sum[WAVES][8];
+    float m = mine < ns ? pm_first : -INFINITY;
+    for (int sI = mine + 64 * WAVES; sI < ns; sI += 64 * WAVES) m = fmaxf(m, pM[(int64_t)sI * n_heads + h]);
+    float M = max64(m);
+    if (together) {
+        if (lane == 0) s_m[wave] = M;
+        __syncthreads();
+        M = s_m[0];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) M = fmaxf(M, s_m[w]);
+    }
+    float den = mine < ns ? wexp(pm_first - M) * pl_first : 0.0f;
+    for (int sI = mine + 64 * WAVES; sI < ns; sI += 64 * WAVES)
         den = fmaf(wexp(pM[(int64_t)sI * n_heads + h] - M), pL[(int64_t)sI * n_heads + h], den);
     den = sum64(den);
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < ns; s0 += 64) {
-        if (s0 > 0) {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int sc = min(s0 + slot + 8 * u, ns - 1);
-                v[u] = pO4[((int64_t)sc * n_heads + h) * NOUT + o_idx];
-                mm[u] = pM[(int64_t)sc * n_heads + h];
-            }
-        }
+    for (int s0 = 64 * wave; s0 < ns; s0 += 64 * WAVES) {
+        if (s0 > 0) fetch(s0, ns);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const bool on = s0 + slot + 8 * u < ns;  // a select, not a zero weight: inactive slots may hold anything
@@ -393,8 +413,20 @@ __global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __r
         r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
         return __uint_as_float(r[0]) + __uint_as_float(r[1]);
     };
+    sum = make_float4(slots(sum.x), slots(sum.y), slots(sum.z), slots(sum.w));
+    if (together) {
+        if (lane < 8) s_sum[wave][lane] = sum;
+        if (lane == 0) s_den[wave] = den;
+        __syncthreads();
+        if (wave > 0) return;
+        for (int w = 1; w < WAVES; ++w) {
+            const float4 t = s_sum[w][lane & 7];
+            sum.x += t.x; sum.y += t.y; sum.z += t.z; sum.w += t.w;
+            den += s_den[w];
+        }
+    }
     const float inv = 1.0f / (den + 1e-10f);  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
-    const float4 o4 = make_float4(slots(sum.x) * inv, slots(sum.y) * inv, slots(sum.z) * inv, slots(sum.w) * inv);
+    const float4 o4 = make_float4(sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv);
     if (lane < 8) reinterpret_cast<float4*>(O)[(int64_t)h * NOUT + o_idx] = o4;
     if (q8_out) {
         // the same vector as Q8 blocks (int8 qs[K] | float d[K/32] | float sum[K/32], K = n_heads * HD) for a Q4_K
@@ -412,16 +444,25 @@ __global__ __launch_bounds__(64) void flash_decode_merge_kernel(const float* __r
     }
 }
 
+template <int HD, int WAVES>
+static void fd_merge_launch(int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O, const int64_t* d_past,
+                            int64_t past_host, int max_seq, uint8_t* q8_out, int chunk_shift, int log2_units) {
+    hipLaunchKernelGGL((flash_decode_merge_kernel<HD, WAVES>), dim3(n_heads, HD / 32), dim3(64 * WAVES), 0, s, pO, pL, pM, O, n_heads, d_past,
+                       past_host, max_seq, q8_out, chunk_shift, log2_units);
+}
+
 static int fd_merge(int head_dim, int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O,
                     const int64_t* d_past, int max_seq, uint8_t* q8_out = nullptr, int64_t past_host = 0,
                     int chunk = FD_CHUNK, int log2_units = 0) {
     const int chunk_shift = chunk < 0 ? -1 : chunk == 128 ? 7 : 6;
-    if (head_dim == 256)
-        hipLaunchKernelGGL(flash_decode_merge_kernel<256>, dim3(n_heads, 8), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
-    else if (head_dim == 128)
-        hipLaunchKernelGGL(flash_decode_merge_kernel<128>, dim3(n_heads, 4), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
-    else
-        hipLaunchKernelGGL(flash_decode_merge_kernel<64>, dim3(n_heads, 2), dim3(64), 0, s, pO, pL, pM, O, n_heads, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units);
+    const int most = chunk_shift < 0 ? (int)FD_LONG_SPLITS : (int)(((int64_t)max_seq + chunk - 1) >> chunk_shift);  // splits there can be
+#define PTM_FDM(HDV, WV) fd_merge_launch<HDV, WV>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units)
+#define PTM_FDMW(HDV) (most <= 64 ? PTM_FDM(HDV, 1) : PTM_FDM(HDV, 4))
+    if (head_dim == 256) PTM_FDMW(256);
+    else if (head_dim == 128) PTM_FDMW(128);
+    else PTM_FDMW(64);
+#undef PTM_FDMW
+#undef PTM_FDM
     return launch_status();
 }
 

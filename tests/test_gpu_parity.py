@@ -563,6 +563,35 @@ def test_flash_decode_merges_any_number_of_splits(dev, po, nh, nkv, hd, T):
     test_flash_decode_vs_oracle(dev, po, True, nh, nkv, hd, T)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,T", [(4, 1, 64, 16384), (4, 1, 64, 16385), (2, 1, 128, 20000), (2, 2, 256, 8192)])
+def test_flash_decode_merges_of_several_waves(dev, po, nh, nkv, hd, T):
+    """More than 64 splits are shared by four waves, 64 each: 256 of them are one turn, 257 take a second."""
+    test_flash_decode_vs_oracle(dev, po, True, nh, nkv, hd, T)
+
+
+@pytest.mark.parametrize("T", [1, 100, 4096, 4097, 4160])
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 64), (4, 4, 128), (2, 1, 256)])
+def test_flash_decode_early_in_a_long_cache(dev, nh, nkv, hd, T):
+    """A long cache changes nothing in the result of the positions in use, to the bit: up to 64 splits one wave merges, beyond four whatever
+    the cache could hold; what lies behind the position is never used."""
+    r = synth.rng_for(48, nh, hd, T)
+    q, outs = cu(synth.make_x(r, nh * hd)), []
+    k, v = (cu(r.standard_normal((T, nkv * hd), dtype=np.float32).astype(np.float16)) for _ in "kv")
+    past = torch.tensor([T - 1], dtype=torch.int64, device="cuda")
+    for max_seq in (T, 20000, 70000):
+        K, V = (torch.full((max_seq, nkv * hd), float("nan"), dtype=torch.float16, device="cuda") for _ in "kv")
+        K[:T], V[:T] = k, v
+        S = ops.flash_decode_num_splits(max_seq)
+        pO, pL, pM = (torch.full((S * nh * n,), float("nan"), device="cuda") for n in (hd, 1, 1))
+        O, q8 = torch.empty(nh * hd, device="cuda"), torch.zeros(ops.q8_bytes(nh * hd), dtype=torch.uint8, device="cuda")
+        ops.flash_decode_window(q, K, V, O, pO, pL, pM, nh, nkv, hd, past, max_seq, hd ** -0.5, o_q8=q8)
+        torch.cuda.synchronize()
+        outs.append((bits(O.cpu().numpy()), q8.cpu().numpy()))
+    assert np.isfinite(O.cpu().numpy()).all()
+    for o, q8 in outs[1:]:
+        assert np.array_equal(o, outs[0][0]) and np.array_equal(q8, outs[0][1])
+
+
 def test_elementwise_embedding_argmax(dev, po):
     r = synth.rng_for(45)
     g = (synth.make_x(r, 9728) * 30).astype(np.float32)
