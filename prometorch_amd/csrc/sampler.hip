@@ -40,7 +40,8 @@ enum {
     SW_CLEAR_WORDS = SW_COUNT + 8
 };
 // The short path: a slice of the vocabulary per workgroup, at most LOCAL_SLICES, and at most LOCAL_SLOTS candidates of each:
-// how many, the largest key that one left out may have (0: none left out), the largest key of each quarter, (key, index) pairs
+// how many, the key of those that were left out for being too many of one (0: none), the largest key of each quarter, (key, index)
+// pairs; the last pair's place holds how many were left out
 enum { LOCAL_MAX_TOPK = 64, LOCAL_SLICES = 128, LOCAL_SLOTS = 128, LOCAL_HEAD = 6, LOCAL_WORDS = LOCAL_HEAD + 2 * LOCAL_SLOTS, SW_WORDS = SW_LOCAL + LOCAL_SLICES * LOCAL_WORDS };
 // wide-path scalars (32-bit words from SW_WIDE): top-k threshold key, largest kept key, sum of exp (64-bit, 2^-32 units),
 // probability mass above the current prefix (64-bit, 2^-40 units), key prefix chosen so far, 1 when every eligible token stays
@@ -233,7 +234,7 @@ __device__ __forceinline__ float running_sums(float v, int n, float& total) {
 struct SamplerLds {
     unsigned long long sort[SAMPLER_MAX_CAND];   // 16 KB
     float p[SAMPLER_MAX_CAND];                   // x, then p, in index order
-    uint32_t idx[SAMPLER_MAX_CAND];
+    __align__(16) uint32_t idx[SAMPLER_MAX_CAND];
     uint8_t keep[SAMPLER_MAX_CAND];
 };
 
@@ -794,16 +795,16 @@ __global__ __launch_bounds__(1024) void sampler_finish_kernel(SamplerArgs a, Sam
 
 // ---- the short path: top-k up to LOCAL_MAX_TOPK ------------------------------------------------------------------------
 // Two launches and one read of the logits instead of seven launches and four reads: a call is a chain of launches and latencies (151 936
-// logits, top-k 40: 34.2 us with histograms, 12.9 so; both read 1.2 MB, under a microsecond).  Beyond 64 candidates per slice the second
+// logits, top-k 40: 34.6 us with histograms, 12.6 so; both read 1.2 MB, under a microsecond).  Beyond 64 candidates per slice the second
 // launch, a single workgroup, would read more than it saves.  What is at or above the k-th largest of the vocabulary is at
 // or above the k-th largest of its slice, so a workgroup leaves only those of its slice, and one workgroup selects among them.
 //
-// The largest T, as far as bits 31 .. low go, with at least k of the wave's R values per lane at or above it (0: fewer than k above 0).
+// The largest T = t + bits `bit` .. low with at least k of the wave's R values per lane at or above it (bits above are in t already; t if there
+// are fewer than k above it).
 template <int R>
-__device__ __forceinline__ uint32_t kth_of_wave(const uint32_t (&v)[R], int k, int low) {
-    uint32_t t = 0;
+__device__ __forceinline__ uint32_t kth_of_wave(const uint32_t (&v)[R], int k, int bit, int low, uint32_t t) {
 #pragma unroll 1
-    for (int bit = 31; bit >= low; --bit) {
+    for (; bit >= low; --bit) {
         const uint32_t with = t | 1u << bit;
         int n = 0;
 #pragma unroll
@@ -812,14 +813,12 @@ __device__ __forceinline__ uint32_t kth_of_wave(const uint32_t (&v)[R], int k, i
     }
     return t;
 }
-// The largest T, as far as its upper 16 bits go, with at least k of the workgroup's E keys per thread at or above it (0 if there are
-// fewer than k; keys left out are zeros): two bits at a time, from the top.  s_cnt: zeros.
+// The same of the workgroup's E keys per thread (keys left out are zeros), two bits at a time.  s_cnt: zeros.
 template <int E>
-__device__ __forceinline__ uint32_t kth_key_bits(const uint32_t (&key)[E], int k, uint32_t (&s_cnt)[8][4]) {
+__device__ __forceinline__ uint32_t kth_key_bits(const uint32_t (&key)[E], int k, uint32_t t, int bit, int low, uint32_t (*s_cnt)[4]) {
     const int lane = threadIdx.x & 63;
-    uint32_t t = 0;
 #pragma unroll 1
-    for (int bit = 30, i = 0; bit >= 16; bit -= 2, ++i) {
+    for (int i = 0; bit >= low; bit -= 2, ++i) {
         uint32_t n[3] = {0, 0, 0};
 #pragma unroll
         for (int j = 0; j < 3; ++j)
@@ -833,17 +832,20 @@ __device__ __forceinline__ uint32_t kth_key_bits(const uint32_t (&key)[E], int k
     return t;
 }
 
-// grid: slices of 1024 E values.  Listed is what reaches the k-th largest of the maxima of four lanes, in its upper 16 bits: k values
-// and a tenth or so, found by one wave.  (Exactly, by all of them, takes eight barriers: 2.7 us against 1.)  Should they not fit, the
-// threshold is made exact, and should ties in its 16 bits still not fit, the list holds what is above them, and says so.
+// grid: slices of 1024 E values.  Greedy: the largest value's first index.  Else listed is what reaches the k-th largest of the maxima of
+// four lanes, in its upper 16 bits: k values and a tenth or so, found by one wave.  (Exactly, by all of them, takes eight barriers: 2.7 us
+// against 1.)  Should they not fit, the threshold is made exact, in 16 bits and then in all; should ties at it still not fit, the
+// list holds what is above them, and says how many there are.
 template <int E>
 __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
-    __shared__ uint32_t s_cnt[8][4];
-    __shared__ uint32_t s_max[256], s_bound, s_n[3];
+    __shared__ uint32_t s_cnt[16][4];
+    __shared__ uint32_t s_max[256], s_bound, s_first, s_n[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, base = blockIdx.x * 1024 * E;
-    if (tid < 32) s_cnt[tid >> 2][tid & 3] = 0;
-    if (tid < 3) s_n[tid] = 0;
+    if (tid < 64) s_cnt[tid >> 2][tid & 3] = 0;
+    if (tid < 4) s_n[tid] = 0;
+    if (tid == 0) s_first = 0xffffffffu;
     const ptm_sampling p = sampler_params(a);
+    const bool greedy = !(p.temperature >= 1e-6f);
     uint32_t key[E], best = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -858,7 +860,14 @@ __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
     uint32_t* seg = a.ws + SW_LOCAL + blockIdx.x * LOCAL_WORDS;
     if (wave == 0) {
         const uint32_t v[4] = {s_max[lane], s_max[lane + 64], s_max[lane + 128], s_max[lane + 192]};
-        const uint32_t t = kth_of_wave(v, sampler_k(p), 16);
+        uint32_t t;
+        if (greedy) {
+            t = max(max(v[0], v[1]), max(v[2], v[3]));
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) t = max(t, (uint32_t)__shfl_xor(t, off, 64));
+        } else {
+            t = kth_of_wave(v, sampler_k(p), 31, 16, 0u);
+        }
         if (lane == 0) s_bound = t;
     } else if (wave <= 4) {  // the quarters' maxima
         uint32_t m = s_max[64 * (wave - 1) + lane];
@@ -867,6 +876,20 @@ __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
         if (lane == 0) seg[1 + wave] = m;
     }
     __syncthreads();
+    if (greedy) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const unsigned long long who = __ballot(base + tid + 1024 * e < a.vocab && key[e] == s_bound);
+            if (who && lane == 0) atomicMin(&s_first, (uint32_t)(base + 1024 * e + 64 * wave) + (uint32_t)__builtin_ctzll(who));
+        }
+        __syncthreads();
+        if (tid == 0) {
+            reinterpret_cast<uint2*>(seg + LOCAL_HEAD)[0] = make_uint2(s_bound, s_first);
+            seg[0] = 1;
+            seg[1] = 0;
+        }
+        return;
+    }
     auto list = [&](uint32_t* count, uint32_t from) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -879,65 +902,69 @@ __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
         __syncthreads();
         return *count;
     };
-    uint32_t n = list(&s_n[0], s_bound), left_out = 0;
+    uint32_t n = list(&s_n[0], s_bound), left_out = 0, ties = 0;
     if (n > LOCAL_SLOTS) {
-        const uint32_t thr = kth_key_bits(key, sampler_k(p), s_cnt);
-        n = list(&s_n[1], thr);
-        if (n > LOCAL_SLOTS) {  // (fewer than k <= 64 are above the whole of thr's 16 bits)
-            left_out = thr | 0xffffu;
-            n = left_out != 0xffffffffu ? list(&s_n[2], left_out + 1) : 0;
+        const int k = sampler_k(p);
+        const uint32_t upper = kth_key_bits(key, k, 0u, 30, 16, s_cnt);
+        n = list(&s_n[1], upper);
+        if (n > LOCAL_SLOTS) {
+            const uint32_t thr = kth_key_bits(key, k, upper, 14, 0, s_cnt + 8), all = list(&s_n[2], thr);
+            n = all;
+            if (all > LOCAL_SLOTS) {  // fewer than k <= 64 are above them
+                left_out = thr;
+                n = thr != 0xffffffffu ? list(&s_n[3], thr + 1) : 0;
+                ties = all - n;
+            }
         }
     }
-    if (tid == 0) { seg[0] = n; seg[1] = left_out; }
+    if (tid == 0) {
+        seg[0] = n;
+        seg[1] = left_out;
+        if (left_out) seg[LOCAL_WORDS - 1] = ties;
+    }
 }
 
 // One workgroup: the candidates of all slices in registers.  A lower bound of the k-th largest is the k-th largest of the quarters'
-// maxima (one wave finds it), which leaves about k of some thousands; of those, the ones with fewer
-// than k greater ones.
-__global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs a, SamplerOut o, int slices) {
+// maxima (one wave finds it), which leaves about k of some thousands; of those, the ones with fewer than k greater ones.  For more than 256
+// of them the k-th largest is found exactly, two bits at a time by all waves (6 us).  151936 logits, top-k 40 / 64: normal 12.6 / 16.4 us,
+// evenly from 0 to 1 23.8 / 25.2, ten above a mask of -inf 543 both (more ties than a list holds: sampler_overflow_body); with
+// histograms 34.6 / 40.3, 32.6 / 38.8, 595.  Ties that a slice left out are more than k of a key, so that none of them and nothing
+// listed below them is kept unless they are the k-th largest themselves; then they are read from their slices.
+__global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs a, SamplerOut o, int slices, int per) {
     __shared__ SamplerLds l;
-    __shared__ uint32_t s_n[3];   // candidates at or above the bound, largest key left out, kept
+    __shared__ uint32_t s_n[4];   // candidates at or above the bound, largest key left out, kept, of them above that key
     __shared__ uint32_t s_bound;
     constexpr int SEGS = LOCAL_SLICES / 16, MAXIMA = LOCAL_SLICES * 4 / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t* const seg0 = a.ws + SW_LOCAL;
-    uint2 head[SEGS], cand[2][SEGS];
+    uint2 head = make_uint2(0, 0), cand[2][SEGS];  // lane g: the head of the wave's slice g
+    if (lane < SEGS && wave + 16 * lane < slices) head = *reinterpret_cast<const uint2*>(seg0 + (wave + 16 * lane) * LOCAL_WORDS);
 #pragma unroll
     for (int g = 0; g < SEGS; ++g) {  // slots are fetched filled or not: one round trip, unless a slice has more than 64
-        head[g] = cand[0][g] = make_uint2(0, 0);
-        if (wave + 16 * g < slices) {
-            const uint32_t* seg = seg0 + (wave + 16 * g) * LOCAL_WORDS;
-            head[g] = *reinterpret_cast<const uint2*>(seg);
-            cand[0][g] = reinterpret_cast<const uint2*>(seg + LOCAL_HEAD)[lane];
-        }
+        cand[0][g] = make_uint2(0, 0);
+        if (wave + 16 * g < slices) cand[0][g] = reinterpret_cast<const uint2*>(seg0 + (wave + 16 * g) * LOCAL_WORDS + LOCAL_HEAD)[lane];
     }
-    if (tid < 3) s_n[tid] = 0;
+    if (tid < 4) s_n[tid] = 0;
     const ptm_sampling p = sampler_params(a);
     const int step = o.d_step ? *o.d_step : 0, k = sampler_k(p);
     const int64_t past_now = o.adv.d_past ? *o.adv.d_past : 0;
     const float r_draw = o.uniforms[step];
+    uint32_t v[MAXIMA], bound = 0;
     if (wave == 0) {
-        uint32_t v[MAXIMA];
 #pragma unroll
         for (int t = 0; t < MAXIMA; ++t) v[t] = lane / 4 + 16 * t < slices ? seg0[(lane / 4 + 16 * t) * LOCAL_WORDS + 2 + lane % 4] : 0u;
-        const uint32_t t = kth_of_wave(v, k, 14);
-        if (lane == 0) s_bound = t;
+        bound = kth_of_wave(v, k, 31, 14, 0u);
+        if (lane == 0) s_bound = bound;
     }
     __syncthreads();
-    const uint32_t bound = s_bound;
-    uint32_t most = 0, left_out = 0;
-#pragma unroll
-    for (int g = 0; g < SEGS; ++g) {
-        most = max(most, head[g].x);
-        left_out = max(left_out, head[g].y);
-    }
-    if (lane == 0 && left_out) atomicMax(&s_n[1], left_out);
-    auto list = [&](int h) {  // one reservation per wave
+    const bool many = __ballot(head.x > 64u) != 0;
+    if (__ballot(head.y != 0u)) atomicMax(&s_n[1], head.y);
+    auto list = [&](int h, uint32_t from) {  // one reservation per wave
         bool in[SEGS];
         uint32_t count = 0;
 #pragma unroll
         for (int g = 0; g < SEGS; ++g) {
-            in[g] = (uint32_t)(lane + 64 * h) < head[g].x && cand[h][g].x >= bound;
+            in[g] = (uint32_t)(lane + 64 * h) < lane_u(head.x, g) && cand[h][g].x >= from;
             count += (uint32_t)__popcll(__ballot(in[g]));
         }
         if (count == 0) return;
@@ -952,16 +979,17 @@ __global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs 
             slot += (uint32_t)__popcll(who);
         }
     };
-    list(0);
-    if (most > 64) {
+    bound = s_bound;
+    list(0, bound);
+    if (many) {
 #pragma unroll
         for (int g = 0; g < SEGS; ++g) cand[1][g] = wave + 16 * g < slices ? reinterpret_cast<const uint2*>(seg0 + (wave + 16 * g) * LOCAL_WORDS + LOCAL_HEAD)[lane + 64] : make_uint2(0, 0);
-        list(1);
+        list(1, bound);
     }
     __syncthreads();
-    const int n = (int)s_n[0];
-    left_out = s_n[1];
-    if (n <= 64 && left_out == 0u) {
+    int n = (int)s_n[0];
+    const uint32_t left_out = s_n[1];
+    if (n <= 64 && (left_out == 0u || left_out < bound)) {
         if (tid >= 64) return;
         const uint32_t key = lane < n ? (uint32_t)l.sort[lane] : 0u, idx = lane < n ? (uint32_t)(l.sort[lane] >> 32) : 0u;
         int greater = 0;
@@ -979,63 +1007,78 @@ __global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs 
         if (tid == 0) sampler_publish(o, token, step, past_now);
         return;
     }
-    // Few slices, ties at the threshold, or a slice's list that was too short.  What was left out does not matter where k candidates are above it.
-    uint32_t thr = 0;
-    bool listed = n <= SAMPLER_MAX_CAND;
-    if (listed) {
-        unsigned long long c[2];
-        bool keep[2];
-        int above = 0;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int i = tid + 1024 * q;
-            c[q] = l.sort[max(0, min(i, n - 1))];
-            int greater = 0;
-            for (int j = 0; j < n; ++j) greater += (uint32_t)l.sort[j] > (uint32_t)c[q];
-            keep[q] = i < n && greater < k;
-            above += i < n && (uint32_t)c[q] > left_out;
-        }
+    if (n > SAMPLER_MAX_CAND) {  // the bound's lower bits
+        __syncthreads();  // s_n and s_bound have been read
+        if (wave == 0) bound = kth_of_wave(v, k, 13, 0, bound);
+        if (tid == 0) { s_bound = bound; s_n[0] = 0; }
         __syncthreads();
+        bound = s_bound;
+        list(0, bound);
+        if (many) list(1, bound);
+        __syncthreads();
+        n = (int)s_n[0];
+    }
+    uint32_t (*const cnt)[4] = reinterpret_cast<uint32_t (*)[4]>(l.p);
+    if (n > 256) {
+        __syncthreads();
+        if (tid < 64) cnt[tid >> 2][tid & 3] = 0;
         if (tid == 0) s_n[0] = 0;
         __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            if (keep[q]) l.sort[atomicAdd(&s_n[2], 1u)] = c[q];
-        if (above) atomicAdd(&s_n[0], (uint32_t)above);
-        __syncthreads();
-        listed = left_out == 0u || s_n[0] >= (uint32_t)k;
     }
-    if (!listed) {  // the vocabulary once more: its k-th largest key, three levels of bins walked from the top
-        uint32_t* hist = reinterpret_cast<uint32_t*>(l.sort);
-        int want = k;
-        for (int level = 0; level < 3; ++level) {
-            const int nb = level == 2 ? 1024 : 2048;
-            __syncthreads();
-            for (int i = tid; i < nb; i += 1024) hist[i] = 0;
-            __syncthreads();
-            for (int i = tid; i < a.vocab; i += 1024) {
-                const uint32_t key = order_key(sampler_value(a, p, i));
-                if (level == 0) atomicAdd(&hist[key >> 21], 1u);
-                else if (level == 1) { if (key >> 21 == thr) atomicAdd(&hist[key >> 10 & 0x7ffu], 1u); }
-                else if (key >> 10 == thr) atomicAdd(&hist[key & 0x3ffu], 1u);
-            }
-            __syncthreads();
-            int b = nb - 1;
-            while (b > 0 && hist[b] < (uint32_t)want) want -= (int)hist[b--];   // every thread the same walk
-            thr = level == 0 ? (uint32_t)b : thr << (level == 1 ? 11 : 10) | (uint32_t)b;
+    uint32_t thr = left_out;
+    bool exact = false;
+    if (n > SAMPLER_MAX_CAND) {  // thousands: the k-th largest of what the registers hold (35 us)
+        uint32_t key[2 * SEGS];
+#pragma unroll
+        for (int q = 0; q < 2 * SEGS; ++q) key[q] = (q < SEGS || many) && (uint32_t)(lane + 64 * (q / SEGS)) < lane_u(head.x, q % SEGS) ? cand[q / SEGS][q % SEGS].x : 0u;
+        thr = max(thr, kth_key_bits(key, k, 0u, 30, 0, cnt));
+        exact = true;
+        list(0, thr);
+        if (many) list(1, thr);
+        __syncthreads();
+        n = (int)s_n[0];
+        if (n > SAMPLER_MAX_CAND) return sampler_overflow_body(a, o, thr, l.sort);
+    }
+    unsigned long long c[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) c[q] = tid + 1024 * q < n ? l.sort[tid + 1024 * q] : 0ull;
+    uint32_t* const keys = l.idx;
+    if (n <= 256) {  // each against all, four keys a read
+        if (tid < 260) keys[tid] = (uint32_t)c[0];
+        __syncthreads();
+        int greater = 0;
+#pragma unroll 4
+        for (int j = 0; j < n; j += 4) {
+            const uint4 x = *reinterpret_cast<const uint4*>(keys + j);
+            greater += (x.x > (uint32_t)c[0]) + (x.y > (uint32_t)c[0]) + (x.z > (uint32_t)c[0]) + (x.w > (uint32_t)c[0]);
+        }
+        if (tid < n && greater >= k) c[0] = 0;
+    } else if (!exact) {
+        const uint32_t key[2] = {(uint32_t)c[0], (uint32_t)c[1]};
+        thr = max(thr, kth_key_bits(key, k, 0u, 30, 0, cnt));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if ((uint32_t)c[q] >= thr && (uint32_t)c[q] > 0u) {
+            l.sort[atomicAdd(&s_n[2], 1u)] = c[q];
+            if ((uint32_t)c[q] > left_out) atomicAdd(&s_n[3], 1u);
+        }
+    __syncthreads();
+    if (left_out && s_n[3] < (uint32_t)k) {  // the left-out ties are the k-th largest
+        const bool again = head.y == left_out;  // (0 in lanes without a slice)
+        if (lane < SEGS) l.keep[wave + 16 * lane] = again;
+        __syncthreads();  // s_n[3] has been read
+        if (again) atomicAdd(&s_n[3], seg0[(wave + 16 * lane + 1) * LOCAL_WORDS - 1] << 8);  // (fewer than 2^18; what it was is below k <= 64)
+        __syncthreads();
+        if (s_n[2] + (s_n[3] >> 8) > SAMPLER_MAX_CAND) return sampler_overflow_body(a, o, left_out, l.sort);
+        __syncthreads();
+        for (int s = 0; s < slices; ++s) {
+            if (!l.keep[s]) continue;
+            for (int i = s * per + tid; i < min(a.vocab, (s + 1) * per); i += 1024)
+                if (order_key(sampler_value(a, p, i)) == left_out) l.sort[min(atomicAdd(&s_n[2], 1u), (uint32_t)SAMPLER_MAX_CAND - 1)] = ((unsigned long long)(uint32_t)i << 32) | left_out;
         }
         __syncthreads();
-        if (tid == 0) s_n[2] = 0;
-        __syncthreads();
-        for (int i = tid; i < a.vocab; i += 1024) {
-            const uint32_t key = order_key(sampler_value(a, p, i));
-            if (key >= thr) {
-                const uint32_t slot = atomicAdd(&s_n[2], 1u);
-                if (slot < SAMPLER_MAX_CAND) l.sort[slot] = ((unsigned long long)(uint32_t)i << 32) | key;
-            }
-        }
-        __syncthreads();
-        if (s_n[2] > SAMPLER_MAX_CAND) return sampler_overflow_body(a, o, thr, l.sort);
     }
     const int m = (int)s_n[2];
     if (m <= 64) {
@@ -1090,7 +1133,7 @@ int sampler_enqueue(const float* logits, int vocab, const int32_t* counts, const
         const int per = vocab <= LOCAL_SLICES * 1024 ? 1024 : 2048, slices = (vocab + per - 1) / per;
         if (per == 1024) hipLaunchKernelGGL(sampler_local_kernel<1>, dim3(slices), dim3(1024), 0, s, a);
         else hipLaunchKernelGGL(sampler_local_kernel<2>, dim3(slices), dim3(1024), 0, s, a);
-        hipLaunchKernelGGL(sampler_local_finish_kernel, dim3(1), dim3(1024), 0, s, a, o, slices);
+        hipLaunchKernelGGL(sampler_local_finish_kernel, dim3(1), dim3(1024), 0, s, a, o, slices, per);
         return launch_status();
     }
     if (!ws_kept_clean) hipLaunchKernelGGL(sampler_clear_kernel, dim3(4), dim3(256), 0, s, a.ws);

@@ -376,3 +376,56 @@ def test_candidates_by_slices(dev, po, vocab, top_k, kind):
             checked += 1
     assert checked >= 4
     assert gpu_sample(x, 0.0, 1, 1.0, 0.5) == int(np.argmax(x))
+
+
+def _close_logits(kind, vocab, g):
+    x = (2 * g.standard_normal(vocab, dtype=np.float32)).astype(np.float32)
+    if kind == "constant":
+        x[:] = 1.25
+    elif kind == "few above a mask":      # fewer than k values, the rest ties at -inf: all of them are kept, most with probability 0
+        keep = g.integers(0, vocab, 9)
+        y = np.full(vocab, -np.inf, np.float32)
+        y[keep] = x[keep]
+        x = y
+    elif kind == "offset":                # a slice's values share their upper 16 bits
+        x = (x + np.float32(1000.0)).astype(np.float32)
+    elif kind == "ramp":
+        x = np.linspace(0, 1, vocab, dtype=np.float32)
+    elif kind == "ties left out":         # some slices with more ties at the k-th largest than their lists hold, others with a few, at edges
+        x = np.minimum(x, np.float32(2.5))
+        x[x == np.float32(2.5)] = 2.0
+        for lo in (0, vocab // 2 - 150, vocab - 140):
+            x[lo:lo + 140] = 3.0
+        x[[5, vocab // 3, vocab - 7]] = 4.0
+    elif kind == "ties below":            # such ties below the k-th largest do not matter
+        x[:300] = 5.0
+        x[vocab // 2:vocab // 2 + 80] = 6.0 + 0.1 * g.random(80, dtype=np.float32)
+    elif kind.startswith("ties listed"):  # forty equal values in each of up to 128 slices, as the k-th largest or below it
+        x = np.minimum(x, np.float32(6.0))
+        x[::25] = 7.0
+        if kind.endswith("below"):
+            x[300:370] = 8.0 + 0.1 * g.random(70, dtype=np.float32)
+    elif kind == "ties at the top":       # as many as k and one more
+        x[g.permutation(vocab)[:65]] = 9.0
+    return x
+
+
+@pytest.mark.parametrize("vocab,top_k", [(1000, 64), (1000, 1), (4096, 64), (32000, 40), (131073, 64), (151936, 40), (262144, 20)])
+@pytest.mark.parametrize("kind", ["constant", "few above a mask", "offset", "ramp", "ties left out", "ties below", "ties listed", "ties listed below", "ties at the top"])
+def test_close_values_and_ties_by_slices(dev, po, vocab, top_k, kind):
+    """What a slice's list cannot hold: equal values, values that differ in their last bits only, and both above or below the top k."""
+    x = _close_logits(kind, vocab, synth.rng_for(93, vocab, top_k))
+    tied = int((x >= np.sort(x)[-min(top_k, vocab)]).sum())
+    checked = 0
+    for r in (0.0031, 0.21371, 0.52193, 0.70937, 0.90173, 0.99731):
+        tok_o, gap, probs = po.sample_token(x, 0.8, top_k, 0.95, r, want_probs=True)
+        tok_g = gpu_sample(x, 0.8, top_k, 0.95, r)
+        if tied > 2048:
+            # the reference adds equal terms one by one, twice (to renormalise and to draw): 2^-25 of the sum off each time, all the same way
+            check_wide_draw(tok_g, tok_o, gap, probs, r, max(GAP_TOL, tied * 2.0 ** -24), vocab)
+            checked += 1
+        elif gap > GAP_TOL:
+            assert tok_g == tok_o, (r, gap)
+            checked += 1
+    assert checked >= 4
+    assert gpu_sample(x, 0.0, 1, 1.0, 0.5) == int(np.argmax(x))
