@@ -205,13 +205,13 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const DenseGemm g) {
 
 // The same product on the tiles of gemm_tile.h, which take rows of both sides from memory to LDS directly.  A launch covers its output
 // with up to four regions of equal tiles.
-typedef GemmTile<gt_b8, 8, 4, 2, 2, 2> Tile0;
-typedef GemmTile<gt_b8, 4, 6, 4, 2, 2> Tile1;
-typedef GemmTile<gt_b8, 4, 4, 2, 2, 3> Tile2;
-typedef GemmTile<gt_b8, 2, 6, 4, 3, 3> Tile3;
-typedef GemmTile<gt_b8, 2, 4, 4, 3, 3> Tile4;
-typedef GemmTile<gt_b8, 2, 4, 2, 3, 3> Tile5;
-typedef GemmTile<gt_b8, 2, 2, 2, 3, 3> Tile6;
+typedef GemmTile<8, 4, 2, 2, 2> Tile0;
+typedef GemmTile<4, 6, 4, 2, 2> Tile1;
+typedef GemmTile<4, 4, 2, 2, 3> Tile2;
+typedef GemmTile<2, 6, 4, 3, 3> Tile3;
+typedef GemmTile<2, 4, 4, 3, 3> Tile4;
+typedef GemmTile<2, 4, 2, 3, 3> Tile5;
+typedef GemmTile<2, 2, 2, 3, 3> Tile6;
 
 template <typename Tile>
 __device__ __forceinline__ void dense_tile(const DenseGemm& g, const GemmRegion& r, int wg, uint8_t* lds) {

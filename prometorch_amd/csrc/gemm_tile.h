@@ -1,4 +1,4 @@
-// The main loop of the prompt products: one workgroup of eight waves, BM rows of X times BN rows of W, 64 values of K per step, fp16 or
+// The main loop of the prompt products: one workgroup of eight waves, BM rows of X times BN rows of W, 64 values of K per step,
 // bfloat16 operands, fp32 sums on v_mfma_f32_16x16x32.
 //
 // LDS holds two or three steps of either side.  A row of a step is 128 bytes, its eight 16-byte pieces stored at piece ^ (row % 8), so the
@@ -19,11 +19,8 @@ namespace ptm {
 
 typedef float gt_f4 __attribute__((ext_vector_type(4)));
 typedef int gt_i4 __attribute__((ext_vector_type(4)));
-typedef _Float16 gt_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 gt_b8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ gt_f4 gt_mfma(gt_h8 a, gt_h8 b, gt_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ gt_f4 gt_mfma(gt_b8 a, gt_b8 b, gt_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // 16 bytes per lane from base + voff + soff to LDS bytes [lds, lds + 1024), lane after lane
 __device__ __forceinline__ void gt_to_lds(uint32_t lds, int voff, gt_i4 base, int soff) {
@@ -42,7 +39,7 @@ __device__ __forceinline__ void gt_arrived() { asm volatile("s_waitcnt vmcnt(%0)
 __device__ __forceinline__ int gt_column(int r) { return (r & ~31) + ((r & 12) << 1) + ((r & 16) >> 2) + (r & 3); }
 
 // RX, RW: 16-row fragments of X and W of a wave; WX waves along the rows of X, 8 / WX along those of W; XN, WN: steps of X and W in LDS
-template <typename F8, int RX, int RW, int WX, int XN, int WN>
+template <int RX, int RW, int WX, int XN, int WN>
 struct GemmTile {
     static_assert((16 * RX * WX) % 64 == 0 && (16 * RW * (8 / WX)) % 64 == 0 && RX % 2 == 0 && RW % 2 == 0, "whole fetch instructions, halves of X, pairs of sums");
     static_assert(XN <= WN && (XN == 2 || XN == 3) && (WN == 2 || WN == 3), "the wait counts");
@@ -67,9 +64,9 @@ struct GemmTile {
         const int p0 = (g ^ (j & 7)) << 4, p1 = ((4 + g) ^ (j & 7)) << 4;
         const uint8_t* x0 = lds + (wx + j) * 128;
         const uint8_t* w0 = lds + XN * XB + (ww + j) * 128;
-        F8 x[2][HX], w[2][RW];
-        auto read_x = [&](int half, int k, int at, int a) { x[half][a] = *reinterpret_cast<const F8*>(x0 + at + (k ? p1 : p0) + (half * HX + a) * 2048); };
-        auto read_w = [&](int k, int at, int b) { w[k][b] = *reinterpret_cast<const F8*>(w0 + at + (k ? p1 : p0) + b * 2048); };
+        gt_b8 x[2][HX], w[2][RW];
+        auto read_x = [&](int half, int k, int at, int a) { x[half][a] = *reinterpret_cast<const gt_b8*>(x0 + at + (k ? p1 : p0) + (half * HX + a) * 2048); };
+        auto read_w = [&](int k, int at, int b) { w[k][b] = *reinterpret_cast<const gt_b8*>(w0 + at + (k ? p1 : p0) + b * 2048); };
         // a quarter of a step: half of the wave's X rows times half of the step's K.  Memory instructions go out between the MFMAs of two X
         // fragments, a few at a time: in one burst behind the barrier they hold up the MFMAs of all eight waves.
         auto quarter = [&](int half, int k, auto&& between) {
@@ -78,7 +75,7 @@ struct GemmTile {
                 between(a);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int b = 0; b < RW; ++b) acc[half * HX + a][b] = gt_mfma(w[k][b], x[half][a], acc[half * HX + a][b]);
+                for (int b = 0; b < RW; ++b) acc[half * HX + a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k][b], x[half][a], acc[half * HX + a][b], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };

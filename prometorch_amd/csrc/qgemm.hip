@@ -691,12 +691,11 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     // W and Xh are deliberately not __restrict__: loads through a restrict pointer may be moved across the
     // compiler fences below, and the prefetch distance of this loop depends on those fences
     constexpr int TM = 32 * MT;                     // rows of X per workgroup (MT tiles of 32)
-    constexpr int NT = 1;                           // 32-column tiles per wave
     constexpr int TN = 32 * WAVES;                  // columns per workgroup
     constexpr int RS = 2 * WAVES;                   // rows of the X tile that one fetch instruction of the workgroup covers
     constexpr int NPIECE = TM / RS;                 // 16-byte pieces of the X tile per thread
-    static_assert((WAVES == 4 && MT <= 2) || (WAVES == 8 && (MT == 4 || MT == 2 || MT == 1)), "wave layouts");
-    static_assert(NPIECE == 2 || NPIECE == 4 || NPIECE == 8 || NPIECE == 16, "pieces per thread");
+    static_assert((WAVES == 4 && (MT == 1 || MT == 2)) || (WAVES == 8 && (MT == 2 || MT == 4)), "wave layouts");
+    static_assert(NPIECE == 4 || NPIECE == 8, "pieces per thread");
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;  // s_a: [2][TM * QF_PITCH]
     const int j = lane & 31, kh = lane >> 5;
     const int m0 = by * TM;
@@ -704,59 +703,41 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     // split K: workgroup z of the grid sums super-blocks [blk0, blk0 + nblk) into its own M x N partial
     const int blk0 = bz * blocks_per_split;
     const int nblk = min(K / 256 - blk0, blocks_per_split);
-    const uint8_t* wrow[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-        wrow[t] = W + (int64_t)min(n_base + 32 * t + j, N - 1) * stride + (int64_t)blk0 * Tile::kBlockBytes;
+    const uint8_t* wrow = W + (int64_t)min(n_base + j, N - 1) * stride + (int64_t)blk0 * Tile::kBlockBytes;
 
-    f32x16 acc[MT][NT];
+    f32x16 acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mt][t][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) acc[mt][r] = 0.0f;
 
-    // X tile of a block = 128 rows x 512 B = 4096 pieces of 16 B; piece q = 256 i + tid (i = 0..15) is row q / 32, bytes
-    // 16 (q % 32): a wave fetches two whole rows per instruction and writes LDS without bank conflicts
+    // X tile of a block = TM rows x 512 B in pieces of 16 B; piece q = 64 WAVES i + tid (i < NPIECE) is row q / 32, bytes 16 (q % 32): a
+    // wave fetches two whole rows per instruction and writes LDS without bank conflicts
     const int64_t x_row_bytes = (int64_t)K * 2;
     const uint8_t* x_src = reinterpret_cast<const uint8_t*>(Xh) + (int64_t)(m0 + (tid >> 5)) * x_row_bytes + 16 * (tid & 31) +
                            (int64_t)blk0 * 512;
     uint8_t* x_dst = s_a + (tid >> 5) * QF_PITCH + 16 * (tid & 31);
     float* s_rs = reinterpret_cast<float*>(s_a + 2 * TM * QF_PITCH);  // the tile's TM row scales (every padded row has one)
     if (tid < TM) s_rs[tid] = rowscale[m0 + tid];
-    // the 16 pieces of the next tile in flight (scalars, not an array: they must stay in registers)
-    static_assert(MT == 1 || MT == 2 || MT == 4, "row tiles per workgroup");
-    uint4 x0, x1, x2, x3, x4, x5, x6, x7, x8, x9, x10, x11, x12, x13, x14, x15;
+    // the pieces of the next tile in flight (scalars, not an array: they must stay in registers)
+    uint4 x0, x1, x2, x3, x4, x5, x6, x7;
     // prologue: tile of block 0 -> LDS buffer 0, weights of block 0, fragments of step 0.  The weight loads go out behind
     // the tile's, before anything waits: one memory round trip for both, not two (a launch of two or three blocks per
     // workgroup, as the K splits of the narrow projections are, is mostly this prologue)
 #define QF_LD0(p) (*reinterpret_cast<const uint4*>(x_src + RS * (p) * x_row_bytes))
 #define QF_ST0(p, v) (*reinterpret_cast<uint4*>(x_dst + RS * (p) * QF_PITCH) = (v))
-    x0 = QF_LD0(0); x1 = QF_LD0(1);
-    if constexpr (NPIECE >= 4) { x2 = QF_LD0(2); x3 = QF_LD0(3); }
-    if constexpr (NPIECE >= 8) { x4 = QF_LD0(4); x5 = QF_LD0(5); x6 = QF_LD0(6); x7 = QF_LD0(7); }
-    if constexpr (NPIECE >= 16) {
-        x8 = QF_LD0(8); x9 = QF_LD0(9); x10 = QF_LD0(10); x11 = QF_LD0(11); x12 = QF_LD0(12);
-        x13 = QF_LD0(13); x14 = QF_LD0(14); x15 = QF_LD0(15);
-    }
+    x0 = QF_LD0(0); x1 = QF_LD0(1); x2 = QF_LD0(2); x3 = QF_LD0(3);
+    if constexpr (NPIECE == 8) { x4 = QF_LD0(4); x5 = QF_LD0(5); x6 = QF_LD0(6); x7 = QF_LD0(7); }
     issue_order_fence();
-    Tile cur[NT], nxt[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) cur[t].load(wrow[t], kh);
+    Tile cur, nxt;
+    cur.load(wrow, kh);
     issue_order_fence();
-    QF_ST0(0, x0); QF_ST0(1, x1);
-    if constexpr (NPIECE >= 4) { QF_ST0(2, x2); QF_ST0(3, x3); }
-    if constexpr (NPIECE >= 8) { QF_ST0(4, x4); QF_ST0(5, x5); QF_ST0(6, x6); QF_ST0(7, x7); }
-    if constexpr (NPIECE >= 16) {
-        QF_ST0(8, x8); QF_ST0(9, x9); QF_ST0(10, x10); QF_ST0(11, x11); QF_ST0(12, x12);
-        QF_ST0(13, x13); QF_ST0(14, x14); QF_ST0(15, x15);
-    }
+    QF_ST0(0, x0); QF_ST0(1, x1); QF_ST0(2, x2); QF_ST0(3, x3);
+    if constexpr (NPIECE == 8) { QF_ST0(4, x4); QF_ST0(5, x5); QF_ST0(6, x6); QF_ST0(7, x7); }
 #undef QF_LD0
 #undef QF_ST0
-    h8 bf[NT][2], bn[NT][2];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) cur[t].frags(0, kh, bf[t][0], bf[t][1]);
+    h8 bf[2], bn[2];
+    cur.frags(0, kh, bf[0], bf[1]);
     __syncthreads();
 
     for (int blk = 0; blk < nblk; ++blk) {
@@ -774,47 +755,30 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
         for (int s = 0; s < 8; ++s) {  // unrolled: the sub-block index selects registers
 #define QF_LD(p) (*reinterpret_cast<const uint4*>(x_from + RS * (p) * x_row_bytes))
 #define QF_ST(p, v) (*reinterpret_cast<uint4*>(x_nxt + RS * (p) * QF_PITCH) = (v))
-            // For the 128-row tile the fetches of the next block are spread over steps 0..3 and the LDS stores of the tile pieces
+            // Where a thread has eight pieces the fetches of the next block are spread over steps 0..3 and the LDS stores of the tile pieces
             // over steps 4..7: issued in one burst at step 0 they held up the vector-memory path for everything behind them
             // (512 x 4096 x 14336: 75.6 -> 72.1 us; a 2048-token prompt 26.3 -> 25.6 ms; prompts of up to 64 rows were 2 % slower
-            // with their few pieces spread, so the small tiles keep the burst).  Tile pieces go FIRST and the weights last (step 3):
+            // with their four pieces spread, so those keep the burst; the 64-row tile of four waves has eight, and the same time either
+            // way: 64 rows, four layers of Qwen3-4B shapes, 537 ... 553 us spread, 549 in a burst).  Tile pieces go FIRST and the weights last (step 3):
             // loads return in order, so a wait for a piece must not have the weight loads (HBM latency, one cache line per
             // lane) in front of it; the weights are first needed at step 7.
-#define QF_W() _Pragma("unroll") for (int t = 0; t < NT; ++t) nxt[t].load(wrow[t] + (int64_t)nb * Tile::kBlockBytes, kh)
             if constexpr (NPIECE == 8) {
                 if (s == 0) { x0 = QF_LD(0); x1 = QF_LD(1); }
                 if (s == 1) { x2 = QF_LD(2); x3 = QF_LD(3); }
                 if (s == 2) { x4 = QF_LD(4); x5 = QF_LD(5); }
-                if (s == 3) { x6 = QF_LD(6); x7 = QF_LD(7); issue_order_fence(); QF_W(); }
+                if (s == 3) { x6 = QF_LD(6); x7 = QF_LD(7); issue_order_fence(); nxt.load(wrow + (int64_t)nb * Tile::kBlockBytes, kh); }
                 if (s == 4) { QF_ST(0, x0); QF_ST(1, x1); }
                 if (s == 5) { QF_ST(2, x2); QF_ST(3, x3); }
                 if (s == 6) { QF_ST(4, x4); QF_ST(5, x5); }
                 if (s == 7) { QF_ST(6, x6); QF_ST(7, x7); }
-            } else if constexpr (NPIECE <= 4) {  // the 64- and 32-row tiles: one burst and one step of stores measured faster there
+            } else {
                 if (s == 0) {
-                    x0 = QF_LD(0); x1 = QF_LD(1);
-                    if constexpr (NPIECE == 4) { x2 = QF_LD(2); x3 = QF_LD(3); }
+                    x0 = QF_LD(0); x1 = QF_LD(1); x2 = QF_LD(2); x3 = QF_LD(3);
                     issue_order_fence();
-                    QF_W();
-                }
-                if (s == 3) {
-                    QF_ST(0, x0); QF_ST(1, x1);
-                    if constexpr (NPIECE == 4) { QF_ST(2, x2); QF_ST(3, x3); }
-                }
-            } else {  // 16 pieces (the four-wave 128-row layout): one burst at step 0, stores in steps 3..6
-                if (s == 0) {
-                    x0 = QF_LD(0); x1 = QF_LD(1); x2 = QF_LD(2); x3 = QF_LD(3); x4 = QF_LD(4); x5 = QF_LD(5); x6 = QF_LD(6); x7 = QF_LD(7);
-                    x8 = QF_LD(8); x9 = QF_LD(9); x10 = QF_LD(10); x11 = QF_LD(11); x12 = QF_LD(12);
-                    x13 = QF_LD(13); x14 = QF_LD(14); x15 = QF_LD(15);
-                    issue_order_fence();
-                    QF_W();
+                    nxt.load(wrow + (int64_t)nb * Tile::kBlockBytes, kh);
                 }
                 if (s == 3) { QF_ST(0, x0); QF_ST(1, x1); QF_ST(2, x2); QF_ST(3, x3); }
-                if (s == 4) { QF_ST(4, x4); QF_ST(5, x5); QF_ST(6, x6); QF_ST(7, x7); }
-                if (s == 5) { QF_ST(8, x8); QF_ST(9, x9); QF_ST(10, x10); QF_ST(11, x11); }
-                if (s == 6) { QF_ST(12, x12); QF_ST(13, x13); QF_ST(14, x14); QF_ST(15, x15); }
             }
-#undef QF_W
 #undef QF_LD
 #undef QF_ST
             issue_order_fence();  // the fetches stay HERE, two steps ahead of their use (the compiler would sink them to it)
@@ -827,7 +791,7 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(af[ks][mt]));
             // X fragments of the NEXT step are read from LDS now and weight fragments of the next step are prepared
-            // while this step's 16 MFMAs (all operands already in registers) run
+            // while this step's MFMAs (all operands already in registers) run
             h8 an[2][MT];
             if (s < 7) {
 #pragma unroll
@@ -836,20 +800,14 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
                     for (int mt = 0; mt < MT; ++mt)
                         an[ks][mt] = *reinterpret_cast<const h8*>(a_cur + (mt * 32 + j) * QF_PITCH + 64 * (s + 1) + 32 * kh + 16 * ks);
             }
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                if (s < 7) cur[t].frags(s + 1, kh, bn[t][0], bn[t][1]);
-                else { nxt[t].pin(); nxt[t].frags(0, kh, bn[t][0], bn[t][1]); }
-            }
+            if (s < 7) cur.frags(s + 1, kh, bn[0], bn[1]);
+            else { nxt.pin(); nxt.frags(0, kh, bn[0], bn[1]); }
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        acc[mt][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks][mt], bf[t][ks], acc[mt][t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) { bf[t][0] = bn[t][0]; bf[t][1] = bn[t][1]; }
+                for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks][mt], bf[ks], acc[mt], 0, 0, 0);
+            bf[0] = bn[0];
+            bf[1] = bn[1];
             if (s < 7) {
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks)
@@ -857,42 +815,38 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
                     for (int mt = 0; mt < MT; ++mt) af[ks][mt] = an[ks][mt];
             }
         }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) cur[t] = nxt[t];
+        cur = nxt;
         __syncthreads();  // next tile complete, this tile no longer read
     }
     // C layout of the 32x32 tile: column j = lane % 32, rows 8 (r / 4) + 4 (lane / 32) + r % 4.  The row scales come from
     // LDS (staged in the prologue), and when accumulating the 16 old values of a tile are fetched together before its 16
     // stores: a load issued behind a store the compiler cannot tell apart from it is one serial memory round trip per value,
     // more than the main loop of a launch with few blocks per workgroup takes.
+    const int n = n_base + j;
+    const bool n_ok = n < N;
+    const int nc = n_ok ? n : N - 1;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int n = n_base + 32 * t + j;
-        const bool n_ok = n < N;
-        const int nc = n_ok ? n : N - 1;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            float old[16];
-            if (!partials && accumulate) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = min(m0 + mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), M - 1);
-                    old[r] = Y[(int64_t)m * N + nc];
-                }
-                issue_order_fence();
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) old[r] = 0.0f;
-            }
+    for (int mt = 0; mt < MT; ++mt) {
+        float old[16];
+        if (!partials && accumulate) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int lr = mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-                const int m = m0 + lr;
-                const float v = acc[mt][t][r] * s_rs[lr];
-                if (m < M && n_ok) {
-                    if (partials) __builtin_nontemporal_store(v, &partials[((int64_t)bz * M + m) * N + n]);
-                    else __builtin_nontemporal_store(accumulate ? old[r] + v : v, &Y[(int64_t)m * N + n]);
-                }
+                const int m = min(m0 + mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), M - 1);
+                old[r] = Y[(int64_t)m * N + nc];
+            }
+            issue_order_fence();
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) old[r] = 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int lr = mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            const int m = m0 + lr;
+            const float v = acc[mt][r] * s_rs[lr];
+            if (m < M && n_ok) {
+                if (partials) __builtin_nontemporal_store(v, &partials[((int64_t)bz * M + m) * N + n]);
+                else __builtin_nontemporal_store(accumulate ? old[r] + v : v, &Y[(int64_t)m * N + n]);
             }
         }
     }
@@ -920,8 +874,8 @@ __device__ __forceinline__ void qf_tile_of(int L, int gx, int gy, int& bx, int& 
     bx = within / rows;
 }
 
-template <typename Tile, int MT, int WAVES = 4>
-__global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : (MT <= 2 ? 2 : 1))) void qgemm_f16_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh,
+template <typename Tile, int MT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh,
                                                         const float* __restrict__ rowscale, float* Y, int M, int K, int N,
                                                         int accumulate, int blocks_per_split, float* partials) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
@@ -932,7 +886,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : (MT <= 2 ? 2 : 1))) v
     qgemm_f16_body<Tile, MT, WAVES>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds);
 }
 
-// Up to three projections of the same rows in ONE launch of the eight-wave 128-row tile (q, k, v of a layer: in a Q4_K_M
+// Up to three projections of the same rows in ONE launch, its tile chosen as below for a single matrix (q, k, v of a layer: in a Q4_K_M
 // file two Q4_K matrices and a Q6_K one).  Each matrix brings its own prepared rows (Q8-rounded for Q4_K, plain for
 // Q6_K), column tiles and K splits; blockIdx.x walks the (column tile, split) slots of the matrices one after the other.
 // Three narrow launches of two or three blocks per workgroup are mostly launch, prologue and epilogue; one launch pays
@@ -1139,9 +1093,9 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     const int tn = narrow ? 128 : QF_TN;
     const dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm, splits);
     const uint8_t* Wb = static_cast<const uint8_t*>(W);
-    // Every tile height runs with eight waves (two per SIMD, one 32-column strip each): against four waves owning two strips
-    // each, 512 x 4096 x 14336 104 -> 92 us (128 rows), 512 x 4096 x 4096 59.8 -> 45.3 us and 96 x 4096 x 2560 57.0 -> 42.7 us
-    // (64 rows), a 16-token prompt 4.09 -> 3.86 ms (32 rows); the 64-row Q6_K tile no longer spills.
+    // 256 columns run with eight waves (two per SIMD, one 32-column strip each): against four waves owning two strips each, 512 x 4096 x
+    // 14336 104 -> 92 us (128 rows), 512 x 4096 x 4096 59.8 -> 45.3 us and 96 x 4096 x 2560 57.0 -> 42.7 us (64 rows).  128 columns have
+    // four waves of one strip.
 #define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials)
     if (q4) {
         if (MT == 4) PTM_QF(Q4Tile, 4, 8);
