@@ -3,7 +3,8 @@ import random
 
 import pytest
 
-from gemm_helpers import DECAY, ELEM, F32, SWIGLU, TILES, plan
+from gemm_helpers import DECAY, ELEM, F32, RELU2, SWIGLU, TILES, plan
+from test_gpu_gemm_tiles import LARGE
 
 
 # outputs of few tiles: up to 256 of 64 x 64, up to 512 where K is short; split, tiles x splits
@@ -58,3 +59,22 @@ def test_plans_cover_each_output():
                 assert lo <= end, (M, N, K, n)
                 end = max(end, hi)
             assert end == M, (M, N, K, n)
+
+
+def test_the_gpu_cases_reach_every_kind_of_tile_and_region():
+    alone, rows, columns, splits = set(), set(), set(), set()
+    for M, N, K, epilogue, section, slabs in LARGE:
+        n, _, regions = plan(M, N, K, epilogue, section, slabs)
+        kinds = [r[0] for r in regions]
+        assert kinds, (M, N, K)
+        if len(kinds) == 1:
+            alone.add((kinds[0], epilogue, section > 0))
+        rows |= {(epilogue, section > 0) for r in regions if r[2] > 0}
+        columns |= {(epilogue, section > 0) for r in regions if r[3] > 0}
+        splits |= {(k, len(kinds) > 1) for k in kinds if n > 1}
+    kinds = {0, 1, 2, 3, 4, 6}  # (64 rows of 256 columns are best where something is left over, or in sections)
+    assert alone >= {(k, e, False) for k in kinds for e in (F32, ELEM, RELU2, SWIGLU, DECAY)} and (5, F32, True) in alone
+    assert rows >= {(e, False) for e in (F32, ELEM, RELU2, SWIGLU, DECAY)} | {(F32, True)}
+    assert columns >= {(e, False) for e in (ELEM, RELU2, SWIGLU, DECAY)} | {(F32, True)}
+    assert splits >= {(3, False), (4, False), (6, False), (5, True)}
+    assert max(len(plan(*c)[2]) for c in LARGE) == 3

@@ -119,6 +119,25 @@ def test_few_tiles(dev, case):
     assert check_product(*case) > 1 or not case[5]
 
 
+# (rows, columns, K, result, section, partial sums): each kind of tile alone with each kind of result, two and three kinds in a launch with
+# columns or rows left over, sections, K splits; tests/test_gemm_plan_cpu.py holds the list against the plans
+LARGE = [(1158, 9988, 72, F32, 0, 0), (555, 13646, 61, F32, 0, 0), (389, 13212, 71, F32, 0, 16), (266, 13268, 64, F32, 0, 16), (133, 11662, 65, F32, 0, 0), (75, 8204, 141, F32, 0, 0),
+         (1472, 8616, 60, ELEM, 0, 0), (515, 13976, 67, ELEM, 0, 0), (464, 12394, 74, ELEM, 0, 0), (259, 13920, 73, ELEM, 0, 0), (257, 6690, 91, ELEM, 0, 0), (67, 8376, 176, ELEM, 0, 0),
+         (1333, 9462, 79, RELU2, 0, 0), (680, 10786, 61, RELU2, 0, 0), (514, 10650, 64, RELU2, 0, 0), (385, 9742, 71, RELU2, 0, 0), (229, 8348, 80, RELU2, 0, 0), (72, 9262, 145, RELU2, 0, 0),
+         (1370, 8996, 69, SWIGLU, 0, 0), (529, 13306, 63, SWIGLU, 0, 0), (393, 13092, 85, SWIGLU, 0, 0), (1041, 3844, 64, SWIGLU, 0, 0), (131, 12082, 98, SWIGLU, 0, 0), (79, 8604, 149, SWIGLU, 0, 0),
+         (1170, 10054, 89, DECAY, 0, 0), (678, 11300, 72, DECAY, 0, 0), (441, 13136, 63, DECAY, 0, 0), (286, 13490, 62, DECAY, 0, 0), (138, 11264, 73, DECAY, 0, 0), (75, 8672, 147, DECAY, 0, 0),
+         (1343, 8192, 79, F32, 2048, 0), (1355, 4608, 83, F32, 1152, 0), (592, 7168, 78, F32, 1792, 0), (406, 10752, 63, F32, 2688, 0), (1468, 11264, 115, F32, 2816, 0), (80, 9216, 150, F32, 2304, 0),
+         (1488, 13894, 124, ELEM, 0, 0), (1468, 12982, 446, SWIGLU, 0, 0), (1175, 13112, 146, RELU2, 0, 0), (1426, 12016, 275, DECAY, 0, 0), (1364, 12288, 357, F32, 3072, 0),
+         (1059, 13522, 97, ELEM, 0, 0), (843, 12602, 69, SWIGLU, 0, 0), (1103, 10638, 147, RELU2, 0, 0), (1356, 8318, 135, DECAY, 0, 0), (1299, 10800, 266, F32, 0, 0), (1132, 10752, 114, F32, 2688, 0),
+         (1325, 13874, 81, ELEM, 0, 0), (1310, 11976, 118, SWIGLU, 0, 0), (1192, 8192, 89, F32, 2048, 0), (1030, 9728, 1000, ELEM, 0, 0), (513, 19458, 500, SWIGLU, 0, 0),
+         (71, 11412, 3312, F32, 0, 16), (68, 9600, 1997, F32, 0, 16), (141, 5788, 2340, F32, 0, 16), (71, 3502, 1168, F32, 0, 16), (138, 13930, 3795, F32, 0, 16)]
+
+
+@pytest.mark.parametrize("i,case", list(enumerate(LARGE)), ids=lambda v: str(v) if isinstance(v, tuple) else "")
+def test_kinds_and_regions(dev, i, case):
+    check_product(*case, pad=i % 8)
+
+
 # the results that are not plain sums (squared ReLU, gated SiLU, decays, 16-bit rows, sections of one product) and their odd sizes
 @pytest.mark.parametrize("design", ["tovasun", "nadozen"])
 def test_prompts_of_many_rows(dev, tmp_path, design):
