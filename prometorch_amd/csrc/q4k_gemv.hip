@@ -40,9 +40,11 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArg
 
 // Gate / up behind RMSNorm, 5 to 16 waves per CU, K <= 4096: in workgroups of four waves each of them normalises and quantises the whole
 // vector, 300 instructions per wave in front of a tile's 250.  One workgroup per CU shares that work; rows, lanes and sums are those
-// of q4k_gemv_kernel.  2816 x 1024 4.68 -> 3.92 us, 6144 x 1536 5.10 -> 4.61, 4096 x 2560 6.02 -> 5.39, 4096 x 4096 6.61 -> 6.07 (in a
-// graph; of 99 sizes from 700 x 256 to 9728 x 4096 none slower).  Its barriers cost more than it saves with more waves (two workgroups of
-// ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80).
+// of q4k_gemv_kernel.  Weights from HBM, in a graph: 2816 x 1024 5.50 -> 4.84 us, 6144 x 1536 6.15 -> 5.66, 4096 x 2560 7.00 -> 6.76, 3472 x
+// 3072 6.98 -> 6.74 (from the caches 4.68 -> 3.92, 5.10 -> 4.61, 6.02 -> 5.39).  Its barriers cost more than it saves with more waves (two
+// workgroups of ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80), and where 14 to 16 waves wait for more
+// than 15 MB together: 14752 x 1024 7.38 -> 7.62, 8192 x 2048 7.53 -> 7.88, 8192 x 2560 8.52 -> 9.01, 3968 x 3584 7.72 -> 7.92 (13 waves,
+// 6248 x 2560, 8.22 -> 7.89; 16 waves, 9.4 MB, 4096 x 1024, 6.22 -> 5.56).
 template <int NB, int NX>
 __global__ __launch_bounds__(1024) void q4k_gemv_wide_kernel(const Q4KArgs a) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -193,8 +195,9 @@ static int q4k_launch(Q4KArgs& a, hipStream_t s) {
     if constexpr (NORM && MODE == 1) {
         const int rows_per_wave = 8 >> a.log2S, total = (a.total_rows + rows_per_wave - 1) / rows_per_wave, per_cu = (total + 255) / 256;
         const int nx = (a.K + 256 * per_cu - 1) / (256 * per_cu);
+        const bool heavy = per_cu > 13 && (int64_t)a.total_rows * (a.K / 256) * 144 > 15000000;
         // K: the sum of squares is taken from 16 values of each of the first 256 threads (longer vectors: the loop of the four-wave form)
-        if (per_cu >= 5 && per_cu <= 16 && nx <= 2 && nb <= 5 && a.K <= 16 * Q4K_THREADS) {
+        if (per_cu >= 5 && per_cu <= 16 && !heavy && nx <= 2 && nb <= 5 && a.K <= 16 * Q4K_THREADS) {
             const dim3 grid((total + per_cu - 1) / per_cu);
 #define PTM_WIDE(NBV, NXV) hipLaunchKernelGGL((q4k_gemv_wide_kernel<NBV, NXV>), grid, dim3(64 * per_cu), lds, s, a)
             switch (2 * nb + nx) {

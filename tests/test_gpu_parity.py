@@ -401,9 +401,11 @@ def test_fused_gate_up_silu_tall_shapes_vs_oracle(dev, po, N, K):
     assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2
 
 
-@pytest.mark.parametrize("N,K", [(5120, 256), (1281, 1024), (2816, 1024), (4096, 1024), (4097, 1024), (1900, 2560), (2100, 4096), (3333, 1536)])
+@pytest.mark.parametrize("N,K", [(5120, 256), (1281, 1024), (2816, 1024), (4096, 1024), (4097, 1024), (1900, 2560), (2100, 4096), (3333, 1536),
+                                 (3472, 3584), (3720, 3584), (3728, 3584)])
 def test_fused_gate_up_silu_one_workgroup_per_cu(dev, po, N, K):
-    """5 to 16 waves per CU (4097 x 1024: the first beyond): one or two values of x per thread, rows that end inside a wave; bars as above."""
+    """5 to 16 waves per CU (4097 x 1024: the first beyond; 3728 x 3584: more than 15 MB): one or two values of x per thread, rows that end inside
+    a wave; bars as above."""
     r = synth.rng_for(58, N, K)
     Wg, Wu = synth.make_q4k(r, N, K), synth.make_q4k(r, N, K)
     x = (synth.make_x(r, K) * 2.0).astype(np.float32)
