@@ -186,8 +186,8 @@ __global__ __launch_bounds__(256) void rowwave_gemv_kernel(const uint8_t* __rest
     }
 }
 
-// y[r] (+)= the row's terms; R rows per wave, four waves per workgroup, C of them (1 or 4) at the same rows
-template <typename Fmt, int R, int C, bool ACC>
+// y[r] (+)= the row's terms; R rows per wave, four waves per workgroup, C of them (1 or 4) at the same rows, U passes over a row requested together
+template <typename Fmt, int R, int C, int U, bool ACC>
 __global__ __launch_bounds__(256) void slots_gemv_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, float* __restrict__ y,
                                                          int K, int N, int64_t stride) {
     __shared__ float part[4][R];
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) void slots_gemv_kernel(const uint8_t* __restri
         acc[i] = 0.0f;
     }
     const int slots = K / Fmt::VALUES;
-    constexpr int U = 2;  // passes requested together; a lane beyond the row repeats the last slot and does not count it
+    // a lane beyond the row repeats the last slot and does not count it
     for (int first = (wave % C) * 64 * U; first < slots; first += 64 * U * C) {
         typename Fmt::X xv[U];
         typename Fmt::Raw w[U][R];
@@ -264,25 +264,32 @@ static int slots_launch(const void* W, const float* x, float* y, int K, int N, i
     const int rc = gemv_check<Fmt>(W, x, y, K, N, stride, per_block, w_align);
     if (rc != PTM_OK) return rc;
     const uint8_t* w = static_cast<const uint8_t*>(W);
-    auto go = [&](auto rows, auto waves) {
-        constexpr int R = decltype(rows)::value, C = decltype(waves)::value;
+    auto go = [&](auto rows, auto waves, auto passes) {
+        constexpr int R = decltype(rows)::value, C = decltype(waves)::value, U = decltype(passes)::value;
         const dim3 grid((N + 4 / C * R - 1) / (4 / C * R)), block(256);
-        if (accumulate) hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, true>), grid, block, 0, s, w, x, y, K, N, stride);
-        else hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, false>), grid, block, 0, s, w, x, y, K, N, stride);
+        if (accumulate) hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, U, true>), grid, block, 0, s, w, x, y, K, N, stride);
+        else hipLaunchKernelGGL((slots_gemv_kernel<Fmt, R, C, U, false>), grid, block, 0, s, w, x, y, K, N, stride);
     };
     using std::integral_constant;
+    constexpr integral_constant<int, 1> one;
+    constexpr integral_constant<int, 2> two;
+    constexpr integral_constant<int, 4> four;
     // Four waves at the same rows where a row has two requests or more for each of them, more rows to share x between the more rows there are.
     // us for one / two rows a wave, then for one / two / four with four waves at them, Q8_0: 9728 x 2560 12.4 10.4 | 11.2 9.5 9.0, 2560 x 9728
     // 12.6 15.4 | 11.9 10.9 10.5, 1024 x 2560 3.3 3.8 | 3.0 2.9 3.0, 700 x 14336 9.7 13.2 | 5.8 6.6 6.3, 9728 x 1024 5.3 5.0 | 7.2 6.2 5.0.
+    // Rows of one pass: a second request would repeat it, Q5_K 2560 x 256 4.0 -> 3.2 us (a wave per row, 32 values a lane: 3.7), 9728 x 1024 7.2 ->
+    // 4.8 (9.2), Q8_0 2560 x 512 3.0 -> 2.8 (3.8).
     const int slots = K / Fmt::VALUES;
     if (slots >= (N >= 2048 ? Fmt::LONG : 256)) {
-        if (N >= 2048) go(integral_constant<int, Fmt::ROWS>{}, integral_constant<int, 4>{});
-        else if (N >= 1024) go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
-        else go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-    } else if (N >= 2048) {
-        go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+        if (N >= 2048) go(integral_constant<int, Fmt::ROWS>{}, four, two);
+        else if (N >= 1024) go(two, four, two);
+        else go(one, four, two);
+    } else if (slots <= 64) {
+        if (N >= 2048) go(two, one, one);
+        else go(one, one, one);
     } else {
-        go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+        if (N >= 2048) go(two, one, two);
+        else go(one, one, two);
     }
     return launch_status();
 }

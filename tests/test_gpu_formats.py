@@ -62,6 +62,19 @@ def test_other_formats_gemv_rows_per_wave(dev, po, qt, N, K):
     assert rel_err(gpu_gemv(qt, W, x), po.gemv(qt, W, x)) <= GEMV_TOL * 1e-2
 
 
+@pytest.mark.parametrize("qt,N,K", [(qt, N, K) for qt, per, once in ((8, 32, 512), (6, 32, 512), (13, 256, 1024)) for N, K in
+                                    ((7, per), (2047, once), (2049, once), (2049, once - per), (2049, once + per))])
+def test_other_formats_gemv_rows_of_one_pass(dev, po, qt, N, K):
+    """Rows of up to 64 slots are requested once, longer ones two passes at a time."""
+    r = synth.rng_for(37, qt, N, K)
+    W = synth.make_weight(r, qt, N, K)
+    x = synth.make_x(r, K)
+    ref = po.gemv(qt, W, x)
+    assert rel_err(gpu_gemv(qt, W, x), ref) <= GEMV_TOL * 1e-2
+    y0 = synth.make_x(r, N)
+    assert np.abs((gpu_gemv(qt, W, x, accumulate=True, y0=y0) - y0) - ref).max() <= 1e-5 * max(np.abs(y0).max(), np.abs(ref).max())
+
+
 @pytest.mark.parametrize("qt,N,K", [(13, 24, 512), (13, 3, 2560), (8, 24, 512), (8, 5, 96)])
 def test_other_formats_dequant_bit_exact(dev, po, seeds, golden_formats, qt, N, K):
     r = synth.rng_for(seeds["blocks"], qt, N, K)
