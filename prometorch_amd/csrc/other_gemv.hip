@@ -24,9 +24,10 @@ __device__ __forceinline__ void load8(const float* __restrict__ x, float (&v)[8]
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-// A format: VALUES of a row per slot, ROWS per wave and from how many slots LONG rows are shared by waves (slots_launch), what a lane loads of the row for slot u, which values of x (two groups of 8 or 4), the slot's term.
+// A format: VALUES of a row per slot; from how many slots LONG rows are shared by waves, then ROWS per wave of 2048 rows and more, FEW of 1024 to
+// 2047 (slots_launch); what a lane loads of the row for slot u, which values of x (two groups of 8 or 4), the slot's term.
 struct FmtQ8_0 {
-    static constexpr int BLOCK_BYTES = 34, VALUES = 8, ROWS = 4, LONG = 256;
+    static constexpr int BLOCK_BYTES = 34, VALUES = 8, ROWS = 4, FEW = 2, LONG = 256;
     struct Raw { u64_a2 q; uint32_t d; };
     struct X { float v[8]; };
     static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
@@ -51,7 +52,7 @@ struct FmtQ8_0 {
 };
 
 struct FmtQ5_0 {
-    static constexpr int BLOCK_BYTES = 22, VALUES = 8, ROWS = 2, LONG = 256;  // four low nibbles and the four high ones of the same bytes, 16 values on
+    static constexpr int BLOCK_BYTES = 22, VALUES = 8, ROWS = 2, FEW = 1, LONG = 256;  // four low nibbles and the four high ones of the same bytes, 16 values on
     struct Raw { uint32_t q, h, d; };
     struct X { float v[8]; };
     static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
@@ -80,7 +81,7 @@ struct FmtQ5_0 {
 };
 
 struct FmtQ5_K {
-    static constexpr int BLOCK_BYTES = 176, VALUES = 16, ROWS = 4, LONG = 512;  // eight low nibbles and the eight high ones of the same bytes, 32 values on
+    static constexpr int BLOCK_BYTES = 176, VALUES = 16, ROWS = 4, FEW = 2, LONG = 512;  // eight low nibbles and the eight high ones of the same bytes, 32 values on
     struct Raw { uint4 hdr; uint2 q, h; };
     struct X { float lo[8], hi[8]; };
     // scale and min of sub-block sb from the 12 packed bytes at p + 4 (get_scale_min_k4, gguf_dequant.h:289-297)
@@ -277,12 +278,14 @@ static int slots_launch(const void* W, const float* x, float* y, int K, int N, i
     // Four waves at the same rows where a row has two requests or more for each of them, more rows to share x between the more rows there are.
     // us for one / two rows a wave, then for one / two / four with four waves at them, Q8_0: 9728 x 2560 12.4 10.4 | 11.2 9.5 9.0, 2560 x 9728
     // 12.6 15.4 | 11.9 10.9 10.5, 1024 x 2560 3.3 3.8 | 3.0 2.9 3.0, 700 x 14336 9.7 13.2 | 5.8 6.6 6.3, 9728 x 1024 5.3 5.0 | 7.2 6.2 5.0.
+    // Q5_0 unpacks more per byte, and of 1024 to 2047 rows one a wave leaves fewer waves without work: 1024 x 2048 3.57 us with two, 3.07 with one (a
+    // wave per row, 32 values a lane: 3.31), 1280 x 4096 4.75 4.36, 2047 x 2048 3.94 3.73, 2047 x 8192 7.97 8.14.
     // Rows of one pass: a second request would repeat it, Q5_K 2560 x 256 4.0 -> 3.2 us (a wave per row, 32 values a lane: 3.7), 9728 x 1024 7.2 ->
     // 4.8 (9.2), Q8_0 2560 x 512 3.0 -> 2.8 (3.8).
     const int slots = K / Fmt::VALUES;
     if (slots >= (N >= 2048 ? Fmt::LONG : 256)) {
         if (N >= 2048) go(integral_constant<int, Fmt::ROWS>{}, four, two);
-        else if (N >= 1024) go(two, four, two);
+        else if (N >= 1024) go(integral_constant<int, Fmt::FEW>{}, four, two);
         else go(one, four, two);
     } else if (slots <= 64) {
         if (N >= 2048) go(two, one, one);
