@@ -226,9 +226,11 @@ __device__ __forceinline__ void dense_tile(const DenseGemm& g, const GemmRegion&
     // two-byte results: a lane's two sums next to each other make one 16-byte store (1030 x 9728 x 2560 63.0 -> 57.7 us); fp32 sums of
     // one fragment are 16 bytes already, and the four lanes of a row then store 64 in a row
     const bool glu = g.epilogue == GEMM_SWIGLU, pairs = g.epilogue == GEMM_ELEM || g.epilogue == GEMM_RELU2;
-    // Offsets count from a wave's first row, which no other of its rows lies in front of (GEMM_SWIGLU: tiles start with whole blocks of 32
-    // columns, and an instruction's 8 rows are gates in the waves without bit 1 and ups, half of W further on, in those with it)
-    const int w0 = weight_row(g, n0 + (glu ? (wave & 2) << 3 : 0));
+    // Offsets count from the tile's first row, which no other of its rows lies in front of (GEMM_SWIGLU: tiles start with whole blocks of 32
+    // columns), and where the ups, half of W further on, are more than 2 GiB away from the wave's first row: an instruction's 8 rows are
+    // gates in the waves without bit 1 and ups in those with it.  (So everywhere, 2048 x 19456 x 2560 takes 185 us instead of 176.)
+    const bool far = glu && (int64_t)g.N * g.ldw >= 0x7fffffff;
+    const int w0 = weight_row(g, n0 + (far ? (wave & 2) << 3 : 0));
     const gt_i4 xs = gt_buffer(A), ws = gt_buffer(g.W + (int64_t)w0 * g.ldw + first * 64);
     const uint32_t piece = ((lane & 7) ^ (lane >> 3)) << 4;
     uint32_t xo[Tile::NX], wo[Tile::NW];

@@ -64,16 +64,19 @@ def test_rows_far_apart(dev, lda, ldw):
     assert ((C.double() - a @ w.T).abs() <= bound).all()
 
 
-def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0):
+def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0, ldw=0):
     """One product as the block decoders' runtime calls it against 64 bits; how many K splits it took."""
     g = torch.Generator(device="cuda").manual_seed(M * 7 + N * 3 + K + epilogue)
     kp, S = (K + 63) // 64 * 64, N // section if section else 1
-    A, W = (torch.zeros(*shape, kp, dtype=torch.bfloat16, device="cuda") for shape in ((S, M), (N,)))
+    A = torch.zeros(S, M, kp, dtype=torch.bfloat16, device="cuda")
+    ldw = ldw or kp
+    W = torch.empty((N - 1) * ldw + kp, dtype=torch.bfloat16, device="cuda").as_strided((N, kp), (ldw, 1))
+    W[:, K:] = 0
     A[..., :K], W[:, :K] = torch.randn(S, M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g) * K ** -0.5
     cols = N // 2 if epilogue == SWIGLU else N
     ldc, bias = cols + pad, torch.randn(N, device="cuda", generator=g) - 1
     out = torch.full((max(1, slabs), M, ldc), float("nan"), device="cuda", dtype=torch.float32 if epilogue in (F32, DECAY) else torch.bfloat16)
-    c = Call(A=A.data_ptr(), W=W.data_ptr(), C=out.data_ptr(), bias=bias.data_ptr(), lda=kp, ldw=kp, ldc=ldc, section_a=M * kp, slab=M * ldc,
+    c = Call(A=A.data_ptr(), W=W.data_ptr(), C=out.data_ptr(), bias=bias.data_ptr(), lda=kp, ldw=ldw, ldc=ldc, section_a=M * kp, slab=M * ldc,
              slab_room=M * ldc * slabs, M=M, N=N, K=K, epilogue=epilogue, section_n=section, may_split=int(slabs > 0))
     splits = C.c_int32()
     torch.cuda.synchronize()
@@ -106,6 +109,12 @@ def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0):
         want, bound = torch.exp(-torch.exp(v + bias.double())), 0.4 * (off + 2.0 ** -23 * (v.abs() + bias.double().abs())) + 2.0 ** -21
     assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
     return splits
+
+
+# gates and ups just under and over 2 GiB apart, and 4.6 GiB
+@pytest.mark.parametrize("ldw", [558656, 558664, 1200000])
+def test_ups_far_from_their_gates(dev, ldw):
+    check_product(1041, 3844, 64, SWIGLU, ldw=ldw)
 
 
 # outputs of few tiles (64 x 64, four waves each): one, all 256 of a round and a little more, split, and every kind of result
