@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
                                                                         int64_t past_host, int max_seq,
                                                                         uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
     constexpr int NOUT = HD / 4;
-    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
+    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
     const float4* pO4 = reinterpret_cast<const float4*>(pO);
     // Every load of the common case goes out before the position is known: chunk slots past the last active one
     // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the first wave makes one
