@@ -116,8 +116,7 @@ int ptm_quant_gemv_supported(uint32_t ggml_type);
 
 /* The dispatcher's other formats, fp32 activations, y (+)= W.x (q8_0_gemv_avx2 cpu_quant_gemv.h:784-826, q5k_gemv_avx2
  * :1091-1185, q5_0_gemv_scalar :1572-1630).  K a multiple of 32 (Q8_0: 34-byte blocks; Q5_0: 22-byte blocks; W and the
- * row stride 2-byte aligned) or of 256 (Q5_K: 176-byte super-blocks, 4-byte aligned); x 16-byte aligned.  No file of
- * the decode path's models holds these types: the kernels are plain row-per-wave ones, not tuned. */
+ * row stride 2-byte aligned) or of 256 (Q5_K: 176-byte super-blocks, 4-byte aligned); x 16-byte aligned. */
 int ptm_q8_0_gemv(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,
                   ptm_stream_t stream);
 int ptm_q5k_gemv(const void* W, const float* x, float* y, int K, int N, int64_t row_stride_bytes, int accumulate,

@@ -6,11 +6,12 @@
 // wave's instruction fills 8 rows, the lanes' global addresses carry the permutation); a step has one barrier, in front of its last quarter,
 // and the fetches behind it are the ones into the LDS it freed.
 //
-// What bounds it (256 x 256, 8192 x 8192 x 8192): MFMAs alone 1670 TFLOP/s at the clock the chip's power leaves, with the fragment reads
-// 1450, with the fetches 1190 ... 1220 (a library's product: 1350 ... 1510).  Reads and fetches in bursts behind the barrier cost 10 % more
-// than spread between the MFMAs; four waves with twice the fragments each read a third less LDS and were slower (1160); workgroups
-// ordered by rows alone, without bands, 900.  Small tiles are bound by how long a fetch takes: three steps in LDS against two
-// bring 128 x 128 from 545 to 760, 128 x 256 from 890 to 1050.
+// What bounds it: 8192 x 8192 x 8192 in 256 x 256 tiles runs at 1190 ... 1400 TFLOP/s on different boxes (a library's product: 1350 ... 1626).  The
+// matrix cores are busy 71 % of the clocks, fragment reads have no bank conflicts, and a wave spends the rest at the barrier of a step and on its
+// reads; 2048 x 19456 x 2560 177 us = 1153 TFLOP/s (the library's 188), busy 50 %, the last round of tiles included.  Reads and fetches in bursts
+// behind the barrier cost 10 % more than spread between the MFMAs; four waves with twice the fragments each read a third less LDS and were slower
+// (1160 where this has 1200); workgroups ordered by rows alone, without bands, 900.  Small tiles are bound by how long a fetch takes: three
+// steps in LDS against two bring 128 x 128 from 545 to 760, 128 x 256 from 890 to 1050.
 #pragma once
 #include "gemm_plan.h"
 #include "ptm_common.h"
@@ -20,7 +21,6 @@ namespace ptm {
 typedef float gt_f4 __attribute__((ext_vector_type(4)));
 typedef int gt_i4 __attribute__((ext_vector_type(4)));
 typedef __bf16 gt_b8 __attribute__((ext_vector_type(8)));
-
 
 // 16 bytes per lane from base + voff + soff to LDS bytes [lds, lds + 1024), lane after lane
 __device__ __forceinline__ void gt_to_lds(uint32_t lds, int voff, gt_i4 base, int soff) {

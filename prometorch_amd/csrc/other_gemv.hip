@@ -5,9 +5,10 @@
 //
 // slots_gemv_kernel: a lane takes 8 values of a row (16 of a Q5_K block: both nibbles of its bytes) at a time, so that neighbouring lanes read
 // neighbouring pieces of x and of the row, and a wave several rows, so that x is loaded once for all of them; two passes over the row are
-// requested together.  Bound by requests in flight: Q8_0 9728 x 2560 9.0 us = 2.9 TB/s, 30000 x 2560 23 us = 3.5 TB/s, 300 x 1024 1.9 us (19.4,
-// 51.5 and 2.4 with a lane per run of 32 values, as the exact Q4_K kernel below still has it: x and the row are then read in pieces 128
-// and 34 bytes apart, and every load instruction touches 64 cache lines).
+// requested together.  Bound by requests in flight: Q8_0 with weights from HBM, in a graph, 9728 x 2560 9.1 us = 2.9 TB/s, 30000 x 2560 19.5 us =
+// 4.2 TB/s, 500 x 1024 2.3 us (19.1, 50.1 and 2.6 with a lane per run of 32 values, as the exact Q4_K kernel below still has it: x and the
+// row are then read in pieces 128 and 34 bytes apart, and every load instruction touches 64 cache lines); 9728 x 2560 called again and again on
+// weights that the caches hold 7.6 us (18.1).
 #include "ptm_common.h"
 
 #include <type_traits>
