@@ -54,6 +54,10 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
 int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool accumulate, const float* gamma, float eps,
                                   int add_one, void* ws_round, void* ws_plain, int M, int K, hipStream_t s);
 int qgemm_f16_splits(int N, int K, int M);
+void qgemm_f16_row_workspace(void* workspace, int M, int K, void** rows, float** rowscale);
+int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
+                           bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
+                           float scale, int kv_fp16, int window, hipStream_t s);
 size_t qgemm_f16_multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M);
 void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits);
 int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const int64_t* strides, const int* N, float* const* Y,
@@ -444,13 +448,19 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
                                                    L.v_cache, local ? d->rope_swa : d->rope, M, c.n_heads, c.n_kv_heads, hd,
                                                    pos0, c.max_seq, c.rms_eps, 0, c.kv_fp16, c.rope_interleaved, s));
         }
-        PTM_TRY(ptm_prefill_attention_window(d->pf_q, L.k_cache, L.v_cache, d->pf_attn, M, c.n_heads, c.n_kv_heads, hd, pos0,
-                                             c.max_seq, 1.0f / sqrtf((float)hd), c.kv_fp16, local ? c.swa_window : 0, s));
+        // the matrix-core attention leaves its rows as the o-projection reads them
+        void* o_rows;
+        float* o_scales;
+        bool o_ready;
+        qgemm_f16_row_workspace(ws_of(L.o), M, qd, &o_rows, &o_scales);
+        PTM_TRY(prefill_attention_rows(d->pf_q, L.k_cache, L.v_cache, d->pf_attn, o_rows, o_scales, L.o.ggml_type == PTM_TYPE_Q4_K, &o_ready,
+                                       M, c.n_heads, c.n_kv_heads, hd, pos0, c.max_seq, 1.0f / sqrtf((float)hd), c.kv_fp16,
+                                       local ? c.swa_window : 0, s));
         if (L.post_attn_norm) {
-            PTM_TRY(gemm(L.o, d->pf_attn, d->pf_h, false, false));
+            PTM_TRY(gemm(L.o, d->pf_attn, d->pf_h, false, o_ready));
             PTM_TRY(ptm_rms_norm_add(d->pf_h, L.post_attn_norm, d->pf_x, M, H, c.rms_eps, 0, s));
         } else {
-            PTM_TRY(gemm(L.o, d->pf_attn, d->pf_x, true, false, H <= 12288 ? &pending : nullptr));  // x += attn . Wo^T
+            PTM_TRY(gemm(L.o, d->pf_attn, d->pf_x, true, o_ready, H <= 12288 ? &pending : nullptr));  // x += attn . Wo^T
         }
         PTM_TRY(norm_rows(pending, L.ffn_norm, uses(PTM_TYPE_Q4_K, {&L.gate, &L.up}), uses(PTM_TYPE_Q6_K, {&L.gate, &L.up})));
         pending = 0;
@@ -494,7 +504,7 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
             PTM_TRY(gemm(L.down, d->pf_gate, d->pf_x, true, act_ready, (li + 1 < c.n_layers && H <= 12288) ? &pending : nullptr));
         }
     }
-    (void)qd; (void)kvd;
+    (void)kvd;
     return PTM_OK;
 #undef PTM_TRY
 }

@@ -450,6 +450,14 @@ __device__ __forceinline__ pf_h4 lds_read_tr16(const uint8_t* p) {
 }
 typedef float pf_f16v __attribute__((ext_vector_type(16)));
 
+// where the rows of the matrix-core kernel go: fp32, or fp16 with their scales (see there)
+struct PrefillAttnOut {
+    float* O;
+    _Float16* rows16;
+    float* rowscale;
+    int q8round;
+};
+
 // v_mfma_f32_32x32x16_f16 operand layout used below: A (32 x 16): lane l holds row l % 32, summation indices
 // 8 (l / 32) + 0..7; B (16 x 32): lane l holds column l % 32, the same indices; C (32 x 32): lane l holds column
 // l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4 for r = 0..15.  The summation index may be permuted freely as long as A
@@ -468,9 +476,14 @@ typedef float pf_f16v __attribute__((ext_vector_type(16)));
 // only one half of the output's head dimension, staging the tiles together.  A wave with the whole 256-wide output would
 // need 128 accumulator registers beside 64 of q fragments and 64 of tile pieces in flight: one wave per SIMD; with the
 // output split a SIMD holds two, and the repeated score MFMAs (half of a tile's work) cost less than the idle pipes would.
+// out.rows16: the rows go out as the fp16 rows of the product that follows (rounded to Q8 blocks of 32 first where that product's
+// weights are Q4_K), not as fp32 rows that a launch of its own reads and converts: a Q8 block is an accumulator tile's 32 dimensions,
+// which two lanes hold, so its maximum is one exchange away.  Their scale is 1: an average of fp16 values fits fp16 as it is.
+// Against the conversion launch, 36 layers of Qwen3-4B shapes: 19 tokens 3343 -> 3240 us, 509 9139 -> 8945; 16 of Llama-3-8B's, 3001 tokens
+// 31276 -> 30899.
 template <int HD, int G, int NG, int DS = 1>
 __global__ __launch_bounds__(256 * NG * DS) void prefill_attn_mfma_kernel(const float* __restrict__ Q, const __half* __restrict__ Kc,
-                                                                const __half* __restrict__ Vc, float* __restrict__ O, int rows,
+                                                                const __half* __restrict__ Vc, const PrefillAttnOut out, int rows,
                                                                 int n_heads, int n_kv_heads, int64_t pos0, float scale, int window) {
     constexpr int GP = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;   // head slots per row
     constexpr int RPW = 32 / GP;       // rows per wave (each with its GP head slots: 32 query vectors)
@@ -722,8 +735,49 @@ __global__ __launch_bounds__(256 * NG * DS) void prefill_attn_mfma_kernel(const 
     }
     const float l = l_run + __shfl_xor(l_run, 32, 64);
     const float inv = 1.0f / (l + 1e-10f);  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
-    if (row < rows && !dead) {
-        float* dst = O + ((int64_t)row * n_heads + head) * HD + 32 * DT * dh + 4 * kh;
+    const bool stored = row < rows && !dead;
+    if (out.rows16) {
+        if (stored && head == 0 && kh == 0 && dh == 0) out.rowscale[row] = 1.0f;
+        _Float16* dst = out.rows16 + ((int64_t)row * n_heads + head) * HD + 32 * DT * dh + 8 * kh;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = acc[dt][r] * inv;
+            if (out.q8round) {  // the arithmetic of q8_quantize4
+                float amax = fabsf(v[0]);
+#pragma unroll
+                for (int r = 1; r < 16; ++r) amax = fmaxf(amax, fabsf(v[r]));
+                amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+                const float d = amax / 127.0f;
+                const float id = d > 0.0f ? 1.0f / d : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) v[r] = d * (float)max(-127, min(127, (int)rintf(v[r] * id)));
+            }
+            // a lane has dimensions 8 q + 4 kh .. +3 of quarter q; quarters 2 p and 2 p + 1 are exchanged between the lane halves so that
+            // each stores eight dimensions in a row
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                union { _Float16 h[4]; uint32_t u[2]; } a, b;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    a.h[i] = (_Float16)v[8 * p + i];
+                    b.h[i] = (_Float16)v[8 * p + 4 + i];
+                }
+                uint32_t w[4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const auto x = __builtin_amdgcn_permlane32_swap(a.u[i], b.u[i], false, false);
+                    w[i] = x[0];
+                    w[2 + i] = x[1];
+                }
+                if (stored) *reinterpret_cast<uint4*>(dst + 32 * dt + 16 * p) = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        return;
+    }
+    if (stored) {
+        float* dst = out.O + ((int64_t)row * n_heads + head) * HD + 32 * DT * dh + 4 * kh;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -734,7 +788,7 @@ __global__ __launch_bounds__(256 * NG * DS) void prefill_attn_mfma_kernel(const 
 }
 
 template <int HD>
-static int prefill_attn_mfma_launch(int G, hipStream_t s, const float* Q, const void* Kc, const void* Vc, float* O, int rows,
+static int prefill_attn_mfma_launch(int G, hipStream_t s, const float* Q, const void* Kc, const void* Vc, const PrefillAttnOut& out, int rows,
                                     int n_heads, int n_kv_heads, int64_t pos0, float scale, int window) {
     const int gp = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
     const int bm = 128 / gp;
@@ -749,13 +803,13 @@ static int prefill_attn_mfma_launch(int G, hipStream_t s, const float* Q, const 
 #define PTM_PA(GG)                                                                                                          \
     if constexpr (HD == 256)                                                                                                \
         hipLaunchKernelGGL((prefill_attn_mfma_kernel<HD, GG, 1, 2>), grid, dim3(512), 0, s, Q, static_cast<const __half*>(Kc), \
-                           static_cast<const __half*>(Vc), O, rows, n_heads, n_kv_heads, pos0, scale, window);              \
+                           static_cast<const __half*>(Vc), out, rows, n_heads, n_kv_heads, pos0, scale, window);              \
     else if (one)                                                                                                                \
         hipLaunchKernelGGL((prefill_attn_mfma_kernel<HD, GG, 1>), grid, dim3(256), 0, s, Q, static_cast<const __half*>(Kc), \
-                           static_cast<const __half*>(Vc), O, rows, n_heads, n_kv_heads, pos0, scale, window);              \
+                           static_cast<const __half*>(Vc), out, rows, n_heads, n_kv_heads, pos0, scale, window);              \
     else                                                                                                                    \
         hipLaunchKernelGGL((prefill_attn_mfma_kernel<HD, GG, 2>), grid, dim3(512), 0, s, Q, static_cast<const __half*>(Kc), \
-                           static_cast<const __half*>(Vc), O, rows, n_heads, n_kv_heads, pos0, scale, window)
+                           static_cast<const __half*>(Vc), out, rows, n_heads, n_kv_heads, pos0, scale, window)
     switch (G) {
         case 1: PTM_PA(1); break;
         case 2: PTM_PA(2); break;
@@ -814,6 +868,42 @@ int qknorm_rope_kv_rows_from_parts(const float* const* P, const int* splits, con
                                             head_dim, pos0, eps, add_one, kv_fp16, rope_interleaved, parts, s);
 }
 
+// Causal attention of `rows` prompt rows.  rows16 / rowscale (optional): where the matrix-core kernel serves the call, the rows are
+// left as the fp16 rows of the next product (rounded to Q8 blocks first when q8round) and *wrote16 is set; O has them otherwise.
+int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
+                           bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
+                           float scale, int kv_fp16, int window, hipStream_t s) {
+    if (!Q || !K_cache || !V_cache || !O) return PTM_E_NULL;
+    if (rows <= 0 || n_heads <= 0 || n_kv_heads <= 0 || max_seq <= 0 || (n_heads % n_kv_heads) != 0) return PTM_E_SHAPE;
+    if (head_dim != 64 && head_dim != 128 && head_dim != 256) return PTM_E_UNSUPPORTED;
+    if (pos0 < 0 || pos0 + rows > max_seq) return PTM_E_RANGE;
+    if (!aligned16(Q) || !aligned16(K_cache) || !aligned16(V_cache) || !aligned16(O)) return PTM_E_ALIGN;
+    if (n_kv_heads > 65535) return PTM_E_UNSUPPORTED;
+    const int G = n_heads / n_kv_heads;
+    const dim3 grid((rows + 3) / 4, n_kv_heads);
+    if (window < 0) window = 0;
+    // the MFMA kernel addresses the caches with 32-bit byte offsets (computed for up to two tiles past the last position
+    // before they are clamped)
+    const bool offsets_fit = (pos0 + rows + 64) * (int64_t)n_kv_heads * head_dim * 2 < ((int64_t)1 << 32);
+    const bool mfma = kv_fp16 && offsets_fit && rows >= PTM_PREFILL_MFMA_MIN_ROWS && G <= 8;
+    const PrefillAttnOut out = {O, static_cast<_Float16*>(rows16), rowscale, q8round ? 1 : 0};
+    if (wrote16) *wrote16 = mfma && rows16;
+    if (head_dim == 256) {  // wide heads (gemma3)
+        if (mfma)
+            return prefill_attn_mfma_launch<256>(G, s, Q, K_cache, V_cache, out, rows, n_heads, n_kv_heads, pos0, scale, window);
+        return kv_fp16 ? prefill_attn_launch<true, 256>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
+                       : prefill_attn_launch<false, 256>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
+    }
+    if (mfma)
+        return head_dim == 128 ? prefill_attn_mfma_launch<128>(G, s, Q, K_cache, V_cache, out, rows, n_heads, n_kv_heads, pos0, scale, window)
+                               : prefill_attn_mfma_launch<64>(G, s, Q, K_cache, V_cache, out, rows, n_heads, n_kv_heads, pos0, scale, window);
+    if (kv_fp16)
+        return head_dim == 128 ? prefill_attn_launch<true, 128>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
+                               : prefill_attn_launch<true, 64>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
+    return head_dim == 128 ? prefill_attn_launch<false, 128>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
+                           : prefill_attn_launch<false, 64>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
+}
+
 }  // namespace ptm
 
 using namespace ptm;
@@ -854,33 +944,8 @@ int ptm_prefill_attention(const float* Q, const void* K_cache, const void* V_cac
 int ptm_prefill_attention_window(const float* Q, const void* K_cache, const void* V_cache, float* O, int rows, int n_heads,
                                  int n_kv_heads, int head_dim, int64_t pos0, int max_seq, float scale, int kv_fp16,
                                  int window, ptm_stream_t stream) {
-    if (!Q || !K_cache || !V_cache || !O) return PTM_E_NULL;
-    if (rows <= 0 || n_heads <= 0 || n_kv_heads <= 0 || max_seq <= 0 || (n_heads % n_kv_heads) != 0) return PTM_E_SHAPE;
-    if (head_dim != 64 && head_dim != 128 && head_dim != 256) return PTM_E_UNSUPPORTED;
-    if (pos0 < 0 || pos0 + rows > max_seq) return PTM_E_RANGE;
-    if (!aligned16(Q) || !aligned16(K_cache) || !aligned16(V_cache) || !aligned16(O)) return PTM_E_ALIGN;
-    if (n_kv_heads > 65535) return PTM_E_UNSUPPORTED;
-    const int G = n_heads / n_kv_heads;
-    const dim3 grid((rows + 3) / 4, n_kv_heads);
-    hipStream_t s = as_stream(stream);
-    if (window < 0) window = 0;
-    // the MFMA kernel addresses the caches with 32-bit byte offsets (computed for up to two tiles past the last position
-    // before they are clamped)
-    const bool offsets_fit = (pos0 + rows + 64) * (int64_t)n_kv_heads * head_dim * 2 < ((int64_t)1 << 32);
-    if (head_dim == 256) {  // wide heads (gemma3)
-        if (kv_fp16 && offsets_fit && rows >= PTM_PREFILL_MFMA_MIN_ROWS && G <= 8)
-            return prefill_attn_mfma_launch<256>(G, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
-        return kv_fp16 ? prefill_attn_launch<true, 256>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
-                       : prefill_attn_launch<false, 256>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
-    }
-    if (kv_fp16 && offsets_fit && rows >= PTM_PREFILL_MFMA_MIN_ROWS && G <= 8)
-        return head_dim == 128 ? prefill_attn_mfma_launch<128>(G, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
-                               : prefill_attn_mfma_launch<64>(G, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
-    if (kv_fp16)
-        return head_dim == 128 ? prefill_attn_launch<true, 128>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
-                               : prefill_attn_launch<true, 64>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
-    return head_dim == 128 ? prefill_attn_launch<false, 128>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window)
-                           : prefill_attn_launch<false, 64>(G, grid, s, Q, K_cache, V_cache, O, rows, n_heads, n_kv_heads, pos0, scale, window);
+    return prefill_attention_rows(Q, K_cache, V_cache, O, nullptr, nullptr, false, nullptr, rows, n_heads, n_kv_heads, head_dim, pos0,
+                                  max_seq, scale, kv_fp16, window, as_stream(stream));
 }
 
 }  // extern "C"

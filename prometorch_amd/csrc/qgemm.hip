@@ -1042,6 +1042,12 @@ static int qgemm_check(const void* W, const void* X, const void* Y, int M, int K
     return PTM_OK;
 }
 
+// where the M rows of K values and their scales lie in a row workspace
+void qgemm_f16_row_workspace(void* workspace, int M, int K, void** rows, float** rowscale) {
+    *rows = workspace;
+    *rowscale = reinterpret_cast<float*>(static_cast<_Float16*>(workspace) + (int64_t)qf_mpad(M) * K);
+}
+
 // Y (+)= X . W^T with X bf16 or fp32 rows; shared by the C entry points and the prefill runtime.
 int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f32, float* Y, int M, int K, int N,
                    int64_t stride, void* workspace, bool accumulate, float* split_ws, size_t split_ws_bytes, bool reuse_rows,

@@ -1,7 +1,14 @@
 // Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
-// splits, which the C ABI's plain product does not have, and how a launch would cover its output.  Host C++ only; built by
+// splits, which the C ABI's plain product does not have, how a launch would cover its output, and the quantised models' prompt attention
+// as theirs calls it.  Host C++ only; built by
 // __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
 #include "gemm_plan.h"
+
+namespace ptm {
+int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
+                           bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
+                           float scale, int kv_fp16, int window, hipStream_t s);
+}
 
 extern "C" {
 
@@ -51,6 +58,16 @@ void gemm_plan(const GemmCall* c, int32_t* out) {
         const ptm::GemmRegion& r = p.regions.r[i];
         for (int v : {r.kind, r.first, r.m0, r.n0, r.n1, r.tiles_m, r.tiles_n}) *out++ = v;
     }
+}
+
+// prompt attention that leaves the rows of the next product; *wrote: whether it did (else O has the rows)
+int prefill_rows16(const float* Q, const void* K, const void* V, float* O, void* rows16, float* rowscale, int q8round, int* wrote, int rows,
+                   int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq, float scale, int kv_fp16, int window, void* stream) {
+    bool w = false;
+    const int rc = ptm::prefill_attention_rows(Q, K, V, O, rows16, rowscale, q8round != 0, &w, rows, n_heads, n_kv_heads, head_dim, pos0,
+                                               max_seq, scale, kv_fp16, window, static_cast<hipStream_t>(stream));
+    *wrote = w ? 1 : 0;
+    return rc;
 }
 
 }  // extern "C"

@@ -15,6 +15,8 @@ rms 3e-3..7e-3 of the logits' spread for 2 and for 36 layers).  test_q8_rounding
 the same growth inside the CPU oracle alone when its input embedding is perturbed by the fp16 GEMM's error.  The
 end-to-end bars are therefore on that scale: logits rms within E2E_RMS_TOL and max within E2E_MAX_TOL of the spread
 of the oracle's logits, greedy tokens identical wherever the oracle's top-2 margin exceeds twice the logit error."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -177,6 +179,41 @@ def test_prefill_attention_vs_oracle(dev, po, kv_fp16, nh, nkv, hd, pos0, rows):
     e = np.abs(got - want).max() / np.abs(want).max()
     print("attention nh %d nkv %d hd %d pos0 %d rows %d fp16 %s: max err / max %.2e" % (nh, nkv, hd, pos0, rows, kv_fp16, e), flush=True)
     assert e <= (1e-3 if kv_fp16 and rows >= 16 else 1e-4)
+
+
+@pytest.mark.parametrize("q8round", [1, 0])
+@pytest.mark.parametrize("kv_fp16,nh,nkv,hd,pos0,rows,window", [(1, 4, 4, 64, 0, 16, 0), (1, 16, 2, 128, 3, 40, 0), (1, 28, 4, 128, 700, 33, 0), (1, 12, 2, 64, 520, 31, 50),
+                                                                (1, 8, 4, 256, 0, 130, 0), (1, 6, 2, 256, 1200, 45, 100), (1, 4, 2, 64, 0, 15, 0), (0, 4, 2, 64, 0, 20, 0)])
+def test_prefill_attention_as_rows_of_the_next_product(dev, kv_fp16, nh, nkv, hd, pos0, rows, window, q8round):
+    """The fp16 rows the matrix-core kernel leaves are its fp32 rows (Q8-rounded where the product asks for it), bit for bit; other calls
+    leave fp32 rows and say so.  Nothing is written past the last row."""
+    from gemm_helpers import harness
+    r = synth.rng_for(72, nh, hd, pos0, rows)
+    max_seq, kvd, qd = pos0 + rows, nkv * hd, nh * hd
+    dt = torch.float16 if kv_fp16 else torch.float32
+    Kc, Vc = cu(r.standard_normal((max_seq, kvd), dtype=np.float32)).to(dt), cu(r.standard_normal((max_seq, kvd), dtype=np.float32)).to(dt)
+    Vc[:, 0] = 60000.0  # no scale for rows beyond 2^14: an average of fp16 values fits fp16
+    Vc[:, hd - 32:hd] = 0.0  # a Q8 block of zeros
+    Q = cu(r.standard_normal((rows, qd), dtype=np.float32))
+    O = torch.full((rows, qd), 9.0, device="cuda")
+    ops.prefill_attention_window(Q, Kc, Vc, O, rows, nh, nkv, hd, pos0, max_seq, hd ** -0.5, bool(kv_fp16), window)
+    rows16, scale = torch.full((rows + 1, qd), 7.0, dtype=torch.float16, device="cuda"), torch.full((rows + 1,), 7.0, device="cuda")
+    O2, wrote = torch.full((rows, qd), 9.0, device="cuda"), ctypes.c_int32(-1)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert harness().prefill_rows16(p(Q), p(Kc), p(Vc), p(O2), p(rows16), p(scale), q8round, ctypes.byref(wrote), rows, nh, nkv, hd, ctypes.c_int64(pos0),
+                                    max_seq, ctypes.c_float(hd ** -0.5), kv_fp16, window, None) == 0
+    torch.cuda.synchronize()
+    v = O.cpu().numpy()
+    if not kv_fp16 or rows < 16:
+        assert wrote.value == 0 and np.array_equal(bits(O2.cpu().numpy()), bits(v))
+        return
+    assert wrote.value == 1 and bool((scale[:rows] == 1).all()) and float(scale[rows]) == 7.0 and bool((rows16[rows] == 7).all())
+    if q8round:
+        b = v.reshape(rows, -1, 32)
+        d = np.abs(b).max(axis=2, keepdims=True) / np.float32(127)
+        inv = np.divide(np.float32(1), d, out=np.zeros_like(d), where=d > 0)
+        v = (d * np.clip(np.rint(b * inv), -127, 127).astype(np.int32).astype(np.float32)).reshape(rows, qd)
+    assert np.array_equal(rows16[:rows].cpu().numpy().view(np.uint16), v.astype(np.float16).view(np.uint16))
 
 
 def test_prefill_attention_rejects_bad_shapes(dev):
