@@ -33,17 +33,19 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 
-// block-wide sum for WAVES waves; red: WAVES floats of LDS
-template <int WAVES>
-__device__ __forceinline__ float block_sum(float v, float* red) {
+// block-wide sum for `waves` waves; red: `waves` floats of LDS
+__device__ __forceinline__ float block_sum(float v, float* red, int waves) {
     v = sum64(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     float s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) s += red[w];
+    for (int w = 0; w < waves; ++w) s += red[w];
     return s;
+}
+template <int WAVES>
+__device__ __forceinline__ float block_sum(float v, float* red) {
+    return block_sum(v, red, WAVES);
 }
 
 enum { GEMV_STORE = 0, GEMV_RELU2 = 1, GEMV_SIDE = 2, GEMV_ARGMAX = 3, GEMV_SWIGLU = 4 };
@@ -58,17 +60,22 @@ constexpr int GEMV_SECTIONS = 8;
 // With tail_n > 0 (no other prologue), values tail0 .. of x are RMS-normed in tail_parts equal parts, times tail_norm * tail_scale.
 // GEMV_SWIGLU: W holds N gate rows, then N up rows; y = silu(gate) * up.
 struct DenseGemv {
+    // what a plain product reads lies in one cache line of kernel arguments, a norm's vectors in the next: a line first read late in the
+    // kernel is a round trip to memory there
     const uint16_t* W = nullptr;
+    const float* x = nullptr;
+    float* y = nullptr;
     int64_t ld = 0;
     int N = 0, K = 0;
-    const float* x = nullptr;
+    int epilogue = GEMV_STORE;
+    float out_scale = 1.0f;          // factor of every stored y
+    int waves = 0, wgs = 0;          // of the launch, set by dense_gemv
+    float eps = 0.0f;
+    int sections = 0;
     const float *h = nullptr, *hw = nullptr, *add0 = nullptr, *add1 = nullptr;
     float* xout = nullptr;
     const float* gamma = nullptr;
     float* xn_out = nullptr;
-    float eps = 0.0f;
-    int epilogue = GEMV_STORE;
-    float* y = nullptr;
     const uint16_t* side = nullptr;  // GEMV_SIDE: row *d_token of the table, from column side_off
     int64_t side_ld = 0;
     int side_off = 0;
@@ -81,13 +88,11 @@ struct DenseGemv {
     const float* mu = nullptr;       // [sections][padded K]
     float* shift = nullptr;          // [2][padded K], by position parity
     const int64_t* d_past = nullptr;
-    int sections = 0;
     int section_row[GEMV_SECTIONS + 1] = {};  // first rows; the last entry is N
     int section_wg[GEMV_SECTIONS + 1] = {};   // first workgroups, set by dense_gemv
     int tail0 = 0, tail_n = 0, tail_parts = 0;
     const float* tail_norm = nullptr;
     float tail_scale = 1.0f;
-    float out_scale = 1.0f;          // factor of every stored y
 };
 int dense_gemv_workgroups(const DenseGemv& g);
 int dense_gemv(DenseGemv g, hipStream_t s);

@@ -1,16 +1,25 @@
 // Decode products over bfloat16 weights: y = W . x with fp32 activations, and the two products a latent-attention step
 // makes around its attention.
 //
-// dense_gemv_kernel: 8 waves per workgroup; LPR lanes share a row (64; fewer for short rows), each taking 8 values (16 bytes)
-// per chunk, R rows x U chunks in flight per lane, the next batch requested before the current one is consumed.  The
-// activation vector lies in LDS as fp32, the two halves of every 8 values in separate planes so that a wave's 16-byte reads
-// are consecutive.  The first weight batch is requested before the prologue, which forms the vector: deferred post-norm and
-// residual add, loop inputs, RMSNorm - recomputed by every workgroup, as the quantised kernels do.
+// dense_gemv_kernel: LPR lanes share a row (64; fewer for short rows), each taking 8 values (16 bytes) per chunk.  A wave walks the chunks
+// of its rows one after the other with D of them in flight, whatever row they belong to: a consumed chunk's registers are refilled at
+// once with the one D further on, and the last D are consumed without a refill.  The activation vector lies in LDS as fp32, the two
+// halves of every 8 values in separate planes so that a wave's 16-byte reads are consecutive.  The first chunks are requested before
+// the prologue, which forms the vector: deferred post-norm and residual add, loop inputs, RMSNorm - recomputed by every workgroup, as the
+// quantised kernels do.  A finished row's sum stays in a lane of its own; what follows it (activation, table row, argmax) runs on up
+// to 64 of them at a time.
+// What bounds it is HBM: 16 waves per CU with 4 or 5 KB in flight each reach what a plain read of the same bytes does, and more in
+// flight is slower (requests past the last row cost the texture path as much as others).  Weights from HBM, in a graph, against batches of 8
+// chunks of up to four rows with the next batch ahead, and that read: 2560 x 9728 14.1 -> 10.7 us (10.1), 9728 x 2560 12.5 -> 9.7 (10.1),
+// 19456 x 2560 20.5 -> 18.0 (18.1), 4096 x 14336 25.1 -> 23.0, 8192 x 2560 10.7 -> 8.9, 2560 x 2560 5.7 -> 5.2 (4.7), 1024 x 2816 3.56 -> 3.55 (3.0).
 #include "dense.h"
+
+#include <type_traits>
 
 namespace ptm {
 
-constexpr int DG_WAVES = 8, DG_THREADS = 64 * DG_WAVES;
+constexpr int DG_WAVES = 8, DG_THREADS = 64 * DG_WAVES;  // of a workgroup whose prologue has a norm or streams
+constexpr int DG_MAX_WAVES = 16;                         // of others
 
 __device__ __forceinline__ float4 ld4(const float* p, int i) { return reinterpret_cast<const float4*>(p)[i]; }
 __device__ __forceinline__ float sq4(float4 v, float s) {
@@ -105,24 +114,22 @@ __device__ __forceinline__ void stream_prologue(const DenseGemv& a, int sec, flo
         finish(i, a.mu ? ld4(a.shift + ((pos & 1) ^ 1) * Kp, i) : make_float4(0.f, 0.f, 0.f, 0.f));
 }
 
-// The vector with its tail normed in equal parts; s_r: one float per part.  AT(e): element e of the vector in LDS.
-template <typename Put, typename At>
-__device__ __forceinline__ void tail_prologue(const DenseGemv& a, float* s_r, float* red, Put put, At at) {
-    const int tid = threadIdx.x, Kp = (a.K + 63) & ~63, n4 = Kp / 4, part = a.tail_n / a.tail_parts;
-    for (int i = tid; i < n4; i += DG_THREADS) put(i, ld4(a.x, i));
-    __syncthreads();
+// Norms the tail of the vector in equal parts; s_r: one float per part.  AT(e): element e of the vector in LDS.
+template <typename At>
+__device__ __forceinline__ void tail_prologue(const DenseGemv& a, float* s_r, float* red, At at) {
+    const int tid = threadIdx.x, nt = 64 * a.waves, part = a.tail_n / a.tail_parts;
     if (a.tail_parts <= 4) {
         for (int p = 0; p < a.tail_parts; ++p) {
             float ss = 0.0f;
-            for (int e = tid; e < part; e += DG_THREADS) {
+            for (int e = tid; e < part; e += nt) {
                 const float v = *at(a.tail0 + p * part + e);
                 ss = fmaf(v, v, ss);
             }
-            ss = block_sum<DG_WAVES>(ss, red);
+            ss = block_sum(ss, red, nt >> 6);
             if (tid == 0) s_r[p] = 1.0f / sqrtf(ss / (float)part + a.eps);
         }
     } else {
-        for (int p = tid >> 6; p < a.tail_parts; p += DG_WAVES) {
+        for (int p = tid >> 6; p < a.tail_parts; p += nt >> 6) {
             float ss = 0.0f;
             for (int e = tid & 63; e < part; e += 64) {
                 const float v = *at(a.tail0 + p * part + e);
@@ -133,24 +140,26 @@ __device__ __forceinline__ void tail_prologue(const DenseGemv& a, float* s_r, fl
         }
     }
     __syncthreads();
-    for (int e = tid; e < a.tail_n; e += DG_THREADS) {
+    for (int e = tid; e < a.tail_n; e += nt) {
         float* v = at(a.tail0 + e);
         *v = *v * s_r[e / part] * a.tail_norm[e] * a.tail_scale;
     }
 }
 
 // PRO: what forms the vector - 0: nothing, 1: residual and RMS norm, 2: streams, 3: the tail's norm
-template <int LPR, int R, int U, int PRO, bool GLU>
-__global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGemv a) {
-    static_assert(!GLU || R % 2 == 0, "a lane holds the gate and the up row of a value");
+template <int LPR, int D, int PRO, bool GLU>
+__global__ __launch_bounds__(PRO == 1 || PRO == 2 ? DG_THREADS : 64 * DG_MAX_WAVES, 4) void dense_gemv_kernel(const DenseGemv a) {
     extern __shared__ __align__(16) float4 s_x[];  // [2][Kp / 8]
-    __shared__ float red[DG_WAVES];
-    __shared__ int redi[DG_WAVES];
-    constexpr int RPP = 64 / LPR, RW = GLU ? RPP * R / 2 : RPP * R;
+    __shared__ float red[DG_MAX_WAVES];
+    __shared__ int redi[DG_MAX_WAVES];
+    constexpr int RPP = 64 / LPR;
+    static_assert(D <= LPR, "a lane for every row a pass can finish");
+    const int waves = PRO == 1 || PRO == 2 ? DG_WAVES : a.waves, nt = 64 * waves;
+    asm volatile("" ::"s"(a.x), "s"(a.y), "s"(a.epilogue), "s"(a.out_scale));  // read now, with the rest of their line
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane % LPR, lr = lane / LPR;
     const int Kp = (a.K + 63) & ~63, n4 = Kp / 4, n8 = Kp / 8;
-    int sec = 0, row0 = 0, rows = a.N, wg = blockIdx.x, wgs = gridDim.x;
+    int sec = 0, row0 = 0, rows = a.N, wg = blockIdx.x, wgs = a.wgs;
     if constexpr (PRO == 2) {
         if (a.sections > 0) {
             while (sec + 1 < a.sections && wg >= a.section_wg[sec + 1]) ++sec;
@@ -160,43 +169,59 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
             rows = a.section_row[sec + 1] - row0;
         }
     }
-    const int groups = (rows + RW - 1) / RW, stride = wgs * DG_WAVES;
-    const int nb = (n8 + LPR * U - 1) / (LPR * U);
+    const int groups = (rows + RPP - 1) / RPP, stride = wgs * waves, g0 = wg * waves + wave;
+    const int nc = (n8 + LPR - 1) / LPR;  // chunks of a row
     const uint32_t bytes = (uint32_t)((int64_t)a.N * a.ld * (GLU ? 4 : 2));
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.W, (int)bytes);
-    auto load = [&](int g, int b, u32x4* w) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            int row;
-            if constexpr (GLU) row = min(g * RW + r / 2 * RPP + lr, rows - 1) + (r & 1) * rows;
-            else row = row0 + min(g * RW + r * RPP + lr, rows - 1);
-            const uint32_t base = (uint32_t)row * (uint32_t)(a.ld * 2);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int kk = (b * U + u) * LPR + li;
-                w[r * U + u] = __builtin_amdgcn_raw_buffer_load_b128(rs, kk < n8 ? base + (uint32_t)kk * 16u : bytes, 0, 0);
-            }
+    u32x4 w[D];
+    int lg = g0, lc = 0, lh = 0;  // the next chunk to request: of which rows, which, of the gate or the up row
+    auto request = [&](u32x4& v) {
+        int row;
+        if constexpr (GLU) row = min(lg * RPP + lr, rows - 1) + lh * rows;
+        else row = row0 + min(lg * RPP + lr, rows - 1);
+        const int kk = lc * LPR + li;
+        v = __builtin_amdgcn_raw_buffer_load_b128(rs, kk < n8 && lg < groups ? (uint32_t)row * (uint32_t)(a.ld * 2) + (uint32_t)kk * 16u : bytes, 0, 0);
+        if (++lc == nc) {
+            lc = 0;
+            if (GLU && lh == 0) { lh = 1; }
+            else { lh = 0; lg += stride; }
         }
+    };
+    auto first_chunks = [&]() {
+#pragma unroll
+        for (int i = 0; i < D; ++i) request(w[i]);
     };
     auto put = [&](int i, float4 v) { s_x[(i & 1) * n8 + (i >> 1)] = v; };
 
-    u32x4 cur[R * U], nxt[R * U];
-    int g = wg * DG_WAVES + wave, b = 0;
     auto at = [&](int e) { return reinterpret_cast<float*>(s_x + ((e >> 2) & 1) * n8 + (e >> 3)) + (e & 3); };
     if constexpr (PRO == 2) {
-        load(min(g, groups - 1), 0, cur);
+        first_chunks();  // in front of the prologue's own requests: behind them 8450 -> 8535 us for the 24 steps of a Nadozen turn
         issue_order_fence();
         stream_prologue(a, sec, red, put, [&](int i) { return s_x[(i & 1) * n8 + (i >> 1)]; });
         __syncthreads();
-    } else if constexpr (PRO == 3) {
-        load(min(g, groups - 1), 0, cur);
-        issue_order_fence();
-        tail_prologue(a, reinterpret_cast<float*>(s_x + 2 * n8), red, put, at);
+    } else if constexpr (PRO == 3 || PRO == 0) {
+        // the vector's first pieces are requested in front of the weights (loads return in order) and without a branch (static load counts)
+        const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, n4 * 16);
+        auto stage = [&](auto pieces) {
+            constexpr int P = decltype(pieces)::value;
+            u32x4 xv[P];
+#pragma unroll
+            for (int u = 0; u < P; ++u) xv[u] = __builtin_amdgcn_raw_buffer_load_b128(rx, min(tid + u * nt, n4) * 16, 0, 0);
+            issue_order_fence();
+            first_chunks();
+            issue_order_fence();
+#pragma unroll
+            for (int u = 0; u < P; ++u)
+                if (tid + u * nt < n4) put(tid + u * nt, __builtin_bit_cast(float4, xv[u]));
+            for (int i = tid + P * nt; i < n4; i += nt) put(i, ld4(a.x, i));
+        };
+        if (n4 <= 2 * nt) stage(std::integral_constant<int, 2>{});
+        else stage(std::integral_constant<int, 4>{});
         __syncthreads();
-    } else if constexpr (PRO == 0) {
-        for (int i = tid; i < n4; i += DG_THREADS) put(i, ld4(a.x, i));
-        load(min(g, groups - 1), 0, cur);
-        __syncthreads();
+        if constexpr (PRO == 3) {
+            tail_prologue(a, reinterpret_cast<float*>(s_x + 2 * n8), red, at);
+            __syncthreads();
+        }
     } else {
         const bool first = blockIdx.x == 0;
         if (n4 <= 2 * DG_THREADS) {  // the vector stays in registers between the passes
@@ -214,7 +239,7 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
                 }
             }
             issue_order_fence();
-            load(min(g, groups - 1), 0, cur);
+            first_chunks();
             if (a.h) {
                 const float r = 1.0f / sqrtf(block_sum<DG_WAVES>(sq4(hv[1], sq4(hv[0], 0.f)), red) / (float)a.K + a.eps);
 #pragma unroll
@@ -235,7 +260,7 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
                 }
             }
         } else {  // long vectors: kept in LDS between the passes
-            load(min(g, groups - 1), 0, cur);
+            first_chunks();
             float rh = 0.0f;
             if (a.h) {
                 float ss = 0.0f;
@@ -272,61 +297,72 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
     const int64_t side_row = a.epilogue == GEMV_SIDE ? (int64_t)*a.d_token * a.side_ld + a.side_off : 0;
     float best = -INFINITY;
     int best_i = 0x7fffffff;
-    float acc[R], glu_gate = 0.0f;
+    float acc = 0.0f, sums = 0.0f, gates = 0.0f;  // lane li of a row's lanes keeps the sum of the li-th finished row
+    int c = 0, half = 0, done = 0, gd = g0;
+    auto finish = [&]() {
+        const int row = (gd + li * stride) * RPP + lr;
+        if (li < done && row < rows) {
+            float v = sums;
+            if constexpr (GLU) {
+                v = silu_f(gates) * v;
+            } else {
+                v *= a.out_scale;
+                if (a.epilogue == GEMV_RELU2) v = v > 0.0f ? v * v : 0.0f;
+                else if (a.epilogue == GEMV_SIDE) v = gelu_tanh(v) * bf16_f(a.side[side_row + row0 + row]);
+                else if (a.epilogue == GEMV_ARGMAX && (v > best || (v == best && row0 + row < best_i))) { best = v; best_i = row0 + row; }
+            }
+            a.y[row0 + row] = v;
+        }
+        gd += done * stride;
+        done = 0;
+    };
+    auto consume = [&](u32x4& v) {
+        const int kc = min(c * LPR + li, n8 - 1);  // a chunk past the end holds zero weights
+        const float4 x0 = s_x[kc], x1 = s_x[n8 + kc];
+        float t = acc;
+        t = fmaf(bf16_lo(v.x), x0.x, t);
+        t = fmaf(bf16_hi(v.x), x0.y, t);
+        t = fmaf(bf16_lo(v.y), x0.z, t);
+        t = fmaf(bf16_hi(v.y), x0.w, t);
+        t = fmaf(bf16_lo(v.z), x1.x, t);
+        t = fmaf(bf16_hi(v.z), x1.y, t);
+        t = fmaf(bf16_lo(v.w), x1.z, t);
+        t = fmaf(bf16_hi(v.w), x1.w, t);
+        acc = t;
+    };
+    auto end_chunk = [&]() {
+        if (++c < nc) return;
+        const float v = LPR == 64 ? sum64(acc) : sum_lanes<LPR == 64 ? 32 : LPR>(acc);
+        c = 0;
+        acc = 0.0f;
+        if (GLU && half == 0) {
+            gates = li == done ? v : gates;
+            half = 1;
+        } else {
+            sums = li == done ? v : sums;
+            half = 0;
+            ++done;
+        }
+    };
+    const int passes = g0 < groups ? (((groups - 1 - g0) / stride + 1) * (GLU ? 2 : 1) * nc + D - 1) / D : 0;
+    for (int p = 1; p <= passes; ++p) {
+        if (done + D > LPR) finish();
+        if (p < passes) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-    while (g < groups) {
-        const bool last = b + 1 == nb;
-        const int ng = last ? g + stride : g, nbb = last ? 0 : b + 1;
-        if (ng < groups) load(ng, nbb, nxt);
+            for (int i = 0; i < D; ++i) {
+                consume(w[i]);
+                request(w[i]);
+                end_chunk();
+            }
+        } else {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int kk = (b * U + u) * LPR + li, kc = min(kk, n8 - 1);  // a chunk past the end holds zero weights
-            const float4 x0 = s_x[kc], x1 = s_x[n8 + kc];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const u32x4 w = cur[r * U + u];
-                float t = acc[r];
-                t = fmaf(bf16_lo(w.x), x0.x, t);
-                t = fmaf(bf16_hi(w.x), x0.y, t);
-                t = fmaf(bf16_lo(w.y), x0.z, t);
-                t = fmaf(bf16_hi(w.y), x0.w, t);
-                t = fmaf(bf16_lo(w.z), x1.x, t);
-                t = fmaf(bf16_hi(w.z), x1.y, t);
-                t = fmaf(bf16_lo(w.w), x1.z, t);
-                t = fmaf(bf16_hi(w.w), x1.w, t);
-                acc[r] = t;
+            for (int i = 0; i < D; ++i) {
+                consume(w[i]);
+                end_chunk();
             }
         }
-        if (last) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                float v = LPR == 64 ? sum64(acc[r]) : sum_lanes<LPR == 64 ? 32 : LPR>(acc[r]);
-                acc[r] = 0.0f;
-                if constexpr (GLU) {
-                    const int pair = g * RW + r / 2 * RPP + lr;
-                    if (r & 1) {
-                        if (li == 0 && pair < rows) a.y[pair] = glu_gate * v;
-                    } else {
-                        glu_gate = silu_f(v);
-                    }
-                    continue;
-                }
-                const int row = row0 + g * RW + r * RPP + lr;
-                if (li == 0 && row < row0 + rows) {
-                    v *= a.out_scale;
-                    if (a.epilogue == GEMV_RELU2) v = v > 0.0f ? v * v : 0.0f;
-                    else if (a.epilogue == GEMV_SIDE) v = gelu_tanh(v) * bf16_f(a.side[side_row + row]);
-                    else if (a.epilogue == GEMV_ARGMAX && (v > best || (v == best && row < best_i))) { best = v; best_i = row; }
-                    a.y[row] = v;
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < R * U; ++i) cur[i] = nxt[i];
-        g = ng;
-        b = nbb;
     }
+    finish();
     if (a.epilogue == GEMV_ARGMAX) {
         for (int off = 1; off < 64; off <<= 1) {
             const float ov = __shfl_xor(best, off, 64);
@@ -337,8 +373,8 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
         if (lane == 0) { red[wave] = best; redi[wave] = best_i; }
         __syncthreads();
         if (tid == 0) {
-            for (int w = 1; w < DG_WAVES; ++w)
-                if (red[w] > best || (red[w] == best && redi[w] < best_i)) { best = red[w]; best_i = redi[w]; }
+            for (int i = 1; i < waves; ++i)
+                if (red[i] > best || (red[i] == best && redi[i] < best_i)) { best = red[i]; best_i = redi[i]; }
             a.part_val[blockIdx.x] = best;
             a.part_idx[blockIdx.x] = best_i;
         }
@@ -346,23 +382,29 @@ __global__ __launch_bounds__(DG_THREADS, 4) void dense_gemv_kernel(const DenseGe
 }
 
 namespace {
-struct GemvShape { int kind, rows_per_wave; };
-// rows shorter than a wave's 512 values share a wave; long rows take more chunks of one row, short ones more rows
+struct GemvShape { int lpr, depth, waves, wgs; };
+int gemv_prologue(const DenseGemv& g) {
+    return g.streams > 0 ? 2 : g.tail_n > 0 ? 3 : g.h || g.add0 || g.add1 || g.gamma || g.xout || g.xn_out ? 1 : 0;
+}
+// Rows shorter than a wave's 512 values share a wave.  Up to 16 rows per CU: one workgroup a CU with a wave for each (8 at least), so that
+// the vector is staged once per CU and no CU has two rows a wave where another has one (2560 x 9728 on 320 workgroups of 8 waves 12.8 us,
+// on 256 of 10 11.4); a prologue with a norm or streams has 8 waves, the threads of its sums.  More rows: two workgroups of 8 waves a CU.
+// A wave with up to 6 chunks requests them all at once; in other cases the chunks in flight are the 4 or 5 that leave fewer requests
+// past a wave's last row (8 in flight where a wave has 8: 4096 x 4096 9.2 us, 8.5 with 4).
 GemvShape gemv_shape(const DenseGemv& g) {
-    const int kp = up64(g.K), ch = (kp + 511) / 512;
-    const bool glu = g.epilogue == GEMV_SWIGLU;
-    if (kp <= 64) return {0, glu ? 16 : 32};
-    if (kp <= 256) return {1, glu ? 4 : 8};
-    if (glu) return ch <= 2 ? GemvShape{2, 2} : GemvShape{3, 1};
-    const bool few = g.N <= 2 * DG_WAVES * 256;  // two rows per wave would leave compute units without work
-    if (ch <= 2) return few ? GemvShape{5, 1} : GemvShape{2, 4};
-    if (ch <= 4 || (ch <= 7 && !few)) return few ? GemvShape{5, 1} : GemvShape{3, 2};
-    return {4, 1};
+    const int kp = up64(g.K), lpr = kp <= 64 ? 8 : kp <= 256 ? 32 : 64, pro = gemv_prologue(g);
+    const int groups = (int)(((int64_t)g.N * lpr + 63) / 64), per_cu = (groups + 255) / 256;
+    const int waves = pro == 1 || pro == 2 || per_cu > DG_MAX_WAVES || per_cu < DG_WAVES ? DG_WAVES : per_cu;
+    int wgs = (groups + waves - 1) / waves;
+    wgs = wgs < 512 ? wgs : 512;
+    const int chunks = (groups + wgs * waves - 1) / (wgs * waves) * ((kp / 8 + lpr - 1) / lpr) * (g.epilogue == GEMV_SWIGLU ? 2 : 1);
+    const int depth = chunks == 6 ? 6 : (4 - chunks % 4) % 4 < (5 - chunks % 5) % 5 ? 4 : 5;
+    return {lpr, lpr < 64 && depth > 5 ? 5 : depth, waves, wgs};
 }
 // At most 512 workgroups (one more would run by itself behind the others): as many as its rows fill for a section of few rows,
 // the rest over the others by their rows.
 void section_workgroups(DenseGemv& g) {
-    const int per = gemv_shape(g).rows_per_wave * DG_WAVES;
+    const int per = 64 / gemv_shape(g).lpr * DG_WAVES;
     int64_t room = 512, rows_left = 0;
     auto rows = [&](int i) { return (int64_t)(g.section_row[i + 1] - g.section_row[i]); };
     auto fill = [&](int i) { return (rows(i) + per - 1) / per; };
@@ -379,27 +421,19 @@ void section_workgroups(DenseGemv& g) {
 }
 }  // namespace
 
-int dense_gemv_workgroups(const DenseGemv& g) {
-    const int groups = (g.N + gemv_shape(g).rows_per_wave - 1) / gemv_shape(g).rows_per_wave;
-    const int wgs = (groups + DG_WAVES - 1) / DG_WAVES;
-    return wgs < 512 ? wgs : 512;
-}
+int dense_gemv_workgroups(const DenseGemv& g) { return gemv_shape(g).wgs; }
 
 template <int PRO>
 static void gemv_attr() {
     const int lds = 150 * 1024;
 #define PTM_DG(...) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(dense_gemv_kernel<__VA_ARGS__>), hipFuncAttributeMaxDynamicSharedMemorySize, lds)
-    PTM_DG(8, 4, 1, PRO, false);
-    PTM_DG(32, 4, 1, PRO, false);
-    PTM_DG(64, 4, 2, PRO, false);
-    PTM_DG(64, 2, 4, PRO, false);
-    PTM_DG(64, 1, 8, PRO, false);
-    PTM_DG(64, 1, 4, PRO, false);
+    PTM_DG(64, 4, PRO, false);
+    PTM_DG(64, 5, PRO, false);
+    PTM_DG(64, 6, PRO, false);
     if constexpr (PRO < 3) {
-        PTM_DG(8, 4, 1, PRO, true);
-        PTM_DG(32, 4, 1, PRO, true);
-        PTM_DG(64, 4, 2, PRO, true);
-        PTM_DG(64, 2, 4, PRO, true);
+        PTM_DG(64, 4, PRO, true);
+        PTM_DG(64, 5, PRO, true);
+        PTM_DG(64, 6, PRO, true);
     }
 #undef PTM_DG
 }
@@ -411,30 +445,23 @@ void dense_gemv_init() {
     gemv_attr<3>();
 }
 
-template <int PRO>
-static void gemv_launch(const DenseGemv& g, dim3 grid, size_t lds, hipStream_t s) {
-    const dim3 block(DG_THREADS);
-#define PTM_DG(...) hipLaunchKernelGGL((dense_gemv_kernel<__VA_ARGS__>), grid, block, lds, s, g)
-    if constexpr (PRO < 3) {
-        if (g.epilogue == GEMV_SWIGLU) {
-            switch (gemv_shape(g).kind) {
-                case 0: PTM_DG(8, 4, 1, PRO, true); break;
-                case 1: PTM_DG(32, 4, 1, PRO, true); break;
-                case 2: PTM_DG(64, 4, 2, PRO, true); break;
-                default: PTM_DG(64, 2, 4, PRO, true); break;
-            }
-            return;
-        }
-    }
-    switch (gemv_shape(g).kind) {
-        case 0: PTM_DG(8, 4, 1, PRO, false); break;
-        case 1: PTM_DG(32, 4, 1, PRO, false); break;
-        case 2: PTM_DG(64, 4, 2, PRO, false); break;
-        case 3: PTM_DG(64, 2, 4, PRO, false); break;
-        case 4: PTM_DG(64, 1, 8, PRO, false); break;
-        default: PTM_DG(64, 1, 4, PRO, false); break;
-    }
+template <int PRO, bool GLU>
+static void gemv_launch(const DenseGemv& g, const GemvShape& sh, dim3 grid, size_t lds, hipStream_t s) {
+    const dim3 block(64 * sh.waves);
+#define PTM_DG(...) hipLaunchKernelGGL((dense_gemv_kernel<__VA_ARGS__, PRO, GLU>), grid, block, lds, s, g)
+    if (sh.lpr == 8) { if (sh.depth == 4) PTM_DG(8, 4); else PTM_DG(8, 5); }
+    else if (sh.lpr == 32) { if (sh.depth == 4) PTM_DG(32, 4); else PTM_DG(32, 5); }
+    else if (sh.depth == 4) PTM_DG(64, 4);
+    else if (sh.depth == 5) PTM_DG(64, 5);
+    else PTM_DG(64, 6);
 #undef PTM_DG
+}
+template <int PRO>
+static void gemv_launch(const DenseGemv& g, const GemvShape& sh, dim3 grid, size_t lds, hipStream_t s) {
+    if constexpr (PRO < 3) {
+        if (g.epilogue == GEMV_SWIGLU) return gemv_launch<PRO, true>(g, sh, grid, lds, s);
+    }
+    gemv_launch<PRO, false>(g, sh, grid, lds, s);
 }
 
 int dense_gemv(DenseGemv g, hipStream_t s) {
@@ -449,21 +476,24 @@ int dense_gemv(DenseGemv g, hipStream_t s) {
             if (g.section_row[i + 1] <= g.section_row[i]) return PTM_E_SHAPE;
         section_workgroups(g);
     }
-    const dim3 grid(g.sections > 0 ? g.section_wg[g.sections] : dense_gemv_workgroups(g));
+    const GemvShape sh = gemv_shape(g);
+    g.waves = sh.waves;
+    g.wgs = g.sections > 0 ? g.section_wg[g.sections] : sh.wgs;
+    const dim3 grid(g.wgs);
     const size_t lds = (size_t)up64(g.K) * 4;
     if (g.streams > 0) {
         if (!g.blend || (g.store && !g.xout) || (g.mu && (!g.shift || !g.d_past)) || (g.beta && !g.gamma)) return PTM_E_NULL;
         if (g.x_stride & 3) return PTM_E_ALIGN;
-        gemv_launch<2>(g, grid, lds, s);
+        gemv_launch<2>(g, sh, grid, lds, s);
     } else if (g.tail_n > 0) {
         if (!g.tail_norm) return PTM_E_NULL;
         if (g.tail_parts <= 0 || g.tail_n % g.tail_parts || g.tail0 + g.tail_n > g.K) return PTM_E_SHAPE;
         if (g.epilogue == GEMV_SWIGLU || g.tail_parts > 512) return PTM_E_UNSUPPORTED;
-        gemv_launch<3>(g, grid, lds + (size_t)g.tail_parts * 4, s);
-    } else if (g.h || g.add0 || g.add1 || g.gamma || g.xout || g.xn_out) {
-        gemv_launch<1>(g, grid, lds, s);
+        gemv_launch<3>(g, sh, grid, lds + (size_t)g.tail_parts * 4, s);
+    } else if (gemv_prologue(g) == 1) {
+        gemv_launch<1>(g, sh, grid, lds, s);
     } else {
-        gemv_launch<0>(g, grid, lds, s);
+        gemv_launch<0>(g, sh, grid, lds, s);
     }
     return launch_status();
 }

@@ -329,6 +329,24 @@ def test_dense_gemv(dev, N, K):
     assert np.abs(y[:N] - ref).max() < 2e-6 * np.sqrt(K) * np.abs(ref).std() + 1e-5 and (y[N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("N,K", [(270000, 64), (270000, 200), (270000, 300), (2305, 2560), (2049, 600), (4095, 3072), (4097, 3072), (3000, 9728), (1024, 2816), (9001, 1024)])
+def test_dense_gemv_many_rows(dev, N, K):
+    """Waves with more finished rows than lanes to keep their sums, workgroups of 9 to 16 waves, and each count of chunks in flight."""
+    import torch
+    L = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    kp = (K + 63) // 64 * 64
+    W = torch.zeros(N, kp, dtype=torch.bfloat16, device="cuda")
+    W[:, :K] = torch.randn(N, K, device="cuda", generator=g)
+    x = torch.zeros(kp, device="cuda")
+    x[:K] = torch.randn(K, device="cuda", generator=g)
+    y = torch.full((N + 3,), 7.0, device="cuda")
+    _lib.check(L.ptm_dense_gemv(W.data_ptr(), x.data_ptr(), y.data_ptr(), K, N, kp, None), "gemv")
+    ref = W.double() @ x.double()
+    # the bound of test_dense_gemv
+    assert float((y[:N] - ref).abs().max()) < 2e-6 * K ** 0.5 * float(ref.std()) + 1e-5 and bool((y[N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("fp32", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1, 3, 8), (2, 70, 40), (31, 257, 100), (33, 65, 320), (64, 64, 64), (100, 130, 192),
                                    (150, 1000, 72), (300, 4100, 200), (1030, 2050, 136)])
