@@ -407,11 +407,7 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
         }
     }
     auto slots = [](float x) {  // over the lanes with equal lane % 8
-        x += dpp_f<0x128>(x);  // row_ror:8
-        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-        x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-        r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        return add32(add16(x + dpp_f<0x128>(x)));  // row_ror:8
     };
     sum = make_float4(slots(sum.x), slots(sum.y), slots(sum.z), slots(sum.w));
     if (together) {
@@ -785,16 +781,12 @@ __device__ __forceinline__ fd_h4 fd_lds_read_tr16(const uint8_t* p) {
 }
 // max / sum over the four 16-lane rows of the wave (lanes with equal lane % 16), result in every lane
 __device__ __forceinline__ float fd_rows_max(float v) {
-    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    LanePair p = pair32(v);
+    p = pair16(fmaxf(p.a, p.b));
+    return fmaxf(p.a, p.b);
 }
 __device__ __forceinline__ float fd_rows_sum(float v) {
-    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    return add16(add32(v));
 }
 
 template <int HD, int G, int TPW, bool BIAS = false>

@@ -284,7 +284,8 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
         for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[u][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const LanePair p = pair32(mx);
+        mx = fmaxf(p.a, p.b);
         const float m_new = fmaxf(m_run, mx), ms = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet
         const float corr = __builtin_amdgcn_exp2f(m_run - ms);
         float psum = 0.0f;
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
                 }
             }
     }
-    const float inv = 1.0f / (l_run + __shfl_xor(l_run, 32, 64));
+    const float inv = 1.0f / (add32(l_run));
     if (!live) return;
     uint16_t* dst = static_cast<uint16_t*>(a.O) + (int64_t)row * a.o_row + (int64_t)head * a.vdim + 4 * kh;
 #pragma unroll
@@ -578,8 +579,9 @@ __global__ __launch_bounds__(256, 1) void decode_mfma_kernel(const DecodeAttenti
             sc[r] = sees(past, k0 + 4 * rg + r, a.window, a.keep_first) ? v : -INFINITY;
             mx = fmaxf(mx, sc[r]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        LanePair p = pair16(mx);
+        p = pair32(fmaxf(p.a, p.b));
+        mx = fmaxf(p.a, p.b);
         if (rg == 0) s_m[wave][j] = mx;
         __syncthreads();
         const float m_new = fmaxf(m_run, fmaxf(fmaxf(s_m[0][j], s_m[1][j]), fmaxf(s_m[2][j], s_m[3][j])));
@@ -617,8 +619,7 @@ __global__ __launch_bounds__(256, 1) void decode_mfma_kernel(const DecodeAttenti
             }
         }
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = add32(add16(l_run));
     if (rg == 0) s_l[wave][j] = l_run;
     __syncthreads();
     if (j >= nh) return;

@@ -225,21 +225,15 @@ __global__ __launch_bounds__(256) void slots_gemv_kernel(const uint8_t* __restri
             }
         }
     }
-#pragma unroll
-    for (int i = 0; i < R; ++i) acc[i] = sum64(acc[i]);
+    float v = sum_rows<R>(acc);
+    const int i = sum_row<R>(lane);
     if constexpr (C > 1) {
-        if (lane == 0)
-#pragma unroll
-            for (int i = 0; i < R; ++i) part[wave][i] = acc[i];
+        if ((lane & (64 / R - 1)) == 0) part[wave][i] = v;
         __syncthreads();
-#pragma unroll
-        for (int i = 0; i < R; ++i) acc[i] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
         if (wave > 0) return;
+        v = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
     }
-    if (lane == 0)
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            if (r0 + i < N) y[r0 + i] = ACC ? y[r0 + i] + acc[i] : acc[i];
+    if ((lane & (64 / R - 1)) == 0 && r0 + i < N) y[r0 + i] = ACC ? y[r0 + i] + v : v;
 }
 
 template <typename Fmt>

@@ -650,7 +650,10 @@ __global__ __launch_bounds__(256 * NG * DS) void prefill_attn_mfma_kernel(const 
         asm("v_max_f32 %0, %0, %1" : "+v"(mx) : "v"(sc[1][0]));
 #pragma unroll
         for (int r = 1; r < 16; ++r) asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx) : "v"(sc[0][r]), "v"(sc[1][r]));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));  // the column's other positions
+        {
+            const LanePair p = pair32(mx);  // the column's other positions
+            mx = fmaxf(p.a, p.b);
+        }
         const float m_new = fmaxf(m_run, mx);
         // group 1 may have seen no visible position of a query yet (-inf): exponentials then take 0 as the reference and are 0
         const float ms = m_new == -INFINITY ? 0.0f : m_new;
@@ -733,7 +736,7 @@ __global__ __launch_bounds__(256 * NG * DS) void prefill_attn_mfma_kernel(const 
         l_run = fmaf(l_run, c0, l1 * c1);
     }
     }
-    const float l = l_run + __shfl_xor(l_run, 32, 64);
+    const float l = add32(l_run);
     const float inv = 1.0f / (l + 1e-10f);  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
     const bool stored = row < rows && !dead;
     if (out.rows16) {

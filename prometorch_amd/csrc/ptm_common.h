@@ -66,12 +66,27 @@ __device__ __forceinline__ float sum16(float v) {
     v += dpp_f<0x140>(v);
     return v;
 }
-// all-reduce over each half of the wave (lanes 0..31, 32..63)
-__device__ __forceinline__ float sum32(float v) {
-    v = sum16(v);
-    v += __shfl_xor(v, 16, 64);
-    return v;
+// The two values of a lane pair 16 / 32 lanes apart, in every lane of the pair the same way round: a lane swap, which is a vector
+// instruction where a shuffle is a trip through LDS.
+struct LanePair { float a, b; };
+__device__ __forceinline__ LanePair pair16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
 }
+__device__ __forceinline__ LanePair pair32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ float add16(float v) {
+    const LanePair p = pair16(v);
+    return p.a + p.b;
+}
+__device__ __forceinline__ float add32(float v) {
+    const LanePair p = pair32(v);
+    return p.a + p.b;
+}
+// all-reduce over each half of the wave (lanes 0..31, 32..63)
+__device__ __forceinline__ float sum32(float v) { return add16(sum16(v)); }
 // sum over groups of LPP = 8, 16 or 32 consecutive lanes
 template <int LPP>
 __device__ __forceinline__ float sum_lanes(float v) {
@@ -82,17 +97,35 @@ __device__ __forceinline__ float sum_lanes(float v) {
 }
 // all-reduce over the whole wave64
 __device__ __forceinline__ float sum64(float v) {
-    v = sum16(v);
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    return v;
+    return add32(sum32(v));
+}
+// The sums over the wave of R = 1, 2 or 4 values in one go: a swap of two registers halves them both.  Lane l has that of value sum_row<R>(l).
+template <int R>
+__device__ __forceinline__ float sum_rows(const float (&v)[R]) {
+    static_assert(R == 1 || R == 2 || R == 4, "registers that halve evenly");
+    auto fold32 = [](float a, float b) {  // lanes 0..31: a, 32..63: b
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    if constexpr (R == 1) {
+        return sum64(v[0]);
+    } else if constexpr (R == 2) {
+        return sum32(fold32(v[0], v[1]));
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(fold32(v[0], v[1])), __float_as_uint(fold32(v[2], v[3])), false, false);
+        return sum16(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+    }
+}
+template <int R>
+__device__ __forceinline__ int sum_row(int lane) {
+    return R == 1 ? 0 : R == 2 ? lane >> 5 : (lane >> 5) + 2 * ((lane >> 4) & 1);
 }
 __device__ __forceinline__ float max64(float v) {
     v = max8(v);
     v = fmaxf(v, dpp_f<0x140>(v));
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    v = fmaxf(v, __shfl_xor(v, 32, 64));
-    return v;
+    LanePair p = pair16(v);
+    p = pair32(fmaxf(p.a, p.b));
+    return fmaxf(p.a, p.b);
 }
 
 // ---- fp16 ---------------------------------------------------------------------------

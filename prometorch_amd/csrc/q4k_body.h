@@ -352,15 +352,15 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
         // reduce: 8 lanes of the group, then the S groups of the row
         float p = sum8(acc);
         if (S >= 2) p += dpp_f<0x128>(p);  // row_ror:8 = the other 8-lane half of the 16-lane row
-        if (S >= 4) p += __shfl_xor(p, 16, 64);
-        if (S >= 8) p += __shfl_xor(p, 32, 64);
+        if (S >= 4) p = add16(p);
+        if (S >= 8) p = add32(p);
 
         if constexpr (MODE == 1) {
-            // gate and up of one row sit S groups apart
+            // gate and up of one row sit S groups apart, the gate in the lower lanes
             float other;
             if (S == 1) other = dpp_f<0x128>(p);
-            else if (S == 2) other = __shfl_xor(p, 16, 64);
-            else other = __shfl_xor(p, 32, 64);
+            else if (S == 2) other = pair16(p).b;
+            else other = pair32(p).b;
             if (live && mat == 0 && sub == 0 && j == 0) a.y[0][local] = a.gelu ? gelu_mul_ref(p, other) : silu_mul_ref(p, other);
         } else {
             float* y = mat == 0 ? a.y[0] : (mat == 1 ? a.y[1] : a.y[2]);
@@ -423,14 +423,14 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
             }
             float p = sum8(acc);
             if (S >= 2) p += dpp_f<0x128>(p);
-            if (S >= 4) p += __shfl_xor(p, 16, 64);
-            if (S >= 8) p += __shfl_xor(p, 32, 64);
+            if (S >= 4) p = add16(p);
+            if (S >= 8) p = add32(p);
             if constexpr (MODE == 1) {
-                // gate and up of one row sit S groups apart
+                // gate and up of one row sit S groups apart, the gate in the lower lanes
                 float other;
                 if (S == 1) other = dpp_f<0x128>(p);
-                else if (S == 2) other = __shfl_xor(p, 16, 64);
-                else other = __shfl_xor(p, 32, 64);
+                else if (S == 2) other = pair16(p).b;
+                else other = pair32(p).b;
                 if (r < total_rows && (r & 1) == 0 && sub == 0 && j == 0)
                     y0[r >> 1] = a.gelu ? gelu_mul_ref(p, other) : silu_mul_ref(p, other);
             } else {

@@ -114,8 +114,8 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
     }
     float p = sum8(acc);
     p += dpp_f<0x128>(p);
-    p += __shfl_xor(p, 16, 64);
-    p += __shfl_xor(p, 32, 64);
+    p = add16(p);
+    p = add32(p);
     if (live && lane == 0) {
         if constexpr (ACC) y[r] += p;
         else y[r] = p;

@@ -181,8 +181,8 @@ __device__ __forceinline__ void q6k_gemv_body(const Q6KArgs a, uint8_t* lds_raw,
     }
     float p = sum8(acc);
     if (S >= 2) p += dpp_f<0x128>(p);
-    if (S >= 4) p += __shfl_xor(p, 16, 64);
-    if (S >= 8) p += __shfl_xor(p, 32, 64);
+    if (S >= 4) p = add16(p);
+    if (S >= 8) p = add32(p);
     if (live && sub == 0 && j == 0 && a.y) {
         if constexpr (ACC) a.y[rr] += p;
         else a.y[rr] = p;

@@ -130,8 +130,8 @@ __global__ __launch_bounds__(64 * MAXW) void q6k_gemv_tall_kernel(const Q6KArgs 
     // same reduction order as q6k_gemv_body
     float p = sum8(acc);
     p += dpp_f<0x128>(p);
-    p += __shfl_xor(p, 16, 64);
-    if (S >= 8) p += __shfl_xor(p, 32, 64);
+    p = add16(p);
+    if (S >= 8) p = add32(p);
     if (live && sub == 0 && j == 0) {
         if constexpr (ACC) a.y[rr] += p;
         else a.y[rr] = p;

@@ -283,8 +283,8 @@ __device__ __forceinline__ void q6k_mfma_gemv_body(const Q6KArgs a, uint8_t* lds
             acc = fmaf(h2f(k.d), t, acc);
         }
     }
-    acc += __shfl_xor(acc, 16, 64);   // the four quarters
-    acc += __shfl_xor(acc, 32, 64);
+    acc = add16(acc);   // the four quarters
+    acc = add32(acc);
     const float p = acc * down;   // row rl of the tile
     if (kq == 0 && live && a.y) {
         if constexpr (ACC) a.y[rr] += p;
