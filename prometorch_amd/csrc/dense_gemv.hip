@@ -155,7 +155,8 @@ __global__ __launch_bounds__(PRO == 1 || PRO == 2 ? DG_THREADS : 64 * DG_MAX_WAV
     constexpr int RPP = 64 / LPR;
     static_assert(D <= LPR, "a lane for every row a pass can finish");
     const int waves = PRO == 1 || PRO == 2 ? DG_WAVES : a.waves, nt = 64 * waves;
-    asm volatile("" ::"s"(a.x), "s"(a.y), "s"(a.epilogue), "s"(a.out_scale));  // read now, with the rest of their line
+    read_now(a.x, a.y, a.epilogue, a.out_scale);
+    if constexpr (PRO > 0) read_now(a.gamma, a.streams, a.d_past, a.section_wg[0], a.tail_n);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane % LPR, lr = lane / LPR;
     const int Kp = (a.K + 63) & ~63, n4 = Kp / 4, n8 = Kp / 8;

@@ -809,6 +809,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     __shared__ __align__(16) float s_o[4][HD][GP];
     __shared__ float s_m[4][GP], s_l[4][GP];
 
+    read_now(a.Q, a.n_heads, a.qb);
     const int64_t past = *a.d_past;
     if (past < 0 || past >= a.max_seq) return;          // never touch memory outside the cache
     const int64_t total = past + 1;
@@ -1143,6 +1144,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_long_kernel(const
     __shared__ __align__(16) float s_o[4][HD][GP];
     __shared__ float s_m[4][GP], s_l[4][GP];
 
+    read_now(a.Q, a.n_heads, a.qb);
     const int64_t past = *a.d_past;
     if (past < 0 || past >= a.max_seq) return;          // never touch memory outside the cache
     const int64_t total = past + 1;

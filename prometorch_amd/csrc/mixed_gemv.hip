@@ -12,6 +12,7 @@ namespace ptm {
 // workgroup 0, a Q6_K one, stores it)
 template <int NB4, int NB6, bool PRE = false>
 __global__ __launch_bounds__(256) void rmsnorm_mixed_gemv_kernel(const Q4KArgs a4, const Q6KArgs a6, int n6_wgs) {
+    read_now(a4.W[0], a4.K, a6.W, a6.gamma, n6_wgs);
     extern __shared__ __align__(16) uint8_t lds[];
     if ((int)blockIdx.x < n6_wgs) q6k_gemv_body<false, false, true, 1, NB6, PRE>(a6, lds, blockIdx.x);
     else q4k_gemv_body<false, true, false, 0, NB4, false, PRE>(a4, lds, (int)blockIdx.x - n6_wgs);

@@ -412,6 +412,7 @@ __device__ __forceinline__ float sumsq_part(const float* p, int n) {  // this th
 
 template <int DQ, int DV, bool RAW, bool V_IS_K>
 __global__ __launch_bounds__(256, 1) void decode_mfma_kernel(const DecodeAttention d, int splits) {
+    read_now(d.a.Q, d.d_past, d.raw, d.k_cache, d.pL, splits);
     constexpr int KS = DQ / 32, DW = DV / 64, QP = DQ * 2 + 16, VP = DV * 2 + 32, PV = V_IS_K ? 1 : DV / 32;
     __shared__ __align__(16) uint8_t s_q[2][16 * QP];
     __shared__ __align__(16) uint8_t s_v[64 * VP];
@@ -641,6 +642,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const float* __restri
                                                            const float* __restrict__ pL, int splits, const ptm_attention_args a,
                                                            float* __restrict__ out) {
     __shared__ float s_sum[4][64];
+    read_now(pO, a.heads, a.vdim, a.sink, a.out_scale, out);
     const int heads = a.heads, vdim = a.vdim;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = blockIdx.x, v = blockIdx.y * 64 + lane, vc = min(v, vdim - 1);
     const float sink = a.sink ? a.sink[h] : -INFINITY, factor = out_factor(a, 0, h, vc);

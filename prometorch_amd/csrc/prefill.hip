@@ -205,6 +205,7 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __r
                                                                       int n_heads, int n_kv_heads, int head_dim, int64_t pos0,
                                                                       float eps, int add_one, int rope_interleaved,
                                                                       const QkvParts parts) {
+    read_now(Q, n_heads, parts.P[0], parts.bias[2]);
     const int m = blockIdx.x, rows = gridDim.x;
     const int lph = head_dim >> 3, hpw = 64 / lph;  // lanes per head, heads per wave
     const int q_blocks = (n_heads + hpw - 1) / hpw;

@@ -27,6 +27,7 @@ namespace ptm {
 
 template <bool XQ8, bool NORM, bool ACC, int MODE, int NB>
 __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_kernel(const Q4KArgs a) {
+    read_now(a.W[0], a.K, a.gamma);
     extern __shared__ __align__(16) uint8_t lds[];
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB>(a, lds, blockIdx.x);
 }
@@ -34,6 +35,7 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_kernel(const Q4KArgs a) 
 // a workgroup walks several row tiles, every tile one pass of NB blocks per lane group: the passes roll across the tiles
 template <bool XQ8, bool NORM, bool ACC, int MODE, int NB>
 __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArgs a) {
+    read_now(a.W[0], a.K, a.gamma);
     extern __shared__ __align__(16) uint8_t lds[];
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB, true>(a, lds, blockIdx.x);
 }
@@ -47,6 +49,7 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArg
 // 6248 x 2560, 8.22 -> 7.89; 16 waves, 9.4 MB, 4096 x 1024, 6.22 -> 5.56).
 template <int NB, int NX>
 __global__ __launch_bounds__(1024) void q4k_gemv_wide_kernel(const Q4KArgs a) {
+    read_now(a.W[0], a.K, a.gamma, a.pre_h);
     extern __shared__ __align__(16) uint8_t lds[];
     q4k_gemv_body<false, true, false, 1, NB, false, false, NX>(a, lds, blockIdx.x);
 }

@@ -205,6 +205,7 @@ __global__ __launch_bounds__(1024) void argmax_partials_kernel(const float* pv, 
                                                                const ArgmaxAdvance adv) {
     __shared__ float bv[16];
     __shared__ int bi[16];
+    read_now(pv, adv.cap);
     int step = 0;
     int64_t past = 0;
     if (threadIdx.x == 0 && adv.d_token) {  // fetched now so that the tail below does not wait on them

@@ -879,6 +879,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_ke
                                                         const float* __restrict__ rowscale, float* Y, int M, int K, int N,
                                                         int accumulate, int blocks_per_split, float* partials) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(W, M);
     const int hw = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     const int L = qf_xcd_order(hw, gridDim.x * gridDim.y * gridDim.z);
     int bx, by, bz;
@@ -905,6 +906,7 @@ struct QfMulti { QfMat m[3]; int n_mat; };
 template <int MT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_multi_kernel(const QfMulti a, int M, int K) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(a.m[0].W, a.m[1].W, a.m[2].W, a.n_mat);
     const int L = qf_xcd_order(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
     int sx, by, unused;
     qf_tile_of(L, gridDim.x, gridDim.y, sx, by, unused);  // sx: the (matrix, split, column tile) slot
