@@ -16,6 +16,7 @@ namespace ptm {
 
 enum { FD_CHUNK = 64, FD_THREADS = 256 };
 enum { FD_LONG_SPLITS = 64 };   // partials per head of the looping kernel for long caches (attn_decode_mfma_long_kernel)
+enum { FD_ONE_WAVES = 8 };       // waves of a workgroup that holds every position of a cache (attn_decode_mfma_kernel, ONE)
 
 // e^x through the hardware base-2 exponential (v_exp_f32, 1 ulp): softmax weights need no more, and the libm
 // expf expands to a dozen instructions on a path whose cost is instruction count.  -inf gives 0.
@@ -488,6 +489,9 @@ struct AttnArgs {
     // biases of the q / k / v projections (qwen2, gguf_model.h:3419-3431), added to the raw vectors before norm and rotation
     // by the kernels instantiated with BIAS; null otherwise
     const float *qb, *kb, *vb;
+    // the finished output (fp32, and Q8 blocks where given) of the kernel that needs no merge
+    float* O;
+    uint8_t* q8;
 };
 
 // one wave: RMSNorm (optional) + NeoX rotation of a head held as pairs (t, t+HD/2); results to dst[HD]
@@ -789,8 +793,11 @@ __device__ __forceinline__ float fd_rows_sum(float v) {
     return add16(add32(v));
 }
 
-template <int HD, int G, int TPW, bool BIAS = false>
-__global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const AttnArgs a) {
+// ONE: a cache of up to 16 WAVES TPW positions in one workgroup per kv head, whose waves' partials are the splits: they are merged in LDS and the
+// output is finished here, as flash_decode_merge_kernel would.  Waves beyond the last position only help with the query heads. 32 heads of 128
+// over 20 positions: 2.9 us a layer less than the two launches, over 110 1.8.
+template <int HD, int G, int TPW, bool BIAS = false, int WAVES = 4, bool ONE = false>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(const AttnArgs a) {
     constexpr int HALF = HD / 2;
     constexpr int KS = HD / 32;          // QK steps (32 head-dim elements each)
     constexpr int DT = HD / 16;          // 16-wide tiles of the output's head dimension
@@ -799,19 +806,20 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     constexpr int VL = 16 / RPL;         // V loads per tile
     constexpr int VP = HD * 2 + 64;      // LDS pitch of a V row: the four rows of a transposing read fall on different banks
     constexpr int GP = G <= 4 ? 4 : 8;   // head slots of the wave partials
-    constexpr int CH = 64 * TPW;         // positions per workgroup
+    constexpr int CH = 16 * WAVES * TPW; // positions per workgroup
     constexpr int PP = (HALF + 63) / 64; // rotation pairs a lane holds in the prologue: pairs lane and (heads of 256) lane + 64
     static_assert(G >= 1 && G <= 8 && (HD == 64 || HD == 128 || (HD == 256 && G <= 4)) && (TPW == 1 || TPW == 2), "shape");
     __shared__ __align__(16) _Float16 s_qh[G][HD];
     __shared__ __align__(16) _Float16 s_ql[G][HD];
     __shared__ __align__(16) _Float16 s_nk[HD];
-    __shared__ __align__(16) uint8_t s_v[4][TPW][16 * VP];
-    __shared__ __align__(16) float s_o[4][HD][GP];
-    __shared__ float s_m[4][GP], s_l[4][GP];
+    __shared__ __align__(16) uint8_t s_v[WAVES][TPW][16 * VP];
+    __shared__ __align__(16) float s_o[WAVES][HD][GP];
+    __shared__ float s_m[WAVES][GP], s_l[WAVES][GP];
 
-    read_now(a.Q, a.n_heads, a.qb);
+    read_now(a.Q, a.n_heads, a.q8);
     const int64_t past = *a.d_past;
-    const int split = fd_split_of(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y), kvh = fd_head_of(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+    const int split = ONE ? 0 : fd_split_of(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+    const int kvh = ONE ? (int)blockIdx.x : fd_head_of(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, rg = lane >> 4;
     const int kv_dim = a.n_kv_heads * HD;
@@ -834,11 +842,11 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
         i0[p] = a.rope_interleaved ? 2 * lh[p] : lh[p];
         i1[p] = a.rope_interleaved ? 2 * lh[p] + 1 : lh[p] + HALF;
     }
-    constexpr int NQ = (G + 3) / 4;  // query heads a wave prepares: wave, wave + 4
+    constexpr int NQ = (G + WAVES - 1) / WAVES;  // query heads a wave prepares: wave, wave + WAVES
     float qx0[NQ][PP], qx1[NQ][PP], qb0[NQ][PP], qb1[NQ][PP];
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-        const int g = wave + 4 * n < G ? wave + 4 * n : 0;
+        const int g = wave + WAVES * n < G ? wave + WAVES * n : 0;
         const float* src = a.Q + (int64_t)(kvh * G + g) * HD;
 #pragma unroll
         for (int p = 0; p < PP; ++p) {
@@ -877,7 +885,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     const int64_t t_begin = (a.window > 0 && total > a.window) ? total - a.window : 0;
     if (t0 + CH <= t_begin) {
         // a chunk wholly in front of the window: an empty partial (weight 2^(-inf - M) = 0 in the merge)
-        for (int e = tid; e < G * HD; e += FD_THREADS) {
+        for (int e = tid; e < G * HD; e += 64 * WAVES) {
             const int g = e / HD, d = e % HD;
             const int64_t oi = (int64_t)split * a.n_heads + kvh * G + g;
             a.pO[oi * HD + d] = 0.0f;
@@ -886,6 +894,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
         return;
     }
     const int64_t wt0 = t0 + (int64_t)wave * (16 * TPW);            // first position of this wave
+    const bool active = !ONE || wt0 < total;                        // wave-uniform
     const bool owner = past >= wt0 && past < wt0 + 16 * TPW;       // wave-uniform: this wave's tiles hold the new position
     const float* cs = a.rope + past * HD;
 #pragma unroll
@@ -899,6 +908,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     const int64_t last_cached = past > 0 ? past - 1 : 0;
     const __half* Kh = static_cast<const __half*>(a.Kc) + (int64_t)kvh * HD;
     const __half* Vh = static_cast<const __half*>(a.Vc) + (int64_t)kvh * HD;
+    if (active) {
 #pragma unroll
     for (int u = 0; u < TPW; ++u) {
         const int64_t tk = wt0 + 16 * u + j;
@@ -915,6 +925,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
             const int64_t tvc = tv < past ? tv : last_cached;
             vreg[u][vl] = *reinterpret_cast<const uint4*>(Vh + tvc * kv_dim + 8 * (lane % LPR));
         }
+    }
     issue_order_fence();
 
     // ---- per-head RMSNorm + rotation of this wave's query heads, scaled into base-2 score units, as two fp16 terms ----
@@ -922,7 +933,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     const float qs = a.scale * 1.44269504088896340736f;
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-        const int g = wave + 4 * n;
+        const int g = wave + WAVES * n;
         if (g >= G) continue;  // wave-uniform
         float x0[PP], x1[PP];
         float ss = 0.0f;
@@ -996,6 +1007,7 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
     }
     __syncthreads();  // the query heads come from the other waves (the new row stays within its wave)
 
+    if (active) {
     // ---- B operands: head column j (columns past G repeat head 0), both terms ----
     fd_h8 qh[KS], ql[KS];
     {
@@ -1109,8 +1121,50 @@ __global__ __launch_bounds__(FD_THREADS) void attn_decode_mfma_kernel(const Attn
             *reinterpret_cast<float4*>(&s_o[wave][16 * dt + j][4 * rg]) = make_float4(acc[dt][0], acc[dt][1], acc[dt][2], acc[dt][3]);
     }
     if (rg == 0 && j < G) { s_m[wave][j] = m; s_l[wave][j] = l; }
+    }
     __syncthreads();
+    if constexpr (ONE) {
+        const int waves = (int)((total + 16 * TPW - 1) / (16 * TPW));
+        for (int e = tid; e < G * HD; e += 64 * WAVES) {  // whole waves: 32 lanes are a Q8 block
+            const int g = e / HD, d = e % HD;
+            // all reads at once; those of waves without positions are selected away, they may hold anything
+            float mw[WAVES], lw[WAVES], ow[WAVES];
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) {
+                mw[w] = s_m[w][g];
+                lw[w] = s_l[w][g];
+                ow[w] = s_o[w][d][g];
+            }
+            float M = mw[0], o = 0.0f, den = 0.0f;
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w) M = w < waves ? fmaxf(M, mw[w]) : M;  // finite: the new position is among them
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) {
+                const float f = __builtin_amdgcn_exp2f(mw[w] - M);
+                o = w < waves ? fmaf(f, ow[w], o) : o;
+                den = w < waves ? fmaf(f, lw[w], den) : den;
+            }
+            const float v = o * (1.0f / (den + 1e-10f));  // reference: inv_sum = 1/(sum_exp + 1e-10f), gguf_model.h:3589
+            const int at = kvh * G * HD + e;
+            a.O[at] = v;
+            if (a.q8) {  // the arithmetic of q8_quantize4
+                LanePair p = pair16(fmaxf(max8(fabsf(v)), dpp_f<0x140>(max8(fabsf(v)))));
+                const float amax = fmaxf(p.a, p.b), q = amax / 127.0f, id = q > 0.0f ? 1.0f / q : 0.0f;
+                const int qi = max(-127, min(127, (int)rintf(v * id)));
+                const int K = a.n_heads * HD;
+                a.q8[at] = (uint8_t)(qi & 0xff);
+                const float sum = sum32((float)qi);  // whole numbers below 2^24: exact
+                if ((e & 31) == 0) {
+                    float* dd = reinterpret_cast<float*>(a.q8 + K);
+                    dd[at / 32] = q;
+                    dd[K / 32 + at / 32] = q * sum;
+                }
+            }
+        }
+        return;
+    }
     // ---- merge the four wave partials into the chunk's partial ----
+    static_assert(ONE || WAVES == 4, "the merge below");
     for (int e = tid; e < G * HD; e += FD_THREADS) {
         const int g = e / HD, d = e % HD;
         const float m0 = s_m[0][g], m1 = s_m[1][g], m2 = s_m[2][g], m3 = s_m[3][g];
@@ -1416,9 +1470,9 @@ static int attn_mfma_long_launch_g(int G, dim3 grid, hipStream_t s, const AttnAr
     return launch_status();
 }
 
-template <int HD, int TPW, bool BIAS>
+template <int HD, int TPW, bool BIAS, int WAVES = 4, bool ONE = false>
 static int attn_mfma_launch_g(int G, dim3 grid, hipStream_t s, const AttnArgs& a) {
-#define PTM_AM(GG) hipLaunchKernelGGL((attn_decode_mfma_kernel<HD, GG, TPW, BIAS>), grid, dim3(FD_THREADS), 0, s, a)
+#define PTM_AM(GG) hipLaunchKernelGGL((attn_decode_mfma_kernel<HD, GG, TPW, BIAS, WAVES, ONE>), grid, dim3(64 * WAVES), 0, s, a)
     if constexpr (HD == 256) {  // up to four query heads per kv head (the wave partials of more would not fit the static LDS)
         switch (G) {
             case 1: PTM_AM(1); break;
@@ -1573,7 +1627,9 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
         if (o_q8 && (reinterpret_cast<uintptr_t>(o_q8) & 15u)) return PTM_E_ALIGN;
         AttnArgs a256{Q, K, V, q_norm_w, k_norm_w, rope_table, K_cache, V_cache, partial_O, partial_lse, partial_max,
                       d_past_len, n_heads, n_kv_heads, max_seq, add_one, scale, eps, rope_interleaved ? 1 : 0,
-                      window > 0 ? window : 0, nullptr, nullptr, nullptr};
+                      window > 0 ? window : 0, nullptr, nullptr, nullptr, O, static_cast<uint8_t*>(o_q8)};
+        if (max_seq <= 16 * FD_ONE_WAVES)
+            return attn_mfma_launch_g<256, 1, false, FD_ONE_WAVES, true>(n_heads / n_kv_heads, dim3(n_kv_heads), as_stream(stream), a256);
         const dim3 grid256(ptm_flash_decode_num_splits(max_seq), n_kv_heads);
         const int rc256 = attn_mfma_launch_g<256, 1, false>(n_heads / n_kv_heads, grid256, as_stream(stream), a256);
         if (rc256 != PTM_OK) return rc256;
@@ -1596,7 +1652,7 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
     }
     AttnArgs a{Q, K, V, q_norm_w, k_norm_w, rope_table, K_cache, V_cache, partial_O, partial_lse, partial_max,
                d_past_len, n_heads, n_kv_heads, max_seq, add_one, scale, eps, rope_interleaved ? 1 : 0, window > 0 ? window : 0,
-               q_bias, k_bias, v_bias};
+               q_bias, k_bias, v_bias, O, static_cast<uint8_t*>(o_q8)};
     const int G = n_heads / n_kv_heads;
     const dim3 grid(ptm_flash_decode_num_splits(max_seq), n_kv_heads);
     hipStream_t s = as_stream(stream);
@@ -1604,6 +1660,17 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
     if (o_q8 && (reinterpret_cast<uintptr_t>(o_q8) & 15u)) return PTM_E_ALIGN;
     if (kv_fp16) {
         // fp16 cache: the matrix-core kernel, chunks of 64 positions; partial maxima in base-2 units
+        // All positions in one workgroup's waves: up to 128, with heads of 64 two tiles a wave for up to 256.  Eight steps, 16 layers of 16 heads
+        // of 64, 30 / 77 / 150 / 240 positions: 2865 / 2874 / 2911 / 2900 us, one tile 2591 / 2610, two 2655 / 2664 / 2713 / 2763 (16 waves of one
+        // 2694 / 2713 / 2802 / 2887); 8 layers of 32 heads of 128, 20 / 110 / 150 / 235: 2849 / 2866 / 2851 / 2861, 2662 / 2751, and 2700 /
+        // 2772 / 2814 / 2889 with two tiles: there half a CU's LDS traffic per head costs what the merge launch does.
+        const dim3 one(n_kv_heads);
+        if (max_seq <= 16 * FD_ONE_WAVES) {
+            if (bias) return head_dim == 128 ? attn_mfma_launch_g<128, 1, true, FD_ONE_WAVES, true>(G, one, s, a) : attn_mfma_launch_g<64, 1, true, FD_ONE_WAVES, true>(G, one, s, a);
+            return head_dim == 128 ? attn_mfma_launch_g<128, 1, false, FD_ONE_WAVES, true>(G, one, s, a) : attn_mfma_launch_g<64, 1, false, FD_ONE_WAVES, true>(G, one, s, a);
+        }
+        if (head_dim == 64 && max_seq <= 32 * FD_ONE_WAVES)
+            return bias ? attn_mfma_launch_g<64, 2, true, FD_ONE_WAVES, true>(G, one, s, a) : attn_mfma_launch_g<64, 2, false, FD_ONE_WAVES, true>(G, one, s, a);
         if (ptm_flash_decode_num_splits(max_seq) > FD_LONG_SPLITS) {
             // a cache of more than 4096 positions: the looping kernel, at most FD_LONG_SPLITS partials per head
             const dim3 grid_long(FD_LONG_SPLITS, n_kv_heads);

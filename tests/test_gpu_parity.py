@@ -755,6 +755,51 @@ def test_attn_decode_fused_q8_output_is_the_quantised_fp32_output(dev, nh, nkv, 
     assert torch.equal(q8, want)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,cap", [(8, 8, 64, 128), (12, 4, 64, 256), (16, 2, 64, 256), (28, 4, 64, 129), (4, 2, 128, 128), (32, 8, 128, 127), (40, 8, 128, 17),
+                                           (16, 2, 128, 128), (4, 4, 256, 128), (6, 2, 256, 64), (8, 2, 256, 128)])
+@pytest.mark.parametrize("norm,bias,interleaved,window", [(1, 0, 0, 0), (0, 1, 1, 0), (1, 0, 0, 23)])
+def test_attn_decode_of_a_short_cache_equals_that_of_a_long_one(dev, nh, nkv, hd, cap, norm, bias, interleaved, window):
+    """A cache that one workgroup's waves hold (no merge launch) against the split kernels, which a larger cache with the same rows takes: the
+    positions at the edges of a wave's tiles, the first and the last, windows, biases, every count of query heads per kv head; NaN behind the
+    position.  fp32 sums over up to 256 positions in another order: 1e-5 of the largest value."""
+    import ctypes as C
+    from prometorch_amd import _lib
+    if hd == 256:
+        bias = 0
+    fn = _lib.load().ptm_attn_decode_fused_bias
+    vp = C.c_void_p
+    fn.restype = C.c_int
+    fn.argtypes = [vp] * 16 + [C.c_int, C.c_int, C.c_int, vp, C.c_int, C.c_float, C.c_float, C.c_int, C.c_int, C.c_int, C.c_int, vp]
+    r = synth.rng_for(51, nh, hd, cap)
+    kvd, qd, long = nkv * hd, nh * hd, 320
+    K0, V0 = [cu(r.standard_normal((long, kvd), dtype=np.float32).astype(np.float16)) for _ in range(2)]
+    Q, K, V = cu(synth.make_x(r, qd) * 3), cu(synth.make_x(r, kvd) * 3), cu(synth.make_x(r, kvd))
+    qw, kw = [cu(1 + 0.1 * synth.make_x(r, hd)) if norm else None for _ in range(2)]
+    bq, bk, bv = [cu(synth.make_x(r, n)) if bias else None for n in (qd, kvd, kvd)]
+    table = ops.rope_table(long, hd, 1e6).cuda()
+    S = ops.flash_decode_num_splits(long)
+    p = lambda t: t.data_ptr() if t is not None else None
+    for past in sorted({0, 1, 15, 16, 17, 31, 32, 63, 64, 100, cap - 2, cap - 1}):
+        if past >= cap:
+            continue
+        res = []
+        for max_seq in (cap, long):
+            Kc, Vc = K0[:max_seq].clone(), V0[:max_seq].clone()
+            Kc[past:], Vc[past:] = float("nan"), float("nan")
+            pO, pL, pM = [torch.full((S * n,), float("nan"), device="cuda") for n in (qd, nh, nh)]
+            O, q8 = torch.empty(qd, device="cuda"), torch.zeros(ops.q8_bytes(qd), dtype=torch.uint8, device="cuda")
+            d_past = torch.full((1,), past, dtype=torch.int64, device="cuda")
+            assert fn(p(Q), p(K), p(V), p(bq), p(bk), p(bv), p(qw), p(kw), p(Kc), p(Vc), p(O), p(q8), p(pO), p(pL), p(pM), p(table), nh, nkv, hd, p(d_past),
+                      max_seq, hd ** -0.5, 1e-6, 0, 1, interleaved, window, None) == 0
+            want = torch.zeros_like(q8)
+            ops.launch_quantize_q8(O, want, qd)
+            torch.cuda.synchronize()
+            assert torch.equal(q8, want), past
+            res.append((O, Kc[:past + 1], Vc[:past + 1]))
+        assert float((res[0][0] - res[1][0]).abs().max()) <= 1e-5 * float(res[1][0].abs().max()), past
+        assert torch.equal(res[0][1].view(torch.int16), res[1][1].view(torch.int16)) and torch.equal(res[0][2].view(torch.int16), res[1][2].view(torch.int16))
+
+
 def test_gemv_random_shapes_vs_oracle(dev, po):
     """A fixed pseudo-random sweep over row counts, row lengths, formats and store modes: every launch rule (lane
     groups per row, blocks per pass, rolling passes, the one-workgroup-per-CU kernel, the plain formats) is met by
