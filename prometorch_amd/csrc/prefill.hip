@@ -172,32 +172,49 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_kernel(float* __restri
     }
 }
 
-// Four values of a q / k / v row that may still be K-split partial sums: slab z holds them at P + z * total + idx
-__device__ __forceinline__ float4 qkv_part_load4(const float* __restrict__ P, int splits, int64_t total, int64_t idx,
-                                                 const float* __restrict__ bias, int col) {
-    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int z0 = 0; z0 < splits; z0 += 4) {  // four slabs per batch, the slab index clamped: in flight together
-        float4 b[4];
+// a lane's two runs of four elements of a row that is still `splits` slabs: B slabs of both per batch, fetched unconditionally (the index clamped)
+template <int B>
+struct QkvRuns {
+    float4 a[B], b[B];
+    __device__ __forceinline__ void fetch(const float* __restrict__ P, int splits, int64_t total, int64_t at, int e0, int e1, int z0) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) b[u] = *reinterpret_cast<const float4*>(P + (int64_t)min(z0 + u, splits - 1) * total + idx);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (z0 + u == 0) a = b[u];
-            else if (z0 + u < splits) { a.x += b[u].x; a.y += b[u].y; a.z += b[u].z; a.w += b[u].w; }
+        for (int u = 0; u < B; ++u) {
+            const float* p = P + (int64_t)min(z0 + u, splits - 1) * total + at;
+            a[u] = *reinterpret_cast<const float4*>(p + e0);
+            b[u] = *reinterpret_cast<const float4*>(p + e1);
         }
     }
-    if (bias) {
-        const float4 bb = *reinterpret_cast<const float4*>(bias + col);
-        a.x += bb.x; a.y += bb.y; a.z += bb.z; a.w += bb.w;
+    // the slabs' sum in their order, the first batch fetched; then the bias
+    __device__ __forceinline__ void sum(const float* __restrict__ P, int splits, int64_t total, int64_t at, int e0, int e1,
+                                        const float* __restrict__ bias, float4& ra, float4& rb) {
+        auto add = [](float4& r, const float4& v) { r.x += v.x; r.y += v.y; r.z += v.z; r.w += v.w; };
+        ra = a[0];
+        rb = b[0];
+        for (int z0 = 0; z0 < splits; z0 += B) {
+            if (z0 > 0) fetch(P, splits, total, at, e0, e1, z0);
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+                if (z0 + u > 0 && z0 + u < splits) {
+                    add(ra, a[u]);
+                    add(rb, b[u]);
+                }
+        }
+        if (bias) {
+            add(ra, *reinterpret_cast<const float4*>(bias + e0));
+            add(rb, *reinterpret_cast<const float4*>(bias + e1));
+        }
     }
-    return a;
-}
+};
+
 
 // The same work with head_dim / 8 lanes per head (head_dim 32, 64, 128 or 256) and 16-byte accesses: a lane owns four
 // rotation pairs (two runs of four elements), a wave 64 / (head_dim / 8) heads of one row.  grid (rows, q head blocks + kv
 // head blocks), one wave.  With one wave per (row, head) and 4-byte accesses the launch was bound by the number of
 // workgroups and requests: 82 k single-wave workgroups for 2048 rows of 40 heads.
-template <bool KV16, bool PART>
+// B: slabs per batch (PART).  A short prompt's launch is its requests' round trips, so a row's slabs (up to 16), the rotation and the norm weights go
+// out together; a long one's rows have one slab, and requesting it four times over cost it the texture path
+// (four at a time, q before k before v, the tables last: 19 rows of 40 heads 7.0 -> 3.8 us, 2048 24.7 -> 18.8 ... 21.3).
+template <bool KV16, bool PART, int B>
 __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __restrict__ Q, float* __restrict__ K,
                                                                       const float* __restrict__ V, const float* __restrict__ qw,
                                                                       const float* __restrict__ kw, void* __restrict__ Kc,
@@ -227,14 +244,26 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __r
     const int w = is_k ? 1 : 0;
     float4 a, b, va, vb;
     va = vb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float* cs = rope + pos * head_dim;
+    const float* nw = is_k ? kw : qw;
+    float4 c4, s4, wa, wb;
+    auto fetch_tables = [&]() {
+        c4 = *reinterpret_cast<const float4*>(cs + 4 * l);
+        s4 = *reinterpret_cast<const float4*>(cs + half + 4 * l);
+        wa = *reinterpret_cast<const float4*>((nw ? nw : cs) + e0);  // a valid address either way
+        wb = *reinterpret_cast<const float4*>((nw ? nw : cs) + e1);
+    };
     if constexpr (PART) {
         const int64_t total = (int64_t)rows * width;
-        a = qkv_part_load4(parts.P[w], parts.splits[w], total, row_off + e0, parts.bias[w], h * head_dim + e0);
-        b = qkv_part_load4(parts.P[w], parts.splits[w], total, row_off + e1, parts.bias[w], h * head_dim + e1);
-        if (is_k) {
-            va = qkv_part_load4(parts.P[2], parts.splits[2], total, row_off + e0, parts.bias[2], h * head_dim + e0);
-            vb = qkv_part_load4(parts.P[2], parts.splits[2], total, row_off + e1, parts.bias[2], h * head_dim + e1);
-        }
+        const int col = h * head_dim;
+        auto bias = [&](int i) { return parts.bias[i] ? parts.bias[i] + col : nullptr; };
+        QkvRuns<B> own, val;
+        own.fetch(parts.P[w], parts.splits[w], total, row_off, e0, e1, 0);
+        if (is_k) val.fetch(parts.P[2], parts.splits[2], total, row_off, e0, e1, 0);
+        fetch_tables();
+        issue_order_fence();
+        own.sum(parts.P[w], parts.splits[w], total, row_off, e0, e1, bias(w), a, b);
+        if (is_k) val.sum(parts.P[2], parts.splits[2], total, row_off, e0, e1, bias(2), va, vb);
     } else {
         a = *reinterpret_cast<const float4*>(vec + e0);
         b = *reinterpret_cast<const float4*>(vec + e1);
@@ -242,10 +271,8 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __r
             va = *reinterpret_cast<const float4*>(V + row_off + e0);
             vb = *reinterpret_cast<const float4*>(V + row_off + e1);
         }
+        fetch_tables();
     }
-    const float* cs = rope + pos * head_dim;
-    const float4 c4 = *reinterpret_cast<const float4*>(cs + 4 * l), s4 = *reinterpret_cast<const float4*>(cs + half + 4 * l);
-    const float* nw = is_k ? kw : qw;
     if (nw) {
         float ss = fmaf(a.x, a.x, 0.0f);
         ss = fmaf(a.y, a.y, ss); ss = fmaf(a.z, a.z, ss); ss = fmaf(a.w, a.w, ss);
@@ -253,7 +280,6 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __r
         for (int o = lph >> 1; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);  // within the head's lanes
         const float rs = 1.0f / sqrtf(ss / (float)head_dim + eps);
         const float one = add_one ? 1.0f : 0.0f;
-        const float4 wa = *reinterpret_cast<const float4*>(nw + e0), wb = *reinterpret_cast<const float4*>(nw + e1);
         a.x = a.x * rs * (wa.x + one); a.y = a.y * rs * (wa.y + one); a.z = a.z * rs * (wa.z + one); a.w = a.w * rs * (wa.w + one);
         b.x = b.x * rs * (wb.x + one); b.y = b.y * rs * (wb.y + one); b.z = b.z * rs * (wb.z + one); b.w = b.w * rs * (wb.w + one);
     }
@@ -310,18 +336,33 @@ static int qknorm_rope_kv_rows_launch(float* Q, float* K, const float* V, const 
     quad = quad && aligned16(Q) && aligned16(K) && aligned16(V) && aligned16(q_norm_w) && aligned16(k_norm_w) &&
            aligned16(K_cache) && aligned16(V_cache) && aligned16(rope_table);
     for (int i = 0; i < 3; ++i) quad = quad && aligned16(parts.P[i]) && aligned16(parts.bias[i]);
-#define PTM_QK(KERNEL, KV16, GRID)                                                                                         \
-    hipLaunchKernelGGL((KERNEL<KV16, PART>), GRID, dim3(64), 0, s, Q, K, V, q_norm_w, k_norm_w, K_cache, V_cache, rope_table, \
+#define PTM_QK(KERNEL, GRID, ...)                                                                                         \
+    hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), GRID, dim3(64), 0, s, Q, K, V, q_norm_w, k_norm_w, K_cache, V_cache, rope_table, \
                        n_heads, n_kv_heads, head_dim, pos0, eps, add_one, rope_interleaved ? 1 : 0, parts)
     if (quad) {
         const int hpw = 64 / (head_dim / 8);
         const dim3 grid(rows, (n_heads + hpw - 1) / hpw + (n_kv_heads + hpw - 1) / hpw);
-        if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, true, grid);
-        else PTM_QK(qknorm_rope_kv_rows_quad_kernel, false, grid);
+        int most = 1;
+        for (int i = 0; i < 3; ++i) most = parts.splits[i] > most ? parts.splits[i] : most;
+        if (!PART || most <= 1) {
+            if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 1);
+            else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 1);
+        } else if constexpr (PART) {
+            if (most <= 2) {
+                if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 2);
+                else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 2);
+            } else if (most <= 4) {
+                if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 4);
+                else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 4);
+            } else {
+                if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 8);
+                else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 8);
+            }
+        }
     } else {
         const dim3 grid(rows, n_heads + n_kv_heads);
-        if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_kernel, true, grid);
-        else PTM_QK(qknorm_rope_kv_rows_kernel, false, grid);
+        if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_kernel, grid, true, PART);
+        else PTM_QK(qknorm_rope_kv_rows_kernel, grid, false, PART);
     }
 #undef PTM_QK
     return launch_status();
