@@ -50,10 +50,14 @@ int q6k_gemv_argmax_impl(const void* W, const float* x, const float* gamma, floa
                          const ArgmaxAdvance adv, hipStream_t s);
 int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f32, float* Y, int M, int K, int N,
                    int64_t stride, void* workspace, bool accumulate, float* split_ws, size_t split_ws_bytes, bool reuse_rows,
-                   hipStream_t s, int* deferred_splits);
+                   hipStream_t s, int* deferred_splits, bool split_scales);
 int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool accumulate, const float* gamma, float eps,
                                   int add_one, void* ws_round, void* ws_plain, int M, int K, hipStream_t s);
 int qgemm_f16_splits(int N, int K, int M);
+int qgemm_f16_blocks_per_split(int N, int K, int M, size_t split_ws_bytes);
+int64_t qgemm_f16_split_scale_bytes(int M);
+bool qgemm_f16_act_rows_fit(int bps, int M, int K);
+int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
 void qgemm_f16_row_workspace(void* workspace, int M, int K, void** rows, float** rowscale);
 int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
                            bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
@@ -356,8 +360,8 @@ static int prefill_alloc(ptm_decoder* d, int rows) {
     const size_t o_h = take(4 * R * H);
     const size_t o_x = take(4 * R * H), o_q = take(4 * R * qd), o_k = take(4 * R * kvd),
                  o_v = take(4 * R * kvd), o_attn = take(4 * R * qd), o_gate = take(4 * R * I), o_up = take(4 * R * I),
-                 o_ws = take((size_t)ptm_qgemm_f16_workspace_bytes(rows, (int)kmax)),
-                 o_ws2 = take((size_t)ptm_qgemm_f16_workspace_bytes(rows, (int)kmax)), o_tok = take(4 * R);
+                 o_ws = take((size_t)(ptm_qgemm_f16_workspace_bytes(rows, (int)kmax) + qgemm_f16_split_scale_bytes(rows))),
+                 o_ws2 = take((size_t)(ptm_qgemm_f16_workspace_bytes(rows, (int)kmax) + qgemm_f16_split_scale_bytes(rows))), o_tok = take(4 * R);
     size_t split_elems = 0;  // widest splits x N over the layer's matrices (all layers have the same shapes)
     for (const ptm_qweight* w : {&d->layers[0].q, &d->layers[0].k, &d->layers[0].v, &d->layers[0].o, &d->layers[0].gate,
                                  &d->layers[0].up, &d->layers[0].down}) {
@@ -410,9 +414,10 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
     // SiLU.up are fused into the conversion (one launch fills both forms); a product whose rows are already in its
     // workspace skips the conversion.
     auto ws_of = [&](const ptm_qweight& w) { return w.ggml_type == PTM_TYPE_Q4_K ? d->pf_ws : d->pf_ws2; };
-    auto gemm = [&](const ptm_qweight& w, const float* X, float* Y, bool acc, bool rows_ready, int* deferred = nullptr) {
+    auto gemm = [&](const ptm_qweight& w, const float* X, float* Y, bool acc, bool rows_ready, int* deferred = nullptr,
+                    bool split_scales = false) {
         return qgemm_f16_impl(w.ggml_type, w.data, X, true, Y, M, w.cols, w.rows, w.row_stride_bytes, ws_of(w), acc,
-                              d->pf_split, d->pf_split_bytes, rows_ready, s, deferred);
+                              d->pf_split, d->pf_split_bytes, rows_ready, s, deferred, split_scales);
     };
     // RMSNorm of the residual rows into the row workspaces; `pending` > 0: the projection before it left that many K-split
     // partial sums in pf_split, which the same launch first adds to the residual rows
@@ -464,6 +469,7 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
         }
         PTM_TRY(norm_rows(pending, L.ffn_norm, uses(PTM_TYPE_Q4_K, {&L.gate, &L.up}), uses(PTM_TYPE_Q6_K, {&L.gate, &L.up})));
         pending = 0;
+        bool act_split = false;  // the down projection's rows have a scale per K split
         {
             // Gate and up share one launch when that fills the chip better.  The eight-wave tile runs one workgroup per CU, so
             // a launch costs ceil(tiles / 256) workgroup times: 2048 rows are 38 x 16 = 608 tiles per matrix, 3 + 3 rounds
@@ -485,7 +491,15 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
                 const void* W2[2] = {L.gate.data, L.up.data};
                 const int64_t s2[2] = {L.gate.row_stride_bytes, L.up.row_stride_bytes};
                 float* Y2[2] = {d->pf_gate, d->pf_up};
-                PTM_TRY(qgemm_f16_multi(2, t2, W2, s2, N2, Y2, M, H, d->pf_ws, d->pf_ws2, d->pf_split, d->pf_split_bytes, s, nullptr, nullptr));
+                // up to 128 rows the K splits are summed by the launch that makes the down projection's rows
+                const int bps = qgemm_f16_blocks_per_split(L.down.rows, I, M, d->pf_split_bytes);
+                const float* P2[2];
+                int sp2[2];
+                act_split = M <= 128 && qgemm_f16_act_rows_fit(bps, M, I);
+                PTM_TRY(qgemm_f16_multi(2, t2, W2, s2, N2, Y2, M, H, d->pf_ws, d->pf_ws2, d->pf_split, d->pf_split_bytes, s, act_split ? P2 : nullptr,
+                                        act_split ? sp2 : nullptr));
+                if (act_split)
+                    PTM_TRY(qgemm_f16_act_rows(P2[0], P2[1], sp2[0], sp2[1], c.ffn_gelu != 0, L.down.ggml_type == PTM_TYPE_Q4_K, ws_of(L.down), bps, M, I, s));
             } else {
                 PTM_TRY(gemm(L.gate, d->pf_x, d->pf_gate, false, true));
                 PTM_TRY(gemm(L.up, d->pf_x, d->pf_up, false, true));
@@ -493,15 +507,16 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
         }
         const bool act_ready = true;
         // SiLU.up (or, flagged through the add_one slot, GELU.up) fused into the conversion for the down projection
-        PTM_TRY(qgemm_f16_prepare_fused(2, d->pf_gate, d->pf_up, 0.0f, c.ffn_gelu ? 1 : 0,
-                                        L.down.ggml_type == PTM_TYPE_Q4_K ? d->pf_ws : nullptr,
-                                        L.down.ggml_type == PTM_TYPE_Q6_K ? d->pf_ws2 : nullptr, M, I, s));
+        if (!act_split)
+            PTM_TRY(qgemm_f16_prepare_fused(2, d->pf_gate, d->pf_up, 0.0f, c.ffn_gelu ? 1 : 0,
+                                            L.down.ggml_type == PTM_TYPE_Q4_K ? d->pf_ws : nullptr,
+                                            L.down.ggml_type == PTM_TYPE_Q6_K ? d->pf_ws2 : nullptr, M, I, s));
         if (L.post_ffn_norm) {
-            PTM_TRY(gemm(L.down, d->pf_gate, d->pf_h, false, act_ready));
+            PTM_TRY(gemm(L.down, d->pf_gate, d->pf_h, false, act_ready, nullptr, act_split));
             PTM_TRY(ptm_rms_norm_add(d->pf_h, L.post_ffn_norm, d->pf_x, M, H, c.rms_eps, 0, s));
         } else {
             // x += act . Wdown^T; before another layer the sum of the K splits is left to that layer's first launch
-            PTM_TRY(gemm(L.down, d->pf_gate, d->pf_x, true, act_ready, (li + 1 < c.n_layers && H <= 12288) ? &pending : nullptr));
+            PTM_TRY(gemm(L.down, d->pf_gate, d->pf_x, true, act_ready, (li + 1 < c.n_layers && H <= 12288) ? &pending : nullptr, act_split));
         }
     }
     (void)kvd;

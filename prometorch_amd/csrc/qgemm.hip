@@ -346,6 +346,18 @@ __global__ __launch_bounds__(256) void qgemm_prepare_rows_f16_kernel(const void*
     }
 }
 
+// silu(g) u and gelu(g) u in the arithmetic of silu_mul_kernel and gelu_mul_kernel
+__device__ __forceinline__ float silu_mul(float g, float u) {
+    float ng = 0.0f - g;
+    ng = fminf(fmaxf(ng, -88.0f), 88.0f);
+    return (g * (1.0f / (1.0f + expf(ng)))) * u;
+}
+__device__ __forceinline__ float gelu_mul(float g, float u) {
+    const float x3 = g * g * g;
+    const float t = tanhf(0.7978845608028654f * (g + 0.044715f * x3));
+    return 0.5f * g * (1.0f + t) * u;
+}
+
 // The same conversion fused with what precedes a projection in the prompt pass, so that the fp32 intermediate is never
 // written: PRE 1 = RMSNorm of the row (x * rs * (gamma + add_one), the arithmetic and reduction order of
 // rms_norm_kernel), PRE 2 = SiLU(gate) * up (the arithmetic of silu_mul_kernel), or tanh-GELU(gate) * up (that of
@@ -386,16 +398,6 @@ __global__ __launch_bounds__(THREADS) void qgemm_prepare_fused_kernel(const floa
         if constexpr (PRE == 1) {
             r.x = a.x * rs * (b.x + one); r.y = a.y * rs * (b.y + one); r.z = a.z * rs * (b.z + one); r.w = a.w * rs * (b.w + one);
         } else {
-            auto silu_mul = [](float g, float u) {
-                float ng = 0.0f - g;
-                ng = fminf(fmaxf(ng, -88.0f), 88.0f);
-                return (g * (1.0f / (1.0f + expf(ng)))) * u;
-            };
-            auto gelu_mul = [](float g, float u) {
-                const float x3 = g * g * g;
-                const float t = tanhf(0.7978845608028654f * (g + 0.044715f * x3));
-                return 0.5f * g * (1.0f + t) * u;
-            };
             if (gelu) { r.x = gelu_mul(a.x, b.x); r.y = gelu_mul(a.y, b.y); r.z = gelu_mul(a.z, b.z); r.w = gelu_mul(a.w, b.w); }
             else { r.x = silu_mul(a.x, b.x); r.y = silu_mul(a.y, b.y); r.z = silu_mul(a.z, b.z); r.w = silu_mul(a.w, b.w); }
         }
@@ -583,6 +585,76 @@ __global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(cons
     }
 }
 
+// SiLU(gate) . up (gelu: tanh-GELU) of a short prompt's rows, gate and up still `sg` / `su` slabs of K splits each, into the fp16 rows of the down
+// projection (rounded: to Q8 blocks first).  A workgroup has `chunk` values of a row, those of one K split of that projection, and they have
+// a scale of their own at rowscale[split * scale_stride + row]: nothing needs the whole row, which one workgroup a row had to
+// walk (19 rows: 19 CUs, behind a launch that summed the slabs on all).  What bounds it is one round trip for the slabs: 19 rows of 9728, three
+// slabs each, 4.1 us (the two launches 4.0 + 5.8).
+constexpr int ACT_CHUNK = 4096;  // values a workgroup holds
+__global__ __launch_bounds__(256) void qgemm_act_rows_kernel(const float* __restrict__ G, const float* __restrict__ U, int sg, int su, int gelu,
+                                                             int rounded, _Float16* __restrict__ Xh, float* __restrict__ rowscale,
+                                                             int scale_stride, int chunk, int M, int K) {
+    read_now(G, Xh, K);
+    __shared__ float red[4];
+    const int m = blockIdx.y, split = blockIdx.x, tid = threadIdx.x;
+    const int first = split * chunk, n4 = min(chunk, K - first) / 4;  // both multiples of 256
+    const int64_t total = (int64_t)M * K, at = (int64_t)m * K + first;
+    constexpr int HOLD = ACT_CHUNK / 1024, B = 4;
+    auto sum = [&](const float* P, int slabs, int i) {
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int z0 = 0; z0 < slabs; z0 += B) {
+            float4 b[B];
+#pragma unroll
+            for (int u = 0; u < B; ++u) b[u] = reinterpret_cast<const float4*>(P + min(z0 + u, slabs - 1) * total + at)[i];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                if (z0 + u == 0) a = b[u];
+                else if (z0 + u < slabs) { a.x += b[u].x; a.y += b[u].y; a.z += b[u].z; a.w += b[u].w; }
+            }
+        }
+        return a;
+    };
+    float4 v[HOLD];
+    float amax = 0.0f;
+#pragma unroll
+    for (int h = 0; h < HOLD; ++h) {
+        const int i = tid + 256 * h;
+        v[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (i < n4) {  // whole waves: n4 is a multiple of 64
+            const float4 g = sum(G, sg, i), u = sum(U, su, i);
+            if (gelu) v[h] = make_float4(gelu_mul(g.x, u.x), gelu_mul(g.y, u.y), gelu_mul(g.z, u.z), gelu_mul(g.w, u.w));
+            else v[h] = make_float4(silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z), silu_mul(g.w, u.w));
+        }
+        amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[h].x), fabsf(v[h].y)), fmaxf(fabsf(v[h].z), fabsf(v[h].w))));
+    }
+    amax = max64(amax);
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    int e = 0;
+    if (amax > 16384.0f) { (void)frexpf(amax, &e); e -= 14; }
+    const float down = ldexpf(1.0f, -e);
+    if (tid == 0) rowscale[split * scale_stride + m] = ldexpf(1.0f, e);
+#pragma unroll
+    for (int h = 0; h < HOLD; ++h) {
+        const int i = tid + 256 * h;
+        if (i >= n4) break;
+        float4 q = v[h];
+        if (rounded) {
+            float d, sm;
+            const uint32_t pk = q8_quantize4(q, d, sm);
+            q = make_float4(d * (float)(int)(int8_t)(pk & 0xff), d * (float)(int)(int8_t)((pk >> 8) & 0xff), d * (float)(int)(int8_t)((pk >> 16) & 0xff),
+                            d * (float)(int)(int8_t)(pk >> 24));
+        }
+        union { _Float16 h4[4]; uint2 u2; } o;
+        o.h4[0] = (_Float16)(q.x * down);
+        o.h4[1] = (_Float16)(q.y * down);
+        o.h4[2] = (_Float16)(q.z * down);
+        o.h4[3] = (_Float16)(q.w * down);
+        reinterpret_cast<uint2*>(Xh + at)[i] = o.u2;
+    }
+}
+
 // 16 small integers (4 dwords of bytes, each < 1024) -> two fragments of 8 fp16 holding (byte - bias) * scale + offset.
 // A byte b becomes the fp16 number 1024 + b by writing it under the exponent byte 0x64 (one v_perm per pair); the
 // subtraction of 1024 + bias is exact, and one packed fp16 FMA applies scale and offset: 2.5 instructions per pair.
@@ -687,7 +759,7 @@ template <typename Tile, int MT, int WAVES>
 __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride, const _Float16* Xh,
                                                const float* __restrict__ rowscale, float* Y, int M, int K, int N,
                                                int accumulate, int blocks_per_split, float* partials, int bx, int by, int bz,
-                                               uint8_t* s_a) {
+                                               uint8_t* s_a, int scale_stride) {
     // W and Xh are deliberately not __restrict__: loads through a restrict pointer may be moved across the
     // compiler fences below, and the prefetch distance of this loop depends on those fences
     constexpr int TM = 32 * MT;                     // rows of X per workgroup (MT tiles of 32)
@@ -718,7 +790,7 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
                            (int64_t)blk0 * 512;
     uint8_t* x_dst = s_a + (tid >> 5) * QF_PITCH + 16 * (tid & 31);
     float* s_rs = reinterpret_cast<float*>(s_a + 2 * TM * QF_PITCH);  // the tile's TM row scales (every padded row has one)
-    if (tid < TM) s_rs[tid] = rowscale[m0 + tid];
+    if (tid < TM) s_rs[tid] = rowscale[bz * scale_stride + m0 + tid];  // scale_stride 0: a row has one scale, not one per K split
     // the pieces of the next tile in flight (scalars, not an array: they must stay in registers)
     uint4 x0, x1, x2, x3, x4, x5, x6, x7;
     // prologue: tile of block 0 -> LDS buffer 0, weights of block 0, fragments of step 0.  The weight loads go out behind
@@ -877,14 +949,14 @@ __device__ __forceinline__ void qf_tile_of(int L, int gx, int gy, int& bx, int& 
 template <typename Tile, int MT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh,
                                                         const float* __restrict__ rowscale, float* Y, int M, int K, int N,
-                                                        int accumulate, int blocks_per_split, float* partials) {
+                                                        int accumulate, int blocks_per_split, float* partials, int scale_stride) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
     read_now(W, M);
     const int hw = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     const int L = qf_xcd_order(hw, gridDim.x * gridDim.y * gridDim.z);
     int bx, by, bz;
     qf_tile_of(L, gridDim.x, gridDim.y, bx, by, bz);
-    qgemm_f16_body<Tile, MT, WAVES>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds);
+    qgemm_f16_body<Tile, MT, WAVES>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
 }
 
 // Up to three projections of the same rows in ONE launch, its tile chosen as below for a single matrix (q, k, v of a layer: in a Q4_K_M
@@ -916,8 +988,8 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_mu
     const QfMat& q = i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]);
     const int local = sx - (i == 0 ? 0 : (i == 1 ? a.m[0].slot_end : a.m[1].slot_end));
     const int bx = local % q.ntiles, bz = local / q.ntiles;
-    if (q.q6) qgemm_f16_body<Q6Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds);
-    else qgemm_f16_body<Q4Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds);
+    if (q.q6) qgemm_f16_body<Q6Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
+    else qgemm_f16_body<Q4Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
 }
 
 // Y (+)= partials[0] + partials[1] + ... in that fixed order (deterministic, unlike atomics)
@@ -972,6 +1044,7 @@ __global__ __launch_bounds__(256) void qgemm_split_reduce_multi_kernel(const QfR
 
 // Row classes of the split rules: up to 128 rows, up to 256, up to 1024, more (2048-row chunks of long prompts: with 16 row
 // tiles per column tile, as many splits as a 512-row launch wants only multiply the partial sums).
+enum { QF_MAX_SPLITS = 16 };
 static inline int qf_row_class(int M) { return M <= 128 ? 1 : (M <= 256 ? 2 : (M <= 1024 ? 4 : 8)); }
 
 // K splits for an N x K weight matrix and M rows: enough workgroups to fill the chip when N alone gives few column
@@ -982,7 +1055,7 @@ int qgemm_f16_splits(int N, int K, int M) {
     const int ntiles = (N + QF_TN - 1) / QF_TN, nblk = K / 256;
     const int row_tiles = qf_row_class(M);
     int s = 256 / (ntiles * row_tiles);
-    const int cap = row_tiles == 1 ? 16 : 8;
+    const int cap = row_tiles == 1 ? QF_MAX_SPLITS : 8;
     s = s > cap ? cap : s;
     s = s > nblk / 2 ? nblk / 2 : s;
     return s < 1 ? 1 : s;
@@ -1044,16 +1117,27 @@ static int qgemm_check(const void* W, const void* X, const void* Y, int M, int K
     return PTM_OK;
 }
 
+// room in a row workspace for a scale per row and K split
+int64_t qgemm_f16_split_scale_bytes(int M) { return (int64_t)QF_MAX_SPLITS * qf_mpad(M) * 4; }
+
 // where the M rows of K values and their scales lie in a row workspace
 void qgemm_f16_row_workspace(void* workspace, int M, int K, void** rows, float** rowscale) {
     *rows = workspace;
     *rowscale = reinterpret_cast<float*>(static_cast<_Float16*>(workspace) + (int64_t)qf_mpad(M) * K);
 }
 
+// super-blocks per K split of qgemm_f16_impl with that much room for partial sums
+int qgemm_f16_blocks_per_split(int N, int K, int M, size_t split_ws_bytes) {
+    int splits = split_ws_bytes ? qgemm_f16_splits(N, K, M) : 1;
+    while (splits > 1 && (size_t)splits * M * N * sizeof(float) > split_ws_bytes) --splits;
+    return (K / 256 + splits - 1) / splits;
+}
+
 // Y (+)= X . W^T with X bf16 or fp32 rows; shared by the C entry points and the prefill runtime.
 int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f32, float* Y, int M, int K, int N,
                    int64_t stride, void* workspace, bool accumulate, float* split_ws, size_t split_ws_bytes, bool reuse_rows,
-                   hipStream_t s, int* deferred_splits) {
+                   hipStream_t s, int* deferred_splits, bool split_scales) {
+    // split_scales (with reuse_rows): the workspace holds a scale per row and K split (qgemm_f16_act_rows)
     // deferred_splits (optional): where K was split, the partial sums are left in split_ws for the caller's next kernel to
     // fold in (qgemm_f16_reduce_norm_prepare) and their count is returned here; 0 = Y is complete
     // reuse_rows: the workspace already holds these rows of X prepared by the previous call for a matrix of the
@@ -1071,10 +1155,9 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     _Float16* Xh = static_cast<_Float16*>(workspace);
     float* rowscale = reinterpret_cast<float*>(Xh + (int64_t)mp * K);
     const int nblk = K / 256;
-    int splits = split_ws ? qgemm_f16_splits(N, K, M) : 1;
-    while (splits > 1 && (size_t)splits * M * N * sizeof(float) > split_ws_bytes) --splits;
-    const int bps = (nblk + splits - 1) / splits;
-    splits = (nblk + bps - 1) / bps;  // no empty split
+    const int bps = qgemm_f16_blocks_per_split(N, K, M, split_ws ? split_ws_bytes : 0);
+    const int splits = (nblk + bps - 1) / bps;  // no empty split
+    const int scale_stride = split_scales ? mp : 0;
     float* partials = splits > 1 ? split_ws : nullptr;
     const int acc = accumulate ? 1 : 0;
     const bool q4 = ggml_type == PTM_TYPE_Q4_K;
@@ -1106,7 +1189,7 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     // 256 columns run with eight waves (two per SIMD, one 32-column strip each): against four waves owning two strips each, 512 x 4096 x
     // 14336 104 -> 92 us (128 rows), 512 x 4096 x 4096 59.8 -> 45.3 us and 96 x 4096 x 2560 57.0 -> 42.7 us (64 rows).  128 columns have
     // four waves of one strip.
-#define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials)
+#define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride)
     if (q4) {
         if (MT == 4) PTM_QF(Q4Tile, 4, 8);
         else if (MT == 2 && narrow) PTM_QF(Q4Tile, 2, 4);
@@ -1263,6 +1346,21 @@ int qgemm_f16_prepare_fused(int pre, const float* X, const float* X2, float eps,
     return launch_status();
 }
 
+// Fills a row workspace of K values with SiLU(gate) . up of M rows that are still G[sg] / U[su] slabs, a scale per row and K split of bps
+// super-blocks (the workspace has room for QF_MAX_SPLITS scales a row).
+bool qgemm_f16_act_rows_fit(int bps, int M, int K) { return M <= 65535 && bps * 256 <= ACT_CHUNK && (K / 256 + bps - 1) / bps <= QF_MAX_SPLITS; }
+int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s) {
+    if (!G || !U || !ws) return PTM_E_NULL;
+    if (M <= 0 || K <= 0 || (K % 256) != 0 || sg < 1 || su < 1 || bps < 1) return PTM_E_SHAPE;
+    if (!qgemm_f16_act_rows_fit(bps, M, K)) return PTM_E_UNSUPPORTED;
+    if (!aligned16(G) || !aligned16(U) || !aligned16(ws)) return PTM_E_ALIGN;
+    const int mp = qf_mpad(M), splits = (K / 256 + bps - 1) / bps;
+    _Float16* rows = static_cast<_Float16*>(ws);
+    hipLaunchKernelGGL(qgemm_act_rows_kernel, dim3(splits, M), dim3(256), 0, s, G, U, sg, su, gelu ? 1 : 0, rounded ? 1 : 0, rows,
+                       reinterpret_cast<float*>(rows + (int64_t)mp * K), mp, bps * 256, M, K);
+    return launch_status();
+}
+
 }  // namespace ptm
 
 using namespace ptm;
@@ -1317,7 +1415,7 @@ int64_t ptm_qgemm_f16_workspace_bytes(int M, int K) {
 int ptm_qgemm_f16(uint32_t ggml_type, const void* W, const void* X_bf16, float* Y, int M, int K, int N, int64_t stride,
                   void* workspace, ptm_stream_t stream) {
     return qgemm_f16_impl(ggml_type, W, X_bf16, false, Y, M, K, N, stride, workspace, false, nullptr, 0, false, as_stream(stream),
-                          nullptr);
+                          nullptr, false);
 }
 
 int64_t ptm_qgemm_f16_f32_workspace_bytes(int M, int K, int N) {
@@ -1335,7 +1433,7 @@ int ptm_qgemm_f16_f32(uint32_t ggml_type, const void* W, const float* X_f32, flo
     const int splits = qgemm_f16_splits(N, K, M);
     return qgemm_f16_impl(ggml_type, W, X_f32, true, Y, M, K, N, stride, workspace, accumulate != 0,
                           splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + base) : nullptr,
-                          splits > 1 ? (size_t)splits * M * N * 4 : 0, false, as_stream(stream), nullptr);
+                          splits > 1 ? (size_t)splits * M * N * 4 : 0, false, as_stream(stream), nullptr, false);
 }
 
 }  // extern "C"

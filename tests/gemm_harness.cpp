@@ -1,13 +1,20 @@
 // Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
-// splits, which the C ABI's plain product does not have, how a launch would cover its output, and the quantised models' prompt attention
-// as theirs calls it.  Host C++ only; built by
+// splits, which the C ABI's plain product does not have, how a launch would cover its output, and the quantised models' prompt attention and
+// down projection as theirs calls them.  Host C++ only; built by
 // __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
 #include "gemm_plan.h"
+#include "ptm.h"
 
 namespace ptm {
 int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
                            bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
                            float scale, int kv_fp16, int window, hipStream_t s);
+int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f32, float* Y, int M, int K, int N,
+                   int64_t stride, void* workspace, bool accumulate, float* split_ws, size_t split_ws_bytes, bool reuse_rows,
+                   hipStream_t s, int* deferred_splits, bool split_scales);
+int qgemm_f16_blocks_per_split(int N, int K, int M, size_t split_ws_bytes);
+int64_t qgemm_f16_split_scale_bytes(int M);
+int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
 }
 
 extern "C" {
@@ -68,6 +75,16 @@ int prefill_rows16(const float* Q, const void* K, const void* V, float* O, void*
                                                max_seq, scale, kv_fp16, window, static_cast<hipStream_t>(stream));
     *wrote = w ? 1 : 0;
     return rc;
+}
+
+int64_t act_down_bytes(int M, int K) { return ptm_qgemm_f16_workspace_bytes(M, K) + ptm::qgemm_f16_split_scale_bytes(M); }
+// Y = down . (act(gate) . up) of rows that are still slabs, in ws of act_down_bytes
+int act_down(uint32_t type, const void* W, int64_t stride, const float* G, const float* U, int sg, int su, int gelu, float* Y, int M, int K, int N, void* ws,
+             float* split_ws, int64_t split_bytes, void* stream) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int bps = ptm::qgemm_f16_blocks_per_split(N, K, M, (size_t)split_bytes);
+    const int rc = ptm::qgemm_f16_act_rows(G, U, sg, su, gelu != 0, type == PTM_TYPE_Q4_K, ws, bps, M, K, s);
+    return rc ? rc : ptm::qgemm_f16_impl(type, W, G, true, Y, M, K, N, stride, ws, false, split_ws, (size_t)split_bytes, true, s, nullptr, true);
 }
 
 }  // extern "C"

@@ -216,6 +216,38 @@ def test_prefill_attention_as_rows_of_the_next_product(dev, kv_fp16, nh, nkv, hd
     assert np.array_equal(rows16[:rows].cpu().numpy().view(np.uint16), v.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N,sg,su,gelu", [(1, 256, 64, 1, 1, 0), (19, 9728, 2560, 3, 3, 0), (5, 2816, 1024, 4, 1, 1), (33, 4096, 300, 5, 9, 0), (128, 2560, 640, 2, 2, 1),
+                                              (2, 14336, 4096, 2, 3, 0)])
+def test_activation_rows_with_a_scale_per_split(dev, po, qt, M, K, N, sg, su, gelu):
+    """SiLU . up (GELU . up) of rows that are still partial sums, and the down projection with a scale per row and K split: rows whose values fit
+    fp16, rows that do not, in one split or in all; against the same in 64 bits (both operands rounded to fp16: the bar of the other products)."""
+    from gemm_helpers import harness
+    h, p = harness(), lambda t: ctypes.c_void_p(t.data_ptr())
+    h.act_down_bytes.restype = ctypes.c_int64
+    r = synth.rng_for(73, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    G, U = [cu(r.standard_normal((s, M, K), dtype=np.float32)) for s in (sg, su)]
+    U[:, M // 2] *= 3e6            # a row beyond fp16
+    U[:, M - 1, K // 2:] *= 1e5    # and half of one
+    gate, up = G.double().sum(0), U.double().sum(0)
+    act = (torch.nn.functional.gelu(gate, approximate="tanh") if gelu else torch.nn.functional.silu(gate)) * up
+    if qt == 12:
+        b = act.reshape(M, -1, 32)
+        d = b.abs().amax(2, keepdim=True) / 127
+        act = (torch.round(b / d) * d).reshape(M, K)
+    want = (act @ cu(po.dequant(qt, W)).double().reshape(N, K).T).cpu().numpy()
+    ws = torch.empty(h.act_down_bytes(M, K), dtype=torch.uint8, device="cuda")
+    split = torch.empty(16 * M * N, device="cuda")
+    Y, Wd = torch.full((M, N), 9.0, device="cuda"), cu(W)
+    assert h.act_down(qt, p(Wd), ctypes.c_int64(W.shape[1]), p(G), p(U), sg, su, gelu, p(Y), M, K, N, p(ws), p(split), ctypes.c_int64(split.numel() * 4), None) == 0
+    torch.cuda.synchronize()
+    got = Y.cpu().numpy()
+    e = np.abs(got - want).max(axis=1) / np.sqrt((want ** 2).mean(axis=1))
+    print("max err / rms per row: %.2e" % e.max(), flush=True)
+    assert e.max() <= PREFILL_TOL
+
+
 def test_prefill_attention_rejects_bad_shapes(dev):
     z = torch.zeros(64 * 64, device="cuda")
     with pytest.raises(PtmError):
