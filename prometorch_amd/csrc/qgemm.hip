@@ -746,6 +746,103 @@ struct Q6Tile {  // Q6_K: the lane's 16 bytes of ql for each (half, pair), of qh
     static constexpr bool kQ8Round = false;
 };
 
+// Where a workgroup's accumulators go.
+// C layout of the 32x32 tile: column j = lane % 32, rows 8 (r / 4) + 4 (lane / 32) + r % 4.  The row scales come from
+// LDS (staged in the prologue), and when accumulating the 16 old values of a tile are fetched together before its 16
+// stores: a load issued behind a store the compiler cannot tell apart from it is one serial memory round trip per value,
+// more than the main loop of a launch with few blocks per workgroup takes.
+template <int MT>
+__device__ __forceinline__ void qf_store(const f32x16 (&acc)[MT], const float* s_rs, float* Y, float* partials, int accumulate, int M, int N, int m0, int n_base,
+                                         int j, int kh, int bz) {
+    const int n = n_base + j;
+    const bool n_ok = n < N;
+    const int nc = n_ok ? n : N - 1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        float old[16];
+        if (!partials && accumulate) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = min(m0 + mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), M - 1);
+                old[r] = Y[(int64_t)m * N + nc];
+            }
+            issue_order_fence();
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) old[r] = 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int lr = mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            const int m = m0 + lr;
+            const float v = acc[mt][r] * s_rs[lr];
+            if (m < M && n_ok) {
+                if (partials) __builtin_nontemporal_store(v, &partials[((int64_t)bz * M + m) * N + n]);
+                else __builtin_nontemporal_store(accumulate ? old[r] + v : v, &Y[(int64_t)m * N + n]);
+            }
+        }
+    }
+}
+
+
+// Up to 32 rows and up to four super-blocks of a K split: 128 columns, four waves of one strip.  Such a workgroup's time is its requests' round trips,
+// one per block where the next block's are out while this one is worked on (half a microsecond's work).  Here all of its blocks, of X
+// (into LDS) and of the weights (registers, up to 120), are requested before any is waited for.  Same sums in the same order.
+// 19 rows, 2560 x 9728 in 13 splits of three: Q6_K 21.6 -> 16.6 us, Q4_K 12.4 -> 11.0; 2 x 9728 x 2560 in three of four 15.8 -> 15.2 (weights in memory order
+// through LDS 17.1; eight waves, 256 columns 17.0).
+template <typename Tile, int NB>
+__device__ __forceinline__ void qgemm_f16_short_body(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale, float* Y, int M,
+                                                     int K, int N, int accumulate, int blocks_per_split, float* partials, int bx, int bz, uint8_t* s_a,
+                                                     int scale_stride) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 31, kh = lane >> 5;
+    const int n_base = bx * 128 + wave * 32;
+    const int blk0 = bz * blocks_per_split, nblk = min(K / 256 - blk0, blocks_per_split);
+    const uint8_t* wrow = W + (int64_t)min(n_base + j, N - 1) * stride + (int64_t)blk0 * Tile::kBlockBytes;
+    const uint8_t* x_src = reinterpret_cast<const uint8_t*>(Xh) + (int64_t)blk0 * 512 + 16 * (tid & 31);
+    float* s_rs = reinterpret_cast<float*>(s_a + NB * 32 * QF_PITCH);
+    // rows past the last repeat it: their sums are not stored
+    u32x4 x[4 * NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            x[4 * b + p] = *reinterpret_cast<const u32x4*>(x_src + (int64_t)min((tid >> 5) + 8 * p, M - 1) * K * 2 + min(b, nblk - 1) * 512);
+    issue_order_fence();
+    Tile w[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) w[b].load(wrow + (int64_t)min(b, nblk - 1) * Tile::kBlockBytes, kh);
+    issue_order_fence();
+    if (tid < 32) s_rs[tid] = rowscale[bz * scale_stride + min(tid, M - 1)];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) *reinterpret_cast<u32x4*>(s_a + (b * 32 + (tid >> 5) + 8 * p) * QF_PITCH + 16 * (tid & 31)) = x[4 * b + p];
+    __syncthreads();
+    f32x16 acc[1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (b >= nblk) break;  // workgroup-uniform
+        w[b].pin();
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            h8 bf[2];
+            w[b].frags(s, kh, bf[0], bf[1]);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const h8 af = *reinterpret_cast<const h8*>(s_a + (b * 32 + j) * QF_PITCH + 64 * s + 32 * kh + 16 * ks);
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[ks], acc[0], 0, 0, 0);
+            }
+        }
+    }
+    qf_store<1>(acc, s_rs, Y, partials, accumulate, M, N, 0, n_base, j, kh, bz);
+}
+// Whether it serves a launch whose longest split has `blocks`: of up to two blocks the other body's prologue and first step request everything, too.
+constexpr int QF_SHORT_BLOCKS = 4;
+static inline bool qf_short(int M, int blocks) { return M <= 32 && blocks > 2 && blocks <= QF_SHORT_BLOCKS; }
+static inline size_t qf_short_lds(int nb) { return (size_t)nb * 32 * QF_PITCH + 4 * 32; }
+
 // X tile of a super-block step in LDS.  The pieces a thread owns of the NEXT block's tile are fetched during the first
 // steps of the current block, followed by the next block's weights, and written to the other LDS buffer during the
 // later steps, so the block ends with the next tile complete behind the only workgroup barrier of the block.  (After the
@@ -890,38 +987,7 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
         cur = nxt;
         __syncthreads();  // next tile complete, this tile no longer read
     }
-    // C layout of the 32x32 tile: column j = lane % 32, rows 8 (r / 4) + 4 (lane / 32) + r % 4.  The row scales come from
-    // LDS (staged in the prologue), and when accumulating the 16 old values of a tile are fetched together before its 16
-    // stores: a load issued behind a store the compiler cannot tell apart from it is one serial memory round trip per value,
-    // more than the main loop of a launch with few blocks per workgroup takes.
-    const int n = n_base + j;
-    const bool n_ok = n < N;
-    const int nc = n_ok ? n : N - 1;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        float old[16];
-        if (!partials && accumulate) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = min(m0 + mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), M - 1);
-                old[r] = Y[(int64_t)m * N + nc];
-            }
-            issue_order_fence();
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) old[r] = 0.0f;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int lr = mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            const int m = m0 + lr;
-            const float v = acc[mt][r] * s_rs[lr];
-            if (m < M && n_ok) {
-                if (partials) __builtin_nontemporal_store(v, &partials[((int64_t)bz * M + m) * N + n]);
-                else __builtin_nontemporal_store(accumulate ? old[r] + v : v, &Y[(int64_t)m * N + n]);
-            }
-        }
-    }
+    qf_store<MT>(acc, s_rs, Y, partials, accumulate, M, N, m0, n_base, j, kh, bz);
 }
 
 // Which tile a workgroup takes.  The hardware deals consecutive workgroup ids round-robin to the 8 XCDs, each with its own
@@ -959,6 +1025,17 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_ke
     qgemm_f16_body<Tile, MT, WAVES>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
 }
 
+// up to 32 rows, NB super-blocks per split
+template <typename Tile, int NB>
+__global__ __launch_bounds__(256, 2) void qgemm_f16_short_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale,
+                                                                 float* Y, int M, int K, int N, int accumulate, int blocks_per_split, float* partials,
+                                                                 int scale_stride) {
+    extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(W, M);
+    const int L = qf_xcd_order(blockIdx.x, gridDim.x), tiles = (N + 127) / 128;
+    qgemm_f16_short_body<Tile, NB>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, L % tiles, L / tiles, qf_lds, scale_stride);
+}
+
 // Up to three projections of the same rows in ONE launch, its tile chosen as below for a single matrix (q, k, v of a layer: in a Q4_K_M
 // file two Q4_K matrices and a Q6_K one).  Each matrix brings its own prepared rows (Q8-rounded for Q4_K, plain for
 // Q6_K), column tiles and K splits; blockIdx.x walks the (column tile, split) slots of the matrices one after the other.
@@ -990,6 +1067,30 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_mu
     const int bx = local % q.ntiles, bz = local / q.ntiles;
     if (q.q6) qgemm_f16_body<Q6Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
     else qgemm_f16_body<Q4Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
+}
+
+// the same for up to 32 rows and up to QF_SHORT_BLOCKS super-blocks per split
+__global__ __launch_bounds__(256, 2) void qgemm_f16_short_multi_kernel(const QfMulti a, int M, int K) {
+    extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(a.m[0].W, a.m[1].W, a.m[2].W, a.n_mat);
+    const int sx = qf_xcd_order(blockIdx.x, gridDim.x);
+    int i = 0;
+    if (a.n_mat > 1 && sx >= a.m[0].slot_end) i = 1;
+    if (a.n_mat > 2 && sx >= a.m[1].slot_end) i = 2;
+    const QfMat& q = i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]);
+    const int local = sx - (i == 0 ? 0 : (i == 1 ? a.m[0].slot_end : a.m[1].slot_end));
+    const int bx = local % q.ntiles, bz = local / q.ntiles;
+#define PTM_QS(TILE, NB) qgemm_f16_short_body<TILE, NB>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, bz, qf_lds, 0)
+    if (q.q6) {
+        if (q.bps <= 2) PTM_QS(Q6Tile, 2);
+        else if (q.bps == 3) PTM_QS(Q6Tile, 3);
+        else PTM_QS(Q6Tile, 4);
+    } else {
+        if (q.bps <= 2) PTM_QS(Q4Tile, 2);
+        else if (q.bps == 3) PTM_QS(Q4Tile, 3);
+        else PTM_QS(Q4Tile, 4);
+    }
+#undef PTM_QS
 }
 
 // Y (+)= partials[0] + partials[1] + ... in that fixed order (deterministic, unlike atomics)
@@ -1174,6 +1275,8 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     static std::once_flag raised;  // two host threads may get here at once: the second waits until the caps are raised
     std::call_once(raised, [] {
         const int big = 2 * 128 * QF_PITCH + 4 * 128, small = 2 * 64 * QF_PITCH + 4 * 64;
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q4Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q6Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
@@ -1189,6 +1292,18 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     // 256 columns run with eight waves (two per SIMD, one 32-column strip each): against four waves owning two strips each, 512 x 4096 x
     // 14336 104 -> 92 us (128 rows), 512 x 4096 x 4096 59.8 -> 45.3 us and 96 x 4096 x 2560 57.0 -> 42.7 us (64 rows).  128 columns have
     // four waves of one strip.
+    if (qf_short(M, bps)) {
+        const size_t short_lds = qf_short_lds(bps);
+#define PTM_QS(TILE, NB) hipLaunchKernelGGL((qgemm_f16_short_kernel<TILE, NB>), dim3(grid.x * grid.z), dim3(256), short_lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride)
+        if (q4) {
+            if (bps == 3) PTM_QS(Q4Tile, 3);
+            else PTM_QS(Q4Tile, 4);
+        } else {
+            if (bps == 3) PTM_QS(Q6Tile, 3);
+            else PTM_QS(Q6Tile, 4);
+        }
+#undef PTM_QS
+    } else {
 #define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride)
     if (q4) {
         if (MT == 4) PTM_QF(Q4Tile, 4, 8);
@@ -1202,6 +1317,7 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         else PTM_QF(Q6Tile, 1, 4);
     }
 #undef PTM_QF
+    }
     if (deferred_splits) *deferred_splits = partials ? splits : 0;
     if (partials && !deferred_splits) {
         const int64_t total = (int64_t)M * N;
@@ -1259,7 +1375,8 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     int sp[3];
     qgemm_f16_multi_plan(n, N, types, K, M, sp);
     const int nblk = K / 256;
-    int wide = 0;
+    int wide = 0, most = 0;  // super-blocks of the longest split
+    for (int i = 0; i < n; ++i) most = (nblk + sp[i] - 1) / sp[i] > most ? (nblk + sp[i] - 1) / sp[i] : most;
     for (int i = 0; i < n; ++i) wide += (N[i] + QF_TN - 1) / QF_TN * sp[i];
     const bool narrow = qf_narrow(M, wide);
     const int tn = narrow ? 128 : QF_TN;
@@ -1311,12 +1428,15 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     std::call_once(raised, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 128 * QF_PITCH + 4 * 128);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(QF_SHORT_BLOCKS));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
     });
-    if (M <= 32)
+    if (qf_short(M, most))
+        hipLaunchKernelGGL(qgemm_f16_short_multi_kernel, dim3(slots), dim3(256), qf_short_lds(most), s, a, M, K);
+    else if (M <= 32)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<1, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)32 * QF_PITCH + 4 * 32, s, a, M, K);
     else if (narrow)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);

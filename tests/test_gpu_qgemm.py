@@ -200,3 +200,29 @@ def test_short_prompt_tiles(dev, po, qt, M, K, N):
     few = gpu_qgemm_f16(qt, W, xb[:M], M, K, N)
     many = gpu_qgemm_f16(qt, W, xb, 65, K, N)
     assert np.array_equal(bits(few), bits(many[:M]))
+
+
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(1, 768, 127), (31, 768, 129), (32, 1024, 385), (17, 1024, 1), (8, 768, 4096)])
+def test_short_prompts_with_all_blocks_requested_at_once(dev, po, qt, M, K, N):
+    """K of three and four super-blocks: rows are the rows of a 65-row call bit for bit."""
+    r = synth.rng_for(47, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    xb, _ = bf16_round(r.standard_normal((65, K), dtype=np.float32))
+    assert np.array_equal(bits(gpu_qgemm_f16(qt, W, xb[:M], M, K, N)), bits(gpu_qgemm_f16(qt, W, xb, 65, K, N)[:M]))
+
+
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(19, 9728, 2560), (32, 14336, 1000), (5, 9728, 2561)])
+def test_short_prompts_whose_last_split_is_shorter(dev, po, qt, M, K, N):
+    """13 splits of three blocks with two in the last, and others: rows are the rows of a 40-row call, which has the same splits, bit for bit."""
+    r = synth.rng_for(48, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    x = torch.from_numpy(r.standard_normal((40, K), dtype=np.float32)).cuda()
+    Wd, out = torch.from_numpy(W).cuda(), []
+    for m in (M, 40):
+        ws = torch.empty(ops.qgemm_f16_f32_workspace_bytes(m, K, N), dtype=torch.uint8, device="cuda")
+        y = torch.full((m, N), 3.0, device="cuda")
+        ops.matmul_q_f16_f32(qt, Wd, x[:m].contiguous(), y, m, K, N, W.shape[1], ws, accumulate=False)
+        out.append(y.cpu().numpy()[:M])
+    assert np.array_equal(bits(out[0]), bits(out[1]))
