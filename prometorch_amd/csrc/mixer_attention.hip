@@ -131,6 +131,9 @@ static int rows_launch(const ptm_attention_args& a, const int64_t* d_past, hipSt
 // v_mfma_f32_32x32x16_bf16: A: lane l holds row l % 32, summation indices 8 (l / 32) + 0..7; B: column l % 32, the same
 // indices; C: column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4.  The 16 keys of a P.V step are the ones the lane already
 // holds in its S^T accumulator, in that order.
+// A tile's vector arithmetic takes longer than its 48 MFMAs, so it is kept short: the cap in three instructions beside 2^x and 1 / x (ten as
+// written: 1030 rows of 32 heads of 128, capped, 54.5 -> 46.4 us), conversions in pairs.  Two groups of waves on alternate tiles, as the quantised
+// models' kernel has, gave 47.3 and 104.7 us (2048 rows, no cap) against 46.4 and 100.5: the chain of a row block is not what it lasts as long as.
 template <int DQ, int DV>
 __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention_mfma_kernel(const ptm_attention_args a) {
     constexpr int KS = DQ / 16, DT = DV / 32, KP = DQ * 2 + 16, VP = DV * 2 + 64;
@@ -221,7 +224,9 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
             }
         }
     };
-    const float sc2 = a.scale * LOG2E, inv_cap = a.softcap > 0.0f ? 1.0f / a.softcap : 0.0f;
+    const float sc2 = a.scale * LOG2E;
+    // scores in base 2, capped: cap tanh(s / cap) = cap - 2 cap / (2^(s turn) + 1), which ends at +-cap for large arguments
+    const float cap2 = a.softcap * LOG2E, turn = a.softcap > 0.0f ? 2.0f * sc2 / a.softcap : 0.0f;
     fetch_k(tile_at(0));
     fetch_v(tile_at(0));
     for (int it = 0; it < ntiles; ++it) {
@@ -243,12 +248,20 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
         for (int u = 0; u < 2; ++u) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) sc[u][r] = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const at_b8 ka = *reinterpret_cast<const at_b8*>(s_k + (32 * u + j) * KP + (16 * ks + 8 * kh) * 2);
-                sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qf[ks], sc[u], 0, 0, 0);
-            }
         }
+        // four fragments are read at a time, of the two halves in turn: the MFMAs wait for a batch, not each for its own read
+#pragma unroll
+        for (int k4 = 0; k4 < KS; k4 += 4)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                at_b8 ka[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) ka[w] = *reinterpret_cast<const at_b8*>(s_k + (32 * u + j) * KP + (16 * (k4 + w) + 8 * kh) * 2);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) asm volatile("" : "+v"(ka[w]));
+#pragma unroll
+                for (int w = 0; w < 4; ++w) sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[w], qf[k4 + w], sc[u], 0, 0, 0);
+            }
         issue_order_fence();
         fetch_v(next);
         issue_order_fence();
@@ -256,7 +269,7 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sc[u][r] = soft_cap(sc[u][r] * a.scale, a.softcap, inv_cap) * LOG2E;
+                for (int r = 0; r < 16; ++r) sc[u][r] = fmaf(-2.0f * cap2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sc[u][r] * turn) + 1.0f), cap2);
         } else {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -310,10 +323,17 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
             for (int ks = 0; ks < 2; ++ks) {
                 at_b8 hi, lo;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float p = sc[u][8 * ks + i];
-                    hi[i] = (__bf16)p;
-                    lo[i] = (__bf16)(p - (float)hi[i]);
+                for (int i = 0; i < 8; i += 2) {  // two conversions an instruction
+                    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+                    typedef float f2 __attribute__((ext_vector_type(2)));
+                    const f2 p = {sc[u][8 * ks + i], sc[u][8 * ks + i + 1]};
+                    const b2 h = __builtin_convertvector(p, b2);
+                    const f2 rest = {p[0] - (float)h[0], p[1] - (float)h[1]};
+                    const b2 l = __builtin_convertvector(rest, b2);
+                    hi[i] = h[0];
+                    hi[i + 1] = h[1];
+                    lo[i] = l[0];
+                    lo[i + 1] = l[1];
                 }
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) {
