@@ -497,13 +497,12 @@ __global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(cons
     __shared__ float red2[THREADS / 64];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int n4 = K / 4;
-    if (m >= M) {  // padding rows: zeros
-        for (int i = tid; i < n4; i += THREADS) {
-            if (Xh_round) reinterpret_cast<uint2*>(Xh_round + (int64_t)m * K)[i] = make_uint2(0, 0);
-            if (Xh_plain) reinterpret_cast<uint2*>(Xh_plain + (int64_t)m * K)[i] = make_uint2(0, 0);
-        }
-        return;
-    }
+    // the norm weights of a thread's first two pieces go out with the slabs: behind the sums they were a round trip of their own (2048 rows of 4096,
+    // two slabs, 29.2 -> 26.8 us; 19 rows in 72 launches of a prompt 2830 -> 2811)
+    float4 g[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) g[u] = reinterpret_cast<const float4*>(gamma)[min(tid + THREADS * u, n4 - 1)];
+    issue_order_fence();
     const int64_t total = (int64_t)M * K;
     float4* x4 = reinterpret_cast<float4*>(X + (int64_t)m * K);
     for (int i = tid; i < n4; i += THREADS) {
@@ -537,17 +536,23 @@ __global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(cons
     ss = (red[0] + red[1]) + (red[2] + red[3]);
     const float rs = 1.0f / sqrtf(ss / (float)K + eps);
     const float one = add_one ? 1.0f : 0.0f;
-    auto value4 = [&](int i) {
-        const float4 a = reinterpret_cast<const float4*>(rn_row)[i], b = reinterpret_cast<const float4*>(gamma)[i];
+    auto value4 = [&](int i, const float4& b) {
+        const float4 a = reinterpret_cast<const float4*>(rn_row)[i];
         float4 r;
         r.x = a.x * rs * (b.x + one); r.y = a.y * rs * (b.y + one); r.z = a.z * rs * (b.z + one); r.w = a.w * rs * (b.w + one);
         return r;
     };
+    // every piece of a thread: the two whose weights are here, then the rest
+    auto pieces = [&](auto take) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (tid + THREADS * u < n4) take(tid + THREADS * u, value4(tid + THREADS * u, g[u]));
+        for (int i = tid + 2 * THREADS; i < n4; i += THREADS) take(i, value4(i, reinterpret_cast<const float4*>(gamma)[i]));
+    };
     float amax = 0.0f;
-    for (int i = tid; i < n4; i += THREADS) {
-        const float4 v = value4(i);
+    pieces([&](int, const float4& v) {
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
+    });
     amax = max64(amax);
     if ((tid & 63) == 0) red2[tid >> 6] = amax;
     __syncthreads();
@@ -569,8 +574,7 @@ __global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(cons
         o.h[3] = (_Float16)(v.w * down);
         reinterpret_cast<uint2*>(dst)[i] = o.u;
     };
-    for (int i = tid; i < n4; i += THREADS) {  // K % 256 == 0: whole waves, aligned groups of 8 lanes = one Q8 block
-        const float4 v = value4(i);
+    pieces([&](int i, const float4& v) {  // K % 256 == 0: whole waves, aligned groups of 8 lanes = one Q8 block
         if (Xh_plain) store4(Xh_plain + (int64_t)m * K, i, v);
         if (Xh_round) {
             float d, sm;
@@ -582,7 +586,7 @@ __global__ __launch_bounds__(THREADS) void qgemm_reduce_norm_prepare_kernel(cons
             q.w = d * (float)(int)(int8_t)(pk >> 24);
             store4(Xh_round + (int64_t)m * K, i, q);
         }
-    }
+    });
 }
 
 // SiLU(gate) . up (gelu: tanh-GELU) of a short prompt's rows, gate and up still `sg` / `su` slabs of K splits each, into the fp16 rows of the down
@@ -886,7 +890,7 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     const uint8_t* x_src = reinterpret_cast<const uint8_t*>(Xh) + (int64_t)(m0 + (tid >> 5)) * x_row_bytes + 16 * (tid & 31) +
                            (int64_t)blk0 * 512;
     uint8_t* x_dst = s_a + (tid >> 5) * QF_PITCH + 16 * (tid & 31);
-    float* s_rs = reinterpret_cast<float*>(s_a + 2 * TM * QF_PITCH);  // the tile's TM row scales (every padded row has one)
+    float* s_rs = reinterpret_cast<float*>(s_a + 2 * TM * QF_PITCH);  // the tile's TM row scales (of rows past M, like the rows, anything: their sums are not stored)
     if (tid < TM) s_rs[tid] = rowscale[bz * scale_stride + m0 + tid];  // scale_stride 0: a row has one scale, not one per K split
     // the pieces of the next tile in flight (scalars, not an array: they must stay in registers)
     uint4 x0, x1, x2, x3, x4, x5, x6, x7;
@@ -1340,7 +1344,7 @@ int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool acc
     _Float16* hp = static_cast<_Float16*>(ws_plain);
     float* rr = hr ? reinterpret_cast<float*>(hr + (int64_t)mp * K) : nullptr;
     float* rp = hp ? reinterpret_cast<float*>(hp + (int64_t)mp * K) : nullptr;
-#define PTM_RN(B, T) hipLaunchKernelGGL((qgemm_reduce_norm_prepare_kernel<B, T>), dim3(mp), dim3(T), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0, gamma, eps, add_one, hr, rr, hp, rp, M, K)
+#define PTM_RN(B, T) hipLaunchKernelGGL((qgemm_reduce_norm_prepare_kernel<B, T>), dim3(M), dim3(T), (size_t)K * 4, s, P, splits, X, accumulate ? 1 : 0, gamma, eps, add_one, hr, rr, hp, rp, M, K)
     // up to 128 rows the launch lasts as long as one row's chain of requests: as many threads as the row has pieces (4 / 8 / 16 slabs of 2560
     // values 9.4 -> 6.5 us).  Beyond, 512 (953 rows of 4096, two slabs: 256 threads 22.6 us, 512 20.8, 1024 22.3; 509 of 2560, six: 12.1,
     // 11.6, 13.5)
