@@ -391,7 +391,9 @@ int gemv_prologue(const DenseGemv& g) {
 // the vector is staged once per CU and no CU has two rows a wave where another has one (2560 x 9728 on 320 workgroups of 8 waves 12.8 us,
 // on 256 of 10 11.4); a prologue with a norm or streams has 8 waves, the threads of its sums.  More rows: two workgroups of 8 waves a CU.
 // A wave with up to 6 chunks requests them all at once; in other cases the chunks in flight are the 4 or 5 that leave fewer requests
-// past a wave's last row (8 in flight where a wave has 8: 4096 x 4096 9.2 us, 8.5 with 4).
+// past a wave's last row (8 in flight where a wave has 8: 4096 x 4096 9.2 us, 8.5 with 4).  Behind a long prologue (streams, a
+// tail's norm) 8 where they divide a wave's chunks: its first requests are what HBM does meanwhile (Nadozen turns of 30 + 24, width 4096, 14244 us
+// with 4, 13837 with 8; 2560, where gates and ups are 30 chunks a wave, 8337 so and 8452 with 10).
 GemvShape gemv_shape(const DenseGemv& g) {
     const int kp = up64(g.K), lpr = kp <= 64 ? 8 : kp <= 256 ? 32 : 64, pro = gemv_prologue(g);
     const int groups = (int)(((int64_t)g.N * lpr + 63) / 64), per_cu = (groups + 255) / 256;
@@ -399,7 +401,7 @@ GemvShape gemv_shape(const DenseGemv& g) {
     int wgs = (groups + waves - 1) / waves;
     wgs = wgs < 512 ? wgs : 512;
     const int chunks = (groups + wgs * waves - 1) / (wgs * waves) * ((kp / 8 + lpr - 1) / lpr) * (g.epilogue == GEMV_SWIGLU ? 2 : 1);
-    const int depth = chunks == 6 ? 6 : (4 - chunks % 4) % 4 < (5 - chunks % 5) % 5 ? 4 : 5;
+    const int depth = lpr == 64 && pro >= 2 && chunks % 8 == 0 ? 8 : chunks == 6 ? 6 : (4 - chunks % 4) % 4 < (5 - chunks % 5) % 5 ? 4 : 5;
     return {lpr, lpr < 64 && depth > 5 ? 5 : depth, waves, wgs};
 }
 // At most 512 workgroups (one more would run by itself behind the others): as many as its rows fill for a section of few rows,
@@ -431,10 +433,12 @@ static void gemv_attr() {
     PTM_DG(64, 4, PRO, false);
     PTM_DG(64, 5, PRO, false);
     PTM_DG(64, 6, PRO, false);
+    if constexpr (PRO >= 2) PTM_DG(64, 8, PRO, false);
     if constexpr (PRO < 3) {
         PTM_DG(64, 4, PRO, true);
         PTM_DG(64, 5, PRO, true);
         PTM_DG(64, 6, PRO, true);
+        if constexpr (PRO == 2) PTM_DG(64, 8, PRO, true);
     }
 #undef PTM_DG
 }
@@ -454,7 +458,8 @@ static void gemv_launch(const DenseGemv& g, const GemvShape& sh, dim3 grid, size
     else if (sh.lpr == 32) { if (sh.depth == 4) PTM_DG(32, 4); else PTM_DG(32, 5); }
     else if (sh.depth == 4) PTM_DG(64, 4);
     else if (sh.depth == 5) PTM_DG(64, 5);
-    else PTM_DG(64, 6);
+    else if (sh.depth == 6) PTM_DG(64, 6);
+    else if constexpr (PRO >= 2) PTM_DG(64, 8);
 #undef PTM_DG
 }
 template <int PRO>

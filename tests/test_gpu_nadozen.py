@@ -404,3 +404,17 @@ def test_feed_forward_sizes(dev, tmp_path, ff):
         for sizes in ([140], [50, 20, 1]):
             assert_close(portions(m, tokens, sizes), want, precision, (ff, sizes))
         m.close()
+
+
+@pytest.mark.parametrize("width,ff", [(3600, 20), (4096, 4100), (1800, 4200)])
+def test_decoding_at_large_widths(dev, tmp_path, width, ff):
+    """Decode products whose waves have whole rings of 8 chunks behind the streams' sums: one row a wave, two, and a ragged last one."""
+    cfg = model([wkv(2, 8, 4, ff=ff), parallel(2, 1, 16, 9, (2, 4, 7, 1, 2, 2), ff=ff)], width, 33, 2)
+    w = fw.random_weights(cfg, width + ff)
+    tokens = np.random.default_rng(ff).integers(0, 33, 6).tolist()
+    want = N.logits(tokens, w, cfg)
+    path = fw.write_model_folder(str(tmp_path / "m"), cfg, w)
+    for precision in ("float32", "bfloat16"):
+        m = registry.load(path, max_seq=8, precision=precision)
+        assert_close(portions(m, tokens, [1]), want, precision, (width, ff))
+        m.close()
