@@ -216,6 +216,40 @@ def test_prefill_attention_as_rows_of_the_next_product(dev, kv_fp16, nh, nkv, hd
     assert np.array_equal(rows16[:rows].cpu().numpy().view(np.uint16), v.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("q8round", [1, 0])
+@pytest.mark.parametrize("nh,nkv,hd,rows", [(4, 4, 64, 200), (16, 2, 128, 90), (8, 4, 256, 150)])
+def test_prefill_attention_rows_at_the_largest_fp16_values(dev, nh, nkv, hd, rows, q8round):
+    """Averages of values at the end of fp16 stay there: the weights are rounded to fp16 and their sum is not, so a row comes out up to 2^-11 beyond its
+    largest value, and fp16 rounds to infinity from 65520.  Here position 0 weighs 1 and all others a weight of 0.5 .. 0.6 that differs from row to
+    row, a half step of fp16 too high in some of them.  What is not finite stays so."""
+    from gemm_helpers import harness
+    kvd, qd, scale = nkv * hd, nh * hd, hd ** -0.5
+    Kc, Vc = torch.zeros(rows, nkv, hd, device="cuda").half(), torch.zeros(rows, nkv, hd, device="cuda").half()
+    Kc[1:, :, 0] = -1.0
+    Vc[:, :, :32], Vc[:, :, 40] = 65504.0, -65504.0
+    if not q8round:
+        Vc[0, :, 50], Vc[0, :, 51] = float("inf"), float("-inf")
+    Q = torch.zeros(rows, nh, hd, device="cuda")
+    Q[:, :, 0] = -torch.log(torch.linspace(0.5, 0.6, rows, device="cuda"))[:, None] / scale
+    O, O2 = torch.empty(rows, qd, device="cuda"), torch.empty(rows, qd, device="cuda")
+    ops.prefill_attention_window(Q, Kc, Vc, O, rows, nh, nkv, hd, 0, rows, scale, True, 0)
+    rows16, ones, wrote = torch.empty(rows, qd, dtype=torch.float16, device="cuda"), torch.empty(rows, device="cuda"), ctypes.c_int32(-1)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert harness().prefill_rows16(p(Q), p(Kc), p(Vc), p(O2), p(rows16), p(ones), q8round, ctypes.byref(wrote), rows, nh, nkv, hd, ctypes.c_int64(0),
+                                    rows, ctypes.c_float(scale), 1, 0, None) == 0
+    torch.cuda.synchronize()
+    assert wrote.value == 1 and bool((ones == 1).all())
+    v, got = O.double().reshape(rows, nh, hd), rows16.double().reshape(rows, nh, hd)
+    assert float(v[:, :, :32].max()) > 65520 and float(v[:, :, 40].min()) < -65520  # the fp32 rows
+    if q8round:  # blocks of equal values, and of one value among zeros: a level is a 127th of it
+        assert bool(((got[:, :, :32] <= 65504) & (got[:, :, :32] >= 65504 * (1 - 2 ** -10))).all())
+        assert bool(((got[:, :, 40] >= -65504) & (got[:, :, 40] <= -65504 * (1 - 2 ** -10))).all())
+    else:
+        want = torch.where(v.isinf(), v, v.clamp(-65504.0, 65504.0)).half().double()  # NaN (a masked weight of 0 times infinity) is NaN
+        assert torch.equal(*[t.nan_to_num(nan=1e9, posinf=2e9, neginf=-2e9) for t in (got, want)])
+        assert not bool(got[:, :, 50:52].isfinite().any()) and bool(got[:, :, :50].isfinite().all())
+
+
 @pytest.mark.parametrize("qt", [12, 14])
 @pytest.mark.parametrize("M,K,N,sg,su,gelu", [(1, 256, 64, 1, 1, 0), (19, 9728, 2560, 3, 3, 0), (5, 2816, 1024, 4, 1, 1), (33, 4096, 300, 5, 9, 0), (128, 2560, 640, 2, 2, 1),
                                               (2, 14336, 4096, 2, 3, 0)])
