@@ -315,6 +315,8 @@ __global__ __launch_bounds__(PRO == 1 || PRO == 2 ? DG_THREADS : 64 * DG_MAX_WAV
             a.y[row0 + row] = v;
         }
         gd += done * stride;
+        // between the gate and the up row of a value: its gate is in the lane that comes next, from now on the first
+        if (GLU && half == 1) gates = __shfl(gates, lr * LPR + done, 64);
         done = 0;
     };
     auto consume = [&](u32x4& v) {

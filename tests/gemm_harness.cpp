@@ -1,7 +1,8 @@
 // Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
-// splits, which the C ABI's plain product does not have, how a launch would cover its output, and the quantised models' prompt attention and
-// down projection as theirs calls them.  Host C++ only; built by
+// splits, which the C ABI's plain product does not have, how a launch would cover its output, their decode product with its epilogues, and the quantised
+// models' prompt attention and down projection as theirs calls them.  Host C++ only; built by
 // __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
+#include "dense_gemv.h"
 #include "gemm_plan.h"
 #include "ptm.h"
 
@@ -65,6 +66,26 @@ void gemm_plan(const GemmCall* c, int32_t* out) {
         const ptm::GemmRegion& r = p.regions.r[i];
         for (int v : {r.kind, r.first, r.m0, r.n0, r.n1, r.tiles_m, r.tiles_n}) *out++ = v;
     }
+}
+
+// y = W . x with one of the epilogues a decode step has; blend (optional): x is a stream of that weight.  GEMV_ARGMAX: (value, index) of
+// every workgroup to part_val, part_idx (room for 512); the number of workgroups is returned in *wgs.
+int gemv_run(const void* W, const float* x, float* y, int K, int N, int64_t ld, int epilogue, const float* blend, float* part_val, int* part_idx, int* wgs,
+             void* stream) {
+    ptm::DenseGemv g;
+    g.W = static_cast<const uint16_t*>(W);
+    g.x = x;
+    g.y = y;
+    g.K = K;
+    g.N = N;
+    g.ld = ld;
+    g.epilogue = epilogue;
+    g.streams = blend ? 1 : 0;
+    g.blend = blend;
+    g.part_val = part_val;
+    g.part_idx = part_idx;
+    *wgs = ptm::dense_gemv_workgroups(g);
+    return ptm::dense_gemv(g, static_cast<hipStream_t>(stream));
 }
 
 // prompt attention that leaves the rows of the next product; *wrote: whether it did (else O has the rows)

@@ -347,6 +347,51 @@ def test_dense_gemv_many_rows(dev, N, K):
     assert float((y[:N] - ref).abs().max()) < 2e-6 * K ** 0.5 * float(ref.std()) + 1e-5 and bool((y[N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("streams,N,K", [(1, 245760, 2560), (1, 475136, 1536), (1, 300000, 200), (0, 70001, 64), (0, 200001, 300), (0, 270000, 520)])
+def test_dense_gemv_gate_up_many_rows(dev, streams, N, K):
+    """silu(gate) . up where a wave finishes more values than it has lanes to keep them, which may happen between a value's gate and its up row."""
+    import ctypes as C
+    import torch
+    from gemm_helpers import harness
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    kp = (K + 63) // 64 * 64
+    W = torch.zeros(2 * N, kp, dtype=torch.bfloat16, device="cuda")
+    x, blend = torch.zeros(kp, device="cuda"), torch.ones(2, device="cuda")
+    x[:K] = torch.randn(K, device="cuda", generator=g)
+    sums = torch.empty(2 * N, dtype=torch.float64, device="cuda")
+    for r in range(0, 2 * N, 1 << 15):
+        W[r:r + (1 << 15), :K] = torch.randn(min(1 << 15, 2 * N - r), K, device="cuda", generator=g)
+        sums[r:r + (1 << 15)] = W[r:r + (1 << 15)].double() @ x.double()
+    y, wgs, p = torch.full((N + 3,), 7.0, device="cuda"), C.c_int32(), lambda t: C.c_void_p(t.data_ptr())
+    assert harness().gemv_run(p(W), p(x), p(y), K, N, C.c_int64(kp), 4, p(blend) if streams else None, None, None, C.byref(wgs), None) == 0
+    gate, up = sums[:N], sums[N:]
+    # a sum is off by up to the bound of test_dense_gemv; silu's slope is at most 1.1
+    off = 2e-6 * K ** 0.5 * float(sums.std()) + 1e-5
+    err = (y[:N] - torch.nn.functional.silu(gate) * up).abs()
+    assert bool((err <= off * (1.1 * up.abs() + gate.abs() + 1)).all()) and bool((y[N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("N,K", [(270000, 64), (270000, 300), (5000, 2560)])
+def test_dense_gemv_argmax_many_rows(dev, N, K):
+    """The largest value and its first row over all finished sums of a wave, with equal values in many rows."""
+    import ctypes as C
+    import torch
+    from gemm_helpers import harness
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    kp = (K + 63) // 64 * 64
+    W = torch.zeros(N, kp, dtype=torch.bfloat16, device="cuda")
+    x, y, wgs = torch.zeros(kp, device="cuda"), torch.empty(N, device="cuda"), C.c_int32()
+    x[:K] = torch.randn(K, device="cuda", generator=g)
+    W[:, :K] = torch.randn(N, K, device="cuda", generator=g)
+    best = torch.randint(N // 3, N, (7,), device="cuda", generator=g)
+    W[best, :K] = torch.where(x[:K] > 0, 4.0, -4.0).to(torch.bfloat16)
+    val, idx, p = torch.full((512,), -9e9, device="cuda"), torch.full((512,), -1, dtype=torch.int32, device="cuda"), lambda t: C.c_void_p(t.data_ptr())
+    assert harness().gemv_run(p(W), p(x), p(y), K, N, C.c_int64(kp), 3, None, p(val), p(idx), C.byref(wgs), None) == 0
+    val, idx = val[:wgs.value], idx[:wgs.value]
+    assert float(val.max()) == float(y.max()) and int(idx[val == val.max()].min()) == int(best.min())
+    assert torch.equal(y[idx.long()], val)
+
+
 @pytest.mark.parametrize("fp32", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1, 3, 8), (2, 70, 40), (31, 257, 100), (33, 65, 320), (64, 64, 64), (100, 130, 192),
                                    (150, 1000, 72), (300, 4100, 200), (1030, 2050, 136)])
