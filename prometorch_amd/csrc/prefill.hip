@@ -206,14 +206,11 @@ struct QkvRuns {
     }
 };
 
-
 // The same work with head_dim / 8 lanes per head (head_dim 32, 64, 128 or 256) and 16-byte accesses: a lane owns four
 // rotation pairs (two runs of four elements), a wave 64 / (head_dim / 8) heads of one row.  grid (rows, q head blocks + kv
 // head blocks), one wave.  With one wave per (row, head) and 4-byte accesses the launch was bound by the number of
 // workgroups and requests: 82 k single-wave workgroups for 2048 rows of 40 heads.
-// B: slabs per batch (PART).  A short prompt's launch is its requests' round trips, so a row's slabs (up to 16), the rotation and the norm weights go
-// out together; a long one's rows have one slab, and requesting it four times over cost it the texture path
-// (four at a time, q before k before v, the tables last: 19 rows of 40 heads 7.0 -> 3.8 us, 2048 24.7 -> 18.8 ... 21.3).
+// B: slabs per batch (PART): the first B slabs of a lane's runs, the rotation and the norm weights go out together (qknorm_slabs_per_batch).
 template <bool KV16, bool PART, int B>
 __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __restrict__ Q, float* __restrict__ K,
                                                                       const float* __restrict__ V, const float* __restrict__ qw,
@@ -326,6 +323,19 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_rows_quad_kernel(float* __r
     }
 }
 
+// Slabs per batch of rows that are up to `most` slabs, in a launch of that many waves.  A launch that lies on the chip as a whole lasts as long as its
+// round trips, so a row's slabs are requested together, up to eight; a larger one lives off the waves a SIMD holds: 2 with eight slabs (170
+// registers), 4 with four (110), 7 with two (72), 8 with one (62).  So: as many as leave all waves on the chip's 1024 SIMDs, one beyond.  Eight
+// against one, 40 heads of 128 in five slabs, 19 / 200 / 256 rows: 3.1 / 6.8 / 8.6 us and 3.6 / 7.1 / 8.1 (four slabs there 8.1); four against one, two to four
+// slabs, 257 / 400 / 509 / 1024 rows: 5.5 / 6.9 / 8.7 / 17.4 and 5.8 / 7.1 / 8.0 / 16.5; two against one, two slabs of 20 heads of 64, 19 / 2048 rows 2.49 / 7.30
+// and 2.63 / 7.40, of 12 of 256, 2048 rows 19.8 and 19.1; four of one slab (three of them requests for the same) 22.1 us at 2048 rows, one 19.6.
+int qknorm_slabs_per_batch(int most, int64_t waves) {
+    if (most > 4 && waves <= 2 * 1024) return 8;
+    if (most > 2 && waves <= 4 * 1024) return 4;
+    if (most == 2 && waves <= 7 * 1024) return 2;
+    return 1;
+}
+
 // launches the 16-byte kernel when the shape and the pointers allow it, the one-wave-per-head kernel otherwise
 template <bool PART>
 static int qknorm_rope_kv_rows_launch(float* Q, float* K, const float* V, const float* q_norm_w, const float* k_norm_w,
@@ -344,14 +354,15 @@ static int qknorm_rope_kv_rows_launch(float* Q, float* K, const float* V, const 
         const dim3 grid(rows, (n_heads + hpw - 1) / hpw + (n_kv_heads + hpw - 1) / hpw);
         int most = 1;
         for (int i = 0; i < 3; ++i) most = parts.splits[i] > most ? parts.splits[i] : most;
-        if (!PART || most <= 1) {
+        const int batch = PART ? qknorm_slabs_per_batch(most, (int64_t)grid.x * grid.y) : 1;
+        if (batch == 1) {
             if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 1);
             else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 1);
         } else if constexpr (PART) {
-            if (most <= 2) {
+            if (batch == 2) {
                 if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 2);
                 else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 2);
-            } else if (most <= 4) {
+            } else if (batch == 4) {
                 if (kv_fp16) PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, true, PART, 4);
                 else PTM_QK(qknorm_rope_kv_rows_quad_kernel, grid, false, PART, 4);
             } else {

@@ -1,6 +1,6 @@
 // Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
 // splits, which the C ABI's plain product does not have, how a launch would cover its output, their decode product with its epilogues, and the quantised
-// models' prompt attention and down projection as theirs calls them.  Host C++ only; built by
+// models' prompt attention, QK-norm and down projection as theirs calls them.  Host C++ only; built by
 // __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
 #include "dense_gemv.h"
 #include "gemm_plan.h"
@@ -15,6 +15,11 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
                    hipStream_t s, int* deferred_splits, bool split_scales);
 int qgemm_f16_blocks_per_split(int N, int K, int M, size_t split_ws_bytes);
 int64_t qgemm_f16_split_scale_bytes(int M);
+int qknorm_slabs_per_batch(int most, int64_t waves);
+int qknorm_rope_kv_rows_from_parts(const float* const* P, const int* splits, const float* const* bias, float* Q,
+                                   const float* q_norm_w, const float* k_norm_w, void* K_cache, void* V_cache,
+                                   const float* rope_table, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0,
+                                   int max_seq, float eps, int add_one, int kv_fp16, int rope_interleaved, hipStream_t s);
 int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
 }
 
@@ -97,6 +102,14 @@ int prefill_rows16(const float* Q, const void* K, const void* V, float* O, void*
     *wrote = w ? 1 : 0;
     return rc;
 }
+
+// QK-norm, rotation and append of rows that are still splits[i] slabs of q, k, v
+int qk_rows(const float* const* P, const int* splits, const float* const* bias, float* Q, const float* qw, const float* kw, void* K, void* V, const float* rope,
+            int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq, int kv_fp16, int interleaved, void* stream) {
+    return ptm::qknorm_rope_kv_rows_from_parts(P, splits, bias, Q, qw, kw, K, V, rope, rows, n_heads, n_kv_heads, head_dim, pos0, max_seq, 1e-6f, 0, kv_fp16,
+                                               interleaved, static_cast<hipStream_t>(stream));
+}
+int qk_rows_batch(int most, int64_t waves) { return ptm::qknorm_slabs_per_batch(most, waves); }
 
 int64_t act_down_bytes(int M, int K) { return ptm_qgemm_f16_workspace_bytes(M, K) + ptm::qgemm_f16_split_scale_bytes(M); }
 // Y = down . (act(gate) . up) of rows that are still slabs, in ws of act_down_bytes

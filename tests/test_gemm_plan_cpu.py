@@ -1,9 +1,10 @@
 """CPU: which tiles cover a prompt product of more than 64 rows, and where a launch of 64 x 64 tiles of four waves takes it instead."""
+import ctypes
 import random
 
 import pytest
 
-from gemm_helpers import DECAY, ELEM, F32, RELU2, SWIGLU, TILES, plan
+from gemm_helpers import DECAY, ELEM, F32, RELU2, SWIGLU, TILES, harness, plan
 from test_gpu_gemm_tiles import LARGE
 
 
@@ -78,3 +79,16 @@ def test_the_gpu_cases_reach_every_kind_of_tile_and_region():
     assert columns >= {(e, False) for e in (ELEM, RELU2, SWIGLU, DECAY)} | {(F32, True)}
     assert splits >= {(3, False), (4, False), (6, False), (5, True)}
     assert max(len(plan(*c)[2]) for c in LARGE) == 3
+
+
+def test_slabs_of_a_qknorm_batch():
+    """A batch takes no more slabs than leave all of a launch's waves on the chip (1024 SIMDs with 2 / 4 / 7 waves of eight / four / two slabs), and never
+    fetches a slab twice over where a smaller batch has them all."""
+    h = harness()
+    h.qk_rows_batch.argtypes = [ctypes.c_int, ctypes.c_int64]
+    for most in range(1, 17):
+        for waves in (1, 2048, 2049, 4096, 4097, 7168, 7169, 20480, 1 << 33):
+            b = h.qk_rows_batch(most, waves)
+            assert b in (1, 2, 4, 8) and (b == 1 or waves <= {8: 2048, 4: 4096, 2: 7168}[b]) and b < 2 * most
+    assert [h.qk_rows_batch(m, 190) for m in (1, 2, 3, 4, 5, 16)] == [1, 2, 4, 4, 8, 8]
+    assert [h.qk_rows_batch(5, w) for w in (2048, 2049, 4096, 4097)] == [8, 4, 4, 1]

@@ -216,6 +216,42 @@ def test_prefill_attention_as_rows_of_the_next_product(dev, kv_fp16, nh, nkv, hd
     assert np.array_equal(rows16[:rows].cpu().numpy().view(np.uint16), v.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("nh,nkv,hd,splits,rows", [
+    (32, 8, 128, (5, 5, 5), (1, 204, 205, 409, 410)), (32, 8, 128, (4, 4, 8), (204, 205)), (8, 4, 256, (4, 3, 5), (341, 342, 682, 683)),
+    (32, 8, 128, (3, 2, 2), (409, 410)), (28, 4, 128, (9, 16, 1), (30, 257, 513)), (16, 4, 64, (2, 2, 2), (2389, 2390)), (6, 2, 32, (1, 2, 5), (50,)), (32, 8, 128, (1, 1, 1), (70,))])
+@pytest.mark.parametrize("kv_fp16,bias,interleaved", [(1, 0, 0), (0, 1, 1)])
+def test_qknorm_of_rows_in_slabs(dev, nh, nkv, hd, splits, rows, kv_fp16, bias, interleaved):
+    """q, k, v rows that are still partial sums, with as many slabs a batch as a launch of that size takes (rows on both sides of each line): bit for bit the
+    result of rows whose slabs were added beforehand in their order."""
+    from gemm_helpers import harness
+    h, widths, p = harness(), (nh * hd, nkv * hd, nkv * hd), lambda t: t.data_ptr() if t is not None else None
+    r = synth.rng_for(75, nh, hd, *splits)
+    dt = torch.float16 if kv_fp16 else torch.float32
+    for M in rows:
+        cap = M + 3
+        parts = [torch.randn(s, M, w, device="cuda", generator=torch.Generator(device="cuda").manual_seed(M + s)) for s, w in zip(splits, widths)]
+        b3 = [cu(synth.make_x(r, w)) if bias else None for w in widths]
+        qw, kw = [cu(1 + 0.1 * synth.make_x(r, hd)) for _ in range(2)]
+        table, res = ops.rope_table(cap, hd, 1e4).cuda(), []
+        for summed in (0, 1):
+            P = parts
+            if summed:
+                P = []
+                for t in parts:
+                    acc = t[0].clone()
+                    for z in range(1, len(t)):
+                        acc += t[z]
+                    P.append(acc)
+            Q = torch.full((M + 1, widths[0]), 7.0, device="cuda")
+            Kc, Vc = torch.full((cap + 1, widths[1]), 7.0, dtype=dt, device="cuda"), torch.full((cap + 1, widths[1]), 7.0, dtype=dt, device="cuda")
+            assert h.qk_rows((ctypes.c_void_p * 3)(*[p(t) for t in P]), (ctypes.c_int * 3)(*([1] * 3 if summed else splits)), (ctypes.c_void_p * 3)(*[p(t) for t in b3]),
+                             *[ctypes.c_void_p(p(t)) for t in (Q, qw, kw, Kc, Vc, table)], M, nh, nkv, hd, ctypes.c_int64(3), cap, kv_fp16, interleaved, None) == 0
+            torch.cuda.synchronize()
+            assert bool((Q[M] == 7).all()) and bool((Kc[:3] == 7).all()) and bool((Kc[cap] == 7).all()) and bool((Vc[:3] == 7).all()) and bool((Vc[cap] == 7).all())
+            res.append((Q, Kc, Vc))
+        assert all(torch.equal(a, b) for a, b in zip(*res)), M
+
+
 @pytest.mark.parametrize("q8round", [1, 0])
 @pytest.mark.parametrize("nh,nkv,hd,rows", [(4, 4, 64, 200), (16, 2, 128, 90), (8, 4, 256, 150)])
 def test_prefill_attention_rows_at_the_largest_fp16_values(dev, nh, nkv, hd, rows, q8round):
