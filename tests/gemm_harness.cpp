@@ -1,6 +1,6 @@
 // Test harness (not part of the library): the block decoders' prompt product as their runtime calls it, with its epilogues, sections and K
 // splits, which the C ABI's plain product does not have, how a launch would cover its output, their decode product with its epilogues, and the quantised
-// models' prompt attention, QK-norm and down projection as theirs calls them.  Host C++ only; built by
+// models' prompt attention, QK-norm, q / k / v and gate / up products and down projection as theirs calls them.  Host C++ only; built by
 // __graft_entry__.build() into tests/libshim_harness.so and driven through ctypes by tests/gemm_helpers.py.
 #include "dense_gemv.h"
 #include "gemm_plan.h"
@@ -20,6 +20,12 @@ int qknorm_rope_kv_rows_from_parts(const float* const* P, const int* splits, con
                                    const float* q_norm_w, const float* k_norm_w, void* K_cache, void* V_cache,
                                    const float* rope_table, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0,
                                    int max_seq, float eps, int add_one, int kv_fp16, int rope_interleaved, hipStream_t s);
+int qgemm_f16_prepare_fused(int pre, const float* X, const float* X2, float eps, int add_one, void* ws_round, void* ws_plain, int M, int K, hipStream_t s);
+int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const int64_t* strides, const int* N, float* const* Y,
+                    int M, int K, void* ws_round, void* ws_plain, float* split_ws, size_t split_ws_bytes, hipStream_t s,
+                    const float** deferred_P, int* deferred_splits);
+size_t qgemm_f16_multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M);
+void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits);
 int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
 }
 
@@ -110,6 +116,16 @@ int qk_rows(const float* const* P, const int* splits, const float* const* bias, 
                                                interleaved, static_cast<hipStream_t>(stream));
 }
 int qk_rows_batch(int most, int64_t waves) { return ptm::qknorm_slabs_per_batch(most, waves); }
+
+// Y[i] = RMSNorm(X; gamma) . W[i]^T of up to three matrices in one launch; P / splits (optional): their slabs instead
+int multi_run(int n, const uint32_t* types, const void* const* W, const int64_t* strides, const int* N, float* const* Y, const float* X, const float* gamma, int M,
+              int K, void* ws_round, void* ws_plain, float* split_ws, int64_t split_bytes, const float** P, int* splits, void* stream) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int rc = ptm::qgemm_f16_prepare_fused(1, X, gamma, 1e-6f, 0, ws_round, ws_plain, M, K, s);
+    return rc ? rc : ptm::qgemm_f16_multi(n, types, W, strides, N, Y, M, K, ws_round, ws_plain, split_ws, (size_t)split_bytes, s, P, splits);
+}
+int64_t multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M) { return (int64_t)ptm::qgemm_f16_multi_split_bytes(n, N, types, K, M); }
+void multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits) { ptm::qgemm_f16_multi_plan(n, N, types, K, M, splits); }
 
 int64_t act_down_bytes(int M, int K) { return ptm_qgemm_f16_workspace_bytes(M, K) + ptm::qgemm_f16_split_scale_bytes(M); }
 // Y = down . (act(gate) . up) of rows that are still slabs, in ws of act_down_bytes

@@ -226,3 +226,62 @@ def test_short_prompts_whose_last_split_is_shorter(dev, po, qt, M, K, N):
         ops.matmul_q_f16_f32(qt, Wd, x[:m].contiguous(), y, m, K, N, W.shape[1], ws, accumulate=False)
         out.append(y.cpu().numpy()[:M])
     assert np.array_equal(bits(out[0]), bits(out[1]))
+
+
+# super-blocks of the longest split of each matrix; types in file order, K that does not divide evenly among the splits, N off the 128-column tiles
+@pytest.mark.parametrize("K,N,types,blocks", [(2560, (4097, 1000, 129), (12, 12, 14), (3, 3, 2)), (2560, (13000, 1000, 515), (14, 12, 12), (3, 4, 4)),
+                                              (4096, (13000, 1000, 515), (12, 14, 14), (4, 2, 3)), (4096, (5000, 700), (14, 12), (2, 3)), (2560, (20000, 300), (12, 14), (4, 2)),
+                                              (1792, (9728, 9728), (12, 12), (3, 3)), (1024, (1000, 70000), (12, 14), (4, 4))])
+def test_short_prompts_of_several_matrices(dev, po, K, N, types, blocks):
+    """q / k / v and gate / up of up to 32 rows: unequal K splits and kinds of weights side by side, shorter last splits.  Rows are the rows of a 40-row call, which
+    has the same splits and another kernel, bit for bit, as sums and as the slabs that a later launch adds; and the product in 64 bits."""
+    import ctypes as C
+    from gemm_helpers import harness
+    h, n, nblk = harness(), len(N), K // 256
+    h.multi_split_bytes.restype = C.c_int64
+    Ns, ts, sp = (C.c_int * n)(*N), (C.c_uint32 * n)(*types), (C.c_int * n)()
+    h.multi_plan(n, Ns, ts, K, 32, sp)
+    assert tuple(-(-nblk // s) for s in sp) == blocks
+    r = synth.rng_for(49, K, *N)
+    Wh = [synth.make_weight(r, t, rows, K) for t, rows in zip(types, N)]
+    W = [torch.from_numpy(w).cuda() for w in Wh]
+    gamma = torch.from_numpy((1 + 0.1 * r.standard_normal(K)).astype(np.float32)).cuda()
+    X = torch.from_numpy(r.standard_normal((40, K), dtype=np.float32)).cuda()
+    ptrs = lambda ts: (C.c_void_p * n)(*[t.data_ptr() for t in ts])
+    p = lambda t: C.c_void_p(t.data_ptr())
+
+    def run(M, deferred):
+        ws = [torch.zeros(ops.qgemm_f16_workspace_bytes(M, K), dtype=torch.uint8, device="cuda") for _ in range(2)]
+        room = h.multi_split_bytes(n, Ns, ts, K, M)
+        split = torch.full((max(room // 4, 4),), 5.0, device="cuda")
+        Y = [torch.full((M, rows), 3.0, device="cuda") for rows in N]
+        P, s = (C.c_void_p * n)(), (C.c_int * n)()
+        rc = h.multi_run(n, ts, ptrs(W), (C.c_int64 * n)(*[w.shape[1] for w in Wh]), Ns, ptrs(Y), p(X), p(gamma), M, K, p(ws[0]), p(ws[1]), p(split),
+                         C.c_int64(split.numel() * 4), P if deferred else None, s if deferred else None, None)
+        assert rc == 0
+        torch.cuda.synchronize()
+        if not deferred:
+            return Y
+        out = []
+        for i in range(n):
+            at = (P[i] - split.data_ptr()) // 4
+            out.append(Y[i][None] if s[i] == 1 else split[at:at + s[i] * M * N[i]].reshape(s[i], M, N[i]))
+        return out
+
+    many, slabs = run(40, False), run(40, True)
+    for M in (1, 19, 32):
+        for i, (a, b) in enumerate(zip(run(M, False), many)):
+            assert torch.equal(a, b[:M]), (M, i)
+        for i, (a, b) in enumerate(zip(run(M, True), slabs)):
+            assert torch.equal(a, b[:, :M]), (M, i)
+    x = X.double() / (X.double().pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * gamma.double()
+    for i, (t, rows) in enumerate(zip(types, N)):
+        xt = x
+        if t == 12:
+            b = x.reshape(40, -1, 32)
+            d = b.abs().amax(2, keepdim=True) / 127
+            xt = (torch.round(b / d) * d).reshape(40, K)
+        want = xt @ torch.from_numpy(po.dequant(t, Wh[i])).cuda().double().reshape(rows, K).T
+        err = float((many[i].double() - want).abs().max() / want.pow(2).mean().sqrt())
+        print("max err / rms: %.2e" % err, flush=True)
+        assert err <= QGEMM_F16_TOL, (i, err)
