@@ -1660,7 +1660,8 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
     if (o_q8 && (reinterpret_cast<uintptr_t>(o_q8) & 15u)) return PTM_E_ALIGN;
     if (kv_fp16) {
         // fp16 cache: the matrix-core kernel, chunks of 64 positions; partial maxima in base-2 units
-        // All positions in one workgroup's waves: up to 128, with heads of 64 two tiles a wave for up to 256.  Eight steps, 16 layers of 16 heads
+        // All positions in one workgroup's waves: a cache with room for up to 128, with heads of 64 two tiles a wave for up to 256.  The room decides and
+        // not the position, which a captured step learns on the device: a cache of thousands takes the kernels below at every position.  Eight steps, 16 layers of 16 heads
         // of 64, 30 / 77 / 150 / 240 positions: 2865 / 2874 / 2911 / 2900 us, one tile 2591 / 2610, two 2655 / 2664 / 2713 / 2763 (16 waves of one
         // 2694 / 2713 / 2802 / 2887); 8 layers of 32 heads of 128, 20 / 110 / 150 / 235: 2849 / 2866 / 2851 / 2861, 2662 / 2751, and 2700 /
         // 2772 / 2814 / 2889 with two tiles: there half a CU's LDS traffic per head costs what the merge launch does.
