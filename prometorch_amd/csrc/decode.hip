@@ -54,6 +54,7 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
 int qgemm_f16_reduce_norm_prepare(const float* P, int splits, float* X, bool accumulate, const float* gamma, float eps,
                                   int add_one, void* ws_round, void* ws_plain, int M, int K, hipStream_t s);
 int qgemm_f16_splits(int N, int K, int M);
+float qgemm_f16_rounds(int tiles, int M, bool q4);
 int qgemm_f16_blocks_per_split(int N, int K, int M, size_t split_ws_bytes);
 int64_t qgemm_f16_split_scale_bytes(int M);
 bool qgemm_f16_act_rows_fit(int bps, int M, int K);
@@ -471,9 +472,9 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
         pending = 0;
         bool act_split = false;  // the down projection's rows have a scale per K split
         {
-            // Gate and up share one launch when that fills the chip better.  The eight-wave tile runs one workgroup per CU, so
-            // a launch costs ceil(tiles / 256) workgroup times: 2048 rows are 38 x 16 = 608 tiles per matrix, 3 + 3 rounds
-            // apart and 5 together; 512 rows, 152 tiles each, gain nothing (1 + 1 against 2).  Up to 256 rows (the two
+            // Gate and up share one launch when that fills the chip better: a tile is a workgroup and has a CU to itself, so a launch takes whole
+            // rounds of 256 (qf_tall).  512 rows of 9728: 152 tiles of 128 rows each, apart two rounds; together 152 of 256 rows, 1.75 (85 -> 70 us);
+            // 2048 rows: 2.75 + 2.75 apart and 4.75 together.  Up to 256 rows (the two
             // short row classes) always together: one launch less, and the launch is the cost there.  Beyond, only when both
             // ways use the same K splits, so that the choice changes no result.
             const uint32_t t2[2] = {L.gate.ggml_type, L.up.ggml_type};
@@ -482,10 +483,10 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
             if (!together) {
                 int sp2[2];
                 qgemm_f16_multi_plan(2, N2, t2, (int)H, M, sp2);
-                const int row_tiles = (M + 127) / 128;
-                const int tg = (N2[0] + 255) / 256 * row_tiles * sp2[0], tu = (N2[1] + 255) / 256 * row_tiles * sp2[1];
+                const int tg = (N2[0] + 255) / 256 * sp2[0], tu = (N2[1] + 255) / 256 * sp2[1];
+                const bool g4 = t2[0] == PTM_TYPE_Q4_K, u4 = t2[1] == PTM_TYPE_Q4_K;
                 together = sp2[0] == qgemm_f16_splits(N2[0], (int)H, M) && sp2[1] == qgemm_f16_splits(N2[1], (int)H, M) &&
-                           (tg + tu + 255) / 256 < (tg + 255) / 256 + (tu + 255) / 256;
+                           qgemm_f16_rounds(tg + tu, M, g4 && u4) < qgemm_f16_rounds(tg, M, g4) + qgemm_f16_rounds(tu, M, u4);
             }
             if (together) {
                 const void* W2[2] = {L.gate.data, L.up.data};

@@ -16,9 +16,11 @@
 // Q6_K (reference row semantics: cpu_quant_gemv.h:883-1020, fp32 activations)
 //   v_mfma_f32_16x16x16_bf16: K = 16 is exactly one scale group of Q6_K.  (q - 32) is exact in bf16 and
 //   X is bf16 by contract, so products are exact; each 16-group sum is scaled by d*scale[n] in fp32.
+#include "gemm_tile.h"
 #include "ptm_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 namespace ptm {
 
@@ -270,9 +272,8 @@ __global__ __launch_bounds__(256) void qgemm_q6k_kernel(const uint8_t* __restric
 //   instruction per pair).  v_mfma_f32_32x32x16_f16 accumulates in fp32 over the whole K, so there is NO per-sub-
 //   block epilogue: VALU work is the dequantisation only, and it is amortised over the 128 rows of X a workgroup
 //   owns.  Result = reference GEMV up to fp16 rounding of the operands (relative 2^-12 per element).
-//   Workgroup: 128 rows of X x 256 columns (wave w: columns 64w..64w+63 = two 32-wide MFMA tiles, all 128 rows =
-//   four 32-high tiles; 8 accumulator tiles = 128 VGPRs).  A 128 x 32 fp16 tile of X per sub-block step is shared
-//   through LDS (double-buffered); each wave dequantises only its own columns.
+//   Workgroup: 32 to 256 rows of X x 256 (128) columns, a 32-column strip a wave; the rows of X are shared through LDS
+//   (double-buffered) and each wave dequantises only its own columns.
 //   The summation index of the MFMA is free to permute: lane half kh takes the 16 CONSECUTIVE elements
 //   [16 kh, 16 kh + 16) of a 32-wide sub-block (first 8 in k-step 0, next 8 in k-step 1), for A and B alike, so a
 //   lane's weights of one sub-block come from one 16-byte load.
@@ -685,6 +686,8 @@ __device__ __forceinline__ void bytes_to_frags(const uint32_t (&b)[4], float bia
 __device__ __forceinline__ void pin4(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
 // ---- per-type weight access: what a lane (column n, element half kh) fetches of a 256-wide super-block ----
+struct Q4Half;
+struct Q6Half;
 struct Q4Tile {  // Q4_K: header + the lane's 16 bytes of each of the 4 groups of 64
     uint4 hdr;
     uint4 qs[4];
@@ -714,6 +717,7 @@ struct Q4Tile {  // Q4_K: header + the lane's 16 bytes of each of the 4 groups o
     }
     static constexpr int kBlockBytes = 144;
     static constexpr bool kQ8Round = true;
+    typedef Q4Half Half;
 };
 struct Q6Tile {  // Q6_K: the lane's 16 bytes of ql for each (half, pair), of qh for each half, scales, d
     uint4 ql[4], qh[2], sc;
@@ -748,6 +752,7 @@ struct Q6Tile {  // Q6_K: the lane's 16 bytes of ql for each (half, pair), of qh
     }
     static constexpr int kBlockBytes = 210;
     static constexpr bool kQ8Round = false;
+    typedef Q6Half Half;
 };
 
 // Where a workgroup's accumulators go.
@@ -994,6 +999,173 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     qf_store<MT>(acc, s_rs, Y, partials, accumulate, M, N, m0, n_base, j, kh, bz);
 }
 
+// ---- 256 rows x 256 columns ----
+// A wave has one strip of 32 columns and all 256 rows (128 accumulators), so each unpacked weight serves twice the products of the 128-row tile, whose
+// time is its matrix and its unpacking instructions one after the other.  A stage is half a super-block: X goes from memory to LDS directly, two stages
+// of 64 KB, and the loop is laid out by hand: behind every MFMA the read of the fragment eight MFMAs on into the registers it has just freed, a
+// piece of the next sub-block's weights behind every fourth, and one barrier a stage, between the last reads of its LDS and the first of the
+// next, with MFMAs on either side.  The same products in the same order as in the 128-row tile: same bits.
+// What bounds it: 2048 x 14336 x 4096 in 235 us (265 in 128-row tiles), Q6_K 2048 x 4096 x 14336 238 (326), 1020 TFLOP/s; the matrix cores are busy 66 %
+// of the clocks of a CU at work (41 % before), at which the card lowers its clock (about 1.7 GHz).  Where the barrier lies, when the weights are
+// requested and how the pieces are spread change it by less than 1 %.  The same loop for 128 rows is 1 to 5 % slower than qgemm_f16_body.
+
+// What a lane (column n, element half kh) holds of half a super-block, and the fragments of its four sub-blocks, four pieces each.
+struct Q4Half {
+    uint4 hdr, qs[2];
+    uint32_t sc4, mn4;
+    __device__ __forceinline__ void load(const uint8_t* blk, int half, int kh) {
+        hdr = *reinterpret_cast<const uint4*>(blk);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) qs[g] = *reinterpret_cast<const uint4*>(blk + 16 + 64 * half + 32 * g + 16 * kh);
+    }
+    // scales and mins of the four sub-blocks, a byte each (q4k_scale_min)
+    __device__ __forceinline__ void arrive(int half, int) {
+        pin4(hdr); pin4(qs[0]); pin4(qs[1]);
+        sc4 = half ? (hdr.w & 0x0f0f0f0fu) | ((hdr.y >> 2) & 0x30303030u) : hdr.y & 0x3f3f3f3fu;
+        mn4 = half ? ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3f3f3f3fu;
+    }
+    __device__ __forceinline__ void scale(int s, h2& sc, h2& of) const {
+        const float dsc = h2f(hdr.x) * (float)((sc4 >> (8 * s)) & 0xffu), dmn = h2f(hdr.x >> 16) * (float)((mn4 >> (8 * s)) & 0xffu);
+        sc = {(_Float16)dsc, (_Float16)dsc};
+        of = {(_Float16)-dmn, (_Float16)-dmn};
+    }
+    __device__ __forceinline__ uint32_t bytes(int s, int w) const {
+        const uint32_t r[4] = {qs[s >> 1].x, qs[s >> 1].y, qs[s >> 1].z, qs[s >> 1].w};
+        return (r[w] >> (4 * (s & 1))) & 0x0f0f0f0fu;
+    }
+    static constexpr float kBias = 0.0f;
+    static constexpr int kBlockBytes = 144;
+};
+struct Q6Half {
+    uint4 ql[2], qh;
+    uint32_t s0, s1, d;
+    __device__ __forceinline__ void load(const uint8_t* blk, int half, int kh) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) ql[c] = ld16_a2(blk + 64 * half + 32 * c + 16 * kh);
+        qh = ld16_a2(blk + 128 + 32 * half + 16 * kh);
+        s0 = ld_u32_a2(blk + 192 + 8 * half);
+        s1 = ld_u32_a2(blk + 196 + 8 * half);
+        d = reinterpret_cast<const u16_a2*>(blk + 208)->v;
+    }
+    __device__ __forceinline__ void arrive(int, int kh) {
+        pin4(ql[0]); pin4(ql[1]); pin4(qh);
+        asm volatile("" : "+v"(s0), "+v"(s1), "+v"(d));
+        s0 >>= 8 * kh;  // scales 2 s + kh in bytes 0 and 2
+        s1 >>= 8 * kh;
+    }
+    __device__ __forceinline__ void scale(int s, h2& sc, h2& of) const {
+        const int sv = (int)(int8_t)(((s >> 1 ? s1 : s0) >> (16 * (s & 1))) & 0xffu);
+        const float v = h2f(d) * (float)sv;
+        sc = {(_Float16)v, (_Float16)v};
+        of = {(_Float16)0.0f, (_Float16)0.0f};
+    }
+    __device__ __forceinline__ uint32_t bytes(int s, int w) const {
+        const uint32_t l[4] = {ql[s & 1].x, ql[s & 1].y, ql[s & 1].z, ql[s & 1].w}, h[4] = {qh.x, qh.y, qh.z, qh.w};
+        return ((l[w] >> (4 * (s >> 1))) & 0x0f0f0f0fu) | (((h[w] >> (2 * s)) & 0x03030303u) << 4);
+    }
+    static constexpr float kBias = 32.0f;
+    static constexpr int kBlockBytes = 210;
+};
+
+
+template <typename Half>
+__device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale, float* Y,
+                                                    int M, int K, int N, int accumulate, int blocks_per_split, float* partials, int bx, int by,
+                                                    int bz, uint8_t* s_a, int scale_stride) {
+    constexpr int MT = 8, TM = 32 * MT, STAGE = TM * 256;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 31, kh = lane >> 5;
+    const int m0 = by * TM, n_base = bx * 256 + 64 * (wave & 3) + 32 * (wave >> 2);
+    const int blk0 = bz * blocks_per_split, nblk = min(K / 256 - blk0, blocks_per_split), nst = 2 * nblk;
+    const uint8_t* wrow = W + (int64_t)min(n_base + j, N - 1) * stride + (int64_t)blk0 * Half::kBlockBytes;
+
+    // X: row r of a stage is 256 bytes of LDS, its sixteen 16-byte pieces at piece ^ (r % 16).  A wave's instruction fetches four rows.
+    const uint32_t row_bytes = (uint32_t)K * 2, last = min(M - 1 - m0, TM - 1), r0 = 4 * wave + (lane >> 4);
+    const uint32_t piece = ((lane & 15) ^ (r0 & 15)) << 4;
+    gt_i4 xs = gt_buffer(reinterpret_cast<const uint8_t*>(Xh) + (int64_t)m0 * K * 2 + (int64_t)blk0 * 512);
+    xs[0] = __builtin_amdgcn_readfirstlane(xs[0]);  // the compiler does not always see that they are the same in every lane
+    xs[1] = __builtin_amdgcn_readfirstlane(xs[1]);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)s_a + wave * 1024;
+    auto fetch = [&](int st, int i) { gt_to_lds(lds0 + (st & 1) * STAGE + i * 8192, (int)(min(r0 + 32 * i, last) * row_bytes + piece), xs, st * 256); };
+
+    float* s_rs = reinterpret_cast<float*>(s_a + 2 * STAGE);
+    f32x16 acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mt][r] = 0.0f;
+    Half w[2];
+    for (int i = 0; i < 8; ++i) fetch(0, i);
+    w[0].load(wrow, 0, kh);
+    issue_order_fence();
+    for (int i = 0; i < 8; ++i) fetch(1, i);
+    if (tid < TM) s_rs[tid] = rowscale[bz * scale_stride + m0 + min(tid, (int)last)];
+    h2 sc, of;
+    uint32_t bf[2][8];  // [buffer][two fragments of four]
+    auto dequant = [&](const Half& h, int s, int q, uint32_t (&out)[8]) {
+        const h2 sub = {(_Float16)(1024.0f + Half::kBias), (_Float16)(1024.0f + Half::kBias)};
+        const uint32_t b = h.bytes(s, q);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const uint32_t hq = __builtin_amdgcn_perm(0x64646464u, b, p ? 0x04030402u : 0x04010400u);
+            h2 x;
+            __builtin_memcpy(&x, &hq, 4);
+            const h2 v = __builtin_elementwise_fma(x - sub, sc, of);
+            __builtin_memcpy(&out[2 * q + p], &v, 4);
+        }
+    };
+    w[0].arrive(0, kh);
+    w[0].scale(0, sc, of);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dequant(w[0], 0, q, bf[0]);
+    gt_arrived<0>();
+    const int a0 = j * 256 + (((2 * kh) ^ (j & 15)) << 4);
+    h8 af[MT];
+    auto read = [&](int from, int mt) { af[mt] = *reinterpret_cast<const h8*>(s_a + from + mt * 8192); };
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) read(a0, mt);
+
+    auto stage = [&](int st, auto half_) {  // 8 groups of 8 MFMAs: 16 values of K each
+        constexpr int half = decltype(half_)::value;
+        Half& cur = w[half];
+        Half& nxt = w[half ^ 1];
+        constexpr int at = half * STAGE;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const int s = g >> 1, ks = g & 1;
+            // where the fragments of the next 16 values of K lie (in assembly: hoisted out of the loop, the sixteen places cost as many registers)
+            int from;
+            asm volatile("v_xor_b32 %0, %1, %2" : "=v"(from) : "v"(a0), "s"(((4 * (((g + 1) >> 1) & 3) + ((g + 1) & 1)) << 4) | (g < 7 ? at : STAGE - at)));
+            h8 b;
+            __builtin_memcpy(&b, &bf[s & 1][4 * ks], 16);
+            if (g == 6) nxt.arrive(half ^ 1, kh);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                __builtin_amdgcn_sched_barrier(0);
+                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], b, acc[mt], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (g < 7) read(from, mt);
+                else if (mt >= 4) { read(from, 2 * mt - 8); read(from, 2 * mt - 7); }
+                // weights of the next sub-block
+                const Half& src = s < 3 ? cur : nxt;
+                const int slot = 8 * ks + mt, sn = (s + 1) & 3;
+                if (slot == 0) src.scale(sn, sc, of);
+                if ((slot & 3) == 2) dequant(src, sn, slot >> 2, bf[(s + 1) & 1]);
+                // the stage after the next, into the half of LDS this one is read from; the next half block of weights
+                if (g == 7 && mt == 3) gt_arrived<0>();
+                if (g == 7 && mt >= 4 && st + 2 < nst) fetch(st + 2, mt - 4);
+                if (g == 0 && mt < 4 && st > 0 && st + 1 < nst) fetch(st + 1, mt + 4);
+                if (g == 2 && mt == 0) nxt.load(wrow + (int64_t)min((st + 1) >> 1, nblk - 1) * Half::kBlockBytes, half ^ 1, kh);
+            }
+        }
+    };
+    for (int st = 0; st < nst; st += 2) {
+        stage(st, std::integral_constant<int, 0>{});
+        stage(st + 1, std::integral_constant<int, 1>{});
+    }
+    qf_store<MT>(acc, s_rs, Y, partials, accumulate, M, N, m0, n_base, j, kh, bz);
+}
+
 // Which tile a workgroup takes.  The hardware deals consecutive workgroup ids round-robin to the 8 XCDs, each with its own
 // L2; taken as they come, the workgroups of one XCD are scattered over all column tiles, row tiles and K splits and share
 // almost nothing (the down projection of a 512-row prompt, 10 x 4 tiles x 6 splits, then pulls 200 MB through the L2s for
@@ -1014,6 +1186,34 @@ __device__ __forceinline__ void qf_tile_of(int L, int gx, int gy, int& bx, int& 
     const int within = r - band * 4 * gx;
     by = 4 * band + within % rows;
     bx = within / rows;
+}
+
+// The first `tall` workgroups of a launch take 256 rows each, in that order of pairs of row tiles; the tiles of 128 rows that are left, two from
+// each pair, follow (qf_tall).  False: a row tile past the last.
+__device__ __forceinline__ bool qf_place(int hw, int nwg, int gx, int gy, int tall, int& bx, int& by, int& bz) {
+    if (tall == 0) {
+        qf_tile_of(qf_xcd_order(hw, nwg), gx, gy, bx, by, bz);
+        return true;
+    }
+    const int rest = hw - tall, L = rest < 0 ? qf_xcd_order(hw, tall) : qf_xcd_order(rest, nwg - tall);
+    qf_tile_of(rest < 0 ? L : tall + (L >> 1), gx, (gy + 1) >> 1, bx, by, bz);
+    if (rest >= 0) by = 2 * by + (L & 1);
+    return rest < 0 || by < gy;
+}
+
+// tiles of 128 and 256 rows by 256 columns
+template <typename Tile>
+__global__ __launch_bounds__(512, 1) void qgemm_f16_rows_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale,
+                                                                float* Y, int M, int K, int N, int accumulate, int blocks_per_split, float* partials,
+                                                                int scale_stride, int tall) {
+    extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(W, M);
+    int bx, by, bz;
+    if (!qf_place(blockIdx.x, gridDim.x, (N + QF_TN - 1) / QF_TN, (M + QF_TM - 1) / QF_TM, tall, bx, by, bz)) return;
+    if ((int)blockIdx.x < tall)
+        qgemm_f16_tall_body<typename Tile::Half>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
+    else
+        qgemm_f16_body<Tile, 4, 8>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
 }
 
 template <typename Tile, int MT, int WAVES>
@@ -1071,6 +1271,29 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_mu
     const int bx = local % q.ntiles, bz = local / q.ntiles;
     if (q.q6) qgemm_f16_body<Q6Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
     else qgemm_f16_body<Q4Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
+}
+
+// the same in tiles of 128 and 256 rows
+__global__ __launch_bounds__(512, 1) void qgemm_f16_rows_multi_kernel(const QfMulti a, int M, int K, int slots, int tall) {
+    extern __shared__ __align__(16) uint8_t qf_lds[];
+    read_now(a.m[0].W, a.m[1].W, a.m[2].W, a.n_mat);
+    int sx, by, unused;
+    if (!qf_place(blockIdx.x, gridDim.x, slots, (M + QF_TM - 1) / QF_TM, tall, sx, by, unused)) return;
+    int i = 0;
+    if (a.n_mat > 1 && sx >= a.m[0].slot_end) i = 1;
+    if (a.n_mat > 2 && sx >= a.m[1].slot_end) i = 2;
+    const QfMat& q = i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]);
+    const int local = sx - (i == 0 ? 0 : (i == 1 ? a.m[0].slot_end : a.m[1].slot_end));
+    const int bx = local % q.ntiles, bz = local / q.ntiles;
+#define PTM_QR(BODY) BODY(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0)
+    if ((int)blockIdx.x < tall) {
+        if (q.q6) PTM_QR(qgemm_f16_tall_body<Q6Half>);
+        else PTM_QR(qgemm_f16_tall_body<Q4Half>);
+    } else {
+        if (q.q6) PTM_QR((qgemm_f16_body<Q6Tile, 4, 8>));
+        else PTM_QR((qgemm_f16_body<Q4Tile, 4, 8>));
+    }
+#undef PTM_QR
 }
 
 // the same for up to 32 rows and up to QF_SHORT_BLOCKS super-blocks per split
@@ -1206,6 +1429,41 @@ static int qgemm_f16_row_tiles(bool q4, int M, int N, int splits) {
     return (q4 && wgs < 128) ? 2 : 4;  // 512 x 2560 x 9728 (152 workgroups): 60 us with 128 rows, 70 with 64; 512 x 4096 x 4096 (64): 80 / 68
 }
 
+// Which tiles of a launch of gx column tiles (slots) and gz K splits have 256 rows: the first `tall` pairs of row tiles in qf_tile_of's order, in whole
+// rounds of the chip or all of them, whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
+// times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there.  Measured, all of
+// 128 rows, all of 256, by this rule: 509 x 19456 x 2560 85, 70, 70 us; 953 x 19456 x 2560 132, 150, 125; 2048 x 9728 x 2560 137, 151, 129; 2048 x 28672 x
+// 4096 in 7 rounds, 7, 6.25; 300 x 14336 x 4096 62, 91, 62; Q6_K 2048 x 4096 x 14336 347, 289, 289, 953 x 18944 x 3584 236, 220, 200.
+static float qf_tall(int gx, int gz, int M, bool q4, int* tall) {
+    const int gy = (M + QF_TM - 1) / QF_TM, pairs = (gy + 1) / 2, plane = gx * pairs, all = plane * gz;
+    const float ratio = q4 ? 1.75f : 1.5f;
+    // 128-row tiles in the pairs from place t of that order on: two each, but one in the last pair of an odd number of row tiles
+    auto left = [&](int t) {
+        const int last_band = (pairs - 1) / 4 * 4, r = t % plane - last_band * gx;
+        const int single = gy & 1 ? gx * gz - (t / plane * gx + (r > 0 ? r / (pairs - last_band) : 0)) : 0;
+        return 2 * (all - t) - single;
+    };
+    float best = (float)((left(0) + 255) / 256);
+    *tall = 0;
+    for (int t : {all / 256 * 256, all}) {
+        if (t == 0) continue;
+        const int rounds = (t + 255) / 256, rest = left(t) - (256 * rounds - t);
+        const float cost = ratio * (float)rounds + (float)(rest > 0 ? (rest + 255) / 256 : 0);
+        if (cost < best) { best = cost; *tall = t; }
+    }
+    return best;
+}
+static int qf_workgroups(int gx, int gz, int M, int tall) {
+    const int gy = (M + QF_TM - 1) / QF_TM;
+    return tall ? tall + 2 * (gx * ((gy + 1) / 2) * gz - tall) : gx * gy * gz;
+}
+
+// rounds of a launch of matrices with `tiles` column tiles and K splits together
+float qgemm_f16_rounds(int tiles, int M, bool q4) {
+    int tall;
+    return qf_tall(tiles, 1, M, q4, &tall);
+}
+
 // Workgroups of 128 columns: always up to 32 rows, up to 64 where the chip then has a CU for each.  Prompts of 19 / 32 / 50 / 64 tokens,
 // Qwen3-4B shapes, 256 columns, this rule, 128 always: 3.53 / 3.67 / 3.97 / 4.12 ms, 3.32 / 3.45 / 3.89 / 4.00, 3.32 / 3.45 / 3.86 / 3.97;
 // Llama-3-8B shapes in 16 layers, 60 tokens: 2.28, 2.28, 2.31; in 8 layers, 5 / 19 / 32 tokens, 256 columns and so: 1.05 / 1.10 / 1.13, 1.00 / 1.05 /
@@ -1281,8 +1539,8 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         const int big = 2 * 128 * QF_PITCH + 4 * 128, small = 2 * 64 * QF_PITCH + 4 * 64;
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q4Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q6Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q4Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q6Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
@@ -1307,16 +1565,21 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
             else PTM_QS(Q6Tile, 4);
         }
 #undef PTM_QS
+    } else if (MT == 4) {
+        int tall;
+        qf_tall(grid.x, splits, M, q4, &tall);
+#define PTM_QR(TILE) hipLaunchKernelGGL((qgemm_f16_rows_kernel<TILE>), dim3(qf_workgroups(grid.x, splits, M, tall)), dim3(512), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride, tall)
+        if (q4) PTM_QR(Q4Tile);
+        else PTM_QR(Q6Tile);
+#undef PTM_QR
     } else {
 #define PTM_QF(TILE, MTV, WV) hipLaunchKernelGGL((qgemm_f16_kernel<TILE, MTV, WV>), grid, dim3(64 * WV), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride)
     if (q4) {
-        if (MT == 4) PTM_QF(Q4Tile, 4, 8);
-        else if (MT == 2 && narrow) PTM_QF(Q4Tile, 2, 4);
+        if (MT == 2 && narrow) PTM_QF(Q4Tile, 2, 4);
         else if (MT == 2) PTM_QF(Q4Tile, 2, 8);
         else PTM_QF(Q4Tile, 1, 4);
     } else {
-        if (MT == 4) PTM_QF(Q6Tile, 4, 8);
-        else if (MT == 2 && narrow) PTM_QF(Q6Tile, 2, 4);
+        if (MT == 2 && narrow) PTM_QF(Q6Tile, 2, 4);
         else if (MT == 2) PTM_QF(Q6Tile, 2, 8);
         else PTM_QF(Q6Tile, 1, 4);
     }
@@ -1430,7 +1693,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     }
     static std::once_flag raised;
     std::call_once(raised, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 128 * QF_PITCH + 4 * 128);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(QF_SHORT_BLOCKS));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1446,8 +1709,13 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
     else if (M <= 64)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 8>), dim3(slots, 1), dim3(512), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
-    else
-        hipLaunchKernelGGL((qgemm_f16_multi_kernel<4, 8>), dim3(slots, (M + 127) / 128), dim3(512), 2 * (size_t)128 * QF_PITCH + 4 * 128, s, a, M, K);
+    else {
+        bool q4 = true;
+        for (int i = 0; i < n; ++i) q4 = q4 && types[i] == PTM_TYPE_Q4_K;
+        int tall;
+        qf_tall(slots, 1, M, q4, &tall);
+        hipLaunchKernelGGL(qgemm_f16_rows_multi_kernel, dim3(qf_workgroups(slots, 1, M, tall)), dim3(512), 2 * (size_t)128 * QF_PITCH + 4 * 128, s, a, M, K, slots, tall);
+    }
     if (r.n > 0 && !deferred_P) hipLaunchKernelGGL(qgemm_split_reduce_multi_kernel, dim3(red_blocks), dim3(256), 0, s, r);
     return launch_status();
 }

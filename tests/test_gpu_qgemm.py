@@ -285,3 +285,49 @@ def test_short_prompts_of_several_matrices(dev, po, K, N, types, blocks):
         err = float((many[i].double() - want).abs().max() / want.pow(2).mean().sqrt())
         print("max err / rms: %.2e" % err, flush=True)
         assert err <= QGEMM_F16_TOL, (i, err)
+
+
+# tiles of 256 rows: all (152 pairs of row tiles), whole rounds and 128-row tiles behind them (K splits off and on), an odd last row tile, ragged N
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(509, 512, 19456), (385, 256, 38000), (953, 512, 19441), (1030, 256, 19456), (2047, 256, 9728), (641, 1024, 14337)])
+def test_tiles_of_256_rows(dev, po, qt, M, K, N):
+    """Rows are the rows of calls of 128 rows, which have tiles of 128, bit for bit (K unsplit)."""
+    r = synth.rng_for(50, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    xb, _ = bf16_round(r.standard_normal((M, K), dtype=np.float32))
+    y = gpu_qgemm_f16(qt, W, xb, M, K, N)
+    for m in list(range(0, M - 127, 384)) + [M - 128]:
+        assert np.array_equal(bits(y[m:m + 128]), bits(gpu_qgemm_f16(qt, W, np.ascontiguousarray(xb[m:m + 128]), 128, K, N))), m
+
+
+@pytest.mark.parametrize("K,N,types,M", [(512, (9728, 9728), (12, 12), 509), (512, (5000, 5001, 5100), (12, 14, 14), 1000), (1024, (4096, 1024, 1000), (12, 12, 14), 2048),
+                                         (512, (14336, 14300), (14, 12), 2000)])
+def test_tiles_of_256_rows_of_several_matrices(dev, po, K, N, types, M):
+    """Slabs and sums are those of calls of fewer rows of the same class (same K splits) in tiles of 128, bit for bit."""
+    import ctypes as C
+    from gemm_helpers import harness
+    h, n, few = harness(), len(N), 260 if M <= 1024 else 1025
+    h.multi_split_bytes.restype = C.c_int64
+    Ns, ts = (C.c_int * n)(*N), (C.c_uint32 * n)(*types)
+    r = synth.rng_for(51, K, *N)
+    Wh = [synth.make_weight(r, t, rows, K) for t, rows in zip(types, N)]
+    W = [torch.from_numpy(w).cuda() for w in Wh]
+    gamma = torch.from_numpy((1 + 0.1 * r.standard_normal(K)).astype(np.float32)).cuda()
+    X = torch.from_numpy(r.standard_normal((M, K), dtype=np.float32)).cuda()
+    ptrs = lambda ts: (C.c_void_p * n)(*[t.data_ptr() for t in ts])
+    p = lambda t: C.c_void_p(t.data_ptr())
+
+    def run(x):
+        m = x.shape[0]
+        ws = [torch.zeros(ops.qgemm_f16_workspace_bytes(m, K), dtype=torch.uint8, device="cuda") for _ in range(2)]
+        split = torch.full((max(h.multi_split_bytes(n, Ns, ts, K, m) // 4, 4),), 5.0, device="cuda")
+        Y = [torch.full((m, rows), 3.0, device="cuda") for rows in N]
+        assert h.multi_run(n, ts, ptrs(W), (C.c_int64 * n)(*[w.shape[1] for w in Wh]), Ns, ptrs(Y), p(x), p(gamma), m, K, p(ws[0]), p(ws[1]), p(split),
+                           C.c_int64(split.numel() * 4), None, None, None) == 0
+        torch.cuda.synchronize()
+        return Y
+
+    y = run(X)
+    for m in (0, M - few):
+        for i, (a, b) in enumerate(zip(run(X[m:m + few].contiguous()), y)):
+            assert torch.equal(a, b[m:m + few]), (m, i)
