@@ -477,7 +477,7 @@ struct BlockStack {
     const double* freq = nullptr;
     int branch = 0, r_branch = 0;  // the next branch's number
     const float *pend_store = nullptr, *r_pend_store = nullptr;
-    float *r_hn = nullptr, *r_conv = nullptr, *r_scan = nullptr, *r_decay = nullptr;
+    float *r_hn = nullptr, *r_conv = nullptr, *r_scan = nullptr, *r_decay = nullptr, *r_tiles = nullptr;
     void *r_mix = nullptr, *r_low = nullptr;
     // all recurrent state, and its copy (blocks_state_copy)
     float *state = nullptr, *saved = nullptr;
@@ -1116,7 +1116,7 @@ int blocks_reserve(BlockStack* b, int rows) {
     const ptm_block_config& c = b->cfg;
     const size_t R = (size_t)rows, es = b->f32 ? 4 : 2, W = (size_t)b->wp;
     const size_t S = (size_t)(c.streams > 0 ? c.streams : 1);
-    size_t proj = 0, q = 0, attn = 0, act = 64, kv = 0, shifted = 0, low = 0, conv = 0, scan = 0, steps = 0;
+    size_t proj = 0, q = 0, attn = 0, act = 64, kv = 0, shifted = 0, low = 0, conv = 0, scan = 0, steps = 0, tiles = 0;
     for (const ptm_block& L : b->blocks) {
         auto grow = [](size_t& v, size_t n) { v = v > n ? v : n; };
         grow(proj, (size_t)(wkv(L) ? 5 * wkv_section(L) : up64(qkv_rows(L))));
@@ -1128,9 +1128,10 @@ int blocks_reserve(BlockStack* b, int rows) {
             grow(q, (size_t)q_cols(L));
         }
         if (has_ssm(L)) {
-            grow(conv, (size_t)ssm_channels(L.ssm));
-            grow(scan, (size_t)scan_slabs(L.ssm.state) * (size_t)(L.ssm.heads * L.ssm.vdim));
+            grow(conv, (size_t)ssm_conv_row(ssm_shape(L.ssm)));
+            grow(scan, (size_t)(L.ssm.heads * L.ssm.vdim));
             grow(steps, 2 * (size_t)L.ssm.heads);
+            grow(tiles, (size_t)ssm_tile_floats(L.ssm.heads, rows));
         }
         grow(attn, (size_t)up64(attn_cols(L)));
         grow(act, (size_t)up64(L.ff));
@@ -1143,7 +1144,7 @@ int blocks_reserve(BlockStack* b, int rows) {
                  o_xn = take(es * R * W), o_q = take(es * R * q), o_at = take(es * R * attn), o_ac = take(es * R * act),
                  o_g = take(es * R * (size_t)up64(c.side_dim > 0 ? c.side_dim : 1)), o_kv = take(es * kv),
                  o_hn = take(4 * shifted), o_mix = take(es * 5 * shifted), o_low = take(es * R * low), o_cv = take(4 * R * conv), o_sc = take(4 * R * scan),
-                 o_st = take(4 * R * steps);
+                 o_st = take(4 * R * steps), o_ti = take(4 * tiles);
     int rc = hip_status(hipMalloc(&b->slab, off));
     if (rc != PTM_OK) return rc;
     if ((rc = hip_status(hipMemset(b->slab, 0, off))) != PTM_OK) return rc;
@@ -1167,6 +1168,7 @@ int blocks_reserve(BlockStack* b, int rows) {
     b->r_conv = (float*)(p + o_cv);
     b->r_scan = (float*)(p + o_sc);
     b->r_decay = (float*)(p + o_st);
+    b->r_tiles = (float*)(p + o_ti);
     b->rows = rows;
     return PTM_OK;
 }
@@ -1320,8 +1322,8 @@ static int attention_prompt(BlockStack* b, const ptm_block& L, const LayerRun& r
         r.state = run.state;
         r.conv = b->r_conv;
         r.decay = b->r_decay;
+        r.tiles = b->r_tiles;
         r.y = b->r_scan;
-        r.y_slab = (int64_t)M * L.ssm.heads * L.ssm.vdim;
         r.out = static_cast<uint8_t*>(b->r_attn) + (size_t)attn_part(L) * es;
         r.out_ld = lda;
         PTM_TRY(ssm_rows(r, f32, s));

@@ -2,6 +2,7 @@
 // mixer_attention.hip).  Host side; not part of the C ABI.
 #pragma once
 #include "dense_gemv.h"
+#include "recurrent.h"
 #include "gemm_plan.h"
 #include "ptm_common.h"
 
@@ -91,76 +92,6 @@ int decode_attention(const DecodeAttention& a, hipStream_t s);
 int decode_attention_merge(const float* pO, const float* pM, const float* pL, int splits, const ptm_attention_args& a, float* out,
                            hipStream_t s);
 int attention_rows(const ptm_attention_args& a, const int64_t* d_past, bool q_fp32_out_fp32, hipStream_t s);
-
-// ---- recurrent mixers (recurrent.hip) ----------------------------------------------------------
-bool recurrent_supported(int keys);
-int64_t recurrent_state_floats(int heads, int keys, int columns);
-
-struct WkvStep {
-    const float* proj;        // [r | k | v | g | low-rank]
-    const uint16_t* w2;       // [heads * dim][w2_ld]
-    int64_t w2_ld;
-    int heads, dim, rank;
-    const float *w0, *u, *norm;
-    float eps;
-    const int64_t* d_past;
-    float* state;
-    float* out;               // [heads * dim]
-};
-int wkv_step(const WkvStep& a, hipStream_t s);
-
-struct WkvRows {
-    const float* proj;        // [M][ld]: r, k, v, g and the decays w, `section` floats apart
-    int64_t ld, section;
-    int M, heads, dim;
-    const float *u, *norm;
-    float eps;
-    int64_t pos0;
-    float* state;
-    float* o;                 // [scan_slabs(dim)][M][o_ld], o_slab floats apart
-    int64_t o_ld, o_slab;
-    int groups;               // set by wkv_rows
-    void* out;                // [M][out_ld]
-    int64_t out_ld;
-    const float* h_last;      // the mixer's last input row, kept for the next token's shift
-    float* shift;
-    int wp;
-};
-int wkv_rows(WkvRows a, bool fp32, hipStream_t s);
-int64_t scan_slabs(int keys);  // partial sums that a scan leaves per row
-int token_shift_rows(const float* h, const float* shift, const float* mu, int n, int rows, int64_t pos0, int wp, bool fp32, void* out, hipStream_t s);
-int tanh_rows(const float* g, int slabs, int64_t slab, int rows, int n, bool fp32, void* out, hipStream_t s);
-
-struct SsmShape {
-    int heads, vdim, state, groups, taps, norm_groups;
-    const float *conv, *conv_b, *dt_bias, *neg_a, *D, *norm;  // neg_a: -exp(A_log)
-    float scale;
-};
-struct SsmStep {
-    SsmShape m;
-    const float* proj;        // [z | x | B | C | dt]
-    const int64_t* d_past;
-    float *ring, *state;      // [taps][channels]; state
-    float* out;               // [heads * vdim], before its norm
-};
-int ssm_step(const SsmStep& a, hipStream_t s);
-struct SsmRows {
-    SsmShape m;
-    const float* proj;        // [M][ld]
-    int64_t ld;
-    int M;
-    int64_t pos0;
-    float eps;
-    float *ring, *state;
-    float* conv;              // [M][x | B | C]
-    float* decay;             // [M][2][heads]
-    float* y;                 // [scan_slabs(state)][M][heads * vdim], y_slab floats apart
-    int64_t y_slab;
-    int key_groups;           // set by ssm_rows
-    void* out;                // [M][out_ld]
-    int64_t out_ld;
-};
-int ssm_rows(SsmRows a, bool fp32, hipStream_t s);
 
 int argmax_finish(const float* part_val, const int* part_idx, int n, int64_t* out_index, const ArgmaxAdvance adv, hipStream_t s);
 

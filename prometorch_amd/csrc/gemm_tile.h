@@ -26,6 +26,10 @@ typedef __bf16 gt_b8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ void gt_to_lds(uint32_t lds, int voff, gt_i4 base, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(base), "s"(soff) : "memory");
 }
+// 4 bytes per lane to LDS bytes [lds, lds + 256)
+__device__ __forceinline__ void gt_word_to_lds(uint32_t lds, int voff, gt_i4 base, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(base), "s"(soff) : "memory");
+}
 __device__ __forceinline__ gt_i4 gt_buffer(const void* p) {
     const uint64_t a = reinterpret_cast<uint64_t>(p);
     return gt_i4{(int)(uint32_t)a, (int)((a >> 32) & 0xffffu), -1, 0x00020000};

@@ -5,8 +5,9 @@
 //
 // A state is stored per value column, its key values consecutive and padded: [heads][columns][16 * KPL].
 // One token: 16 lanes share a column, KPL key values each, so a wave holds four columns and a read of the state is consecutive.
-// Prompt rows: neither the columns nor the keys of a state depend on each other, only the sum over the keys does.  A lane is a value
-// column and a wave has KPL keys of 64 columns in registers, so what belongs to a key (r, k, w; B, C) is one value for the whole
+// Prompt rows, ssm: 16 tokens at a time on the fp32 matrix cores (ssm_scan_kernel).
+// Prompt rows, wkv: neither the columns nor the keys of a state depend on each other, only the sum over the keys does.  A lane is a value
+// column and a wave has KPL keys of 64 columns in registers, so what belongs to a key (r, k, w) is one value for the whole
 // wave: it is loaded once into a row of 16 lanes and broadcast as a DPP operand of the arithmetic, three instructions per key and
 // token.  A workgroup's four waves add their sums through LDS; up to four workgroups share a head and leave partial sums, which the
 // row kernel behind the scan adds.  The next tile's vectors are on their way while a tile of tokens is used.
@@ -14,10 +15,14 @@
 // What a token needs from earlier ones besides the state (the token shift's vector, the convolution's inputs) lies in rings
 // indexed by position; a slot is never read and written by the same launch.
 #include "dense.h"
+#include "gemm_tile.h"
 
+#include <mutex>
 #include <type_traits>
 
 namespace ptm {
+
+typedef float rc_f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
@@ -386,8 +391,16 @@ __global__ __launch_bounds__(64) void tanh_rows_kernel(const float* __restrict__
     }
 }
 
-// grid (ceil(rows / 8), ceil(channels / 256) + 1): convolution and silu of x, B and C, [rows][channels], eight rows per thread;
-// the last column of workgroups leaves decay and dt, [rows][2][heads]
+// Where x, B and C of a convolved row lie: x padded to 4, then B and C of every group padded to KP, all padding zeros.
+__host__ __device__ inline int conv_x(const SsmShape& m) { return (m.heads * m.vdim + 3) & ~3; }
+static int padded_keys(int n) { return 16 * keys_per_lane(n); }
+int64_t ssm_conv_row(const SsmShape& m) { return conv_x(m) + 2 * (int64_t)m.groups * padded_keys(m.state); }
+// per 16 tokens and head: what the tokens take from each other [16 from][16 to], the state's decay up to each, each one's share of the new state
+constexpr int SSM_TILE = 288;
+int64_t ssm_tile_floats(int heads, int rows) { return (int64_t)((rows + 15) / 16) * heads * SSM_TILE; }
+
+// grid (ceil(rows / 8), ceil(row / 256) + 1): convolution and silu of x, B and C, eight rows per thread; the last column of workgroups leaves
+// decay and dt, [rows][2][heads]
 constexpr int CONV_ROWS = 8;
 __global__ __launch_bounds__(256) void ssm_conv_rows_kernel(const SsmRows a) {
     const SsmShape& m = a.m;
@@ -402,14 +415,23 @@ __global__ __launch_bounds__(256) void ssm_conv_rows_kernel(const SsmRows a) {
         }
         return;
     }
-    const int ch = blockIdx.y * 256 + threadIdx.x;
-    if (ch >= channels) return;
+    const int at = blockIdx.y * 256 + threadIdx.x;
+    if (at >= a.conv_ld) return;
+    int ch = at;
+    if (at >= conv_x(m)) {
+        const int kp = a.keys, q = at - conv_x(m), n = q % kp;
+        ch = n < m.state ? inner + q / kp * m.state + n : channels;
+    } else if (at >= inner) ch = channels;
+    if (ch == channels) {
+        for (int r = 0; r < rows; ++r) a.conv[(int64_t)(r0 + r) * a.conv_ld + at] = 0.0f;
+        return;
+    }
     const float *x = a.proj + inner + ch, *w = m.conv + (int64_t)ch * m.taps, bias = m.conv_b[ch];
     auto input = [&](int row) {  // of row r0 + row, also of rows and positions before
         const int64_t p = a.pos0 + r0 + row;
         return r0 + row >= 0 ? x[(int64_t)min(r0 + row, a.M - 1) * a.ld] : p >= 0 ? a.ring[p % m.taps * channels + ch] : 0.0f;
     };
-    float* out = a.conv + (int64_t)r0 * channels + ch;
+    float* out = a.conv + (int64_t)r0 * a.conv_ld + at;
     if (m.taps <= 4) {
         float in[CONV_ROWS + 3], t[4];
 #pragma unroll
@@ -418,177 +440,315 @@ __global__ __launch_bounds__(256) void ssm_conv_rows_kernel(const SsmRows a) {
         for (int i = 0; i < CONV_ROWS + 3; ++i) in[i] = 3 - i < m.taps ? input(i - 3) : 0.0f;
 #pragma unroll
         for (int r = 0; r < CONV_ROWS; ++r)
-            if (r < rows) out[(int64_t)r * channels] = silu_f(fmaf(t[3], in[r], fmaf(t[2], in[r + 1], fmaf(t[1], in[r + 2], fmaf(t[0], in[r + 3], bias)))));
+            if (r < rows) out[(int64_t)r * a.conv_ld] = silu_f(fmaf(t[3], in[r], fmaf(t[2], in[r + 1], fmaf(t[1], in[r + 2], fmaf(t[0], in[r + 3], bias)))));
     } else {
         for (int r = 0; r < rows; ++r) {
             float acc = bias;
             for (int j = 0; j < m.taps; ++j) acc = fmaf(w[m.taps - 1 - j], input(r - j), acc);
-            out[(int64_t)r * channels] = silu_f(acc);
+            out[(int64_t)r * a.conv_ld] = silu_f(acc);
         }
     }
 }
 
-// Four keys of 64 columns take four tokens: S <- decay S + B dx, y += C S.  p[t]: a row of lanes with B at lanes B0 .. and C at
-// C0 .. .
-#define PTM_DECAY(S, D) "v_mul_f32 %" S ", %" D ", %" S "\n\t"
-#define PTM_SSM_TAKE(P, X)                                       \
-    "v_fmac_f32_dpp %0, %" P ", %" X PTM_DPP("%20")              \
-    "v_fmac_f32_dpp %1, %" P ", %" X PTM_DPP("%21")              \
-    "v_fmac_f32_dpp %2, %" P ", %" X PTM_DPP("%22")              \
-    "v_fmac_f32_dpp %3, %" P ", %" X PTM_DPP("%23")
-#define PTM_SSM_GIVE(Y, P, S, C) "v_fmac_f32_dpp %" Y ", %" P ", %" S PTM_DPP("%" C)
-#define PTM_SSM_GIVE_NEXT(Y, P, D)                               \
-    PTM_SSM_GIVE(Y, P, "0", "24") PTM_DECAY("0", D)              \
-    PTM_SSM_GIVE(Y, P, "1", "25") PTM_DECAY("1", D)              \
-    PTM_SSM_GIVE(Y, P, "2", "26") PTM_DECAY("2", D)              \
-    PTM_SSM_GIVE(Y, P, "3", "27") PTM_DECAY("3", D)
-template <int B0, int C0>
-__device__ __forceinline__ void ssm_keys4(float* s, float (&y)[4], float p0, float p1, float p2, float p3, const float* decay, const float* dx) {
-    asm(PTM_DECAY("0", "12") PTM_DECAY("1", "12") PTM_DECAY("2", "12") PTM_DECAY("3", "12")
-        PTM_SSM_TAKE("8", "16") PTM_SSM_GIVE_NEXT("4", "8", "13")
-        PTM_SSM_TAKE("9", "17") PTM_SSM_GIVE_NEXT("5", "9", "14")
-        PTM_SSM_TAKE("10", "18") PTM_SSM_GIVE_NEXT("6", "10", "15")
-        PTM_SSM_TAKE("11", "19")
-        PTM_SSM_GIVE("7", "11", "0", "24") PTM_SSM_GIVE("7", "11", "1", "25") PTM_SSM_GIVE("7", "11", "2", "26") PTM_SSM_GIVE("7", "11", "3", "27")
-        : "+&v"(s[0]), "+&v"(s[1]), "+&v"(s[2]), "+&v"(s[3]), "+&v"(y[0]), "+&v"(y[1]), "+&v"(y[2]), "+&v"(y[3])
-        : "v"(p0), "v"(p1), "v"(p2), "v"(p3), "v"(decay[0]), "v"(decay[1]), "v"(decay[2]), "v"(decay[3]), "v"(dx[0]), "v"(dx[1]), "v"(dx[2]), "v"(dx[3]),
-          "n"(B0), "n"(B0 + 1), "n"(B0 + 2), "n"(B0 + 3), "n"(C0), "n"(C0 + 1), "n"(C0 + 2), "n"(C0 + 3));
+// What 16 tokens of a head take from each other: M[s][t] = (C_t . B_s) dt_s prod(s < q <= t) decay_q, with the skip D on the diagonal, the products P_t =
+// prod(q <= t) and Q_s = dt_s prod(q > s) beside it.  Products of decays, never quotients.  grid (ceil(rows / 16), ceil(heads of a group / 4 each),
+// groups), `each` heads a wave (a head for few rows: 30 rows 5.0 us; two where the chip is full: 2048 rows of 40 heads 14.8 -> 11.2); tokens past the
+// last leave everything as it is.
+__global__ __launch_bounds__(256) void ssm_tiles_kernel(const SsmRows a, int each) {
+    const SsmShape& m = a.m;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g4 = lane >> 4, t0 = blockIdx.x * 16, per = m.heads / m.groups;
+    const int first = (blockIdx.y * 4 + wave) * each, end = min(first + each, per);
+    if (first >= per) return;
+    const int64_t row = (int64_t)min(t0 + j, a.M - 1);
+    const bool here = t0 + j < a.M;
+    float next_decay, next_Q, next_dt[4], next_skip;
+    auto fetch = [&](int in_group) {
+        const int h = blockIdx.z * per + in_group;
+        const float* step = a.decay + h;
+        next_decay = step[row * 2 * m.heads];
+        next_Q = step[(row * 2 + 1) * m.heads];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) next_dt[i] = step[((int64_t)min(t0 + 4 * g4 + i, a.M - 1) * 2 + 1) * m.heads];
+        next_skip = m.D[h];
+    };
+    fetch(first);
+    const float* at = a.conv + row * a.conv_ld + conv_x(m) + (int64_t)blockIdx.z * a.keys + 4 * g4;
+    rc_f4 dot = {0.f, 0.f, 0.f, 0.f}, odd = dot;  // rows s = 4 g4 + i, column t = j
+    for (int k = 0; k < a.keys; k += 64) {
+        rc_f4 B[4], C[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            B[i] = *reinterpret_cast<const rc_f4*>(at + k + 16 * i);
+            C[i] = *reinterpret_cast<const rc_f4*>(at + k + 16 * i + (int64_t)m.groups * a.keys);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                dot = __builtin_amdgcn_mfma_f32_16x16x4f32(B[i][e], C[i][e], dot, 0, 0, 0);
+                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(B[i][e + 1], C[i][e + 1], odd, 0, 0, 0);
+            }
+    }
+    dot += odd;
+    for (int n = first; n < end; ++n) {
+        const int h = blockIdx.z * per + n;
+        const float decay = here ? next_decay : 1.0f, skip = next_skip, dt[4] = {next_dt[0], next_dt[1], next_dt[2], next_dt[3]};
+        float p[4] = {1.f, 1.f, 1.f, 1.f}, P = 1.0f, Q = here ? next_Q : 0.0f;
+        if (n + 1 < end) fetch(n + 1);
+        static_for<16>([&](auto T) {
+            constexpr int q = decltype(T)::value;
+            const float d = row_lane<q>(decay), to = q <= j ? d : 1.0f;
+            P *= to;
+            Q *= q > j ? d : 1.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] *= q > 4 * g4 + i ? to : 1.0f;
+        });
+        float* out = a.tiles + ((int64_t)h * gridDim.x + blockIdx.x) * SSM_TILE;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int from = 4 * g4 + i;
+            const float v = dot[i] * (dt[i] * p[i]);
+            out[16 * from + j] = from > j || t0 + from >= a.M ? 0.0f : from == j ? v + skip : v;
+        }
+        if (g4 == 0) {
+            out[256 + j] = P;
+            out[272 + j] = Q;
+        }
+    }
 }
 
-// grid (heads, key groups * ceil(vdim / 64)), 256 threads; without the skip D x, which the row kernel behind it adds
-template <int KPL>
-__global__ __launch_bounds__(256, 1) void ssm_scan_kernel(const SsmRows a) {
-    constexpr int KP = 16 * KPL, KQ = KPL < 8 ? KPL : 8, Q = KPL / KQ, TT = 16 / Q;  // Q rows of [B | C] of KQ keys per token
-    constexpr int NG = (TT + 7) / 8;
-    __shared__ float s_o[2][4][TT][64];
+constexpr int ssm_tile_lds(int keys) { return 128 * keys + 4096 + 1024; }
+constexpr int ssm_stages(int keys) { return keys <= 128 ? 4 : keys <= 256 ? 3 : 2; }
+static int ssm_scan_lds(int waves, int keys) { return 2048 * waves + ssm_stages(keys) * ssm_tile_lds(keys); }
+
+// The state goes from 16 tokens to the next 16: y_t = P_t (C_t S) + sum(s <= t) M[s][t] x_s,  S <- P_15 S + sum(s) B_s Q_s x_s, on
+// v_mfma_f32_16x16x4_f32.  grid (heads, ceil(vdim / 16)), W waves: a wave has 16 columns and KT tiles of 16 keys of the state, as sums (row r of tile q is
+// key KT r + q of the wave's), which are, register by register, also the operand of C S.  The waves' sums meet in LDS.
+// A tile of tokens comes through LDS, STAGES of them in flight, with full instructions (B and C: 16-byte pieces, piece ^ row).
+// What bounds it: a turn (0.65 us) has 544 clocks of MFMAs on a SIMD and as many of LDS traffic on the CU, behind a barrier for the waves' sums; 40 heads are
+// 160 workgroups.  2048 tokens of 40 heads of 64, 128 keys: 89 us, 11 for the tiles in front; token by token on the vector units 217.  Four waves of
+// twice the keys 98, operands from memory straight to registers 104 (without loads 63, without the barrier 75).
+template <int W, int KT>
+__global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
+    constexpr int KP = 16 * W * KT, ROW = KP / 2, STAGES = ssm_stages(KP), TILE = ssm_tile_lds(KP), BC = 128 * KP;  // ROW: pieces of a row's B and C
+    constexpr int BCI = 2 * KT, PER = W == 8 ? BCI + 1 : BCI + 2;  // a wave's instructions for B and C of a tile, for all of it
+    extern __shared__ __align__(16) uint8_t ss_lds[];              // s_y, then the tiles: B and C, M with P and Q, x
+    float (*s_y)[W][256] = reinterpret_cast<float (*)[W][256]>(ss_lds);
+    constexpr int TILES = 2 * W * 1024;
     const SsmShape& m = a.m;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.x, N = m.state;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = wave & 3, j = lane & 15, g4 = lane >> 4, h = blockIdx.x, N = m.state;
     const int per = m.heads / m.groups, g = h / per, inner = m.heads * m.vdim, channels = inner + 2 * m.groups * N;
-    const int kg = blockIdx.y % a.key_groups, c0 = blockIdx.y / a.key_groups * 64, c = min(c0 + lane, m.vdim - 1), k0 = (4 * kg + wave) * KPL;
+    const int c0 = blockIdx.y * 16, c = min(c0 + j, m.vdim - 1), tiles = (a.M + 15) / 16;
     // the ring takes the inputs of the last positions
-    for (int j = 0; j < m.taps && j < a.M; ++j) {
-        const float* row = a.proj + (int64_t)(a.M - 1 - j) * a.ld + inner;
-        float* slot = a.ring + (a.pos0 + a.M - 1 - j) % m.taps * channels;
-        if (kg == 0 && wave == 0 && c0 + lane < m.vdim) slot[h * m.vdim + c] = row[h * m.vdim + c];
+    for (int q = 0; q < m.taps && q < a.M; ++q) {
+        const float* row = a.proj + (int64_t)(a.M - 1 - q) * a.ld + inner;
+        float* slot = a.ring + (a.pos0 + a.M - 1 - q) % m.taps * channels;
+        if (tid < 16 && c0 + tid < m.vdim) slot[h * m.vdim + c] = row[h * m.vdim + c];
         if (h % per == 0 && blockIdx.y == 0)
-            for (int i = tid; i < 2 * N; i += 256) {
+            for (int i = tid; i < 2 * N; i += 64 * W) {
                 const int ch = inner + (i < N ? 0 : m.groups * N) + g * N + i % N;
                 slot[ch] = row[ch];
             }
     }
-    float* state = a.state + ((int64_t)h * m.vdim + c) * KP + k0;
-    float S[KPL];
-    if (a.pos0 > 0) load_keys<KPL>(S, state);
-    else
+    float* state = a.state + ((int64_t)h * m.vdim + c) * KP + 16 * KT * wave + 4 * KT * g4;
+    rc_f4 S[KT];
+    {
+        float keys[4 * KT];
+        load_keys<4 * KT>(keys, state);
 #pragma unroll
-        for (int i = 0; i < KPL; ++i) S[i] = 0.0f;
-    // lane j of a row of lanes: B (j < KQ) or C (KQ <= j < 2 KQ) of key k0 + KQ q + j % KQ; the other lanes, and keys past the end,
-    // are zeros
-    const uint32_t step = (uint32_t)channels * 4, bytes = (uint32_t)a.M * step;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.conv, (int)bytes);
-    uint32_t off[Q];
+        for (int q = 0; q < KT; ++q)
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = lane & 15, key = k0 + KQ * q + j % KQ;
-        off[q] = key < N && j < 2 * KQ ? (uint32_t)(inner + (j < KQ ? 0 : m.groups * N) + g * N + key) * 4 : bytes;
+            for (int i = 0; i < 4; ++i) S[q][i] = a.pos0 > 0 ? keys[KT * i + q] : 0.0f;
     }
-    const uint32_t xoff = (uint32_t)(h * m.vdim + c) * 4;
-    const float* dsrc = a.decay + (lane & 8 ? m.heads : 0) + h;
-    struct Tile { float p[TT][Q], x[TT], d[NG]; } A, B;
-    const uint32_t last = bytes - step;
-    auto fetch = [&](Tile& x, int t0) {  // rows past the last repeat it and are not used
-        uint32_t row = min((uint32_t)t0 * step, last);
+    // memory -> LDS; rows past the last repeat it and count nothing, columns of x past the last are what lies there and are not stored
+    const uint32_t step = (uint32_t)a.conv_ld * 4, last = (uint32_t)(a.M - 1) * step;
+    const gt_i4 rows = gt_buffer(a.conv), pairs = gt_buffer(a.tiles + (int64_t)h * tiles * SSM_TILE);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)ss_lds + TILES;
+    uint32_t row_of[BCI], col_of[BCI];
 #pragma unroll
-        for (int i = 0; i < NG; ++i) x.d[i] = dsrc[(int64_t)min(t0 + 8 * i + (lane & 7), a.M - 1) * 2 * m.heads];  // decay, then dt, of eight tokens
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-#pragma unroll
-            for (int q = 0; q < Q; ++q) x.p[t][q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off[q], row, 0));
-            x.x[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, xoff, row, 0));
-            row = min(row + step, last);
-        }
-        issue_order_fence();
+    for (int i = 0; i < BCI; ++i) {
+        const int p = (BCI * wave + i) * 64 + lane, q = (p % ROW) ^ (p / ROW & 15);
+        row_of[i] = p / ROW * step;
+        col_of[i] = 4 * (conv_x(m) + (q < ROW / 2 ? g * KP : (m.groups + g) * KP) + 4 * (q % (ROW / 2)));
+    }
+    const uint32_t x_row = (4 * g4 + w4) * step, x_col = 4 * (h * m.vdim + c0 + j), pair_at = 16 * (18 * w4 + min(lane, 17));
+    auto fetch = [&](int n, int i) {
+        const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + n % STAGES * TILE), t0 = 16 * n * step;
+        if (i < BCI) gt_to_lds(at + (BCI * wave + i) * 1024, (int)(min(t0 + row_of[i], last) + col_of[i]), rows, 0);
+        else if (W == 8 ? wave < 4 : i == BCI) gt_to_lds(at + BC + w4 * 1024, (int)pair_at, pairs, n * SSM_TILE * 4);
+        else gt_word_to_lds(at + BC + 4096 + w4 * 256, (int)(min(t0 + x_row, last) + x_col), rows, 0);
     };
-    float* out = a.y + kg * a.y_slab + h * m.vdim + c0;
-    TileSums<TT> sums;
-    auto run = [&](Tile& x, int t0, int buf) {  // a token past the last leaves the state as it is
-        if (t0 > 0) sums.read(s_o[buf ^ 1]);
-        float decay[TT], dx[TT];
-        static_for<TT>([&](auto T) {
-            constexpr int t = decltype(T)::value;
-            decay[t] = row_lane<t % 8>(x.d[t / 8]);
-            dx[t] = row_lane<8 + t % 8>(x.d[t / 8]) * x.x[t];
-        });
-        if (t0 + TT > a.M) {
+    // LDS -> registers
+    struct Tile {
+        rc_f4 P, Q;
+        float C[4 * KT], B[4][KT], x[4], xw, from, end;
+    } T0, T1;
+    auto pair = [&](int f) { return BC + f / 72 * 1024 + f % 72 * 4; };  // where float f of M, P, Q lies in a tile
+    const int from_at = pair(16 * (4 * g4 + w4) + j), p_at = pair(256 + 4 * g4), q_at = pair(272 + 4 * g4), end_at = pair(271);
+    const int x_at = BC + 4096 + 64 * g4 + 4 * j;                        // of row 4 g4: row 4 g4 + i 256 i further on
+    constexpr int READS = KT + 6;
+    auto read = [&](Tile& v, int n, int part) {
+        const uint8_t* t = ss_lds + TILES + n % STAGES * TILE;
+        if (part < KT) {
+            const int q = part;
+            const float4 x = *reinterpret_cast<const float4*>(t + (j * ROW + ((ROW / 2 + (4 * wave + g4) * KT + q) ^ j)) * 16);
+            v.C[4 * q] = x.x; v.C[4 * q + 1] = x.y; v.C[4 * q + 2] = x.z; v.C[4 * q + 3] = x.w;
+        } else if (part < KT + 4) {
+            const int i = part - KT, r = 4 * g4 + i, k = (16 * wave + j) * KT;
+            const uint8_t* b = t + (r * ROW + ((k >> 2) ^ r)) * 16 + (k & 3) * 4;
+            if constexpr (KT == 1) v.B[i][0] = *reinterpret_cast<const float*>(b);
+            else if constexpr (KT == 2) {
+                const float2 x = *reinterpret_cast<const float2*>(b);
+                v.B[i][0] = x.x; v.B[i][1] = x.y;
+            } else {
+                const float4 x = *reinterpret_cast<const float4*>(b);
+                v.B[i][0] = x.x; v.B[i][1] = x.y; v.B[i][2] = x.z; v.B[i][3] = x.w;
+            }
+            v.x[i] = *reinterpret_cast<const float*>(t + x_at + 256 * i);
+        } else if (part == KT + 4) {
+            v.xw = *reinterpret_cast<const float*>(t + x_at + 256 * w4);
+            v.from = *reinterpret_cast<const float*>(t + from_at);
+            v.end = *reinterpret_cast<const float*>(t + end_at);
+        } else {
+            v.P = *reinterpret_cast<const rc_f4*>(t + p_at);
+            v.Q = *reinterpret_cast<const rc_f4*>(t + q_at);
+        }
+    };
+    // the waves' sums of a tile (waves 0 .. 3), on their way from LDS while the next tile is used
+    float sums[W];
+    auto read_sums = [&](int n) {
+        if (wave < 4)
 #pragma unroll
-            for (int t = 0; t < TT; ++t)
-                if (t0 + t >= a.M) {
-                    decay[t] = 1.0f;
-                    dx[t] = 0.0f;
+            for (int w = 0; w < W; ++w) sums[w] = s_y[n & 1][w][tid & 255];
+    };
+    const bool stored = tid < 256 && c0 + j < m.vdim;
+    float* y = a.y + (int64_t)(tid >> 4 & 15) * inner + h * m.vdim + c0 + j;
+    auto put = [&](int n) {
+        if (!stored || 16 * n + (tid >> 4) >= a.M) return;
+        float v = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+        if constexpr (W == 8) v += (sums[4] + sums[5]) + (sums[6] + sums[7]);
+        y[(int64_t)16 * n * inner] = v;
+    };
+    auto run = [&](const Tile& v, Tile& next, int n) {
+        // the next tile has arrived in every wave's part; the one used now lies in registers, and its LDS takes one more
+        if (n + STAGES - 1 < tiles) gt_arrived<(STAGES - 2) * PER>();
+        else gt_arrived<0>();
+        rc_f4 old[KT], here = {0.f, 0.f, 0.f, 0.f}, next_S[KT];
+        float dx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dx[i] = v.x[i] * v.Q[i];
+#pragma unroll
+        for (int q = 0; q < KT; ++q) {
+            old[q] = rc_f4{0.f, 0.f, 0.f, 0.f};
+            next_S[q] = S[q] * v.end;
+        }
+        // sums that do not depend on each other take turns, and what is read and requested for later tiles goes out between them
+        constexpr int OPS = 1 + READS + PER, SLOTS = 4 * KT;
+        const bool more = n + STAGES < tiles;
+        auto between = [&](int slot) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int o = 0; o < OPS; ++o)
+                if (o * SLOTS / OPS == slot) {
+                    if (o == 0) read_sums(n + 1);  // n - 1
+                    else if (o <= READS) read(next, n + 1, o - 1);
+                    else if (more) fetch(n + STAGES, o - 1 - READS);
                 }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (wave < 4) here = __builtin_amdgcn_mfma_f32_16x16x4f32(v.from, v.xw, here, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < KT; ++q) {
+                old[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.C[KT * i + q], S[q][i], old[q], 0, 0, 0);
+                next_S[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.B[i][q], dx[i], next_S[q], 0, 0, 0);
+                between(KT * i + q);
+            }
+        if (n > 0) put(n - 1);
+#pragma unroll
+        for (int q = 0; q < KT; ++q) S[q] = next_S[q];
+#pragma unroll
+        for (int q = 1; q < KT; ++q) old[0] += old[q];
+        if (__builtin_expect(wave < 4 && __builtin_amdgcn_ballot_w64(!(fabsf(v.xw) < INFINITY)) != 0, 0)) {  // 0 times infinity: no token takes from a later one
+            here = rc_f4{0.f, 0.f, 0.f, 0.f};
+            const float* t = a.tiles + ((int64_t)h * tiles + n) * SSM_TILE;
+            for (int b = 0; b < 4; ++b) {
+                const float xs = __shfl(v.xw, 16 * b + j, 64);
+                const int from = 4 * b + wave;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (from <= 4 * g4 + i) here[i] = fmaf(t[16 * from + 4 * g4 + i], xs, here[i]);
+            }
         }
 #pragma unroll
-        for (int t = 0; t < TT; t += 4) {
-            float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            static_for<KPL / 4>([&](auto I) {
-                constexpr int i = 4 * decltype(I)::value, b0 = i % KQ, q = i / KQ;
-                ssm_keys4<b0, KQ + b0>(S + i, y, x.p[t][q], x.p[t + 1][q], x.p[t + 2][q], x.p[t + 3][q], decay + t, dx + t);
-            });
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s_o[buf][wave][t + i][lane] = y[i];
-        }
-        if (t0 > 0) sums.store(out, inner, t0 - TT, a.M, m.vdim - c0);
-        __syncthreads();
+        for (int i = 0; i < 4; ++i) s_y[n & 1][wave][16 * (4 * g4 + i) + j] = fmaf(v.P[i], old[0][i], here[i]);
     };
-    fetch(A, 0);
-    int t0 = 0;
-    for (;; t0 += 2 * TT) {
-        fetch(B, t0 + TT);
-        run(A, t0, 0);
-        if (t0 + TT >= a.M) break;
-        fetch(A, t0 + 2 * TT);
-        run(B, t0 + TT, 1);
-        if (t0 + 2 * TT >= a.M) { t0 += TT; break; }
+#pragma unroll
+    for (int n = 0; n < STAGES; ++n)
+        if (n < tiles)
+#pragma unroll
+            for (int i = 0; i < PER; ++i) fetch(n, i);
+    if (tiles >= STAGES) gt_arrived<(STAGES - 1) * PER>();
+    else gt_arrived<0>();
+#pragma unroll
+    for (int i = 0; i < READS; ++i) read(T0, 0, i);
+    for (int n = 0; n < tiles; n += 2) {
+        run(T0, T1, n);
+        if (n + 1 < tiles) run(T1, T0, n + 1);
     }
-    sums.read(s_o[t0 / TT & 1]);
-    sums.store(out, inner, t0, a.M, m.vdim - c0);
-    if (c0 + lane < m.vdim) store_keys<KPL>(state, S);
+    __syncthreads();
+    read_sums(tiles - 1);
+    put(tiles - 1);
+    if (c0 + j < m.vdim) {
+        float keys[4 * KT];
+#pragma unroll
+        for (int q = 0; q < KT; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) keys[KT * i + q] = S[q][i];
+        store_keys<4 * KT>(state, keys);
+    }
 }
 
-// grid rows: (the scan's sums + D x) * silu(z), normed in equal parts, times norm and the branch's scale
+// grid rows: the scan's y * silu(z), normed in equal parts, times norm and the branch's scale.  All that a row reads goes out together (2560 values, each
+// piece's loads behind the use of the one before: 16 rows 10.3 us, 2048 24).
 template <bool F32>
 __global__ __launch_bounds__(256) void ssm_out_rows_kernel(const SsmRows a) {
     __shared__ float red[4];
     const SsmShape& m = a.m;
-    const int tid = threadIdx.x, inner = m.heads * m.vdim, channels = inner + 2 * m.groups * m.state, part = inner / m.norm_groups;
-    const float *y = a.y + (int64_t)blockIdx.x * inner, *x = a.conv + (int64_t)blockIdx.x * channels, *z = a.proj + blockIdx.x * a.ld;
-    auto value = [&](int c) {
-        float s[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[k] = k < a.key_groups ? y[k * a.y_slab + c] : 0.0f;
-        return fmaf(m.D[c / m.vdim], x[c], (s[0] + s[1]) + (s[2] + s[3])) * silu_f(z[c]);
-    };
+    const int tid = threadIdx.x, inner = m.heads * m.vdim, part = inner / m.norm_groups;
+    const float *y = a.y + (int64_t)blockIdx.x * inner, *z = a.proj + blockIdx.x * a.ld;
     constexpr int NS = 16;  // values kept in registers: parts of up to 4096
+    const int pieces = min((part + 255) / 256, NS);
     for (int p = 0; p < m.norm_groups; ++p) {
         const int c0 = p * part;
-        float v[NS], ss = 0.0f;
+        float v[NS], g[NS], n[NS], ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            const int c = tid + 256 * i;
-            v[i] = c < part ? value(c0 + c) : 0.0f;
-            ss = fmaf(v[i], v[i], ss);
-        }
+        for (int i = 0; i < NS; ++i)
+            if (i < pieces) {
+                const int c = c0 + min(tid + 256 * i, part - 1);
+                v[i] = y[c];
+                g[i] = z[c];
+                n[i] = m.norm[c];
+            }
+        issue_order_fence();
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+            if (i < pieces) {
+                v[i] = tid + 256 * i < part ? v[i] * silu_f(g[i]) : 0.0f;
+                ss = fmaf(v[i], v[i], ss);
+            }
         for (int c = tid + 256 * NS; c < part; c += 256) {
-            const float t = value(c0 + c);
+            const float t = y[c0 + c] * silu_f(z[c0 + c]);
             ss = fmaf(t, t, ss);
         }
         const float r = 1.0f / sqrtf(block_sum<4>(ss, red) / (float)part + a.eps) * m.scale;
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             const int c = tid + 256 * i;
-            if (c < part) put_elem<F32>(a.out, blockIdx.x * a.out_ld + c0 + c, v[i] * r * m.norm[c0 + c]);
+            if (c < part) put_elem<F32>(a.out, blockIdx.x * a.out_ld + c0 + c, v[i] * r * n[i]);
         }
-        for (int c = tid + 256 * NS; c < part; c += 256) put_elem<F32>(a.out, blockIdx.x * a.out_ld + c0 + c, value(c0 + c) * r * m.norm[c0 + c]);
+        for (int c = tid + 256 * NS; c < part; c += 256) put_elem<F32>(a.out, blockIdx.x * a.out_ld + c0 + c, y[c0 + c] * silu_f(z[c0 + c]) * r * m.norm[c0 + c]);
     }
 }
 
@@ -655,12 +815,25 @@ int wkv_rows(WkvRows a, bool fp32, hipStream_t s) {
 int ssm_rows(SsmRows a, bool fp32, hipStream_t s) {
     const SsmShape& m = a.m;
     if (!recurrent_supported(m.state)) return PTM_E_UNSUPPORTED;
-    const int channels = m.heads * m.vdim + 2 * m.groups * m.state;
-    a.key_groups = key_groups(m.state);
-    hipLaunchKernelGGL(ssm_conv_rows_kernel, dim3((a.M + CONV_ROWS - 1) / CONV_ROWS, (channels + 255) / 256 + 1), dim3(256), 0, s, a);
-    const dim3 grid(m.heads, a.key_groups * ((m.vdim + 63) / 64));
-#define PTM_RUN(KPL) hipLaunchKernelGGL(ssm_scan_kernel<KPL>, grid, dim3(256), 0, s, a)
-    PTM_KPL(m.state, PTM_RUN)
+    a.keys = padded_keys(m.state);
+    a.conv_ld = ssm_conv_row(m);
+    hipLaunchKernelGGL(ssm_conv_rows_kernel, dim3((a.M + CONV_ROWS - 1) / CONV_ROWS, (unsigned)((a.conv_ld + 255) / 256 + 1)), dim3(256), 0, s, a);
+    const int per = m.heads / m.groups, each = (int64_t)(a.M + 15) / 16 * m.heads > 4096 ? 2 : 1;
+    hipLaunchKernelGGL(ssm_tiles_kernel, dim3((a.M + 15) / 16, (per + 4 * each - 1) / (4 * each), m.groups), dim3(256), 0, s, a, each);
+    const dim3 grid(m.heads, (m.vdim + 15) / 16);
+    static std::once_flag raised;
+    std::call_once(raised, [] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 128));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 256));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 512));
+    });
+#define PTM_RUN(W, KT) hipLaunchKernelGGL((ssm_scan_kernel<W, KT>), grid, dim3(64 * W), ssm_scan_lds(W, a.keys), s, a)
+    switch (a.keys) {
+        case 64: PTM_RUN(4, 1); break;
+        case 128: PTM_RUN(8, 1); break;
+        case 256: PTM_RUN(8, 2); break;
+        default: PTM_RUN(8, 4);
+    }
 #undef PTM_RUN
     if (fp32) hipLaunchKernelGGL(ssm_out_rows_kernel<true>, dim3(a.M), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(ssm_out_rows_kernel<false>, dim3(a.M), dim3(256), 0, s, a);

@@ -5,6 +5,7 @@
 #include "dense_gemv.h"
 #include "gemm_plan.h"
 #include "ptm.h"
+#include "recurrent.h"
 
 namespace ptm {
 int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
@@ -136,5 +137,35 @@ int act_down(uint32_t type, const void* W, int64_t stride, const float* G, const
     const int rc = ptm::qgemm_f16_act_rows(G, U, sg, su, gelu != 0, type == PTM_TYPE_Q4_K, ws, bps, M, K, s);
     return rc ? rc : ptm::qgemm_f16_impl(type, W, G, true, Y, M, K, N, stride, ws, false, split_ws, (size_t)split_bytes, true, s, nullptr, true);
 }
+
+// prompt rows of a state-space mixer, fp32: weights w = conv, conv_b, dt_bias, neg_a, D, norm; scratch = conv rows, decays, tiles, y
+int64_t ssm_scratch(int heads, int vdim, int state, int groups, int M, int what) {
+    ptm::SsmShape m{};
+    m.heads = heads;
+    m.vdim = vdim;
+    m.state = state;
+    m.groups = groups;
+    return what == 0 ? ptm::ssm_conv_row(m) * M : what == 1 ? 2 * (int64_t)heads * M : what == 2 ? ptm::ssm_tile_floats(heads, M) : (int64_t)heads * vdim * M;
+}
+int ssm_run(const int* shape, const float* const* w, const float* proj, int M, int64_t pos0, float* ring, float* state, float* const* scratch, float* out, void* stream) {
+    ptm::SsmRows r{};
+    r.m = {shape[0], shape[1], shape[2], shape[3], shape[4], 1, w[0], w[1], w[2], w[3], w[4], w[5], 1.0f};
+    const int inner = r.m.heads * r.m.vdim;
+    r.proj = proj;
+    r.ld = 2 * inner + 2 * r.m.groups * r.m.state + r.m.heads;
+    r.M = M;
+    r.pos0 = pos0;
+    r.eps = 1e-6f;
+    r.ring = ring;
+    r.state = state;
+    r.conv = scratch[0];
+    r.decay = scratch[1];
+    r.tiles = scratch[2];
+    r.y = scratch[3];
+    r.out = out;
+    r.out_ld = inner;
+    return ptm::ssm_rows(r, true, static_cast<hipStream_t>(stream));
+}
+int64_t ssm_state_floats(int heads, int state, int vdim) { return ptm::recurrent_state_floats(heads, state, vdim); }
 
 }  // extern "C"

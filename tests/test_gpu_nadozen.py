@@ -418,3 +418,68 @@ def test_decoding_at_large_widths(dev, tmp_path, width, ff):
         m = registry.load(path, max_seq=8, precision=precision)
         assert_close(portions(m, tokens, [1]), want, precision, (width, ff))
         m.close()
+
+
+# ---- the scan over 16 tokens at a time ------------------------------------------------------------------
+def ssm_reference(w, proj, m, pos0, ring, S):
+    """Token by token in 64 bits: (y * silu(z) before the norm's row kernel, normed), state."""
+    import torch
+    H, V, n, G, taps = m
+    inner, ch = H * V, H * V + 2 * G * n
+    conv, cb, dtb, neg_a, D, norm = [t.double() for t in w]
+    p = proj.double()
+    past = [ring[(pos0 - taps + 1 + j) % taps].double() if pos0 - taps + 1 + j >= 0 else torch.zeros(ch, device="cuda", dtype=torch.float64) for j in range(taps - 1)]
+    x = torch.cat([torch.stack(past)] * (taps > 1) + [p[:, inner:inner + ch]])
+    c = torch.nn.functional.silu(sum(x[j:j + len(p)] * conv[:, j] for j in range(taps)) + cb)
+    dt = torch.nn.functional.softplus(p[:, inner + ch:] + dtb)
+    out = []
+    for t in range(len(p)):
+        xt, B, C = c[t, :inner].reshape(H, V), *(c[t, inner + i * G * n:inner + (i + 1) * G * n].reshape(G, n).repeat_interleave(H // G, 0) for i in (0, 1))
+        S = torch.exp(neg_a * dt[t])[:, None, None] * S + dt[t][:, None, None] * xt[:, :, None] * B[:, None, :]
+        y = (S * C[:, None, :]).sum(2) + D[:, None] * xt
+        y = y.reshape(-1) * torch.nn.functional.silu(p[t, :inner])
+        out.append(y / (y.pow(2).mean() + 1e-6).sqrt() * norm)
+    return torch.stack(out), S
+
+
+# every number of key tiles a wave has, states and columns off the tiles, groups, more rows than tiles in flight, tokens off 16
+@pytest.mark.parametrize("heads,vdim,state,groups,taps,rows", [(2, 16, 64, 1, 4, 16), (3, 5, 20, 1, 2, 15), (4, 64, 128, 1, 4, 97), (4, 33, 100, 2, 3, 130), (2, 17, 200, 1, 4, 49),
+                                                               (2, 16, 256, 2, 4, 17), (2, 20, 300, 1, 4, 70), (1, 64, 512, 1, 6, 33), (18, 8, 16, 2, 4, 1)])
+@pytest.mark.parametrize("pos0", [0, 21])
+def test_state_space_scan(dev, heads, vdim, state, groups, taps, rows, pos0):
+    """One call against the recurrence in 64 bits.  A sum of up to 512 products, 16 decays deep, is off by some 1e-6 of its terms; a first value that is
+    infinite reaches no token before its own."""
+    import torch
+    from gemm_helpers import harness
+    h = harness()
+    for f in ("ssm_scratch", "ssm_state_floats"):
+        getattr(h, f).restype = C.c_int64
+    g = torch.Generator(device="cuda").manual_seed(rows + state)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    inner, ch = heads * vdim, heads * vdim + 2 * groups * state
+    w = [rand(ch, taps) * taps ** -0.5, 0.1 * rand(ch), rand(heads) - 2, -torch.exp(0.8 * rand(heads)), rand(heads), 1 + 0.1 * rand(inner)]
+    proj, ring = rand(rows, inner + ch + heads), rand(taps, ch)
+    kp = h.ssm_state_floats(1, state, 1)
+    S0 = torch.zeros(heads, vdim, kp, device="cuda")
+    S0[:, :, :state] = rand(heads, vdim, state)
+
+    def run(proj):
+        S, r, out = S0.clone(), ring.clone(), torch.empty(rows, inner, device="cuda")
+        scratch = [torch.full((h.ssm_scratch(heads, vdim, state, groups, rows, i),), float("nan"), device="cuda") for i in range(4)]
+        ptrs = lambda ts: (C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+        assert h.ssm_run((C.c_int * 5)(heads, vdim, state, groups, taps), ptrs(w), C.c_void_p(proj.data_ptr()), rows, C.c_int64(pos0), C.c_void_p(r.data_ptr()),
+                         C.c_void_p(S.data_ptr()), ptrs(scratch), C.c_void_p(out.data_ptr()), None) == 0
+        torch.cuda.synchronize()
+        return out, S, r
+
+    out, S, r = run(proj)
+    want, want_S = ssm_reference(w, proj, (heads, vdim, state, groups, taps), pos0, ring, (S0[:, :, :state] if pos0 else 0 * S0[:, :, :state]).double())
+    for a, b in ((out, want), (S[:, :, :state], want_S)):
+        assert float((a.double() - b).abs().max() / b.pow(2).mean().sqrt()) < 3e-5
+    assert (S[:, :, state:] == 0).all()
+    for j in range(min(taps, rows)):
+        assert torch.equal(r[(pos0 + rows - 1 - j) % taps], proj[rows - 1 - j, inner:inner + ch])
+    if rows > 9:
+        loud = proj.clone()
+        loud[9, inner] = float("inf")
+        assert torch.equal(run(loud)[0][:9], out[:9])
