@@ -16,9 +16,8 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",
 ]
-# Per-file additions.  prefill.hip, mixer_attention.hip: their matrix-core attention rescales the output accumulators between MFMAs with vector
-# arithmetic, which cannot touch accumulation registers; with the accumulators there the compiler copies all 64 of them
-# out and back on every tile.  One wave per SIMD leaves room for them in ordinary registers.
+# Per-file additions.  The matrix-core attention rescales its output accumulators between MFMAs with vector arithmetic, the recurrent scans the state,
+# and vector arithmetic cannot touch accumulation registers; with the accumulators there the compiler copies all of them out and back on every tile.  One wave per SIMD leaves room for them in ordinary registers.
 FILE_FLAGS = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("prefill.hip", "mixer_attention.hip", "prompt_attention.hip", "recurrent.hip")}
 
 

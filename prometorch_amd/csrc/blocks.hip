@@ -1123,7 +1123,8 @@ int blocks_reserve(BlockStack* b, int rows) {
         if (wkv(L)) {
             shifted = R * W;
             grow(low, (size_t)up64(L.wkv.rank));
-            grow(scan, (size_t)scan_slabs(L.wkv.dim) * (size_t)(L.wkv.heads * L.wkv.dim));
+            grow(scan, (size_t)(L.wkv.heads * L.wkv.dim));
+            grow(tiles, (size_t)wkv_tile_floats(L.wkv.heads, L.wkv.dim, rows));
         } else {
             grow(q, (size_t)q_cols(L));
         }
@@ -1233,9 +1234,9 @@ static int wkv_prompt(BlockStack* b, const ptm_block& L, const LayerRun& run, in
     w.eps = b->cfg.eps;
     w.pos0 = pos0;
     w.state = run.state;
+    w.tiles = b->r_tiles;
     w.o = b->r_scan;
     w.o_ld = hd;
-    w.o_slab = (int64_t)M * hd;
     w.out = b->r_attn;
     w.out_ld = up64(attn_cols(L));
     w.h_last = b->r_hn + (int64_t)(M - 1) * b->wp;

@@ -30,9 +30,10 @@ struct WkvRows {
     float eps;
     int64_t pos0;
     float* state;
-    float* o;                 // [scan_slabs(dim)][M][o_ld], o_slab floats apart
-    int64_t o_ld, o_slab;
-    int groups;               // set by wkv_rows
+    float* tiles;             // wkv_tile_floats, 16-byte aligned
+    float* o;                 // [M][o_ld]
+    int64_t o_ld;
+    int keys;                 // set by wkv_rows
     void* out;                // [M][out_ld]
     int64_t out_ld;
     const float* h_last;      // the mixer's last input row, kept for the next token's shift
@@ -40,7 +41,7 @@ struct WkvRows {
     int wp;
 };
 int wkv_rows(WkvRows a, bool fp32, hipStream_t s);
-int64_t scan_slabs(int keys);  // partial sums that a scan leaves per row
+int64_t wkv_tile_floats(int heads, int dim, int rows);
 int token_shift_rows(const float* h, const float* shift, const float* mu, int n, int rows, int64_t pos0, int wp, bool fp32, void* out, hipStream_t s);
 int tanh_rows(const float* g, int slabs, int64_t slab, int rows, int n, bool fp32, void* out, hipStream_t s);
 

@@ -5,12 +5,7 @@
 //
 // A state is stored per value column, its key values consecutive and padded: [heads][columns][16 * KPL].
 // One token: 16 lanes share a column, KPL key values each, so a wave holds four columns and a read of the state is consecutive.
-// Prompt rows, ssm: 16 tokens at a time on the fp32 matrix cores (ssm_scan_kernel).
-// Prompt rows, wkv: neither the columns nor the keys of a state depend on each other, only the sum over the keys does.  A lane is a value
-// column and a wave has KPL keys of 64 columns in registers, so what belongs to a key (r, k, w) is one value for the whole
-// wave: it is loaded once into a row of 16 lanes and broadcast as a DPP operand of the arithmetic, three instructions per key and
-// token.  A workgroup's four waves add their sums through LDS; up to four workgroups share a head and leave partial sums, which the
-// row kernel behind the scan adds.  The next tile's vectors are on their way while a tile of tokens is used.
+// Prompt rows: 16 tokens at a time on the fp32 matrix cores (scan_columns); a launch in front leaves what the 16 take from each other.
 // A sequence's first position starts from zeros instead of the stored state, so nothing has to be cleared between sequences.
 // What a token needs from earlier ones besides the state (the token shift's vector, the convolution's inputs) lies in rings
 // indexed by position; a slot is never read and written by the same launch.
@@ -196,159 +191,52 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const SsmStep a) {
 }
 
 // ---- prompt rows ---------------------------------------------------------------------------------
-// workgroups that share the keys of a head, four waves of KPL keys each
-static int key_groups(int keys) { return (keys + 4 * keys_per_lane(keys) - 1) / (4 * keys_per_lane(keys)); }
-
 // value of lane N of each row of 16 lanes, as an operand of the next instruction
 template <int N>
 __device__ __forceinline__ float row_lane(float v) { return dpp_f<0x150 + N>(v); }
 
-// The waves' sums of a tile of TT tokens (s_o [4][TT][64]), on their way from LDS while the next tile is used: this wave's rows
-// wave, wave + 4, ...
-template <int TT>
-struct TileSums {
-    float v[TT / 4][4];
-    __device__ __forceinline__ void read(const float (*s_o)[TT][64]) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int q = 0; q < TT / 4; ++q)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) v[q][w] = s_o[w][wave + 4 * q][lane];
-    }
-    __device__ __forceinline__ void store(float* out, int64_t ld, int t0, int M, int columns) const {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int q = 0; q < TT / 4; ++q) {
-            const int t = t0 + wave + 4 * q;
-            if (t < M && lane < columns) out[(int64_t)t * ld + lane] = (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
-        }
-    }
-};
+static int padded_keys(int n) { return 16 * keys_per_lane(n); }
 
-// Four keys of 64 columns take four tokens: o += S^T r, S <- diag(w) S + k v^T.  p[t]: a row of lanes [r | k | w | -], four each.
-// (One block, because the compiler does not fold the broadcasts into the multiply-adds; the wait states are for p.)
-#define PTM_DPP(n) " row_newbcast:" n " row_mask:0xf bank_mask:0xf\n\t"
-#define PTM_WKV_TOKEN(O, P, V)                                   \
-    "v_fmac_f32_dpp %" O ", %" P ", %0" PTM_DPP("0")             \
-    "v_mul_f32_dpp %0, %" P ", %0" PTM_DPP("8")                  \
-    "v_fmac_f32_dpp %" O ", %" P ", %1" PTM_DPP("1")             \
-    "v_mul_f32_dpp %1, %" P ", %1" PTM_DPP("9")                  \
-    "v_fmac_f32_dpp %" O ", %" P ", %2" PTM_DPP("2")             \
-    "v_mul_f32_dpp %2, %" P ", %2" PTM_DPP("10")                 \
-    "v_fmac_f32_dpp %" O ", %" P ", %3" PTM_DPP("3")             \
-    "v_mul_f32_dpp %3, %" P ", %3" PTM_DPP("11")                 \
-    "v_fmac_f32_dpp %0, %" P ", %" V PTM_DPP("4")                \
-    "v_fmac_f32_dpp %1, %" P ", %" V PTM_DPP("5")                \
-    "v_fmac_f32_dpp %2, %" P ", %" V PTM_DPP("6")                \
-    "v_fmac_f32_dpp %3, %" P ", %" V PTM_DPP("7")
-__device__ __forceinline__ void wkv_keys4(float* s, float (&o)[4], float p0, float p1, float p2, float p3, float v0, float v1, float v2, float v3) {
-    asm("s_nop 1\n\t" PTM_WKV_TOKEN("4", "8", "12") PTM_WKV_TOKEN("5", "9", "13") PTM_WKV_TOKEN("6", "10", "14") PTM_WKV_TOKEN("7", "11", "15")
-        : "+&v"(s[0]), "+&v"(s[1]), "+&v"(s[2]), "+&v"(s[3]), "+&v"(o[0]), "+&v"(o[1]), "+&v"(o[2]), "+&v"(o[3])
-        : "v"(p0), "v"(p1), "v"(p2), "v"(p3), "v"(v0), "v"(v1), "v"(v2), "v"(v3));
+// The scan's o of each row and head over its root mean square, times norm and silu(gate).  It moves memory: four values a lane and G lanes a head where the
+// addresses allow, 1024 / G heads a workgroup (2048 rows of 40 heads of 64: a wave per head 22.2 us, this 12.9).  grid ceil(rows * heads / (256 / G))
+template <bool F32, int G>
+__global__ __launch_bounds__(256) void wkv_out_fours_kernel(const WkvRows a) {
+    const int at = blockIdx.x * (256 / G) + threadIdx.x / G, row = at / a.heads, h = at % a.heads, d = a.dim, e = 4 * (threadIdx.x % G);
+    if (row >= a.M) return;
+    const bool in = e < d;
+    const int c = h * d + (in ? e : 0);
+    const rc_f4 o = *reinterpret_cast<const rc_f4*>(a.o + row * a.o_ld + c), g = *reinterpret_cast<const rc_f4*>(a.proj + row * a.ld + 3 * a.section + c),
+                n = *reinterpret_cast<const rc_f4*>(a.norm + c);
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss = fmaf(o[i], o[i], ss);
+    const float r = 1.0f / sqrtf(sum_lanes<G>(in ? ss : 0.0f) / (float)d + a.eps);
+    rc_f4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = o[i] * r * n[i] * silu_f(g[i]);
+    if (!in) return;
+    if constexpr (F32) *reinterpret_cast<rc_f4*>(static_cast<float*>(a.out) + row * a.out_ld + c) = v;
+    else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + row * a.out_ld + c) =
+             make_uint2((uint32_t)f_bf16(v[0]) | ((uint32_t)f_bf16(v[1]) << 16), (uint32_t)f_bf16(v[2]) | ((uint32_t)f_bf16(v[3]) << 16));
 }
-
-// grid (heads, key groups * ceil(dim / 64)), 256 threads.  Without the bonus, which the row kernel behind it adds.
-template <int KPL>
-__global__ __launch_bounds__(256, 1) void wkv_scan_kernel(const WkvRows a) {
-    constexpr int KP = 16 * KPL, Q = KPL / 4, TT = Q < 4 ? 16 / Q : 4;  // Q rows of [r | k | w] of four keys per token
-    __shared__ float s_o[2][4][TT][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.x, d = a.dim;
-    const int kg = blockIdx.y % a.groups, c0 = blockIdx.y / a.groups * 64, c = min(c0 + lane, d - 1), k0 = (4 * kg + wave) * KPL;
-    if (h == 0 && blockIdx.y == 0)  // the next token's shift reads the last row
-        for (int i = tid; i < a.wp; i += 256) a.shift[(a.pos0 + a.M - 1) % 2 * a.wp + i] = a.h_last[i];
-    float* state = a.state + ((int64_t)h * d + c) * KP + k0;
-    float S[KPL];
-    if (a.pos0 > 0) load_keys<KPL>(S, state);
-    else
-#pragma unroll
-        for (int i = 0; i < KPL; ++i) S[i] = 0.0f;
-    // lane j of a row of lanes: r (0..3), k (4..7), w (8..11) of key k0 + 4 q + j % 4; keys past the end, and lanes 12..15, are zeros
-    const uint32_t step = (uint32_t)a.ld * 4, bytes = (uint32_t)a.M * step, part = (lane >> 2) & 3;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.proj, (int)bytes);
-    uint32_t off[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int key = k0 + 4 * q + (lane & 3);
-        off[q] = key < d && part < 3 ? (uint32_t)((part == 2 ? 4 : part) * a.section + h * d + key) * 4 : bytes;
-    }
-    const uint32_t voff = (uint32_t)(2 * a.section + h * d + c) * 4;
-    struct Tile { float p[TT][Q], v[TT]; } A, B;
-    const uint32_t last = bytes - step;
-    auto fetch = [&](Tile& x, int t0) {  // rows past the last repeat it and are not used
-        uint32_t row = min((uint32_t)t0 * step, last);
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-#pragma unroll
-            for (int q = 0; q < Q; ++q) x.p[t][q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off[q], row, 0));
-            x.v[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, voff, row, 0));
-            row = min(row + step, last);
-        }
-        issue_order_fence();
-    };
-    float* out = a.o + kg * a.o_slab + (int64_t)h * d + c0;
-    TileSums<TT> sums;
-    auto run = [&](Tile& x, int t0, int buf) {  // a token past the last leaves the state as it is
-        if (t0 > 0) sums.read(s_o[buf ^ 1]);
-        if (t0 + TT > a.M) {
-            const float keep = part == 2 ? 1.0f : 0.0f;
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-                if (t0 + t >= a.M)
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) x.p[t][q] = keep;
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t += 4) {
-            float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-                wkv_keys4(S + 4 * q, o, x.p[t][q], x.p[t + 1][q], x.p[t + 2][q], x.p[t + 3][q], x.v[t], x.v[t + 1], x.v[t + 2], x.v[t + 3]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s_o[buf][wave][t + i][lane] = o[i];
-        }
-        if (t0 > 0) sums.store(out, a.o_ld, t0 - TT, a.M, d - c0);
-        __syncthreads();
-    };
-    fetch(A, 0);
-    int t0 = 0;
-    for (;; t0 += 2 * TT) {
-        fetch(B, t0 + TT);
-        run(A, t0, 0);
-        if (t0 + TT >= a.M) break;
-        fetch(A, t0 + 2 * TT);
-        run(B, t0 + TT, 1);
-        if (t0 + 2 * TT >= a.M) { t0 += TT; break; }
-    }
-    sums.read(s_o[t0 / TT & 1]);
-    sums.store(out, a.o_ld, t0, a.M, d - c0);
-    if (c0 + lane < d) store_keys<KPL>(state, S);
-}
-
-// grid (rows, ceil(heads / 4)), a wave per head: o = the scan's sums + the bonus; over its root mean square, times norm and
-// silu(gate).  NV: values per lane.
+// the same for any head and alignment, grid (rows, ceil(heads / 4)), a wave per head, NV values a lane
 template <bool F32, int NV>
 __global__ __launch_bounds__(256) void wkv_out_rows_kernel(const WkvRows a) {
     const int lane = threadIdx.x & 63, h = blockIdx.y * 4 + (threadIdx.x >> 6), d = a.dim;
     if (h >= a.heads) return;
     const float *p = a.proj + blockIdx.x * a.ld + h * d, *o = a.o + blockIdx.x * a.o_ld + h * d;
-    float x[NV][4], v[NV], g[NV], n[NV], b[NV];
+    float v[NV], g[NV], n[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int e = min(lane + 64 * i, d - 1);
-#pragma unroll
-        for (int z = 0; z < 4; ++z) x[i][z] = z < a.groups ? o[z * a.o_slab + e] : 0.0f;
-        v[i] = p[2 * a.section + e];
+        v[i] = o[e];
         g[i] = p[3 * a.section + e];
         n[i] = a.norm[h * d + e];
-        b[i] = p[e] * a.u[h * d + e] * p[a.section + e];
     }
-    float bonus = 0.0f, ss = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) bonus += lane + 64 * i < d ? b[i] : 0.0f;
-    bonus = sum64(bonus);
+    float ss = 0.0f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        v[i] = lane + 64 * i < d ? fmaf(bonus, v[i], (x[i][0] + x[i][1]) + (x[i][2] + x[i][3])) : 0.0f;
+        v[i] = lane + 64 * i < d ? v[i] : 0.0f;
         ss = fmaf(v[i], v[i], ss);
     }
     const float r = 1.0f / sqrtf(sum64(ss) / (float)d + a.eps);
@@ -393,7 +281,6 @@ __global__ __launch_bounds__(64) void tanh_rows_kernel(const float* __restrict__
 
 // Where x, B and C of a convolved row lie: x padded to 4, then B and C of every group padded to KP, all padding zeros.
 __host__ __device__ inline int conv_x(const SsmShape& m) { return (m.heads * m.vdim + 3) & ~3; }
-static int padded_keys(int n) { return 16 * keys_per_lane(n); }
 int64_t ssm_conv_row(const SsmShape& m) { return conv_x(m) + 2 * (int64_t)m.groups * padded_keys(m.state); }
 // per 16 tokens and head: what the tokens take from each other [16 from][16 to], the state's decay up to each, each one's share of the new state
 constexpr int SSM_TILE = 288;
@@ -517,40 +404,47 @@ __global__ __launch_bounds__(256) void ssm_tiles_kernel(const SsmRows a, int eac
     }
 }
 
-constexpr int ssm_tile_lds(int keys) { return 128 * keys + 4096 + 1024; }
-constexpr int ssm_stages(int keys) { return keys <= 128 ? 4 : keys <= 256 ? 3 : 2; }
-static int ssm_scan_lds(int waves, int keys) { return 2048 * waves + ssm_stages(keys) * ssm_tile_lds(keys); }
+constexpr int scan_tile_lds(int keys) { return 128 * keys + 4096 + 1024; }
+constexpr int scan_stages(int keys) { return keys <= 128 ? 4 : keys <= 256 ? 3 : 2; }
+static int scan_lds(int waves, int keys) { return 2048 * waves + scan_stages(keys) * scan_tile_lds(keys); }
 
-// The state goes from 16 tokens to the next 16: y_t = P_t (C_t S) + sum(s <= t) M[s][t] x_s,  S <- P_15 S + sum(s) B_s Q_s x_s, on
-// v_mfma_f32_16x16x4_f32.  grid (heads, ceil(vdim / 16)), W waves: a wave has 16 columns and KT tiles of 16 keys of the state, as sums (row r of tile q is
-// key KT r + q of the wave's), which are, register by register, also the operand of C S.  The waves' sums meet in LDS.
+// What a scan over the tokens reads and leaves for one head and 16 columns from c0 on.
+struct Scan {
+    int M, tiles, columns, c0;
+    bool from_zero;
+    const float* bc;            // SSM: rows of B and C, `bc_step` bytes a token, at bytes b_at and c_at.  WKV: the tiles
+    uint32_t bc_step, b_at, c_at;
+    const float* pairs;         // SSM: M, P and Q of each tile.  WKV: M and the keys' decays, behind the rows of the tiles
+    uint32_t tile_bytes;        // from one tile's to the next's
+    const float* x;
+    uint32_t x_step, x_at;
+    float* state;               // of the head's first column
+    float* y;                   // of the head's first column
+    int64_t y_ld;
+};
+constexpr int wkv_tile(int keys) { return 33 * keys + 256; }  // floats: [16][k | r] with the decays to the tile's edges, M, the decays of the whole tile
+
+// The state goes from 16 tokens to the next 16 on v_mfma_f32_16x16x4_f32:
+//   ssm  y_t = P_t (C_t S) + sum(s <= t) M[s][t] x_s,  S <- P_15 S + sum(s) B_s Q_s x_s
+//   wkv  the same with the decays inside r and k (C and B) and per key in front of S, and the bonus on M's diagonal
+// A wave has 16 columns and KT tiles of 16 keys of the state, as sums (row r of tile q is key KT r + q of the wave's), which are, register by
+// register, also the operand of C S.  The waves' sums meet in LDS.
 // A tile of tokens comes through LDS, STAGES of them in flight, with full instructions (B and C: 16-byte pieces, piece ^ row).
 // What bounds it: a turn (0.65 us) has 544 clocks of MFMAs on a SIMD and as many of LDS traffic on the CU, behind a barrier for the waves' sums; 40 heads are
-// 160 workgroups.  2048 tokens of 40 heads of 64, 128 keys: 89 us, 11 for the tiles in front; token by token on the vector units 217.  Four waves of
+// 160 workgroups.  SSM, 2048 tokens of 40 heads of 64, 128 keys: 89 us, 11 for the tiles in front; token by token on the vector units 217.  Four waves of
 // twice the keys 98, operands from memory straight to registers 104 (without loads 63, without the barrier 75).
-template <int W, int KT>
-__global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
-    constexpr int KP = 16 * W * KT, ROW = KP / 2, STAGES = ssm_stages(KP), TILE = ssm_tile_lds(KP), BC = 128 * KP;  // ROW: pieces of a row's B and C
+// WKV, 2048 tokens of 40 heads of 64: 64 us, 31 for the tiles in front; token by token, with a slab of sums per 16 keys, 157 and 9 more to add the slabs.
+template <int W, int KT, bool WKV>
+__device__ __forceinline__ void scan_columns(const Scan& a, uint8_t* ss_lds) {
+    constexpr int KP = 16 * W * KT, ROW = KP / 2, STAGES = scan_stages(KP), TILE = scan_tile_lds(KP), BC = 128 * KP;  // ROW: pieces of a row's B and C
     constexpr int BCI = 2 * KT, PER = W == 8 ? BCI + 1 : BCI + 2;  // a wave's instructions for B and C of a tile, for all of it
-    extern __shared__ __align__(16) uint8_t ss_lds[];              // s_y, then the tiles: B and C, M with P and Q, x
+    constexpr int PIECES = WKV ? 16 + KP / 16 : 18;               // a wave's share of M and what lies behind it
+    // LDS: s_y, then the tiles: B and C, M and what lies behind it, x
     float (*s_y)[W][256] = reinterpret_cast<float (*)[W][256]>(ss_lds);
     constexpr int TILES = 2 * W * 1024;
-    const SsmShape& m = a.m;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = wave & 3, j = lane & 15, g4 = lane >> 4, h = blockIdx.x, N = m.state;
-    const int per = m.heads / m.groups, g = h / per, inner = m.heads * m.vdim, channels = inner + 2 * m.groups * N;
-    const int c0 = blockIdx.y * 16, c = min(c0 + j, m.vdim - 1), tiles = (a.M + 15) / 16;
-    // the ring takes the inputs of the last positions
-    for (int q = 0; q < m.taps && q < a.M; ++q) {
-        const float* row = a.proj + (int64_t)(a.M - 1 - q) * a.ld + inner;
-        float* slot = a.ring + (a.pos0 + a.M - 1 - q) % m.taps * channels;
-        if (tid < 16 && c0 + tid < m.vdim) slot[h * m.vdim + c] = row[h * m.vdim + c];
-        if (h % per == 0 && blockIdx.y == 0)
-            for (int i = tid; i < 2 * N; i += 64 * W) {
-                const int ch = inner + (i < N ? 0 : m.groups * N) + g * N + i % N;
-                slot[ch] = row[ch];
-            }
-    }
-    float* state = a.state + ((int64_t)h * m.vdim + c) * KP + 16 * KT * wave + 4 * KT * g4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = wave & 3, j = lane & 15, g4 = lane >> 4;
+    const int c0 = a.c0, c = min(c0 + j, a.columns - 1), tiles = a.tiles;
+    float* state = a.state + (int64_t)c * KP + 16 * KT * wave + 4 * KT * g4;
     rc_f4 S[KT];
     {
         float keys[4 * KT];
@@ -558,33 +452,38 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
 #pragma unroll
         for (int q = 0; q < KT; ++q)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[q][i] = a.pos0 > 0 ? keys[KT * i + q] : 0.0f;
+            for (int i = 0; i < 4; ++i) S[q][i] = a.from_zero ? 0.0f : keys[KT * i + q];
     }
     // memory -> LDS; rows past the last repeat it and count nothing, columns of x past the last are what lies there and are not stored
-    const uint32_t step = (uint32_t)a.conv_ld * 4, last = (uint32_t)(a.M - 1) * step;
-    const gt_i4 rows = gt_buffer(a.conv), pairs = gt_buffer(a.tiles + (int64_t)h * tiles * SSM_TILE);
+    const uint32_t last = (uint32_t)(a.M - 1) * a.bc_step, x_last = (uint32_t)(a.M - 1) * a.x_step;
+    const gt_i4 rows = gt_buffer(a.bc), pairs = gt_buffer(a.pairs), xs = gt_buffer(a.x);
     const uint32_t lds0 = (uint32_t)(uintptr_t)ss_lds + TILES;
     uint32_t row_of[BCI], col_of[BCI];
 #pragma unroll
     for (int i = 0; i < BCI; ++i) {
         const int p = (BCI * wave + i) * 64 + lane, q = (p % ROW) ^ (p / ROW & 15);
-        row_of[i] = p / ROW * step;
-        col_of[i] = 4 * (conv_x(m) + (q < ROW / 2 ? g * KP : (m.groups + g) * KP) + 4 * (q % (ROW / 2)));
+        row_of[i] = p / ROW * (WKV ? 16 * ROW : a.bc_step);
+        col_of[i] = WKV ? 16 * q : (q < ROW / 2 ? a.b_at : a.c_at) + 16 * (q % (ROW / 2));
     }
-    const uint32_t x_row = (4 * g4 + w4) * step, x_col = 4 * (h * m.vdim + c0 + j), pair_at = 16 * (18 * w4 + min(lane, 17));
+    const uint32_t x_row = (4 * g4 + w4) * a.x_step, x_col = a.x_at + 4 * (c0 + j), pair_at = 16 * (PIECES * w4 + min(lane, PIECES - 1));
     auto fetch = [&](int n, int i) {
-        const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + n % STAGES * TILE), t0 = 16 * n * step;
-        if (i < BCI) gt_to_lds(at + (BCI * wave + i) * 1024, (int)(min(t0 + row_of[i], last) + col_of[i]), rows, 0);
-        else if (W == 8 ? wave < 4 : i == BCI) gt_to_lds(at + BC + w4 * 1024, (int)pair_at, pairs, n * SSM_TILE * 4);
-        else gt_word_to_lds(at + BC + 4096 + w4 * 256, (int)(min(t0 + x_row, last) + x_col), rows, 0);
+        const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + n % STAGES * TILE);
+        if (i < BCI) {
+            if constexpr (WKV) gt_to_lds(at + (BCI * wave + i) * 1024, (int)(row_of[i] + col_of[i]), rows, n * a.tile_bytes);
+            else gt_to_lds(at + (BCI * wave + i) * 1024, (int)(min(16 * n * a.bc_step + row_of[i], last) + col_of[i]), rows, 0);
+        } else if (W == 8 ? wave < 4 : i == BCI) gt_to_lds(at + BC + w4 * 1024, (int)pair_at, pairs, n * a.tile_bytes);
+        else gt_word_to_lds(at + BC + 4096 + w4 * 256, (int)(min(16 * n * a.x_step + x_row, x_last) + x_col), xs, 0);
     };
     // LDS -> registers
     struct Tile {
         rc_f4 P, Q;
-        float C[4 * KT], B[4][KT], x[4], xw, from, end;
+        float C[4 * KT], B[4][KT], x[4], xw, from, end, decay[4 * KT];  // P, Q and end: SSM; decay: WKV
     } T0, T1;
-    auto pair = [&](int f) { return BC + f / 72 * 1024 + f % 72 * 4; };  // where float f of M, P, Q lies in a tile
+    auto pair = [&](int f) { return BC + f / (4 * PIECES) * 1024 + f % (4 * PIECES) * 4; };  // where float f of M and what lies behind it is in a tile
     const int from_at = pair(16 * (4 * g4 + w4) + j), p_at = pair(256 + 4 * g4), q_at = pair(272 + 4 * g4), end_at = pair(271);
+    int decay_at[KT];
+#pragma unroll
+    for (int q = 0; q < KT; ++q) decay_at[q] = pair(256 + 16 * KT * wave + 4 * KT * g4 + 4 * q);
     const int x_at = BC + 4096 + 64 * g4 + 4 * j;                        // of row 4 g4: row 4 g4 + i 256 i further on
     constexpr int READS = KT + 6;
     auto read = [&](Tile& v, int n, int part) {
@@ -608,7 +507,13 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
         } else if (part == KT + 4) {
             v.xw = *reinterpret_cast<const float*>(t + x_at + 256 * w4);
             v.from = *reinterpret_cast<const float*>(t + from_at);
-            v.end = *reinterpret_cast<const float*>(t + end_at);
+            if constexpr (!WKV) v.end = *reinterpret_cast<const float*>(t + end_at);
+        } else if constexpr (WKV) {
+#pragma unroll
+            for (int q = 0; q < KT; ++q) {
+                const float4 x = *reinterpret_cast<const float4*>(t + decay_at[q]);
+                v.decay[4 * q] = x.x; v.decay[4 * q + 1] = x.y; v.decay[4 * q + 2] = x.z; v.decay[4 * q + 3] = x.w;
+            }
         } else {
             v.P = *reinterpret_cast<const rc_f4*>(t + p_at);
             v.Q = *reinterpret_cast<const rc_f4*>(t + q_at);
@@ -621,13 +526,13 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
 #pragma unroll
             for (int w = 0; w < W; ++w) sums[w] = s_y[n & 1][w][tid & 255];
     };
-    const bool stored = tid < 256 && c0 + j < m.vdim;
-    float* y = a.y + (int64_t)(tid >> 4 & 15) * inner + h * m.vdim + c0 + j;
+    const bool stored = tid < 256 && c0 + j < a.columns;
+    float* y = a.y + (int64_t)(tid >> 4 & 15) * a.y_ld + c0 + j;
     auto put = [&](int n) {
         if (!stored || 16 * n + (tid >> 4) >= a.M) return;
         float v = (sums[0] + sums[1]) + (sums[2] + sums[3]);
         if constexpr (W == 8) v += (sums[4] + sums[5]) + (sums[6] + sums[7]);
-        y[(int64_t)16 * n * inner] = v;
+        y[(int64_t)16 * n * a.y_ld] = v;
     };
     auto run = [&](const Tile& v, Tile& next, int n) {
         // the next tile has arrived in every wave's part; the one used now lies in registers, and its LDS takes one more
@@ -636,11 +541,14 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
         rc_f4 old[KT], here = {0.f, 0.f, 0.f, 0.f}, next_S[KT];
         float dx[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dx[i] = v.x[i] * v.Q[i];
+        for (int i = 0; i < 4; ++i) dx[i] = WKV ? v.x[i] : v.x[i] * v.Q[i];
 #pragma unroll
         for (int q = 0; q < KT; ++q) {
             old[q] = rc_f4{0.f, 0.f, 0.f, 0.f};
-            next_S[q] = S[q] * v.end;
+            if constexpr (WKV) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) next_S[q][i] = S[q][i] * v.decay[KT * i + q];
+            } else next_S[q] = S[q] * v.end;
         }
         // sums that do not depend on each other take turns, and what is read and requested for later tiles goes out between them
         constexpr int OPS = 1 + READS + PER, SLOTS = 4 * KT;
@@ -672,7 +580,7 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
         for (int q = 1; q < KT; ++q) old[0] += old[q];
         if (__builtin_expect(wave < 4 && __builtin_amdgcn_ballot_w64(!(fabsf(v.xw) < INFINITY)) != 0, 0)) {  // 0 times infinity: no token takes from a later one
             here = rc_f4{0.f, 0.f, 0.f, 0.f};
-            const float* t = a.tiles + ((int64_t)h * tiles + n) * SSM_TILE;
+            const float* t = a.pairs + (int64_t)n * (a.tile_bytes / 4);
             for (int b = 0; b < 4; ++b) {
                 const float xs = __shfl(v.xw, 16 * b + j, 64);
                 const int from = 4 * b + wave;
@@ -682,7 +590,7 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s_y[n & 1][wave][16 * (4 * g4 + i) + j] = fmaf(v.P[i], old[0][i], here[i]);
+        for (int i = 0; i < 4; ++i) s_y[n & 1][wave][16 * (4 * g4 + i) + j] = WKV ? old[0][i] + here[i] : fmaf(v.P[i], old[0][i], here[i]);
     };
 #pragma unroll
     for (int n = 0; n < STAGES; ++n)
@@ -700,7 +608,7 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
     __syncthreads();
     read_sums(tiles - 1);
     put(tiles - 1);
-    if (c0 + j < m.vdim) {
+    if (c0 + j < a.columns) {
         float keys[4 * KT];
 #pragma unroll
         for (int q = 0; q < KT; ++q)
@@ -708,6 +616,139 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
             for (int i = 0; i < 4; ++i) keys[KT * i + q] = S[q][i];
         store_keys<4 * KT>(state, keys);
     }
+}
+
+
+// grid (heads, ceil(vdim / 16)), W waves
+template <int W, int KT>
+__global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
+    extern __shared__ __align__(16) uint8_t scan_mem[];
+    const SsmShape& m = a.m;
+    const int tid = threadIdx.x, h = blockIdx.x, N = m.state, per = m.heads / m.groups, g = h / per, inner = m.heads * m.vdim, channels = inner + 2 * m.groups * N;
+    const int c0 = blockIdx.y * 16;
+    // the ring takes the inputs of the last positions
+    for (int q = 0; q < m.taps && q < a.M; ++q) {
+        const float* row = a.proj + (int64_t)(a.M - 1 - q) * a.ld + inner;
+        float* slot = a.ring + (a.pos0 + a.M - 1 - q) % m.taps * channels;
+        if (tid < 16 && c0 + tid < m.vdim) slot[h * m.vdim + c0 + tid] = row[h * m.vdim + c0 + tid];
+        if (h % per == 0 && blockIdx.y == 0)
+            for (int i = tid; i < 2 * N; i += 64 * W) {
+                const int ch = inner + (i < N ? 0 : m.groups * N) + g * N + i % N;
+                slot[ch] = row[ch];
+            }
+    }
+    Scan s;
+    s.M = a.M;
+    s.tiles = (a.M + 15) / 16;
+    s.columns = m.vdim;
+    s.c0 = c0;
+    s.from_zero = a.pos0 == 0;
+    s.bc = s.x = a.conv;
+    s.bc_step = s.x_step = (uint32_t)a.conv_ld * 4;
+    s.b_at = 4 * (conv_x(m) + g * a.keys);
+    s.c_at = 4 * (conv_x(m) + (m.groups + g) * a.keys);
+    s.pairs = a.tiles + (int64_t)h * s.tiles * SSM_TILE;
+    s.tile_bytes = SSM_TILE * 4;
+    s.x_at = 4 * h * m.vdim;
+    s.state = a.state + (int64_t)h * m.vdim * a.keys;
+    s.y = a.y + h * m.vdim;
+    s.y_ld = inner;
+    scan_columns<W, KT, false>(s, scan_mem);
+}
+
+// What 16 tokens of a head take from each other, and their r and k with the decays to the edges of the tile.  M[s][t] = sum over keys of
+// r_t k_s prod(s < q < t) w_q, the bonus r_t u k_s on its diagonal.  A pair of tokens meets at one size B of 1, 2, 4 and 8: the highest bit in which
+// their places differ.  There the product is that of the decays behind s in its block of B times those in front of t in the next: products of
+// decays, never quotients, and one matrix product a size.  It moves memory (2048 rows of 40 heads of 64: 63 MB in, 47 out, 31 us).
+// grid (ceil(rows / 16), heads), four waves that share the keys; tokens past the last leave everything as it is.
+__global__ __launch_bounds__(256) void wkv_tiles_kernel(const WkvRows a) {
+    __shared__ float s_m[4][256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 15, g4 = lane >> 4, t0 = blockIdx.x * 16, h = blockIdx.y, d = a.dim, kp = a.keys;
+    const bool here = t0 + j < a.M, fours = !((d | a.ld | a.section) & 3) && !(reinterpret_cast<uintptr_t>(a.u) & 15);
+    const float *p = a.proj + (int64_t)min(t0 + j, a.M - 1) * a.ld + h * d, *u = a.u + h * d;
+    float* out = a.tiles + ((int64_t)h * gridDim.x + blockIdx.x) * wkv_tile(kp);
+    float m[4] = {0.f, 0.f, 0.f, 0.f};  // from 4 g4 + i to j
+    for (int k0 = 16 * wave; k0 < kp; k0 += 64) {
+        const int key = k0 + 4 * g4;
+        rc_f4 r, k, w, b;
+        if (fours) {
+            const int at = min(key, d - 4);
+            r = *reinterpret_cast<const rc_f4*>(p + at);
+            k = *reinterpret_cast<const rc_f4*>(p + a.section + at);
+            w = *reinterpret_cast<const rc_f4*>(p + 4 * a.section + at);
+            b = *reinterpret_cast<const rc_f4*>(u + at);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int at = min(key + i, d - 1);
+                r[i] = p[at];
+                k[i] = p[a.section + at];
+                w[i] = p[4 * a.section + at];
+                b[i] = u[at];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool in = here && key + i < d;
+            r[i] = in ? r[i] : 0.0f;
+            k[i] = in ? k[i] : 0.0f;
+            w[i] = in ? w[i] : 1.0f;
+            b[i] = key + i < d ? b[i] : 0.0f;
+        }
+        rc_f4 dot = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dot = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i] * b[i], r[i], dot, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] += 4 * g4 + i == j ? dot[i] : 0.0f;
+        static_for<4>([&](auto L) {  // r and k: with the decays in front of and behind the token in its block of B, w: those of the whole block
+            constexpr int B = 1 << decltype(L)::value, other = B == 1 ? 0xB1 : B == 2 ? 0x4E : B == 4 ? 0x141 : 0x140;
+            rc_f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], r[i], sum, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int from = 4 * g4 + i;
+                m[i] += ((from ^ j) & ~(2 * B - 1)) == 0 && !(from & B) && (j & B) ? sum[i] : 0.0f;
+                const float next = dpp_f<other>(w[i]);
+                r[i] *= j & B ? next : 1.0f;
+                k[i] *= j & B ? 1.0f : next;
+                w[i] *= next;
+            }
+        });
+        *reinterpret_cast<rc_f4*>(out + j * 2 * kp + key) = k;
+        *reinterpret_cast<rc_f4*>(out + j * 2 * kp + kp + key) = r;
+        if (j == 0) *reinterpret_cast<rc_f4*>(out + 32 * kp + 256 + key) = w;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_m[wave][16 * (4 * g4 + i) + j] = m[i];
+    __syncthreads();
+    out[32 * kp + tid] = (s_m[0][tid] + s_m[1][tid]) + (s_m[2][tid] + s_m[3][tid]);
+}
+
+// grid (heads, ceil(dim / 16)), W waves
+template <int W, int KT>
+__global__ __launch_bounds__(64 * W, 1) void wkv_scan_kernel(const WkvRows a) {
+    extern __shared__ __align__(16) uint8_t scan_mem[];
+    const int h = blockIdx.x;
+    if (h == 0 && blockIdx.y == 0)  // the next token's shift reads the last row
+        for (int i = threadIdx.x; i < a.wp; i += 64 * W) a.shift[(a.pos0 + a.M - 1) % 2 * a.wp + i] = a.h_last[i];
+    Scan s;
+    s.M = a.M;
+    s.tiles = (a.M + 15) / 16;
+    s.columns = a.dim;
+    s.c0 = blockIdx.y * 16;
+    s.from_zero = a.pos0 == 0;
+    s.tile_bytes = wkv_tile(a.keys) * 4;
+    s.bc = a.tiles + (int64_t)h * s.tiles * wkv_tile(a.keys);
+    s.bc_step = s.b_at = s.c_at = 0;
+    s.pairs = s.bc + 32 * a.keys;
+    s.x = a.proj;
+    s.x_step = (uint32_t)a.ld * 4;
+    s.x_at = (uint32_t)(2 * a.section + h * a.dim) * 4;
+    s.state = a.state + (int64_t)h * a.dim * a.keys;
+    s.y = a.o + h * a.dim;
+    s.y_ld = a.o_ld;
+    scan_columns<W, KT, true>(s, scan_mem);
 }
 
 // grid rows: the scan's y * silu(z), normed in equal parts, times norm and the branch's scale.  All that a row reads goes out together (2560 values, each
@@ -792,22 +833,42 @@ int tanh_rows(const float* g, int slabs, int64_t slab, int rows, int n, bool fp3
     return launch_status();
 }
 
-int64_t scan_slabs(int keys) { return key_groups(keys); }
+int64_t wkv_tile_floats(int heads, int dim, int rows) { return (int64_t)((rows + 15) / 16) * heads * wkv_tile(padded_keys(dim)); }
 
 int wkv_rows(WkvRows a, bool fp32, hipStream_t s) {
     if (!recurrent_supported(a.dim)) return PTM_E_UNSUPPORTED;
-    a.groups = key_groups(a.dim);
-    const dim3 grid(a.heads, a.groups * ((a.dim + 63) / 64));
-#define PTM_RUN(KPL) hipLaunchKernelGGL(wkv_scan_kernel<KPL>, grid, dim3(256), 0, s, a)
-    PTM_KPL(a.dim, PTM_RUN)
+    a.keys = padded_keys(a.dim);
+    hipLaunchKernelGGL(wkv_tiles_kernel, dim3((a.M + 15) / 16, a.heads), dim3(256), 0, s, a);
+    static std::once_flag raised;
+    std::call_once(raised, [] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&wkv_scan_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 128));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&wkv_scan_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 256));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&wkv_scan_kernel<8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 512));
+    });
+    const dim3 grid(a.heads, (a.dim + 15) / 16);
+#define PTM_RUN(W, KT) hipLaunchKernelGGL((wkv_scan_kernel<W, KT>), grid, dim3(64 * W), scan_lds(W, a.keys), s, a)
+    switch (a.keys) {
+        case 64: PTM_RUN(4, 1); break;
+        case 128: PTM_RUN(8, 1); break;
+        case 256: PTM_RUN(8, 2); break;
+        default: PTM_RUN(8, 4);
+    }
 #undef PTM_RUN
+    const bool fours = !((a.dim | a.ld | a.section | a.o_ld | a.out_ld) & 3) &&
+                       !((reinterpret_cast<uintptr_t>(a.o) | reinterpret_cast<uintptr_t>(a.proj) | reinterpret_cast<uintptr_t>(a.norm) | reinterpret_cast<uintptr_t>(a.out)) & 15);
     const dim3 out_grid(a.M, (a.heads + 3) / 4);
+#define PTM_FOURS(G)                                                                                                                                         \
+    if (fp32) hipLaunchKernelGGL((wkv_out_fours_kernel<true, G>), dim3((unsigned)(((int64_t)a.M * a.heads * G + 255) / 256)), dim3(256), 0, s, a);           \
+    else hipLaunchKernelGGL((wkv_out_fours_kernel<false, G>), dim3((unsigned)(((int64_t)a.M * a.heads * G + 255) / 256)), dim3(256), 0, s, a)
 #define PTM_RUN(NV)                                                                                                  \
     if (fp32) hipLaunchKernelGGL((wkv_out_rows_kernel<true, NV>), out_grid, dim3(256), 0, s, a);                     \
     else hipLaunchKernelGGL((wkv_out_rows_kernel<false, NV>), out_grid, dim3(256), 0, s, a)
-    if (a.dim <= 64) { PTM_RUN(1); }
+    if (fours && a.dim <= 64) { PTM_FOURS(16); }
+    else if (fours && a.dim <= 128) { PTM_FOURS(32); }
+    else if (a.dim <= 64) { PTM_RUN(1); }
     else if (a.dim <= 128) { PTM_RUN(2); }
     else { PTM_RUN(8); }
+#undef PTM_FOURS
 #undef PTM_RUN
     return launch_status();
 }
@@ -823,11 +884,11 @@ int ssm_rows(SsmRows a, bool fp32, hipStream_t s) {
     const dim3 grid(m.heads, (m.vdim + 15) / 16);
     static std::once_flag raised;
     std::call_once(raised, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 128));
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 256));
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, ssm_scan_lds(8, 512));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 128));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 256));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<8, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds(8, 512));
     });
-#define PTM_RUN(W, KT) hipLaunchKernelGGL((ssm_scan_kernel<W, KT>), grid, dim3(64 * W), ssm_scan_lds(W, a.keys), s, a)
+#define PTM_RUN(W, KT) hipLaunchKernelGGL((ssm_scan_kernel<W, KT>), grid, dim3(64 * W), scan_lds(W, a.keys), s, a)
     switch (a.keys) {
         case 64: PTM_RUN(4, 1); break;
         case 128: PTM_RUN(8, 1); break;

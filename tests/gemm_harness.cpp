@@ -166,6 +166,32 @@ int ssm_run(const int* shape, const float* const* w, const float* proj, int M, i
     r.out_ld = inner;
     return ptm::ssm_rows(r, true, static_cast<hipStream_t>(stream));
 }
+// prompt rows of a WKV mixer, fp32: proj rows of r, k, v, g and decays
+int64_t wkv_scratch(int heads, int dim, int M, int what) { return what == 0 ? ptm::wkv_tile_floats(heads, dim, M) : (int64_t)heads * dim * M; }
+int wkv_run(int heads, int dim, const float* proj, const float* u, const float* norm, int M, int64_t pos0, float* state, float* const* scratch, const float* h_last, float* shift,
+            float* out, void* stream) {
+    ptm::WkvRows w{};
+    w.proj = proj;
+    w.section = (int64_t)heads * dim;
+    w.ld = 5 * w.section;
+    w.M = M;
+    w.heads = heads;
+    w.dim = dim;
+    w.u = u;
+    w.norm = norm;
+    w.eps = 1e-6f;
+    w.pos0 = pos0;
+    w.state = state;
+    w.tiles = scratch[0];
+    w.o = scratch[1];
+    w.o_ld = w.section;
+    w.out = out;
+    w.out_ld = w.section;
+    w.h_last = h_last;
+    w.shift = shift;
+    w.wp = 64;
+    return ptm::wkv_rows(w, true, static_cast<hipStream_t>(stream));
+}
 int64_t ssm_state_floats(int heads, int state, int vdim) { return ptm::recurrent_state_floats(heads, state, vdim); }
 
 }  // extern "C"

@@ -483,3 +483,50 @@ def test_state_space_scan(dev, heads, vdim, state, groups, taps, rows, pos0):
         loud = proj.clone()
         loud[9, inner] = float("inf")
         assert torch.equal(run(loud)[0][:9], out[:9])
+
+
+# every number of key tiles a wave has, dims off 4 and off the tiles, tokens off 16, one head and many; decays next to 1, next to 0 and 0
+@pytest.mark.parametrize("heads,dim,rows", [(2, 64, 16), (3, 5, 15), (1, 1, 2), (4, 62, 97), (3, 100, 130), (40, 64, 33), (2, 200, 49), (1, 300, 70), (1, 512, 17), (2, 128, 1)])
+@pytest.mark.parametrize("pos0", [0, 21])
+def test_wkv_scan(dev, heads, dim, rows, pos0):
+    """One call against the recurrence in 64 bits.  A sum of up to 512 products, 16 decays deep, is off by some 1e-6 of its terms; a value that is
+    infinite reaches no token before its own."""
+    import torch
+    from gemm_helpers import harness
+    h = harness()
+    for f in ("wkv_scratch", "ssm_state_floats"):
+        getattr(h, f).restype = C.c_int64
+    gen = torch.Generator(device="cuda").manual_seed(rows + dim)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    proj = rand(rows, 5, heads, dim)
+    proj[:, 4] = torch.exp(-torch.exp(3 * rand(rows, heads, dim)))
+    proj[rows // 2, 4, 0] = 0.0
+    u, norm, last = rand(heads, dim), 1 + 0.1 * rand(heads, dim), rand(64)
+    kp = h.ssm_state_floats(1, dim, 1)
+    S0 = torch.zeros(heads, dim, kp, device="cuda")
+    S0[:, :, :dim] = rand(heads, dim, dim)
+
+    def run(proj):
+        S, out, shift = S0.clone(), torch.empty(rows, heads, dim, device="cuda"), torch.zeros(2, 64, device="cuda")
+        scratch = [torch.full((h.wkv_scratch(heads, dim, rows, i),), float("nan"), device="cuda") for i in range(2)]
+        p = lambda t: C.c_void_p(t.data_ptr())
+        assert h.wkv_run(heads, dim, p(proj), p(u), p(norm), rows, C.c_int64(pos0), p(S), (C.c_void_p * 2)(*[t.data_ptr() for t in scratch]), p(last), p(shift), p(out), None) == 0
+        torch.cuda.synchronize()
+        return out, S, shift
+
+    out, S, shift = run(proj)
+    r, k, v, g, w = proj.double().unbind(1)
+    want, want_S = [], (S0[:, :, :dim] if pos0 else 0 * S0[:, :, :dim]).double()  # [head][column][key]
+    for t in range(rows):
+        kv = v[t, :, :, None] * k[t, :, None, :]
+        o = ((want_S + u.double()[:, None, :] * kv) * r[t, :, None, :]).sum(2)
+        want_S = w[t, :, None, :] * want_S + kv
+        want.append(o / (o.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * norm.double() * torch.nn.functional.silu(g[t]))
+    for a, b in ((out, torch.stack(want)), (S[:, :, :dim], want_S)):
+        assert float((a.double() - b).abs().max() / b.pow(2).mean().sqrt()) < 3e-5
+    assert (S[:, :, dim:] == 0).all() and torch.equal(shift[(pos0 + rows - 1) % 2], last)
+    if rows > 9:
+        for part in (0, 1, 2):
+            loud = proj.clone()
+            loud[9, part, 0, 0] = float("inf")
+            assert torch.equal(run(loud)[0][:9], out[:9])
