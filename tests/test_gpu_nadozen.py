@@ -389,6 +389,45 @@ def test_attention_rows_sink_and_gate(dev, case, fp32):
     assert err.max() < (2e-5 if fp32 else 2.5e-2), err.max()
 
 
+# workgroups of one round of the chip, of two with long row blocks beside short ones (257 .. 512), of more; heads off 8 and off the size classes; a scale
+# that is negative or zero, capped scores, scores that move the softmax's reference by more and by less than 2^8, gates off 16 bytes
+@pytest.mark.parametrize("rows,heads,kv_heads,dim,scale,cap,loud,shift", [
+    (130, 4, 2, 64, -1.0, 0.0, 1, 0), (40, 2, 1, 40, 0.0, 0.0, 1, 0), (40, 2, 2, 128, 0.0, 5.0, 1, 1), (150, 3, 1, 104, 1.0, 9.0, 1, 2), (150, 3, 1, 104, -1.0, 9.0, 4, 0),
+    (257, 2, 1, 128, 1.0, 0.0, 8, 0), (257, 2, 1, 200, 1.0, 0.0, 24, 1), (255, 64, 4, 16, 1.0, 0.0, 3, 0), (257, 128, 4, 32, 1.0, 0.0, 3, 1), (512, 128, 4, 16, 1.0, 20.0, 3, 0),
+    (516, 128, 4, 16, -1.0, 0.0, 1, 3)])
+def test_prompt_attention_forms(dev, rows, heads, kv_heads, dim, scale, cap, loud, shift):
+    """Against 64 bits.  Values and gates are at most some 5 * 0.7; what is stored is off by 2^-9 of that, the weights by 2^-16."""
+    import torch
+    pos0, window = 11, 200
+    rng = np.random.default_rng(rows + heads + dim)
+    n = pos0 + rows
+    rnd = lambda *s: fw.from_bf16(fw.to_bf16(rng.standard_normal(s, np.float32)))
+    q, k, v = rnd(rows, heads, dim), rnd(n, kv_heads, dim), rnd(n, kv_heads, dim)
+    k = fw.from_bf16(fw.to_bf16(k * np.where(np.arange(n) % 64 == 37, loud, 1).astype(np.float32)[:, None, None]))
+    gate = rng.standard_normal(rows * heads * (dim - shift) + 4).astype(np.float32)
+    sink = rng.standard_normal(heads).astype(np.float32)
+    scale, see = scale * 2.0 / np.sqrt(dim), N.visible(n, {"size": window})[pos0:]
+    want = np.zeros((rows, heads, dim))
+    for h in range(heads):
+        g = h // (heads // kv_heads)
+        s = q[:, h].astype(np.float64) @ k[:, g].T.astype(np.float64) * scale
+        s = np.where(see, cap * np.tanh(s / cap) if cap else s, -np.inf)
+        want[:, h] = N.sink_softmax(s, float(sink[h])) @ v[:, g] * 0.7
+    gates = gate[shift:shift + rows * heads * (dim - shift)].reshape(rows, heads, dim - shift)
+    want[:, :, :dim - shift] *= N.sigmoid(gates.astype(np.float64))
+    put = lambda a: torch.from_numpy(fw.to_bf16(a).view(np.int16)).cuda()
+    Q, K, V = put(q), put(k), put(v)
+    O = torch.zeros((rows, heads, dim), dtype=torch.bfloat16, device="cuda")
+    S, Gt = torch.from_numpy(sink).cuda(), torch.from_numpy(gate).cuda()
+    a = _lib.AttentionArgs(Q=Q.data_ptr(), K1=K.data_ptr(), V=V.data_ptr(), O=O.data_ptr(), q_row=heads * dim, k1_row=kv_heads * dim, k1_head=dim, v_row=kv_heads * dim,
+                           v_head=dim, o_row=heads * dim, rows=rows, heads=heads, kv_heads=kv_heads, dim1=dim, vdim=dim, window=window, pos0=pos0, scale=scale, softcap=cap,
+                           fp32=0, sink=S.data_ptr(), gate=Gt.data_ptr() + 4 * shift, gate_row=heads * (dim - shift), gate_head=dim - shift, out_scale=0.7)
+    _lib.check(_lib.load().ptm_attention_rows(C.byref(a), None), "attention_rows")
+    torch.cuda.synchronize()
+    err = np.abs(O.float().cpu().numpy() - want)
+    assert err.max() < 1e-2, err.max()
+
+
 # ---- products with the gated epilogue are reached through the models; shapes around their tile edges -------------
 @pytest.mark.parametrize("ff", [1, 15, 16, 17, 64, 100, 257])
 def test_feed_forward_sizes(dev, tmp_path, ff):

@@ -52,6 +52,23 @@ def test_prompt_portions_and_decode(dev, built, name, precision):
     m.close()
 
 
+# heads of multiples of 8 values, taken four values at a time: fewer and more than a walk of 4096, rotated in whole, in part, not in fours (one by one)
+@pytest.mark.parametrize("mixer", [attention(40, 2, 128, 128, rot=64, sharp=1.0), attention(2, 1, 8, 8, rot=4), attention(3, 1, 24, 16, rot=20), attention(2, 2, 40, 40, rot=18),
+                                   attention(1, 1, 256, 104, sharp=1.0), latent(24, 128, 64, 512, 64, sharp=1.0), latent(1, 8, 8, 8, 8), latent(3, 24, 16, 40, 8),
+                                   latent(2, 16, 6, 24, 16)], ids=lambda m: "-".join(str(m[k]) for k in ("heads", "dim", "vdim")))
+def test_head_sizes(dev, tmp_path, mixer):
+    cfg = model([layer(mixer)], 64, 90)
+    w = fw.random_weights(cfg, 5)
+    tokens = np.random.default_rng(6).integers(0, 90, 70).tolist()
+    want = T.logits(tokens, w, cfg)
+    path = fw.write_model_folder(str(tmp_path / "m"), cfg, w)
+    for precision in ("float32", "bfloat16"):
+        m = registry.load(path, max_seq=71, precision=precision)
+        for sizes in ([70], [33, 2, 1]):
+            assert_close(portions(m, tokens, sizes), want, precision, (mixer, precision, sizes))
+        m.close()
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_random_designs(dev, tmp_path, seed):
     cfg = random_model(seed)
