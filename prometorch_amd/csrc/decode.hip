@@ -473,8 +473,8 @@ static int prefill_chunk(ptm_decoder* d, const int* tokens_host, int M, int64_t 
         bool act_split = false;  // the down projection's rows have a scale per K split
         {
             // Gate and up share one launch when that fills the chip better: a tile is a workgroup and has a CU to itself, so a launch takes whole
-            // rounds of 256 (qf_tall).  512 rows of 9728: 152 tiles of 128 rows each, apart two rounds; together 152 of 256 rows, 1.75 (85 -> 70 us);
-            // 2048 rows: 2.75 + 2.75 apart and 4.75 together.  Up to 256 rows (the two
+            // rounds of 256 (qf_tall).  512 rows of 9728: 152 tiles of 128 rows each, apart two rounds; together 228 of 192 rows, one of 1.5 (85 -> 64
+            // us); 2048 rows: 2.75 + 2.75 apart and 4.75 together.  Up to 256 rows (the two
             // short row classes) always together: one launch less, and the launch is the cost there.  Beyond, only when both
             // ways use the same K splits, so that the choice changes no result.
             const uint32_t t2[2] = {L.gate.ggml_type, L.up.ggml_type};

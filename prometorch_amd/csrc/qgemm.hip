@@ -999,12 +999,13 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
     qf_store<MT>(acc, s_rs, Y, partials, accumulate, M, N, m0, n_base, j, kh, bz);
 }
 
-// ---- 256 rows x 256 columns ----
+// ---- 256 and 192 rows x 256 columns ----
 // A wave has one strip of 32 columns and all 256 rows (128 accumulators), so each unpacked weight serves twice the products of the 128-row tile, whose
 // time is its matrix and its unpacking instructions one after the other.  A stage is half a super-block: X goes from memory to LDS directly, two stages
 // of 64 KB, and the loop is laid out by hand: behind every MFMA the read of the fragment eight MFMAs on into the registers it has just freed, a
 // piece of the next sub-block's weights behind every fourth, and one barrier a stage, between the last reads of its LDS and the first of the
-// next, with MFMAs on either side.  The same products in the same order as in the 128-row tile: same bits.
+// next, with MFMAs on either side.  The same products in the same order as in the 128-row tile: same bits.  With 192 rows, for launches that would
+// leave CUs idle, everything is three quarters of that but the unpacking.
 // What bounds it: 2048 x 14336 x 4096 in 235 us (265 in 128-row tiles), Q6_K 2048 x 4096 x 14336 238 (326), 1020 TFLOP/s; the matrix cores are busy 66 %
 // of the clocks of a CU at work (41 % before), at which the card lowers its clock (about 1.7 GHz).  Where the barrier lies, when the weights are
 // requested and how the pieces are spread change it by less than 1 %.  The same loop for 128 rows is 1 to 5 % slower than qgemm_f16_body.
@@ -1068,11 +1069,12 @@ struct Q6Half {
 };
 
 
-template <typename Half>
+template <typename Half, int MT>
 __device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale, float* Y,
                                                     int M, int K, int N, int accumulate, int blocks_per_split, float* partials, int bx, int by,
                                                     int bz, uint8_t* s_a, int scale_stride) {
-    constexpr int MT = 8, TM = 32 * MT, STAGE = TM * 256;
+    static_assert(MT == 8 || MT == 6, "row tiles of 32");
+    constexpr int TM = 32 * MT, STAGE = TM * 256, H = MT / 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, kh = lane >> 5;
     const int m0 = by * TM, n_base = bx * 256 + 64 * (wave & 3) + 32 * (wave >> 2);
@@ -1095,10 +1097,10 @@ __device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t st
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mt][r] = 0.0f;
     Half w[2];
-    for (int i = 0; i < 8; ++i) fetch(0, i);
+    for (int i = 0; i < MT; ++i) fetch(0, i);
     w[0].load(wrow, 0, kh);
     issue_order_fence();
-    for (int i = 0; i < 8; ++i) fetch(1, i);
+    for (int i = 0; i < MT; ++i) fetch(1, i);
     if (tid < TM) s_rs[tid] = rowscale[bz * scale_stride + m0 + min(tid, (int)last)];
     h2 sc, of;
     uint32_t bf[2][8];  // [buffer][two fragments of four]
@@ -1125,7 +1127,7 @@ __device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t st
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) read(a0, mt);
 
-    auto stage = [&](int st, auto half_) {  // 8 groups of 8 MFMAs: 16 values of K each
+    auto stage = [&](int st, auto half_) {  // 8 groups of MT MFMAs: 16 values of K each
         constexpr int half = decltype(half_)::value;
         Half& cur = w[half];
         Half& nxt = w[half ^ 1];
@@ -1145,16 +1147,16 @@ __device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t st
                 acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], b, acc[mt], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (g < 7) read(from, mt);
-                else if (mt >= 4) { read(from, 2 * mt - 8); read(from, 2 * mt - 7); }
+                else if (mt >= H) { read(from, 2 * (mt - H)); read(from, 2 * (mt - H) + 1); }
                 // weights of the next sub-block
                 const Half& src = s < 3 ? cur : nxt;
-                const int slot = 8 * ks + mt, sn = (s + 1) & 3;
+                const int slot = MT * ks + mt, sn = (s + 1) & 3;
                 if (slot == 0) src.scale(sn, sc, of);
-                if ((slot & 3) == 2) dequant(src, sn, slot >> 2, bf[(s + 1) & 1]);
+                if (slot % H == H / 2) dequant(src, sn, slot / H, bf[(s + 1) & 1]);
                 // the stage after the next, into the half of LDS this one is read from; the next half block of weights
-                if (g == 7 && mt == 3) gt_arrived<0>();
-                if (g == 7 && mt >= 4 && st + 2 < nst) fetch(st + 2, mt - 4);
-                if (g == 0 && mt < 4 && st > 0 && st + 1 < nst) fetch(st + 1, mt + 4);
+                if (g == 7 && mt == H - 1) gt_arrived<0>();
+                if (g == 7 && mt >= H && st + 2 < nst) fetch(st + 2, mt - H);
+                if (g == 0 && mt < H && st > 0 && st + 1 < nst) fetch(st + 1, mt + H);
                 if (g == 2 && mt == 0) nxt.load(wrow + (int64_t)min((st + 1) >> 1, nblk - 1) * Half::kBlockBytes, half ^ 1, kh);
             }
         }
@@ -1189,9 +1191,11 @@ __device__ __forceinline__ void qf_tile_of(int L, int gx, int gy, int& bx, int& 
 }
 
 // The first `tall` workgroups of a launch take 256 rows each, in that order of pairs of row tiles; the tiles of 128 rows that are left, two from
-// each pair, follow (qf_tall).  False: a row tile past the last.
-__device__ __forceinline__ bool qf_place(int hw, int nwg, int gx, int gy, int tall, int& bx, int& by, int& bz) {
-    if (tall == 0) {
+// each pair, follow (qf_tall).  QF_192: all take 192.  False: a row tile past the last.
+constexpr int QF_192 = -1;
+__device__ __forceinline__ bool qf_place(int hw, int nwg, int gx, int M, int tall, int& bx, int& by, int& bz) {
+    const int gy = tall == QF_192 ? (M + 191) / 192 : (M + QF_TM - 1) / QF_TM;
+    if (tall <= 0) {
         qf_tile_of(qf_xcd_order(hw, nwg), gx, gy, bx, by, bz);
         return true;
     }
@@ -1201,7 +1205,7 @@ __device__ __forceinline__ bool qf_place(int hw, int nwg, int gx, int gy, int ta
     return rest < 0 || by < gy;
 }
 
-// tiles of 128 and 256 rows by 256 columns
+// tiles of 128, 192 and 256 rows by 256 columns
 template <typename Tile>
 __global__ __launch_bounds__(512, 1) void qgemm_f16_rows_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale,
                                                                 float* Y, int M, int K, int N, int accumulate, int blocks_per_split, float* partials,
@@ -1209,9 +1213,11 @@ __global__ __launch_bounds__(512, 1) void qgemm_f16_rows_kernel(const uint8_t* W
     extern __shared__ __align__(16) uint8_t qf_lds[];
     read_now(W, M);
     int bx, by, bz;
-    if (!qf_place(blockIdx.x, gridDim.x, (N + QF_TN - 1) / QF_TN, (M + QF_TM - 1) / QF_TM, tall, bx, by, bz)) return;
-    if ((int)blockIdx.x < tall)
-        qgemm_f16_tall_body<typename Tile::Half>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
+    if (!qf_place(blockIdx.x, gridDim.x, (N + QF_TN - 1) / QF_TN, M, tall, bx, by, bz)) return;
+    if (tall == QF_192)
+        qgemm_f16_tall_body<typename Tile::Half, 6>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
+    else if ((int)blockIdx.x < tall)
+        qgemm_f16_tall_body<typename Tile::Half, 8>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
     else
         qgemm_f16_body<Tile, 4, 8>(W, stride, Xh, rowscale, Y, M, K, N, accumulate, blocks_per_split, partials, bx, by, bz, qf_lds, scale_stride);
 }
@@ -1273,12 +1279,12 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_mu
     else qgemm_f16_body<Q4Tile, MT, WAVES>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0);
 }
 
-// the same in tiles of 128 and 256 rows
+// the same in tiles of 128, 192 and 256 rows
 __global__ __launch_bounds__(512, 1) void qgemm_f16_rows_multi_kernel(const QfMulti a, int M, int K, int slots, int tall) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
     read_now(a.m[0].W, a.m[1].W, a.m[2].W, a.n_mat);
     int sx, by, unused;
-    if (!qf_place(blockIdx.x, gridDim.x, slots, (M + QF_TM - 1) / QF_TM, tall, sx, by, unused)) return;
+    if (!qf_place(blockIdx.x, gridDim.x, slots, M, tall, sx, by, unused)) return;
     int i = 0;
     if (a.n_mat > 1 && sx >= a.m[0].slot_end) i = 1;
     if (a.n_mat > 2 && sx >= a.m[1].slot_end) i = 2;
@@ -1286,9 +1292,12 @@ __global__ __launch_bounds__(512, 1) void qgemm_f16_rows_multi_kernel(const QfMu
     const int local = sx - (i == 0 ? 0 : (i == 1 ? a.m[0].slot_end : a.m[1].slot_end));
     const int bx = local % q.ntiles, bz = local / q.ntiles;
 #define PTM_QR(BODY) BODY(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, by, bz, qf_lds, 0)
-    if ((int)blockIdx.x < tall) {
-        if (q.q6) PTM_QR(qgemm_f16_tall_body<Q6Half>);
-        else PTM_QR(qgemm_f16_tall_body<Q4Half>);
+    if (tall == QF_192) {
+        if (q.q6) PTM_QR((qgemm_f16_tall_body<Q6Half, 6>));
+        else PTM_QR((qgemm_f16_tall_body<Q4Half, 6>));
+    } else if ((int)blockIdx.x < tall) {
+        if (q.q6) PTM_QR((qgemm_f16_tall_body<Q6Half, 8>));
+        else PTM_QR((qgemm_f16_tall_body<Q4Half, 8>));
     } else {
         if (q.q6) PTM_QR((qgemm_f16_body<Q6Tile, 4, 8>));
         else PTM_QR((qgemm_f16_body<Q4Tile, 4, 8>));
@@ -1430,10 +1439,14 @@ static int qgemm_f16_row_tiles(bool q4, int M, int N, int splits) {
 }
 
 // Which tiles of a launch of gx column tiles (slots) and gz K splits have 256 rows: the first `tall` pairs of row tiles in qf_tile_of's order, in whole
-// rounds of the chip or all of them, whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
+// rounds of the chip or all of them - or whether all tiles have 192 - whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
 // times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there.  Measured, all of
 // 128 rows, all of 256, by this rule: 509 x 19456 x 2560 85, 70, 70 us; 953 x 19456 x 2560 132, 150, 125; 2048 x 9728 x 2560 137, 151, 129; 2048 x 28672 x
 // 4096 in 7 rounds, 7, 6.25; 300 x 14336 x 4096 62, 91, 62; Q6_K 2048 x 4096 x 14336 347, 289, 289, 953 x 18944 x 3584 236, 220, 200.
+// A tile of 192 rows takes 1.4 to 1.6 (Q6_K 1.35) of 128-row tiles, by how much of the chip the other tiles leave idle, that is to say how far they let it
+// clock.  The best of the others and 192: 509 x 19456 x 2560 (152 tiles of 256, 228 of 192) 70, 64 us, Q6_K 78, 71; 192 x 65536 x 2560 (512 of 128, 256) 86, 71;
+// 384 x 28672 x 4096 (224 half empty, 224) 117, 93; 953 x 19456 x 2560 (256 + 96, 380) 119, 116; 953 x 28672 x 4096 (256 + 384, 560) 236, 267; 300 x 14336 x
+// 4096 (168 of 128, 112) 56, 71.
 static float qf_tall(int gx, int gz, int M, bool q4, int* tall) {
     const int gy = (M + QF_TM - 1) / QF_TM, pairs = (gy + 1) / 2, plane = gx * pairs, all = plane * gz;
     const float ratio = q4 ? 1.75f : 1.5f;
@@ -1451,11 +1464,13 @@ static float qf_tall(int gx, int gz, int M, bool q4, int* tall) {
         const float cost = ratio * (float)rounds + (float)(rest > 0 ? (rest + 255) / 256 : 0);
         if (cost < best) { best = cost; *tall = t; }
     }
+    const float cost = (q4 ? 1.5f : 1.35f) * (float)((gx * gz * ((M + 191) / 192) + 255) / 256);
+    if (cost < best) { best = cost; *tall = QF_192; }
     return best;
 }
 static int qf_workgroups(int gx, int gz, int M, int tall) {
     const int gy = (M + QF_TM - 1) / QF_TM;
-    return tall ? tall + 2 * (gx * ((gy + 1) / 2) * gz - tall) : gx * gy * gz;
+    return tall == QF_192 ? gx * ((M + 191) / 192) * gz : tall ? tall + 2 * (gx * ((gy + 1) / 2) * gz - tall) : gx * gy * gz;
 }
 
 // rounds of a launch of matrices with `tiles` column tiles and K splits together

@@ -287,9 +287,11 @@ def test_short_prompts_of_several_matrices(dev, po, K, N, types, blocks):
         assert err <= QGEMM_F16_TOL, (i, err)
 
 
-# tiles of 256 rows: all (152 pairs of row tiles), whole rounds and 128-row tiles behind them (K splits off and on), an odd last row tile, ragged N
+# tiles of 256 rows: all (236 pairs of row tiles), whole rounds and 128-row tiles behind them (K splits off and on), an odd last row tile, ragged N; of 192
+# rows: 3 and 2 row tiles, whole and ragged, one of 129 rows
 @pytest.mark.parametrize("qt", [12, 14])
-@pytest.mark.parametrize("M,K,N", [(509, 512, 19456), (385, 256, 38000), (953, 512, 19441), (1030, 256, 19456), (2047, 256, 9728), (641, 1024, 14337)])
+@pytest.mark.parametrize("M,K,N", [(509, 512, 19456), (385, 256, 38000), (953, 512, 19441), (1030, 256, 19456), (2047, 256, 9728), (641, 1024, 14337), (510, 512, 30001), (384, 256, 28672),
+                                   (129, 512, 65000), (192, 768, 40001), (576, 256, 19456)])
 def test_tiles_of_256_rows(dev, po, qt, M, K, N):
     """Rows are the rows of calls of 128 rows, which have tiles of 128, bit for bit (K unsplit)."""
     r = synth.rng_for(50, qt, M, K, N)
