@@ -1,7 +1,8 @@
 // Prompt products over bfloat16 weights: C[M][N] = A[M][K] . W[N][K]^T on the matrix cores.
 //
 // dense_gemm_tiles_kernel (more than 64 bfloat16 rows): the tiles of gemm_tile.h, as plan_tiles lays them out.
-// dense_gemm_kernel (up to 64 bfloat16 rows, outputs of few tiles, rows far apart): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
+// dense_gemm_few_kernel (up to 64 bfloat16 rows, outputs of up to 1280 tiles of 32 x 32).
+// dense_gemm_kernel (up to 64 bfloat16 rows and more columns, outputs of few tiles, rows far apart): 4 waves, BM x BN output tile, 64 values of K per step.  Tiles go global -> registers ->
 // LDS; two register sets and two LDS buffers, so a step has one barrier and the loads of the next two steps are in flight
 // while its MFMAs run.
 // LDS rows are 128 bytes, the eight 16-byte pieces of row r stored at piece ^ (r % 8): the fragment reads (32 rows, one
@@ -98,6 +99,97 @@ __device__ __forceinline__ void store_glu(const DenseGemm& g, int m, int n, int 
         if (v < o.N)
             store4<F32>(o, 0, m, v, silu_f(acc[4 * q]) * acc[8 + 4 * q], silu_f(acc[4 * q + 1]) * acc[9 + 4 * q],
                         silu_f(acc[4 * q + 2]) * acc[10 + 4 * q], silu_f(acc[4 * q + 3]) * acc[11 + 4 * q]);
+    }
+}
+
+// Few rows: a workgroup has 32 rows and 32 columns, its four waves take steps of K in turn, and their sums meet at the end.  A wave's steps come to LDS
+// of its own, two of them in flight, W and X alike in whole 128-byte rows, and nothing but the end has a barrier.
+// What bounds it: how much of W is on its way, 4 KB a step, which is why a workgroup has few columns (64: 30 x 2560 x 2560 13.5 us where this takes
+// 9.6, 30 x 10240 x 2560 15.7 and 17.5; 64 rows at a time: 48 x 2560 x 2560 11.8 and 8.6).  Weights from HBM, in a graph, against the tiles of
+// dense_gemm_kernel: 30 x 10240 x 2560 24.3 -> 17.5 us, 30 x 19456 x 2560 30.8 -> 26.7, 30 x 2560 x 9728 70.7 -> 25.3, 19 x 5632 x 2560 23.0 -> 9.7,
+// 64 x 2560 x 9728 68.3 -> 25.0.
+constexpr int FEW_WAVES = 4, FEW_STEPS = 2;
+__global__ __launch_bounds__(64 * FEW_WAVES, 2) void dense_gemm_few_kernel(const DenseGemm g) {
+    constexpr int STEP = 8192, PIECES = 8;  // 32 rows of W, 32 of X, and a wave's instructions for them
+    __shared__ __align__(16) uint8_t s_t[FEW_WAVES * FEW_STEPS * STEP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 31, kh = lane >> 5;
+    const int tiles_n = (g.tile_cols + 31) / 32, tiles_m = (g.M + 31) / 32, split = blockIdx.x / (tiles_m * tiles_n);
+    int tm, tn;
+    tile_of(blockIdx.x - split * tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
+    const int m0 = 32 * tm, n0 = 32 * tn, all = (g.K + 63) / 64, first = all * split / g.splits + wave, end = all * (split + 1) / g.splits;
+    const uint16_t* A = static_cast<const uint16_t*>(g.A);
+    if (g.section_n > 0) A += n0 / g.section_n * g.section_a;
+    gt_i4 ws = gt_buffer(g.W), xs = gt_buffer(A);
+    xs[0] = __builtin_amdgcn_readfirstlane(xs[0]);
+    xs[1] = __builtin_amdgcn_readfirstlane(xs[1]);
+    const int piece = ((lane & 7) ^ (lane >> 3)) << 4;  // piece p of row r lies at p ^ (r % 8)
+    int wo[4], xo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        wo[i] = weight_row(g, n0 + r) * (int)g.ldw * 2 + piece;
+        xo[i] = min(m0 + r, g.M - 1) * (int)g.lda * 2 + piece;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)s_t + wave * (FEW_STEPS * STEP);
+    auto fetch = [&](int slot, int st) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gt_to_lds(lds0 + slot * STEP + i * 1024, wo[i], ws, st * 128);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gt_to_lds(lds0 + slot * STEP + 4096 + i * 1024, xo[i], xs, st * 128);
+    };
+    gm_f16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    auto step = [&](int slot, int st) {  // used, and its place given to the step FEW_STEPS on
+        if (st + FEW_WAVES < end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const uint8_t* t = s_t + (wave * FEW_STEPS + slot) * STEP + j * 128;
+        gm_b8 w[4], x[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int at = ((2 * ks + kh) ^ (j & 7)) << 4;
+            w[ks] = *reinterpret_cast<const gm_b8*>(t + at);
+            x[ks] = *reinterpret_cast<const gm_b8*>(t + 4096 + at);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (st + FEW_STEPS * FEW_WAVES < end) fetch(slot, st + FEW_STEPS * FEW_WAVES);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ks], x[ks], acc, 0, 0, 0);
+    };
+    if (first < end) fetch(0, first);
+    if (first + FEW_WAVES < end) fetch(1, first + FEW_WAVES);
+    for (int st = first; st < end; st += 2 * FEW_WAVES) {
+        step(0, st);
+        if (st + FEW_WAVES < end) step(1, st + FEW_WAVES);
+    }
+    __syncthreads();
+    float4* sums = reinterpret_cast<float4*>(s_t);  // [wave][four columns][lane]
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sums[(4 * wave + q) * 64 + lane] = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    __syncthreads();
+    auto sum = [&](int q) {
+        float4 v = sums[q * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < FEW_WAVES; ++w) {
+            const float4 o = sums[(4 * w + q) * 64 + lane];
+            v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
+        }
+        return v;
+    };
+    const int m = m0 + j;
+    const bool glu = g.epilogue == GEMM_SWIGLU;
+    if (m >= g.M || (glu && wave >= 2)) return;
+    const float4 v = sum(wave);
+    if (glu) {  // columns 0 .. 15 of the 32 are gates
+        const float4 u = sum(wave + 2);
+        DenseGemm o = g;
+        o.epilogue = GEMM_ELEM;
+        o.N = g.N / 2;
+        const int n = n0 / 2 + 8 * wave + 4 * kh;
+        if (n < o.N) store4<false>(o, 0, m, n, silu_f(v.x) * u.x, silu_f(v.y) * u.y, silu_f(v.z) * u.z, silu_f(v.w) * u.w);
+    } else {
+        const int n = n0 + 8 * wave + 4 * kh;
+        if (n < g.N) store4<false>(g, split, m, n, v.x, v.y, v.z, v.w);
     }
 }
 
@@ -377,6 +469,11 @@ TilePlan dense_gemm_plan(const DenseGemm& g, bool may_split) {
     return p;
 }
 
+// Up to so many tiles of 32 x 32 dense_gemm_few_kernel has the few rows; with more of them, larger tiles fill the chip, too, and read X less often:
+// 32 x 28672 x 4096 (896) 51.7 us there and 51.3 with few, 64 x 19456 x 2560 (1216) 37.0 and 35.3, 64 x 28672 x 4096 (1792) 56.3 and 68.6, 30 x 65536 x
+// 1024 (2048) 28.2 and 31.6.
+constexpr int64_t FEW_TILES = 1280;
+
 int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (!g.A || !g.W || !g.C) return PTM_E_NULL;
     const int kp = up64(g.K);
@@ -388,7 +485,7 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (!aligned16(g.A) || !aligned16(g.W) || !aligned16(g.C) || (g.lda & 7) || (g.ldw & 7)) return PTM_E_ALIGN;
     const int cols = g.tile_cols = tile_columns(g);
     auto tiles = [&](int bm, int bn) { return ((int64_t)g.M + bm - 1) / bm * ((cols + bn - 1) / bn); };
-    if (tiles(32, 64) * 16 > 0x7fffffff) return PTM_E_UNSUPPORTED;
+    if (tiles(32, 32) * 16 > 0x7fffffff) return PTM_E_UNSUPPORTED;
     // splits that bring `t` tiles to about `target` workgroups, each with at least four steps of K
     auto split = [&](int64_t t, int64_t target) {
         g.splits = 1;
@@ -402,6 +499,10 @@ int dense_gemm(DenseGemm g, hipStream_t s, int* splits) {
     if (g.a_fp32) {
         g.splits = 1;
         hipLaunchKernelGGL(dense_gemm_f32_kernel, dim3((unsigned)tiles(64, 64)), dim3(256), 0, s, g);
+    } else if (g.M <= 64 && tiles(32, 32) <= FEW_TILES && g.lda <= 1 << 22 && (int64_t)g.N * g.ldw < 1 << 30) {  // (offsets of 32 bits)
+        split(tiles(32, 32), 512);
+        if (g.splits > kp / 512) g.splits = kp / 512 > 1 ? kp / 512 : 1;  // two steps a wave
+        hipLaunchKernelGGL(dense_gemm_few_kernel, dim3((unsigned)(tiles(32, 32) * g.splits)), dim3(64 * FEW_WAVES), 0, s, g);
     } else if (g.M <= 32) {
         split(tiles(32, 128), 512);
         hipLaunchKernelGGL((dense_gemm_kernel<32, 128, 32, 32>), dim3((unsigned)(tiles(32, 128) * g.splits)), dim3(256), 0, s, g);

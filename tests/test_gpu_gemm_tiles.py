@@ -112,6 +112,16 @@ def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0, ldw=0):
 
 
 # gates and ups just under and over 2 GiB apart, and 4.6 GiB
+# up to 64 rows in tiles of 32 x 32 and a step: one, fewer steps than waves, steps that are no multiple of the waves, K split, sections, every epilogue,
+# and the last output that these tiles take with the first that they do not
+@pytest.mark.parametrize("M,N,K,epilogue,section,slabs", [
+    (1, 1, 8, F32, 0, 0), (1, 32, 64, ELEM, 0, 0), (31, 257, 100, F32, 0, 0), (32, 64, 576, RELU2, 0, 0), (33, 65, 320, DECAY, 0, 0), (64, 96, 1030, SWIGLU, 0, 0),
+    (17, 90, 200, SWIGLU, 0, 0), (30, 512, 2560, F32, 128, 0), (64, 40, 9728, F32, 0, 16), (30, 2560, 1536, F32, 0, 16), (32, 40960, 64, F32, 0, 0),
+    (32, 40961, 64, F32, 0, 0), (64, 20480, 192, ELEM, 0, 0), (64, 20481, 192, ELEM, 0, 0)])
+def test_few_rows(dev, M, N, K, epilogue, section, slabs):
+    check_product(M, N, K, epilogue, section, slabs)
+
+
 @pytest.mark.parametrize("ldw", [558656, 558664, 1200000])
 def test_ups_far_from_their_gates(dev, ldw):
     check_product(1041, 3844, 64, SWIGLU, ldw=ldw)
