@@ -279,9 +279,12 @@ __global__ __launch_bounds__(64) void tanh_rows_kernel(const float* __restrict__
     }
 }
 
-// Where x, B and C of a convolved row lie: x padded to 4, then B and C of every group padded to KP, all padding zeros.
+// Where x, B and C of a convolved row lie: x, then B and C of every group, each padded to 4, then sixteen zeros, which stand for the keys that the matrix
+// products have beyond these (and end the 16 columns of the last head).  All padding is zeros.  Padded to the keys of the products instead, up to 64 for one,
+// a row of thousands of small groups is megabytes, and 2048 of them pass the 32 bits of an offset.
 __host__ __device__ inline int conv_x(const SsmShape& m) { return (m.heads * m.vdim + 3) & ~3; }
-int64_t ssm_conv_row(const SsmShape& m) { return conv_x(m) + 2 * (int64_t)m.groups * padded_keys(m.state); }
+__host__ __device__ inline int conv_keys(const SsmShape& m) { return (m.state + 3) & ~3; }
+int64_t ssm_conv_row(const SsmShape& m) { return conv_x(m) + 2 * (int64_t)m.groups * conv_keys(m) + 16; }
 // per 16 tokens and head: what the tokens take from each other [16 from][16 to], the state's decay up to each, each one's share of the new state
 constexpr int SSM_TILE = 288;
 int64_t ssm_tile_floats(int heads, int rows) { return (int64_t)((rows + 15) / 16) * heads * SSM_TILE; }
@@ -306,8 +309,8 @@ __global__ __launch_bounds__(256) void ssm_conv_rows_kernel(const SsmRows a) {
     if (at >= a.conv_ld) return;
     int ch = at;
     if (at >= conv_x(m)) {
-        const int kp = a.keys, q = at - conv_x(m), n = q % kp;
-        ch = n < m.state ? inner + q / kp * m.state + n : channels;
+        const int keys = conv_keys(m), q = at - conv_x(m), n = q % keys;
+        ch = n < m.state && q / keys < 2 * m.groups ? inner + q / keys * m.state + n : channels;
     } else if (at >= inner) ch = channels;
     if (ch == channels) {
         for (int r = 0; r < rows; ++r) a.conv[(int64_t)(r0 + r) * a.conv_ld + at] = 0.0f;
@@ -359,14 +362,16 @@ __global__ __launch_bounds__(256) void ssm_tiles_kernel(const SsmRows a, int eac
         next_skip = m.D[h];
     };
     fetch(first);
-    const float* at = a.conv + row * a.conv_ld + conv_x(m) + (int64_t)blockIdx.z * a.keys + 4 * g4;
+    const float* conv = a.conv + row * a.conv_ld;
+    const int keys = conv_keys(m), b_at = conv_x(m) + blockIdx.z * keys, c_at = b_at + m.groups * keys, zeros = (int)a.conv_ld - 4;
     rc_f4 dot = {0.f, 0.f, 0.f, 0.f}, odd = dot;  // rows s = 4 g4 + i, column t = j
     for (int k = 0; k < a.keys; k += 64) {
         rc_f4 B[4], C[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            B[i] = *reinterpret_cast<const rc_f4*>(at + k + 16 * i);
-            C[i] = *reinterpret_cast<const rc_f4*>(at + k + 16 * i + (int64_t)m.groups * a.keys);
+            const int key = k + 16 * i + 4 * g4;
+            B[i] = *reinterpret_cast<const rc_f4*>(conv + (key < keys ? b_at + key : zeros));
+            C[i] = *reinterpret_cast<const rc_f4*>(conv + (key < keys ? c_at + key : zeros));
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -412,8 +417,9 @@ static int scan_lds(int waves, int keys) { return 2048 * waves + scan_stages(key
 struct Scan {
     int M, tiles, columns, c0;
     bool from_zero;
-    const float* bc;            // SSM: rows of B and C, `bc_step` bytes a token, at bytes b_at and c_at.  WKV: the tiles
-    uint32_t bc_step, b_at, c_at;
+    const float* bc;            // SSM: rows of B and C, `bc_step` bytes a token (all tokens in 32 bits), at bytes b_at and c_at.  WKV: the tiles
+    uint32_t bc_step, b_at, c_at, zeros_at;
+    int pieces;                 // SSM: 16-byte pieces of B; the others are at zeros_at
     const float* pairs;         // SSM: M, P and Q of each tile.  WKV: M and the keys' decays, behind the rows of the tiles
     uint32_t tile_bytes;        // from one tile's to the next's
     const float* x;
@@ -461,9 +467,9 @@ __device__ __forceinline__ void scan_columns(const Scan& a, uint8_t* ss_lds) {
     uint32_t row_of[BCI], col_of[BCI];
 #pragma unroll
     for (int i = 0; i < BCI; ++i) {
-        const int p = (BCI * wave + i) * 64 + lane, q = (p % ROW) ^ (p / ROW & 15);
+        const int p = (BCI * wave + i) * 64 + lane, q = (p % ROW) ^ (p / ROW & 15), of = q % (ROW / 2);
         row_of[i] = p / ROW * (WKV ? 16 * ROW : a.bc_step);
-        col_of[i] = WKV ? 16 * q : (q < ROW / 2 ? a.b_at : a.c_at) + 16 * (q % (ROW / 2));
+        col_of[i] = WKV ? 16 * q : of < a.pieces ? (q < ROW / 2 ? a.b_at : a.c_at) + 16 * of : a.zeros_at;
     }
     const uint32_t x_row = (4 * g4 + w4) * a.x_step, x_col = a.x_at + 4 * (c0 + j), pair_at = 16 * (PIECES * w4 + min(lane, PIECES - 1));
     auto fetch = [&](int n, int i) {
@@ -645,8 +651,10 @@ __global__ __launch_bounds__(64 * W, 1) void ssm_scan_kernel(const SsmRows a) {
     s.from_zero = a.pos0 == 0;
     s.bc = s.x = a.conv;
     s.bc_step = s.x_step = (uint32_t)a.conv_ld * 4;
-    s.b_at = 4 * (conv_x(m) + g * a.keys);
-    s.c_at = 4 * (conv_x(m) + (m.groups + g) * a.keys);
+    s.b_at = 4 * (conv_x(m) + g * conv_keys(m));
+    s.c_at = 4 * (conv_x(m) + (m.groups + g) * conv_keys(m));
+    s.zeros_at = s.bc_step - 16;
+    s.pieces = conv_keys(m) / 4;
     s.pairs = a.tiles + (int64_t)h * s.tiles * SSM_TILE;
     s.tile_bytes = SSM_TILE * 4;
     s.x_at = 4 * h * m.vdim;
@@ -740,7 +748,8 @@ __global__ __launch_bounds__(64 * W, 1) void wkv_scan_kernel(const WkvRows a) {
     s.from_zero = a.pos0 == 0;
     s.tile_bytes = wkv_tile(a.keys) * 4;
     s.bc = a.tiles + (int64_t)h * s.tiles * wkv_tile(a.keys);
-    s.bc_step = s.b_at = s.c_at = 0;
+    s.bc_step = s.b_at = s.c_at = s.zeros_at = 0;
+    s.pieces = 0;
     s.pairs = s.bc + 32 * a.keys;
     s.x = a.proj;
     s.x_step = (uint32_t)a.ld * 4;
@@ -837,6 +846,7 @@ int64_t wkv_tile_floats(int heads, int dim, int rows) { return (int64_t)((rows +
 
 int wkv_rows(WkvRows a, bool fp32, hipStream_t s) {
     if (!recurrent_supported(a.dim)) return PTM_E_UNSUPPORTED;
+    if (a.M * a.ld >= (int64_t)1 << 30) return PTM_E_UNSUPPORTED;  // 32-bit offsets of the scan; not reached by 2048 rows of what a decoder accepts
     a.keys = padded_keys(a.dim);
     hipLaunchKernelGGL(wkv_tiles_kernel, dim3((a.M + 15) / 16, a.heads), dim3(256), 0, s, a);
     static std::once_flag raised;
@@ -878,6 +888,7 @@ int ssm_rows(SsmRows a, bool fp32, hipStream_t s) {
     if (!recurrent_supported(m.state)) return PTM_E_UNSUPPORTED;
     a.keys = padded_keys(m.state);
     a.conv_ld = ssm_conv_row(m);
+    if (a.M * a.conv_ld >= (int64_t)1 << 30) return PTM_E_UNSUPPORTED;  // 32-bit offsets of the scan; not reached by 2048 rows of what a decoder accepts
     hipLaunchKernelGGL(ssm_conv_rows_kernel, dim3((a.M + CONV_ROWS - 1) / CONV_ROWS, (unsigned)((a.conv_ld + 255) / 256 + 1)), dim3(256), 0, s, a);
     const int per = m.heads / m.groups, each = (int64_t)(a.M + 15) / 16 * m.heads > 4096 ? 2 : 1;
     hipLaunchKernelGGL(ssm_tiles_kernel, dim3((a.M + 15) / 16, (per + 4 * each - 1) / (4 * each), m.groups), dim3(256), 0, s, a, each);

@@ -184,3 +184,15 @@ def test_decode_attention_args_are_checked():
     import ctypes as C
     a = _lib.AttentionArgs(Q=16, K1=16, V=16, O=16, rows=1, heads=2, kv_heads=2, dim1=8, vdim=8, gate=16)
     assert L.ptm_attention_rows(C.byref(a), None) == E_SHAPE             # a gate without its columns
+
+
+# ---- prompt rows of state-space mixers --------------------------------------------------------------
+@pytest.mark.parametrize("heads,vdim,state,groups", [(40, 64, 128, 1), (4096, 9, 9, 4096), (36864, 1, 1, 36864), (12288, 3, 3, 12288), (72, 512, 512, 72), (7372, 5, 5, 7372)])
+def test_convolved_rows_of_2048_tokens_have_32_bit_offsets(heads, vdim, state, groups):
+    """The scan reads the rows with byte offsets of 32 bits.  The shapes are at the limits of what a decoder accepts: 36864 values, 36864 keys of all groups."""
+    import ctypes
+    from gemm_helpers import harness
+    h = harness()
+    h.ssm_scratch.restype = ctypes.c_int64
+    floats = h.ssm_scratch(heads, vdim, state, groups, 2048, 0)
+    assert 2048 * (heads * vdim + 2 * groups * state) <= floats < 2**30
