@@ -460,7 +460,7 @@ __device__ __forceinline__ void scan_columns(const Scan& a, uint8_t* ss_lds) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) S[q][i] = a.from_zero ? 0.0f : keys[KT * i + q];
     }
-    // memory -> LDS; rows past the last repeat it and count nothing, columns of x past the last are what lies there and are not stored
+    // memory -> LDS; rows past the last repeat it and are taken out again in registers, columns of x past the last are what lies there and are not stored
     const uint32_t last = (uint32_t)(a.M - 1) * a.bc_step, x_last = (uint32_t)(a.M - 1) * a.x_step;
     const gt_i4 rows = gt_buffer(a.bc), pairs = gt_buffer(a.pairs), xs = gt_buffer(a.x);
     const uint32_t lds0 = (uint32_t)(uintptr_t)ss_lds + TILES;
@@ -540,10 +540,19 @@ __device__ __forceinline__ void scan_columns(const Scan& a, uint8_t* ss_lds) {
         if constexpr (W == 8) v += (sums[4] + sums[5]) + (sums[6] + sums[7]);
         y[(int64_t)16 * n * a.y_ld] = v;
     };
-    auto run = [&](const Tile& v, Tile& next, int n) {
+    auto run = [&](Tile& v, Tile& next, int n) {
         // the next tile has arrived in every wave's part; the one used now lies in registers, and its LDS takes one more
         if (n + STAGES - 1 < tiles) gt_arrived<(STAGES - 2) * PER>();
         else gt_arrived<0>();
+        if (16 * n + 16 > a.M)  // what repeats the last row may be infinite, and a factor of zero does not take it out of the state
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (16 * n + 4 * g4 + i >= a.M) {
+                    v.x[i] = 0.0f;
+                    if constexpr (!WKV)  // (their k are zeros in the tiles)
+#pragma unroll
+                        for (int q = 0; q < KT; ++q) v.B[i][q] = 0.0f;
+                }
         rc_f4 old[KT], here = {0.f, 0.f, 0.f, 0.f}, next_S[KT];
         float dx[4];
 #pragma unroll

@@ -523,6 +523,12 @@ def test_state_space_scan(dev, heads, vdim, state, groups, taps, rows, pos0):
         loud = proj.clone()
         loud[9, inner] = float("inf")
         assert torch.equal(run(loud)[0][:9], out[:9])
+    # a last token's x and B that are infinite leave the states that they enter infinite, and all others alone
+    for at, where in ((0, (0, 0)), (inner, (slice(heads // groups), slice(None), 0))):
+        loud, mask = proj.clone(), torch.zeros(heads, vdim, state, dtype=torch.bool, device="cuda")
+        loud[-1, inner + at], mask[where] = float("inf") * float(w[0][at, -1].sign()), True
+        got = run(loud)[1][:, :, :state]
+        assert torch.equal(got.isinf(), mask) and not got.isnan().any(), at
 
 
 # every number of key tiles a wave has, dims off 4 and off the tiles, tokens off 16, one head and many; decays next to 1, next to 0 and 0
@@ -570,3 +576,8 @@ def test_wkv_scan(dev, heads, dim, rows, pos0):
             loud = proj.clone()
             loud[9, part, 0, 0] = float("inf")
             assert torch.equal(run(loud)[0][:9], out[:9])
+    for part, where in ((2, (0, 0)), (1, (0, slice(None), 0))):  # a last token's v and k that are infinite
+        loud, mask = proj.clone(), torch.zeros(heads, dim, dim, dtype=torch.bool, device="cuda")
+        loud[-1, part, 0, 0], mask[where] = float("inf"), True
+        got = run(loud)[1][:, :, :dim]
+        assert torch.equal(got.isinf(), mask) and not got.isnan().any(), part
