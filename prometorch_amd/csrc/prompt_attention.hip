@@ -11,10 +11,11 @@ namespace ptm {
 // holds in its S^T accumulator, in that order.
 // A tile's vector arithmetic takes longer than its 48 MFMAs, so it is kept short: the cap in three instructions beside 2^x and 1 / x (ten as
 // written: 1030 rows of 32 heads of 128, capped, 54.5 -> 46.4 us) in a kernel of its own, conversions in pairs, scale and reference of an exponent in one
-// multiply-add, no branch around a piece that is padding (it is read from zeros), rescaling only where the reference moves by 2^8.  With the
-// pairing of long row blocks and short ones: 2048 rows of 32 heads of 128, gated, 104 -> 83 us (without the second bfloat16 term of the weights 71,
-// without fetches, staging and barriers 69), 1500 rows 75 -> 62, 1030 rows of 192 and 128 54 -> 50, capped 47 -> 44.  Two groups of waves on alternate
-// tiles, and the scores of the next 32 keys formed between the parts of a softmax (K a tile ahead in LDS), were no faster: 47.3 and 47.8 us, capped.
+// multiply-add, no branch around a piece that is padding (it is read from zeros).  With the pairing of long row blocks and short ones, launches in a row:
+// 2048 rows of 32 heads of 128, gated, 88 -> 79 us, 1500 rows 66 -> 59, 1030 rows of 192 and 128 46.6 -> 45.1, capped 42.6 -> 40.2.  A reference that moves
+// only when it is passed by 2^8 takes 1 to 7 us less, but then the largest weight is no longer 1, and a tenth to a third more of the results were not the
+// bfloat16 number nearest to the exact one.  Two groups of waves on alternate tiles, and the scores of the next 32 keys formed between the parts of a softmax (K
+// a tile ahead in LDS), were no faster: 47.3 and 47.8 us, capped.
 __device__ const uint4 zero_piece = {0, 0, 0, 0};
 
 template <int DQ, int DV, bool CAP>
@@ -177,19 +178,10 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[u][r]);
         const LanePair p = pair32(mx);
         mx = fmaxf(p.a, p.b);
-        // The reference of a query's weights is its largest exponent so far to within 2^8: sums and values are rescaled when it is passed by more, which
-        // after the first tiles is seldom.
+        // The reference of a query's weights is its largest exponent so far: the largest weight is 1, which two bfloat16 terms hold exactly.
         mx *= mul;
-        if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.0f) != 0) {
-            const float m_new = mx > m_run + 8.0f ? mx : m_run, corr = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= corr;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[dt][r] *= corr;
-            m_run = m_new;
-        }
-        const float ms = m_run == -INFINITY ? 0.0f : m_run;  // nothing visible yet
+        const float m_new = fmaxf(m_run, mx), ms = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet
+        const float corr = __builtin_amdgcn_exp2f(m_run - ms);
         float psum = 0.0f;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -198,7 +190,14 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
                 sc[u][r] = __builtin_amdgcn_exp2f(fmaf(sc[u][r], mul, -ms));
                 psum += sc[u][r];
             }
-        l_run += psum;
+        l_run = fmaf(l_run, corr, psum);
+        if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[dt][r] *= corr;
+        }
+        m_run = m_new;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -244,7 +243,7 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
             else z[i] = make_float4(gate[min(v, gates - 1)], gate[min(v + 1, gates - 1)], gate[min(v + 2, gates - 1)], gate[min(v + 3, gates - 1)]);
         }
     }
-    auto factor = [&](int v, float z) { return v < gates ? scale * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -LOG2E)) : scale; };
+    auto factor = [&](int v, float z) { return v < gates ? scale * sigmoid_f(z) : scale; };  // out_factor
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll

@@ -428,6 +428,49 @@ def test_prompt_attention_forms(dev, rows, heads, kv_heads, dim, scale, cap, lou
     assert err.max() < 1e-2, err.max()
 
 
+@pytest.mark.parametrize("dim,vdim,cap", [(64, 64, 0.0), (128, 64, 0.0), (128, 128, 0.0), (192, 128, 0.0), (256, 256, 0.0), (128, 128, 50.0)])
+@pytest.mark.parametrize("part", ["weights", "gate"])
+def test_prompt_attention_rounds_like_64_bits(dev, dim, vdim, cap, part):
+    """The share of values that are not the nearest bfloat16 number to the 64-bit result.  Borders are 2^-7 of the power of two below apart and a value is up to
+    twice that power: relative errors of e take 256 e of the values past one.
+    weights: a score of 2^7 to 2^8 times the weight of the first comes in a later tile.  Its own weight is 1, which has no rounding; what the first weighs,
+    2^-7, is rounded at 2^-17, and five operations at 2^-24: e < 4e-7, 1e-4 of the values.  Measured against another score than the largest it is itself off by
+    up to 2^-17, and 2e-4 to 3e-4 differed.
+    gate: one visible key, so that the gate is all that is computed: 1 / (1 + e^-z) in 32 bits, z down to -80, and two products: e < 4e-7 again.  With z
+    times log2(e) rounded in front of the exponential, 3e-6 at z = -80, 1.35e-4 to 1.9e-4 differed."""
+    import torch
+    rows, heads, pos0 = 260, 4, 200
+    rng = np.random.default_rng(dim + vdim)
+    n = pos0 + rows
+    rnd = lambda *s: fw.from_bf16(fw.to_bf16(rng.standard_normal(s, np.float32)))
+    gates = np.zeros((rows, heads, vdim), np.float32)
+    if part == "weights":
+        q, k = np.zeros((rows, heads, dim), np.float32), np.zeros((n, 1, dim), np.float32)
+        q[..., 0], q[..., 1] = 1, fw.from_bf16(fw.to_bf16(rng.random((rows, heads), np.float32)))
+        k[:, 0, 0] = -120
+        k[0, 0, 0], k[150, 0, :2] = 0, (5, 0.4375)
+    else:
+        q, k = rnd(rows, heads, dim), rnd(n, 1, dim)
+        gates = (-80 * rng.random((rows, heads, vdim))).astype(np.float32)
+    v = rnd(n, 1, vdim)
+    see = N.visible(n, {"size": 1} if part == "gate" else None)[pos0:]
+    s = np.einsum("rhd,nd->hrn", q.astype(np.float64), k[:, 0].astype(np.float64))
+    s = np.where(see, cap * np.tanh(s / cap) if cap else s, -np.inf)
+    p = np.exp(s - s.max(2, keepdims=True))
+    want = np.einsum("hrn,nv->rhv", p / p.sum(2, keepdims=True), v[:, 0].astype(np.float64)) / (1 + np.exp(-gates.astype(np.float64)) if part == "gate" else 1)
+    put = lambda a: torch.from_numpy(fw.to_bf16(a).view(np.int16)).cuda()
+    Q, K, V, G = put(q), put(k), put(v), torch.from_numpy(gates).cuda()
+    O = torch.zeros((rows, heads, vdim), dtype=torch.bfloat16, device="cuda")
+    a = _lib.AttentionArgs(Q=Q.data_ptr(), K1=K.data_ptr(), V=V.data_ptr(), O=O.data_ptr(), q_row=heads * dim, k1_row=dim, k1_head=dim, v_row=vdim, v_head=vdim,
+                           o_row=heads * vdim, rows=rows, heads=heads, kv_heads=1, dim1=dim, vdim=vdim, window=1 if part == "gate" else 0, pos0=pos0, scale=1.0, softcap=cap,
+                           fp32=0, gate=G.data_ptr() if part == "gate" else None, gate_row=heads * vdim, gate_head=vdim if part == "gate" else 0)
+    _lib.check(_lib.load().ptm_attention_rows(C.byref(a), None), "attention_rows")
+    torch.cuda.synchronize()
+    differ = (O.cpu() != torch.from_numpy(want).to(torch.bfloat16)).double().mean().item()
+    print("differ: %.2e" % differ, flush=True)
+    assert differ <= 1e-4
+
+
 # ---- products with the gated epilogue are reached through the models; shapes around their tile edges -------------
 @pytest.mark.parametrize("ff", [1, 15, 16, 17, 64, 100, 257])
 def test_feed_forward_sizes(dev, tmp_path, ff):
