@@ -4,6 +4,8 @@
 // 52 launches took 1 % longer with them in one).
 #include "attention.h"
 
+#include <type_traits>
+
 namespace ptm {
 
 // v_mfma_f32_32x32x16_bf16: A: lane l holds row l % 32, summation indices 8 (l / 32) + 0..7; B: column l % 32, the same
@@ -18,8 +20,17 @@ namespace ptm {
 // a tile ahead in LDS), were no faster: 47.3 and 47.8 us, capped.
 __device__ const uint4 zero_piece = {0, 0, 0, 0};
 
+// Workgroups of a class that share a CU.  (Of 256 and 256 the registers leave room for one.)
+constexpr int mfma_resident(int DQ, int DV) { return DQ <= 192 && DV <= 128 ? 2 : 1; }
+// Row blocks go longest first.  Where two workgroups share a CU and all are there at once, the second 256 come shortest first, so that the longest row block
+// has the shortest beside it: heads of 128, 512 workgroups 85 -> 79 us, 328 43 -> 41; where only a few share (heads of 64, 264) 23.9 -> 24.5.  With one a CU
+// it would put long ones last: heads of 256, 512 workgroups 165 us, and 134 so.
+__host__ __device__ constexpr int mfma_order(int id, int grid, int resident) {
+    return resident == 2 && grid > 256 && grid <= 512 && id >= 256 ? grid - 1 - (id - 256) : id;
+}
+
 template <int DQ, int DV, bool CAP>
-__global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention_mfma_kernel(const ptm_attention_args a) {
+__global__ __launch_bounds__(256, mfma_resident(DQ, DV)) void attention_mfma_kernel(const ptm_attention_args a) {
     constexpr int KS = DQ / 16, DT = DV / 32, KP = DQ * 2 + 16, VP = DV * 2 + 64;
     __shared__ __align__(16) uint8_t s_k[64 * KP];
     __shared__ __align__(16) uint8_t s_v[64 * VP];
@@ -28,10 +39,8 @@ __global__ __launch_bounds__(256, DQ <= 192 && DV <= 128 ? 2 : 1) void attention
     int sh = 0;  // a row takes 1 << sh slots (heads) of a wave's 32 query vectors
     while ((1 << sh) < per && sh < 5) ++sh;
     const int htiles = (per + 31) / 32, rpw = 32 >> sh, bm = 4 * rpw;
-    // Longest row blocks first, all kv heads of a block together.  Two workgroups share a CU: where all are there at once, the second 256 come
-    // shortest first, so that the longest row block has the shortest beside it.
-    int id = blockIdx.x;
-    if (gridDim.x <= 512 && id >= 256) id = gridDim.x - 1 - (id - 256);
+    // all kv heads of a row block together
+    const int id = mfma_order(blockIdx.x, gridDim.x, mfma_resident(DQ, DV));
     const int gh = id % (a.kv_heads * htiles), g = gh / htiles, ht = gh % htiles;
     const int m_base = ((a.rows + bm - 1) / bm - 1 - id / (a.kv_heads * htiles)) * bm;
     const int slot = (j & ((1 << sh) - 1)) + 32 * ht, row = m_base + wave * rpw + (j >> sh);
@@ -280,13 +289,23 @@ static int mfma_launch(const ptm_attention_args& a, hipStream_t s) {
     return launch_status();
 }
 
+// f(key size, value size) of the class that has such heads
+template <typename F>
+static int mfma_class(int dq, int dv, F f) {
+    using std::integral_constant;
+    if (dq <= 64 && dv <= 64) return f(integral_constant<int, 64>{}, integral_constant<int, 64>{});
+    if (dq <= 128 && dv <= 64) return f(integral_constant<int, 128>{}, integral_constant<int, 64>{});
+    if (dq <= 128 && dv <= 128) return f(integral_constant<int, 128>{}, integral_constant<int, 128>{});
+    if (dq <= 192 && dv <= 128) return f(integral_constant<int, 192>{}, integral_constant<int, 128>{});
+    return f(integral_constant<int, 256>{}, integral_constant<int, 256>{});
+}
+
 int attention_mfma(const ptm_attention_args& a, hipStream_t s) {
-    const int dq = a.dim1 + a.dim2;
-    if (dq <= 64 && a.vdim <= 64) return mfma_launch<64, 64>(a, s);
-    if (dq <= 128 && a.vdim <= 64) return mfma_launch<128, 64>(a, s);
-    if (dq <= 128 && a.vdim <= 128) return mfma_launch<128, 128>(a, s);
-    if (dq <= 192 && a.vdim <= 128) return mfma_launch<192, 128>(a, s);
-    return mfma_launch<256, 256>(a, s);
+    return mfma_class(a.dim1 + a.dim2, a.vdim, [&](auto dq, auto dv) { return mfma_launch<decltype(dq)::value, decltype(dv)::value>(a, s); });
+}
+// which row block's turn a workgroup's is, counted from the longest
+int attention_mfma_order(int dq, int dv, int id, int grid) {
+    return mfma_class(dq, dv, [&](auto q, auto v) { return mfma_order(id, grid, mfma_resident(decltype(q)::value, decltype(v)::value)); });
 }
 
 }  // namespace ptm

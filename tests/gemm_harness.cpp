@@ -8,6 +8,7 @@
 #include "recurrent.h"
 
 namespace ptm {
+int attention_mfma_order(int dq, int dv, int id, int grid);
 int prefill_attention_rows(const float* Q, const void* K_cache, const void* V_cache, float* O, void* rows16, float* rowscale,
                            bool q8round, bool* wrote16, int rows, int n_heads, int n_kv_heads, int head_dim, int64_t pos0, int max_seq,
                            float scale, int kv_fp16, int window, hipStream_t s);
@@ -193,5 +194,7 @@ int wkv_run(int heads, int dim, const float* proj, const float* u, const float* 
     return ptm::wkv_rows(w, true, static_cast<hipStream_t>(stream));
 }
 int64_t ssm_state_floats(int heads, int state, int vdim) { return ptm::recurrent_state_floats(heads, state, vdim); }
+
+int attention_order(int dq, int dv, int id, int grid) { return ptm::attention_mfma_order(dq, dv, id, grid); }
 
 }  // extern "C"

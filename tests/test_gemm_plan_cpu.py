@@ -92,3 +92,36 @@ def test_slabs_of_a_qknorm_batch():
             assert b in (1, 2, 4, 8) and (b == 1 or waves <= {8: 2048, 4: 4096, 2: 7168}[b]) and b < 2 * most
     assert [h.qk_rows_batch(m, 190) for m in (1, 2, 3, 4, 5, 16)] == [1, 2, 4, 4, 8, 8]
     assert [h.qk_rows_batch(5, w) for w in (2048, 2049, 4096, 4097)] == [8, 4, 4, 1]
+
+
+# ---- prompt attention -----------------------------------------------------------------------------
+@pytest.mark.parametrize("dq,dv,resident", [(64, 64, 2), (128, 64, 2), (104, 128, 2), (192, 128, 2), (128, 200, 1), (200, 128, 1), (256, 256, 1)])
+@pytest.mark.parametrize("heads,blocks", [(8, 16), (8, 33), (8, 50), (8, 64), (4, 128), (8, 65), (4, 200)])
+def test_row_blocks_that_take_long_do_not_come_last(dq, dv, resident, heads, blocks):
+    """Row block i of a causal prompt takes about i + 1 turns.  `resident` workgroups share a CU, which then takes as long as both together; 256 CUs take the
+    workgroups in the order of their ids.  None is left out, and the launch is no longer than with the longest first."""
+    h, grid = harness(), heads * blocks
+    got = [h.attention_order(dq, dv, i, grid) for i in range(grid)]
+    assert sorted(got) == list(range(grid))
+
+    def lasts(order):
+        cus = [[] for _ in range(256)]  # what is left of a CU's workgroups
+        todo, t = [blocks - o // heads for o in order], 0
+        for s in range(resident):
+            for cu in cus:
+                if todo:
+                    cu.append(todo.pop(0))
+        while any(cus):
+            step = min(min(cu) * len(cu) for cu in cus if cu)
+            t += step
+            for cu in cus:
+                n = len(cu)
+                for i in range(n - 1, -1, -1):
+                    cu[i] -= step / n
+                    if cu[i] < 1e-9:
+                        del cu[i]
+                        if todo:
+                            cu.append(todo.pop(0))
+        return t
+
+    assert lasts(got) <= lasts(range(grid)) + 1e-6
