@@ -285,6 +285,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // LDS holds the fp16 X tile of a whole super-block step: 128 rows x 256 k, row pitch 528 B (16 consecutive lanes
 // x 16 B then hit all 64 banks once), double-buffered: 2 x 66 KB of the CU's 160 KB.
 enum { QF_TM = 128, QF_TN = 256, QF_PITCH = 528 };
+// LDS of a launch in tiles of 128, 192 and 256 rows: two X tiles and the row scales of 128 rows, which take more than those of 256 (qgemm_f16_tall_body)
+enum { QF_ROWS_LDS = 2 * 128 * QF_PITCH + 4 * 128 };
 
 __host__ __device__ inline int qf_mpad(int M) { return (M + QF_TM - 1) / QF_TM * QF_TM; }
 
@@ -1075,6 +1077,7 @@ __device__ __forceinline__ void qgemm_f16_tall_body(const uint8_t* W, int64_t st
                                                     int bz, uint8_t* s_a, int scale_stride) {
     static_assert(MT == 8 || MT == 6, "row tiles of 32");
     constexpr int TM = 32 * MT, STAGE = TM * 256, H = MT / 2;
+    static_assert(2 * STAGE + 4 * TM <= QF_ROWS_LDS, "two stages and the row scales");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, kh = lane >> 5;
     const int m0 = by * TM, n_base = bx * 256 + 64 * (wave & 3) + 32 * (wave >> 2);
@@ -1548,14 +1551,14 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     // rows per workgroup: 32, 64 or 128 (see qgemm_f16_row_tiles)
     const int MT = qgemm_f16_row_tiles(q4, M, N, splits);
     const int tm = 32 * MT;
-    const size_t lds = 2 * (size_t)tm * QF_PITCH + 4 * (size_t)tm;  // 132 KB / 66 KB (two X tiles) + the row scales: above the default 64 KB cap of dynamic LDS
+    const size_t lds = 2 * (size_t)tm * QF_PITCH + 4 * (size_t)tm;  // two X tiles (64 rows: 66 KB) and the row scales: above the default 64 KB cap of dynamic LDS
     static std::once_flag raised;  // two host threads may get here at once: the second waits until the caps are raised
     std::call_once(raised, [] {
-        const int big = 2 * 128 * QF_PITCH + 4 * 128, small = 2 * 64 * QF_PITCH + 4 * 64;
+        const int small = 2 * 64 * QF_PITCH + 4 * 64;
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q4Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_kernel<Q6Tile, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(4));
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q4Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q6Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, big);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q4Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, QF_ROWS_LDS);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_kernel<Q6Tile>), hipFuncAttributeMaxDynamicSharedMemorySize, QF_ROWS_LDS);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
@@ -1583,7 +1586,7 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
     } else if (MT == 4) {
         int tall;
         qf_tall(grid.x, splits, M, q4, &tall);
-#define PTM_QR(TILE) hipLaunchKernelGGL((qgemm_f16_rows_kernel<TILE>), dim3(qf_workgroups(grid.x, splits, M, tall)), dim3(512), lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride, tall)
+#define PTM_QR(TILE) hipLaunchKernelGGL((qgemm_f16_rows_kernel<TILE>), dim3(qf_workgroups(grid.x, splits, M, tall)), dim3(512), QF_ROWS_LDS, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride, tall)
         if (q4) PTM_QR(Q4Tile);
         else PTM_QR(Q6Tile);
 #undef PTM_QR
@@ -1708,8 +1711,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     }
     static std::once_flag raised;
     std::call_once(raised, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  2 * 128 * QF_PITCH + 4 * 128);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, QF_ROWS_LDS);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(QF_SHORT_BLOCKS));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
@@ -1729,7 +1731,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
         for (int i = 0; i < n; ++i) q4 = q4 && types[i] == PTM_TYPE_Q4_K;
         int tall;
         qf_tall(slots, 1, M, q4, &tall);
-        hipLaunchKernelGGL(qgemm_f16_rows_multi_kernel, dim3(qf_workgroups(slots, 1, M, tall)), dim3(512), 2 * (size_t)128 * QF_PITCH + 4 * 128, s, a, M, K, slots, tall);
+        hipLaunchKernelGGL(qgemm_f16_rows_multi_kernel, dim3(qf_workgroups(slots, 1, M, tall)), dim3(512), QF_ROWS_LDS, s, a, M, K, slots, tall);
     }
     if (r.n > 0 && !deferred_P) hipLaunchKernelGGL(qgemm_split_reduce_multi_kernel, dim3(red_blocks), dim3(256), 0, s, r);
     return launch_status();

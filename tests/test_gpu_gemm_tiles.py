@@ -111,7 +111,6 @@ def check_product(M, N, K, epilogue=F32, section=0, slabs=0, pad=0, ldw=0):
     return splits
 
 
-# gates and ups just under and over 2 GiB apart, and 4.6 GiB
 # up to 64 rows in tiles of 32 x 32 and a step: one, fewer steps than waves, steps that are no multiple of the waves, K split, sections, every epilogue,
 # and the last output that these tiles take with the first that they do not
 @pytest.mark.parametrize("M,N,K,epilogue,section,slabs", [
@@ -122,6 +121,14 @@ def test_few_rows(dev, M, N, K, epilogue, section, slabs):
     check_product(M, N, K, epilogue, section, slabs)
 
 
+# outputs of more tiles than that, in tiles of 32 x 128 and 64 x 64: gated, with a bias, sections, steps of K with a rest
+@pytest.mark.parametrize("M,N,K,epilogue,section", [(33, 28672, 330, SWIGLU, 0), (64, 28672, 330, SWIGLU, 0), (19, 41002, 330, SWIGLU, 0), (32, 41000, 200, DECAY, 0),
+                                                    (1, 41001, 130, F32, 0), (40, 24001, 200, RELU2, 0), (30, 49152, 330, F32, 16384), (50, 24576, 330, ELEM, 8192)])
+def test_few_rows_of_wide_outputs(dev, M, N, K, epilogue, section):
+    check_product(M, N, K, epilogue, section)
+
+
+# gates and ups just under and over 2 GiB apart, and 4.6 GiB
 @pytest.mark.parametrize("ldw", [558656, 558664, 1200000])
 def test_ups_far_from_their_gates(dev, ldw):
     check_product(1041, 3844, 64, SWIGLU, ldw=ldw)

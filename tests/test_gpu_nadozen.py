@@ -524,10 +524,12 @@ def ssm_reference(w, proj, m, pos0, ring, S):
     return torch.stack(out), S
 
 
-# every number of key tiles a wave has, states and columns off the tiles, groups, more rows than tiles in flight, tokens off 16
+# every number of key tiles a wave has, states and columns off the tiles, groups, more rows than tiles in flight, tokens off 16, many heads of one group and of
+# two (two heads a wave, the last by itself)
 @pytest.mark.parametrize("heads,vdim,state,groups,taps,rows", [(2, 16, 64, 1, 4, 16), (3, 5, 20, 1, 2, 15), (4, 64, 128, 1, 4, 97), (4, 33, 100, 2, 3, 130), (2, 17, 200, 1, 4, 49),
                                                                (2, 16, 256, 2, 4, 17), (2, 20, 300, 1, 4, 70), (1, 64, 512, 1, 6, 33), (18, 8, 16, 2, 4, 1),
-                                                               (40, 9, 9, 40, 4, 33), (6, 1, 1, 6, 4, 40)])
+                                                               (40, 9, 9, 40, 4, 33), (6, 1, 1, 6, 4, 40),
+                                                               (65, 4, 8, 1, 4, 1030), (66, 3, 70, 2, 2, 1030)])
 @pytest.mark.parametrize("pos0", [0, 21])
 def test_state_space_scan(dev, heads, vdim, state, groups, taps, rows, pos0):
     """One call against the recurrence in 64 bits.  A sum of up to 512 products, 16 decays deep, is off by some 1e-6 of its terms; a first value that is
