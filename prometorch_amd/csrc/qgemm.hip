@@ -1008,8 +1008,8 @@ __device__ __forceinline__ void qgemm_f16_body(const uint8_t* W, int64_t stride,
 // piece of the next sub-block's weights behind every fourth, and one barrier a stage, between the last reads of its LDS and the first of the
 // next, with MFMAs on either side.  The same products in the same order as in the 128-row tile: same bits.  With 192 rows, for launches that would
 // leave CUs idle, everything is three quarters of that but the unpacking.
-// What bounds it: 2048 x 14336 x 4096 in 235 us (265 in 128-row tiles), Q6_K 2048 x 4096 x 14336 238 (326), 1020 TFLOP/s; the matrix cores are busy 66 %
-// of the clocks of a CU at work (41 % before), at which the card lowers its clock (about 1.7 GHz).  Where the barrier lies, when the weights are
+// What bounds it: 2048 x 14336 x 4096 in 236 us (276 in 128-row tiles), Q6_K 257 to 291 (427), 1020 TFLOP/s; the matrix cores are busy 67 % of the time that
+// a workgroup is there (59 % in 128-row tiles), at which the card lowers its clock (1.8 GHz; 1.6 at 2048 x 28672 x 4096).  Where the barrier lies, when the weights are
 // requested and how the pieces are spread change it by less than 1 %.  The same loop for 128 rows is 1 to 5 % slower than qgemm_f16_body.
 
 // What a lane (column n, element half kh) holds of half a super-block, and the fragments of its four sub-blocks, four pieces each.
@@ -1443,13 +1443,19 @@ static int qgemm_f16_row_tiles(bool q4, int M, int N, int splits) {
 
 // Which tiles of a launch of gx column tiles (slots) and gz K splits have 256 rows: the first `tall` pairs of row tiles in qf_tile_of's order, in whole
 // rounds of the chip or all of them - or whether all tiles have 192 - whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
-// times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there.  Measured, all of
-// 128 rows, all of 256, by this rule: 509 x 19456 x 2560 85, 70, 70 us; 953 x 19456 x 2560 132, 150, 125; 2048 x 9728 x 2560 137, 151, 129; 2048 x 28672 x
-// 4096 in 7 rounds, 7, 6.25; 300 x 14336 x 4096 62, 91, 62; Q6_K 2048 x 4096 x 14336 347, 289, 289, 953 x 18944 x 3584 236, 220, 200.
-// A tile of 192 rows takes 1.4 to 1.6 (Q6_K 1.35) of 128-row tiles, by how much of the chip the other tiles leave idle, that is to say how far they let it
-// clock.  The best of the others and 192: 509 x 19456 x 2560 (152 tiles of 256, 228 of 192) 70, 64 us, Q6_K 78, 71; 192 x 65536 x 2560 (512 of 128, 256) 86, 71;
-// 384 x 28672 x 4096 (224 half empty, 224) 117, 93; 953 x 19456 x 2560 (256 + 96, 380) 119, 116; 953 x 28672 x 4096 (256 + 384, 560) 236, 267; 300 x 14336 x
-// 4096 (168 of 128, 112) 56, 71.
+// times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there; a tile of 192 rows
+// 1.4 to 1.6 times (Q6_K 1.35), by how much of the chip the other tiles leave idle, that is to say how far they let it clock.  In us, all of 128 rows, all
+// of 256, whole rounds of 256 and 128 behind them, 192, and by this rule (a run of its own: the same plan again differs by up to 12 %):
+//   509 x 19456 x 2560     82  79   -   68   63 (192)        Q6_K  107  77   -   70   72 (192)
+//   953 x 19456 x 2560    133 154  129 120  123 (256, 128)
+//   953 x 28672 x 4096    273 234  254 265  238 (256)
+//   953 x 14336 x 4096    131 120   -  167  118 (256)        Q6_K  170 124   -  199  125 (256)
+//   2048 x 9728 x 2560    132 147  123 121  122 (256, 128)
+//   2048 x 14336 x 4096   276 236  256 269  237 (256)        Q6_K  427 257  314 322  291 (256)
+//   2048 x 28672 x 4096   496 471  451 477  459 (256, 128)
+//   300 x 14336 x 4096     59  94   -   74   59 (128)        953 x 18944 x 3584, Q6_K  236 214  195 188  195 (256, 128)
+//   384 x 28672 x 4096    121 117   -   93   92 (192)        2048 x 4096 x 14336, Q6_K 317 350   -  314  300 (128)
+// A launch of several matrices counts as Q6_K where one of them is (v beside q and k): up to 50 column tiles and 2048 rows both counts choose the same.
 static float qf_tall(int gx, int gz, int M, bool q4, int* tall) {
     const int gy = (M + QF_TM - 1) / QF_TM, pairs = (gy + 1) / 2, plane = gx * pairs, all = plane * gz;
     const float ratio = q4 ? 1.75f : 1.5f;

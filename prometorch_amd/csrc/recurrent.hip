@@ -198,7 +198,8 @@ __device__ __forceinline__ float row_lane(float v) { return dpp_f<0x150 + N>(v);
 static int padded_keys(int n) { return 16 * keys_per_lane(n); }
 
 // The scan's o of each row and head over its root mean square, times norm and silu(gate).  It moves memory: four values a lane and G lanes a head where the
-// addresses allow, 1024 / G heads a workgroup (2048 rows of 40 heads of 64: a wave per head 22.2 us, this 12.9).  grid ceil(rows * heads / (256 / G))
+// addresses allow, 256 / G heads a workgroup (2048 rows of 40 heads of 64: a wave per head 22.2 us, this 12.9; from 64 values on a wave per head has every
+// lane at work, too, and heads of more than 128 have no form here).  grid ceil(rows * heads / (256 / G))
 template <bool F32, int G>
 __global__ __launch_bounds__(256) void wkv_out_fours_kernel(const WkvRows a) {
     const int at = blockIdx.x * (256 / G) + threadIdx.x / G, row = at / a.heads, h = at % a.heads, d = a.dim, e = 4 * (threadIdx.x % G);
@@ -342,8 +343,8 @@ __global__ __launch_bounds__(256) void ssm_conv_rows_kernel(const SsmRows a) {
 
 // What 16 tokens of a head take from each other: M[s][t] = (C_t . B_s) dt_s prod(s < q <= t) decay_q, with the skip D on the diagonal, the products P_t =
 // prod(q <= t) and Q_s = dt_s prod(q > s) beside it.  Products of decays, never quotients.  grid (ceil(rows / 16), ceil(heads of a group / 4 each),
-// groups), `each` heads a wave (a head for few rows: 30 rows 5.0 us; two where the chip is full: 2048 rows of 40 heads 14.8 -> 11.2); tokens past the
-// last leave everything as it is.
+// groups), `each` heads a wave (ssm_rows); tokens past the last
+// leave everything as it is.
 __global__ __launch_bounds__(256) void ssm_tiles_kernel(const SsmRows a, int each) {
     const SsmShape& m = a.m;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g4 = lane >> 4, t0 = blockIdx.x * 16, per = m.heads / m.groups;
@@ -899,6 +900,7 @@ int ssm_rows(SsmRows a, bool fp32, hipStream_t s) {
     a.conv_ld = ssm_conv_row(m);
     if (a.M * a.conv_ld >= (int64_t)1 << 30) return PTM_E_UNSUPPORTED;  // 32-bit offsets of the scan; not reached by 2048 rows of what a decoder accepts
     hipLaunchKernelGGL(ssm_conv_rows_kernel, dim3((a.M + CONV_ROWS - 1) / CONV_ROWS, (unsigned)((a.conv_ld + 255) / 256 + 1)), dim3(256), 0, s, a);
+    // One head a wave, or two, which read B and C once: 128 keys, 16 to 1600 heads of tiles 6.3 and 7.0 us, 2600 8.7 and 8.3, 4120 11.6 and 9.8, 12288 23.8 and 16.9.
     const int per = m.heads / m.groups, each = (int64_t)(a.M + 15) / 16 * m.heads > 4096 ? 2 : 1;
     hipLaunchKernelGGL(ssm_tiles_kernel, dim3((a.M + 15) / 16, (per + 4 * each - 1) / (4 * each), m.groups), dim3(256), 0, s, a, each);
     const dim3 grid(m.heads, (m.vdim + 15) / 16);
