@@ -31,6 +31,23 @@ __device__ __forceinline__ void read_now(const T&... v) {
     (void)std::initializer_list<int>{(([](auto x) { asm volatile("" ::"s"(x)); })(v), 0)...};
 }
 
+// A uniform value that the compiler takes as it is, not as the load it comes from.  A pointer is then one it knows nothing of: in_global
+// says where it points (a load through a pointer to anywhere is waited for with LDS accesses, too).
+template <typename T>
+__device__ __forceinline__ T in_registers(T v) {
+    asm("" : "+s"(v));
+    return v;
+}
+typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
+typedef __attribute__((address_space(1))) float* GlobalFloats;
+__device__ __forceinline__ GlobalBytes in_global(const uint8_t* p) { return (GlobalBytes)in_registers(p); }
+__device__ __forceinline__ GlobalFloats in_global(float* p) { return (GlobalFloats)in_registers(p); }
+__device__ __forceinline__ uint4 load16(GlobalBytes p) {
+    typedef uint32_t vec __attribute__((ext_vector_type(4)));
+    const vec v = *(const __attribute__((address_space(1))) vec*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // Bookkeeping of a decode step done by the thread that finishes the argmax (all NULL: plain argmax):
 // publish the token, feed it back as the next input, advance the position.
 struct ArgmaxAdvance {
@@ -167,26 +184,54 @@ struct __attribute__((packed, aligned(2))) u16_a2 { uint16_t v; };
 // Q8 activation layout in memory: int8 qs[K] | float d[K/32] | float sum[K/32]
 __host__ __device__ inline int64_t q8_bytes(int K) { return (int64_t)K + K / 4; }
 
+// the low bytes of four values, the first lowest
+__device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+}
+
+// d = amax / 127 and id = 1 / d, 0 where d is, both correctly rounded: a quotient from a correctly rounded reciprocal (of 127 a constant, of d the
+// hardware's with one Newton step) is put right by one exact remainder (Markstein, IBM J. Res. Dev. 34, 1990).  6 instructions where the IEEE
+// sequences take 24; equal to them for every amax and d of 2^-100 .. 2^100, each compared.  Other amax, 0 and NaN among them: the IEEE sequences.
+__device__ __forceinline__ void q8_scales(float amax, float& d, float& id) {
+    const float r127 = 1.0f / 127.0f, q = amax * r127;
+    d = fmaf(fmaf(-127.0f, q, amax), r127, q);
+    const float r = __builtin_amdgcn_rcpf(d);
+    id = fmaf(fmaf(-d, r, 1.0f), r, r);
+    if (!(amax >= 0x1p-90f && amax <= 0x1p90f)) {
+        d = amax / 127.0f;
+        id = d > 0.0f ? 1.0f / d : 0.0f;
+    }
+}
+
 // Quantise the 32 floats held as float4 by the 8 lanes of an aligned lane group.
 // Returns the packed 4 int8 of this lane; d and sum (d * sum q) are group-uniform.
 // Same rule as quantize_x_q8 (reference: torch/io/cpu_quant_gemv.h:147-198).
 __device__ __forceinline__ uint32_t q8_quantize4(float4 v, float& d, float& sum) {
     float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
     amax = max8(amax);
-    d = amax / 127.0f;
-    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    float id;
+    q8_scales(amax, d, id);
     int q0 = (int)rintf(v.x * id), q1 = (int)rintf(v.y * id), q2 = (int)rintf(v.z * id), q3 = (int)rintf(v.w * id);
     q0 = max(-127, min(127, q0));
     q1 = max(-127, min(127, q1));
     q2 = max(-127, min(127, q2));
     q3 = max(-127, min(127, q3));
-    const int s = sum8i(q0 + q1 + q2 + q3);
-    sum = d * (float)s;
-    return (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) |
-           ((uint32_t)(q3 & 0xff) << 24);
+    const uint32_t q = pack_bytes((uint32_t)q0, (uint32_t)q1, (uint32_t)q2, (uint32_t)q3);
+    sum = d * (float)sum8i(__builtin_amdgcn_sdot4((int)q, 0x01010101, 0, false));
+    return q;
 }
 
-// Block-wide sum for blockDim.x = 256 (4 waves); red is 4 floats of LDS.
+// Block-wide sum over `waves` <= 16 waves; red is 16 floats of LDS.
+__device__ __forceinline__ float block_sum(float v, float* red, int waves) {
+    v = sum64(v);
+    const int w = threadIdx.x >> 6;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[w] = v;
+    __syncthreads();
+    const int i = threadIdx.x & 15;
+    return sum16(i < waves ? red[i] : 0.0f);
+}
+// for blockDim.x = 256 (4 waves)
 __device__ __forceinline__ float block_sum256(float v, float* red) {
     v = sum64(v);
     const int w = threadIdx.x >> 6;

@@ -32,6 +32,19 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_kernel(const Q4KArgs a) 
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB>(a, lds, blockIdx.x);
 }
 
+// The same where a row's blocks are one pass of 1 << LS lane groups, in workgroups of up to ten waves (q4k_one).  What bounds a launch of 14 to 40
+// MB is the order in which a CU's waves get their requests out: a wave that asks for all its blocks at once stands in the queue of the memory path for
+// up to 5 us, x behind the weights of others, and only then starts to stage x.  Here x goes out first (wave priority 3), then EARLY blocks, then
+// the staging (priority 2, in front of other waves' products), then the other blocks; 2.5 blocks of 20 waves, 40 KB a CU, keep HBM busy.  Weights
+// from HBM, in a graph behind a launch that writes x, that launch (2.1 us) included: gate / up 9728 x 2560 12.0 -> 9.6 us, 6144 x 4096 11.7 -> 9.9, q / k / v
+// 6144 x 2560 7.1 -> 6.3, 6144 x 4096 8.5 -> 7.7, o 2560 x 4096 5.7 -> 5.3.
+template <bool XQ8, bool NORM, bool ACC, int MODE, int NB, int LS, int PIECES>
+__global__ __launch_bounds__(64 * Q4K_ONE_WAVES) void q4k_gemv_one_kernel(const Q4KArgs a) {
+    read_now(a.W[0], a.K, a.gamma);
+    extern __shared__ __align__(16) uint8_t lds[];
+    q4k_gemv_body<XQ8, NORM, ACC, MODE, NB, false, false, LS, PIECES, MODE == 1 ? 1 : (NB + 1) / 2>(a, lds, blockIdx.x);
+}
+
 // a workgroup walks several row tiles, every tile one pass of NB blocks per lane group: the passes roll across the tiles
 template <bool XQ8, bool NORM, bool ACC, int MODE, int NB>
 __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArgs a) {
@@ -40,34 +53,28 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_tall_kernel(const Q4KArg
     q4k_gemv_body<XQ8, NORM, ACC, MODE, NB, true>(a, lds, blockIdx.x);
 }
 
-// Gate / up behind RMSNorm, 5 to 16 waves per CU, K <= 4096: in workgroups of four waves each of them normalises and quantises the whole
-// vector, 300 instructions per wave in front of a tile's 250.  One workgroup per CU shares that work; rows, lanes and sums are those
-// of q4k_gemv_kernel.  Weights from HBM, in a graph: 2816 x 1024 5.50 -> 4.84 us, 6144 x 1536 6.15 -> 5.66, 4096 x 2560 7.00 -> 6.76, 3472 x
-// 3072 6.98 -> 6.74 (from the caches 4.68 -> 3.92, 5.10 -> 4.61, 6.02 -> 5.39).  Its barriers cost more than it saves with more waves (two
-// workgroups of ten, 9728 x 2560: 9.74 -> 10.07) and for q / k / v (6144 x 2560: 5.66 -> 5.80), and where 14 to 16 waves wait for more
-// than 15 MB together: 14752 x 1024 7.38 -> 7.62, 8192 x 2048 7.53 -> 7.88, 8192 x 2560 8.52 -> 9.01, 3968 x 3584 7.72 -> 7.92 (13 waves,
-// 6248 x 2560, 8.22 -> 7.89; 16 waves, 9.4 MB, 4096 x 1024, 6.22 -> 5.56).
-template <int NB, int NX>
-__global__ __launch_bounds__(1024) void q4k_gemv_wide_kernel(const Q4KArgs a) {
-    read_now(a.W[0], a.K, a.gamma, a.pre_h);
-    extern __shared__ __align__(16) uint8_t lds[];
-    q4k_gemv_body<false, true, false, 1, NB, false, false, NX>(a, lds, blockIdx.x);
-}
-
 // Few rows, long rows (a Q4_K down projection: 2560 x 9728, as in the layers of a Q4_K_M file whose ffn_down is Q4_K): with
 // four rows per workgroup, 640 workgroups would each quantise the whole 9728-value activation vector for four rows' worth
-// of weights.  Here a workgroup is `waves` waves of one row each (the row's super-blocks strided over the wave's 8 lane
-// groups, two or three blocks of a group in flight, passes rolling), sized so that the launch is one workgroup per CU (two
-// for 17 to 32 rows per CU): x is quantised once per workgroup, one to three half blocks of 16 values per thread.
-// Block-to-lane assignment and reduction order are those of q4k_gemv_body with 8 lane groups per row, so the result is
-// bit-identical to that kernel's.  Against that kernel: 3584 x 18944 15.2 -> 11.3 us, 4096 x 14336 12.0 -> 9.8,
-// 5120 x 17408 15.9 -> 14.2, 8192 x 28672 31.1 -> 28.1.
+// of weights.  Here a workgroup is blockDim.x / 64 waves of one row each (the row's super-blocks strided over the wave's 8 lane
+// groups), sized so that the launch is one workgroup per CU (two for 17 to 32 rows per CU): x is quantised once per workgroup, up to eight
+// 16-byte pieces per thread.  Of a group's blocks two are requested in front of the staging, three are in flight.  Block-to-lane assignment and
+// reduction order are those of q4k_gemv_body with 8 lane groups per row, so the result is bit-identical to that kernel's.  Against passes
+// of three blocks in a loop, weights from HBM, in a graph with two small launches in front (3.7 us, included): 2560 x 9728 10.6 -> 9.7 us, 4096 x
+// 14336 13.8 -> 12.7, 3584 x 11008 12.0 -> 11.2; two workgroups of eight waves instead of one of 16, 4096 x 14336: 13.4.
+template <bool ACC, int NB, int PIECES>
+__global__ __launch_bounds__(1024) void q4k_gemv_rows_kernel(const Q4KArgs a) {
+    read_now(a.W[0], a.K);
+    extern __shared__ __align__(16) uint8_t lds[];
+    q4k_gemv_body<false, false, ACC, 0, NB, false, false, 3, PIECES, NB < 2 ? NB : 2, NB < 3 ? NB : 3>(a, lds, blockIdx.x);
+}
+
+// The same for rows of more than ten blocks a lane group, or x of more than eight pieces a thread: passes of two blocks, rolling
+// as in q4k_gemv_body.  XL: values of x a thread quantises, by 16
 enum { Q4K_LONGROW_MAX_WAVES = 16 };
-// XL: half blocks of x a thread quantises (rows longer than 16 values per thread: up to three rounds); MAXW: the most waves
-// an instantiation is launched with
-template <bool ACC, int NB, int XL = 1, int MAXW = 12>
-__global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8_t* __restrict__ W, int64_t stride,
-                                                                  const float* __restrict__ x, float* y, int N, int K) {
+template <bool ACC, int XL>
+__global__ __launch_bounds__(64 * Q4K_LONGROW_MAX_WAVES) void q4k_gemv_longrow_kernel(const uint8_t* __restrict__ W, int64_t stride,
+                                                                                       const float* __restrict__ x, float* y, int N, int K) {
+    constexpr int NB = 2;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6, j = lane & 7, sub = lane >> 3;
     const int nblk = K / 256;
@@ -76,9 +83,8 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
     const uint8_t* row = W + (int64_t)(live ? r : N - 1) * stride;
     // activation loads first (range-checked: zeros past the end), then the weights, then the Q8 arithmetic
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(x, K * 4);
-    float4 xv[XL][4];
-#pragma unroll
-    for (int u = 0; u < XL; ++u) q4k_load16(rx, 16 * (tid + nthr * u), xv[u]);
+    float4 xv[4 * XL];
+    q4k_load(rx, tid, nthr, xv);
     issue_order_fence();
     uint4 hdr[NB], qv[NB];
 #pragma unroll
@@ -89,12 +95,9 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
     }
     issue_order_fence();
 #pragma unroll
-    for (int u = 0; u < XL; ++u) {  // lanes t, t ^ 1 share a block: both inside or both outside (nthr is a multiple of 64)
-        const int unit = tid + nthr * u;
-        if (16 * unit < K) q4k_quantize16_store<false>(xv[u], xv[u], 1.0f, 0.0f, unit, lds, K);
-    }
+    for (int u = 0; u < 4 * XL; ++u) q4k_quantize4_store<false>(xv[u], xv[u], 1.0f, 0.0f, tid + nthr * u, lds, K);  // (nthr is a multiple of 64)
     __syncthreads();
-    // passes roll as in q4k_gemv_body: a consumed block's registers are refilled from the next pass at once
+    const Q4KLane ln = q4k_lane(lds, K, j);
     const int nb_max = (nblk + 7) >> 3;
     float acc = 0.0f;
     int i0 = 0;
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             const int b = sub + 8 * (i0 + u);
-            const float t = q4k_block_term(hdr[u], qv[u], lds, K, min(b, nblk - 1), j);
+            const float t = q4k_block_term(hdr[u], qv[u], ln, min(b, nblk - 1));
             acc += b < nblk ? t : 0.0f;
             const uint8_t* p = row + (int64_t)min(sub + 8 * (i0 + NB + u), nblk - 1) * 144;
             hdr[u] = *reinterpret_cast<const uint4*>(p);
@@ -112,7 +115,7 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
         const int b = sub + 8 * (i0 + u);
-        const float t = q4k_block_term(hdr[u], qv[u], lds, K, min(b, nblk - 1), j);
+        const float t = q4k_block_term(hdr[u], qv[u], ln, min(b, nblk - 1));
         acc += b < nblk ? t : 0.0f;
     }
     float p = sum8(acc);
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(64 * MAXW) void q4k_gemv_longrow_kernel(const uint8
     }
 }
 
-// waves per workgroup and half blocks of x per thread of that launch, or waves = 0 when the shape is not one for it.  Up to
+// waves per workgroup and values of x per thread, by 16, of that launch, or waves = 0 when the shape is not one for it.  Up to
 // 16 rows per CU make one workgroup per CU, up to 32 two (each quantises x for itself).
 struct Q4KLongrow { int waves, xl; };
 static Q4KLongrow q4k_longrow_shape(int N, int K) {
@@ -140,33 +143,72 @@ static Q4KLongrow q4k_longrow_shape(int N, int K) {
     return {waves, xl};
 }
 
-template <bool ACC, int NB>
-static int q4k_launch_longrow_nb(const void* W, int64_t stride, const float* x, float* y, int N, int K, Q4KLongrow sh, hipStream_t s) {
-    const dim3 grid((N + sh.waves - 1) / sh.waves), block(64 * sh.waves);
-    const size_t lds = (size_t)q8_bytes(K);
-    const uint8_t* Wb = static_cast<const uint8_t*>(W);
-#define PTM_LR(XL, MAXW) hipLaunchKernelGGL((q4k_gemv_longrow_kernel<ACC, NB, XL, MAXW>), grid, block, lds, s, Wb, stride, x, y, N, K)
-    if (sh.waves <= 12) {
-        if (sh.xl == 1) PTM_LR(1, 12);
-        else if (sh.xl == 2) PTM_LR(2, 12);
-        else PTM_LR(3, 12);
-    } else {
-        if (sh.xl == 1) PTM_LR(1, 16);
-        else if (sh.xl == 2) PTM_LR(2, 16);
-        else PTM_LR(3, 16);
+template <bool ACC, int PIECES>
+static void (*q4k_rows_kernel(int nb))(const Q4KArgs) {
+    switch (nb) {
+        case 2: return q4k_gemv_rows_kernel<ACC, 2, PIECES>;
+        case 3: return q4k_gemv_rows_kernel<ACC, 3, PIECES>;
+        case 4: return q4k_gemv_rows_kernel<ACC, 4, PIECES>;
+        case 5: return q4k_gemv_rows_kernel<ACC, 5, PIECES>;
+        case 6: return q4k_gemv_rows_kernel<ACC, 6, PIECES>;
+        case 7: return q4k_gemv_rows_kernel<ACC, 7, PIECES>;
+        case 8: return q4k_gemv_rows_kernel<ACC, 8, PIECES>;
+        case 9: return q4k_gemv_rows_kernel<ACC, 9, PIECES>;
+        default: return q4k_gemv_rows_kernel<ACC, 10, PIECES>;
     }
+}
+template <bool ACC>
+static int q4k_launch_longrow(const Q4KArgs& a, Q4KLongrow sh, hipStream_t s) {
+    const dim3 grid((a.total_rows + sh.waves - 1) / sh.waves), block(64 * sh.waves);
+    const size_t lds = (size_t)q8_bytes(a.K);
+    const int nb = (a.K / 256 + 7) / 8, pieces = (a.K / 4 + 64 * sh.waves - 1) / (64 * sh.waves);
+    if (nb <= 10 && pieces <= 8 && a.stride < 1ll << 31) {
+        const auto kernel = pieces <= 4 ? q4k_rows_kernel<ACC, 4>(nb) : q4k_rows_kernel<ACC, 8>(nb);
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, a);
+        return launch_status();
+    }
+    const float* x = static_cast<const float*>(a.x);
+#define PTM_LR(XL) hipLaunchKernelGGL((q4k_gemv_longrow_kernel<ACC, XL>), grid, block, lds, s, a.W[0], a.stride, x, a.y[0], a.total_rows, a.K)
+    if (sh.xl == 1) PTM_LR(1);
+    else if (sh.xl == 2) PTM_LR(2);
+    else PTM_LR(3);
 #undef PTM_LR
     return launch_status();
 }
 
-template <bool ACC>
-static int q4k_launch_longrow(const void* W, int64_t stride, const float* x, float* y, int N, int K, Q4KLongrow sh, hipStream_t s) {
-    // blocks in flight per lane group: two; three for workgroups of up to ten waves (2560 x 9728, 10 waves, five blocks per
-    // group: 1 / 2 / 3 / 5 in flight 7.5 / 7.0 / 6.9 / 7.0 us; 2048 x 11008, 8 waves: 2 / 3 in flight 6.6 / 6.2;
-    // 3072 x 8192, 12 waves: 5.9 / 6.5; 3584 x 18944, 14 waves: 1 / 2 / 3 in flight 12.8 / 11.3 / 12.2)
-    const int nb = (K / 256 + 7) / 8;
-    if (nb > 2 && sh.waves <= 10) return q4k_launch_longrow_nb<ACC, 3>(W, stride, x, y, N, K, sh, s);
-    return q4k_launch_longrow_nb<ACC, 2>(W, stride, x, y, N, K, sh, s);
+// How a launch is laid out for q4k_gemv_one_kernel (waves 0: not at all): a row's blocks in one pass of up to five a lane group, the waves of a CU
+// in workgroups of at most ten, which share the staging of x (one of 15 or 16 waves instead of two: 7376 x 1024 6.15 -> 6.45 us, 8192 x 2048 7.9 -> 8.3; of
+// four instead of ten, 9728 x 2560: 9.45 -> 9.9), at most two 16-byte pieces of x a thread.
+struct Q4KOne { int waves, nb, ls, pieces; };
+template <bool XQ8, bool NORM, int MODE>
+static Q4KOne q4k_one(const Q4KArgs& a) {
+    const int nblk = a.K / 256;
+    int ls = a.log2S;
+    // q / k / v: six waves a CU with more blocks each are better than twelve (6144 x 2560: 6.5 -> 6.3 us)
+    if (NORM && MODE == 0 && ls > 1 && (nblk + (1 << (ls - 1)) - 1) >> (ls - 1) <= 5 && (int64_t)a.total_rows << (ls - 1) >= 12288) --ls;
+    const int nb = (nblk + (1 << ls) - 1) >> ls;
+    if (ls < 1 || nb > 5 || a.add_one || a.stride >= 1ll << 31) return {0, 0, 0, 0};
+    const int rows_per_wave = 8 >> ls, total = (a.total_rows + rows_per_wave - 1) / rows_per_wave, per_cu = (total + 255) / 256;
+    const int wgs = (per_cu + Q4K_ONE_WAVES - 1) / Q4K_ONE_WAVES;
+    const int waves = per_cu < 4 ? 4 : (per_cu + wgs - 1) / wgs;
+    const int pieces = ((XQ8 ? (a.K + a.K / 4) / 16 : a.K / 4) + 64 * waves - 1) / (64 * waves);
+    return {pieces <= 2 ? waves : 0, nb, ls, pieces};
+}
+template <bool XQ8, bool NORM, bool ACC, int MODE, int LS, int PIECES>
+static void (*q4k_one_kernel(int nb))(const Q4KArgs) {
+    switch (nb) {
+        case 1: return q4k_gemv_one_kernel<XQ8, NORM, ACC, MODE, 1, LS, PIECES>;
+        case 2: return q4k_gemv_one_kernel<XQ8, NORM, ACC, MODE, 2, LS, PIECES>;
+        case 3: return q4k_gemv_one_kernel<XQ8, NORM, ACC, MODE, 3, LS, PIECES>;
+        case 4: return q4k_gemv_one_kernel<XQ8, NORM, ACC, MODE, 4, LS, PIECES>;
+        default: return q4k_gemv_one_kernel<XQ8, NORM, ACC, MODE, 5, LS, PIECES>;
+    }
+}
+template <bool XQ8, bool NORM, bool ACC, int MODE, int PIECES>
+static void (*q4k_one_kernel(const Q4KOne& o))(const Q4KArgs) {
+    if (o.ls == 1) return q4k_one_kernel<XQ8, NORM, ACC, MODE, 1, PIECES>(o.nb);
+    if (MODE == 1 || o.ls == 2) return q4k_one_kernel<XQ8, NORM, ACC, MODE, 2, PIECES>(o.nb);
+    return q4k_one_kernel<XQ8, NORM, ACC, MODE, MODE == 1 ? 2 : 3, PIECES>(o.nb);
 }
 
 template <bool XQ8, bool NORM, bool ACC, int MODE>
@@ -195,25 +237,13 @@ static int q4k_launch(Q4KArgs& a, hipStream_t s) {
             return launch_status();
         }
     }
-    if constexpr (NORM && MODE == 1) {
-        const int rows_per_wave = 8 >> a.log2S, total = (a.total_rows + rows_per_wave - 1) / rows_per_wave, per_cu = (total + 255) / 256;
-        const int nx = (a.K + 256 * per_cu - 1) / (256 * per_cu);
-        const bool heavy = per_cu > 13 && (int64_t)a.total_rows * (a.K / 256) * 144 > 15000000;
-        // K: the sum of squares is taken from 16 values of each of the first 256 threads (longer vectors: the loop of the four-wave form)
-        if (per_cu >= 5 && per_cu <= 16 && !heavy && nx <= 2 && nb <= 5 && a.K <= 16 * Q4K_THREADS) {
-            const dim3 grid((total + per_cu - 1) / per_cu);
-#define PTM_WIDE(NBV, NXV) hipLaunchKernelGGL((q4k_gemv_wide_kernel<NBV, NXV>), grid, dim3(64 * per_cu), lds, s, a)
-            switch (2 * nb + nx) {
-                case 5: PTM_WIDE(2, 1); break;
-                case 6: PTM_WIDE(2, 2); break;
-                case 7: PTM_WIDE(3, 1); break;
-                case 8: PTM_WIDE(3, 2); break;
-                case 9: PTM_WIDE(4, 1); break;
-                case 10: PTM_WIDE(4, 2); break;
-                case 11: PTM_WIDE(5, 1); break;
-                default: PTM_WIDE(5, 2); break;
-            }
-#undef PTM_WIDE
+    if constexpr ((NORM && !ACC) || (XQ8 && MODE == 0)) {  // the launches of a decode step
+        const Q4KOne o = a.tiles_per_wg == 1 ? q4k_one<XQ8, NORM, MODE>(a) : Q4KOne{};
+        if (o.waves > 0) {
+            a.log2S = o.ls;
+            const int rows = o.waves * (8 >> o.ls);
+            const auto kernel = XQ8 || o.pieces == 2 ? q4k_one_kernel<XQ8, NORM, ACC, MODE, 2>(o) : q4k_one_kernel<XQ8, NORM, ACC, MODE, XQ8 ? 2 : 1>(o);
+            hipLaunchKernelGGL(kernel, dim3((a.total_rows + rows - 1) / rows), dim3(64 * o.waves), lds, s, a);
             return launch_status();
         }
     }
@@ -267,9 +297,7 @@ int q4k_gemv_multi(int n_mat, const void* const* W, float* const* y, const int* 
     if (x_is_q8) return accumulate ? q4k_launch<true, false, true, 0>(a, s) : q4k_launch<true, false, false, 0>(a, s);
     if (n_mat == 1) {
         const Q4KLongrow sh = q4k_longrow_shape(N[0], K);
-        if (sh.waves > 0)
-            return accumulate ? q4k_launch_longrow<true>(W[0], stride, static_cast<const float*>(x), y[0], N[0], K, sh, s)
-                              : q4k_launch_longrow<false>(W[0], stride, static_cast<const float*>(x), y[0], N[0], K, sh, s);
+        if (sh.waves > 0) return accumulate ? q4k_launch_longrow<true>(a, sh, s) : q4k_launch_longrow<false>(a, sh, s);
     }
     return accumulate ? q4k_launch<false, false, true, 0>(a, s) : q4k_launch<false, false, false, 0>(a, s);
 }

@@ -438,6 +438,34 @@ def test_fused_gate_up_silu_norm_of_long_vectors(dev, po, N, K):
     assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[N:] == 5.0)
 
 
+@pytest.mark.parametrize("nq,nk,nv,K", [(300, 41, 7, 256), (1030, 513, 255, 768), (1024, 256, 256, 1024), (2049, 511, 513, 1280), (4096, 1024, 1024, 2560),
+                                        (4091, 1030, 1023, 2304), (3584, 512, 512, 3584), (4096, 1024, 1024, 4096), (701, 300, 20, 5120), (9000, 33, 100, 512)])
+def test_one_pass_projections_vs_oracle(dev, po, nq, nk, nv, K):
+    """Rows of one pass of blocks per lane group: two, four and eight groups a row, one to five blocks a group, the last one there for some groups
+    only, four to ten waves with one or two pieces of x a thread, matrices that meet inside a wave.  RMSNorm + three matrices (bars as above)
+    and Q8 blocks (added to y: the plain result and y, bit for bit)."""
+    r = synth.rng_for(60, nq, K)
+    W = [synth.make_q4k(r, n, K) for n in (nq, nk, nv)]
+    x = (synth.make_x(r, K) * 2.0).astype(np.float32)
+    gam = (1.0 + 0.1 * r.standard_normal(K)).astype(np.float32)
+    y = [torch.full((n + 4,), 5.0, device="cuda") for n in (nq, nk, nv)]
+    ops.launch_q4km_fused_rmsnorm_qkv_gemv(cu(x), cu(gam), *map(cu, W), *y, K, nq, nk, nv, W[0].shape[1], 1e-6, False)
+    q8, xd = torch.empty(ops.q8_bytes(K), dtype=torch.uint8, device="cuda"), cu(x)
+    ops.launch_quantize_q8(xd, q8, K)
+    plain, added = torch.full((nq + 4,), 5.0, device="cuda"), torch.full((nq + 4,), 0.5, device="cuda")
+    ops.launch_q4km_q8_gemv(cu(W[0]), q8, plain, K, nq, W[0].shape[1])
+    ops.launch_q4km_q8_gemv(cu(W[0]), q8, added, K, nq, W[0].shape[1], accumulate=True)
+    torch.cuda.synchronize()
+    xn = po.rmsnorm(x, gam, 1e-6)
+    for w, got in zip(W, y):
+        ref, got = po.gemv(12, w, xn), got.cpu().numpy()
+        err = np.abs(got[:-4].astype(np.float64) - ref) / np.sqrt((ref.astype(np.float64) ** 2).mean())
+        assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[-4:] == 5.0)
+    plain, added = plain.cpu().numpy(), added.cpu().numpy()
+    assert rel_err(plain[:-4], po.gemv(12, W[0], x)) <= GEMV_TOL and np.all(plain[-4:] == 5.0)
+    assert np.array_equal(bits(added[:-4]), bits(np.float32(0.5) + plain[:-4])) and np.all(added[-4:] == 0.5)
+
+
 # ---------------------------------------------------------------------------------------------
 # glue
 # ---------------------------------------------------------------------------------------------
