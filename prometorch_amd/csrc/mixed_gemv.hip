@@ -18,6 +18,48 @@ __global__ __launch_bounds__(256) void rmsnorm_mixed_gemv_kernel(const Q4KArgs a
     else q4k_gemv_body<false, true, false, 0, NB4, false, PRE>(a4, lds, (int)blockIdx.x - n6_wgs);
 }
 
+// The same where rows are one pass of blocks: 1 << L4 lane groups a Q4_K row with NB4 blocks each, 1 << L6 a Q6_K row with NT6, in workgroups of
+// blockDim.x / 64 waves that share the staging of x (mixed_one; why: q4k_gemv_one_kernel).  Weights from HBM, in a graph with two small launches in front (3.7
+// us, included): 5120 + 1024 x 2560 9.4 -> 8.7 us, 5120 + 1024 x 4096 10.3 -> 9.4, 1280 + 256 x 1024 7.6 -> 6.4.
+template <int NB4, int L4, int NT6, int L6, bool PRE>
+__global__ __launch_bounds__(64 * Q4K_ONE_WAVES) void rmsnorm_mixed_one_kernel(const Q4KArgs a4, const Q6KArgs a6, int n6_wgs) {
+    read_now(a4.W[0], a4.K, a6.W, a6.gamma, n6_wgs);
+    extern __shared__ __align__(16) uint8_t lds[];
+    if ((int)blockIdx.x < n6_wgs) q6k_one_body<false, true, PRE, L6, NT6, NT6 < 2 ? NT6 : 2, 2>(a6, lds, blockIdx.x);
+    else q4k_gemv_body<false, true, false, 0, NB4, false, PRE, L4, 2, (NB4 + 1) / 2>(a4, lds, (int)blockIdx.x - n6_wgs);
+}
+
+typedef void (*MixedOneKernel)(const Q4KArgs, const Q6KArgs, int);
+struct MixedOne { MixedOneKernel kernel; int waves, l4, l6; };
+// Two lane groups a Q4_K row, four of more than five blocks or where the launch would have less than three waves per CU; Q6_K rows, fewer and with more
+// arithmetic per byte, one step finer while every group has a block (5120 + 1024 x 4096: 4 / 8 groups 9.4 us, 2 / 4 9.7).  The waves of a CU in
+// workgroups of at most ten, one more each while they don't fit (257 workgroups of seven waves: 9.4 us, 224 of eight 8.8).
+template <bool PRE>
+static MixedOne mixed_one(const Q4KArgs& a4, const Q6KArgs& a6) {
+    const int nblk = a4.K / 256;
+    for (int l4 = 1; l4 <= 2; ++l4) {
+        const int l6 = nblk >= 2 << l4 ? l4 + 1 : l4, nb4 = (nblk + (1 << l4) - 1) >> l4;
+        auto waves_of = [](int rows, int l) { return (rows + (8 >> l) - 1) / (8 >> l); };
+        const int w4 = waves_of(a4.total_rows, l4), w6 = waves_of(a6.N, l6), per_cu = (w4 + w6 + 255) / 256;
+        if (nb4 > 5 || (l4 < 2 && w4 + w6 < 768 && nb4 > 1)) continue;
+        if (nblk < 1 << l4) break;
+        const int wgs = (per_cu + Q4K_ONE_WAVES - 1) / Q4K_ONE_WAVES;
+        int waves = (per_cu + wgs - 1) / wgs;
+        if (waves < 4) waves = 4;
+        while (waves < Q4K_ONE_WAVES && (w4 + waves - 1) / waves + (w6 + waves - 1) / waves > 256 * wgs) ++waves;
+        if (a4.add_one || a4.stride >= 1ll << 31 || a4.K / 4 > 2 * 64 * waves) break;
+        MixedOneKernel k;
+        if (l4 == 1 && l6 == 1) break;
+        if (l4 == 1) k = nb4 == 2 ? rmsnorm_mixed_one_kernel<2, 1, 1, 2, PRE> : nb4 == 3 ? rmsnorm_mixed_one_kernel<3, 1, 2, 2, PRE>
+                       : nb4 == 4 ? rmsnorm_mixed_one_kernel<4, 1, 2, 2, PRE> : rmsnorm_mixed_one_kernel<5, 1, 3, 2, PRE>;
+        else if (l6 == 2) k = nb4 == 1 ? rmsnorm_mixed_one_kernel<1, 2, 1, 2, PRE> : rmsnorm_mixed_one_kernel<2, 2, 2, 2, PRE>;
+        else k = nb4 == 2 ? rmsnorm_mixed_one_kernel<2, 2, 1, 3, PRE> : nb4 == 3 ? rmsnorm_mixed_one_kernel<3, 2, 2, 3, PRE>
+                 : nb4 == 4 ? rmsnorm_mixed_one_kernel<4, 2, 2, 3, PRE> : rmsnorm_mixed_one_kernel<5, 2, 3, 3, PRE>;
+        return {k, waves, l4, l6};
+    }
+    return {nullptr, 0, 0, 0};
+}
+
 template <int NB4, bool PRE>
 static void mixed_launch6(int nb6, dim3 grid, size_t lds, hipStream_t s, const Q4KArgs& a4, const Q6KArgs& a6, int n6) {
     switch (nb6) {
@@ -91,6 +133,13 @@ int rmsnorm_mixed_gemv(int n4, const void* const* W4, float* const* y4, const in
     a4.pre_h = pre_h;
     a4.pre_w = pre_w;
     a4.pre_out = nullptr;  // the Q6_K workgroup 0 stores the sum
+    if (const MixedOne o = pre ? mixed_one<true>(a4, a6) : mixed_one<false>(a4, a6); o.kernel) {
+        a4.log2S = o.l4;
+        a6.log2S = o.l6;
+        const int r4 = o.waves * (8 >> o.l4), r6 = o.waves * (8 >> o.l6), g6 = (N6 + r6 - 1) / r6;
+        hipLaunchKernelGGL(o.kernel, dim3(g6 + (total + r4 - 1) / r4), dim3(64 * o.waves), q6k_x_lds_bytes(K), s, a4, a6, g6);
+        return launch_status();
+    }
     const int n6 = (N6 + (32 >> l6) - 1) / (32 >> l6), n4w = q4k_workgroups(total, a4.log2S);
     const size_t lds = q6k_x_lds_bytes(K);  // the Q6_K body's fp32 x + per-16 sums; Q4_K needs less
     static const int cand6[] = {2, 3, 5};

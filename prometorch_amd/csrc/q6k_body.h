@@ -209,6 +209,106 @@ __device__ __forceinline__ void q6k_gemv_body(const Q6KArgs a, uint8_t* lds_raw,
     }
 }
 
+// Rows whose blocks are NT per lane group (1 << LS groups a row), in workgroups of blockDim.x / 64 waves that share the staging of x (PIECES 16-byte pieces
+// a thread, add_one == 0).  What the waves of a CU ask for goes out in an order: x at raised priority and the old y, one block, x to LDS (in
+// front of other waves' products), then up to DEPTH blocks in flight (see q4k_gemv_one_kernel).  Blocks, lanes and sums are those of q6k_gemv_body.
+template <bool ACC, bool NORM, bool PRE, int LS, int NT, int DEPTH, int PIECES>
+__device__ __forceinline__ void q6k_one_body(const Q6KArgs a, uint8_t* lds_raw, int wg) {
+    static_assert(!PRE || NORM, "the deferred post-norm comes with the RMSNorm prologue");
+    constexpr int S = 1 << LS, ROWS = 8 >> LS;
+    float* xf = reinterpret_cast<float*>(lds_raw);
+    float* xsum16 = xf + q6k_x_floats(a.K);
+    __shared__ float red[16];
+    const int tid = threadIdx.x, threads = blockDim.x, waves = threads >> 6, n4 = a.K / 4, nblk = a.K / 256;
+    const int lane = tid & 63, wave = tid >> 6, j = lane & 7, grp = lane >> 3, sub = grp & (S - 1);
+    const int r = (wg * waves + wave) * ROWS + (grp >> LS);
+    const bool live = r < a.N;
+    const int rr = live ? r : a.N - 1;
+    const int qh_off = 128 + 32 * (j >> 2) + 16 * (j & 1);
+    const int sc_off = 192 + 8 * (j >> 2) + 2 * ((j & 3) >> 1) + (j & 1);
+    auto load = [&](const float* p, float4 (&v)[PIECES]) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p, a.K * 4);  // zeros past the end
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, (tid + threads * u) * 16, 0, 0);
+            v[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
+        }
+    };
+    auto squares = [&](const float4 (&v)[PIECES]) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) ss = fmaf(v[u].w, v[u].w, fmaf(v[u].z, v[u].z, fmaf(v[u].y, v[u].y, fmaf(v[u].x, v[u].x, ss))));
+        return block_sum(ss, red, waves);
+    };
+    __builtin_amdgcn_s_setprio(3);
+    float4 x[PIECES], g[PIECES], h[PIECES], w[PIECES];
+    if constexpr (PRE) {
+        load(a.pre_h, h);
+        load(a.pre_w, w);
+    }
+    load(a.x, x);
+    if constexpr (NORM) load(a.gamma, g);
+    float y_old = 0.0f;
+    if constexpr (ACC) y_old = a.y[rr];
+    issue_order_fence();
+    __builtin_amdgcn_s_setprio(0);
+    const uint8_t* row = a.W + (int64_t)rr * a.stride;
+    const uint8_t* first = row + sub * 210;
+    const uint8_t* last = row + min(sub + S * (NT - 1), nblk - 1) * 210;
+    Q6Blk blk[DEPTH];
+    auto request = [&](int u) { blk[u % DEPTH] = q6k_load(u < NT - 1 ? first + S * u * 210 : last, j, qh_off, sc_off); };
+    request(0);
+    issue_order_fence();
+    __builtin_amdgcn_s_setprio(2);
+    float rs = 1.0f;
+    if constexpr (PRE) {
+        const float rsh = 1.0f / sqrtf(squares(h) / (float)a.K + a.eps);
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            x[u].x += h[u].x * rsh * w[u].x;
+            x[u].y += h[u].y * rsh * w[u].y;
+            x[u].z += h[u].z * rsh * w[u].z;
+            x[u].w += h[u].w * rsh * w[u].w;
+            const int i = tid + threads * u;
+            if (wg == 0 && a.pre_out && i < n4) reinterpret_cast<float4*>(a.pre_out)[i] = x[u];
+        }
+    }
+    if constexpr (NORM) rs = 1.0f / sqrtf(squares(x) / (float)a.K + a.eps);
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u) {
+        const int i = tid + threads * u;
+        if (i >= n4) break;  // whole waves: K is a multiple of 256
+        float4 v = x[u];
+        if constexpr (NORM) v = make_float4(v.x * rs * g[u].x, v.y * rs * g[u].y, v.z * rs * g[u].z, v.w * rs * g[u].w);
+        reinterpret_cast<float4*>(xf)[q6k_xslot(i)] = v;
+        float sm = (v.x + v.y) + (v.z + v.w);
+        sm += dpp_f<0xB1>(sm);
+        sm += dpp_f<0x4E>(sm);
+        if ((tid & 3) == 0) xsum16[i >> 2] = sm;
+    }
+    __syncthreads();
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int u = 1; u < DEPTH; ++u) request(u);
+    issue_order_fence();
+    float acc = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+        const int b = sub + S * u;
+        const float t = q6k_block_term(blk[u % DEPTH], xf, xsum16, u < NT - 1 ? b : min(b, nblk - 1), j);
+        acc += u < NT - 1 || b < nblk ? t : 0.0f;
+        if (u + DEPTH < NT) {
+            request(u + DEPTH);
+            issue_order_fence();
+        }
+    }
+    float p = sum8(acc);
+    if (S >= 2) p += dpp_f<0x128>(p);
+    if (S >= 4) p = add16(p);
+    if (S >= 8) p = add32(p);
+    if (live && sub == 0 && j == 0) a.y[rr] = ACC ? y_old + p : p;
+}
+
 // Lane groups per row: the fewest that still give the chip enough workgroups, with a group's blocks in at most two
 // rolling passes (the vocabulary projection 151936 x 2560 then runs one group per row, two passes of 5 blocks:
 // 94 -> 88 us with the argmax against two groups per row and one pass, for half the stagings of x).

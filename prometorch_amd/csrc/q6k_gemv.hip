@@ -34,10 +34,23 @@ __global__ __launch_bounds__(Q6K_THREADS) __attribute__((amdgpu_waves_per_eu(3, 
     q6k_mfma_gemv_body<ACC, ARGMAX, NORM, XL, NB>(a, lds_raw);
 }
 
-// Few rows, long rows (a down projection: 2560 x 9728, 4096 x 14336): with 4 rows per workgroup every workgroup
+// Up to 16 rows per CU (down projections): a row per wave, its super-blocks strided over the wave's 8 lane groups, NT of them a group, one workgroup
+// per CU, so that x is staged once per CU instead of once per 4 rows.  Two blocks of a group in flight, one of them requested in front of the
+// staging (2560 x 9728 with one / two / three: 12.0 / 11.4 / 12.2 us).  Against passes in a loop, which pad the last one, weights from HBM, in a
+// graph with two small launches in front (3.7 us, included): 2560 x 9728 11.7 -> 11.4 us, 4096 x 14336 (eight waves of two rows) 17.1 -> 16.0, 1024 x 2816
+// (four rows a workgroup) 7.2 -> 6.9.
+enum { Q6K_ROWS_MAX_WAVES = 16 };
+template <bool ACC, int NT, int PIECES>
+__global__ __launch_bounds__(64 * Q6K_ROWS_MAX_WAVES) void q6k_gemv_rows_kernel(const Q6KArgs a) {
+    read_now(a.W, a.K);
+    extern __shared__ __align__(16) uint8_t lds_raw[];
+    q6k_one_body<ACC, false, false, 3, NT, NT < 2 ? NT : 2, PIECES>(a, lds_raw, blockIdx.x);
+}
+
+// The same for rows that kernel has not (17 to 32 a CU, more than 20480 values): with 4 rows per workgroup every workgroup
 // would stage the whole activation vector for 4 rows' worth of weights, and the staging traffic through L2 would
 // exceed the weights'.  Here a workgroup is `waves` waves of 8 >> LOG2S rows each (a row's super-blocks strided over
-// 1 << LOG2S lane groups), sized so that the launch is one workgroup per CU: x is staged once per CU.
+// 1 << LOG2S lane groups), sized so that the launch is one workgroup per CU.
 // XL = float4 loads of x per thread.
 enum { Q6K_TALL_MAX_WAVES = 16 };
 // XMORE: rows of more than XL float4 per thread are staged in further rounds of loads (its own instantiation: the loop's
@@ -139,10 +152,8 @@ __global__ __launch_bounds__(64 * MAXW) void q6k_gemv_tall_kernel(const Q6KArgs 
 }
 
 // Shape of a tall launch: waves per workgroup and lane groups per row, or waves = 0 when the shape is not one for
-// it.  Rows that fill the chip once at one workgroup per CU: 8 lane groups per row while that needs at most 16 waves
-// (2560 x 9728: 10 waves; 3584 x 18944, the down projection of a 7B model: 14 waves - on the four-row kernel, where 896
-// workgroups each staged 76 KB of x, that launch took 33 us), else 4 groups per row and two rows per wave
-// (4096 x 14336: 8 waves of 2 rows).
+// it.  Rows that fill the chip once at one workgroup per CU: 8 lane groups per row while that needs at most 16 waves, else 4 groups
+// per row and two rows per wave (3584 x 18944 on the four-row kernel, where 896 workgroups each staged 76 KB of x: 33 us).
 struct Q6KTall { int waves, log2S; };
 inline Q6KTall q6k_tall_shape(int N, int K) {
     if (K < 4096 || K > 32768) return {0, 0};   // x and its sums in LDS: 4.4 bytes per value, at most 141 KB
@@ -178,7 +189,7 @@ static int q6k_launch_tall_nb(const Q6KArgs& a, int waves, hipStream_t s) {
     if (waves > 12) {
         if (xl <= 8) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, false, 16>), dim3(grid), dim3(64 * waves), lds, s, a);
         else hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, true, 16>), dim3(grid), dim3(64 * waves), lds, s, a);
-    } else if (xl <= 4) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 4, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
+    } else if (LOG2S == 2 && xl <= 4) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, LOG2S == 2 ? 4 : 8, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
     else if (xl <= 8) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
     else hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, true>), dim3(grid), dim3(64 * waves), lds, s, a);
     return launch_status();
@@ -272,9 +283,9 @@ static void q6k_raise_lds_cap() {
 template <bool ACC, int LOG2S>
 static void q6k_raise_lds_cap_tall() {
     const int cap = 144 * 1024;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 4, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, LOG2S == 2 ? 4 : 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 4, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, LOG2S == 2 ? 4 : 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 8, LOG2S, true>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S, true>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
@@ -282,6 +293,14 @@ static void q6k_raise_lds_cap_tall() {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S, false, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 8, LOG2S, true, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S, true, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+}
+// (seven blocks a lane group: rows of up to 14336 values, which 64 KB hold)
+template <bool ACC, int PIECES>
+static void q6k_raise_lds_cap_rows() {
+    const int cap = 144 * 1024;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_rows_kernel<ACC, 8, PIECES>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_rows_kernel<ACC, 9, PIECES>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_rows_kernel<ACC, 10, PIECES>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
 }
 template <bool ACC, bool ARGMAX, bool NORM, int XCH>
 static void q6k_raise_lds_cap_nb() {
@@ -301,6 +320,10 @@ void q6k_init_attributes() {
     q6k_raise_lds_cap_nb<false, true, false, 1>();
     q6k_raise_lds_cap_nb<false, true, true, 1>();
     q6k_raise_lds_cap_nb<false, false, true, 1>();
+    q6k_raise_lds_cap_rows<false, 4>();
+    q6k_raise_lds_cap_rows<false, 8>();
+    q6k_raise_lds_cap_rows<true, 4>();
+    q6k_raise_lds_cap_rows<true, 8>();
     q6k_raise_lds_cap_tall<false, 2>();
     q6k_raise_lds_cap_tall<false, 3>();
     q6k_raise_lds_cap_tall<true, 2>();
@@ -342,6 +365,27 @@ static int q6k_launch_mfma(const Q6KArgs& a, hipStream_t s) {
     return launch_status();
 }
 
+template <bool ACC, int PIECES>
+static void (*q6k_rows_kernel(int nt))(const Q6KArgs) {
+    switch (nt) {
+        case 1: return q6k_gemv_rows_kernel<ACC, 1, PIECES>;
+        case 2: return q6k_gemv_rows_kernel<ACC, 2, PIECES>;
+        case 3: return q6k_gemv_rows_kernel<ACC, 3, PIECES>;
+        case 4: return q6k_gemv_rows_kernel<ACC, 4, PIECES>;
+        case 5: return q6k_gemv_rows_kernel<ACC, 5, PIECES>;
+        case 6: return q6k_gemv_rows_kernel<ACC, 6, PIECES>;
+        case 7: return q6k_gemv_rows_kernel<ACC, 7, PIECES>;
+        case 8: return q6k_gemv_rows_kernel<ACC, 8, PIECES>;
+        case 9: return q6k_gemv_rows_kernel<ACC, 9, PIECES>;
+        default: return q6k_gemv_rows_kernel<ACC, 10, PIECES>;
+    }
+}
+// the waves of that launch, 0 where rows or blocks are too many or a thread would have more than eight pieces of x
+static int q6k_rows_waves(int N, int K) {
+    const int per_cu = (N + 255) / 256, waves = per_cu < 2 ? 2 : per_cu;
+    return per_cu <= Q6K_ROWS_MAX_WAVES && K <= 10 * 8 * 256 && (K / 4 + 64 * waves - 1) / (64 * waves) <= 8 ? waves : 0;
+}
+
 template <bool ACC, bool ARGMAX, bool NORM>
 static int q6k_launch(Q6KArgs& a, hipStream_t s) {
     if (q6k_mfma_shape(a.N, a.K)) return q6k_launch_mfma<ACC, ARGMAX, NORM>(a, s);
@@ -349,6 +393,13 @@ static int q6k_launch(Q6KArgs& a, hipStream_t s) {
     const int grid = q6k_workgroups(a.N, a.K);
     const size_t lds = q6k_x_lds_bytes(a.K);
     if constexpr (!ARGMAX && !NORM) {
+        if (const int waves = q6k_rows_waves(a.N, a.K)) {
+            if (lds > 64 * 1024) q6k_init_attributes();
+            const int nt = (a.K / 256 + 7) / 8;
+            const auto kernel = a.K / 4 <= 4 * 64 * waves ? q6k_rows_kernel<ACC, 4>(nt) : q6k_rows_kernel<ACC, 8>(nt);
+            hipLaunchKernelGGL(kernel, dim3((a.N + waves - 1) / waves), dim3(64 * waves), lds, s, a);
+            return launch_status();
+        }
         const Q6KTall tall = q6k_tall_shape(a.N, a.K);
         if (tall.waves > 0)
             return tall.log2S == 3 ? q6k_launch_tall<ACC, 3>(a, tall.waves, s) : q6k_launch_tall<ACC, 2>(a, tall.waves, s);

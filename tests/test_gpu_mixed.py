@@ -252,3 +252,22 @@ def test_random_architectures_decode_and_prefill_vs_oracle(dev, po, seed):
     print("logit err/std", np.array2string(errs, precision=2), flush=True)
     assert errs.max() <= LOGIT_TOL_FLIP and np.median(errs) <= LOGIT_TOL, errs
     dec.close()
+
+
+@pytest.mark.parametrize("hidden,heads,kv_heads,inter", [(512, 4, 1, 768), (768, 8, 1, 2816), (1024, 20, 4, 2816), (1280, 12, 12, 512), (1792, 16, 2, 768),
+                                                         (2304, 40, 8, 1024), (2560, 64, 16, 512), (4096, 64, 16, 512), (5120, 12, 4, 256), (5376, 4, 2, 256)])
+def test_widths_of_the_mixed_launch(dev, po, seeds, hidden, heads, kv_heads, inter):
+    """RMSNorm + q, k (Q4_K) + v (Q6_K) where rows are one pass of two or four lane groups (one to five blocks a group, the last not there for every
+    group; Q6_K rows as many groups or twice as many; a workgroup's last rows past the end) and either side of it, and down projections of one to
+    eleven blocks, against the oracle: two layers, three steps.  A wrong row or block is an error of order 1; the bar is that of a step with an
+    activation on a Q8 rounding boundary."""
+    from prometorch_amd.decode import Decoder
+    cfg = dict(synth.TINY, hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, inter=inter)
+    layers, head = [synth.make_layer(seeds["tiny"], i, cfg) for i in range(2)], synth.make_head(seeds["tiny"], cfg)
+    om = po.OracleModel(cfg, layers, head, 64, kv_fp16=True)
+    dec = Decoder(cfg, layers, head, max_seq=64, kv_fp16=True, use_graph=True)
+    for st in range(3):
+        om.step(synth.MIXED_FEED[st])
+        dec.step(synth.MIXED_FEED[st])
+        assert np.abs(dec.logits() - om.logits).max() <= LOGIT_TOL_FLIP * om.logits.std(), st
+    dec.close()

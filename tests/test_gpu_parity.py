@@ -244,6 +244,18 @@ def test_gemv_shapes_vs_oracle(dev, po, qt, N, K):
     assert e <= GEMV_TOL
 
 
+@pytest.mark.parametrize("N,K", [(3, 512), (257, 2048), (1024, 2816), (2560, 9728), (4096, 14336), (4095, 4352), (3584, 18944), (2000, 20480), (2000, 20736),
+                                 (4097, 2304)])
+def test_q6k_rows_vs_oracle(dev, po, N, K):
+    """A row per wave (up to 16 rows per CU, one to ten blocks a lane group, the last not there for every group; four or eight pieces of x a thread, two
+    waves at least) and one row or block more: plain, and added to y bit for bit."""
+    r = synth.rng_for(61, N, K)
+    W, x, y0 = synth.make_q6k(r, N, K), synth.make_x(r, K), synth.make_x(r, N)
+    y = gpu_gemv(14, W, x)
+    assert rel_err(y, po.gemv(14, W, x)) <= GEMV_TOL
+    assert np.array_equal(bits(gpu_gemv(14, W, x, accumulate=True, y0=y0)), bits(y0 + y))
+
+
 def test_gemv_ragged_vs_reference_golden(dev, golden, seeds):
     rr = synth.rng_for(seeds["ragged"])
     for i, (qt, N, K) in enumerate([(12, 33, 512), (12, 1, 256), (12, 77, 2560), (14, 7, 256), (14, 45, 1024)]):
