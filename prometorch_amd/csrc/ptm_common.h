@@ -222,7 +222,7 @@ __device__ __forceinline__ uint32_t q8_quantize4(float4 v, float& d, float& sum)
 }
 
 // Block-wide sum over `waves` <= 16 waves; red is 16 floats of LDS.
-__device__ __forceinline__ float block_sum(float v, float* red, int waves) {
+__device__ __forceinline__ float sum_of_waves(float v, float* red, int waves) {
     v = sum64(v);
     const int w = threadIdx.x >> 6;
     __syncthreads();

@@ -109,7 +109,7 @@ __device__ __forceinline__ Q4KStage<NX> q4k_stage_issue(const Q4KArgs a, uint8_t
                     q4k_load(rx, base + tid, threads, t);
                     ss = q4k_sumsq(t, ss);
                 }
-                ss = block_sum(ss, red, threads >> 6);
+                ss = sum_of_waves(ss, red, threads >> 6);
                 st.rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
             }
             for (int base = NX * threads; 4 * base < a.K; base += 4 * threads) {
@@ -145,7 +145,7 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q
         }
     } else if constexpr (PRE) {
         // x + RMSNorm(h) * w first (threads past the end hold zeros), then the kernel's own RMSNorm of that sum
-        const float ssh = block_sum(q4k_sumsq(st.h, 0.0f), red, threads >> 6);
+        const float ssh = sum_of_waves(q4k_sumsq(st.h, 0.0f), red, threads >> 6);
         const float rsh = 1.0f / sqrtf(ssh / (float)a.K + a.eps);
         float4 xv[NX];
 #pragma unroll
@@ -160,7 +160,7 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q
             for (int u = 0; u < NX; ++u)
                 if (4 * (tid + threads * u) < a.K) reinterpret_cast<float4*>(a.pre_out)[tid + threads * u] = xv[u];
         }
-        const float ss = block_sum(q4k_sumsq(xv, 0.0f), red, threads >> 6);
+        const float ss = sum_of_waves(q4k_sumsq(xv, 0.0f), red, threads >> 6);
         const float rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
 #pragma unroll
         for (int u = 0; u < NX; ++u) q4k_quantize4_store<true>(xv[u], st.g[u], rs, one, tid + threads * u, lds, a.K);
@@ -168,7 +168,7 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q
         float rs = st.rs;
         if constexpr (NORM) {
             if (SHORT || a.K <= 4 * NX * threads) {
-                const float ss = block_sum(q4k_sumsq(st.x, 0.0f), red, threads >> 6);
+                const float ss = sum_of_waves(q4k_sumsq(st.x, 0.0f), red, threads >> 6);
                 rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
             }
         }

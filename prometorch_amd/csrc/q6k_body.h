@@ -238,7 +238,7 @@ __device__ __forceinline__ void q6k_one_body(const Q6KArgs a, uint8_t* lds_raw, 
         float ss = 0.0f;
 #pragma unroll
         for (int u = 0; u < PIECES; ++u) ss = fmaf(v[u].w, v[u].w, fmaf(v[u].z, v[u].z, fmaf(v[u].y, v[u].y, fmaf(v[u].x, v[u].x, ss))));
-        return block_sum(ss, red, waves);
+        return sum_of_waves(ss, red, waves);
     };
     __builtin_amdgcn_s_setprio(3);
     float4 x[PIECES], g[PIECES], h[PIECES], w[PIECES];
