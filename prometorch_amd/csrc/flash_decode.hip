@@ -331,18 +331,17 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
                                                                         const float* __restrict__ pM, float* __restrict__ O,
                                                                         int n_heads, const int64_t* __restrict__ d_past,
                                                                         int64_t past_host, int max_seq,
-                                                                        uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
+                                                                        uint8_t* __restrict__ q8_out, int chunk_arg, int log2_units) {
     constexpr int NOUT = HD / 4;
     const int h = blockIdx.x, lane = threadIdx.x & 63, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
     const float4* pO4 = reinterpret_cast<const float4*>(pO);
     // Every load of the common case goes out before the position is known: chunk slots past the last active one
     // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the first wave makes one
     // memory round trip, not one for the position and a second for the data; the others are there for long contexts only.
-    // chunk_shift < 0: the partials of the looping kernel (at most FD_LONG_SPLITS of them, cpw chunks of 64 positions each)
-    const bool long_mode = chunk_shift < 0;
-    const int chunk = long_mode ? FD_CHUNK : 1 << chunk_shift;  // positions per chunk
-    const int cs_ = long_mode ? 6 : chunk_shift;
-    const int ns_max = long_mode ? min((max_seq + chunk - 1) >> cs_, (int)FD_LONG_SPLITS) : (max_seq + chunk - 1) >> cs_;
+    // chunk < 0: the partials of the looping kernel (at most FD_LONG_SPLITS of them, cpw chunks of 64 positions each)
+    const bool long_mode = chunk_arg < 0;
+    const int chunk = long_mode ? (int)FD_CHUNK : chunk_arg;  // positions per chunk
+    const int ns_max = long_mode ? min((max_seq + chunk - 1) / chunk, (int)FD_LONG_SPLITS) : (max_seq + chunk - 1) / chunk;
     const int64_t past = d_past ? *d_past : past_host;
     // partial maxima are natural-log scores, or base-2 ones (log2_units) from the matrix-core kernel
     const float ek = log2_units ? 1.0f : 1.44269504088896340736f;
@@ -372,7 +371,7 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
     int64_t total = past + 1;
     if (total > max_seq) total = max_seq;
     if (total <= 0) return;
-    const int n_chunks = (int)((total + chunk - 1) >> cs_);
+    const int n_chunks = ((int)total + chunk - 1) / chunk;
     const int cpw_ = long_mode ? (n_chunks + (int)FD_LONG_SPLITS - 1) / (int)FD_LONG_SPLITS : 1;
     const int ns = long_mode ? (n_chunks + cpw_ - 1) / cpw_ : n_chunks;
     const bool together = WAVES > 1 && ns > 64;  // the same in every thread
@@ -443,17 +442,16 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
 
 template <int HD, int WAVES>
 static void fd_merge_launch(int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O, const int64_t* d_past,
-                            int64_t past_host, int max_seq, uint8_t* q8_out, int chunk_shift, int log2_units) {
+                            int64_t past_host, int max_seq, uint8_t* q8_out, int chunk_arg, int log2_units) {
     hipLaunchKernelGGL((flash_decode_merge_kernel<HD, WAVES>), dim3(n_heads, HD / 32), dim3(64 * WAVES), 0, s, pO, pL, pM, O, n_heads, d_past,
-                       past_host, max_seq, q8_out, chunk_shift, log2_units);
+                       past_host, max_seq, q8_out, chunk_arg, log2_units);
 }
 
 static int fd_merge(int head_dim, int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O,
                     const int64_t* d_past, int max_seq, uint8_t* q8_out = nullptr, int64_t past_host = 0,
                     int chunk = FD_CHUNK, int log2_units = 0) {
-    const int chunk_shift = chunk < 0 ? -1 : chunk == 128 ? 7 : 6;
-    const int most = chunk_shift < 0 ? (int)FD_LONG_SPLITS : (int)(((int64_t)max_seq + chunk - 1) >> chunk_shift);  // splits there can be
-#define PTM_FDM(HDV, WV) fd_merge_launch<HDV, WV>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units)
+    const int most = chunk < 0 ? (int)FD_LONG_SPLITS : (int)(((int64_t)max_seq + chunk - 1) / chunk);  // splits there can be
+#define PTM_FDM(HDV, WV) fd_merge_launch<HDV, WV>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, chunk, log2_units)
 #define PTM_FDMW(HDV) (most <= 64 ? PTM_FDM(HDV, 1) : PTM_FDM(HDV, 4))
     if (head_dim == 256) PTM_FDMW(256);
     else if (head_dim == 128) PTM_FDMW(128);
@@ -1163,20 +1161,25 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(const Attn
         }
         return;
     }
-    // ---- merge the four wave partials into the chunk's partial ----
-    static_assert(ONE || WAVES == 4, "the merge below");
-    for (int e = tid; e < G * HD; e += FD_THREADS) {
+    // ---- merge the wave partials into the chunk's partial ----
+    for (int e = tid; e < G * HD; e += 64 * WAVES) {
         const int g = e / HD, d = e % HD;
-        const float m0 = s_m[0][g], m1 = s_m[1][g], m2 = s_m[2][g], m3 = s_m[3][g];
-        const float M = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));  // finite: the chunk holds at least one valid position
-        const float w0 = __builtin_amdgcn_exp2f(m0 - M), w1 = __builtin_amdgcn_exp2f(m1 - M),
-                    w2 = __builtin_amdgcn_exp2f(m2 - M), w3 = __builtin_amdgcn_exp2f(m3 - M);
-        const float o = (w0 * s_o[0][d][g] + w1 * s_o[1][d][g]) + (w2 * s_o[2][d][g] + w3 * s_o[3][d][g]);
+        float mw[WAVES], w[WAVES], M = -INFINITY;  // finite in the end: the chunk holds at least one valid position
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) M = fmaxf(M, mw[i] = s_m[i][g]);
+        float o = 0.0f, l = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) {
+            w[i] = __builtin_amdgcn_exp2f(mw[i] - M);
+            o += w[i] * s_o[i][d][g];
+        }
         const int64_t oi = (int64_t)split * a.n_heads + kvh * G + g;
         a.pO[oi * HD + d] = o;
         if (d == 0) {
+#pragma unroll
+            for (int i = 0; i < WAVES; ++i) l += w[i] * s_l[i][g];
             a.pM[oi] = M;
-            a.pL[oi] = (w0 * s_l[0][g] + w1 * s_l[1][g]) + (w2 * s_l[2][g] + w3 * s_l[3][g]);
+            a.pL[oi] = l;
         }
     }
 }
@@ -1680,6 +1683,17 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
             if (rc != PTM_OK) return rc;
             return fd_merge(head_dim, n_heads, s, partial_O, partial_lse, partial_max, O, d_past_len, max_seq,
                             static_cast<uint8_t*>(o_q8), 0, -1, 1);
+        }
+        // Chunks of 80 positions, five waves, where those of 64 make a few workgroups more than the chip has CUs: a CU's L1 returns what was asked of it
+        // in order, and a second workgroup's query, rotation row and keys come behind the rows of the first, 0.8 us of the launch's 3.9 behind its
+        // arguments.  Eight steps of Qwen3-4B shapes at 2048 positions (264 workgroups of four waves, 208 of five) 9835 -> 9705 us; six waves 9750,
+        // eight 9825.
+        const int wide = (max_seq + 79) / 80;
+        if (head_dim == 128 && (int)grid.x * n_kv_heads > 256 && wide * n_kv_heads <= 256) {
+            const dim3 grid5(wide, n_kv_heads);
+            rc = bias ? attn_mfma_launch_g<128, 1, true, 5>(G, grid5, s, a) : attn_mfma_launch_g<128, 1, false, 5>(G, grid5, s, a);
+            if (rc != PTM_OK) return rc;
+            return fd_merge(head_dim, n_heads, s, partial_O, partial_lse, partial_max, O, d_past_len, max_seq, static_cast<uint8_t*>(o_q8), 0, 80, 1);
         }
         if (bias) rc = head_dim == 128 ? attn_mfma_launch_g<128, 1, true>(G, grid, s, a) : attn_mfma_launch_g<64, 1, true>(G, grid, s, a);
         else rc = head_dim == 128 ? attn_mfma_launch_g<128, 1, false>(G, grid, s, a) : attn_mfma_launch_g<64, 1, false>(G, grid, s, a);

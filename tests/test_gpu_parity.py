@@ -735,6 +735,13 @@ def test_attn_decode_fused_vs_oracle(dev, po, kv_fp16, nh, nkv, hd, past):
         kf[pos] = krow                                               # continue from what the cache really holds
 
 
+@pytest.mark.parametrize("nh,nkv,past", [(8, 8, 1998), (24, 8, 2077), (40, 8, 2156), (64, 8, 2239), (56, 8, 2398), (36, 9, 1840)])
+def test_attn_decode_five_waves_vs_oracle(dev, po, nh, nkv, past):
+    """Caches whose chunks of 64 would be more than 256 workgroups and those of 80 are not: three tokens over the ends of a wave's 16 positions and of a
+    chunk, one to eight query heads per kv head."""
+    test_attn_decode_fused_vs_oracle(dev, po, True, nh, nkv, 128, past)
+
+
 @pytest.mark.parametrize("N,K,accumulate", [(2500, 9728, True), (300, 4096, False), (77, 14336, True), (3000, 6912, False),
                                             (4096, 14336, True), (3300, 8192, False), (5119, 13824, False),  # two rows per wave
                                             # rows beyond 14336 values (more than 64 KB of LDS), 13 to 16 waves per workgroup
