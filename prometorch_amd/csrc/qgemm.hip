@@ -759,42 +759,57 @@ struct Q6Tile {  // Q6_K: the lane's 16 bytes of ql for each (half, pair), of qh
 
 // Where a workgroup's accumulators go.
 // C layout of the 32x32 tile: column j = lane % 32, rows 8 (r / 4) + 4 (lane / 32) + r % 4.  The row scales come from
-// LDS (staged in the prologue), and when accumulating the 16 old values of a tile are fetched together before its 16
+// LDS (staged in the prologue) four at a time, and a value's place is the lane's first plus rows that are the same for the wave: 64-bit products
+// per value, each behind its own read of a scale and its own branches, were 42 instructions and a wait where this has three (EDGE: six).
+// ADD: the 16 old values of a tile are fetched together before its 16
 // stores: a load issued behind a store the compiler cannot tell apart from it is one serial memory round trip per value,
 // more than the main loop of a launch with few blocks per workgroup takes.
-template <int MT>
-__device__ __forceinline__ void qf_store(const f32x16 (&acc)[MT], const float* s_rs, float* Y, float* partials, int accumulate, int M, int N, int m0, int n_base,
-                                         int j, int kh, int bz) {
-    const int n = n_base + j;
-    const bool n_ok = n < N;
-    const int nc = n_ok ? n : N - 1;
+// p: the lane's column in row m0 + 4 kh, `left` rows from there on; rows: M < m0 + 32 MT or N within the workgroup's columns (EDGE).
+// Few rows' sums are read by the next kernel from the caches, where plain stores leave them (19 rows of 36 layers 2823 -> 2749 us); many
+// rows' pass by them (509 rows: 8353 us plain, 8248 so).
+template <int MT, bool EDGE, bool ADD>
+__device__ __forceinline__ void qf_store_rows(const f32x16 (&acc)[MT], const float* s_rs, float* p, int N, int left, bool n_ok, int kh) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
+        float4 sc[4];
         float old[16];
-        if (!partials && accumulate) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sc[q] = *reinterpret_cast<const float4*>(s_rs + 32 * mt + 8 * q + 4 * kh);
+        if constexpr (ADD) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m = min(m0 + mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), M - 1);
-                old[r] = Y[(int64_t)m * N + nc];
+                const int row = 32 * mt + 8 * (r >> 2) + (r & 3);
+                old[r] = p[(int64_t)(EDGE ? min(row, left - 1) : row) * N];
             }
             issue_order_fence();
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) old[r] = 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int lr = mt * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            const int m = m0 + lr;
-            const float v = acc[mt][r] * s_rs[lr];
-            if (m < M && n_ok) {
-                if (partials) __builtin_nontemporal_store(v, &partials[((int64_t)bz * M + m) * N + n]);
-                else __builtin_nontemporal_store(accumulate ? old[r] + v : v, &Y[(int64_t)m * N + n]);
+            const int row = 32 * mt + 8 * (r >> 2) + (r & 3);
+            const float4 s4 = sc[r >> 2];
+            float v = acc[mt][r] * ((r & 3) == 0 ? s4.x : (r & 3) == 1 ? s4.y : (r & 3) == 2 ? s4.z : s4.w);
+            if constexpr (ADD) v = old[r] + v;
+            if (!EDGE || (row < left && n_ok)) {
+                if constexpr (MT == 1) p[(int64_t)row * N] = v;
+                else __builtin_nontemporal_store(v, &p[(int64_t)row * N]);
             }
         }
     }
 }
-
+template <int MT>
+__device__ __forceinline__ void qf_store(const f32x16 (&acc)[MT], const float* s_rs, float* Y, float* partials, int accumulate, int M, int N, int m0, int n_base,
+                                         int j, int kh, int bz) {
+    const int n = n_base + j, left = M - m0 - 4 * kh;
+    float* p = (partials ? partials + (int64_t)bz * M * N : Y) + (int64_t)(m0 + 4 * kh) * N + min(n, N - 1);
+    const bool add = !partials && accumulate, edge = MT == 1 || m0 + 32 * MT > M || __builtin_amdgcn_readfirstlane(n_base) + 32 > N;
+    if (edge) {
+        if (add) qf_store_rows<MT, true, true>(acc, s_rs, p, N, left, n < N, kh);
+        else qf_store_rows<MT, true, false>(acc, s_rs, p, N, left, n < N, kh);
+    } else {
+        if (add) qf_store_rows<MT, false, true>(acc, s_rs, p, N, left, true, kh);
+        else qf_store_rows<MT, false, false>(acc, s_rs, p, N, left, true, kh);
+    }
+}
 
 // Up to 32 rows and up to four super-blocks of a K split: 128 columns, four waves of one strip.  Such a workgroup's time is its requests' round trips,
 // one per block where the next block's are out while this one is worked on (half a microsecond's work).  Here all of its blocks, of X

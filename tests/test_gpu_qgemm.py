@@ -228,6 +228,26 @@ def test_short_prompts_whose_last_split_is_shorter(dev, po, qt, M, K, N):
     assert np.array_equal(bits(out[0]), bits(out[1]))
 
 
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(1, 256, 31), (5, 768, 128), (32, 768, 33), (33, 768, 129), (64, 512, 256), (65, 768, 255), (128, 256, 513), (129, 768, 256), (192, 512, 20000),
+                                   (257, 768, 6500), (260, 512, 40000)])
+def test_sums_onto_what_is_there(dev, po, qt, M, K, N):
+    """Every tile height, whole tiles and ones with rows and columns past the edge: added onto Y is what is stored plus Y, bit for bit, and
+    nothing behind the last row is written."""
+    r = synth.rng_for(51, qt, M, K, N)
+    W = torch.from_numpy(synth.make_weight(r, qt, N, K)).cuda()
+    x = torch.from_numpy(r.standard_normal((M, K), dtype=np.float32)).cuda()
+    old = torch.from_numpy(r.standard_normal((M + 1, N), dtype=np.float32)).cuda()
+    ws = torch.empty(ops.qgemm_f16_f32_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda")
+    out = []
+    for accumulate in (False, True):
+        y = old.clone()
+        ops.matmul_q_f16_f32(qt, W, x, y, M, K, N, W.shape[1], ws, accumulate=accumulate)
+        assert torch.equal(y[M], old[M])
+        out.append(y[:M])
+    assert torch.equal(out[1], out[0] + old[:M]) or torch.equal(out[1], old[:M] + out[0])
+
+
 # super-blocks of the longest split of each matrix; types in file order, K that does not divide evenly among the splits, N off the 128-column tiles
 @pytest.mark.parametrize("K,N,types,blocks", [(2560, (4097, 1000, 129), (12, 12, 14), (3, 3, 2)), (2560, (13000, 1000, 515), (14, 12, 12), (3, 4, 4)),
                                               (4096, (13000, 1000, 515), (12, 14, 14), (4, 2, 3)), (4096, (5000, 700), (14, 12), (2, 3)), (2560, (20000, 300), (12, 14), (4, 2)),
