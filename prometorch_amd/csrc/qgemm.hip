@@ -815,7 +815,8 @@ __device__ __forceinline__ void qf_store(const f32x16 (&acc)[MT], const float* s
 // one per block where the next block's are out while this one is worked on (half a microsecond's work).  Here all of its blocks, of X
 // (into LDS) and of the weights (registers, up to 120), are requested before any is waited for.  Same sums in the same order.
 // 19 rows, 2560 x 9728 in 13 splits of three: Q6_K 21.6 -> 16.6 us, Q4_K 12.4 -> 11.0; 2 x 9728 x 2560 in three of four 15.8 -> 15.2 (weights in memory order
-// through LDS 17.1; eight waves, 256 columns 17.0).
+// through LDS 17.1; eight waves, 256 columns 17.0).  Then its time is unpacking, behind the weights: 2 x 9728 x 2560 12.3 us without X and stores, 7.3 with one
+// line of weights for all.  Up to two blocks three of them fit a SIMD: 36 layers of 19 rows 2749 -> 2728 us, most of it in q / k / v and o.
 template <typename Tile, int NB>
 __device__ __forceinline__ void qgemm_f16_short_body(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale, float* Y, int M,
                                                      int K, int N, int accumulate, int blocks_per_split, float* partials, int bx, int bz, uint8_t* s_a,
@@ -864,9 +865,9 @@ __device__ __forceinline__ void qgemm_f16_short_body(const uint8_t* W, int64_t s
     }
     qf_store<1>(acc, s_rs, Y, partials, accumulate, M, N, 0, n_base, j, kh, bz);
 }
-// Whether it serves a launch whose longest split has `blocks`: of up to two blocks the other body's prologue and first step request everything, too.
+// Whether it serves a launch whose longest split has `blocks`
 constexpr int QF_SHORT_BLOCKS = 4;
-static inline bool qf_short(int M, int blocks) { return M <= 32 && blocks > 2 && blocks <= QF_SHORT_BLOCKS; }
+static inline bool qf_short(int M, int blocks) { return M <= 32 && blocks <= QF_SHORT_BLOCKS; }
 static inline size_t qf_short_lds(int nb) { return (size_t)nb * 32 * QF_PITCH + 4 * 32; }
 
 // X tile of a super-block step in LDS.  The pieces a thread owns of the NEXT block's tile are fetched during the first
@@ -1255,7 +1256,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES == 8 ? 1 : 2)) void qgemm_f16_ke
 
 // up to 32 rows, NB super-blocks per split
 template <typename Tile, int NB>
-__global__ __launch_bounds__(256, 2) void qgemm_f16_short_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale,
+__global__ __launch_bounds__(256, (NB <= 2 ? 3 : 2)) void qgemm_f16_short_kernel(const uint8_t* W, int64_t stride, const _Float16* Xh, const float* __restrict__ rowscale,
                                                                  float* Y, int M, int K, int N, int accumulate, int blocks_per_split, float* partials,
                                                                  int scale_stride) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
@@ -1323,8 +1324,9 @@ __global__ __launch_bounds__(512, 1) void qgemm_f16_rows_multi_kernel(const QfMu
 #undef PTM_QR
 }
 
-// the same for up to 32 rows and up to QF_SHORT_BLOCKS super-blocks per split
-__global__ __launch_bounds__(256, 2) void qgemm_f16_short_multi_kernel(const QfMulti a, int M, int K) {
+// the same for up to 32 rows and up to NB super-blocks per split
+template <int NB>
+__global__ __launch_bounds__(256, (NB <= 2 ? 3 : 2)) void qgemm_f16_short_multi_kernel(const QfMulti a, int M, int K) {
     extern __shared__ __align__(16) uint8_t qf_lds[];
     read_now(a.m[0].W, a.m[1].W, a.m[2].W, a.n_mat);
     const int sx = qf_xcd_order(blockIdx.x, gridDim.x);
@@ -1334,8 +1336,16 @@ __global__ __launch_bounds__(256, 2) void qgemm_f16_short_multi_kernel(const QfM
     const QfMat& q = i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]);
     const int local = sx - (i == 0 ? 0 : (i == 1 ? a.m[0].slot_end : a.m[1].slot_end));
     const int bx = local % q.ntiles, bz = local / q.ntiles;
-#define PTM_QS(TILE, NB) qgemm_f16_short_body<TILE, NB>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, bz, qf_lds, 0)
-    if (q.q6) {
+#define PTM_QS(TILE, B) qgemm_f16_short_body<TILE, B>(q.W, q.stride, q.Xh, q.rowscale, q.Y, M, K, q.N, 0, q.bps, q.partials, bx, bz, qf_lds, 0)
+    if constexpr (NB <= 2) {
+        if (q.q6) {
+            if (q.bps == 1) PTM_QS(Q6Tile, 1);
+            else PTM_QS(Q6Tile, 2);
+        } else {
+            if (q.bps == 1) PTM_QS(Q4Tile, 1);
+            else PTM_QS(Q4Tile, 2);
+        }
+    } else if (q.q6) {
         if (q.bps <= 2) PTM_QS(Q6Tile, 2);
         else if (q.bps == 3) PTM_QS(Q6Tile, 3);
         else PTM_QS(Q6Tile, 4);
@@ -1403,9 +1413,13 @@ enum { QF_MAX_SPLITS = 16 };
 static inline int qf_row_class(int M) { return M <= 128 ? 1 : (M <= 256 ? 2 : (M <= 1024 ? 4 : 8)); }
 
 // K splits for an N x K weight matrix and M rows: enough workgroups to fill the chip when N alone gives few column
-// tiles (a 2560-wide projection is 10 tiles).  M enters only through its class (up to 128 rows, up to 256, up to 1024, more), so
+// tiles (a 2560-wide projection is 10 tiles).  M enters only through its class, so
 // that the summation order of a row does not change with how many rows share the launch within a class; short
 // prompts (one row tile) get up to 16 splits, because there the launch is bound by how many workgroups stream weights.
+// Where workgroups have 128 columns (below), a few more of them than a round of the chip double what some CUs do: then more
+// blocks a split (2560 x 9728, 19 rows: 13 splits of three blocks, 260 workgroups, Q6_K 15.9 us, Q4_K 10.1; 247 of them 11.3 and 8.1; ten of four, 200, 13.5 and 9.4;
+// 19 of two 11.8 and 8.4, but as many more sums for the next kernel).  18 layers of Qwen3-4B shapes, 19 rows 1364 -> 1343 us, 40 rows 1676 -> 1606, 64
+// rows 1713 -> 1645, 100 rows 2181 and 2185, 128 rows 2222 and 2237; 12 of Gemma-3-4B shapes, 30 rows 1276 -> 1254.
 int qgemm_f16_splits(int N, int K, int M) {
     const int ntiles = (N + QF_TN - 1) / QF_TN, nblk = K / 256;
     const int row_tiles = qf_row_class(M);
@@ -1413,7 +1427,16 @@ int qgemm_f16_splits(int N, int K, int M) {
     const int cap = row_tiles == 1 ? QF_MAX_SPLITS : 8;
     s = s > cap ? cap : s;
     s = s > nblk / 2 ? nblk / 2 : s;
-    return s < 1 ? 1 : s;
+    s = s < 1 ? 1 : s;
+    if (M <= 128 && s > 1) {
+        const int tiles = (N + 127) / 128, from = (nblk + s - 1) / s;
+        auto blocks = [&](int bps) { return (tiles * ((nblk + bps - 1) / bps) + 255) / 256 * bps; };
+        int best = from;
+        for (int bps = from + 1; bps <= QF_SHORT_BLOCKS; ++bps)
+            if (blocks(bps) < blocks(best)) best = bps;
+        s = (nblk + best - 1) / best;
+    }
+    return s;
 }
 
 // K splits of the matrices of a multi-matrix launch.  All (column tile, split) slots of all matrices must fit one round of
@@ -1421,6 +1444,8 @@ int qgemm_f16_splits(int N, int K, int M) {
 // workgroup: starting from one split each, the matrix whose workgroups have the most work (blocks per split, a Q6_K block
 // weighing 1.6 Q4_K blocks: measured 8 against 5 us) gets its next split count until the slots run out.  A function of
 // the shapes, the types and M's class only, like qgemm_f16_splits.
+// Up to 128 rows one more split where, in workgroups of 128 columns, that takes a fifth off what the busiest CU does: gate and up of 18944 x 3584 in one split are
+// 296 workgroups of 14 blocks, two on some CUs, in two 592 of seven (25 rows, 8 layers: 1002 -> 975 us).
 void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits) {
     const int nblk = K / 256;
     const int row_tiles = qf_row_class(M);
@@ -1443,6 +1468,15 @@ void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int
         slots += ntile[j] * (next - splits[j]);
         splits[j] = next;
     }
+    if (M > 128) return;
+    int tiles = 0;
+    for (int i = 0; i < n; ++i) {
+        if (splits[i] != splits[0]) return;
+        tiles += (N[i] + 127) / 128;
+    }
+    auto blocks = [&](int s) { return (tiles * s + 255) / 256 * ((nblk + s - 1) / s); };
+    if (splits[0] < cap && 5 * blocks(splits[0] + 1) <= 4 * blocks(splits[0]))
+        for (int i = 0; i < n; ++i) ++splits[i];
 }
 
 // Rows per workgroup in tiles of 32: 4 (128 rows: each dequantised weight serves twice as many products) unless that
@@ -1597,10 +1631,14 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         const size_t short_lds = qf_short_lds(bps);
 #define PTM_QS(TILE, NB) hipLaunchKernelGGL((qgemm_f16_short_kernel<TILE, NB>), dim3(grid.x * grid.z), dim3(256), short_lds, s, Wb, stride, Xh, rowscale, Y, M, K, N, acc, bps, partials, scale_stride)
         if (q4) {
-            if (bps == 3) PTM_QS(Q4Tile, 3);
+            if (bps == 1) PTM_QS(Q4Tile, 1);
+            else if (bps == 2) PTM_QS(Q4Tile, 2);
+            else if (bps == 3) PTM_QS(Q4Tile, 3);
             else PTM_QS(Q4Tile, 4);
         } else {
-            if (bps == 3) PTM_QS(Q6Tile, 3);
+            if (bps == 1) PTM_QS(Q6Tile, 1);
+            else if (bps == 2) PTM_QS(Q6Tile, 2);
+            else if (bps == 3) PTM_QS(Q6Tile, 3);
             else PTM_QS(Q6Tile, 4);
         }
 #undef PTM_QS
@@ -1734,14 +1772,16 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     std::call_once(raised, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_rows_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, QF_ROWS_LDS);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<4, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, QF_ROWS_LDS);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_multi_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(QF_SHORT_BLOCKS));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_short_multi_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)qf_short_lds(QF_SHORT_BLOCKS));
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_multi_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   2 * 64 * QF_PITCH + 4 * 64);
     });
-    if (qf_short(M, most))
-        hipLaunchKernelGGL(qgemm_f16_short_multi_kernel, dim3(slots), dim3(256), qf_short_lds(most), s, a, M, K);
+    if (qf_short(M, most) && most <= 2)
+        hipLaunchKernelGGL(qgemm_f16_short_multi_kernel<2>, dim3(slots), dim3(256), qf_short_lds(most), s, a, M, K);
+    else if (qf_short(M, most))
+        hipLaunchKernelGGL(qgemm_f16_short_multi_kernel<4>, dim3(slots), dim3(256), qf_short_lds(most), s, a, M, K);
     else if (M <= 32)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<1, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)32 * QF_PITCH + 4 * 32, s, a, M, K);
     else if (narrow)

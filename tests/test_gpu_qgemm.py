@@ -229,6 +229,16 @@ def test_short_prompts_whose_last_split_is_shorter(dev, po, qt, M, K, N):
 
 
 @pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(1, 256, 129), (32, 256, 127), (19, 512, 1), (31, 512, 385), (19, 1280, 130), (32, 4096, 2560)])
+def test_short_prompts_of_one_and_two_blocks(dev, po, qt, M, K, N):
+    """Splits of one and of two super-blocks, the last shorter or not: rows are the rows of a 40-row call, which has the same splits, bit for bit."""
+    r = synth.rng_for(50, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    xb, _ = bf16_round(r.standard_normal((40, K), dtype=np.float32))
+    assert np.array_equal(bits(gpu_qgemm_f16(qt, W, xb[:M], M, K, N)), bits(gpu_qgemm_f16(qt, W, xb, 40, K, N)[:M]))
+
+
+@pytest.mark.parametrize("qt", [12, 14])
 @pytest.mark.parametrize("M,K,N", [(1, 256, 31), (5, 768, 128), (32, 768, 33), (33, 768, 129), (64, 512, 256), (65, 768, 255), (128, 256, 513), (129, 768, 256), (192, 512, 20000),
                                    (257, 768, 6500), (260, 512, 40000)])
 def test_sums_onto_what_is_there(dev, po, qt, M, K, N):
