@@ -335,6 +335,48 @@ __device__ __forceinline__ void dense_tile(const DenseGemm& g, const GemmRegion&
     t.run(lds, steps, [&](int st, int i, int at) { gt_to_lds(base + at + i * 8192, (int)xo[i], xs, st * 128); },
           [&](int st, int i, int at) { gt_to_lds(base + at + i * 8192, (int)wo[i], ws, st * 128); });
     const int m1 = min(g.M, r.m0 + r.tiles_m * Tile::BM), n1 = min(g.N, r.n1);
+    // Tiles that end within the columns (and rows that hold whole vectors): one place per lane, a test per row.  With its own place, its tests and its kind of
+    // result decided for every store, the end of a 256 x 256 tile took 64 instructions per eight values.
+    const int row0 = Tile::lane_row(), col0 = Tile::lane_col(), g4 = (lane >> 4) * 4;
+    auto rows = [&](auto&& store) {
+#pragma unroll
+        for (int a = 0; a < Tile::ROWS; ++a)
+            if (m0 + row0 + 16 * a < m1)
+#pragma unroll
+                for (int b = 0; b < Tile::COLS; b += 2) store(a, b, (int64_t)(16 * a) * g.ldc, t.acc[a][b], t.acc[a][b + 1]);
+    };
+    if (n0 + Tile::BN <= n1 && (!glu || (g.ldc & 3) == 0)) {
+        const int64_t first = (int64_t)(m0 + row0) * g.ldc;
+        auto pack = [](float lo, float hi) { return (uint32_t)f_bf16(lo) | ((uint32_t)f_bf16(hi) << 16); };
+        if (glu) {
+            uint16_t* p = static_cast<uint16_t*>(g.C) + first + (n0 + col0 - g4) / 2 + g4;
+            rows([&](int, int b, int64_t at, const gt_f4& x, const gt_f4& u) {
+                *reinterpret_cast<uint2*>(p + at + 8 * b) = make_uint2(pack(silu_f(x[0]) * u[0], silu_f(x[1]) * u[1]), pack(silu_f(x[2]) * u[2], silu_f(x[3]) * u[3]));
+            });
+            return;
+        }
+        if (pairs && (g.ldc & 7) == 0) {
+            uint16_t* p = static_cast<uint16_t*>(g.C) + first + n0 + col0 + g4;
+            auto put = [&](int b, int64_t at, const gt_f4& x, const gt_f4& y) {
+                *reinterpret_cast<uint4*>(p + at + 16 * b) = make_uint4(pack(x[0], x[1]), pack(x[2], x[3]), pack(y[0], y[1]), pack(y[2], y[3]));
+            };
+            if (g.epilogue == GEMM_RELU2)
+                rows([&](int, int b, int64_t at, const gt_f4& x, const gt_f4& y) {
+                    put(b, at, gt_f4{relu2(x[0]), relu2(x[1]), relu2(x[2]), relu2(x[3])}, gt_f4{relu2(y[0]), relu2(y[1]), relu2(y[2]), relu2(y[3])});
+                });
+            else
+                rows([&](int, int b, int64_t at, const gt_f4& x, const gt_f4& y) { put(b, at, x, y); });
+            return;
+        }
+        if (g.epilogue == GEMM_F32 && (g.ldc & 3) == 0) {
+            float* p = static_cast<float*>(g.C) + first + n0 + col0 + split * g.slab;
+            rows([&](int, int b, int64_t at, const gt_f4& x, const gt_f4& y) {
+                *reinterpret_cast<gt_f4*>(p + at + 16 * b) = x;
+                *reinterpret_cast<gt_f4*>(p + at + 16 * b + 16) = y;
+            });
+            return;
+        }
+    }
     if (glu) {  // even W fragments are gates, the odd ones behind them the ups of the same values
         DenseGemm o = g;
         o.epilogue = GEMM_ELEM;

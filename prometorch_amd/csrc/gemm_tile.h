@@ -132,6 +132,10 @@ struct GemmTile {
         }
     }
 
+    // where the lane's sums acc[0][0] lie: row of X, first of four rows of W; acc[a][b] are 16 a and 16 b on
+    static __device__ __forceinline__ int lane_row() { return ((threadIdx.x >> 6) % WX) * 16 * RX + (threadIdx.x & 15); }
+    static __device__ __forceinline__ int lane_col() { return ((threadIdx.x >> 6) / WX) * 16 * RW + 4 * ((threadIdx.x >> 4) & 3); }
+    static constexpr int ROWS = RX, COLS = RW;
     // use(a, b, row of X, row of W): the sums acc[a][b] and acc[a][b + 1] are of rows .. + 0, 1, 2, 3 and .. + 16, 17, 18, 19 of W in LDS
     template <typename Use>
     __device__ __forceinline__ void each(Use&& use) const {
