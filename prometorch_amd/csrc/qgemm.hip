@@ -1479,17 +1479,6 @@ void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int
         for (int i = 0; i < n; ++i) ++splits[i];
 }
 
-// Rows per workgroup in tiles of 32: 4 (128 rows: each dequantised weight serves twice as many products) unless that
-// leaves most of the chip idle; then 2 (64 rows: twice the workgroups).  Prompts of up to 64 / 32 rows take the 64- / 32-row
-// tile: a quarter of the X tile traffic, LDS reads and MFMAs per block.  A row's sum does not depend on the choice (same K
-// order).  Threshold swept on the Qwen3-4B shapes: 128 workgroups, Q4_K only, is the best or tied at every prompt length.
-static int qgemm_f16_row_tiles(bool q4, int M, int N, int splits) {
-    if (M <= 32) return 1;
-    if (M <= 64) return 2;
-    const int wgs = ((N + QF_TN - 1) / QF_TN) * ((M + 127) / 128) * splits;
-    return (q4 && wgs < 128) ? 2 : 4;  // 512 x 2560 x 9728 (152 workgroups): 60 us with 128 rows, 70 with 64; 512 x 4096 x 4096 (64): 80 / 68
-}
-
 // Which tiles of a launch of gx column tiles (slots) and gz K splits have 256 rows: the first `tall` pairs of row tiles in qf_tile_of's order, in whole
 // rounds of the chip or all of them - or whether all tiles have 192 - whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
 // times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there; a tile of 192 rows
@@ -1537,12 +1526,16 @@ float qgemm_f16_rounds(int tiles, int M, bool q4) {
     return qf_tall(tiles, 1, M, q4, &tall);
 }
 
-// Workgroups of 128 columns: always up to 32 rows, up to 64 where the chip then has a CU for each.  Prompts of 19 / 32 / 50 / 64 tokens,
-// Qwen3-4B shapes, 256 columns, this rule, 128 always: 3.53 / 3.67 / 3.97 / 4.12 ms, 3.32 / 3.45 / 3.89 / 4.00, 3.32 / 3.45 / 3.86 / 3.97;
+// Workgroups of 128 columns (and up to 64 rows): always up to 32 rows, up to 64 where the chip then has a CU for each, with more rows where two
+// of them fit every CU: half the columns and half the rows are half the unpacking and a quarter of the products of a workgroup that leaves CUs idle.  Prompts of
+// 19 / 32 / 50 / 64 tokens, Qwen3-4B shapes, 256 columns, this rule, 128 always: 3.53 / 3.67 / 3.97 / 4.12 ms, 3.32 / 3.45 / 3.89 / 4.00, 3.32 / 3.45 / 3.86 / 3.97;
 // Llama-3-8B shapes in 16 layers, 60 tokens: 2.28, 2.28, 2.31; in 8 layers, 5 / 19 / 32 tokens, 256 columns and so: 1.05 / 1.10 / 1.13, 1.00 / 1.05 /
 // 1.09.  Up to 32 rows a single product is 10 to 25 % faster where 256 columns are up to 128 workgroups, and the same within -3 to 3 % where they are
-// more (32 x 4096 x 14336 22.5 -> 23.2 us, 2 x 9728 x 16384 41.7 -> 40.7).  A row's sum does not depend on the choice.
-static bool qf_narrow(int M, int wide_workgroups) { return M <= 32 || (M <= 64 && wide_workgroups <= 128); }
+// more (32 x 4096 x 14336 22.5 -> 23.2 us, 2 x 9728 x 16384 41.7 -> 40.7).  More than 64 rows, 256 columns and so, and with three of them to two CUs: 70 / 128 rows,
+// 18 layers of Qwen3-4B shapes 2039 / 2191 -> 1978 / 2122 us, 16 of width 1024 (66, 128, 250, 600, 1500 rows) 1183 1164 1415 1707 2868 -> 896 921 1157 1592 2818, the
+// last three then 1141 1585 2925; 12 layers of Qwen3-4B, 160 / 250 rows 1898 / 2088, 1847 / 2078, 1909 / 2204; 6 of Llama-3-8B, 190 rows 1301, 1296, 1457.
+// A row's sum does not depend on the choice.
+static bool qf_narrow(int M, int wide_workgroups) { return M <= 32 || (M <= 64 ? wide_workgroups <= 128 : (int64_t)wide_workgroups * ((M + 63) / 64) <= 256); }
 
 static int qgemm_check(const void* W, const void* X, const void* Y, int M, int K, int N, int64_t stride, int blk_bytes) {
     if (!W || !X || !Y) return PTM_E_NULL;
@@ -1603,8 +1596,9 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         else if (x_is_f32) hipLaunchKernelGGL((qgemm_prepare_rows_f16_kernel<false, true>), dim3(mp), dim3(256), 0, s, X, Xh, rowscale, M, K);
         else hipLaunchKernelGGL((qgemm_prepare_rows_f16_kernel<false, false>), dim3(mp), dim3(256), 0, s, X, Xh, rowscale, M, K);
     }
-    // rows per workgroup: 32, 64 or 128 (see qgemm_f16_row_tiles)
-    const int MT = qgemm_f16_row_tiles(q4, M, N, splits);
+    const int wide = (N + QF_TN - 1) / QF_TN * splits;
+    const bool narrow = qf_narrow(M, wide);
+    const int MT = M <= 32 ? 1 : M <= 64 || narrow ? 2 : 4;  // tiles of 32 rows
     const int tm = 32 * MT;
     const size_t lds = 2 * (size_t)tm * QF_PITCH + 4 * (size_t)tm;  // two X tiles (64 rows: 66 KB) and the row scales: above the default 64 KB cap of dynamic LDS
     static std::once_flag raised;  // two host threads may get here at once: the second waits until the caps are raised
@@ -1619,8 +1613,6 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q4Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&qgemm_f16_kernel<Q6Tile, 2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, small);
     });
-    const int wide = (N + QF_TN - 1) / QF_TN * splits;
-    const bool narrow = qf_narrow(M, wide);
     const int tn = narrow ? 128 : QF_TN;
     const dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm, splits);
     const uint8_t* Wb = static_cast<const uint8_t*>(W);
@@ -1785,7 +1777,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
     else if (M <= 32)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<1, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)32 * QF_PITCH + 4 * 32, s, a, M, K);
     else if (narrow)
-        hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 4>), dim3(slots, 1), dim3(256), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
+        hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 4>), dim3(slots, (M + 63) / 64), dim3(256), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
     else if (M <= 64)
         hipLaunchKernelGGL((qgemm_f16_multi_kernel<2, 8>), dim3(slots, 1), dim3(512), 2 * (size_t)64 * QF_PITCH + 4 * 64, s, a, M, K);
     else {

@@ -317,6 +317,53 @@ def test_short_prompts_of_several_matrices(dev, po, K, N, types, blocks):
         assert err <= QGEMM_F16_TOL, (i, err)
 
 
+@pytest.mark.parametrize("K,N,types", [(1024, (1000, 129, 257), (12, 12, 14)), (2560, (4097, 1000), (14, 12)), (256, (300, 300), (12, 12))])
+def test_several_matrices_in_128_columns_and_several_row_tiles(dev, po, K, N, types):
+    """65 to 128 rows in workgroups of 64 rows and 128 columns: their first 40 rows are those of a 40-row call, which has the same splits, bit for
+    bit, and so are rows 64 on of those of a call of them alone."""
+    import ctypes as C
+    from gemm_helpers import harness
+    h, n = harness(), len(N)
+    h.multi_split_bytes.restype = C.c_int64
+    Ns, ts = (C.c_int * n)(*N), (C.c_uint32 * n)(*types)
+    r = synth.rng_for(52, K, *N)
+    W = [torch.from_numpy(synth.make_weight(r, t, rows, K)).cuda() for t, rows in zip(types, N)]
+    gamma = torch.from_numpy((1 + 0.1 * r.standard_normal(K)).astype(np.float32)).cuda()
+    X = torch.from_numpy(r.standard_normal((128, K), dtype=np.float32)).cuda()
+    ptrs = lambda ts: (C.c_void_p * n)(*[t.data_ptr() for t in ts])
+    p = lambda t: C.c_void_p(t.data_ptr())
+
+    def run(x):
+        M = x.shape[0]
+        ws = [torch.zeros(ops.qgemm_f16_workspace_bytes(M, K), dtype=torch.uint8, device="cuda") for _ in range(2)]
+        split = torch.full((max(h.multi_split_bytes(n, Ns, ts, K, M) // 4, 4),), 5.0, device="cuda")
+        Y = [torch.full((M + 1, rows), 3.0, device="cuda") for rows in N]
+        assert h.multi_run(n, ts, ptrs(W), (C.c_int64 * n)(*[w.shape[1] for w in W]), Ns, ptrs(Y), p(x), p(gamma), M, K, p(ws[0]), p(ws[1]), p(split),
+                           C.c_int64(split.numel() * 4), None, None, None) == 0
+        torch.cuda.synchronize()
+        assert all(bool((y[M] == 3.0).all()) for y in Y)
+        return [y[:M] for y in Y]
+
+    few = run(X[:40].contiguous())
+    for M in (65, 100, 128):
+        tail = run(X[64:M].contiguous())
+        for i, y in enumerate(run(X[:M].contiguous())):
+            assert torch.equal(y[:40], few[i]), (M, i)
+            assert torch.equal(y[64:], tail[i]), (M, i)
+
+
+@pytest.mark.parametrize("qt", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(65, 768, 257), (128, 2560, 1000), (127, 9728, 129)])
+def test_128_columns_and_several_row_tiles(dev, po, qt, M, K, N):
+    """65 to 128 rows in workgroups of 64 rows and 128 columns: rows are those of a 40-row call, which has the same splits, bit for bit."""
+    r = synth.rng_for(53, qt, M, K, N)
+    W = synth.make_weight(r, qt, N, K)
+    xb, _ = bf16_round(r.standard_normal((M, K), dtype=np.float32))
+    y = gpu_qgemm_f16(qt, W, xb, M, K, N)
+    assert np.array_equal(bits(y[:40]), bits(gpu_qgemm_f16(qt, W, xb[:40], 40, K, N)))
+    assert np.array_equal(bits(y[64:]), bits(gpu_qgemm_f16(qt, W, xb[64:], M - 64, K, N)))
+
+
 # tiles of 256 rows: all (236 pairs of row tiles), whole rounds and 128-row tiles behind them (K splits off and on), an odd last row tile, ragged N; of 192
 # rows: 3 and 2 row tiles, whole and ragged, one of 129 rows
 @pytest.mark.parametrize("qt", [12, 14])
