@@ -5,10 +5,10 @@
 //
 // slots_gemv_kernel: a lane takes 8 values of a row (16 of a Q5_K block: both nibbles of its bytes) at a time, so that neighbouring lanes read
 // neighbouring pieces of x and of the row, and a wave several rows, so that x is loaded once for all of them; two passes over the row are
-// requested together.  Bound by requests in flight: Q8_0 with weights from HBM, in a graph, 9728 x 2560 9.1 us = 2.9 TB/s, 30000 x 2560 19.5 us =
-// 4.2 TB/s, 500 x 1024 2.3 us (19.1, 50.1 and 2.6 with a lane per run of 32 values, as the exact Q4_K kernel below still has it: x and the
+// requested together; split_gemv_kernel: a wave per pass.  Bound by requests in flight: Q8_0 with weights from HBM, in a graph, 9728 x 2560 7.9 us = 3.3 TB/s
+// (two passes at a time 8.7), 30000 x 2560 19.5 us = 4.2 TB/s with two passes at a time, 500 x 1024 2.3 us (19.1, 50.1 and 2.6 with a lane per run of 32 values, as the exact Q4_K kernel below still has it: x and the
 // row are then read in pieces 128 and 34 bytes apart, and every load instruction touches 64 cache lines); 9728 x 2560 called again and again on
-// weights that the caches hold 7.6 us (18.1).
+// weights that the caches hold 6.1 us (6.6; 18.1).
 #include "ptm_common.h"
 
 #include <type_traits>
@@ -25,10 +25,11 @@ __device__ __forceinline__ void load8(const float* __restrict__ x, float (&v)[8]
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-// A format: VALUES of a row per slot; from how many slots LONG rows are shared by waves, then ROWS per wave of 2048 rows and more, FEW of 1024 to
-// 2047 (slots_launch); what a lane loads of the row for slot u, which values of x (two groups of 8 or 4), the slot's term.
+// A format: VALUES of a row per slot; where waves share rows ROWS per wave of 2048 rows and more, FEW of 1024 to 2047; whether fewer than 2048 rows,
+// too, have a wave for each pass (slots_launch); what a lane loads of the row for slot u, which values of x (two groups of 8 or 4), the slot's term.
 struct FmtQ8_0 {
-    static constexpr int BLOCK_BYTES = 34, VALUES = 8, ROWS = 4, FEW = 2, LONG = 256;
+    static constexpr int BLOCK_BYTES = 34, VALUES = 8, ROWS = 4, FEW = 2;
+    static constexpr bool SPLIT_FEW = false;
     struct Raw { u64_a2 q; uint32_t d; };
     struct X { float v[8]; };
     static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
@@ -53,7 +54,8 @@ struct FmtQ8_0 {
 };
 
 struct FmtQ5_0 {
-    static constexpr int BLOCK_BYTES = 22, VALUES = 8, ROWS = 2, FEW = 1, LONG = 256;  // four low nibbles and the four high ones of the same bytes, 16 values on
+    static constexpr int BLOCK_BYTES = 22, VALUES = 8, ROWS = 2, FEW = 1;  // four low nibbles and the four high ones of the same bytes, 16 values on
+    static constexpr bool SPLIT_FEW = false;
     struct Raw { uint32_t q, h, d; };
     struct X { float v[8]; };
     static __device__ __forceinline__ void load(const uint8_t* __restrict__ row, int u, Raw& r) {
@@ -69,20 +71,26 @@ struct FmtQ5_0 {
         o.v[4] = b.x; o.v[5] = b.y; o.v[6] = b.z; o.v[7] = b.w;
     }
     static __device__ __forceinline__ float term(const Raw& r, const X& x, int u) {
+        // four values at a time: the fifth bits spread to their bytes (times 1 + 2^7 + 2^14 + 2^21), 16 subtracted within each byte, which the conversion
+        // then takes with its sign (9728 x 2560 7.5 -> 6.4 us; byte by byte a value was eight instructions, so it is four)
         const uint32_t h = r.h >> (4 * (u & 3));
+        auto less16 = [](uint32_t nibbles, uint32_t high) {
+            return (((nibbles & 0x0f0f0f0fu) | (((high & 0xfu) * 0x00204081u) & 0x01010101u) << 4 | 0x80808080u) - 0x10101010u) ^ 0x80808080u;
+        };
+        const uint32_t lo = less16(r.q, h), hi = less16(r.q >> 4, h >> 16);
         float s = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t b = (r.q >> (8 * i)) & 0xffu;
-            s = fmaf((float)((int)((b & 0xfu) | (((h >> i) & 1u) << 4)) - 16), x.v[i], s);
-            s = fmaf((float)((int)((b >> 4) | (((h >> (16 + i)) & 1u) << 4)) - 16), x.v[4 + i], s);
+            s = fmaf((float)(int8_t)((lo >> (8 * i)) & 0xffu), x.v[i], s);
+            s = fmaf((float)(int8_t)((hi >> (8 * i)) & 0xffu), x.v[4 + i], s);
         }
         return h2f(r.d) * s;
     }
 };
 
 struct FmtQ5_K {
-    static constexpr int BLOCK_BYTES = 176, VALUES = 16, ROWS = 4, FEW = 2, LONG = 512;  // eight low nibbles and the eight high ones of the same bytes, 32 values on
+    static constexpr int BLOCK_BYTES = 176, VALUES = 16, ROWS = 4, FEW = 2;  // eight low nibbles and the eight high ones of the same bytes, 32 values on
+    static constexpr bool SPLIT_FEW = true;
     struct Raw { uint4 hdr; uint2 q, h; };
     struct X { float lo[8], hi[8]; };
     // scale and min of sub-block sb from the 12 packed bytes at p + 4 (get_scale_min_k4, gguf_dequant.h:289-297)
@@ -236,6 +244,37 @@ __global__ __launch_bounds__(256) void slots_gemv_kernel(const uint8_t* __restri
     if ((lane & (64 / R - 1)) == 0 && r0 + i < N) y[r0 + i] = ACC ? y[r0 + i] + v : v;
 }
 
+// The same for rows of up to SPLIT_PASSES passes: a wave for each pass, all of them at the same R rows, so that nothing is requested twice, no wave is without
+// work (2560 values of Q8_0 are five passes: in twos for four waves, the last has none) and x, which goes out first, is read once for R rows.
+constexpr int SPLIT_PASSES = 10;
+template <typename Fmt, int R, bool ACC>
+__global__ __launch_bounds__(64 * SPLIT_PASSES) void split_gemv_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, float* __restrict__ y,
+                                                                       int K, int N, int64_t stride) {
+    __shared__ float part[SPLIT_PASSES][R];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = blockIdx.x * R, slots = K / Fmt::VALUES, at = 64 * wave + lane, u = min(at, slots - 1);
+    typename Fmt::X xv;
+    typename Fmt::Raw w[R];
+    Fmt::load_x(x, u, xv);
+    issue_order_fence();
+#pragma unroll
+    for (int i = 0; i < R; ++i) Fmt::load(W + (int64_t)min(r0 + i, N - 1) * stride, u, w[i]);
+    float acc[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const float t = Fmt::term(w[i], xv, u);
+        acc[i] = at < slots ? t : 0.0f;  // a lane beyond the row repeats the last slot and does not count it
+    }
+    const float v = sum_rows<R>(acc);
+    if ((lane & (64 / R - 1)) == 0) part[wave][sum_row<R>(lane)] = v;
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i >= R || r0 + i >= N) return;
+    float s = part[0][i];
+    for (int c = 1; c < (int)blockDim.x / 64; ++c) s += part[c][i];
+    y[r0 + i] = ACC ? y[r0 + i] + s : s;
+}
+
 template <typename Fmt>
 __global__ __launch_bounds__(256) void elementwise_dequant_kernel(const uint8_t* __restrict__ blocks, float* __restrict__ out,
                                                                   int64_t n) {
@@ -277,8 +316,22 @@ static int slots_launch(const void* W, const float* x, float* y, int K, int N, i
     // wave per row, 32 values a lane: 3.31), 1280 x 4096 4.75 4.36, 2047 x 2048 3.94 3.73, 2047 x 8192 7.97 8.14.
     // Rows of one pass: a second request would repeat it, Q5_K 2560 x 256 4.0 -> 3.2 us (a wave per row, 32 values a lane: 3.7), 9728 x 1024 7.2 ->
     // 4.8 (9.2), Q8_0 2560 x 512 3.0 -> 2.8 (3.8).
-    const int slots = K / Fmt::VALUES;
-    if (slots >= (N >= 2048 ? Fmt::LONG : 256)) {
+    const int slots = K / Fmt::VALUES, all = (slots + 63) / 64;
+    // Three to ten passes, a wave for each.  us as below and so, on weights that the caches hold, Q8_0 9728 x 1536 5.5, 4.5, x 2560 6.6, 6.1, 2048 x 2560 2.8, 2.6,
+    // 6000 x 5120 7.1, 6.9, 14336 x 4096 10.3, 10.4, 30000 x 3584 27.3, 24.9 (from HBM 9728 x 2560 8.7, 7.9, 14336 x 4096 15.1, 14.7); Q5_K 9728 x 2560 9.7, 7.2,
+    // 2560 x 9728 10.2, 7.7, 30000 x 3584 22.4, 20.0; Q5_0 9728 x 2560 9.8, 6.4, 6000 x 5120 9.8, 7.3.  Of two passes, 9728 x 1024, they are within 2 % (Q5_K x 1536
+    // 5.66, 5.71), of fourteen Q8_0 3000 x 7168 5.7, 5.6.  Fewer rows, two a workgroup, are faster for Q5_K alone: 1200 x 4096 3.6, 3.1 (Q8_0 2.9, 3.0),
+    // 400 x 10240 3.4, 3.1, 300 x 2560 2.7, 2.3 (2.2, 2.2).
+    auto split = [&](auto rows) {
+        constexpr int R = decltype(rows)::value;
+        const dim3 grid((N + R - 1) / R), block(64 * all);
+        if (accumulate) hipLaunchKernelGGL((split_gemv_kernel<Fmt, R, true>), grid, block, 0, s, w, x, y, K, N, stride);
+        else hipLaunchKernelGGL((split_gemv_kernel<Fmt, R, false>), grid, block, 0, s, w, x, y, K, N, stride);
+    };
+    if (all >= 3 && all <= SPLIT_PASSES && (N >= 2048 || Fmt::SPLIT_FEW)) {
+        if (N >= 2048) split(four);
+        else if constexpr (Fmt::SPLIT_FEW) split(two);
+    } else if (slots >= 256) {
         if (N >= 2048) go(integral_constant<int, Fmt::ROWS>{}, four, two);
         else if (N >= 1024) go(integral_constant<int, Fmt::FEW>{}, four, two);
         else go(one, four, two);

@@ -75,6 +75,21 @@ def test_other_formats_gemv_rows_of_one_pass(dev, po, qt, N, K):
     assert np.abs((gpu_gemv(qt, W, x, accumulate=True, y0=y0) - y0) - ref).max() <= 1e-5 * max(np.abs(y0).max(), np.abs(ref).max())
 
 
+@pytest.mark.parametrize("qt,N,K", [(qt, N, K) for qt, per, once in ((8, 32, 512), (6, 32, 512), (13, 256, 1024)) for N, K in
+                                    ((2048, 2 * once + per), (2049, 3 * once), (2051, 5 * once - per), (2050, 10 * once), (2050, 10 * once + per), (2, 3 * once), (1, 10 * once))])
+def test_other_formats_gemv_wave_per_pass(dev, po, qt, N, K):
+    """Three to ten passes over a row, the last whole or not, rows past the last of a workgroup; as stored and as added."""
+    r = synth.rng_for(38, qt, N, K)
+    W = synth.make_weight(r, qt, N, K)
+    x = synth.make_x(r, K)
+    Wd, xd, y = torch.from_numpy(W).cuda(), torch.from_numpy(x).cuda(), torch.full((N + 8,), 7.0, device="cuda")
+    ops.quant_gemv(qt, Wd, xd, y, K, N, W.shape[1])
+    got = y[:N].cpu().numpy()
+    assert rel_err(got, po.gemv(qt, W, x)) <= GEMV_TOL * 1e-2
+    ops.quant_gemv(qt, Wd, xd, y, K, N, W.shape[1], accumulate=True)
+    assert np.array_equal(y[:N].cpu().numpy(), got + got) and bool((y[N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("qt,N,K", [(13, 24, 512), (13, 3, 2560), (8, 24, 512), (8, 5, 96)])
 def test_other_formats_dequant_bit_exact(dev, po, seeds, golden_formats, qt, N, K):
     r = synth.rng_for(seeds["blocks"], qt, N, K)
