@@ -795,10 +795,14 @@ __global__ __launch_bounds__(1024) void sampler_finish_kernel(SamplerArgs a, Sam
 
 // ---- the short path: top-k up to LOCAL_MAX_TOPK ------------------------------------------------------------------------
 // Two launches and one read of the logits instead of seven launches and four reads: a call is a chain of launches and latencies (151 936
-// logits, top-k 40: 34.6 us with histograms, 12.6 so; both read 1.2 MB, under a microsecond).  Beyond 64 candidates per slice the second
+// logits, top-k 40: 34.6 us with histograms, 11.2 so; both read 1.2 MB, under a microsecond).  Beyond 64 candidates per slice the second
 // launch, a single workgroup, would read more than it saves.  What is at or above the k-th largest of the vocabulary is at
 // or above the k-th largest of its slice, so a workgroup leaves only those of its slice, and one workgroup selects among them.
 //
+// Up to this k among 128 maxima, two a lane: a bit then takes a third of the time, and what is left above the bound (48 of k = 40, of more
+// maxima 43) still fits a wave.  Top-k 20 and 40 of 151936 logits 11.2 -> 9.8 and 12.7 -> 11.2 us; 64 would leave 89 and the longer way.
+enum { LOCAL_PAIRS_TOPK = 40 };
+
 // The largest T = t + bits `bit` .. low with at least k of the wave's R values per lane at or above it (bits above are in t already; t if there
 // are fewer than k above it).
 template <int R>
@@ -860,13 +864,15 @@ __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
     uint32_t* seg = a.ws + SW_LOCAL + blockIdx.x * LOCAL_WORDS;
     if (wave == 0) {
         const uint32_t v[4] = {s_max[lane], s_max[lane + 64], s_max[lane + 128], s_max[lane + 192]};
+        const uint32_t pairs[2] = {max(v[0], v[1]), max(v[2], v[3])};
         uint32_t t;
         if (greedy) {
             t = max(max(v[0], v[1]), max(v[2], v[3]));
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) t = max(t, (uint32_t)__shfl_xor(t, off, 64));
         } else {
-            t = kth_of_wave(v, sampler_k(p), 31, 16, 0u);
+            const int k = sampler_k(p);
+            t = k <= LOCAL_PAIRS_TOPK ? kth_of_wave(pairs, k, 31, 16, 0u) : kth_of_wave(v, k, 31, 16, 0u);
         }
         if (lane == 0) s_bound = t;
     } else if (wave <= 4) {  // the quarters' maxima
@@ -926,8 +932,8 @@ __global__ __launch_bounds__(1024) void sampler_local_kernel(SamplerArgs a) {
 
 // One workgroup: the candidates of all slices in registers.  A lower bound of the k-th largest is the k-th largest of the quarters'
 // maxima (one wave finds it), which leaves about k of some thousands; of those, the ones with fewer than k greater ones.  For more than 256
-// of them the k-th largest is found exactly, two bits at a time by all waves (6 us).  151936 logits, top-k 40 / 64: normal 12.6 / 16.4 us,
-// evenly from 0 to 1 23.8 / 25.2, ten above a mask of -inf 543 both (more ties than a list holds: sampler_overflow_body); with
+// of them the k-th largest is found exactly, two bits at a time by all waves (6 us).  151936 logits, top-k 20 / 40 / 64: normal 9.8 / 11.2 / 16.3 us,
+// evenly from 0 to 1 13.5 / 14.8 / 19.1, ten above a mask of -inf 543 both (more ties than a list holds: sampler_overflow_body); with
 // histograms 34.6 / 40.3, 32.6 / 38.8, 595.  Ties that a slice left out are more than k of a key, so that none of them and nothing
 // listed below them is kept unless they are the k-th largest themselves; then they are read from their slices.
 __global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs a, SamplerOut o, int slices, int per) {
@@ -953,7 +959,10 @@ __global__ __launch_bounds__(1024) void sampler_local_finish_kernel(SamplerArgs 
     if (wave == 0) {
 #pragma unroll
         for (int t = 0; t < MAXIMA; ++t) v[t] = lane / 4 + 16 * t < slices ? seg0[(lane / 4 + 16 * t) * LOCAL_WORDS + 2 + lane % 4] : 0u;
-        bound = kth_of_wave(v, k, 31, 14, 0u);
+        uint32_t pairs[2] = {0, 0};
+#pragma unroll
+        for (int t = 0; t < MAXIMA; ++t) pairs[t & 1] = max(pairs[t & 1], v[t]);
+        bound = k <= LOCAL_PAIRS_TOPK ? kth_of_wave(pairs, k, 31, 14, 0u) : kth_of_wave(v, k, 31, 14, 0u);
         if (lane == 0) s_bound = bound;
     }
     __syncthreads();

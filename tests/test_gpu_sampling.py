@@ -410,6 +410,12 @@ def _close_logits(kind, vocab, g):
     return x
 
 
+@pytest.mark.parametrize("top_k", [39, 41])
+@pytest.mark.parametrize("kind", ["normal", "one_slice", "close"])
+def test_candidates_by_pairs_of_maxima(dev, po, top_k, kind):
+    test_candidates_by_slices(dev, po, 151936, top_k, kind)
+
+
 @pytest.mark.parametrize("vocab,top_k", [(1000, 64), (1000, 1), (4096, 64), (32000, 40), (131073, 64), (151936, 40), (262144, 20)])
 @pytest.mark.parametrize("kind", ["constant", "few above a mask", "offset", "ramp", "ties left out", "ties below", "ties listed", "ties listed below", "ties at the top"])
 def test_close_values_and_ties_by_slices(dev, po, vocab, top_k, kind):
