@@ -8,7 +8,8 @@
 //
 // What bounds it: 8192 x 8192 x 8192 in 256 x 256 tiles runs at 1190 ... 1400 TFLOP/s on different boxes (a library's product: 1350 ... 1626).  The
 // matrix cores are busy 71 % of the clocks, fragment reads have no bank conflicts, and a wave spends the rest at the barrier of a step and on its
-// reads; 2048 x 19456 x 2560 177 us = 1153 TFLOP/s (the library's 188), busy 50 %, the last round of tiles included.  Reads and fetches in bursts
+// reads; 2048 x 19456 x 2560 177 us = 1153 TFLOP/s (the library's 188), busy 50 %, the last round of tiles included, before the tiles' ends took a sixth
+// of the instructions (gates and ups so, under a tracer, 182 -> 171).  Reads and fetches in bursts
 // behind the barrier cost 10 % more than spread between the MFMAs; four waves with twice the fragments each read a third less LDS and were slower
 // (1160 where this has 1200); workgroups ordered by rows alone, without bands, 900.  Small tiles are bound by how long a fetch takes: three
 // steps in LDS against two bring 128 x 128 from 545 to 760, 128 x 256 from 890 to 1050.

@@ -1483,7 +1483,8 @@ void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int
 // rounds of the chip or all of them - or whether all tiles have 192 - whichever lets the launch end first; returns its time in rounds of 128-row tiles.  A tile of 256 rows takes 1.75
 // times (Q6_K, more to unpack: 1.5 times) as long as one of 128, and where its last round leaves CUs idle, 128-row tiles run there; a tile of 192 rows
 // 1.4 to 1.6 times (Q6_K 1.35), by how much of the chip the other tiles leave idle, that is to say how far they let it clock.  In us, all of 128 rows, all
-// of 256, whole rounds of 256 and 128 behind them, 192, and by this rule (a run of its own: the same plan again differs by up to 12 %):
+// of 256, whole rounds of 256 and 128 behind them, 192, and by this rule (a run of its own: the same plan again differs by up to 12 %; since then
+// qf_store takes 3 to 10 us less of each):
 //   509 x 19456 x 2560     82  79   -   68   63 (192)        Q6_K  107  77   -   70   72 (192)
 //   953 x 19456 x 2560    133 154  129 120  123 (256, 128)
 //   953 x 28672 x 4096    273 234  254 265  238 (256)
