@@ -1444,8 +1444,8 @@ int qgemm_f16_splits(int N, int K, int M) {
 // workgroup: starting from one split each, the matrix whose workgroups have the most work (blocks per split, a Q6_K block
 // weighing 1.6 Q4_K blocks: measured 8 against 5 us) gets its next split count until the slots run out.  A function of
 // the shapes, the types and M's class only, like qgemm_f16_splits.
-// Up to 128 rows one more split where, in workgroups of 128 columns, that takes a fifth off what the busiest CU does: gate and up of 18944 x 3584 in one split are
-// 296 workgroups of 14 blocks, two on some CUs, in two 592 of seven (25 rows, 8 layers: 1002 -> 975 us).
+// (A split more where workgroups of 128 columns would do a fifth less on the busiest CU: 2 x 22016 x 4096, 5 / 32 rows 49.3 / 50.8 -> 45.3 / 48.8 us, but the rows of
+// a class share their splits: 40 / 100 / 128 rows 57.0 / 66.6 / 68.8 -> 67.0 / 87.6 / 90.5; 2 x 24576 x 2048, 32 / 128 rows 30.9 / 43.9 -> 34.1 / 66.3.)
 void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits) {
     const int nblk = K / 256;
     const int row_tiles = qf_row_class(M);
@@ -1468,15 +1468,6 @@ void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int
         slots += ntile[j] * (next - splits[j]);
         splits[j] = next;
     }
-    if (M > 128) return;
-    int tiles = 0;
-    for (int i = 0; i < n; ++i) {
-        if (splits[i] != splits[0]) return;
-        tiles += (N[i] + 127) / 128;
-    }
-    auto blocks = [&](int s) { return (tiles * s + 255) / 256 * ((nblk + s - 1) / s); };
-    if (splits[0] < cap && 5 * blocks(splits[0] + 1) <= 4 * blocks(splits[0]))
-        for (int i = 0; i < n; ++i) ++splits[i];
 }
 
 // Which tiles of a launch of gx column tiles (slots) and gz K splits have 256 rows: the first `tall` pairs of row tiles in qf_tile_of's order, in whole

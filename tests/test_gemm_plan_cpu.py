@@ -125,3 +125,21 @@ def test_row_blocks_that_take_long_do_not_come_last(dq, dv, resident, heads, blo
         return t
 
     assert lasts(got) <= lasts(range(grid)) + 1e-6
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 128, 129, 256, 300, 2048])
+def test_several_quantised_matrices_fit_one_round(rows):
+    """All (column tile, K split) slots of a launch of several matrices in one round of the chip over the row tiles of the rows' class, but for the one split a
+    matrix has at least: a split more leaves CUs with two workgroups of half the blocks, and adds its partial sums."""
+    h, r = harness(), random.Random(5)
+    of_class = 1 if rows <= 128 else 2 if rows <= 256 else 4 if rows <= 1024 else 8
+    shapes = [((24576, 24576), 2048), ((22016, 22016), 4096), ((28672, 28672), 8192), ((9728, 9728), 2560), ((4096, 1024, 1024), 2560)]
+    shapes += [(tuple(256 * r.randint(1, 120) - r.randint(0, 255) for _ in range(r.randint(1, 3))), 256 * r.randint(1, 64)) for _ in range(300)]
+    for N, K in shapes:
+        n = len(N)
+        types = [r.choice([12, 14]) for _ in N]
+        sp = (ctypes.c_int * n)()
+        h.multi_plan(n, (ctypes.c_int * n)(*N), (ctypes.c_uint32 * n)(*types), K, rows, sp)
+        tiles = [-(-x // 256) for x in N]
+        assert sum(t * s for t, s in zip(tiles, sp)) <= max(256 // of_class, sum(tiles)), (N, K, list(sp))
+        assert all(1 <= s <= max(1, min(16 if of_class == 1 else 8, K // 512)) for s in sp)
