@@ -35,7 +35,7 @@ enum { Q4K_THREADS = 256, Q4K_ONE_WAVES = 10 };
 
 // ---- prologue: bring the Q8 activation into LDS; loads first (q4k_stage_issue), the arithmetic after the
 // weight prefetch has been issued (q4k_stage_finish) --------------------------------------------------
-// fp32 x: thread t takes the 16 bytes at t, t + 256, ... - whole lines per instruction.  What bounds these kernels is how fast a CU's waves get
+// fp32 x of the workgroups that share it among many waves or tiles: thread t takes the 16 bytes at t, t + threads, ... - whole lines per instruction.  What bounds these kernels is how fast a CU's waves get
 // their loads out, and an instruction takes a clock for every 64 bytes it touches: with 16 consecutive values a thread (64 bytes apart from lane
 // to lane) the eight loads of x and the norm's weights took the time of 32, and the last of 1216 workgroups had its loads out 5.4 us behind the first.
 template <int NX>
@@ -131,6 +131,20 @@ __device__ __forceinline__ Q4KStage<NX> q4k_stage_issue(const Q4KArgs a, uint8_t
     return st;
 }
 
+// x + RMSNorm(h) * w, h's sum of squares being ssh
+template <int NX>
+__device__ __forceinline__ void q4k_add_normed(const float4 (&x)[NX], const float4 (&h)[NX], const float4 (&w)[NX], float ssh, float one, const Q4KArgs& a,
+                                               float4 (&xv)[NX]) {
+    const float rsh = 1.0f / sqrtf(ssh / (float)a.K + a.eps);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+        xv[u].x = x[u].x + h[u].x * rsh * (w[u].x + one);
+        xv[u].y = x[u].y + h[u].y * rsh * (w[u].y + one);
+        xv[u].z = x[u].z + h[u].z * rsh * (w[u].z + one);
+        xv[u].w = x[u].w + h[u].w * rsh * (w[u].w + one);
+    }
+}
+
 template <bool XQ8, bool NORM, bool PRE, bool SHORT, int NX>
 __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q4KArgs a, uint8_t* lds, float* red, int wg, int threads) {
     const int tid = threadIdx.x;
@@ -144,17 +158,9 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q
             if (i < n16) dst[i] = make_uint4(st.q8[u].x, st.q8[u].y, st.q8[u].z, st.q8[u].w);
         }
     } else if constexpr (PRE) {
-        // x + RMSNorm(h) * w first (threads past the end hold zeros), then the kernel's own RMSNorm of that sum
-        const float ssh = sum_of_waves(q4k_sumsq(st.h, 0.0f), red, threads >> 6);
-        const float rsh = 1.0f / sqrtf(ssh / (float)a.K + a.eps);
+        // the sum first (threads past the end hold zeros), then the kernel's own RMSNorm of it
         float4 xv[NX];
-#pragma unroll
-        for (int u = 0; u < NX; ++u) {
-            xv[u].x = st.x[u].x + st.h[u].x * rsh * (st.w[u].x + one);
-            xv[u].y = st.x[u].y + st.h[u].y * rsh * (st.w[u].y + one);
-            xv[u].z = st.x[u].z + st.h[u].z * rsh * (st.w[u].z + one);
-            xv[u].w = st.x[u].w + st.h[u].w * rsh * (st.w[u].w + one);
-        }
+        q4k_add_normed(st.x, st.h, st.w, sum_of_waves(q4k_sumsq(st.h, 0.0f), red, threads >> 6), one, a, xv);
         if (wg == 0 && a.pre_out) {
 #pragma unroll
             for (int u = 0; u < NX; ++u)
@@ -174,6 +180,119 @@ __device__ __forceinline__ void q4k_stage_finish(const Q4KStage<NX>& st, const Q
         }
 #pragma unroll
         for (int u = 0; u < NX; ++u) q4k_quantize4_store<NORM, SHORT>(st.x[u], st.g[u], rs, one, tid + threads * u, lds, a.K);
+    }
+    __syncthreads();
+}
+
+// Workgroups of four waves that stage x for one tile take half a Q8 block a thread: the 16 consecutive values [16t, 16t + 16) (lanes t, t ^ 1 share a
+// block), so that the quotients of the Q8 rule and what crosses lanes are paid once per 16 values; there each wave's instructions in front of its
+// tile count for more than the lines its loads touch.  q / k / v behind a launch that writes x, in pieces as above and so: 6144 x 4096 8.76, 8.10 us, 3072 x 3584
+// 7.40, 6.87, gate / up 2 x 1536 x 4096 7.46, 6.88, a product of 1024 x 9728 8.28, 6.97, 512 x 18944 10.72, 8.36; the other way round, 0.16, for 2560 to 4096 x 1024
+// and 5120 to 8192 x 512.  (Several tiles a workgroup, pieces: 2 x 14336 x 2560 13.4 us, halves 14.2; 2 x 11008 x 2048 10.2, 9.9.)
+struct Q4KHalves { float4 x[4], g[4], h[4], w[4]; float rs; };
+
+__device__ __forceinline__ void q4k_load16(__amdgpu_buffer_rsrc_t r, int first, float4 (&v)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, (first + 4 * u) * 4, 0, 0);  // zeros past the end
+        v[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
+    }
+}
+// Q8 rule of quantize_x_q8 (reference: torch/io/cpu_quant_gemv.h:147-198) on the half block `unit` (16 values).
+template <bool NORM>
+__device__ __forceinline__ void q4k_quantize16_store(const float4 (&xv)[4], const float4 (&gv)[4], float rs, float one,
+                                                     int unit, uint8_t* lds, int K) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        float4 t = xv[u];
+        if constexpr (NORM) t = norm4(t, gv[u], rs, one);
+        v[4 * u] = t.x; v[4 * u + 1] = t.y; v[4 * u + 2] = t.z; v[4 * u + 3] = t.w;
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    amax = fmaxf(amax, dpp_f<0xB1>(amax));
+    float d, id;
+    q8_scales(amax, d, id);
+    int isum = 0;
+    uint32_t w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        uint32_t q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = (uint32_t)max(-127, min(127, (int)rintf(v[4 * u + i] * id)));
+        w[u] = pack_bytes(q[0], q[1], q[2], q[3]);
+        isum = __builtin_amdgcn_sdot4((int)w[u], 0x01010101, isum, false);
+    }
+    isum += dpp_i<0xB1>(isum);
+    *reinterpret_cast<uint4*>(lds + 16 * unit) = make_uint4(w[0], w[1], w[2], w[3]);
+    if ((unit & 1) == 0) {
+        float* xd = reinterpret_cast<float*>(lds + K);
+        xd[unit >> 1] = d;
+        xd[K / 32 + (unit >> 1)] = d * (float)isum;
+    }
+}
+
+template <bool NORM, bool PRE>
+__device__ __forceinline__ Q4KHalves q4k_halves_issue(const Q4KArgs a, uint8_t* lds, float* red) {
+    static_assert(!PRE || NORM, "the deferred post-norm comes with the RMSNorm prologue");
+    Q4KHalves st;
+    const int tid = threadIdx.x;
+    st.rs = 1.0f;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, a.K * 4);
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(NORM ? static_cast<const void*>(a.gamma) : a.x, a.K * 4);
+    if (a.K > 16 * Q4K_THREADS) {  // first, as above
+        if constexpr (NORM) {
+            float ss = 0.0f;
+            for (int base = 0; base < a.K; base += 16 * Q4K_THREADS) {
+                float4 t[4];
+                q4k_load16(rx, base + 16 * tid, t);
+                ss = q4k_sumsq(t, ss);
+            }
+            ss = block_sum256(ss, red);
+            st.rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+        }
+        for (int base = 16 * Q4K_THREADS; base < a.K; base += 16 * Q4K_THREADS) {
+            float4 t[4], g[4];
+            q4k_load16(rx, base + 16 * tid, t);
+            if constexpr (NORM) q4k_load16(rg, base + 16 * tid, g);
+            if (base + 16 * tid < a.K) q4k_quantize16_store<NORM>(t, g, st.rs, a.add_one ? 1.0f : 0.0f, base / 16 + tid, lds, a.K);
+        }
+    }
+    issue_order_fence();
+    if constexpr (PRE) {
+        q4k_load16(make_rsrc(a.pre_h, a.K * 4), 16 * tid, st.h);
+        q4k_load16(make_rsrc(a.pre_w, a.K * 4), 16 * tid, st.w);
+    }
+    q4k_load16(rx, 16 * tid, st.x);
+    if constexpr (NORM) q4k_load16(rg, 16 * tid, st.g);
+    return st;
+}
+
+template <bool NORM, bool PRE>
+__device__ __forceinline__ void q4k_halves_finish(const Q4KHalves& st, const Q4KArgs a, uint8_t* lds, float* red, int wg) {
+    const int tid = threadIdx.x;
+    const float one = a.add_one ? 1.0f : 0.0f;
+    if constexpr (PRE) {
+        float4 xv[4];
+        q4k_add_normed(st.x, st.h, st.w, block_sum256(q4k_sumsq(st.h, 0.0f), red), one, a, xv);
+        if (wg == 0 && a.pre_out && 16 * tid < a.K) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) reinterpret_cast<float4*>(a.pre_out)[4 * tid + u] = xv[u];
+        }
+        const float ss = block_sum256(q4k_sumsq(xv, 0.0f), red);
+        const float rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+        if (16 * tid < a.K) q4k_quantize16_store<true>(xv, st.g, rs, one, tid, lds, a.K);
+    } else {
+        float rs = st.rs;
+        if constexpr (NORM) {
+            if (a.K <= 16 * Q4K_THREADS) {
+                const float ss = block_sum256(q4k_sumsq(st.x, 0.0f), red);
+                rs = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+            }
+        }
+        if (16 * tid < a.K) q4k_quantize16_store<NORM>(st.x, st.g, rs, one, tid, lds, a.K);
     }
     __syncthreads();
 }
@@ -259,7 +378,7 @@ __device__ __forceinline__ float silu_mul_ref(float g, float u) {
 //     staging.  Addresses are then one base and constants: 70 -> 56 instructions a block, and a launch's setup a third.
 template <bool XQ8, bool NORM, bool ACC, int MODE, int NB, bool ROLLT = false, bool PRE = false, int LS = -1, int PIECES = 4, int EARLY = NB, int DEPTH = NB>
 __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int wg) {
-    constexpr bool ONE = LS >= 0;
+    constexpr bool ONE = LS >= 0, HALVES = !ONE && !XQ8 && !ROLLT;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 7, grp = lane >> 3;
     const int log2S = ONE ? LS : a.log2S;
@@ -389,7 +508,14 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
         });
         return;
     }
-    const auto stg = q4k_stage_issue<XQ8, NORM, PRE, false, XQ8 ? 2 : PIECES>(a, lds, red, Q4K_THREADS);
+    const auto stg = [&] {
+        if constexpr (HALVES) return q4k_halves_issue<NORM, PRE>(a, lds, red);
+        else return q4k_stage_issue<XQ8, NORM, PRE, false, XQ8 ? 2 : PIECES>(a, lds, red, Q4K_THREADS);
+    }();
+    auto finish = [&] {
+        if constexpr (HALVES) q4k_halves_finish<NORM, PRE>(stg, a, lds, red, wg);
+        else q4k_stage_finish<XQ8, NORM, PRE, false>(stg, a, lds, red, wg, Q4K_THREADS);
+    };
     if constexpr (ROLLT) {
         // MODE 0: one matrix (a.W[0], a.y[0]); MODE 1: virtual row 2 r = gate row r (a.W[0]), 2 r + 1 = up row r (a.W[1]).
         // The pointers are taken out of the argument struct once: a select over its arrays per tile would push it to scratch.
@@ -416,7 +542,7 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
             qv[u] = *reinterpret_cast<const uint4*>(p + 16 + 16 * j);
         }
         issue_order_fence();
-        q4k_stage_finish<XQ8, NORM, false, false>(stg, a, lds, red, wg, Q4K_THREADS);
+        finish();
         for (; tile < tile_end; ++tile) {
             const int r_next = tile + 1 < tile_end ? r + 4 * rows_per_wave : r;
             const uint8_t* row_next = row_ptr(r_next);
@@ -452,7 +578,7 @@ __device__ __forceinline__ void q4k_gemv_body(const Q4KArgs a, uint8_t* lds, int
         }
         return;
     }
-    run_tile(wg * tpw, [&] { q4k_stage_finish<XQ8, NORM, PRE, false>(stg, a, lds, red, wg, Q4K_THREADS); });
+    run_tile(wg * tpw, finish);
     // further tiles reuse the staged activations: the quantisation of x is paid once per workgroup
     for (int k = 1; k < tpw; ++k) {
         const int tile = wg * tpw + k;

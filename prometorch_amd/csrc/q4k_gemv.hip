@@ -68,13 +68,12 @@ __global__ __launch_bounds__(1024) void q4k_gemv_rows_kernel(const Q4KArgs a) {
     q4k_gemv_body<false, false, ACC, 0, NB, false, false, 3, PIECES, NB < 2 ? NB : 2, NB < 3 ? NB : 3>(a, lds, blockIdx.x);
 }
 
-// The same for rows of more than ten blocks a lane group, or x of more than eight pieces a thread: passes of two blocks, rolling
-// as in q4k_gemv_body.  XL: values of x a thread quantises, by 16
+// The same for rows of more than ten blocks a lane group and x of more than eight pieces a thread: passes of NB blocks, rolling as in q4k_gemv_body, x staged by half
+// blocks (q4k_halves_issue says why), XL of them a thread.  In pieces 4096 x 25600 took 18.0 us, so 17.4, 2048 x 25600 18.1 and 15.0.
 enum { Q4K_LONGROW_MAX_WAVES = 16 };
-template <bool ACC, int XL>
+template <bool ACC, int NB, int XL>
 __global__ __launch_bounds__(64 * Q4K_LONGROW_MAX_WAVES) void q4k_gemv_longrow_kernel(const uint8_t* __restrict__ W, int64_t stride,
                                                                                        const float* __restrict__ x, float* y, int N, int K) {
-    constexpr int NB = 2;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = tid >> 6, j = lane & 7, sub = lane >> 3;
     const int nblk = K / 256;
@@ -83,8 +82,9 @@ __global__ __launch_bounds__(64 * Q4K_LONGROW_MAX_WAVES) void q4k_gemv_longrow_k
     const uint8_t* row = W + (int64_t)(live ? r : N - 1) * stride;
     // activation loads first (range-checked: zeros past the end), then the weights, then the Q8 arithmetic
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(x, K * 4);
-    float4 xv[4 * XL];
-    q4k_load(rx, tid, nthr, xv);
+    float4 xv[XL][4];
+#pragma unroll
+    for (int u = 0; u < XL; ++u) q4k_load16(rx, 16 * (tid + nthr * u), xv[u]);
     issue_order_fence();
     uint4 hdr[NB], qv[NB];
 #pragma unroll
@@ -95,9 +95,13 @@ __global__ __launch_bounds__(64 * Q4K_LONGROW_MAX_WAVES) void q4k_gemv_longrow_k
     }
     issue_order_fence();
 #pragma unroll
-    for (int u = 0; u < 4 * XL; ++u) q4k_quantize4_store<false>(xv[u], xv[u], 1.0f, 0.0f, tid + nthr * u, lds, K);  // (nthr is a multiple of 64)
+    for (int u = 0; u < XL; ++u) {  // lanes t, t ^ 1 share a block: both inside or both outside (nthr is a multiple of 64)
+        const int unit = tid + nthr * u;
+        if (16 * unit < K) q4k_quantize16_store<false>(xv[u], xv[u], 1.0f, 0.0f, unit, lds, K);
+    }
     __syncthreads();
     const Q4KLane ln = q4k_lane(lds, K, j);
+    // passes roll as in q4k_gemv_body: a consumed block's registers are refilled from the next pass at once
     const int nb_max = (nblk + 7) >> 3;
     float acc = 0.0f;
     int i0 = 0;
@@ -128,7 +132,7 @@ __global__ __launch_bounds__(64 * Q4K_LONGROW_MAX_WAVES) void q4k_gemv_longrow_k
     }
 }
 
-// waves per workgroup and values of x per thread, by 16, of that launch, or waves = 0 when the shape is not one for it.  Up to
+// waves per workgroup and half blocks of x per thread of that launch, or waves = 0 when the shape is not one for it.  Up to
 // 16 rows per CU make one workgroup per CU, up to 32 two (each quantises x for itself).
 struct Q4KLongrow { int waves, xl; };
 static Q4KLongrow q4k_longrow_shape(int N, int K) {
@@ -168,10 +172,17 @@ static int q4k_launch_longrow(const Q4KArgs& a, Q4KLongrow sh, hipStream_t s) {
         return launch_status();
     }
     const float* x = static_cast<const float*>(a.x);
-#define PTM_LR(XL) hipLaunchKernelGGL((q4k_gemv_longrow_kernel<ACC, XL>), grid, block, lds, s, a.W[0], a.stride, x, a.y[0], a.total_rows, a.K)
-    if (sh.xl == 1) PTM_LR(1);
-    else if (sh.xl == 2) PTM_LR(2);
-    else PTM_LR(3);
+#define PTM_LR(NB, XL) hipLaunchKernelGGL((q4k_gemv_longrow_kernel<ACC, NB, XL>), grid, block, lds, s, a.W[0], a.stride, x, a.y[0], a.total_rows, a.K)
+    // blocks in flight per lane group: two; three for workgroups of up to ten waves (2560 x 9728, 10 waves, five blocks per
+    // group: 1 / 2 / 3 / 5 in flight 7.5 / 7.0 / 6.9 / 7.0 us; 3584 x 18944, 14 waves: 1 / 2 / 3 in flight 12.8 / 11.3 / 12.2).  A half block a
+    // thread and more than eight pieces are not both there; ten blocks a group and one half block a thread need a row of 2 GiB.
+    if (sh.waves <= 10) {
+        if (sh.xl <= 2) PTM_LR(3, 2);
+        else PTM_LR(3, 3);
+    } else {
+        if (sh.xl <= 2) PTM_LR(2, 2);
+        else PTM_LR(2, 3);
+    }
 #undef PTM_LR
     return launch_status();
 }

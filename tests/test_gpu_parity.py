@@ -478,6 +478,32 @@ def test_one_pass_projections_vs_oracle(dev, po, nq, nk, nv, K):
     assert np.array_equal(bits(added[:-4]), bits(np.float32(0.5) + plain[:-4])) and np.all(added[-4:] == 0.5)
 
 
+@pytest.mark.parametrize("N,K,add_one", [(300, 256, False), (256, 2816, True), (1024, 4096, True), (777, 4352, False), (768, 4096, False), (3072, 3584, False), (40, 8192, True),
+                                         (1025, 9728, False), (513, 9472, False), (700, 20736, False), (2817, 21248, False), (2100, 32768, False), (512, 18944, False)])
+def test_q4k_staging_by_half_blocks_vs_oracle(dev, po, N, K, add_one):
+    """Workgroups of four waves, 16 values of x a thread: one round of them or more, the last threads without any, behind RMSNorm (bars as above) and plain; rows of long
+    vectors, two and three rounds, two and three blocks of a group in flight.  Plain is also the product of the Q8 blocks, and what is added to y."""
+    r = synth.rng_for(62, N, K)
+    W, x = synth.make_q4k(r, N, K), synth.make_x(r, K)
+    stride, Wd, xd = W.shape[1], cu(W), cu(x)
+    y, q8 = torch.full((N + 4,), 5.0, device="cuda"), torch.empty(ops.q8_bytes(K), dtype=torch.uint8, device="cuda")
+    ops.quant_gemv(12, Wd, xd, y, K, N, stride)
+    plain = y.cpu().numpy()
+    assert rel_err(plain[:N], po.gemv(12, W, x)) <= GEMV_TOL and np.all(plain[N:] == 5.0)
+    ops.quant_gemv(12, Wd, xd, y, K, N, stride, accumulate=True)
+    assert np.array_equal(bits(y.cpu().numpy()[:N]), bits(plain[:N] + plain[:N]))
+    ops.launch_quantize_q8(xd, q8, K)
+    ops.launch_q4km_q8_gemv(Wd, q8, y, K, N, stride)
+    assert np.abs(y.cpu().numpy()[:N] - plain[:N]).max() <= 1e-5 * np.abs(plain[:N]).max()  # the same Q8 blocks: 32-bit sums in another order
+    gam = (0.1 * r.standard_normal(K) + (0.0 if add_one else 1.0)).astype(np.float32)
+    y.fill_(5.0)
+    ops.launch_q4km_fused_rmsnorm_gemv(xd, cu(gam), Wd, y, K, N, stride, 1e-6, add_one)
+    ref = po.gemv(12, W, po.rmsnorm(x, gam + np.float32(1.0) if add_one else gam, 1e-6)).astype(np.float64)
+    got = y.cpu().numpy()
+    err = np.abs(got[:N] - ref) / np.sqrt((ref ** 2).mean())
+    assert np.median(err) <= GEMV_TOL and err.max() <= 2e-2 and np.all(got[N:] == 5.0)
+
+
 # ---------------------------------------------------------------------------------------------
 # glue
 # ---------------------------------------------------------------------------------------------
