@@ -68,7 +68,7 @@ __global__ __launch_bounds__(1024) void q4k_gemv_rows_kernel(const Q4KArgs a) {
     q4k_gemv_body<false, false, ACC, 0, NB, false, false, 3, PIECES, NB < 2 ? NB : 2, NB < 3 ? NB : 3>(a, lds, blockIdx.x);
 }
 
-// The same for rows of more than ten blocks a lane group and x of more than eight pieces a thread: passes of NB blocks, rolling as in q4k_gemv_body, x staged by half
+// The same for rows of more than ten blocks a lane group, x of more than eight pieces a thread and where it is faster (q4k_rows_in_order): passes of NB blocks, rolling as in q4k_gemv_body, x staged by half
 // blocks (q4k_halves_issue says why), XL of them a thread.  In pieces 4096 x 25600 took 18.0 us, so 17.4, 2048 x 25600 18.1 and 15.0.
 enum { Q4K_LONGROW_MAX_WAVES = 16 };
 template <bool ACC, int NB, int XL>
@@ -161,12 +161,20 @@ static void (*q4k_rows_kernel(int nb))(const Q4KArgs) {
         default: return q4k_gemv_rows_kernel<ACC, 10, PIECES>;
     }
 }
+// Whether x in pieces and blocks in an order (q4k_gemv_rows_kernel) is faster than the passes of the other, for rows of up to ten blocks a lane group.  us behind a launch
+// that writes x, so and in passes: two and three waves are too few to share the staging, 512 x 4096 6.09, 5.20, 768 x 6144 6.21, 5.65.  Of two
+// blocks a group (4096 values) nothing is left to request in order, and it is the staging of 12 waves and more that counts: 2816 x 4096 5.89, 6.07, 3584 6.51,
+// 6.32, 4096 6.69, 6.28; two workgroups a CU, 5120 x 4096 7.44, 7.21, 6144 7.66, 7.27, but 7168 8.49, 8.74, 8192 8.41, 8.43.  Others 0.1 to 1.3 less so.
+bool q4k_rows_in_order(int N, int K, int waves) {
+    return waves >= 4 && (K > 4096 || (N <= 256 * Q4K_LONGROW_MAX_WAVES ? waves <= 11 : waves > 12));
+}
+
 template <bool ACC>
 static int q4k_launch_longrow(const Q4KArgs& a, Q4KLongrow sh, hipStream_t s) {
     const dim3 grid((a.total_rows + sh.waves - 1) / sh.waves), block(64 * sh.waves);
     const size_t lds = (size_t)q8_bytes(a.K);
     const int nb = (a.K / 256 + 7) / 8, pieces = (a.K / 4 + 64 * sh.waves - 1) / (64 * sh.waves);
-    if (nb <= 10 && pieces <= 8 && a.stride < 1ll << 31) {
+    if (q4k_rows_in_order(a.total_rows, a.K, sh.waves) && nb <= 10 && pieces <= 8 && a.stride < 1ll << 31) {
         const auto kernel = pieces <= 4 ? q4k_rows_kernel<ACC, 4>(nb) : q4k_rows_kernel<ACC, 8>(nb);
         hipLaunchKernelGGL(kernel, grid, block, lds, s, a);
         return launch_status();
@@ -174,13 +182,14 @@ static int q4k_launch_longrow(const Q4KArgs& a, Q4KLongrow sh, hipStream_t s) {
     const float* x = static_cast<const float*>(a.x);
 #define PTM_LR(NB, XL) hipLaunchKernelGGL((q4k_gemv_longrow_kernel<ACC, NB, XL>), grid, block, lds, s, a.W[0], a.stride, x, a.y[0], a.total_rows, a.K)
     // blocks in flight per lane group: two; three for workgroups of up to ten waves (2560 x 9728, 10 waves, five blocks per
-    // group: 1 / 2 / 3 / 5 in flight 7.5 / 7.0 / 6.9 / 7.0 us; 3584 x 18944, 14 waves: 1 / 2 / 3 in flight 12.8 / 11.3 / 12.2).  A half block a
-    // thread and more than eight pieces are not both there; ten blocks a group and one half block a thread need a row of 2 GiB.
-    if (sh.waves <= 10) {
+    // group: 1 / 2 / 3 / 5 in flight 7.5 / 7.0 / 6.9 / 7.0 us; 3584 x 18944, 14 waves: 1 / 2 / 3 in flight 12.8 / 11.3 / 12.2).  One half block
+    // of x a thread is there for 4096 values only: of more, eight pieces are.
+    if (nb > 2 && sh.waves <= 10) {
         if (sh.xl <= 2) PTM_LR(3, 2);
         else PTM_LR(3, 3);
     } else {
-        if (sh.xl <= 2) PTM_LR(2, 2);
+        if (sh.xl == 1) PTM_LR(2, 1);
+        else if (sh.xl == 2) PTM_LR(2, 2);
         else PTM_LR(2, 3);
     }
 #undef PTM_LR

@@ -478,6 +478,22 @@ def test_one_pass_projections_vs_oracle(dev, po, nq, nk, nv, K):
     assert np.array_equal(bits(added[:-4]), bits(np.float32(0.5) + plain[:-4])) and np.all(added[-4:] == 0.5)
 
 
+@pytest.mark.parametrize("N,K", [(257, 4096), (512, 4096), (700, 6144), (768, 4608), (2816, 4096), (2820, 4096), (4093, 4096), (4100, 4096), (6140, 4096), (6150, 4096)])
+def test_q4k_rows_in_passes_vs_oracle(dev, po, N, K):
+    """Two and three waves a workgroup, and rows of 4096 values either side of the lines: plain, added to y bit for bit, and the product of the Q8 blocks."""
+    r = synth.rng_for(63, N, K)
+    W, x = synth.make_q4k(r, N, K), synth.make_x(r, K)
+    Wd, xd, y, q8 = cu(W), cu(x), torch.full((N + 4,), 5.0, device="cuda"), torch.empty(ops.q8_bytes(K), dtype=torch.uint8, device="cuda")
+    ops.quant_gemv(12, Wd, xd, y, K, N, W.shape[1])
+    plain = y.cpu().numpy()
+    assert rel_err(plain[:N], po.gemv(12, W, x)) <= GEMV_TOL and np.all(plain[N:] == 5.0)
+    ops.quant_gemv(12, Wd, xd, y, K, N, W.shape[1], accumulate=True)
+    assert np.array_equal(bits(y.cpu().numpy()[:N]), bits(plain[:N] + plain[:N]))
+    ops.launch_quantize_q8(xd, q8, K)
+    ops.launch_q4km_q8_gemv(Wd, q8, y, K, N, W.shape[1])
+    assert np.abs(y.cpu().numpy()[:N] - plain[:N]).max() <= 1e-5 * np.abs(plain[:N]).max()  # the same Q8 blocks: 32-bit sums in another order
+
+
 @pytest.mark.parametrize("N,K,add_one", [(300, 256, False), (256, 2816, True), (1024, 4096, True), (777, 4352, False), (768, 4096, False), (3072, 3584, False), (40, 8192, True),
                                          (1025, 9728, False), (513, 9472, False), (700, 20736, False), (2817, 21248, False), (2100, 32768, False), (512, 18944, False)])
 def test_q4k_staging_by_half_blocks_vs_oracle(dev, po, N, K, add_one):
