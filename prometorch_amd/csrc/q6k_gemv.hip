@@ -47,7 +47,7 @@ __global__ __launch_bounds__(64 * Q6K_ROWS_MAX_WAVES) void q6k_gemv_rows_kernel(
     q6k_one_body<ACC, false, false, 3, NT, NT < 2 ? NT : 2, PIECES>(a, lds_raw, blockIdx.x);
 }
 
-// The same for rows that kernel has not (17 to 32 a CU, more than 20480 values): with 4 rows per workgroup every workgroup
+// The same for rows that kernel has not (17 to 32 a CU, more than 20480 values; q6k_rows_waves): with 4 rows per workgroup every workgroup
 // would stage the whole activation vector for 4 rows' worth of weights, and the staging traffic through L2 would
 // exceed the weights'.  Here a workgroup is `waves` waves of 8 >> LOG2S rows each (a row's super-blocks strided over
 // 1 << LOG2S lane groups), sized so that the launch is one workgroup per CU.
@@ -189,7 +189,7 @@ static int q6k_launch_tall_nb(const Q6KArgs& a, int waves, hipStream_t s) {
     if (waves > 12) {
         if (xl <= 8) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, false, 16>), dim3(grid), dim3(64 * waves), lds, s, a);
         else hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, true, 16>), dim3(grid), dim3(64 * waves), lds, s, a);
-    } else if (LOG2S == 2 && xl <= 4) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, LOG2S == 2 ? 4 : 8, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
+    } else if (xl <= 4) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 4, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
     else if (xl <= 8) hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S>), dim3(grid), dim3(64 * waves), lds, s, a);
     else hipLaunchKernelGGL((q6k_gemv_tall_kernel<ACC, NB, 8, LOG2S, true>), dim3(grid), dim3(64 * waves), lds, s, a);
     return launch_status();
@@ -283,9 +283,9 @@ static void q6k_raise_lds_cap() {
 template <bool ACC, int LOG2S>
 static void q6k_raise_lds_cap_tall() {
     const int cap = 144 * 1024;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, LOG2S == 2 ? 4 : 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 4, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, LOG2S == 2 ? 4 : 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 4, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 1, 8, LOG2S, true>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_gemv_tall_kernel<ACC, 2, 8, LOG2S, true>), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
@@ -380,10 +380,25 @@ static void (*q6k_rows_kernel(int nt))(const Q6KArgs) {
         default: return q6k_gemv_rows_kernel<ACC, 10, PIECES>;
     }
 }
-// the waves of that launch, 0 where rows or blocks are too many or a thread would have more than eight pieces of x
-static int q6k_rows_waves(int N, int K) {
-    const int per_cu = (N + 255) / 256, waves = per_cu < 2 ? 2 : per_cu;
-    return per_cu <= Q6K_ROWS_MAX_WAVES && K <= 10 * 8 * 256 && (K / 4 + 64 * waves - 1) / (64 * waves) <= 8 ? waves : 0;
+// The waves of that launch, 0 where the kernels it goes in front of are faster or it cannot be (rows, blocks, or more than eight pieces of x a thread).
+// us behind a launch that writes x, so and before.  Where not every lane group of a wave has a block, each wave's way to its tile is too long for many
+// of them: 4096 x 256 5.34, 4.44, x 512 5.76, 4.89, x 1024 5.71, 5.38; 2048 x 512 within 0.1, 1024 x 512 0.3 to 0.55 less so.  One block a group: 0.3 to 0.9 less.  Two,
+// added to y, whose old values go out first: up to 0.5 less, but of most rows and less than 3584 values 0.1 to 0.3 more (4096 x 2560); as stored up to
+// 0.54 more (4096 x 2560 7.72, 7.25), but of five and six rows a CU (eleven, of more than 3072 values), and of 4096 values from 13, 0.1 to 0.4 less.  Three to ten,
+// added: up to 1.5 less, but 16 rows of 4352 to 5120 values, added or not, 0.3 more.  As stored, up to twelve rows of four blocks 0.2 to 0.6 more
+// (1024 x 8192), twelve and more of seven 0.1 to 0.4, of eight to ten up to 1.1 (3328 x 20480); others 0.45 more (1536 x 12288) to 1.0 less.  The sums are the same on
+// both sides but of 16 rows a CU, where added and stored are on the same (14336 values, as stored, within 0.16).
+int q6k_rows_waves(int N, int K, bool accumulate) {
+    const int nblk = K / 256, blocks = (nblk + 7) / 8, per_cu = (N + 255) / 256, waves = per_cu < 2 ? 2 : per_cu;
+    if (per_cu > Q6K_ROWS_MAX_WAVES || blocks > 10 || (K / 4 + 64 * waves - 1) / (64 * waves) > 8) return 0;
+    bool faster;
+    if (blocks == 1) faster = nblk > 4 || per_cu <= (nblk > 2 ? 12 : 6);
+    else if (blocks == 3 && nblk <= 20 && per_cu == 16) faster = false;
+    else if (accumulate) faster = blocks > 2 || nblk >= 14 || per_cu <= 14;
+    else if (blocks == 2) faster = nblk == 16 ? per_cu >= 13 : per_cu >= 5 && per_cu <= (nblk > 12 ? 11 : 6);
+    else if (blocks == 4) faster = per_cu >= 13;
+    else faster = blocks < 7 || per_cu <= 11 || (per_cu == 16 && K < 16384);
+    return faster ? waves : 0;
 }
 
 template <bool ACC, bool ARGMAX, bool NORM>
@@ -393,7 +408,7 @@ static int q6k_launch(Q6KArgs& a, hipStream_t s) {
     const int grid = q6k_workgroups(a.N, a.K);
     const size_t lds = q6k_x_lds_bytes(a.K);
     if constexpr (!ARGMAX && !NORM) {
-        if (const int waves = q6k_rows_waves(a.N, a.K)) {
+        if (const int waves = q6k_rows_waves(a.N, a.K, ACC)) {
             if (lds > 64 * 1024) q6k_init_attributes();
             const int nt = (a.K / 256 + 7) / 8;
             const auto kernel = a.K / 4 <= 4 * 64 * waves ? q6k_rows_kernel<ACC, 4>(nt) : q6k_rows_kernel<ACC, 8>(nt);

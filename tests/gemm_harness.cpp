@@ -29,6 +29,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
 size_t qgemm_f16_multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M);
 void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits);
 bool q4k_rows_in_order(int N, int K, int waves);
+int q6k_rows_waves(int N, int K, bool accumulate);
 int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
 }
 
@@ -131,6 +132,7 @@ int64_t multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int
 void multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits) { ptm::qgemm_f16_multi_plan(n, N, types, K, M, splits); }
 
 int q4k_rows_in_order(int N, int K, int waves) { return ptm::q4k_rows_in_order(N, K, waves) ? 1 : 0; }
+int q6k_rows_waves(int N, int K, int accumulate) { return ptm::q6k_rows_waves(N, K, accumulate != 0); }
 
 int64_t act_down_bytes(int M, int K) { return ptm_qgemm_f16_workspace_bytes(M, K) + ptm::qgemm_f16_split_scale_bytes(M); }
 // Y = down . (act(gate) . up) of rows that are still slabs, in ws of act_down_bytes

@@ -14,3 +14,14 @@ def _waves(N):
 def test_q4k_long_rows(N, K, in_order):
     """Sides of the lines as they were measured: few waves, and rows of 4096 values in the largest workgroups, go in passes."""
     assert harness().q4k_rows_in_order(N, K, _waves(N)) == in_order
+
+
+@pytest.mark.parametrize("N,K,stored,added", [(1536, 256, 6, 6), (1537, 256, 0, 0), (4096, 512, 0, 0), (3072, 768, 12, 12), (3073, 1024, 0, 0), (4096, 1280, 16, 16), (1, 2048, 2, 2),
+                                              (4096, 2560, 0, 0), (3584, 2560, 0, 14), (1280, 2304, 5, 5), (1536, 3840, 6, 6), (1537, 2816, 0, 7), (2816, 3328, 11, 11), (2817, 3840, 0, 12),
+                                              (4096, 4352, 0, 0), (3841, 5120, 0, 0), (3840, 4608, 15, 15), (4096, 5376, 16, 16), (4096, 3584, 0, 16),
+                                              (3073, 4096, 13, 13), (3072, 4096, 0, 12), (2560, 9728, 10, 10), (3072, 8192, 0, 12), (3073, 6400, 13, 13), (2816, 14336, 11, 11),
+                                              (3072, 13312, 0, 12), (4096, 14336, 16, 16), (4096, 16384, 0, 16), (4097, 2304, 0, 0), (2560, 20736, 0, 0)])
+def test_q6k_rows_a_wave(N, K, stored, added):
+    """Waves of the kernel with a row per wave, 0 where the ones before it are faster: sides of the lines as they were measured."""
+    h = harness()
+    assert (h.q6k_rows_waves(N, K, 0), h.q6k_rows_waves(N, K, 1)) == (stored, added)

@@ -256,6 +256,13 @@ def test_q6k_rows_vs_oracle(dev, po, N, K):
     assert np.array_equal(bits(gpu_gemv(14, W, x, accumulate=True, y0=y0)), bits(y0 + y))
 
 
+@pytest.mark.parametrize("N,K", [(1536, 256), (1537, 512), (3072, 1024), (3073, 768), (1281, 2304), (1540, 2816), (3585, 3328), (3590, 3584), (3072, 4096), (3073, 4096), (3070, 7168), (3080, 8192),
+                                 (2816, 13312), (3072, 14336), (4090, 14592), (4096, 18944)])
+def test_q6k_rows_around_the_lines_vs_oracle(dev, po, N, K):
+    """Either side of where a row per wave takes over, which is another place for sums that are stored and for ones that are added: they stay the same sums."""
+    test_q6k_rows_vs_oracle(dev, po, N, K)
+
+
 def test_gemv_ragged_vs_reference_golden(dev, golden, seeds):
     rr = synth.rng_for(seeds["ragged"])
     for i, (qt, N, K) in enumerate([(12, 33, 512), (12, 1, 256), (12, 77, 2560), (14, 7, 256), (14, 45, 1024)]):
