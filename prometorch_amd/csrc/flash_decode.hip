@@ -326,22 +326,24 @@ __global__ __launch_bounds__(FD_THREADS) void flash_decode_partial_kernel(
 // LDS behind three barriers: 3.9).  Where a cache can hold more, four WAVES take 64 each in turn:
 // 16 heads of 64 over 4 kv heads, 33000 / 131072 positions, partials and merge 22.0 / 59.6 us (one wave 27.7 / 83.5, the workgroup of
 // four 23.2 / 64.0); the three waves cost 0.3 us where a cache that long is still short.
-template <int HD, int WAVES>
+template <int HD, int WAVES, bool CHUNKS_OF_80>
 __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const float* __restrict__ pO, const float* __restrict__ pL,
                                                                         const float* __restrict__ pM, float* __restrict__ O,
                                                                         int n_heads, const int64_t* __restrict__ d_past,
                                                                         int64_t past_host, int max_seq,
-                                                                        uint8_t* __restrict__ q8_out, int chunk_arg, int log2_units) {
+                                                                        uint8_t* __restrict__ q8_out, int chunk_shift, int log2_units) {
     constexpr int NOUT = HD / 4;
     const int h = blockIdx.x, lane = threadIdx.x & 63, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = lane >> 3, o_idx = blockIdx.y * 8 + (lane & 7);
     const float4* pO4 = reinterpret_cast<const float4*>(pO);
     // Every load of the common case goes out before the position is known: chunk slots past the last active one
     // are clamped into the allocation (ns_max chunks) and dropped by selects below, so the first wave makes one
     // memory round trip, not one for the position and a second for the data; the others are there for long contexts only.
-    // chunk < 0: the partials of the looping kernel (at most FD_LONG_SPLITS of them, cpw chunks of 64 positions each)
-    const bool long_mode = chunk_arg < 0;
-    const int chunk = long_mode ? (int)FD_CHUNK : chunk_arg;  // positions per chunk
-    const int ns_max = long_mode ? min((max_seq + chunk - 1) / chunk, (int)FD_LONG_SPLITS) : (max_seq + chunk - 1) / chunk;
+    // chunk_shift < 0: the partials of the looping kernel (at most FD_LONG_SPLITS of them, cpw chunks of 64 positions each)
+    const bool long_mode = !CHUNKS_OF_80 && chunk_shift < 0;
+    const int cs_ = long_mode ? 6 : chunk_shift;
+    // of 80 a constant, of the others a shift: a division by an argument put 0.1 us in front of every merge
+    auto chunks_of = [cs_](int n) { return CHUNKS_OF_80 ? (n + 79) / 80 : (n + (1 << cs_) - 1) >> cs_; };
+    const int ns_max = long_mode ? min(chunks_of(max_seq), (int)FD_LONG_SPLITS) : chunks_of(max_seq);
     const int64_t past = d_past ? *d_past : past_host;
     // partial maxima are natural-log scores, or base-2 ones (log2_units) from the matrix-core kernel
     const float ek = log2_units ? 1.0f : 1.44269504088896340736f;
@@ -371,7 +373,7 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
     int64_t total = past + 1;
     if (total > max_seq) total = max_seq;
     if (total <= 0) return;
-    const int n_chunks = ((int)total + chunk - 1) / chunk;
+    const int n_chunks = chunks_of((int)total);
     const int cpw_ = long_mode ? (n_chunks + (int)FD_LONG_SPLITS - 1) / (int)FD_LONG_SPLITS : 1;
     const int ns = long_mode ? (n_chunks + cpw_ - 1) / cpw_ : n_chunks;
     const bool together = WAVES > 1 && ns > 64;  // the same in every thread
@@ -440,18 +442,23 @@ __global__ __launch_bounds__(64 * WAVES) void flash_decode_merge_kernel(const fl
     }
 }
 
-template <int HD, int WAVES>
+template <int HD, int WAVES, bool CHUNKS_OF_80 = false>
 static void fd_merge_launch(int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O, const int64_t* d_past,
-                            int64_t past_host, int max_seq, uint8_t* q8_out, int chunk_arg, int log2_units) {
-    hipLaunchKernelGGL((flash_decode_merge_kernel<HD, WAVES>), dim3(n_heads, HD / 32), dim3(64 * WAVES), 0, s, pO, pL, pM, O, n_heads, d_past,
-                       past_host, max_seq, q8_out, chunk_arg, log2_units);
+                            int64_t past_host, int max_seq, uint8_t* q8_out, int chunk_shift, int log2_units) {
+    hipLaunchKernelGGL((flash_decode_merge_kernel<HD, WAVES, CHUNKS_OF_80>), dim3(n_heads, HD / 32), dim3(64 * WAVES), 0, s, pO, pL, pM, O, n_heads, d_past,
+                       past_host, max_seq, q8_out, chunk_shift, log2_units);
 }
 
 static int fd_merge(int head_dim, int n_heads, hipStream_t s, const float* pO, const float* pL, const float* pM, float* O,
                     const int64_t* d_past, int max_seq, uint8_t* q8_out = nullptr, int64_t past_host = 0,
                     int chunk = FD_CHUNK, int log2_units = 0) {
-    const int most = chunk < 0 ? (int)FD_LONG_SPLITS : (int)(((int64_t)max_seq + chunk - 1) / chunk);  // splits there can be
-#define PTM_FDM(HDV, WV) fd_merge_launch<HDV, WV>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, chunk, log2_units)
+    if (chunk == 80) {  // heads of 128, at most 51 chunks
+        fd_merge_launch<128, 1, true>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, 0, log2_units);
+        return launch_status();
+    }
+    const int chunk_shift = chunk < 0 ? -1 : chunk == 128 ? 7 : 6;
+    const int most = chunk_shift < 0 ? (int)FD_LONG_SPLITS : (int)(((int64_t)max_seq + chunk - 1) >> chunk_shift);  // splits there can be
+#define PTM_FDM(HDV, WV) fd_merge_launch<HDV, WV>(n_heads, s, pO, pL, pM, O, d_past, past_host, max_seq, q8_out, chunk_shift, log2_units)
 #define PTM_FDMW(HDV) (most <= 64 ? PTM_FDM(HDV, 1) : PTM_FDM(HDV, 4))
     if (head_dim == 256) PTM_FDMW(256);
     else if (head_dim == 128) PTM_FDMW(128);
@@ -1161,24 +1168,23 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(const Attn
         }
         return;
     }
-    // ---- merge the wave partials into the chunk's partial ----
+    // ---- merge the four or five wave partials into the chunk's partial ----
+    static_assert(ONE || WAVES == 4 || WAVES == 5, "the merge below");
     for (int e = tid; e < G * HD; e += 64 * WAVES) {
         const int g = e / HD, d = e % HD;
-        float mw[WAVES], w[WAVES], M = -INFINITY;  // finite in the end: the chunk holds at least one valid position
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) M = fmaxf(M, mw[i] = s_m[i][g]);
-        float o = 0.0f, l = 0.0f;
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) {
-            w[i] = __builtin_amdgcn_exp2f(mw[i] - M);
-            o += w[i] * s_o[i][d][g];
-        }
+        const float m0 = s_m[0][g], m1 = s_m[1][g], m2 = s_m[2][g], m3 = s_m[3][g];
+        float M = fmaxf(fmaxf(m0, m1), fmaxf(m2, m3));  // finite in the end: the chunk holds at least one valid position
+        if constexpr (WAVES == 5) M = fmaxf(M, s_m[4][g]);
+        const float w0 = __builtin_amdgcn_exp2f(m0 - M), w1 = __builtin_amdgcn_exp2f(m1 - M),
+                    w2 = __builtin_amdgcn_exp2f(m2 - M), w3 = __builtin_amdgcn_exp2f(m3 - M);
+        float o = (w0 * s_o[0][d][g] + w1 * s_o[1][d][g]) + (w2 * s_o[2][d][g] + w3 * s_o[3][d][g]);
+        if constexpr (WAVES == 5) o += __builtin_amdgcn_exp2f(s_m[4][g] - M) * s_o[4][d][g];
         const int64_t oi = (int64_t)split * a.n_heads + kvh * G + g;
         a.pO[oi * HD + d] = o;
         if (d == 0) {
-#pragma unroll
-            for (int i = 0; i < WAVES; ++i) l += w[i] * s_l[i][g];
             a.pM[oi] = M;
+            float l = (w0 * s_l[0][g] + w1 * s_l[1][g]) + (w2 * s_l[2][g] + w3 * s_l[3][g]);
+            if constexpr (WAVES == 5) l += __builtin_amdgcn_exp2f(s_m[4][g] - M) * s_l[4][g];
             a.pL[oi] = l;
         }
     }
