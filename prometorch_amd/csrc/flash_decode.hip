@@ -1548,6 +1548,18 @@ static int fd_launch_g(int G, dim3 grid, hipStream_t s, const float* Q, const vo
     return launch_status();
 }
 
+// Chunks of 80 positions, five waves, where those of 64 make more workgroups than the chip has CUs and those of 80 do not: a CU's L1 returns what was asked of it in
+// order, and a second workgroup's query, rotation row and keys come behind the rows of the first, 0.8 us of the launch's 3.9 behind its arguments.
+// At few positions the fifth wave costs 0.2 to 0.6 us of 8 to 10.  Both launches behind one that writes Q, over the positions of a cache, in 16
+// steps: 32 heads on 8, room for 2240 / 2304 / 2368 / 2496 0.21 / 0.35 / 0.34 / 0.11 us less on average (0.3 to 0.9 more up to position 140,
+// 0.4 to 0.6 less from 1000 on); 40 on 10, 1750 / 1850 / 2000 0.36 / 0.40 / 0.43; 64 on 8, 2304 0.28; 32 on 16, 1088 0.23.  Of eight workgroups more than CUs it is
+// faster behind position 1600 only, 0.17 (32 on 8, 2064) to 0.38 us (64 on 8) slower on average; one query head a kv head is up to 0.14 slower at
+// any room (8 on 8, 2304: 0.03 less).
+bool attn_five_waves(int head_dim, int n_heads, int n_kv_heads, int max_seq) {
+    const int64_t chunks = ((int64_t)max_seq + FD_CHUNK - 1) / FD_CHUNK, wide = ((int64_t)max_seq + 79) / 80;
+    return head_dim == 128 && n_heads > n_kv_heads && chunks <= FD_LONG_SPLITS && chunks * n_kv_heads > 264 && wide * n_kv_heads <= 256;
+}
+
 }  // namespace ptm
 
 using namespace ptm;
@@ -1690,13 +1702,8 @@ int ptm_attn_decode_fused_bias(const float* Q, const float* K, const float* V, c
             return fd_merge(head_dim, n_heads, s, partial_O, partial_lse, partial_max, O, d_past_len, max_seq,
                             static_cast<uint8_t*>(o_q8), 0, -1, 1);
         }
-        // Chunks of 80 positions, five waves, where those of 64 make a few workgroups more than the chip has CUs: a CU's L1 returns what was asked of it
-        // in order, and a second workgroup's query, rotation row and keys come behind the rows of the first, 0.8 us of the launch's 3.9 behind its
-        // arguments.  Eight steps of Qwen3-4B shapes at 2048 positions (264 workgroups of four waves, 208 of five) 9835 -> 9705 us; six waves 9750,
-        // eight 9825.
-        const int wide = (max_seq + 79) / 80;
-        if (head_dim == 128 && (int)grid.x * n_kv_heads > 256 && wide * n_kv_heads <= 256) {
-            const dim3 grid5(wide, n_kv_heads);
+        if (attn_five_waves(head_dim, n_heads, n_kv_heads, max_seq)) {
+            const dim3 grid5((max_seq + 79) / 80, n_kv_heads);
             rc = bias ? attn_mfma_launch_g<128, 1, true, 5>(G, grid5, s, a) : attn_mfma_launch_g<128, 1, false, 5>(G, grid5, s, a);
             if (rc != PTM_OK) return rc;
             return fd_merge(head_dim, n_heads, s, partial_O, partial_lse, partial_max, O, d_past_len, max_seq, static_cast<uint8_t*>(o_q8), 0, 80, 1);

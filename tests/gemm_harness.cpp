@@ -28,6 +28,7 @@ int qgemm_f16_multi(int n, const uint32_t* types, const void* const* W, const in
                     const float** deferred_P, int* deferred_splits);
 size_t qgemm_f16_multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M);
 void qgemm_f16_multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits);
+bool attn_five_waves(int head_dim, int n_heads, int n_kv_heads, int max_seq);
 bool q4k_rows_in_order(int N, int K, int waves);
 int q6k_rows_waves(int N, int K, bool accumulate);
 int qgemm_f16_act_rows(const float* G, const float* U, int sg, int su, bool gelu, bool rounded, void* ws, int bps, int M, int K, hipStream_t s);
@@ -131,6 +132,7 @@ int multi_run(int n, const uint32_t* types, const void* const* W, const int64_t*
 int64_t multi_split_bytes(int n, const int* N, const uint32_t* types, int K, int M) { return (int64_t)ptm::qgemm_f16_multi_split_bytes(n, N, types, K, M); }
 void multi_plan(int n, const int* N, const uint32_t* types, int K, int M, int* splits) { ptm::qgemm_f16_multi_plan(n, N, types, K, M, splits); }
 
+int attn_five_waves(int head_dim, int n_heads, int n_kv_heads, int max_seq) { return ptm::attn_five_waves(head_dim, n_heads, n_kv_heads, max_seq) ? 1 : 0; }
 int q4k_rows_in_order(int N, int K, int waves) { return ptm::q4k_rows_in_order(N, K, waves) ? 1 : 0; }
 int q6k_rows_waves(int N, int K, int accumulate) { return ptm::q6k_rows_waves(N, K, accumulate != 0); }
 

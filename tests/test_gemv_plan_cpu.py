@@ -1,4 +1,4 @@
-"""CPU: which kernel takes a product of few long rows, where two of them could."""
+"""CPU: which kernel takes a product of few long rows, or a step's attention, where two of them could."""
 import pytest
 
 from gemm_helpers import harness
@@ -25,3 +25,11 @@ def test_q6k_rows_a_wave(N, K, stored, added):
     """Waves of the kernel with a row per wave, 0 where the ones before it are faster: sides of the lines as they were measured."""
     h = harness()
     assert (h.q6k_rows_waves(N, K, 0), h.q6k_rows_waves(N, K, 1)) == (stored, added)
+
+
+@pytest.mark.parametrize("dim,heads,kv_heads,room,five", [(128, 32, 8, 2048, 0), (128, 32, 8, 2112, 0), (128, 32, 8, 2113, 1), (128, 32, 8, 2560, 1), (128, 32, 8, 2561, 0), (128, 8, 8, 2304, 0),
+                                                          (128, 40, 10, 1664, 0), (128, 40, 10, 1700, 1), (128, 32, 16, 1025, 1), (128, 32, 32, 600, 0), (128, 64, 32, 600, 1),
+                                                          (64, 32, 8, 2304, 0), (128, 20, 5, 4096, 0), (128, 20, 5, 4080, 1), (128, 32, 4, 4096, 0), (128, 32, 8, 1 << 30, 0)])
+def test_attention_in_chunks_of_80(dim, heads, kv_heads, room, five):
+    """Sides of the lines as they were measured over the positions of a cache: not for a few workgroups more than CUs, nor for one query head a kv head."""
+    assert harness().attn_five_waves(dim, heads, kv_heads, room) == five

@@ -786,8 +786,14 @@ def test_attn_decode_fused_vs_oracle(dev, po, kv_fp16, nh, nkv, hd, past):
 
 @pytest.mark.parametrize("nh,nkv,past", [(8, 8, 1998), (24, 8, 2077), (40, 8, 2156), (64, 8, 2239), (56, 8, 2398), (36, 9, 1840)])
 def test_attn_decode_five_waves_vs_oracle(dev, po, nh, nkv, past):
-    """Caches whose chunks of 64 would be more than 256 workgroups and those of 80 are not: three tokens over the ends of a wave's 16 positions and of a
+    """Caches whose chunks of 64 would be more than 256 workgroups and those of 80 are not, in chunks of either: three tokens over the ends of a wave's 16 positions and of a
     chunk, one to eight query heads per kv head."""
+    test_attn_decode_fused_vs_oracle(dev, po, True, nh, nkv, 128, past)
+
+
+@pytest.mark.parametrize("nh,nkv,past", [(16, 8, 2077), (32, 8, 2238), (40, 8, 79), (64, 8, 2398), (48, 8, 2492), (36, 9, 1902), (20, 10, 1758), (56, 7, 2556)])
+def test_attn_decode_chunks_of_80_vs_oracle(dev, po, nh, nkv, past):
+    """Caches that five waves a chunk take, and either side of their rule: three tokens over the ends of a wave's 16 positions, of a chunk and of the room."""
     test_attn_decode_fused_vs_oracle(dev, po, True, nh, nkv, 128, past)
 
 
