@@ -191,7 +191,8 @@ __device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t 
 
 // d = amax / 127 and id = 1 / d, 0 where d is, both correctly rounded: a quotient from a correctly rounded reciprocal (of 127 a constant, of d the
 // hardware's with one Newton step) is put right by one exact remainder (Markstein, IBM J. Res. Dev. 34, 1990).  6 instructions where the IEEE
-// sequences take 24; equal to them for every amax and d of 2^-100 .. 2^100, each compared.  Other amax, 0 and NaN among them: the IEEE sequences.
+// sequences take 24.  One step does not round every reciprocal of every hardware correctly; here it does, for each of the 2^23 amax of a binade and so,
+// by their scaling, of all from 2^-90 to 2^90 (test_quantize_q8_scales_are_ieee_quotients).  Other amax, 0 and NaN among them: the IEEE sequences.
 __device__ __forceinline__ void q8_scales(float amax, float& d, float& id) {
     const float r127 = 1.0f / 127.0f, q = amax * r127;
     d = fmaf(fmaf(-127.0f, q, amax), r127, q);

@@ -120,6 +120,43 @@ def test_quantize_q8_bit_exact(dev, po, golden):
     assert np.array_equal(q2, qo) and np.array_equal(bits(d2), bits(do)) and np.array_equal(bits(s2), bits(so))
 
 
+def _q8_of_maxima(amax):
+    """Blocks with these largest values, the others half way between two whole values (31 of 0.5 .. 122.5 times the scale, signs in turn): scale, sum and values of the
+    kernel, and of the IEEE quotients on the host."""
+    with np.errstate(all="ignore"):
+        d = amax / np.float32(127.0)
+        inv = np.where(d > 0, np.float32(1.0) / d, np.float32(0.0)).astype(np.float32)
+    D, I = cu(d), cu(inv)
+    ties = torch.arange(31, device="cuda").to(torch.float32) * 4 + torch.tensor([0.5, 1.5, 2.5], device="cuda").repeat(11)[:31]
+    x = torch.cat([cu(amax)[:, None], torch.minimum(D[:, None] * ties, cu(amax)[:, None])], 1)
+    x[:, 2::2].neg_()
+    K = x.numel()
+    buf = torch.zeros(ops.q8_bytes(K), dtype=torch.uint8, device="cuda")
+    ops.launch_quantize_q8(x, buf, K)
+    q = torch.clamp(torch.round(x * I[:, None]), -127, 127)
+    f = buf[K:].view(torch.float32)
+    n = len(amax)
+    return (f[:n], f[n:], buf[:K].view(torch.int8)), (D, D * q.sum(1), q.reshape(-1).to(torch.int8))
+
+
+def test_quantize_q8_scales_are_ieee_quotients(dev):
+    """d = amax / 127 and 1 / d, which the kernels make without the division sequences, for every largest value of a binade: scales and sums bit for bit, and the values, halves that
+    a scale's neighbour would round the other way; fewer of other binades out to where the sequences take over (2^-90, 2^90), the values beside those, and none."""
+    def same(amax):
+        got, want = _q8_of_maxima(amax)
+        for a, b in zip(got, want):
+            assert torch.equal(a.view(torch.int32) if a.dtype == torch.float32 else a, b.view(torch.int32) if b.dtype == torch.float32 else b)
+    for part in range(8):
+        same((np.arange(part << 20, (part + 1) << 20, dtype=np.uint32) + np.uint32(127 << 23)).view(np.float32))
+    for e in range(-90, 90, 12):
+        same((np.arange(e & 63, 1 << 23, 64, dtype=np.uint32) + np.uint32((127 + e) << 23)).view(np.float32))
+    edge = []
+    for e in (-118, -100, -91, -90, -89, 89, 90, 91, 100, 120):
+        v = np.float32(2.0) ** np.float32(e)
+        edge += [np.nextafter(v, np.float32(0.0)), v, np.nextafter(v, np.float32(np.inf)), v * np.float32(1.3)]
+    same(np.array(edge + [0.0] * 8, dtype=np.float32))
+
+
 # ---------------------------------------------------------------------------------------------
 # GEMV
 # ---------------------------------------------------------------------------------------------
