@@ -1529,6 +1529,14 @@ float qgemm_f16_rounds(int tiles, int M, bool q4) {
 // A row's sum does not depend on the choice.
 static bool qf_narrow(int M, int wide_workgroups) { return M <= 32 || (M <= 64 ? wide_workgroups <= 128 : (int64_t)wide_workgroups * ((M + 63) / 64) <= 256); }
 
+// Q4_K products of one split (where K may be split, 257 to 384 rows of 8193 to 10752 columns): where workgroups of 64 rows and 256 columns leave no CU two and would be more than half
+// the chip, but ones of 128 rows would not be, they are faster than twice as many of 128 columns, whose X each needs again: 280 / 384 rows, 9728 x 2560 31.4 / 33.2 ->
+// 29.4 / 32.2 us, x 4096 45.3 / 48.1 -> 43.2 / 46.7, 9216 x 1024 16.6 / 16.9 -> 15.6 / 16.6; of 512 values and of 8192 up to 4 % slower, of 14336
+// 3 % either way.  (Q6_K, more to unpack, 9728 x 2560: 54 us so, 46 narrow.)
+static bool qf_flat(int M, int K, int wide_workgroups) {
+    return M > 64 && K >= 1024 && K <= 4096 && wide_workgroups * ((M + 127) / 128) < 128 && (int64_t)wide_workgroups * ((M + 63) / 64) > 128;
+}
+
 static int qgemm_check(const void* W, const void* X, const void* Y, int M, int K, int N, int64_t stride, int blk_bytes) {
     if (!W || !X || !Y) return PTM_E_NULL;
     if (M <= 0 || N <= 0 || K <= 0 || (K % 256) != 0) return PTM_E_SHAPE;
@@ -1589,8 +1597,9 @@ int qgemm_f16_impl(uint32_t ggml_type, const void* W, const void* X, bool x_is_f
         else hipLaunchKernelGGL((qgemm_prepare_rows_f16_kernel<false, false>), dim3(mp), dim3(256), 0, s, X, Xh, rowscale, M, K);
     }
     const int wide = (N + QF_TN - 1) / QF_TN * splits;
-    const bool narrow = qf_narrow(M, wide);
-    const int MT = M <= 32 ? 1 : M <= 64 || narrow ? 2 : 4;  // tiles of 32 rows
+    const bool flat = q4 && splits == 1 && qf_flat(M, K, wide);
+    const bool narrow = !flat && qf_narrow(M, wide);
+    const int MT = M <= 32 ? 1 : M <= 64 || narrow || flat ? 2 : 4;  // tiles of 32 rows
     const int tm = 32 * MT;
     const size_t lds = 2 * (size_t)tm * QF_PITCH + 4 * (size_t)tm;  // two X tiles (64 rows: 66 KB) and the row scales: above the default 64 KB cap of dynamic LDS
     static std::once_flag raised;  // two host threads may get here at once: the second waits until the caps are raised

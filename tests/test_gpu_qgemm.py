@@ -364,6 +364,18 @@ def test_128_columns_and_several_row_tiles(dev, po, qt, M, K, N):
     assert np.array_equal(bits(y[64:]), bits(gpu_qgemm_f16(qt, W, xb[64:], M - 64, K, N)))
 
 
+@pytest.mark.parametrize("M,K,N", [(257, 1024, 8449), (320, 2560, 9728), (321, 1280, 10751), (384, 1024, 10752), (385, 1024, 9000), (300, 4096, 8200), (300, 4352, 8200), (300, 768, 9000),
+                                   (300, 1024, 8192), (190, 1024, 13001)])
+def test_64_rows_of_256_columns_in_several_row_tiles(dev, po, M, K, N):
+    """Q4_K products in one split, and beside the rule for these tiles: rows are those of calls of 64 rows, which have 128 columns, bit for bit."""
+    r = synth.rng_for(54, M, K, N)
+    W = synth.make_weight(r, 12, N, K)
+    xb, _ = bf16_round(r.standard_normal((M, K), dtype=np.float32))
+    y = gpu_qgemm_f16(12, W, xb, M, K, N)
+    for m in (0, 64, 100, M - 64):
+        assert np.array_equal(bits(y[m:m + 64]), bits(gpu_qgemm_f16(12, W, np.ascontiguousarray(xb[m:m + 64]), 64, K, N))), m
+
+
 # tiles of 256 rows: all (236 pairs of row tiles), whole rounds and 128-row tiles behind them (K splits off and on), an odd last row tile, ragged N; of 192
 # rows: 3 and 2 row tiles, whole and ragged, one of 129 rows
 @pytest.mark.parametrize("qt", [12, 14])
