@@ -1554,7 +1554,8 @@ static int fd_launch_g(int G, dim3 grid, hipStream_t s, const float* Q, const vo
 // steps: 32 heads on 8, room for 2240 / 2304 / 2368 / 2496 0.21 / 0.35 / 0.34 / 0.11 us less on average (0.3 to 0.9 more up to position 140,
 // 0.4 to 0.6 less from 1000 on); 40 on 10, 1750 / 1850 / 2000 0.36 / 0.40 / 0.43; 64 on 8, 2304 0.28; 32 on 16, 1088 0.23.  Of eight workgroups more than CUs it is
 // faster behind position 1600 only, 0.17 (32 on 8, 2064) to 0.38 us (64 on 8) slower on average; one query head a kv head is up to 0.14 slower at
-// any room (8 on 8, 2304: 0.03 less).
+// any room (8 on 8, 2304: 0.03 less).  Eight steps of twelve layers of 32 heads on 8, width 2560, room for 2064: five waves and four from position 500 3685, 3646 us,
+// 1300 3700, 3648, 2048 3706, 3735.
 bool attn_five_waves(int head_dim, int n_heads, int n_kv_heads, int max_seq) {
     const int64_t chunks = ((int64_t)max_seq + FD_CHUNK - 1) / FD_CHUNK, wide = ((int64_t)max_seq + 79) / 80;
     return head_dim == 128 && n_heads > n_kv_heads && chunks <= FD_LONG_SPLITS && chunks * n_kv_heads > 264 && wide * n_kv_heads <= 256;

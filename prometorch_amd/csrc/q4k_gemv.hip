@@ -36,8 +36,9 @@ __global__ __launch_bounds__(Q4K_THREADS) void q4k_gemv_kernel(const Q4KArgs a) 
 // MB is the order in which a CU's waves get their requests out: a wave that asks for all its blocks at once stands in the queue of the memory path for
 // up to 5 us, x behind the weights of others, and only then starts to stage x.  Here x goes out first (wave priority 3), then EARLY blocks, then
 // the staging (priority 2, in front of other waves' products), then the other blocks; 2.5 blocks of 20 waves, 40 KB a CU, keep HBM busy.  Weights
-// from HBM, in a graph behind a launch that writes x, that launch (2.1 us) included: gate / up 9728 x 2560 12.0 -> 9.6 us, 6144 x 4096 11.7 -> 9.9, q / k / v
-// 6144 x 2560 7.1 -> 6.3, 6144 x 4096 8.5 -> 7.7, o 2560 x 4096 5.7 -> 5.3.
+// from HBM, in a graph behind a launch that writes x, that launch (2.1 us) included: gate / up 9728 x 2560 12.0 -> 9.6 us, q / k / v 6144 x 2560 7.1 -> 6.3,
+// o 2560 x 4096 5.7 -> 5.3.  More than two pieces of x a thread are no gain (q / k / v 6144 x 4096 8.2 -> 8.1, gate / up 11.2 either way) and stay with
+// q4k_gemv_kernel.
 template <bool XQ8, bool NORM, bool ACC, int MODE, int NB, int LS, int PIECES>
 __global__ __launch_bounds__(64 * Q4K_ONE_WAVES) void q4k_gemv_one_kernel(const Q4KArgs a) {
     read_now(a.W[0], a.K, a.gamma);
@@ -204,7 +205,9 @@ template <bool XQ8, bool NORM, int MODE>
 static Q4KOne q4k_one(const Q4KArgs& a) {
     const int nblk = a.K / 256;
     int ls = a.log2S;
-    // q / k / v: six waves a CU with more blocks each are better than twelve (6144 x 2560: 6.5 -> 6.3 us)
+    // q / k / v: six waves a CU with more blocks each are better than twelve (6144 x 2560: 6.5 -> 6.3 us), from 6144 rows of four lane groups and 3072 of eight on: with twice the
+    // blocks and with the lane groups as they are 6144 x 2560 6.57, 7.03, 3072 x 2560 5.48, 5.93, but 5120 x 2560 6.33, 6.13, 2048 x 2560 5.81, 5.42 (5376 to
+    // 5888 rows, which stay with the latter, 0.2 to 0.4 less with the former).
     if (NORM && MODE == 0 && ls > 1 && (nblk + (1 << (ls - 1)) - 1) >> (ls - 1) <= 5 && (int64_t)a.total_rows << (ls - 1) >= 12288) --ls;
     const int nb = (nblk + (1 << ls) - 1) >> ls;
     if (ls < 1 || nb > 5 || a.add_one || a.stride >= 1ll << 31) return {0, 0, 0, 0};

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(Q6K_THREADS) __attribute__((amdgpu_waves_per_eu(3, 
 // Up to 16 rows per CU (down projections): a row per wave, its super-blocks strided over the wave's 8 lane groups, NT of them a group, one workgroup
 // per CU, so that x is staged once per CU instead of once per 4 rows.  Two blocks of a group in flight, one of them requested in front of the
 // staging (2560 x 9728 with one / two / three: 12.0 / 11.4 / 12.2 us).  Against passes in a loop, which pad the last one, weights from HBM, in a
-// graph with two small launches in front (3.7 us, included): 2560 x 9728 11.7 -> 11.4 us, 4096 x 14336 (eight waves of two rows) 17.1 -> 16.0, 1024 x 2816
+// graph with two small launches in front (3.7 us, included), results added to y (stored ones: q6k_rows_waves): 2560 x 9728 11.7 -> 11.4 us, 4096 x 14336 (eight waves of two rows) 17.1 -> 16.0, 1024 x 2816
 // (four rows a workgroup) 7.2 -> 6.9.
 enum { Q6K_ROWS_MAX_WAVES = 16 };
 template <bool ACC, int NT, int PIECES>
