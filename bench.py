@@ -472,9 +472,9 @@ def main():
     # and the Q6_K down projection accumulating into the residual.  `roofline` is the one that costs more per token.
     traffic, traffic_commit = measured_traffic()
     kernels = {
-        "gate_up": {"kernel": "q4k_gemv_kernel<fused rmsnorm + gate/up + silu> 2x9728x2560", "bytes_per_launch": gate_up_bytes,
+        "gate_up": {"kernel": "q4k_gemv_one_kernel<fused rmsnorm + gate/up + silu> 2x9728x2560", "bytes_per_launch": gate_up_bytes,
                     "us_per_launch": ms * 1e3, "launches_per_token": nL},
-        "down": {"kernel": "q6k_gemv_tall_kernel<accumulate> 2560x9728", "bytes_per_launch": b2, "us_per_launch": ms2 * 1e3,
+        "down": {"kernel": "q6k_gemv_rows_kernel<accumulate> 2560x9728", "bytes_per_launch": b2, "us_per_launch": ms2 * 1e3,
                  "launches_per_token": nL},
     }
     for key, kq in kernels.items():
